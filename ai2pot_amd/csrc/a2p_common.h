@@ -7,6 +7,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstdarg>
+#include <cstring>
 #include <string>
 
 #include "../../include/ai2pot_hip.h"
@@ -65,6 +66,10 @@ enum StatusBits {
     ST_SEG_OVERFLOW = 8,   // more pairs name one atom than its reduction segment holds (a list that is not symmetric)
     ST_GRID_BOUND = 16,    // neighbour list built without reading the extents back: the bin box outgrew its bound
 };
+
+// Copies nwords (< 32) 4-byte words from device memory to the host behind the work queued on `stream` and waits for
+// them; not for streams under capture.
+int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t stream);
 
 inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 

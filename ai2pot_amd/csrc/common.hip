@@ -1,6 +1,8 @@
 // Error state, per-device workspace and small utility kernels of libai2pot_hip.so.
 #include "a2p_common.h"
 
+#include <atomic>
+#include <chrono>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -98,6 +100,74 @@ int ws_release()
         b.bytes = 0;
     }
     g_ws_generation++;
+    return A2P_OK;
+}
+
+// ---- small results read back to the host -----------------------------------------------------
+// A status word or a dozen extents: one wavefront writes them to pinned host memory and then a sequence number, and
+// the host polls that number.  Bound by latency alone.  A copy to pageable memory and a stream synchronisation cost
+// 23 us behind a short kernel on an MI355X, the synchronisation alone 11.5 us, this 9.6 us: the write crosses the bus
+// as the kernel ends, with no completion signal, interrupt or staging buffer behind it.
+namespace {
+constexpr int RB_SLOTS = 64, RB_WORDS = 32;          // words per slot; word 0 is the sequence number
+std::mutex g_rb_mutex;
+int* g_rb_page = nullptr;                            // one pinned allocation for the process (8 KiB)
+std::atomic<unsigned long long> g_rb_used{0};        // slots in use, one bit each: a call holds one while it waits
+std::atomic<int> g_rb_seq{0};
+
+__global__ void read_back_kernel(const int* __restrict__ src, int nwords, int* host, int seq)
+{
+    const int l = (int)threadIdx.x;
+    if (l < nwords) __hip_atomic_store(host + 1 + l, src[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();                          // the words of all lanes (one wavefront) before the number
+    if (l == 0) __hip_atomic_store(host, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+}  // namespace
+
+int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t stream)
+{
+    A2P_REQUIRE(nwords > 0 && nwords < RB_WORDS, A2P_ERR_INVALID, "read_back: %d words", nwords);
+    {
+        std::lock_guard<std::mutex> lock(g_rb_mutex);
+        if (!g_rb_page) {
+            void* p = nullptr;
+            A2P_HIP_CHECK(hipHostMalloc(&p, RB_SLOTS * RB_WORDS * sizeof(int), hipHostMallocPortable));
+            for (int i = 0; i < RB_SLOTS * RB_WORDS; i++) ((int*)p)[i] = 0;
+            g_rb_page = (int*)p;
+        }
+    }
+    int slot = -1;
+    for (unsigned long long used = g_rb_used.load(); ~used != 0ull;) {
+        const int free_slot = __builtin_ctzll(~used);
+        if (g_rb_used.compare_exchange_weak(used, used | (1ull << free_slot))) { slot = free_slot; break; }
+    }
+    if (slot < 0) {                                  // more threads wait at once than there are slots
+        A2P_HIP_CHECK(hipMemcpyAsync(host_dst, device_src, (size_t)nwords * sizeof(int), hipMemcpyDeviceToHost, stream));
+        A2P_HIP_CHECK(hipStreamSynchronize(stream));
+        return A2P_OK;
+    }
+    int* const word = g_rb_page + slot * RB_WORDS;
+    int seq;
+    do seq = g_rb_seq.fetch_add(1) + 1; while (seq == 0 || seq == __atomic_load_n(word, __ATOMIC_RELAXED));
+    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, (const int*)device_src, nwords, word, seq);
+    hipError_t err = hipGetLastError();
+    if (err == hipSuccess) {
+        // polling pays while the wait is short; behind a long queue (or after a fault, when the number never
+        // arrives) the runtime's own wait takes over
+        const auto began = std::chrono::steady_clock::now();
+        bool there = false;
+        while (!(there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq)) {
+            for (int i = 0; i < 16; i++) __builtin_ia32_pause();
+            if (std::chrono::steady_clock::now() - began > std::chrono::milliseconds(1)) break;
+        }
+        if (!there) {
+            err = hipStreamSynchronize(stream);
+            if (err == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) err = hipErrorUnknown;
+        }
+        if (err == hipSuccess) memcpy(host_dst, word + 1, (size_t)nwords * sizeof(int));
+    }
+    g_rb_used.fetch_and(~(1ull << slot));
+    A2P_HIP_CHECK(err);
     return A2P_OK;
 }
 
@@ -351,8 +421,8 @@ int a2p_check_status(void* stream_)
     int rc = a2p::ws_get(a2p::WS_FLAGS, 64, &flags);
     if (rc) return rc;
     int host = 0;
-    A2P_HIP_CHECK(hipMemcpyAsync(&host, flags, sizeof(int), hipMemcpyDeviceToHost, stream));
-    A2P_HIP_CHECK(hipStreamSynchronize(stream));
+    rc = a2p::read_back(flags, 1, &host, stream);
+    if (rc) return rc;
     if (host == 0) return A2P_OK;
     rc = a2p::fill_zero(flags, 64, stream);
     if (rc) return rc;

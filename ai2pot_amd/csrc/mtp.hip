@@ -2117,8 +2117,8 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
     rc = exclusive_scan_i32(nnc, pair_off, rows + 1, tmp, stream);
     if (rc) return rc;
     int npairs = 0;                         // sizes the pair buffer: one read-back per call
-    A2P_HIP_CHECK(hipMemcpyAsync(&npairs, pair_off + rows, sizeof(int), hipMemcpyDeviceToHost, stream));
-    A2P_HIP_CHECK(hipStreamSynchronize(stream));
+    rc = read_back(pair_off + rows, 1, &npairs, stream);
+    if (rc) return rc;
     if (npairs < 0) npairs = 0;
     // pair derivatives | row sums | scalar moments | list of the pairs that name each atom
     const size_t n_pb = (size_t)std::max(npairs, 1) * 3 * S, n_rp = (size_t)rows * 12 * S, n_desc = (size_t)rows * S;

@@ -1327,8 +1327,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                            cap[2], big_coord, status);
     } else {
         T ext[12];
-        A2P_HIP_CHECK(hipMemcpyAsync(ext, ext_dev, sizeof(ext), hipMemcpyDeviceToHost, stream));
-        A2P_HIP_CHECK(hipStreamSynchronize(stream));
+        rc = read_back(ext_dev, (int)(sizeof(ext) / 4), ext, stream);
+        if (rc) return rc;
 
         // find_pl_info4nblist + bin counts (structure.h:1013-1061, binLinkedList.h:685-688)
         for (int a = 0; a < 3; a++) {
@@ -1404,8 +1404,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     long long total = (long long)N * g.nimg;
     if (total * (long long)(4 * sizeof(T)) > (2ll << 30)) {
         int counted = 0;
-        A2P_HIP_CHECK(hipMemcpyAsync(&counted, offsets + nregion, sizeof(int), hipMemcpyDeviceToHost, stream));
-        A2P_HIP_CHECK(hipStreamSynchronize(stream));
+        rc = read_back(offsets + nregion, 1, &counted, stream);
+        if (rc) return rc;
         total = counted;
     }
 
@@ -1546,8 +1546,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                            numneigh, N, status + 1);
         prof_end(stream);
         int st[2] = {0, 0};
-        A2P_HIP_CHECK(hipMemcpyAsync(st, status, sizeof(st), hipMemcpyDeviceToHost, stream));
-        A2P_HIP_CHECK(hipStreamSynchronize(stream));
+        rc = read_back(status, 2, st, stream);
+        if (rc) return rc;
         *max_nn_host = st[1];
         if (st[1] > umax) {
             rc = fill_zero(status, sizeof(int), stream);

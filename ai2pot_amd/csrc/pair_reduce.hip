@@ -491,9 +491,7 @@ extern "C" int a2p_pair_incoming_max(int batch, int natoms_pad, int umax, int ng
     hipLaunchKernelGGL(incoming_max_kernel, dim3(std::min(ceil_div((long long)n, 256), 1024)), dim3(256), 0, stream,
                        (const int*)counts, (int)n, counts + n);
     A2P_HIP_CHECK(hipGetLastError());
-    A2P_HIP_CHECK(hipMemcpyAsync(max_incoming, counts + n, sizeof(int), hipMemcpyDeviceToHost, stream));
-    A2P_HIP_CHECK(hipStreamSynchronize(stream));
-    return A2P_OK;
+    return read_back(counts + n, 1, max_incoming, stream);
 }
 
 extern "C" int a2p_pair_ranks(int batch, int natoms_pad, int umax, int nghost, const int* binum, const int* bnumneigh,
