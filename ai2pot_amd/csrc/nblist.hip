@@ -506,7 +506,13 @@ constexpr int NBL_UNROLL = 4;
 constexpr int NBL_ENT_CAP = 256;   // flat candidate list per atom (entries); longer lists search the runs
 
 template <typename T>
-inline size_t rowbuf_bytes(int umax, bool rank) { return (size_t)umax * (4 + 3 * sizeof(T) + (rank ? 4 : 0)); }
+inline size_t rowbuf_bytes(int umax, bool rank, bool sort = false)
+{
+    return (size_t)umax * (4 + 3 * sizeof(T) + (rank ? 4 : 0) + (sort ? sizeof(T) : 0));
+}
+// Rows up to this long are put in order by the wavefront that built them (four entries per lane in registers; an
+// entry's place fits a byte in sort_tied_rows_kernel).
+constexpr int NBL_SORT_CAP = 256;
 
 // Run of supercell entries that column `lane` of the (2e+1)^2 columns around the bin of the atom at
 // c can contribute: start index and length (0 for lanes without a column or with nothing in reach).
@@ -629,9 +635,10 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
              int umax, int* __restrict__ ilist, int* __restrict__ numneigh, int* __restrict__ firstneigh,
              T* __restrict__ rcs, int* __restrict__ types_out, T* __restrict__ keys,
              int* __restrict__ status, int update, int* __restrict__ rank_out, int* __restrict__ incoming,
-             const CompactEmit<T> ce, const GridDyn<T>* __restrict__ gd)
+             const CompactEmit<T> ce, const GridDyn<T>* __restrict__ gd, int* __restrict__ tied = nullptr)
 {
     static_assert(!COMPACT || (ROWBUF && !SORT && !RANK), "compact lists are cut from the row held in LDS");
+    static_assert(!(SORT && RANK), "places belong to unsorted rows");
     const Grid<T> g = with_dyn(g_in, gd);
     __shared__ int sh_start[NBL_BLOCK / 64][64];
     __shared__ int sh_base[NBL_BLOCK / 64][64];
@@ -646,10 +653,12 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     T* rb_rcs = nullptr;
     int* rb_first = nullptr;
     int* rb_rank = nullptr;
+    T* rb_key = nullptr;
     if (ROWBUF) {
-        unsigned char* mine = sh_rows + (size_t)wv * umax * (4 + 3 * sizeof(T) + (RANK ? 4 : 0));
+        unsigned char* mine = sh_rows + (size_t)wv * umax * (4 + 3 * sizeof(T) + (RANK ? 4 : 0) + (SORT ? sizeof(T) : 0));
         rb_rcs = (T*)mine;
-        rb_first = (int*)(mine + (size_t)umax * 3 * sizeof(T));
+        rb_key = rb_rcs + (size_t)umax * 3;                            // SORT: the rounded distances
+        rb_first = (int*)(mine + (size_t)umax * (SORT ? 4 : 3) * sizeof(T));
         rb_rank = rb_first + umax;
     }
     // A row costs three dependent trips to memory (coordinates, column runs, candidates).  The
@@ -777,7 +786,8 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
                     rcs[(rowi + slot) * 3 + 1] = dy;
                     rcs[(rowi + slot) * 3 + 2] = dz;
                 }
-                if (SORT) keys[rowi + slot] = (T)__dsqrt_rn(d2d);      // neighborList.h:318-322
+                if (SORT && ROWBUF) rb_key[slot] = (T)__dsqrt_rn(d2d); // neighborList.h:318-322
+                else if (SORT) keys[rowi + slot] = (T)__dsqrt_rn(d2d);
                 if (RANK) {
                     rk[u] = atomicAdd(&incoming[sj[u]], 1);
                     rs[u] = slot;
@@ -856,6 +866,59 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         // the padded row lists plain indices
         if (rows)
             for (int e = lane; e < used; e += 64) rb_first[e] &= CL_IMAGE_BIT - 1;
+    }
+    if (SORT && ROWBUF) {
+        // The row in order of distance.  With no two distances equal the order is unique: an entry's place is the
+        // number of smaller distances, counted over the keys in LDS (every lane reads the same one: a broadcast, four
+        // keys per 16-byte read in fp32), and the entries go from registers to their places.  A row with equal
+        // distances keeps the order it was found in and is flagged for sort_tied_rows_kernel, which repeats the
+        // reference's own sequence of moves.  Bound by the padded rows written: 131072 atoms, 36 neighbours, fp64,
+        // umax 200 take 0.156 ms (4.7 TB/s); rows through global memory, a sort by a thread per row and a gather took
+        // 0.176 + 0.898 + 0.241 ms.
+        __builtin_amdgcn_wave_barrier();
+        const int used = min(cnt, umax);          // wave-uniform, at most NBL_SORT_CAP
+        const int quads = (used + 3) / 4;
+        if (lane < quads * 4 - used) rb_key[used + lane] = (T)INFINITY;        // umax is a multiple of 4
+        __builtin_amdgcn_wave_barrier();
+        int place[NBL_SORT_CAP / 64];
+        bool tie = false;
+#pragma unroll
+        for (int u = 0; u < NBL_SORT_CAP / 64; u++) {
+            if (u * 64 >= used) break;
+            const int e = u * 64 + lane;
+            const bool have = e < used;
+            const T k = rb_key[have ? e : 0];
+            int less = 0, same = 0;
+            for (int q = 0; q < quads; q++) {
+                struct alignas(16) Quad { T v[4]; };
+                const Quad o = reinterpret_cast<const Quad*>(rb_key)[q];
+#pragma unroll
+                for (int i = 0; i < 4; i++) { less += o.v[i] < k ? 1 : 0; same += o.v[i] == k ? 1 : 0; }
+            }
+            place[u] = less;
+            tie |= have && same != 1;
+        }
+        const bool tied_row = __ballot(tie) != 0ull;
+        if (lane == 0) tied[p] = tied_row ? 1 : 0;
+        if (!tied_row) {
+            int ef[NBL_SORT_CAP / 64];
+            T ex[NBL_SORT_CAP / 64], ey[NBL_SORT_CAP / 64], ez[NBL_SORT_CAP / 64];
+#pragma unroll
+            for (int u = 0; u < NBL_SORT_CAP / 64; u++) {
+                if (u * 64 >= used) break;
+                const int e = min(u * 64 + lane, used - 1);
+                ef[u] = rb_first[e]; ex[u] = rb_rcs[e * 3]; ey[u] = rb_rcs[e * 3 + 1]; ez[u] = rb_rcs[e * 3 + 2];
+            }
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int u = 0; u < NBL_SORT_CAP / 64; u++) {
+                if (u * 64 >= used) break;
+                if (u * 64 + lane < used) {
+                    const int e = place[u];
+                    rb_first[e] = ef[u]; rb_rcs[e * 3] = ex[u]; rb_rcs[e * 3 + 1] = ey[u]; rb_rcs[e * 3 + 2] = ez[u];
+                }
+            }
+        }
     }
     if (ROWBUF && rows) {
         __builtin_amdgcn_wave_barrier();
@@ -985,12 +1048,12 @@ compact_symmetry_kernel(const Grid<T> g_in, const GridDyn<T>* __restrict__ gd, c
 // Introsort: median-of-three quicksort down to partitions of 16, heap sort beyond depth
 // 2*floor(log2 n), then one insertion sort pass.  Only the sequence of comparisons and moves
 // decides where equal keys end up, so the published algorithm is followed step by step.
-template <typename T>
+template <typename T, typename I>
 struct IdxSorter {
-    int* v;          // index array being sorted
+    I* v;            // index array being sorted
     const T* d;      // keys
     __device__ bool less(int a, int b) const { return d[a] < d[b]; }
-    __device__ void iter_swap(int i, int j) { int t = v[i]; v[i] = v[j]; v[j] = t; }
+    __device__ void iter_swap(int i, int j) { I t = v[i]; v[i] = v[j]; v[j] = t; }
 
     __device__ void move_median_to_first(int result, int a, int b, int c)
     {
@@ -1120,8 +1183,75 @@ __global__ void sort_rows_kernel(int N, int umax, const int* __restrict__ numnei
     const int n = min(numneigh[p], umax);
     int* v = order + (size_t)p * umax;
     for (int j = 0; j < n; j++) v[j] = j;
-    IdxSorter<T> s{v, keys + (size_t)p * umax};
+    IdxSorter<T, int> s{v, keys + (size_t)p * umax};
     s.sort(n);
+}
+
+// Rows with equal distances (flagged by the list kernel; every row of a perfect crystal, none or a handful otherwise).
+// A wavefront looks at 64 rows.  The keys of as many flagged rows as fit its LDS are formed from the rows as they
+// stand, one lane per row runs the reference's moves there, and the wavefront puts the rows in order.  A serial chain
+// of dependent LDS reads bounds it; the same chain over global memory took 0.90 ms for 131072 rows of 36.
+template <typename T>
+__global__ void __launch_bounds__(64)
+sort_tied_rows_kernel(int N, int umax, int lds_bytes, const int* __restrict__ numneigh, const int* __restrict__ tied,
+                      int* __restrict__ firstneigh, T* __restrict__ rcs)
+{
+    extern __shared__ __align__(16) unsigned char sh_tied[];
+    const int lane = (int)threadIdx.x, p0 = (int)blockIdx.x * 64;
+    const bool mine = p0 + lane < N && tied[p0 + lane] != 0;
+    unsigned long long todo = __ballot(mine);
+    if (todo == 0ull) return;
+    const int n_mine = mine ? min(numneigh[p0 + lane], umax) : 0;
+    const int stride = (wave_max(n_mine) + 3) & ~3;                   // entries per row, at most umax
+    const int group = min(64, lds_bytes / (stride * (int)(sizeof(T) + 1)));
+    T* const keys = (T*)sh_tied;
+    unsigned char* const order = sh_tied + (size_t)group * stride * sizeof(T);
+    while (todo != 0ull) {
+        unsigned long long chosen = 0ull;
+        int slot = -1, rows = 0;                                      // the LDS row of this lane's row, if chosen
+        for (; rows < group && todo != 0ull; rows++) {
+            const int l = __builtin_ctzll(todo);
+            todo &= todo - 1ull;
+            chosen |= 1ull << l;
+            if (l == lane) slot = rows;
+        }
+        int k = 0;
+        for (unsigned long long left = chosen; left != 0ull; left &= left - 1ull, k++) {
+            const int l = __builtin_ctzll(left), n = __shfl(n_mine, l, 64);
+            const T* const r = rcs + (size_t)(p0 + l) * umax * 3;
+            for (int e = lane; e < n; e += 64) {
+                keys[k * stride + e] = (T)__dsqrt_rn(dist2_double<T>(r[e * 3], r[e * 3 + 1], r[e * 3 + 2]));
+                order[k * stride + e] = (unsigned char)e;
+            }
+        }
+        __syncthreads();
+        if (slot >= 0) {
+            IdxSorter<T, unsigned char> s{order + slot * stride, keys + (size_t)slot * stride};
+            s.sort(n_mine);
+        }
+        __syncthreads();
+        k = 0;
+        for (unsigned long long left = chosen; left != 0ull; left &= left - 1ull, k++) {
+            const int l = __builtin_ctzll(left), n = __shfl(n_mine, l, 64);
+            int* const f = firstneigh + (size_t)(p0 + l) * umax;
+            T* const r = rcs + (size_t)(p0 + l) * umax * 3;
+            int ef[NBL_SORT_CAP / 64];
+            T ex[NBL_SORT_CAP / 64], ey[NBL_SORT_CAP / 64], ez[NBL_SORT_CAP / 64];
+#pragma unroll
+            for (int u = 0; u < NBL_SORT_CAP / 64; u++) {
+                if (u * 64 >= n) break;
+                const int src = order[k * stride + min(u * 64 + lane, n - 1)];
+                ef[u] = f[src]; ex[u] = r[src * 3]; ey[u] = r[src * 3 + 1]; ez[u] = r[src * 3 + 2];
+            }
+#pragma unroll
+            for (int u = 0; u < NBL_SORT_CAP / 64; u++) {
+                if (u * 64 >= n) break;
+                const int e = u * 64 + lane;
+                if (e < n) { f[e] = ef[u]; r[e * 3] = ex[u]; r[e * 3 + 1] = ey[u]; r[e * 3 + 2] = ez[u]; }
+            }
+        }
+        __syncthreads();
+    }
 }
 
 // out row = tmp row gathered through `order` (SingleNeighborListArrangement, neighborList.h:46-67)
@@ -1410,7 +1540,15 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     }
 
     size_t sorted_bytes = (size_t)total * 4 * sizeof(T) + 256;
-    size_t sort_bytes = sort ? (size_t)N * umax * (2 * sizeof(int) + 4 * sizeof(T)) + 256 : 0;
+    // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
+    // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;
+    // otherwise through global memory by a thread per row
+    const bool sort_in_place = sort && umax % 4 == 0 && umax <= NBL_SORT_CAP && (uintptr_t)firstneigh % 16 == 0 &&
+                               (uintptr_t)rcs % 16 == 0 &&
+                               rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64) <= 48 * 1024;
+    size_t sort_bytes = sort_in_place ? (size_t)N * sizeof(int) + 256
+                        : sort        ? (size_t)N * umax * (2 * sizeof(int) + 4 * sizeof(T)) + 256
+                                      : 0;
     void* wsC = nullptr;
     rc = ws_get(WS_MISC, sorted_bytes + sort_bytes, &wsC);
     if (rc) return rc;
@@ -1420,7 +1558,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     T* keys = nullptr;
     int* order = nullptr;
     int* tmp_first = nullptr;
-    if (sort) {
+    int* const tied = (int*)sort_base;
+    if (sort && !sort_in_place) {
         tmp_rcs = (T*)sort_base;
         keys = tmp_rcs + (size_t)N * umax * 3;
         order = (int*)(keys + (size_t)N * umax);
@@ -1498,6 +1637,11 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         hipLaunchKernelGGL((lists_kernel<T, false, true, false, true>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds,
                            stream, g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out,
                            keys, status, update, nullptr, nullptr, ce, (const GridDyn<T>*)gd);
+    else if (sort_in_place)
+        hipLaunchKernelGGL((lists_kernel<T, true, true, false>), dim3(list_blocks), dim3(NBL_BLOCK),
+                           rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64), stream, g, x, types, offsets, s_rec, umax,
+                           ilist, numneigh, firstneigh, rcs, types_out, keys, status, update, nullptr, nullptr,
+                           CompactEmit<T>{}, (const GridDyn<T>*)gd, tied);
     else if (sort)
         hipLaunchKernelGGL((lists_kernel<T, true, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, tmp_first, tmp_rcs, types_out, keys,
@@ -1525,7 +1669,13 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                            stream, g, (const GridDyn<T>*)gd, (const T*)x, ce, umax, status);
         prof_end(stream);
     }
-    if (sort) {
+    if (sort_in_place) {
+        constexpr int lds = 32 * 1024;            // a row of NBL_SORT_CAP fp64 keys and places takes 2304 bytes of it
+        prof_begin("nbl_sort_rows", stream);
+        hipLaunchKernelGGL(sort_tied_rows_kernel<T>, dim3(ceil_div(N, 64)), dim3(64), lds, stream, N, umax, lds,
+                           (const int*)numneigh, (const int*)tied, firstneigh, rcs);
+        prof_end(stream);
+    } else if (sort) {
         prof_begin("nbl_sort_rows", stream);
         hipLaunchKernelGGL(sort_rows_kernel<T>, dim3(ceil_div(N, 64)), dim3(64), 0, stream, N, umax, numneigh,
                            keys, order);
