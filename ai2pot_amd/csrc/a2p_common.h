@@ -70,6 +70,17 @@ enum StatusBits {
 // Copies nwords (< 32) 4-byte words from device memory to the host behind the work queued on `stream` and waits for
 // them; not for streams under capture.
 int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t stream);
+// The same in two steps, so that the host can queue more work in between.  Every post is waited for, once.
+struct ReadBack {
+    const void* src;
+    int nwords, slot, seq;
+    hipStream_t stream;
+};
+int read_back_post(const void* device_src, int nwords, hipStream_t stream, ReadBack* rb);
+int read_back_wait(const ReadBack& rb, void* host_dst);
+// Called where every check of the call's inputs has been queued: posts the status word if the calling thread asked
+// for it (a2p_status_early).
+int status_post_early(hipStream_t stream);
 
 inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 

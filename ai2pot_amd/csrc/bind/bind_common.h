@@ -110,14 +110,20 @@ inline void check_device_status(const at::Tensor& t)
 // A list that names an atom more often than a row is long (half lists, ghosts collecting the pairs of
 // several rows) overflows the fixed reduction segments of the fast kernels: the status says so and
 // the call is repeated once with segments sized for the list at hand.
+// early: a loss call, whose status is final before its gradient kernels run; the host then goes on (to the backward
+// call, as a rule) while they do.
 template <class Call>
 inline void run_checked(const at::Tensor& brcs, const at::Tensor& binum, const at::Tensor& bnumneigh,
-                        const at::Tensor& bfirstneigh, int nghost, Call&& call)
+                        const at::Tensor& bfirstneigh, int nghost, Call&& call, bool early = false)
 {
-    check_rc(call());
+    early = early && validate_flag();
+    if (early) a2p_status_early(1);
+    int rc = call();
+    if (early && rc != A2P_OK) a2p_status_early(0);
+    check_rc(rc);
     if (!validate_flag()) return;
     void* st = current_stream(brcs);
-    int rc = a2p_check_status(st);
+    rc = early ? a2p_check_status_early(st) : a2p_check_status(st);
     if (rc == A2P_ERR_SEGMENT) {
         int most = 0;
         check_rc(a2p_pair_incoming_max((int)brcs.size(0), (int)brcs.size(1), (int)brcs.size(2), nghost,
@@ -198,6 +204,95 @@ inline at::Tensor zbl_esites(double zbl_rmax, double zbl_rmin, const at::Tensor&
     check_rc(rc);
     check_device_status(brcs);
     return out;
+}
+
+// What the loss functions of the three families share around their library call.
+
+// Tensor over elements [beg, beg + numel(shape)) of a one-dimensional one, without the view relation to it: an
+// operator's outputs that share an allocation can then be written in place by their owner like any others.
+inline at::Tensor piece(const at::Tensor& flat, int64_t beg, at::IntArrayRef shape)
+{
+    at::AutoDispatchBelowADInplaceOrView guard;
+    int64_t n = 1;
+    for (int64_t d : shape) n *= d;
+    return flat.narrow(0, beg, n).view(shape);
+}
+
+// Per-structure gradients of the parameters in one allocation: [B, numel(p)] of each parameter behind one another.
+struct GradRows {
+    at::Tensor flat;
+    int64_t B = 0;
+    std::vector<int64_t> numel;          // of each parameter
+    GradRows(int64_t B_, std::initializer_list<const at::Tensor*> params, const at::TensorOptions& opt, bool fresh) : B(B_)
+    {
+        int64_t total = 0;
+        for (auto* p : params) { numel.push_back(p->numel()); total += p->numel(); }
+        flat = fresh ? at::empty({B * total}, opt) : at::zeros({B * total}, opt);
+    }
+    template <typename T>
+    T* ptr(int i) const
+    {
+        int64_t beg = 0;
+        for (int k = 0; k < i; k++) beg += numel[k];
+        return flat.data_ptr<T>() + B * beg;
+    }
+};
+
+inline void save_grad_rows(torch::autograd::AutogradContext* ctx, bool need, const GradRows* rows,
+                           std::initializer_list<const at::Tensor*> params)
+{
+    std::vector<int64_t> shapes;         // dimensions and sizes of each parameter
+    if (need) {
+        ctx->save_for_backward({rows->flat});
+        for (auto* p : params) {
+            shapes.push_back(p->dim());
+            shapes.insert(shapes.end(), p->sizes().begin(), p->sizes().end());
+        }
+    }
+    ctx->saved_data["shapes"] = shapes;  // empty: no parameter wants a gradient
+}
+
+// grad_output @ dloss/dtheta of every parameter, in one launch; out[first + i] receives parameter i's.
+inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tensor& grad_output,
+                          torch::autograd::variable_list& out, int first)
+{
+    const std::vector<int64_t> shapes = ctx->saved_data["shapes"].toIntVector();
+    if (shapes.empty()) return;
+    const at::Tensor flat = ctx->get_saved_variables()[0];
+    const at::Tensor gl = grad_output.contiguous();
+    const int64_t B = gl.numel();
+    std::vector<std::vector<int64_t>> shape;
+    std::vector<long long> numel;
+    long long total = 0;
+    for (size_t i = 0; i < shapes.size(); i += 1 + shapes[i]) {
+        shape.emplace_back(shapes.begin() + i + 1, shapes.begin() + i + 1 + shapes[i]);
+        long long n = 1;
+        for (int64_t d : shape.back()) n *= d;
+        numel.push_back(n);
+        total += n;
+    }
+    const int np = (int)shape.size();
+    // a backward pass that is itself differentiated (in grad_output) goes through operators autograd knows
+    if (B == 0 || (at::GradMode::is_enabled() && gl.requires_grad())) {
+        for (int64_t i = 0, beg = 0; i < np; beg += numel[i] * B, i++)
+            out[first + i] = torch::matmul(gl, flat.narrow(0, beg, numel[i] * B).view({B, (int64_t)numel[i]})).view(shape[i]);
+        return;
+    }
+    DeviceGuard guard(flat);
+    const at::Tensor sums = at::empty({(int64_t)total}, flat.options());
+    void* st = current_stream(flat);
+    int rc;
+    if (flat.scalar_type() == at::kDouble) {
+        std::vector<const double*> parts;
+        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) parts.push_back(flat.data_ptr<double>() + beg);
+        rc = a2p_weighted_rows_f64((int)B, gl.data_ptr<double>(), np, parts.data(), numel.data(), sums.data_ptr<double>(), st);
+    } else {
+        std::vector<const float*> parts;
+        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) parts.push_back(flat.data_ptr<float>() + beg);
+        rc = a2p_weighted_rows_f32((int)B, gl.data_ptr<float>(), np, parts.data(), numel.data(), sums.data_ptr<float>(), st);
+    }
+    check_rc(rc);
+    for (int64_t i = 0, beg = 0; i < np; beg += numel[i], i++) out[first + i] = piece(sums, beg, shape[i]);
 }
 
 // Labels of a loss operator with the ZBL pair repulsion taken out.  The correction does not depend

@@ -108,54 +108,45 @@ struct LossFunction : public torch::autograd::Function<LossFunction> {
                     "label tensors must have shapes [B], [B, P, 3], [B, 9]");
         const bool need = coeffs.requires_grad() || lin.requires_grad() || bias.requires_grad();
         // the library writes every element of these outputs when the batch is not empty
-        auto out = [&](at::IntArrayRef shape) { return B > 0 && P > 0 ? at::empty(shape, opt) : at::zeros(shape, opt); };
-        at::Tensor bloss = out({B}), rmse = out({3}), e = out({B}), f = out({B, P, 3}), v = out({B, 9}), dc, dl, db;
-        if (need) {
-            dc = out({B, coeffs.numel()});
-            dl = out({B, lin.numel()});
-            db = out({B, bias.numel()});
-        }
+        const bool fresh = B > 0 && P > 0;
+        auto out = [&](int64_t n) { return fresh ? at::empty({n}, opt) : at::zeros({n}, opt); };
+        const int64_t nf = (int64_t)B * P * 3;
+        at::Tensor bloss = out(B), rmse = out(3), efv = out(B + nf + (int64_t)B * 9);
+        const GradRows rows(need ? B : 0, {&coeffs, &lin, &bias}, opt, fresh);
         void* st = current_stream(brcs);
         auto call = [&]() -> int {
             int rc;
             if (brcs.scalar_type() == at::kDouble) {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<double>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<double>(); };
+                auto g = [&](int i) { return need ? rows.ptr<double>(i) : nullptr; };
                 rc = a2p_mtp_loss_f64(c.plan.handle, e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft),
                                       (int)K, scaling, p(coeffs), p(lin), p(bias), (int)nmus, c.ntypes, p(q_scaler),
                                       rmax, rmin, B, P, c.s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(),
                                       bnumneigh.data_ptr<int>(), bfirstneigh.data_ptr<int>(), p(brcs),
-                                      btypes.data_ptr<int>(), p(bloss), p(rmse), p(e), p(f), p(v), p(dc), p(dl), p(db),
+                                      btypes.data_ptr<int>(), p(bloss), p(rmse), p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2),
                                       st);
             } else {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<float>(); };
+                auto g = [&](int i) { return need ? rows.ptr<float>(i) : nullptr; };
                 rc = a2p_mtp_loss_f32(c.plan.handle, e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft),
                                       (int)K, scaling, p(coeffs), p(lin), p(bias), (int)nmus, c.ntypes, p(q_scaler),
                                       rmax, rmin, B, P, c.s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(),
                                       bnumneigh.data_ptr<int>(), bfirstneigh.data_ptr<int>(), p(brcs),
-                                      btypes.data_ptr<int>(), p(bloss), p(rmse), p(e), p(f), p(v), p(dc), p(dl), p(db),
+                                      btypes.data_ptr<int>(), p(bloss), p(rmse), p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2),
                                       st);
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
-        ctx->saved_data["need"] = need;
-        if (need) ctx->save_for_backward({dc, dl, db});
-        ctx->saved_data["shape_c"] = coeffs.sizes().vec();
-        ctx->saved_data["shape_l"] = lin.sizes().vec();
-        ctx->saved_data["shape_b"] = bias.sizes().vec();
-        if (with_virial) return {bloss, rmse.slice(0, 0, 1).clone(), rmse.slice(0, 1, 2).clone(), rmse.slice(0, 2, 3).clone()};
-        return {bloss, rmse.slice(0, 0, 1).clone(), rmse.slice(0, 1, 2).clone()};
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        save_grad_rows(ctx, need, &rows, {&coeffs, &lin, &bias});
+        if (with_virial) return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1}), piece(rmse, 2, {1})};
+        return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1})};
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         variable_list out(28);                   // one slot per forward argument after ctx
-        if (!ctx->saved_data["need"].toBool()) return out;
-        auto saved = ctx->get_saved_variables();
-        at::Tensor gl = grads[0].contiguous();
-        out[9] = torch::matmul(gl, saved[0]).reshape(ctx->saved_data["shape_c"].toIntVector());
-        out[10] = torch::matmul(gl, saved[1]).reshape(ctx->saved_data["shape_l"].toIntVector());
-        out[11] = torch::matmul(gl, saved[2]).reshape(ctx->saved_data["shape_b"].toIntVector());
+        grad_products(ctx, grads[0], out, 9);    // coeffs, linear_coeffs, type_bias
         return out;
     }
 };

@@ -183,57 +183,43 @@ struct NepLossFunction : public torch::autograd::Function<NepLossFunction> {
         const bool need = coeffs.requires_grad() || w0.requires_grad() || b0.requires_grad() ||
                           w1.requires_grad() || bias.requires_grad();
         // the library writes every element of these outputs when the batch is not empty
-        auto out = [&](at::IntArrayRef shape) { return B > 0 && P > 0 ? at::empty(shape, opt) : at::zeros(shape, opt); };
-        at::Tensor bloss = out({B}), rmse = out({3}), e = out({B}), f = out({B, P, 3}), v = out({B, 9}), dc, dw0, db0, dw1, db;
-        if (need) {
-            dc = out({B, coeffs.numel()});
-            dw0 = out({B, w0.numel()});
-            db0 = out({B, b0.numel()});
-            dw1 = out({B, w1.numel()});
-            db = out({B, bias.numel()});
-        }
+        const bool fresh = B > 0 && P > 0;
+        auto out = [&](int64_t n) { return fresh ? at::empty({n}, opt) : at::zeros({n}, opt); };
+        const int64_t nf = (int64_t)B * P * 3;
+        at::Tensor bloss = out(B), rmse = out(3), efv = out(B + nf + (int64_t)B * 9);
+        const GradRows rows(need ? B : 0, {&coeffs, &w0, &b0, &w1, &bias}, opt, fresh);
         void* st = current_stream(brcs);
         auto call = [&]() -> int {
             int rc;
             if (brcs.scalar_type() == at::kDouble) {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<double>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<double>(); };
+                auto g = [&](int i) { return need ? rows.ptr<double>(i) : nullptr; };
                 rc = a2p_nep_loss_f64(e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft), m.K, m.n_r, m.n_a,
                                       m.l_max, m.H, m.ntypes, p(coeffs), p(w0), p(b0), p(w1), p(bias), p(q_scaler), rr, ra,
                                       B, P, s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(), bnumneigh.data_ptr<int>(),
                                       bfirstneigh.data_ptr<int>(), p(brcs), btypes.data_ptr<int>(), p(bloss), p(rmse),
-                                      p(e), p(f), p(v), p(dc), p(dw0), p(db0), p(dw1), p(db), st);
+                                      p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2), g(3), g(4), st);
             } else {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<float>(); };
+                auto g = [&](int i) { return need ? rows.ptr<float>(i) : nullptr; };
                 rc = a2p_nep_loss_f32(e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft), m.K, m.n_r, m.n_a,
                                       m.l_max, m.H, m.ntypes, p(coeffs), p(w0), p(b0), p(w1), p(bias), p(q_scaler), rr, ra,
                                       B, P, s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(), bnumneigh.data_ptr<int>(),
                                       bfirstneigh.data_ptr<int>(), p(brcs), btypes.data_ptr<int>(), p(bloss), p(rmse),
-                                      p(e), p(f), p(v), p(dc), p(dw0), p(db0), p(dw1), p(db), st);
+                                      p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2), g(3), g(4), st);
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
-        ctx->saved_data["need"] = need;
-        if (need) ctx->save_for_backward({dc, dw0, db0, dw1, db});
-        ctx->saved_data["shape_c"] = coeffs.sizes().vec();
-        ctx->saved_data["shape_w0"] = w0.sizes().vec();
-        ctx->saved_data["shape_b0"] = b0.sizes().vec();
-        ctx->saved_data["shape_w1"] = w1.sizes().vec();
-        ctx->saved_data["shape_b"] = bias.sizes().vec();
-        if (with_virial)
-            return {bloss, rmse.slice(0, 0, 1).clone(), rmse.slice(0, 1, 2).clone(), rmse.slice(0, 2, 3).clone()};
-        return {bloss, rmse.slice(0, 0, 1).clone(), rmse.slice(0, 1, 2).clone()};
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        save_grad_rows(ctx, need, &rows, {&coeffs, &w0, &b0, &w1, &bias});
+        if (with_virial) return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1}), piece(rmse, 2, {1})};
+        return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1})};
     }
 
     static variable_list backward(torch::autograd::AutogradContext* ctx, variable_list grads)
     {
         variable_list out(27);                   // one slot per forward argument after ctx
-        if (!ctx->saved_data["need"].toBool()) return out;
-        auto saved = ctx->get_saved_variables();
-        at::Tensor gl = grads[0].contiguous();
-        const char* keys[5] = {"shape_c", "shape_w0", "shape_b0", "shape_w1", "shape_b"};
-        for (int i = 0; i < 5; i++)              // coeffs, w0, b0, w1, type_bias are arguments 11..15
-            out[11 + i] = torch::matmul(gl, saved[i]).reshape(ctx->saved_data[keys[i]].toIntVector());
+        grad_products(ctx, grads[0], out, 11);   // coeffs, w0, b0, w1, type_bias are arguments 11..15
         return out;
     }
 };

@@ -230,58 +230,47 @@ struct NNLossFunction : public torch::autograd::Function<NNLossFunction> {
         TORCH_CHECK(e_dft.numel() == B && f_dft.numel() == (int64_t)B * P * 3 && v_dft.numel() == (int64_t)B * 9,
                     "label tensors must have shapes [B], [B, P, 3], [B, 9]");
         const bool need = coeffs.requires_grad() || w0.requires_grad() || w1.requires_grad() || bias.requires_grad();
-        at::Tensor bloss = at::zeros({B}, opt), e = at::zeros({B}, opt), f = at::zeros({B, P, 3}, opt),
-                   v = at::zeros({B, 9}, opt), dc, d0, d1, db;
-        if (need) {
-            dc = at::zeros({B, coeffs.numel()}, opt);
-            d0 = at::zeros({B, w0.numel()}, opt);
-            d1 = at::zeros({B, w1.numel()}, opt);
-            db = at::zeros({B, bias.numel()}, opt);
-        }
+        // the library writes every element of these outputs when the batch is not empty
+        const bool fresh = B > 0 && P > 0;
+        auto out = [&](int64_t n) { return fresh ? at::empty({n}, opt) : at::zeros({n}, opt); };
+        const int64_t nf = (int64_t)B * P * 3;
+        at::Tensor bloss = out(B), efv = out(B + nf + (int64_t)B * 9);
+        const GradRows rows(need ? B : 0, {&coeffs, &w0, &w1, &bias}, opt, fresh);
         const char* env = std::getenv("A2P_NNMTP_EXACT_GRADIENT");
         const int exact = env && env[0] == '1';
         void* st = current_stream(brcs);
         auto call = [&]() -> int {
             int rc;
             if (brcs.scalar_type() == at::kDouble) {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<double>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<double>(); };
+                auto g = [&](int i) { return need ? rows.ptr<double>(i) : nullptr; };
                 rc = a2p_nnmtp_loss_f64(plan.handle, e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft), (int)K,
                                         H, p(coeffs), p(w0), p(w1), p(bias), (int)nmus, ntypes, p(q_shifter), p(q_scaler),
                                         rmax, rmin, B, P, s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(),
                                         bnumneigh.data_ptr<int>(), bfirstneigh.data_ptr<int>(), p(brcs),
-                                        btypes.data_ptr<int>(), p(bloss), p(e), p(f), p(v), p(dc), p(d0), p(d1), p(db),
+                                        btypes.data_ptr<int>(), p(bloss), p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2), g(3),
                                         exact, st);
             } else {
-                auto p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<float>() : nullptr; };
+                auto p = [](const at::Tensor& t) { return t.data_ptr<float>(); };
+                auto g = [&](int i) { return need ? rows.ptr<float>(i) : nullptr; };
                 rc = a2p_nnmtp_loss_f32(plan.handle, e_w, f_w, with_virial ? v_w : 0.0, p(e_dft), p(f_dft), p(v_dft), (int)K,
                                         H, p(coeffs), p(w0), p(w1), p(bias), (int)nmus, ntypes, p(q_shifter), p(q_scaler),
                                         rmax, rmin, B, P, s.U, binum.data_ptr<int>(), bilist.data_ptr<int>(),
                                         bnumneigh.data_ptr<int>(), bfirstneigh.data_ptr<int>(), p(brcs),
-                                        btypes.data_ptr<int>(), p(bloss), p(e), p(f), p(v), p(dc), p(d0), p(d1), p(db),
+                                        btypes.data_ptr<int>(), p(bloss), p(efv), p(efv) + B, p(efv) + B + nf, g(0), g(1), g(2), g(3),
                                         exact, st);
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
-        ctx->saved_data["need"] = need;
-        if (need) ctx->save_for_backward({dc, d0, d1, db});
-        ctx->saved_data["shape_c"] = coeffs.sizes().vec();
-        ctx->saved_data["shape_0"] = w0.sizes().vec();
-        ctx->saved_data["shape_1"] = w1.sizes().vec();
-        ctx->saved_data["shape_b"] = bias.sizes().vec();
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        save_grad_rows(ctx, need, &rows, {&coeffs, &w0, &w1, &bias});
         return {bloss};
     }
 
     static variable_list backward(AutogradContext* ctx, variable_list grads)
     {
         variable_list out(29);                   // one slot per forward argument after ctx
-        if (!ctx->saved_data["need"].toBool()) return out;
-        auto saved = ctx->get_saved_variables();
-        at::Tensor gl = grads[0].contiguous();
-        out[8] = torch::matmul(gl, saved[0]).reshape(ctx->saved_data["shape_c"].toIntVector());
-        out[9] = torch::matmul(gl, saved[1]).reshape(ctx->saved_data["shape_0"].toIntVector());
-        out[10] = torch::matmul(gl, saved[2]).reshape(ctx->saved_data["shape_1"].toIntVector());
-        out[11] = torch::matmul(gl, saved[3]).reshape(ctx->saved_data["shape_b"].toIntVector());
+        grad_products(ctx, grads[0], out, 8);    // coeffs, w0, w1, type_bias
         return out;
     }
 };

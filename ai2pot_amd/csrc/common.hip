@@ -124,7 +124,7 @@ __global__ void read_back_kernel(const int* __restrict__ src, int nwords, int* h
 }
 }  // namespace
 
-int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t stream)
+int read_back_post(const void* device_src, int nwords, hipStream_t stream, ReadBack* rb)
 {
     A2P_REQUIRE(nwords > 0 && nwords < RB_WORDS, A2P_ERR_INVALID, "read_back: %d words", nwords);
     {
@@ -136,39 +136,71 @@ int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t st
             g_rb_page = (int*)p;
         }
     }
-    int slot = -1;
+    rb->src = device_src; rb->nwords = nwords; rb->stream = stream; rb->slot = -1;
     for (unsigned long long used = g_rb_used.load(); ~used != 0ull;) {
         const int free_slot = __builtin_ctzll(~used);
-        if (g_rb_used.compare_exchange_weak(used, used | (1ull << free_slot))) { slot = free_slot; break; }
+        if (g_rb_used.compare_exchange_weak(used, used | (1ull << free_slot))) { rb->slot = free_slot; break; }
     }
-    if (slot < 0) {                                  // more threads wait at once than there are slots
-        A2P_HIP_CHECK(hipMemcpyAsync(host_dst, device_src, (size_t)nwords * sizeof(int), hipMemcpyDeviceToHost, stream));
-        A2P_HIP_CHECK(hipStreamSynchronize(stream));
-        return A2P_OK;
-    }
-    int* const word = g_rb_page + slot * RB_WORDS;
-    int seq;
-    do seq = g_rb_seq.fetch_add(1) + 1; while (seq == 0 || seq == __atomic_load_n(word, __ATOMIC_RELAXED));
-    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, (const int*)device_src, nwords, word, seq);
-    hipError_t err = hipGetLastError();
-    if (err == hipSuccess) {
-        // polling pays while the wait is short; behind a long queue (or after a fault, when the number never
-        // arrives) the runtime's own wait takes over
-        const auto began = std::chrono::steady_clock::now();
-        bool there = false;
-        while (!(there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == seq)) {
-            for (int i = 0; i < 16; i++) __builtin_ia32_pause();
-            if (std::chrono::steady_clock::now() - began > std::chrono::milliseconds(1)) break;
-        }
-        if (!there) {
-            err = hipStreamSynchronize(stream);
-            if (err == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) != seq) err = hipErrorUnknown;
-        }
-        if (err == hipSuccess) memcpy(host_dst, word + 1, (size_t)nwords * sizeof(int));
-    }
-    g_rb_used.fetch_and(~(1ull << slot));
+    if (rb->slot < 0) return A2P_OK;                 // more waiters than slots: read_back_wait copies instead
+    int* const word = g_rb_page + rb->slot * RB_WORDS;
+    do rb->seq = g_rb_seq.fetch_add(1) + 1; while (rb->seq == 0 || rb->seq == __atomic_load_n(word, __ATOMIC_RELAXED));
+    hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, (const int*)device_src, nwords, word, rb->seq);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) g_rb_used.fetch_and(~(1ull << rb->slot));
     A2P_HIP_CHECK(err);
     return A2P_OK;
+}
+
+int read_back_wait(const ReadBack& rb, void* host_dst)
+{
+    if (rb.slot < 0) {
+        A2P_HIP_CHECK(hipMemcpyAsync(host_dst, rb.src, (size_t)rb.nwords * sizeof(int), hipMemcpyDeviceToHost, rb.stream));
+        A2P_HIP_CHECK(hipStreamSynchronize(rb.stream));
+        return A2P_OK;
+    }
+    // polling pays while the wait is short; behind a long queue (or after a fault, when the number never arrives) the
+    // runtime's own wait takes over
+    int* const word = g_rb_page + rb.slot * RB_WORDS;
+    hipError_t err = hipSuccess;
+    const auto began = std::chrono::steady_clock::now();
+    bool there = false;
+    while (!(there = __atomic_load_n(word, __ATOMIC_ACQUIRE) == rb.seq)) {
+        for (int i = 0; i < 16; i++) __builtin_ia32_pause();
+        if (std::chrono::steady_clock::now() - began > std::chrono::milliseconds(1)) break;
+    }
+    if (!there) {
+        err = hipStreamSynchronize(rb.stream);
+        if (err == hipSuccess && __atomic_load_n(word, __ATOMIC_ACQUIRE) != rb.seq) err = hipErrorUnknown;
+    }
+    if (err == hipSuccess) memcpy(host_dst, word + 1, (size_t)rb.nwords * sizeof(int));
+    g_rb_used.fetch_and(~(1ull << rb.slot));
+    A2P_HIP_CHECK(err);
+    return A2P_OK;
+}
+
+int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t stream)
+{
+    ReadBack rb;
+    const int rc = read_back_post(device_src, nwords, stream, &rb);
+    return rc ? rc : read_back_wait(rb, host_dst);
+}
+
+// The status word of a call that checks its inputs in its first kernels can be on its way to the host while the rest
+// of the call runs: see a2p_status_early.
+namespace {
+thread_local bool g_early_asked = false, g_early_posted = false;
+thread_local ReadBack g_early;
+}  // namespace
+
+int status_post_early(hipStream_t stream)
+{
+    if (!g_early_asked || g_early_posted) return A2P_OK;
+    void* flags = nullptr;
+    int rc = ws_get(WS_FLAGS, 64, &flags);
+    if (rc) return rc;
+    rc = read_back_post(flags, 1, stream, &g_early);
+    g_early_posted = rc == A2P_OK;
+    return rc;
 }
 
 // ---- per-kernel timing ---------------------------------------------------------------------
@@ -349,9 +381,86 @@ template int finish_energy_virial<double>(double*, double*, const double*, int, 
 template int finish_partials<float>(float*, const double*, int, int, int, int, int, hipStream_t, bool);
 template int finish_partials<double>(double*, const double*, int, int, int, int, int, hipStream_t, bool);
 
+// Weighted sums of the per-structure gradient rows.  64 elements per workgroup, the structures in four runs (one per
+// wavefront) whose sums are added in run order: a batch of 64 is sixteen loads per lane, eight of them in flight, and the
+// few thousand parameters of a model still make dozens of workgroups.  Bound by the launch and one trip to the L2, where
+// the rows lie (1.1 MB for a NEP model and 64 structures).
+constexpr int WR_PARTS = 8;
+template <typename T>
+struct WeightedRows {
+    const T* part[WR_PARTS];
+    long long beg[WR_PARTS + 1];       // first element of each part in out
+    int nparts;
+};
+template <typename T>
+__global__ void __launch_bounds__(256)
+weighted_rows_kernel(int B, const T* __restrict__ w, const WeightedRows<T> a, T* __restrict__ out)
+{
+    __shared__ double red[4][64];
+    const int lane = threadIdx.x & 63, run = threadIdx.x >> 6;
+    const long long e = (long long)blockIdx.x * 64 + lane, total = a.beg[a.nparts];
+    double acc = 0.0;
+    if (e < total) {
+        const T* src = a.part[0];
+        long long beg = 0, n = a.beg[1];
+#pragma unroll
+        for (int p = 1; p < WR_PARTS; p++)
+            if (p < a.nparts && e >= a.beg[p]) { src = a.part[p]; beg = a.beg[p]; n = a.beg[p + 1] - beg; }
+        src += e - beg;
+        const int len = (B + 3) / 4, b1 = min(B, (run + 1) * len);
+        for (int b0 = run * len; b0 < b1; b0 += 8) {
+            T v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = src[(long long)min(b0 + u, b1 - 1) * n];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (b0 + u < b1) acc += (double)w[b0 + u] * (double)v[u];
+        }
+    }
+    red[run][lane] = acc;
+    __syncthreads();
+    if (run == 0 && e < total) out[e] = (T)(((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
+}
+
+template <typename T>
+int weighted_rows(int B, const T* w, int nparts, const T* const* parts, const long long* sizes, T* out, hipStream_t stream)
+{
+    A2P_REQUIRE(B >= 1 && nparts >= 1 && nparts <= WR_PARTS && w && parts && sizes && out, A2P_ERR_INVALID,
+                "weighted_rows: need a batch, 1 to %d parts and non-null pointers", WR_PARTS);
+    WeightedRows<T> a;
+    a.nparts = nparts;
+    a.beg[0] = 0;
+    for (int p = 0; p < WR_PARTS; p++) {
+        const bool have = p < nparts;
+        A2P_REQUIRE(!have || (parts[p] && sizes[p] >= 0), A2P_ERR_INVALID, "weighted_rows: part %d", p);
+        a.part[p] = have ? parts[p] : nullptr;
+        a.beg[p + 1] = a.beg[p] + (have ? sizes[p] : 0);
+    }
+    const long long total = a.beg[nparts];
+    if (total == 0) return A2P_OK;
+    A2P_REQUIRE(total < (1ll << 36), A2P_ERR_INVALID, "weighted_rows: too many elements");
+    prof_begin("weighted_rows", stream);
+    hipLaunchKernelGGL(weighted_rows_kernel<T>, dim3(ceil_div(total, 64)), dim3(256), 0, stream, B, w, a, out);
+    prof_end(stream);
+    A2P_HIP_CHECK(hipGetLastError());
+    return A2P_OK;
+}
+
 }  // namespace a2p
 
 extern "C" {
+
+int a2p_weighted_rows_f32(int batch, const float* w, int nparts, const float* const* parts, const long long* sizes,
+                          float* out, void* stream)
+{
+    return a2p::weighted_rows<float>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+}
+
+int a2p_weighted_rows_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
+                          double* out, void* stream)
+{
+    return a2p::weighted_rows<double>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+}
 
 const char* a2p_last_error(void) { return a2p::last_error(); }
 
@@ -414,6 +523,8 @@ int a2p_profile_report(char* buf, size_t buflen)
     return A2P_OK;
 }
 
+static int a2p_report_status(int host, void* flags, hipStream_t stream);
+
 int a2p_check_status(void* stream_)
 {
     hipStream_t stream = (hipStream_t)stream_;
@@ -423,8 +534,37 @@ int a2p_check_status(void* stream_)
     int host = 0;
     rc = a2p::read_back(flags, 1, &host, stream);
     if (rc) return rc;
+    return a2p_report_status(host, flags, stream);
+}
+
+void a2p_status_early(int on)
+{
+    if (a2p::g_early_posted) {          // left over from a call that failed: its slot is free once the word has arrived
+        int word;
+        (void)a2p::read_back_wait(a2p::g_early, &word);
+        a2p::g_early_posted = false;
+    }
+    a2p::g_early_asked = on != 0;
+}
+
+int a2p_check_status_early(void* stream_)
+{
+    if (!a2p::g_early_posted) {         // the call had no early point
+        a2p::g_early_asked = false;
+        return a2p_check_status(stream_);
+    }
+    int host = 0;
+    const int rc = a2p::read_back_wait(a2p::g_early, &host);
+    a2p::g_early_asked = a2p::g_early_posted = false;
+    if (rc) return rc;
     if (host == 0) return A2P_OK;
-    rc = a2p::fill_zero(flags, 64, stream);
+    return a2p_check_status(stream_);   // behind the whole call: the word is cleared with nothing of the call to come
+}
+
+static int a2p_report_status(int host, void* flags, hipStream_t stream)
+{
+    if (host == 0) return A2P_OK;
+    int rc = a2p::fill_zero(flags, 64, stream);
     if (rc) return rc;
     A2P_HIP_CHECK(hipStreamSynchronize(stream));
     if (host & a2p::ST_SEG_OVERFLOW) {

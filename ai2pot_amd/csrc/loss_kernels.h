@@ -54,17 +54,24 @@ loss_forward_kernel(int P, const int* __restrict__ binum, const int* __restrict_
     }
 }
 
+// One wavefront: the structures' squared errors by lane, then by a fixed tree (a single thread over 64 structures took
+// 8 us, all of it the latency of its loads).
 template <typename T>
-__global__ void loss_rmse_kernel(int B, const int* __restrict__ binum, const double* __restrict__ sq,
-                                T* __restrict__ rmse)
+__global__ void __launch_bounds__(64)
+loss_rmse_kernel(int B, const int* __restrict__ binum, const double* __restrict__ sq, T* __restrict__ rmse)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    double e = 0, f = 0, v = 0;
-    long nf = 0;
-    for (int b = 0; b < B; b++) { e += sq[b * 3]; f += sq[b * 3 + 1]; v += sq[b * 3 + 2]; nf += 3L * binum[b]; }
-    rmse[0] = (T)sqrt(e / B);
-    rmse[1] = (T)sqrt(f / (double)nf);
-    rmse[2] = (T)sqrt(v / (9.0 * B));
+    const int lane = (int)threadIdx.x;
+    double e = 0, f = 0, v = 0, nf = 0;
+    for (int b = lane; b < B; b += 64) {
+        e += sq[b * 3]; f += sq[b * 3 + 1]; v += sq[b * 3 + 2];
+        nf += 3.0 * binum[b];
+    }
+    e = wave_sum(e); f = wave_sum(f); v = wave_sum(v); nf = wave_sum(nf);
+    if (lane == 0) {
+        rmse[0] = (T)sqrt(e / B);
+        rmse[1] = (T)sqrt(f / nf);
+        rmse[2] = (T)sqrt(v / (9.0 * B));
+    }
 }
 
 }  // namespace losskern

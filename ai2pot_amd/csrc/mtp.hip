@@ -1852,6 +1852,8 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
                         binum, bilist, bnumneigh, bfirstneigh, brcs, btypes, etot, force, virial, stream);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
+    rc = status_post_early(stream);      // the gradient kernel looks at the same entries of the same lists
+    if (rc) return rc;
     MtpPlan* plan = nullptr;
     rc = plan_check(handle, &plan);
     if (rc) return rc;
@@ -1913,6 +1915,8 @@ int nnmtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft,
                         bilist, bnumneigh, bfirstneigh, brcs, btypes, etot, force, virial, stream, &net);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
+    rc = status_post_early(stream);      // the gradient kernel looks at the same entries of the same lists
+    if (rc) return rc;
     MtpPlan* plan = nullptr;
     rc = plan_check(handle, &plan);
     if (rc) return rc;

@@ -417,6 +417,8 @@ int nep_loss(double e_w, double f_w, double v_w, const T* e_dft, const T* f_dft,
                       bilist, bnumneigh, bfirstneigh, brcs, btypes, etot, force, virial, (void*)stream);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
+    rc = status_post_early(stream);      // the gradient kernel looks at the same entries of the same lists
+    if (rc) return rc;
     NepLossArgs<T> a;
     a.K = K; a.n_r = n_r; a.n_a = n_a; a.l_max = l_max; a.H = H; a.ntypes = ntypes;
     a.D = (l_max == 0) ? n_r : n_r + n_a * l_max;

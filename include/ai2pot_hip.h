@@ -53,6 +53,21 @@ unsigned long long a2p_workspace_generation(void);
  * Synchronises `stream`.  Returns A2P_OK, A2P_ERR_INPUT, A2P_ERR_OVERFLOW, A2P_ERR_SEGMENT or A2P_ERR_GRID.  The reference has no such check: it asserts or overflows
  * (source/nblist/include/neighborList.h:550, commented-out assert). */
 int a2p_check_status(void* stream);
+/* The same for the loss entry points, whose first kernels make every check: a2p_status_early(1) before such a call
+ * sends the status word to the host behind those kernels, and a2p_check_status_early after it waits for that word
+ * only, while the gradient kernels of the call may still run (a raised bit is then confirmed by a2p_check_status behind
+ * the whole call).  Per host thread, for one call; after a call of another kind it is a2p_check_status. */
+void a2p_status_early(int on);
+int a2p_check_status_early(void* stream);
+
+/* out[c] = sum_b w[b] * parts[p][b, i] for every part p and i < sizes[p] (parts [batch, sizes[p]], laid one behind
+ * the other in out): the products grad_output @ dloss/dtheta of all parameters of a loss operator in one launch
+ * (one matmul per parameter in the reference, mtpr/src/linearMtpOp.cc:1740-1742).  Sums in double, in a fixed order.
+ * `parts` (device pointers) and `sizes` are host arrays of at most 8 entries. */
+int a2p_weighted_rows_f32(int batch, const float* w, int nparts, const float* const* parts, const long long* sizes,
+                          float* out, void* stream);
+int a2p_weighted_rows_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
+                          double* out, void* stream);
 
 /* Per-kernel timing for benchmarks (no counterpart in the reference, which leaves timing to
  * commented-out std::chrono calls, interface/lammps/AI2POT/pair_ai2pot.cpp:392-442).  While
