@@ -144,44 +144,29 @@ __device__ __forceinline__ int wave_inclusive_scan(int v)
 // ---- shared device routines (pair_reduce.hip) --------------------------------------------
 // Deterministic reduction of per-pair derivatives g[row, slot, 3] onto atoms:
 //   force[b, j] = own[b, j] - sum over pairs (row, slot) of structure b whose neighbour is j.
-// `force` must already hold the `own` part (zero for atoms without a row).  Integer atomics
-// build the incoming lists; the floating-point sums are order-independent (terms rounded to a
-// common quantum chosen from the per-target maximum, then added exactly), so results are
-// reproducible run to run.
+// With `own` the sum over the row of centre j is formed here; otherwise `force` must already hold it (zero for atoms
+// without a row) and bilist is not read.  Integer atomics deal out the places of the pairs in their targets'
+// segments; the floating-point sums are order-independent (terms rounded to a common quantum chosen from the
+// per-target maximum, then added exactly), so results are reproducible run to run.  Any list is summed in full.
 template <typename T>
-int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, const int* binum,
-                const int* bnumneigh, const int* bfirstneigh, hipStream_t stream);
+int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, const int* binum, const int* bilist,
+                const int* bnumneigh, const int* bfirstneigh, bool own, hipStream_t stream);
 
-// The same reduction for a producer that stores each pair derivative straight into its
-// target's segment, without the intermediate [row, slot, 3] array:
-//   pair_csr_begin   counts the incoming pairs per target and scans them into segment offsets;
-//                    with_rank: every valid pair (row, slot) also gets rank[row*U + slot], its
-//                    place inside its target's segment (-1 for an index out of range);
-//   the producer     stores seg_g[pos*3 .. pos*3+2] at  pos = offsets[t] + rank[row*U + slot]
-//                    for EVERY valid pair (zeros where the derivative vanishes), or, without
-//                    ranks, claims  pos = offsets[t] + atomicAdd(&cursor[t], 1)  and may skip pairs;
-//   pair_csr_finish  sums the filled part of every segment onto `force` as above.
+// The same reduction for a producer that stores each pair derivative straight into its target's segment, without the
+// intermediate [row, slot, 3] array (pair_fixed_begin, the producer, pair_csr_finish).
 // Capacity of the fixed reduction segments: umax unless the calling thread asked for more with
 // a2p_pair_segment_capacity (lists in which an atom is named by more pairs than a row holds).
 int pair_segment_capacity(int U);
-// pair_fixed_begin skips counting: every target owns a segment of fixed capacity seg_cap (umax by default)
+// pair_fixed_begin: every target owns a segment of fixed capacity seg_cap (umax by default)
 // (a cutoff-built list sends an atom no more pairs than its own row could hold); the producer
 // claims  rank = atomicAdd(&cursor[t], 1),  stores at  pos = t*seg_cap + rank  when rank < seg_cap
 // and otherwise raises ST_SEG_OVERFLOW and stores at the spare entry n*seg_cap.
 struct PairCsr {
-    int* counts;
-    int* offsets;
     int* cursor;
-    int* rank;      // [B*P, U] or null
     void* seg_g;
     int n;          // B * (P + nghost) targets
-    int seg_cap;    // > 0: fixed-capacity segments (offsets, counts and rank are null)
+    int seg_cap;
 };
-template <typename T>
-int pair_csr_begin(PairCsr* csr, bool with_rank, int B, int P, int U, int nghost, const int* binum,
-                   const int* bnumneigh, const int* bfirstneigh, hipStream_t stream);
-// also_zero / also_bytes: a second range cleared by the same launch that clears the cursors
-// (the force array of the caller, as a rule)
 template <typename T>
 int pair_fixed_begin(PairCsr* csr, int B, int P, int U, int nghost, hipStream_t stream, void* also_zero = nullptr,
                      size_t also_bytes = 0, int* cursor_ext = nullptr, bool cursor_final = false);

@@ -106,6 +106,15 @@ inline void check_device_status(const at::Tensor& t)
     if (validate_flag()) check_rc(a2p_check_status(current_stream(t)));
 }
 
+// Asks the next library call to send its status word ahead of its last kernels (a2p_status_early); what was sent and
+// not read is dropped when the scope ends.
+struct EarlyStatus {
+    bool on;
+    explicit EarlyStatus(bool on_ = true) : on(on_) { if (on) a2p_status_early(1); }
+    ~EarlyStatus() { if (on) a2p_status_early(0); }
+    int read(const at::Tensor& t) { return a2p_check_status_early(current_stream(t)); }
+};
+
 // Runs an energy / force / virial (or loss) call and, with validation on, reads the device status.
 // A list that names an atom more often than a row is long (half lists, ghosts collecting the pairs of
 // several rows) overflows the fixed reduction segments of the fast kernels: the status says so and
@@ -116,14 +125,11 @@ template <class Call>
 inline void run_checked(const at::Tensor& brcs, const at::Tensor& binum, const at::Tensor& bnumneigh,
                         const at::Tensor& bfirstneigh, int nghost, Call&& call, bool early = false)
 {
-    early = early && validate_flag();
-    if (early) a2p_status_early(1);
-    int rc = call();
-    if (early && rc != A2P_OK) a2p_status_early(0);
-    check_rc(rc);
+    EarlyStatus status(early && validate_flag());
+    check_rc(call());
     if (!validate_flag()) return;
     void* st = current_stream(brcs);
-    rc = early ? a2p_check_status_early(st) : a2p_check_status(st);
+    int rc = early ? status.read(brcs) : a2p_check_status(st);
     if (rc == A2P_ERR_SEGMENT) {
         int most = 0;
         check_rc(a2p_pair_incoming_max((int)brcs.size(0), (int)brcs.size(1), (int)brcs.size(2), nghost,
@@ -238,18 +244,20 @@ struct GradRows {
     }
 };
 
-inline void save_grad_rows(torch::autograd::AutogradContext* ctx, bool need, const GradRows* rows,
+inline void save_grad_rows(torch::autograd::AutogradContext* ctx, bool need, const GradRows& rows,
                            std::initializer_list<const at::Tensor*> params)
 {
     std::vector<int64_t> shapes;         // dimensions and sizes of each parameter
     if (need) {
-        ctx->save_for_backward({rows->flat});
+        ctx->save_for_backward({rows.flat});
         for (auto* p : params) {
             shapes.push_back(p->dim());
             shapes.insert(shapes.end(), p->sizes().begin(), p->sizes().end());
         }
     }
     ctx->saved_data["shapes"] = shapes;  // empty: no parameter wants a gradient
+    ctx->saved_data["batch"] = rows.B;
+    ctx->set_materialize_grads(false);   // the RMSEs' gradients are not used: no zeros are filled in for them
 }
 
 // grad_output @ dloss/dtheta of every parameter, in one launch; out[first + i] receives parameter i's.
@@ -259,8 +267,9 @@ inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tenso
     const std::vector<int64_t> shapes = ctx->saved_data["shapes"].toIntVector();
     if (shapes.empty()) return;
     const at::Tensor flat = ctx->get_saved_variables()[0];
-    const at::Tensor gl = grad_output.contiguous();
-    const int64_t B = gl.numel();
+    const int64_t B = ctx->saved_data["batch"].toInt();
+    // (an output that took no part in what is differentiated has no gradient: zero)
+    const at::Tensor gl = grad_output.defined() ? grad_output.contiguous() : at::zeros({B}, flat.options());
     std::vector<std::vector<int64_t>> shape;
     std::vector<long long> numel;
     long long total = 0;

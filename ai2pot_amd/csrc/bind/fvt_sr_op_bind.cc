@@ -191,8 +191,9 @@ TORCH_LIBRARY(fvt, m)
                               bilist.numel() == dei.size(0) * dei.size(1) &&
                               bnumneigh.numel() == dei.size(0) * dei.size(1) && binum.numel() == dei.size(0),
                           "neighbour tensors do not match bdei_drij");
+              EarlyStatus status(validate_flag());
               at::Tensor f = ForceSr::apply(dei, binum, bilist, bnumneigh, bfirstneigh, nghost);
-              check_device_status(dei);
+              if (validate_flag()) check_rc(status.read(dei));
               return {f};
           });
     m.def("VirialSrOp",
@@ -207,8 +208,17 @@ TORCH_LIBRARY(fvt, m)
                           "brcs must match bdei_drij in dtype and device");
               check_device_int(dei, bnumneigh, "bnumneigh");
               TORCH_CHECK(bnumneigh.numel() == dei.size(0) * dei.size(1), "bnumneigh must have shape [B, nlocal]");
-              if (bnumneigh.numel())
-                  TORCH_CHECK(bnumneigh.max().item<int>() <= umax, "a neighbour count exceeds umax_num_neighs");
-              return {VirialSr::apply(brcs, dei, bnumneigh)};
+              // the kernel reports a row that is too long; with validation off its status word is left alone
+              const char* too_long = "a neighbour count exceeds umax_num_neighs";
+              const bool any = bnumneigh.numel() > 0;
+              if (any && !validate_flag()) TORCH_CHECK(bnumneigh.max().item<int>() <= umax, too_long);
+              EarlyStatus status(any && validate_flag());
+              at::Tensor v = VirialSr::apply(brcs, dei, bnumneigh);
+              if (any && validate_flag()) {
+                  const int rc = status.read(dei);
+                  TORCH_CHECK(rc != A2P_ERR_OVERFLOW, too_long);
+                  check_rc(rc);
+              }
+              return {v};
           });
 }

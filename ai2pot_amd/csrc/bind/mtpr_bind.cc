@@ -138,7 +138,7 @@ struct LossFunction : public torch::autograd::Function<LossFunction> {
             return rc;
         };
         run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
-        save_grad_rows(ctx, need, &rows, {&coeffs, &lin, &bias});
+        save_grad_rows(ctx, need, rows, {&coeffs, &lin, &bias});
         if (with_virial) return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1}), piece(rmse, 2, {1})};
         return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1})};
     }

@@ -2,8 +2,8 @@
 // vector-Jacobian products, for gfx950.
 //
 //   force : F[c] = sum_s g[ii,s] - sum over pairs whose neighbour is c of g   (c = ilist[ii])
-//           reference: source/fvt/include/force_sr.h:50-84.  The own-row sum is one wavefront
-//           per row; the neighbour part is a2p::pair_reduce (no floating-point atomics).
+//           reference: source/fvt/include/force_sr.h:50-84.  a2p::pair_reduce: the own-row sum is formed by the
+//           wavefront that deals out the row's places (no floating-point atomics).
 //   virial: V[a,b] = - sum_{ii,s} g[ii,s,a] r[ii,s,b]          source/fvt/include/virial_sr.h:24-51
 // The reference materialises dense Jacobians [(nlocal+nghost)*3, nlocal*umax] and
 // [9, nlocal*umax] (src/force_sr_op.cc:44, src/virial_sr_op.cc:31-32) and multiplies by them
@@ -16,30 +16,6 @@
 
 namespace a2p {
 namespace {
-
-template <typename T>
-__global__ void __launch_bounds__(256)
-force_own_kernel(T* __restrict__ force, const T* __restrict__ g, int B, int P, int U, int NF,
-                 const int* __restrict__ binum, const int* __restrict__ bilist,
-                 const int* __restrict__ bnumneigh, int* __restrict__ status)
-{
-    const int row = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (row >= B * P) return;
-    const int b = row / P, ii = row - b * P;
-    if (ii >= binum[b]) return;
-    int nn = bnumneigh[row];
-    if (nn > U) { if (lane == 0) atomicOr(status, ST_NEIGH_OVERFLOW); nn = U; }
-    const int c = bilist[row];
-    if ((unsigned)c >= (unsigned)NF) { if (lane == 0) atomicOr(status, ST_BAD_NEIGHBOR); return; }
-    const T* gr = g + (size_t)row * U * 3;
-    T sx = 0, sy = 0, sz = 0;
-    for (int s = lane; s < nn; s += 64) { sx += gr[s * 3]; sy += gr[s * 3 + 1]; sz += gr[s * 3 + 2]; }
-    sx = wave_sum(sx); sy = wave_sum(sy); sz = wave_sum(sz);
-    if (lane == 0) {
-        T* f = force + ((size_t)b * NF + c) * 3;
-        f[0] = sx; f[1] = sy; f[2] = sz;
-    }
-}
 
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -76,11 +52,12 @@ force_bwd_kernel(T* __restrict__ gout, const T* __restrict__ gF, int B, int P, i
 template <typename T>
 __global__ void __launch_bounds__(256)
 virial_rows_kernel(double* __restrict__ partial, const T* __restrict__ g, const T* __restrict__ r, int B,
-                   int P, int U, const int* __restrict__ bnumneigh)
+                   int P, int U, const int* __restrict__ bnumneigh, int* __restrict__ status)
 {
     const int row = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (row >= B * P) return;
     const int nn = min(bnumneigh[row], U);
+    if (status && lane == 0 && bnumneigh[row] > U) atomicOr(status, ST_NEIGH_OVERFLOW);
     const T* gr = g + (size_t)row * U * 3;
     const T* rr = r + (size_t)row * U * 3;
     double v[9];
@@ -143,17 +120,7 @@ int force_fwd(int B, int P, int U, int nghost, const int* binum, const int* bili
     A2P_REQUIRE(binum && bilist && bnumneigh && bfirstneigh && dei && force, A2P_ERR_INVALID,
                 "fvt force: null pointer");
     if (B == 0 || P == 0) return A2P_OK;
-    void* flags = nullptr;
-    rc = ws_get(WS_FLAGS, 64, &flags);
-    if (rc) return rc;
-    rc = fill_zero(force, (size_t)B * (P + nghost) * 3 * sizeof(T), stream);
-    if (rc) return rc;
-    prof_begin("fvt_force_own", stream);
-    hipLaunchKernelGGL(force_own_kernel<T>, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
-                       force, dei, B, P, U, P + nghost, binum, bilist, bnumneigh, (int*)flags);
-    prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
-    return pair_reduce<T>(force, dei, B, P, U, nghost, binum, bnumneigh, bfirstneigh, stream);
+    return pair_reduce<T>(force, dei, B, P, U, nghost, binum, bilist, bnumneigh, bfirstneigh, true, stream);
 }
 
 template <typename T>
@@ -183,13 +150,18 @@ int virial_fwd(int B, int P, int U, const int* bnumneigh, const T* rcs, const T*
     if (B == 0) return A2P_OK;
     if (P == 0) return fill_zero(virial, (size_t)B * 9 * sizeof(T), stream);
     void* ws = nullptr;
+    rc = ws_get(WS_FLAGS, 64, &ws);
+    if (rc) return rc;
+    int* const status = (int*)ws;
     rc = ws_get(WS_PARTIAL, (size_t)B * P * 9 * sizeof(double), &ws);
     if (rc) return rc;
     prof_begin("fvt_virial_rows", stream);
     hipLaunchKernelGGL(virial_rows_kernel<T>, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
-                       (double*)ws, dei, rcs, B, P, U, bnumneigh);
+                       (double*)ws, dei, rcs, B, P, U, bnumneigh, status);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
+    rc = status_post_early(stream);
+    if (rc) return rc;
     return finish_partials<T>(virial, (const double*)ws, B, P, 9, 9, 9, stream);
 }
 
@@ -258,7 +230,7 @@ int virial_fwd_noalloc(int B, int P, int U, const int* bnumneigh, const float* r
     // what an earlier call left in the buffer never shows; nlocal == 0 leaves nothing to sum (zeros)
     if (P > 0) {
         hipLaunchKernelGGL(virial_rows_kernel<float>, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
-                           partial, dei, rcs, B, P, U, bnumneigh);
+                           partial, dei, rcs, B, P, U, bnumneigh, (int*)nullptr);
         A2P_HIP_CHECK(hipGetLastError());
     }
     return finish_partials<float>(virial, (const double*)partial, B, P, 9, 9, 9, stream, false);

@@ -536,7 +536,7 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
             rc = launch<T, 16, 12, 8, 4, false>(a, lds, stream);
         if (rc) return rc;
         if (force) {
-            rc = pair_reduce<T>(force, a.pair_g, B, P, U, nghost, binum, bnumneigh, bfirstneigh, stream);
+            rc = pair_reduce<T>(force, a.pair_g, B, P, U, nghost, binum, bilist, bnumneigh, bfirstneigh, false, stream);
             if (rc) return rc;
         }
     }

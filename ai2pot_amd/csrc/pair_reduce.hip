@@ -3,16 +3,19 @@
 // neighbour is j  on top of the sum over its own row that the producing kernel stored.
 //
 // Steps (all on `stream`):
-//   1. count  : integer histogram of neighbour indices            (HBM: reads valid firstneigh)
-//   2. scan   : exclusive prefix sum -> segment offsets
-//   3. fill   : pair derivatives copied into their target's segment (position by integer
-//               atomic; the order inside a segment is therefore arbitrary)
-//   4. reduce : per target, order-independent sum: every term is converted to 64-bit fixed
+//   1. clear  : a cursor per target, the overflow count (and the caller's force array)
+//   2. claim  : every pair takes an entry of its target's segment (a returning integer atomic; the order inside a
+//               segment is therefore arbitrary) and leaves its number there.  Segments hold as many pairs as a row: a
+//               list built with one cutoff never needs more, and what does not fit goes to one list for all targets
+//   3. reduce : per target, order-independent sum over the pairs named: every term is converted to 64-bit fixed
 //               point against the segment's largest magnitude, integers are added (exact,
 //               associative), the total is converted back.  The result is identical for
 //               any arrival order, so the output is bit-reproducible run to run; the
 //               conversion error per term is below 2^-37 (fp32 inputs) / 2^-52 (fp64 inputs)
 //               of the largest term, i.e. below the rounding error of a floating sum.
+// Three short launches, bound by their latency for systems of a few thousand atoms (counting, a prefix sum in three
+// launches and a copy of the derivatives in place of the claim took ten; force and virial of 4 x 1000 atoms with their
+// gradients, fp64, 146 -> 103 us).
 // No floating-point atomics are used.
 #include "a2p_common.h"
 
@@ -124,38 +127,61 @@ __global__ void scan_apply(const int* __restrict__ in, int* __restrict__ out,
     }
 }
 
-template <typename T>
-__global__ void fill_kernel(T* __restrict__ seg_g, int* __restrict__ cursor,
-                            const int* __restrict__ offsets, const T* __restrict__ pair_g, int B,
-                            int P, int U, int NF, const int* __restrict__ binum,
-                            const int* __restrict__ bnumneigh, const int* __restrict__ bfirstneigh)
+// Claims of step 2, one wavefront per row.  With OWN the wavefront also sums the row itself and stores it as the force
+// on the row's centre (a centre has one row).
+template <typename T, bool OWN>
+__global__ void __launch_bounds__(256)
+claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum, const int* __restrict__ bilist,
+             const int* __restrict__ bnumneigh, const int* __restrict__ bfirstneigh, const T* __restrict__ pair_g,
+             int* __restrict__ cursor, int* __restrict__ seg, int2* __restrict__ spill, int* __restrict__ nspill,
+             T* __restrict__ force, int* __restrict__ status)
 {
-    const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const int lane = threadIdx.x & 63;
-    if (wave >= B * P) return;
-    const int b = wave / P, ii = wave - b * P;
+    const int row = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (row >= B * P) return;
+    const int b = row / P, ii = row - b * P;
     if (ii >= binum[b]) return;
-    int nn = min(bnumneigh[wave], U);
-    const int* row = bfirstneigh + (size_t)wave * U;
-    const T* grow = pair_g + (size_t)wave * U * 3;
+    int nn = bnumneigh[row];
+    if (nn > U) {
+        if (lane == 0) atomicOr(status, ST_NEIGH_OVERFLOW);
+        nn = U;
+    }
+    const int* first = bfirstneigh + (size_t)row * U;
+    const T* g = pair_g + (size_t)row * U * 3;
+    T sx = (T)0, sy = (T)0, sz = (T)0;
     for (int s = lane; s < nn; s += 64) {
-        int j = row[s];
-        if ((unsigned)j >= (unsigned)NF) continue;
-        size_t t = (size_t)b * NF + j;
-        int pos = offsets[t] + atomicAdd(&cursor[t], 1);
-        seg_g[(size_t)pos * 3 + 0] = grow[s * 3 + 0];
-        seg_g[(size_t)pos * 3 + 1] = grow[s * 3 + 1];
-        seg_g[(size_t)pos * 3 + 2] = grow[s * 3 + 2];
+        const int j = first[s];
+        if (OWN) { sx += g[s * 3]; sy += g[s * 3 + 1]; sz += g[s * 3 + 2]; }
+        if ((unsigned)j >= (unsigned)NF) {
+            atomicOr(status, ST_BAD_NEIGHBOR);
+            continue;
+        }
+        const int t = b * NF + j;
+        const int k = atomicAdd(&cursor[t], 1);
+        if (k < cap) seg[(size_t)t * cap + k] = row * U + s;
+        else spill[atomicAdd(nspill, 1)] = make_int2(t, row * U + s);      // at most one entry per pair
+    }
+    if (OWN) {
+        sx = wave_sum(sx); sy = wave_sum(sy); sz = wave_sum(sz);
+        const int c = bilist[row];
+        if ((unsigned)c >= (unsigned)NF) {
+            if (lane == 0) atomicOr(status, ST_BAD_NEIGHBOR);
+        } else if (lane == 0) {
+            T* f = force + ((size_t)b * NF + c) * 3;
+            f[0] = sx; f[1] = sy; f[2] = sz;
+        }
     }
 }
 
 // 16 lanes per target atom.  Workgroups from `reduce_blocks` on sum the energy / virial partials
 // instead (one component of one structure each), which saves small systems a launch.
-template <typename T>
-__global__ void reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g,
-                              const int* __restrict__ offsets, const int* __restrict__ counts, int NT,
-                              int seg_cap, int reduce_blocks, T* __restrict__ etot, T* __restrict__ virial,
-                              const double* __restrict__ partial, int nblocks)
+// NAMED: the segments hold the numbers of the pairs (claim_kernel), otherwise the derivatives themselves.
+// The first four entries of every lane stay in registers between the two passes (largest magnitude, then the sum).
+template <typename T, bool NAMED>
+__global__ void __launch_bounds__(256)
+reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __restrict__ counts, int NT, int seg_cap,
+              const int* __restrict__ seg_pair, const int2* __restrict__ spill, const int* __restrict__ nspill,
+              int reduce_blocks, T* __restrict__ etot, T* __restrict__ virial, const double* __restrict__ partial,
+              int nblocks)
 {
     if ((int)blockIdx.x >= reduce_blocks) {
         __shared__ double sh[256];
@@ -163,51 +189,62 @@ __global__ void reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g
         finish_ev_body<T>(etot, virial, partial, nblocks, id / 10, id % 10, sh);
         return;
     }
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    const int t = gid >> 4;
-    const int sub = gid & 15;
-    const bool live = t < NT;
-    // seg_cap > 0: segments of fixed capacity, target t owns entries [t*seg_cap, (t+1)*seg_cap)
-    const int beg = !live ? 0 : seg_cap > 0 ? t * seg_cap : offsets[t];
-    const int cnt = !live ? 0 : seg_cap > 0 ? min(counts[t], seg_cap) : counts[t];
+    const int t = (int)(blockIdx.x * 16u + (threadIdx.x >> 4));       // 256 threads
+    const int sub = threadIdx.x & 15;
+    // target t owns entries [t*seg_cap, (t+1)*seg_cap); uniform over the 16 lanes of a target
+    const int all = t < NT ? counts[t] : 0;
+    const int cnt = min(all, seg_cap);
+    if (all == 0) return;
+    const size_t beg = (size_t)t * seg_cap;
+    auto entry = [&](int e) __attribute__((always_inline)) -> const T* {
+        return seg_g + (NAMED ? (size_t)seg_pair[beg + e] : beg + e) * 3;
+    };
+    // calls f on every entry beyond the four in registers: the rest of the segment, then the target's pairs among
+    // those that did not fit (a scan of the whole list; no list built with one cutoff gets here)
+    auto others = [&](auto&& f) __attribute__((always_inline)) {
+        for (int e = sub + 64; e < cnt; e += 16) f(entry(e));
+        if (NAMED && all > seg_cap) {
+            const int n = *nspill;
+            for (int i = sub; i < n; i += 16)
+                if (spill[i].x == t) f(seg_g + (size_t)spill[i].y * 3);
+        }
+    };
+    T gx[4], gy[4], gz[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int e = sub + 16 * k;
+        gx[k] = (T)0; gy[k] = (T)0; gz[k] = (T)0;
+        if (e < cnt) {
+            const T* g = entry(e);
+            gx[k] = g[0]; gy[k] = g[1]; gz[k] = g[2];
+        }
+    }
+    T* const fo = force + (size_t)t * 3;
     if constexpr (sizeof(T) == 4) {
         // fp32 segments: every value is rounded to a multiple of 2^q, q chosen from the segment's
         // largest magnitude and its length so that any partial sum of the rounded values fits the
-        // 53 bits of a double: the additions are then exact in whatever order they happen.  The
-        // first four entries of every lane stay in registers between the two passes.
-        float gx[4], gy[4], gz[4];
+        // 53 bits of a double: the additions are then exact in whatever order they happen.
         float mf = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int e = sub + 16 * k;
-            gx[k] = 0.0f; gy[k] = 0.0f; gz[k] = 0.0f;
-            if (e < cnt) {
-                const float* g = seg_g + (size_t)(beg + e) * 3;
-                gx[k] = g[0]; gy[k] = g[1]; gz[k] = g[2];
-            }
-            mf = fmaxf(mf, fmaxf(fabsf(gx[k]), fmaxf(fabsf(gy[k]), fabsf(gz[k]))));
+        auto larger = [&](float a0, float a1, float a2) __attribute__((always_inline)) {
             // fmaxf drops a NaN operand: keep it
-            if (gx[k] != gx[k] || gy[k] != gy[k] || gz[k] != gz[k]) mf = NAN;
-        }
-        for (int e = sub + 64; e < cnt; e += 16) {
-            const float* g = seg_g + (size_t)(beg + e) * 3;
-            const float a0 = g[0], a1 = g[1], a2 = g[2];
             if (!(mf != mf)) mf = fmaxf(mf, fmaxf(fabsf(a0), fmaxf(fabsf(a1), fabsf(a2))));
             if (a0 != a0 || a1 != a1 || a2 != a2) mf = NAN;
-        }
+        };
+#pragma unroll
+        for (int k = 0; k < 4; k++) larger(gx[k], gy[k], gz[k]);
+        others([&](const T* g) __attribute__((always_inline)) { larger(g[0], g[1], g[2]); });
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) {
             const float o = __shfl_xor(mf, off, 64);
             mf = (mf != mf || o != o) ? NAN : fmaxf(mf, o);
         }
-        if (cnt == 0) return;               // uniform over the 16 lanes of a target
         const bool finite = mf < 3.0e38f && mf == mf;
         double s0 = 0.0, s1 = 0.0, s2 = 0.0;
         const bool any = finite && mf > 0.0f;
         if (any) {
             // |v| < 2^(ex+1), fewer than 2^hb of them: sums stay below 2^(ex+1+hb), so q = ex + hb - 52;
             // (v + C) - C with C = 1.5 * 2^(52+q) rounds v to a multiple of 2^q (needs hb >= 2)
-            const int hb = max(32 - __clz(cnt), 2);
+            const int hb = max(32 - __clz(all), 2);
             const double C = ldexp(1.5, ilogbf(mf) + hb);
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -215,12 +252,11 @@ __global__ void reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g
                 s1 += ((double)gy[k] + C) - C;
                 s2 += ((double)gz[k] + C) - C;
             }
-            for (int e = sub + 64; e < cnt; e += 16) {
-                const float* g = seg_g + (size_t)(beg + e) * 3;
+            others([&](const T* g) __attribute__((always_inline)) {
                 s0 += ((double)g[0] + C) - C;
                 s1 += ((double)g[1] + C) - C;
                 s2 += ((double)g[2] + C) - C;
-            }
+            });
         }
 #pragma unroll
         for (int off = 8; off > 0; off >>= 1) {
@@ -229,54 +265,57 @@ __global__ void reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g
             s2 += __shfl_xor(s2, off, 64);
         }
         if (sub == 0) {
-            T* f = force + (size_t)t * 3;
             if (!finite) {
-                f[0] = f[1] = f[2] = (T)NAN;
+                fo[0] = fo[1] = fo[2] = (T)NAN;
             } else if (any) {
-                f[0] = (T)((double)f[0] - s0);
-                f[1] = (T)((double)f[1] - s1);
-                f[2] = (T)((double)f[2] - s2);
+                fo[0] = (T)((double)fo[0] - s0);
+                fo[1] = (T)((double)fo[1] - s1);
+                fo[2] = (T)((double)fo[2] - s2);
             }
         }
-        return;
-    }
-    // pass 1: largest magnitude of the segment
-    double m = 0.0;
-    for (int e = sub; e < cnt; e += 16) {
-        const T* g = seg_g + (size_t)(beg + e) * 3;
-        m = fmax(m, fmax(fabs((double)g[0]), fmax(fabs((double)g[1]), fabs((double)g[2]))));
-    }
+    } else {
+        double m = 0.0;
+        auto larger = [&](double a0, double a1, double a2) __attribute__((always_inline)) {
+            m = fmax(m, fmax(fabs(a0), fmax(fabs(a1), fabs(a2))));
+        };
 #pragma unroll
-    for (int off = 8; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
-    if (cnt == 0) return;               // uniform over the 16 lanes of a target
-    long long s0 = 0, s1 = 0, s2 = 0;
-    double scale = 0.0;
-    const bool finite = m < 1.0e300 && m == m;
-    if (m < 1.0e-280) m = 0.0;          // nothing but (sub)normal dust: contributes zero
-    if (m > 0.0 && finite) {
-        int bits = 61 - (32 - __clz(cnt));          // head-room for cnt additions
-        scale = ldexp(1.0, bits - 1 - ilogb(m));
-        for (int e = sub; e < cnt; e += 16) {
-            const T* g = seg_g + (size_t)(beg + e) * 3;
-            s0 += __double2ll_rn((double)g[0] * scale);
-            s1 += __double2ll_rn((double)g[1] * scale);
-            s2 += __double2ll_rn((double)g[2] * scale);
+        for (int k = 0; k < 4; k++) larger(gx[k], gy[k], gz[k]);
+        others([&](const T* g) __attribute__((always_inline)) { larger(g[0], g[1], g[2]); });
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+        long long s0 = 0, s1 = 0, s2 = 0;
+        double scale = 0.0;
+        const bool finite = m < 1.0e300 && m == m;
+        if (m < 1.0e-280) m = 0.0;          // nothing but (sub)normal dust: contributes zero
+        if (m > 0.0 && finite) {
+            const int bits = 61 - (32 - __clz(all));    // head-room for that many additions
+            scale = ldexp(1.0, bits - 1 - ilogb(m));
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                s0 += __double2ll_rn(gx[k] * scale);
+                s1 += __double2ll_rn(gy[k] * scale);
+                s2 += __double2ll_rn(gz[k] * scale);
+            }
+            others([&](const T* g) __attribute__((always_inline)) {
+                s0 += __double2ll_rn(g[0] * scale);
+                s1 += __double2ll_rn(g[1] * scale);
+                s2 += __double2ll_rn(g[2] * scale);
+            });
         }
-    }
 #pragma unroll
-    for (int off = 8; off > 0; off >>= 1) {
-        s0 += shfl_xor_ll(s0, off);
-        s1 += shfl_xor_ll(s1, off);
-        s2 += shfl_xor_ll(s2, off);
-    }
-    if (sub == 0) {
-        T* f = force + (size_t)t * 3;
-        if (!finite) {
-            f[0] = f[1] = f[2] = (T)NAN;
-        } else if (m > 0.0) {
-            f[0] = (T)((double)f[0] - (double)s0 / scale);
-            f[1] = (T)((double)f[1] - (double)s1 / scale);
-            f[2] = (T)((double)f[2] - (double)s2 / scale);
+        for (int off = 8; off > 0; off >>= 1) {
+            s0 += shfl_xor_ll(s0, off);
+            s1 += shfl_xor_ll(s1, off);
+            s2 += shfl_xor_ll(s2, off);
+        }
+        if (sub == 0) {
+            if (!finite) {
+                fo[0] = fo[1] = fo[2] = (T)NAN;
+            } else if (m > 0.0) {
+                fo[0] = (T)((double)fo[0] - (double)s0 / scale);
+                fo[1] = (T)((double)fo[1] - (double)s1 / scale);
+                fo[2] = (T)((double)fo[2] - (double)s2 / scale);
+            }
         }
     }
 }
@@ -302,51 +341,6 @@ int exclusive_scan_i32(const int* in, int* out, int n, int* tmp, hipStream_t str
     return A2P_OK;
 }
 
-template <typename T>
-int pair_csr_begin(PairCsr* csr, bool with_rank, int B, int P, int U, int nghost, const int* binum,
-                   const int* bnumneigh, const int* bfirstneigh, hipStream_t stream)
-{
-    const int NF = P + nghost;
-    const long long NT = (long long)B * NF;
-    const long long rows = (long long)B * P;
-    A2P_REQUIRE(NT < (1ll << 31) - SCAN_TILE && rows * U < (1ll << 31), A2P_ERR_INVALID,
-                "pair_reduce: batch too large for 32-bit pair indexing");
-    const int n = (int)NT;
-    const int ntiles = ceil_div(n, SCAN_TILE);
-    // workspace: counts[n] | offsets[n] | cursor[n] | tile[ntiles] | total[1] | seg_g[rows*U*3] | rank[rows*U]
-    size_t ints = (size_t)n * 3 + ntiles + 8;
-    size_t bytes = ((ints * sizeof(int) + 255) / 256) * 256;
-    size_t seg_bytes = (((size_t)rows * U * 3 * sizeof(T) + 255) / 256) * 256;
-    size_t rank_bytes = with_rank ? (size_t)rows * U * sizeof(int) : 0;
-    void* ws = nullptr;
-    int rc = ws_get(WS_CSR, bytes + seg_bytes + rank_bytes, &ws);
-    if (rc) return rc;
-    void* flags = nullptr;
-    rc = ws_get(WS_FLAGS, 64, &flags);
-    if (rc) return rc;
-    csr->n = n;
-    csr->seg_cap = 0;
-    csr->counts = (int*)ws;
-    csr->offsets = csr->counts + n;
-    csr->cursor = csr->offsets + n;
-    int* tiles = csr->cursor + n;
-    csr->seg_g = (void*)((char*)ws + bytes);
-    csr->rank = with_rank ? (int*)((char*)ws + bytes + seg_bytes) : nullptr;
-
-    // counts and cursor are adjacent and start at zero (offsets is fully overwritten)
-    rc = fill_zero(csr->counts, (size_t)n * sizeof(int), stream);
-    if (rc) return rc;
-    rc = fill_zero(csr->cursor, (size_t)n * sizeof(int), stream);
-    if (rc) return rc;
-
-    const int wave_blocks = ceil_div(rows * 64, 256);
-    prof_begin("reduce_count", stream);
-    hipLaunchKernelGGL(count_kernel, dim3(wave_blocks), dim3(256), 0, stream, csr->counts, csr->rank, B, P,
-                       U, NF, binum, bnumneigh, bfirstneigh, (int*)flags);
-    prof_end(stream);
-    return exclusive_scan_i32(csr->counts, csr->offsets, n, tiles, stream);
-}
-
 static thread_local int g_seg_capacity = 0;
 
 int pair_segment_capacity(int U) { return g_seg_capacity > U ? g_seg_capacity : U; }
@@ -368,9 +362,6 @@ int pair_fixed_begin(PairCsr* csr, int B, int P, int U_rows, int nghost, hipStre
     if (rc) return rc;
     csr->n = n;
     csr->seg_cap = U;
-    csr->counts = nullptr;
-    csr->offsets = nullptr;
-    csr->rank = nullptr;
     csr->cursor = (int*)ws;
     csr->seg_g = (void*)((char*)ws + bytes);
     if (cursor_ext) csr->cursor = cursor_ext;            // the caller keeps the counts
@@ -403,45 +394,67 @@ template <typename T>
 int pair_csr_finish(T* force, const PairCsr& csr, hipStream_t stream, T* etot, T* virial, const double* partial,
                     int B, int nblocks)
 {
-    // with ranks every counted pair has its place in the segment; otherwise the cursor holds
-    // how many entries were filled
     const int reduce_blocks = ceil_div((long long)csr.n * 16, 256);
     const int ev_blocks = (etot || virial) ? 10 * B : 0;
     prof_begin("reduce_sum", stream);
-    hipLaunchKernelGGL(reduce_kernel<T>, dim3(reduce_blocks + ev_blocks), dim3(256), 0, stream,
-                       force, (const T*)csr.seg_g, csr.offsets, csr.rank ? csr.counts : csr.cursor, csr.n,
-                       csr.seg_cap, reduce_blocks, etot, virial, partial, nblocks);
+    hipLaunchKernelGGL((reduce_kernel<T, false>), dim3(reduce_blocks + ev_blocks), dim3(256), 0, stream,
+                       force, (const T*)csr.seg_g, (const int*)csr.cursor, csr.n, csr.seg_cap, (const int*)nullptr,
+                       (const int2*)nullptr, (const int*)nullptr, reduce_blocks, etot, virial, partial, nblocks);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
 }
 
 template <typename T>
-int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, const int* binum,
-                const int* bnumneigh, const int* bfirstneigh, hipStream_t stream)
+int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, const int* binum, const int* bilist,
+                const int* bnumneigh, const int* bfirstneigh, bool own, hipStream_t stream)
 {
-    PairCsr csr;
-    int rc = pair_csr_begin<T>(&csr, false, B, P, U, nghost, binum, bnumneigh, bfirstneigh, stream);
+    const int NF = P + nghost;
+    const long long NT = (long long)B * NF, rows = (long long)B * P;
+    A2P_REQUIRE(NT < (1ll << 31) - 1 && rows * U < (1ll << 31), A2P_ERR_INVALID,
+                "pair_reduce: batch too large for 32-bit pair indexing");
+    const int n = (int)NT;
+    // workspace: cursor[n] | nspill[1] | seg[n*U] | spill[rows*U] (8 bytes each)
+    const size_t head = (((size_t)n + 1) * sizeof(int) + 255) / 256 * 256;
+    const size_t seg_bytes = ((size_t)n * U * sizeof(int) + 255) / 256 * 256;
+    void* ws = nullptr;
+    int rc = ws_get(WS_CSR, head + seg_bytes + (size_t)rows * U * sizeof(int2), &ws);
     if (rc) return rc;
-    const long long rows = (long long)B * P;
-    const int wave_blocks = ceil_div(rows * 64, 256);
-    prof_begin("reduce_fill", stream);
-    hipLaunchKernelGGL(fill_kernel<T>, dim3(wave_blocks), dim3(256), 0, stream, (T*)csr.seg_g, csr.cursor,
-                       csr.offsets, pair_g, B, P, U, P + nghost, binum, bnumneigh, bfirstneigh);
+    int* cursor = (int*)ws;
+    int* nspill = cursor + n;
+    int* seg = (int*)((char*)ws + head);
+    int2* spill = (int2*)((char*)ws + head + seg_bytes);
+    rc = ws_get(WS_FLAGS, 64, &ws);
+    if (rc) return rc;
+    // own: the rows' own sums are formed here, and atoms without a row start from zero
+    rc = fill_zero2(cursor, ((size_t)n + 1) * sizeof(int), own ? (void*)force : nullptr, own ? (size_t)n * 3 * sizeof(T) : 0,
+                    stream);
+    if (rc) return rc;
+    prof_begin("reduce_claim", stream);
+    hipLaunchKernelGGL((own ? claim_kernel<T, true> : claim_kernel<T, false>), dim3(ceil_div(rows * 64, 256)), dim3(256), 0,
+                       stream, B, P, U, NF, U, binum, bilist, bnumneigh, bfirstneigh, pair_g, cursor, seg, spill, nspill,
+                       force, (int*)ws);
     prof_end(stream);
-    return pair_csr_finish<T>(force, csr, stream);
+    rc = status_post_early(stream);
+    if (rc) return rc;
+    const int reduce_blocks = ceil_div((long long)n * 16, 256);
+    prof_begin("reduce_sum", stream);
+    hipLaunchKernelGGL((reduce_kernel<T, true>), dim3(reduce_blocks), dim3(256), 0, stream, force, pair_g,
+                       (const int*)cursor, n, U, (const int*)seg, (const int2*)spill, (const int*)nspill, reduce_blocks,
+                       (T*)nullptr, (T*)nullptr, (const double*)nullptr, 0);
+    prof_end(stream);
+    A2P_HIP_CHECK(hipGetLastError());
+    return A2P_OK;
 }
 
-template int pair_csr_begin<float>(PairCsr*, bool, int, int, int, int, const int*, const int*, const int*, hipStream_t);
-template int pair_csr_begin<double>(PairCsr*, bool, int, int, int, int, const int*, const int*, const int*, hipStream_t);
 template int pair_fixed_begin<float>(PairCsr*, int, int, int, int, hipStream_t, void*, size_t, int*, bool);
 template int pair_fixed_begin<double>(PairCsr*, int, int, int, int, hipStream_t, void*, size_t, int*, bool);
 template int pair_csr_finish<float>(float*, const PairCsr&, hipStream_t, float*, float*, const double*, int, int);
 template int pair_csr_finish<double>(double*, const PairCsr&, hipStream_t, double*, double*, const double*, int, int);
-template int pair_reduce<float>(float*, const float*, int, int, int, int, const int*, const int*,
-                                const int*, hipStream_t);
-template int pair_reduce<double>(double*, const double*, int, int, int, int, const int*, const int*,
-                                 const int*, hipStream_t);
+template int pair_reduce<float>(float*, const float*, int, int, int, int, const int*, const int*, const int*, const int*,
+                                bool, hipStream_t);
+template int pair_reduce<double>(double*, const double*, int, int, int, int, const int*, const int*, const int*,
+                                 const int*, bool, hipStream_t);
 
 }  // namespace a2p
 
