@@ -48,6 +48,7 @@ enum WsSlot {
     WS_MISC,
     WS_GRID,           // neighbor-list: the bin grid derived on the device (builds without read-back)
     WS_NEP_CLAIMS,     // NEP on compact lists: counters of claimed places and spare rows; zero between calls
+    WS_HOST_LISTS,     // neighbour lists on their way to host arrays
     WS_NSLOTS
 };
 // Returns a device pointer valid until the next ws_get on the same slot with a larger size.
@@ -57,6 +58,11 @@ int ws_get(int slot, size_t bytes, void** out);
 int ws_drop(int slot); // synchronises the device and frees one buffer of the current device (its contents are suspect)
 size_t ws_bytes();     // held on the current device
 int ws_release();      // synchronises the device, frees the current device's buffers
+
+// Host memory for arrays that are copied from or to the device, pinned (and reused) while the library's share of
+// pinned memory lasts, ordinary otherwise; given back with host_free from any thread.
+void* host_alloc(size_t bytes, bool* pinned);
+void host_free(void* p);
 
 // Device status word bits written by kernels when inputs violate the contract.
 enum StatusBits {

@@ -3,27 +3,18 @@
 //       -> (inum, ilist, numneigh, firstneigh, rcs, types, nghost)
 // (source/nblist/bind/nblist_bind.cc:35-207): same positional signature, same type checks
 // (TypeError), NumPy arrays in and out, float32 / float64 selected by the dtype of coords.
-// The list is built on the current HIP device by libai2pot_hip.so; inputs are copied to the
-// device and results back.  Unlike the reference, more than `umax` neighbours raises
+// The list is built on the current HIP device by libai2pot_hip.so (a2p_nblist_host_*); the arrays
+// returned share one block of host memory, owned by the last of them.  Unlike the reference, more than `umax` neighbours raises
 // RuntimeError instead of overrunning the output arrays.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #define NPY_NO_DEPRECATED_API NPY_1_7_API_VERSION
 #include <numpy/arrayobject.h>
-#include <hip/hip_runtime_api.h>
-
 #include <string>
-#include <vector>
 
 #include "../../../include/ai2pot_hip.h"
 
 namespace {
-
-struct DeviceBuf {
-    void* p = nullptr;
-    ~DeviceBuf() { if (p) (void)hipFree(p); }
-    bool alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess; }
-};
 
 PyObject* fail(PyObject* exc, const std::string& msg)
 {
@@ -31,47 +22,51 @@ PyObject* fail(PyObject* exc, const std::string& msg)
     return nullptr;
 }
 
-template <typename T>
+void free_block(PyObject* capsule)
+{
+    a2p_host_lists_free(PyCapsule_GetPointer(capsule, "a2p_host_lists"));
+}
+
+// An array over part of the block, which lives as long as any of its arrays.
+PyObject* array_over(PyObject* owner, int nd, npy_intp* dims, int type, void* data)
+{
+    PyObject* a = PyArray_SimpleNewFromData(nd, dims, type, data);
+    if (!a) return nullptr;
+    Py_INCREF(owner);
+    if (PyArray_SetBaseObject((PyArrayObject*)a, owner) != 0) {
+        Py_DECREF(a);
+        return nullptr;
+    }
+    return a;
+}
+
 PyObject* run(PyArrayObject* lattice, PyArrayObject* types, PyArrayObject* coords, double rcut, int umax,
               bool is_cart, const int* pbc, bool sort, int npy_float)
 {
     const int n = (int)PyArray_DIM(coords, 0);
     if (n <= 0) return fail(PyExc_RuntimeError, "the structure has no atoms");
-    DeviceBuf d_types, d_coords, d_ilist, d_nn, d_first, d_rcs, d_tout;
-    const size_t row = (size_t)n * umax;
-    if (!d_types.alloc(sizeof(int) * n) || !d_coords.alloc(sizeof(T) * n * 3) || !d_ilist.alloc(sizeof(int) * n) ||
-        !d_nn.alloc(sizeof(int) * n) || !d_first.alloc(sizeof(int) * row) || !d_rcs.alloc(sizeof(T) * row * 3) ||
-        !d_tout.alloc(sizeof(int) * n))
-        return fail(PyExc_MemoryError, "hipMalloc failed");
-    if (hipMemcpy(d_types.p, PyArray_DATA(types), sizeof(int) * n, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(d_coords.p, PyArray_DATA(coords), sizeof(T) * n * 3, hipMemcpyHostToDevice) != hipSuccess)
-        return fail(PyExc_RuntimeError, "copy to the device failed");
-    int max_nn = 0, rc;
-    if (sizeof(T) == 4)
-        rc = a2p_nblist_build_f32((const float*)PyArray_DATA(lattice), (const int*)d_types.p,
-                                  (const float*)d_coords.p, n, rcut, umax, is_cart, pbc, sort, (int*)d_ilist.p,
-                                  (int*)d_nn.p, (int*)d_first.p, (float*)d_rcs.p, (int*)d_tout.p, &max_nn, nullptr);
-    else
-        rc = a2p_nblist_build_f64((const double*)PyArray_DATA(lattice), (const int*)d_types.p,
-                                  (const double*)d_coords.p, n, rcut, umax, is_cart, pbc, sort, (int*)d_ilist.p,
-                                  (int*)d_nn.p, (int*)d_first.p, (double*)d_rcs.p, (int*)d_tout.p, &max_nn, nullptr);
+    a2p_host_lists out;
+    const int rc = npy_float == NPY_FLOAT32
+        ? a2p_nblist_host_f32((const float*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
+                              (const float*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, &out)
+        : a2p_nblist_host_f64((const double*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
+                              (const double*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, &out);
     if (rc != A2P_OK) return fail(PyExc_RuntimeError, std::string("libai2pot_hip: ") + a2p_last_error());
-
+    PyObject* owner = PyCapsule_New(out.block, "a2p_host_lists", free_block);
+    if (!owner) {
+        a2p_host_lists_free(out.block);
+        return nullptr;
+    }
     npy_intp d1[1] = {n}, d2[2] = {n, umax}, d3[3] = {n, umax, 3};
-    PyObject* ilist = PyArray_SimpleNew(1, d1, NPY_INT32);
-    PyObject* nn = PyArray_SimpleNew(1, d1, NPY_INT32);
-    PyObject* first = PyArray_SimpleNew(2, d2, NPY_INT32);
-    PyObject* rcs = PyArray_SimpleNew(3, d3, npy_float);
-    PyObject* tout = PyArray_SimpleNew(1, d1, NPY_INT32);
-    bool ok = ilist && nn && first && rcs && tout;
-    ok = ok && hipMemcpy(PyArray_DATA((PyArrayObject*)ilist), d_ilist.p, sizeof(int) * n, hipMemcpyDeviceToHost) == hipSuccess;
-    ok = ok && hipMemcpy(PyArray_DATA((PyArrayObject*)nn), d_nn.p, sizeof(int) * n, hipMemcpyDeviceToHost) == hipSuccess;
-    ok = ok && hipMemcpy(PyArray_DATA((PyArrayObject*)first), d_first.p, sizeof(int) * row, hipMemcpyDeviceToHost) == hipSuccess;
-    ok = ok && hipMemcpy(PyArray_DATA((PyArrayObject*)rcs), d_rcs.p, sizeof(T) * row * 3, hipMemcpyDeviceToHost) == hipSuccess;
-    ok = ok && hipMemcpy(PyArray_DATA((PyArrayObject*)tout), d_tout.p, sizeof(int) * n, hipMemcpyDeviceToHost) == hipSuccess;
-    if (!ok) {
+    PyObject* ilist = array_over(owner, 1, d1, NPY_INT32, out.ilist);
+    PyObject* nn = array_over(owner, 1, d1, NPY_INT32, out.numneigh);
+    PyObject* first = array_over(owner, 2, d2, NPY_INT32, out.firstneigh);
+    PyObject* rcs = array_over(owner, 3, d3, npy_float, out.rcs);
+    PyObject* tout = array_over(owner, 1, d1, NPY_INT32, out.types);
+    Py_DECREF(owner);
+    if (!(ilist && nn && first && rcs && tout)) {
         Py_XDECREF(ilist); Py_XDECREF(nn); Py_XDECREF(first); Py_XDECREF(rcs); Py_XDECREF(tout);
-        return fail(PyExc_RuntimeError, "copy from the device failed");
+        return nullptr;
     }
     return Py_BuildValue("(iNNNNNi)", n, ilist, nn, first, rcs, tout, 0);
 }
@@ -108,12 +103,9 @@ PyObject* py_find_info4mlff(PyObject*, PyObject* args)
     const long umax_l = PyLong_AsLong(umax);
     PyObject* out;
     if (umax_l <= 0 || umax_l > (1 << 20)) out = fail(PyExc_RuntimeError, "umax must be positive");
-    else if (ft == NPY_FLOAT32)
-        out = run<float>(c_lat, c_types, c_coords, PyFloat_AsDouble(rcut), (int)umax_l, PyObject_IsTrue(is_cart),
-                         pbc_i, PyObject_IsTrue(sort), NPY_FLOAT32);
     else
-        out = run<double>(c_lat, c_types, c_coords, PyFloat_AsDouble(rcut), (int)umax_l, PyObject_IsTrue(is_cart),
-                          pbc_i, PyObject_IsTrue(sort), NPY_FLOAT64);
+        out = run(c_lat, c_types, c_coords, PyFloat_AsDouble(rcut), (int)umax_l, PyObject_IsTrue(is_cart), pbc_i,
+                  PyObject_IsTrue(sort), ft);
     Py_DECREF(c_lat); Py_DECREF(c_coords); Py_DECREF(c_types);
     return out;
 }

@@ -3,6 +3,7 @@
 
 #include <atomic>
 #include <chrono>
+#include <cstdlib>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -22,6 +23,77 @@ void set_error(const char* fmt, ...)
 }
 
 const char* last_error() { return g_err.c_str(); }
+
+// ---- host blocks ---------------------------------------------------------------------------------------
+// Copies from pageable memory are staged by the runtime (90 KB took 36 us down and up to 100 us up, 9 us from pinned
+// memory) and pinning costs more than a small list: blocks are pinned once and kept.  The library holds at most
+// kPinnedMost bytes pinned, in use and idle together; a larger share, or a block above kPinnedBlock, is ordinary memory.
+namespace {
+constexpr size_t kPinnedMost = (size_t)256 << 20, kPinnedBlock = (size_t)64 << 20, kPinnedStep = 64 << 10;
+struct HostBlock {
+    char* ptr;
+    size_t bytes;
+    bool idle;
+};
+std::mutex g_host_mutex;
+std::vector<HostBlock> g_host_blocks;      // the pinned ones
+size_t g_host_pinned = 0;
+
+// frees idle blocks until `want` more bytes fit the share (all of them with want = kPinnedMost)
+void host_trim(size_t want)
+{
+    for (size_t i = 0; i < g_host_blocks.size() && g_host_pinned + want > kPinnedMost;) {
+        if (!g_host_blocks[i].idle) { i++; continue; }
+        (void)hipHostFree(g_host_blocks[i].ptr);
+        g_host_pinned -= g_host_blocks[i].bytes;
+        g_host_blocks.erase(g_host_blocks.begin() + i);
+    }
+}
+}  // namespace
+
+void* host_alloc(size_t bytes, bool* pinned)
+{
+    *pinned = false;
+    if (bytes <= kPinnedBlock) {
+        std::lock_guard<std::mutex> lock(g_host_mutex);
+        HostBlock* best = nullptr;
+        for (HostBlock& b : g_host_blocks)
+            if (b.idle && b.bytes >= bytes && b.bytes <= 2 * bytes + kPinnedStep && (!best || b.bytes < best->bytes)) best = &b;
+        if (best) {
+            // its last owner may have queued a copy that still reads it
+            if (hipDeviceSynchronize() == hipSuccess) {
+                best->idle = false;
+                *pinned = true;
+                return best->ptr;
+            }
+            return nullptr;
+        }
+        const size_t want = (bytes + kPinnedStep - 1) / kPinnedStep * kPinnedStep;
+        if (g_host_pinned + want > kPinnedMost) host_trim(want);
+        if (g_host_pinned + want <= kPinnedMost) {
+            void* p = nullptr;
+            if (hipHostMalloc(&p, want, hipHostMallocPortable) == hipSuccess && p) {
+                g_host_blocks.push_back({(char*)p, want, false});
+                g_host_pinned += want;
+                *pinned = true;
+                return p;
+            }
+            (void)hipGetLastError();
+        }
+    }
+    return malloc(bytes ? bytes : 1);
+}
+
+void host_free(void* p)
+{
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lock(g_host_mutex);
+        for (HostBlock& b : g_host_blocks)
+            if (b.ptr == (char*)p) { b.idle = true; return; }
+    }
+    free(p);
+}
 
 namespace {
 struct Buf {
@@ -92,6 +164,10 @@ int ws_release()
     int dev = 0;
     A2P_HIP_CHECK(hipGetDevice(&dev));
     A2P_HIP_CHECK(hipDeviceSynchronize());          // no kernel of any stream still uses the buffers
+    {
+        std::lock_guard<std::mutex> host_lock(g_host_mutex);
+        host_trim(kPinnedMost);
+    }
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     if ((int)g_ws.size() <= dev) return A2P_OK;
     for (Buf& b : g_ws[dev].slot) {

@@ -189,6 +189,22 @@ int a2p_nblist_build_f64(const double* lattice, const int* types, const double* 
                          int* numneigh, int* firstneigh, double* rcs, int* types_out, int* max_numneigh,
                          void* stream);
 
+/* The list with host arrays in and out, as nblist.find_info4mlff has them (source/nblist/bind/nblist_bind.cc:35-189):
+ * types int32[natoms] and coords [natoms, 3] are host pointers; the results lie in one host block that the caller hands
+ * back to a2p_host_lists_free (any thread; the library keeps pinned blocks for later calls, at most 256 MiB in all).
+ * Runs on the null stream and waits for it.  A neighbour count above umax is A2P_ERR_OVERFLOW, and nothing is returned. */
+typedef struct {
+    void* block;          /* owns the five arrays */
+    void* rcs;            /* [natoms, umax, 3] of the type of coords */
+    int *firstneigh, *ilist, *numneigh, *types;
+    int max_numneigh;
+} a2p_host_lists;
+int a2p_nblist_host_f32(const float* lattice, const int* types, const float* coords, int natoms, double rcut, int umax,
+                        int is_cart, const int* pbc, int sort, a2p_host_lists* out);
+int a2p_nblist_host_f64(const double* lattice, const int* types, const double* coords, int natoms, double rcut, int umax,
+                        int is_cart, const int* pbc, int sort, a2p_host_lists* out);
+void a2p_host_lists_free(void* block);
+
 /* Rebuild into buffers that already hold a list.  Same arguments and results as
  * a2p_nblist_build_*, for a caller that keeps its list buffers between steps (molecular
  * dynamics; the reference allocates fresh arrays per call, nblist_bind.cc:95-134, so it has no
