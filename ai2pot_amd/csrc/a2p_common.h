@@ -84,6 +84,16 @@ struct ReadBack {
 };
 int read_back_post(const void* device_src, int nwords, hipStream_t stream, ReadBack* rb);
 int read_back_wait(const ReadBack& rb, void* host_dst);
+// For a kernel that posts by itself: the slot's words (1.. are the data, word 0 the number rb->seq, written last and
+// with system scope: read_back_store), or null when no slot is free; the caller launches and then waits as above.
+int* read_back_take(int nwords, hipStream_t stream, ReadBack* rb);
+void read_back_drop(const ReadBack& rb);       // a taken slot whose kernel was not launched
+// By one lane.
+__device__ __forceinline__ void read_back_store(int* slot, int seq, const int* words, int n)
+{
+    for (int i = 0; i < n; i++) __hip_atomic_store(slot + 1 + i, words[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(slot, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 // Called where every check of the call's inputs has been queued: posts the status word if the calling thread asked
 // for it (a2p_status_early).
 int status_post_early(hipStream_t stream);

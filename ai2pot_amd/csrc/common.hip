@@ -200,26 +200,40 @@ __global__ void read_back_kernel(const int* __restrict__ src, int nwords, int* h
 }
 }  // namespace
 
-int read_back_post(const void* device_src, int nwords, hipStream_t stream, ReadBack* rb)
+int* read_back_take(int nwords, hipStream_t stream, ReadBack* rb)
 {
-    A2P_REQUIRE(nwords > 0 && nwords < RB_WORDS, A2P_ERR_INVALID, "read_back: %d words", nwords);
+    rb->src = nullptr; rb->nwords = nwords; rb->stream = stream; rb->slot = -1;
+    if (nwords < 1 || nwords >= RB_WORDS) return nullptr;
     {
         std::lock_guard<std::mutex> lock(g_rb_mutex);
         if (!g_rb_page) {
             void* p = nullptr;
-            A2P_HIP_CHECK(hipHostMalloc(&p, RB_SLOTS * RB_WORDS * sizeof(int), hipHostMallocPortable));
+            if (hipHostMalloc(&p, RB_SLOTS * RB_WORDS * sizeof(int), hipHostMallocPortable) != hipSuccess) return nullptr;
             for (int i = 0; i < RB_SLOTS * RB_WORDS; i++) ((int*)p)[i] = 0;
             g_rb_page = (int*)p;
         }
     }
-    rb->src = device_src; rb->nwords = nwords; rb->stream = stream; rb->slot = -1;
     for (unsigned long long used = g_rb_used.load(); ~used != 0ull;) {
         const int free_slot = __builtin_ctzll(~used);
         if (g_rb_used.compare_exchange_weak(used, used | (1ull << free_slot))) { rb->slot = free_slot; break; }
     }
-    if (rb->slot < 0) return A2P_OK;                 // more waiters than slots: read_back_wait copies instead
+    if (rb->slot < 0) return nullptr;
     int* const word = g_rb_page + rb->slot * RB_WORDS;
     do rb->seq = g_rb_seq.fetch_add(1) + 1; while (rb->seq == 0 || rb->seq == __atomic_load_n(word, __ATOMIC_RELAXED));
+    return word;
+}
+
+void read_back_drop(const ReadBack& rb)
+{
+    if (rb.slot >= 0) g_rb_used.fetch_and(~(1ull << rb.slot));
+}
+
+int read_back_post(const void* device_src, int nwords, hipStream_t stream, ReadBack* rb)
+{
+    A2P_REQUIRE(nwords > 0 && nwords < RB_WORDS, A2P_ERR_INVALID, "read_back: %d words", nwords);
+    int* const word = read_back_take(nwords, stream, rb);
+    rb->src = device_src;
+    if (!word) return A2P_OK;                        // more waiters than slots: read_back_wait copies instead
     hipLaunchKernelGGL(read_back_kernel, dim3(1), dim3(64), 0, stream, (const int*)device_src, nwords, word, rb->seq);
     const hipError_t err = hipGetLastError();
     if (err != hipSuccess) g_rb_used.fetch_and(~(1ull << rb->slot));

@@ -28,6 +28,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <atomic>
 #include <climits>
 #include <cmath>
 #include <vector>
@@ -110,6 +111,38 @@ __device__ __forceinline__ int bin_of(T c, T mn, T bin_size)      // binLinkedLi
 }
 
 // ---- 1. coordinates and extents --------------------------------------------------------------
+// Cartesian coordinates of atom p, and the extremes of its images (v[0..2] minima, v[3..5] maxima).
+template <typename T>
+__device__ __forceinline__ void atom_extremes(const Grid<T>& g, const T* __restrict__ coords, int p, T (&c)[3], T (&v)[6])
+{
+    if (g.is_cart) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) c[a] = coords[(size_t)p * 3 + a];
+    } else {                                         // calc_cart_coords, structure.h:561-579
+        const T f0 = coords[(size_t)p * 3], f1 = coords[(size_t)p * 3 + 1], f2 = coords[(size_t)p * 3 + 2];
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+            c[a] = add_rn(add_rn(mul_rn(f0, g.b[0][a]), mul_rn(f1, g.b[1][a])), mul_rn(f2, g.b[2][a]));
+    }
+    // Extremes over the atom's images (structure.h:1018-1052 takes them over the whole supercell).  Rounded
+    // multiplication and addition are monotone in each operand, so image_coord is monotone in each image
+    // index, rising or falling with the sign of the lattice component: the extremes sit at the ends of
+    // the index ranges, and two images per axis give the same values as the loop over all of them.
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        int lo[3], hi[3];
+#pragma unroll
+        for (int w = 0; w < 3; w++) {
+            const int first = g.img_lo[w], last = g.img_lo[w] + g.img_dim[w] - 1;
+            const bool rising = g.b[w][a] >= (T)0;
+            lo[w] = rising ? first : last;
+            hi[w] = rising ? last : first;
+        }
+        v[a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], lo[0], lo[1], lo[2]);
+        v[3 + a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], hi[0], hi[1], hi[2]);
+    }
+}
+
 template <typename T>
 __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coords, T* __restrict__ x,
                                      T* __restrict__ partial)
@@ -123,38 +156,15 @@ __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coor
         v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
     }
     if (p < g.N) {
-        T c[3];
-        if (g.is_cart) {
-#pragma unroll
-            for (int a = 0; a < 3; a++) c[a] = coords[(size_t)p * 3 + a];
-        } else {                                         // calc_cart_coords, structure.h:561-579
-            const T f0 = coords[(size_t)p * 3], f1 = coords[(size_t)p * 3 + 1], f2 = coords[(size_t)p * 3 + 2];
-#pragma unroll
-            for (int a = 0; a < 3; a++)
-                c[a] = add_rn(add_rn(mul_rn(f0, g.b[0][a]), mul_rn(f1, g.b[1][a])), mul_rn(f2, g.b[2][a]));
-        }
+        T c[3], w[6];
+        atom_extremes<T>(g, coords, p, c, w);
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             x[(size_t)p * 3 + a] = c[a];
+            v[a] = w[a];
+            v[3 + a] = w[3 + a];
             v[6 + a] = c[a];
             v[9 + a] = c[a];
-        }
-        // Extremes over the atom's images (structure.h:1018-1052 takes them over the whole supercell).  Rounded
-        // multiplication and addition are monotone in each operand, so image_coord is monotone in each image
-        // index, rising or falling with the sign of the lattice component: the extremes sit at the ends of
-        // the index ranges, and two images per axis give the same values as the loop over all of them.
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            int lo[3], hi[3];
-#pragma unroll
-            for (int w = 0; w < 3; w++) {
-                const int first = g.img_lo[w], last = g.img_lo[w] + g.img_dim[w] - 1;
-                const bool rising = g.b[w][a] >= (T)0;
-                lo[w] = rising ? first : last;
-                hi[w] = rising ? last : first;
-            }
-            v[a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], lo[0], lo[1], lo[2]);
-            v[3 + a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], hi[0], hi[1], hi[2]);
         }
     }
 #pragma unroll
@@ -211,6 +221,36 @@ __global__ void minmax_finish_kernel(const T* __restrict__ partial, int nblocks,
 // otherwise (or if an extent is not finite) the box
 // is made empty, so that no kernel indexes beyond the bound, and ST_GRID_BOUND is raised.
 template <typename T>
+__device__ __forceinline__ bool grid_axis(const Grid<T>& g, const T* ext, GridDyn<T>* gd, int a, int cap, double big_bound)
+{
+    bool ok = true;
+    const T lo = ext[a], hi = ext[3 + a];
+    if (!(fabs((double)lo) < 1.0e30) || !(fabs((double)hi) < 1.0e30)) ok = false;    // NaN, infinity or absurd
+    const T mn = sub_rn(lo, (T)kMargin);
+    const T mx = add_rn(hi, (T)kMargin);
+    const T pl = sub_rn(mx, mn);
+    if (!((double)pl / (double)g.bin_size < 1.0e9)) ok = false;       // the bin counts below must fit an int
+    const int nbin = (int)ceil(div_rn(pl, g.bin_size));
+    const int cb_lo = (int)floor(div_rn(sub_rn(ext[6 + a], mn), g.bin_size));
+    const int cb_hi = (int)floor(div_rn(sub_rn(ext[9 + a], mn), g.bin_size));
+    const int rlo = max(cb_lo - g.ext_bins, 0);
+    const int rhi = min(cb_hi + g.ext_bins, nbin - 1);
+    const int rdim = rhi - rlo + 1;
+    if (rdim <= 0 || rdim > cap) ok = false;
+    const double big = fmax(fabs((double)mn), fabs((double)mx));
+    const double slack = 1.0e-3 * (double)g.bin_size + 1.0e-5 * (big + (double)pl);
+    gd->mn[a] = mn;
+    gd->nbin[a] = nbin;
+    gd->rlo[a] = rlo;
+    gd->rdim[a] = rdim;
+    gd->keep_lo[a] = (T)((double)mn + (double)rlo * (double)g.bin_size - slack);
+    gd->keep_hi[a] = (T)((double)mn + (double)(rlo + rdim) * (double)g.bin_size + slack);
+    // the host sized the symmetry band of the compact lists for coordinates within big_bound
+    if (fmax(fabs((double)gd->keep_lo[a]), fabs((double)gd->keep_hi[a])) > big_bound) ok = false;
+    return ok;
+}
+
+template <typename T>
 __global__ void grid_setup_kernel(const Grid<T> g, const T* __restrict__ ext, GridDyn<T>* __restrict__ gd, int cap0,
                                   int cap1, int cap2, double big_bound, int* __restrict__ status)
 {
@@ -219,30 +259,8 @@ __global__ void grid_setup_kernel(const Grid<T> g, const T* __restrict__ ext, Gr
     bool ok = true;
     long long nregion = 1;
     for (int a = 0; a < 3; a++) {
-        const T lo = ext[a], hi = ext[3 + a];
-        if (!(fabs((double)lo) < 1.0e30) || !(fabs((double)hi) < 1.0e30)) ok = false;    // NaN, infinity or absurd
-        const T mn = sub_rn(lo, (T)kMargin);
-        const T mx = add_rn(hi, (T)kMargin);
-        const T pl = sub_rn(mx, mn);
-        if (!((double)pl / (double)g.bin_size < 1.0e9)) ok = false;       // the bin counts below must fit an int
-        const int nbin = (int)ceil(div_rn(pl, g.bin_size));
-        const int cb_lo = (int)floor(div_rn(sub_rn(ext[6 + a], mn), g.bin_size));
-        const int cb_hi = (int)floor(div_rn(sub_rn(ext[9 + a], mn), g.bin_size));
-        const int rlo = max(cb_lo - g.ext_bins, 0);
-        const int rhi = min(cb_hi + g.ext_bins, nbin - 1);
-        int rdim = rhi - rlo + 1;
-        if (rdim <= 0 || rdim > cap[a]) ok = false;
-        const double big = fmax(fabs((double)mn), fabs((double)mx));
-        const double slack = 1.0e-3 * (double)g.bin_size + 1.0e-5 * (big + (double)pl);
-        gd->mn[a] = mn;
-        gd->nbin[a] = nbin;
-        gd->rlo[a] = rlo;
-        gd->rdim[a] = rdim;
-        gd->keep_lo[a] = (T)((double)mn + (double)rlo * (double)g.bin_size - slack);
-        gd->keep_hi[a] = (T)((double)mn + (double)(rlo + rdim) * (double)g.bin_size + slack);
-        // the host sized the symmetry band of the compact lists for coordinates within big_bound
-        if (fmax(fabs((double)gd->keep_lo[a]), fabs((double)gd->keep_hi[a])) > big_bound) ok = false;
-        nregion *= rdim > 0 ? rdim : 0;
+        if (!grid_axis<T>(g, ext, gd, a, cap[a], big_bound)) ok = false;
+        nregion *= gd->rdim[a] > 0 ? gd->rdim[a] : 0;
     }
     if (!ok) {
         for (int a = 0; a < 3; a++) { gd->rdim[a] = 0; gd->keep_lo[a] = (T)1; gd->keep_hi[a] = (T)-1; }
@@ -413,6 +431,227 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
         // compact lists: the species, and whether this is an image outside the cell (image number != central)
         entry_store<T>(s_rec + (size_t)i * 4, x, y, z,
                        types ? at | ((types[at] & 15) << CL_TYPE_SHIFT) | (idx / natoms != central ? CL_IMAGE_BIT : 0) : at);
+    }
+}
+
+// ---- 1-5 in one workgroup: structures of up to NBS_ATOMS atoms --------------------------------------------
+// Such a build is bound by the latency of nine short launches and of the wait for the extents (51 us of GPU time for
+// 4096 atoms of which 38 in kernels; 28 us for 108).  One workgroup of 1024 threads does the same with its counters in
+// LDS: extents, grid, counts, prefix sum, image numbers dealt to their bins, and every record written once, to its final
+// place (an image's place in its bin is the number of larger image numbers there).  The images of an atom are found per
+// axis when the lattice is diagonal and an axis has at most three images and kept in three
+// registers per atom, else one by one.  What the grid turned out to be goes to the host while the rest runs; a box or image count
+// beyond the LDS empties the lists and is reported, and the host then takes the general route.
+constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 11264, NBS_IMAGES = 15360;
+constexpr int NBS_AXIS = 254;                     // bins per axis: a bin is a byte, 255 marks an image outside the box
+constexpr int NBS_PER = NBS_ATOMS / NBS_THREADS;  // atoms per thread
+constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_IMAGES * 6;
+
+// posted to the host: [0] 1 if the lists are complete, [1..3] the box, [4..5] the largest |coordinate| kept (a double)
+constexpr int NBS_WORDS = 6;
+
+template <typename T>
+__global__ void __launch_bounds__(NBS_THREADS)
+small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restrict__ x, GridDyn<T>* __restrict__ gd,
+                  int* __restrict__ offsets, T* __restrict__ s_rec, const int* __restrict__ types, int* __restrict__ ilist,
+                  int* __restrict__ types_out, int* __restrict__ incoming, int mark_types, int separable, int cap0, int cap1,
+                  int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq)
+{
+    extern __shared__ __align__(16) unsigned char sh_small[];
+    int* const cnt = (int*)sh_small;                             // per bin: count, then end of the bin's records
+    int* const num = cnt + NBS_BINS;                             // image numbers, by bin
+    unsigned short* const bin_of_num = (unsigned short*)(num + NBS_IMAGES);
+    __shared__ T sh_ext[NBS_THREADS / 64][12];
+    __shared__ T ext[12];
+    __shared__ GridDyn<T> dyn;
+    __shared__ int sh_ok[3], sh_scan[NBS_THREADS / 64], sh_bad;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int N = g_in.N;
+    if (tid == 0) sh_bad = 0;
+    __syncthreads();
+
+    // 1. coordinates, extents
+    T c[NBS_PER][3], v[12];
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        v[a] = (T)INT_MAX; v[3 + a] = (T)INT_MIN;       // structure.h:1018-1022
+        v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
+    }
+#pragma unroll
+    for (int u = 0; u < NBS_PER; u++) {
+        const int p = u * NBS_THREADS + tid;
+        c[u][0] = c[u][1] = c[u][2] = (T)0;
+        if (p < N) {
+            T w[6];
+            atom_extremes<T>(g_in, coords, p, c[u], w);
+            if (ilist) { ilist[p] = p; types_out[p] = types[p]; }      // neighborList.h:548-553
+            if (incoming) incoming[p] = 0;                             // counted up by the list kernel
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                x[(size_t)p * 3 + a] = c[u][a];
+                if (!(fabs((double)c[u][a]) < 1.0e30)) sh_bad = 1;     // the comparisons below pass a NaN by
+                v[a] = w[a] < v[a] ? w[a] : v[a];
+                v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
+                v[6 + a] = c[u][a] < v[6 + a] ? c[u][a] : v[6 + a];
+                v[9 + a] = c[u][a] > v[9 + a] ? c[u][a] : v[9 + a];
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < 12; q++) {
+        const bool is_min = (q % 6) < 3;
+        T r = v[q];
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const T o = __shfl_xor(r, off, 64);
+            r = is_min ? (o < r ? o : r) : (o > r ? o : r);
+        }
+        if (lane == 0) sh_ext[wv][q] = r;
+    }
+    __syncthreads();
+    if (tid < 12) {
+        const bool is_min = (tid % 6) < 3;
+        T r = sh_ext[0][tid];
+        for (int w = 1; w < NBS_THREADS / 64; w++) {
+            const T o = sh_ext[w][tid];
+            r = is_min ? (o < r ? o : r) : (o > r ? o : r);
+        }
+        ext[tid] = r;
+    }
+    __syncthreads();
+    if (tid < 3) sh_ok[tid] = grid_axis<T>(g_in, ext, &dyn, tid, tid == 0 ? cap0 : tid == 1 ? cap1 : cap2, big_bound) ? 1 : 0;
+    __syncthreads();
+    const long long nregion_ll = (long long)max(dyn.rdim[0], 0) * max(dyn.rdim[1], 0) * max(dyn.rdim[2], 0);
+    bool ok = !sh_bad && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform
+    const int nregion = ok ? (int)nregion_ll : 0;
+    const Grid<T> g = with_dyn<T>(g_in, &dyn);
+
+    // 2. counts
+    // separable: an axis' images inside the box, 10 bits each (image index, bin), and how many above bit 30
+    unsigned pk[NBS_PER][3];
+    for (int i = tid; i < nregion; i += NBS_THREADS) cnt[i] = 0;
+    __syncthreads();
+    if (ok && separable) {
+#pragma unroll
+        for (int u = 0; u < NBS_PER; u++) {
+            const bool have = u * NBS_THREADS + tid < N;
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                unsigned w = 0, n = 0;
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    // (the other axes' indices only add zeros: their lattice components along this axis vanish)
+                    const T ci = add_rn(c[u][a], mul_rn(g.b[a][a], (T)(g.img_lo[a] + i)));
+                    if (have && i < g.img_dim[a] && !(ci < g.keep_lo[a] || ci > g.keep_hi[a])) {
+                        const int b = bin_of(ci, g.mn[a], g.bin_size) - g.rlo[a];
+                        if (b >= 0 && b < g.rdim[a]) { w |= ((unsigned)i << 8 | (unsigned)b) << (10 * n); n++; }
+                    }
+                }
+                pk[u][a] = w | n << 30;
+            }
+        }
+    }
+    // calls f(image number, bin) on every image of the thread's atoms that lies in the box; a thread walks its own
+    // images only, so a wavefront takes as many trips as its atom with the most (eight next to a corner of the cell)
+    auto images = [&](auto&& f) __attribute__((always_inline)) {
+        if (separable) {
+#pragma unroll
+            for (int u = 0; u < NBS_PER; u++) {
+                if (u * NBS_THREADS >= N) break;                                  // uniform
+                const unsigned n0 = pk[u][0] >> 30, n1 = pk[u][1] >> 30, n2 = pk[u][2] >> 30, n = n0 * n1 * n2;
+                unsigned w0 = pk[u][0], w1 = pk[u][1], w2 = pk[u][2], j = 0, k = 0;
+                for (unsigned q = 0; q < n; q++) {
+                    const int bin = (int)(((w0 & 0xffu) * g.rdim[1] + (w1 & 0xffu)) * g.rdim[2] + (w2 & 0xffu));
+                    const int im = (int)((((w0 >> 8) & 3u) * g.img_dim[1] + ((w1 >> 8) & 3u)) * g.img_dim[2] + ((w2 >> 8) & 3u));
+                    f(im * N + u * NBS_THREADS + tid, bin);
+                    w2 >>= 10;
+                    if (++k == n2) {
+                        k = 0; w2 = pk[u][2];
+                        w1 >>= 10;
+                        if (++j == n1) { j = 0; w1 = pk[u][1]; w0 >>= 10; }
+                    }
+                }
+            }
+        } else {
+            for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
+                const int m = w / N, p = w - m * N;
+                const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
+                const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+                T ci[3];
+                const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
+                if (b >= 0) f(w, b);
+            }
+        }
+    };
+    if (ok) images([&](int, int b) __attribute__((always_inline)) { atomicAdd(&cnt[b], 1); });
+    __syncthreads();
+
+    // 3. prefix sum in place: a thread takes consecutive bins
+    const int per = (nregion + NBS_THREADS - 1) / NBS_THREADS;
+    const int b0 = min(tid * per, nregion), b1 = min(b0 + per, nregion);
+    int mine = 0;
+    for (int b = b0; b < b1; b++) mine += cnt[b];
+    const int incl = wave_inclusive_scan(mine);
+    if (lane == 63) sh_scan[wv] = incl;
+    __syncthreads();
+    int run = incl - mine, total = 0;
+    for (int w = 0; w < NBS_THREADS / 64; w++) {
+        if (w < wv) run += sh_scan[w];
+        total += sh_scan[w];
+    }
+    ok = ok && total <= NBS_IMAGES;                              // uniform
+    for (int b = b0; b < b1; b++) {
+        const int n = cnt[b];
+        cnt[b] = run;
+        if (ok) offsets[b] = run;
+        run += n;
+    }
+    if (tid == 0) {
+        if (!ok) {
+            for (int a = 0; a < 3; a++) { dyn.rdim[a] = 0; dyn.keep_lo[a] = (T)1; dyn.keep_hi[a] = (T)-1; }
+            if (raise) atomicOr(status, ST_GRID_BOUND);
+        }
+        dyn.nregion = ok ? nregion : 0;
+        if (ok) offsets[nregion] = total;
+        double big = 0;
+        for (int a = 0; a < 3; a++) big = fmax(big, fmax(fabs((double)dyn.keep_lo[a]), fabs((double)dyn.keep_hi[a])));
+        *gd = dyn;
+        if (slot) {
+            const long long bits = __double_as_longlong(big);
+            const int words[NBS_WORDS] = {ok ? 1 : 0, dyn.rdim[0], dyn.rdim[1], dyn.rdim[2], (int)(bits & 0xffffffffll),
+                                          (int)(bits >> 32)};
+            read_back_store(slot, seq, words, NBS_WORDS);
+        }
+    }
+    if (!ok) return;
+    __syncthreads();
+
+    // 4. image numbers to their bins; afterwards cnt[b] is where bin b ends, and bin b + 1 begins
+    images([&](int m, int b) __attribute__((always_inline)) {
+        const int pos = atomicAdd(&cnt[b], 1);
+        num[pos] = m;
+        bin_of_num[pos] = (unsigned short)b;
+    });
+    __syncthreads();
+
+    // 5. records in descending image number within a bin (head insertion, binLinkedList.h:833)
+    const int central = ((-g.img_lo[0]) * g.img_dim[1] + (-g.img_lo[1])) * g.img_dim[2] + (-g.img_lo[2]);
+    for (int e = tid; e < total; e += NBS_THREADS) {
+        const int b = bin_of_num[e], m = num[e];
+        const int beg = b > 0 ? cnt[b - 1] : 0, end = cnt[b];
+        int place = beg;
+        for (int q = beg; q < end; q++) place += num[q] > m ? 1 : 0;
+        const int im = m / N, p = m - im * N;
+        const int k = im % g.img_dim[2], ij = im / g.img_dim[2];
+        const int i = ij / g.img_dim[1], j = ij % g.img_dim[1];
+        T ci[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++)
+            ci[a] = image_coord(x[(size_t)p * 3 + a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + i, g.img_lo[1] + j,
+                                g.img_lo[2] + k);
+        // as binsort_kernel leaves it
+        entry_store<T>(s_rec + (size_t)place * 4, ci[0], ci[1], ci[2],
+                       mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
     }
 }
 
@@ -1330,6 +1569,7 @@ struct GridBound {
     double lattice[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, rcut = 0;
     int rdim[3] = {0, 0, 0};
     double big = 0;    // largest |coordinate| of the box kept by that build
+    bool large = false;    // the box did not fit one workgroup (small_bins_kernel)
 };
 // a few structures per host thread (two calculators used in turn keep both of their bounds), oldest replaced first
 constexpr size_t kMaxBounds = 8;
@@ -1340,7 +1580,7 @@ template <typename T>
 int nblist_build(const T* lattice, const int* types, const T* coords, int N, double rcut_in, int umax,
                  int is_cart, const int* pbc, int sort, int* ilist, int* numneigh, int* firstneigh,
                  T* rcs, int* types_out, int* max_nn_host, hipStream_t stream, int update = 0,
-                 int* rank = nullptr, int* incoming = nullptr, const CompactOut* co = nullptr)
+                 int* rank = nullptr, int* incoming = nullptr, const CompactOut* co = nullptr, bool large = false)
 {
     const bool want_rows = !co || (ilist || numneigh || firstneigh || rcs || types_out);
     if (co) {
@@ -1415,18 +1655,11 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     int* status = (int*)flags;
 
     for (int a = 0; a < 3; a++) { g.mn[a] = 0; g.nbin[a] = 0; g.rlo[a] = 0; g.rdim[a] = 0; }
-    prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(nblocks), dim3(NBL_BLOCK), 0, stream, g, coords, x,
-                       partial);
-    prof_end(stream);
-    prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(12 * 64), 0, stream, partial, nblocks, ext_dev);
-    prof_end(stream);
     // the bin box: read back from the extents, or bounded by the box of the last synchronised build of this structure
     int device = 0;
     A2P_HIP_CHECK(hipGetDevice(&device));
-    const GridBound* bound = nullptr;
-    for (const GridBound& gb : g_bounds) {
+    GridBound* bound = nullptr;
+    for (GridBound& gb : g_bounds) {
         bool same = gb.valid && gb.device == device && gb.N == N && gb.is_cart == is_cart && gb.rcut == (double)g.rcut;
         for (int a = 0; a < 3 && same; a++) same = gb.pbc[a] == (pbc[a] ? 1 : 0);
         for (int q = 0; q < 9 && same; q++) same = gb.lattice[q] == (double)lattice[q];
@@ -1435,19 +1668,145 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     const bool same = bound != nullptr;
     const bool sync_free = g_sync_free && same && !max_nn_host &&
                            (long long)N * g.nimg * (long long)(4 * sizeof(T)) <= (2ll << 30);
-    GridDyn<T>* gd = nullptr;
-    long long nregion = 1;
+    auto remember = [&](const int (&rdim)[3], double big) {
+        GridBound nb;
+        nb.big = big;
+        nb.valid = true;
+        nb.large = large;
+        nb.device = device; nb.N = N; nb.is_cart = is_cart; nb.rcut = (double)g.rcut;
+        for (int a = 0; a < 3; a++) { nb.pbc[a] = pbc[a] ? 1 : 0; nb.rdim[a] = rdim[a]; }
+        for (int q = 0; q < 9; q++) nb.lattice[q] = (double)lattice[q];
+        if (bound) { *bound = nb; return; }
+        if (g_bounds.size() >= kMaxBounds) g_bounds.erase(g_bounds.begin());
+        g_bounds.push_back(nb);
+    };
+    // How far the box of a sync-free build may reach beyond the remembered one, and its coordinates with it.
+    int cap[3] = {NBS_AXIS, NBS_AXIS, NBS_AXIS};
     double big_coord = 0;                               // bound of the coordinates the build keeps
     if (sync_free) {
-        int cap[3];
         int grow = 0;
         for (int a = 0; a < 3; a++) {
             cap[a] = bound->rdim[a] + std::max(2, bound->rdim[a] / 8);
-            g.rdim[a] = cap[a];                         // host copies of the box serve launch and scratch sizes only
-            nregion *= cap[a];
             grow = std::max(grow, cap[a] - bound->rdim[a]);
         }
         big_coord = bound->big + (double)(grow + 2) * (double)g.bin_size;   // the box cannot have moved further
+    }
+
+    // One workgroup bins the whole structure (small_bins_kernel) when its images can be told axis by axis or are few, and
+    // the box expected of atoms inside the cell, a bin to spare on each side, fits its LDS.
+    bool diagonal = true;
+    for (int i = 0; i < 3; i++)
+        for (int j = 0; j < 3; j++) diagonal = diagonal && (i == j || g.b[i][j] == (T)0);
+    const bool separable = diagonal && g.img_dim[0] <= 3 && g.img_dim[1] <= 3 && g.img_dim[2] <= 3;
+    bool small = !large && !(same && bound->large) && N <= NBS_ATOMS && (separable || (long long)N * g.nimg <= NBS_IMAGES);
+    if (small) {
+        double bins = 1, images = N;
+        for (int a = 0; a < 3; a++) {
+            const double len = std::fabs((double)g.b[0][a]) + std::fabs((double)g.b[1][a]) + std::fabs((double)g.b[2][a]);
+            const double n = std::ceil(len / (double)g.bin_size) + 2 + 2 * g.ext_bins;
+            small = small && n <= NBS_AXIS;
+            bins *= n;
+            images *= std::min((double)g.img_dim[a], n * (double)g.bin_size / len);
+        }
+        small = small && bins < NBS_BINS && (!separable || images <= NBS_IMAGES);
+    }
+    // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
+    // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;
+    // otherwise through global memory by a thread per row
+    const bool sort_in_place = sort && umax % 4 == 0 && umax <= NBL_SORT_CAP && (uintptr_t)firstneigh % 16 == 0 &&
+                               (uintptr_t)rcs % 16 == 0 &&
+                               rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64) <= 48 * 1024;
+    size_t sort_bytes = sort_in_place ? (size_t)N * sizeof(int) + 256
+                        : sort        ? (size_t)N * umax * (2 * sizeof(int) + 4 * sizeof(T)) + 256
+                                      : 0;
+    ReadBack post;
+    bool posted = false;
+    struct Settle {                                     // a post that an early return leaves behind is still waited for
+        const ReadBack& rb;
+        const bool& open;
+        ~Settle() { int words[NBS_WORDS]; if (open) (void)read_back_wait(rb, words); }
+    } settle{post, posted};
+    auto box_of_post = [&]() -> int {                   // waits; 1: the box did not fit
+        int words[NBS_WORDS];
+        const int rcw = read_back_wait(post, words);
+        posted = false;
+        if (rcw) return -rcw;
+        if (!words[0]) return 1;
+        const long long bits = (long long)(unsigned)words[4] | (long long)words[5] << 32;
+        memcpy(&big_coord, &bits, sizeof(big_coord));
+        for (int a = 0; a < 3; a++) g.rdim[a] = words[1 + a];
+        remember({words[1], words[2], words[3]}, big_coord);
+        return 0;
+    };
+    auto general = [&]() {                              // (the rows of the abandoned build are empty: written in full)
+        return nblist_build<T>(lattice, types, coords, N, rcut_in, umax, is_cart, pbc, sort, ilist, numneigh, firstneigh, rcs,
+                               types_out, max_nn_host, stream, 0, rank, incoming, co, true);
+    };
+    int* post_slot = nullptr;
+    if (small && !sync_free) {
+        post_slot = read_back_take(NBS_WORDS, stream, &post);
+        small = post_slot != nullptr;                   // (every slot in use: the general route)
+    }
+    const dim3 pair_grid(ceil_div(N, NBL_BLOCK));
+    GridDyn<T>* gd = nullptr;
+    int* offsets = nullptr;
+    long long total = 0;
+    if (small) {
+        posted = !sync_free;
+        void* wsG = nullptr;
+        rc = ws_get(WS_GRID, 256, &wsG);
+        if (rc == A2P_OK) rc = ws_get(WS_NBL_B, (NBS_BINS + 1) * sizeof(int), (void**)&offsets);
+        gd = (GridDyn<T>*)wsG;
+        total = NBS_IMAGES;
+    }
+
+    if (small && rc == A2P_OK) {
+        void* wsC0 = nullptr;
+        rc = ws_get(WS_MISC, (size_t)NBS_IMAGES * 4 * sizeof(T) + 256 + sort_bytes, &wsC0);
+        static std::atomic<unsigned long long> lds_set{0};          // devices on which the kernel may use its LDS
+        if (rc == A2P_OK && (device > 63 || !(lds_set.load() & (1ull << device)))) {
+            if (hipFuncSetAttribute((const void*)small_bins_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)NBS_LDS) != hipSuccess) rc = A2P_ERR_HIP;
+            else if (device <= 63) lds_set.fetch_or(1ull << device);
+        }
+        if (rc == A2P_OK) {
+            const double bound_of_coords = sync_free ? big_coord : 1.0e30;
+            prof_begin("nbl_small_bins", stream);
+            hipLaunchKernelGGL(small_bins_kernel<T>, dim3(1), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x, gd, offsets,
+                               (T*)wsC0, types, want_rows ? ilist : (int*)nullptr, types_out, incoming, co ? 1 : 0,
+                               separable ? 1 : 0, cap[0], cap[1], cap[2], bound_of_coords, sync_free ? 1 : 0, status,
+                               posted ? post_slot : nullptr, post.seq);
+            prof_end(stream);
+            if (hipGetLastError() != hipSuccess) rc = A2P_ERR_HIP;
+        }
+        if (rc == A2P_OK && posted && co) {                 // the band of the compact lists needs the box
+            const int b = box_of_post();
+            if (b == 1) return general();
+            rc = -b;
+        }
+        for (int a = 0; a < 3 && (sync_free || !co); a++) g.rdim[a] = cap[a];     // (a bound for the order's keys)
+    }
+    if (small && rc != A2P_OK) {
+        if (rc == A2P_ERR_HIP) set_error("nblist: launch failed: %s", hipGetErrorString(hipGetLastError()));
+        if (posted) { read_back_drop(post); posted = false; }
+        return rc;
+    }
+    long long nregion = 1;
+    int split = 1, *cursor = nullptr;
+    dim3 image_grid;
+    if (!small) {
+    prof_begin("nbl_coords_minmax", stream);
+    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(nblocks), dim3(NBL_BLOCK), 0, stream, g, coords, x,
+                       partial);
+    prof_end(stream);
+    prof_begin("nbl_coords_minmax", stream);
+    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(12 * 64), 0, stream, partial, nblocks, ext_dev);
+    prof_end(stream);
+    if (sync_free) {
+        for (int a = 0; a < 3; a++) {
+            g.rdim[a] = cap[a];                         // host copies of the box serve launch and scratch sizes only
+            nregion *= cap[a];
+        }
         A2P_REQUIRE(nregion < (1ll << 30), A2P_ERR_INVALID, "nblist: %lld bins around the centre atoms", nregion);
         void* wsG = nullptr;
         rc = ws_get(WS_GRID, 256, &wsG);
@@ -1490,18 +1849,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                     nregion);
         for (int a = 0; a < 3; a++)
             big_coord = std::max(big_coord, std::max(std::fabs((double)g.keep_lo[a]), std::fabs((double)g.keep_hi[a])));
-        GridBound nb;
-        nb.big = big_coord;
-        nb.valid = true;
-        nb.device = device; nb.N = N; nb.is_cart = is_cart; nb.rcut = (double)g.rcut;
-        for (int a = 0; a < 3; a++) { nb.pbc[a] = pbc[a] ? 1 : 0; nb.rdim[a] = g.rdim[a]; }
-        for (int q = 0; q < 9; q++) nb.lattice[q] = (double)lattice[q];
-        if (bound) {
-            g_bounds[bound - g_bounds.data()] = nb;
-        } else {
-            if (g_bounds.size() >= kMaxBounds) g_bounds.erase(g_bounds.begin());
-            g_bounds.push_back(nb);
-        }
+        remember({g.rdim[0], g.rdim[1], g.rdim[2]}, big_coord);
     }
     const int nb1 = (int)nregion + 1;
 
@@ -1513,15 +1861,14 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     rc = ws_get(WS_NBL_B, ints * sizeof(int), &wsB);
     if (rc) return rc;
     int* counts = (int*)wsB;
-    int* offsets = counts + nb1;
-    int* cursor = offsets + nb1;
+    offsets = counts + nb1;
+    cursor = offsets + nb1;
     int* tmp = cursor + nb1;
     rc = fill_zero2(counts, (size_t)nb1 * sizeof(int), cursor, (size_t)nb1 * sizeof(int), stream);
     if (rc) return rc;
-    const dim3 pair_grid(ceil_div(N, NBL_BLOCK));
     // binning: a thread per atom, or per x-layer of an atom's images while the structure is small
-    const int split = (N < 65536 && g.img_dim[0] > 1) ? g.img_dim[0] : 1;
-    const dim3 image_grid(ceil_div((long long)N * split, NBL_BLOCK));
+    split = (N < 65536 && g.img_dim[0] > 1) ? g.img_dim[0] : 1;
+    image_grid = dim3(ceil_div((long long)N * split, NBL_BLOCK));
     prof_begin("nbl_count", stream);
     hipLaunchKernelGGL(count_kernel<T>, image_grid, dim3(NBL_BLOCK), 0, stream, g, x, counts, incoming,
                        (const GridDyn<T>*)gd, types, want_rows ? ilist : (int*)nullptr, types_out, split);
@@ -1531,24 +1878,16 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     // Entries of the sorted image arrays.  Every (atom, image) pair can own at most one: while that
     // bound stays below 2 GiB the arrays are simply sized for it and the host never learns the count
     // (one synchronisation less per build); beyond, the count is read back.
-    long long total = (long long)N * g.nimg;
+    total = (long long)N * g.nimg;
     if (total * (long long)(4 * sizeof(T)) > (2ll << 30)) {
         int counted = 0;
         rc = read_back(offsets + nregion, 1, &counted, stream);
         if (rc) return rc;
         total = counted;
     }
+    }
 
     size_t sorted_bytes = (size_t)total * 4 * sizeof(T) + 256;
-    // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
-    // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;
-    // otherwise through global memory by a thread per row
-    const bool sort_in_place = sort && umax % 4 == 0 && umax <= NBL_SORT_CAP && (uintptr_t)firstneigh % 16 == 0 &&
-                               (uintptr_t)rcs % 16 == 0 &&
-                               rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64) <= 48 * 1024;
-    size_t sort_bytes = sort_in_place ? (size_t)N * sizeof(int) + 256
-                        : sort        ? (size_t)N * umax * (2 * sizeof(int) + 4 * sizeof(T)) + 256
-                                      : 0;
     void* wsC = nullptr;
     rc = ws_get(WS_MISC, sorted_bytes + sort_bytes, &wsC);
     if (rc) return rc;
@@ -1566,6 +1905,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         tmp_first = order + (size_t)N * umax;
     }
 
+    if (!small) {
     prof_begin("nbl_fill", stream);
 
     hipLaunchKernelGGL(fill_kernel<T>, image_grid, dim3(NBL_BLOCK), 0, stream, g, x, offsets, cursor,
@@ -1577,6 +1917,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                        (int)nregion, offsets, s_rec, g.N, co ? types : (const int*)nullptr, (const GridDyn<T>*)gd,
                        ((-g.img_lo[0]) * g.img_dim[1] + (-g.img_lo[1])) * g.img_dim[2] + (-g.img_lo[2]));
     prof_end(stream);
+    }
     CompactEmit<T> ce{};
     if (co) {
         // processing order: atoms sorted by the Morton code of their bin (ties by index: the sort is stable)
@@ -1684,6 +2025,11 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         hipLaunchKernelGGL(gather_rows_kernel<T>, dim3(ceil_div(N, NBL_BLOCK / 64)), dim3(NBL_BLOCK), 0, stream, N, umax,
                            numneigh, order, tmp_first, tmp_rcs, firstneigh, rcs);
         prof_end(stream);
+    }
+    if (posted) {                                       // the rest of the build is queued: now see how the binning went
+        const int b = box_of_post();
+        if (b == 1) return general();
+        if (b) return -b;
     }
     A2P_HIP_CHECK(hipGetLastError());
 

@@ -1,0 +1,79 @@
+"""Lists of structures whose binning one workgroup does (csrc/nblist.hip, small_bins_kernel): atom counts around its
+threads and its limit, cells told axis by axis and cells whose images are tried one by one, open boundaries, and boxes
+that do not fit (atoms far outside the cell), where the build starts over on the general route."""
+import numpy as np
+import pytest
+
+from ai2pot_amd import synth
+from test_gpu_nblist import assert_same, gpu_list
+
+pytestmark = pytest.mark.gpu
+
+
+def jittered(n, seed, density=0.04, shape=(1.0, 1.2, 0.9)):
+    m = int(np.ceil(n ** (1 / 3)))
+    L = np.array(shape) * (n / density / np.prod(shape)) ** (1 / 3)
+    site = np.argsort(synth.rng_uniform(seed, m ** 3), kind="stable")[:n]       # any order of the atoms
+    f = (np.stack([site // (m * m), site // m % m, site % m], 1) + 0.25 * synth.rng_uniform(seed + 1, 3 * n).reshape(n, 3)) / m
+    return L, f
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 2, 63, 65, 500, 1023, 1024, 1025, 2049, 4095, 4096, 4097])
+def test_atom_counts(oracle, dt, n):
+    L, f = jittered(n, n)
+    ty = synth.rng_randint(n, n, 3)
+    for sort in (False, True):
+        args = (np.diag(L).astype(dt), ty, (f * L).astype(dt), 5.0, 120)
+        assert_same(gpu_list(*args, sort=sort), oracle.nblist(*args, sort=sort))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("pbc", [(True, True, True), (True, False, True), (False, False, False)])
+@pytest.mark.parametrize("n,tilt,rcut", [(7, 0.0, 6.0), (90, 0.3, 6.0), (560, 0.3, 6.0), (600, 0.3, 6.0), (120, 0.0, 7.5), (30, 0.0, 12.0)])
+def test_cells(oracle, dt, pbc, n, tilt, rcut):
+    """Five and more images along an axis, triclinic cells on both sides of the limit (atoms x images), fractional input."""
+    L, f = jittered(n, 7 * n)
+    lat = np.diag(L)
+    lat[1, 0], lat[2, 1] = tilt * L[0], -tilt * L[1]
+    ty = synth.rng_randint(n, n, 2)
+    for is_cart in (True, False):
+        x = (f @ lat if is_cart else f).astype(dt)
+        args = (lat.astype(dt), ty, x, rcut, 400)
+        a = gpu_list(*args, is_cart=is_cart, pbc=pbc)
+        assert_same(a, oracle.nblist(*args, is_cart=is_cart, pbc=pbc))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_atoms_outside_the_cell(oracle, dt):
+    """A few bins beyond the cell (fits), a dozen cells away (does not), and back, into fresh and into kept buffers."""
+    import torch
+    from ai2pot_amd.calculator import NepCalculator
+    n = 800
+    L, f = jittered(n, 5)
+    ty = synth.rng_randint(3, n, 3)
+    lat = np.diag(L).astype(dt)
+    m = synth.nep_model(rmax_radial=5.0, rmax_angular=4.0)
+    calc = NepCalculator(m, n, lat, ty, umax=120, dtype=torch.float32 if dt == np.float32 else torch.float64, path="segments")
+    for far in (0.0, 0.2, 12.0, 0.1, 12.0, 0.0):
+        x = f * L
+        x[::3, 0] += far * L[0]
+        x[1::3, 2] -= 0.5 * far * L[2]
+        args = (lat, ty, x.astype(dt), 5.0, 120)
+        want = oracle.nblist(*args)
+        assert_same(gpu_list(*args), want)
+        calc.step(torch.from_numpy(x.astype(dt)).to("cuda:0"))
+        calc.check()
+        nn = calc.numneigh.cpu().numpy()
+        assert np.array_equal(nn, want[2])
+        first, rcs = calc.firstneigh.cpu().numpy(), calc.rcs.cpu().numpy()
+        for i in range(n):
+            assert np.array_equal(first[i, :nn[i]], want[3][i, :nn[i]]) and np.array_equal(rcs[i, :nn[i]], want[4][i, :nn[i]])
+    bad = (f * L).astype(dt)
+    bad[401] = np.nan
+    try:
+        gpu_list(lat, ty, bad, 5.0, 120)
+    except RuntimeError:
+        pass
+    args = (lat, ty, (f * L).astype(dt), 5.0, 120)
+    assert_same(gpu_list(*args), oracle.nblist(*args))            # still usable
