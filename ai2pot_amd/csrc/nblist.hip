@@ -436,16 +436,24 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
 
 // ---- 1-5 in one workgroup: structures of up to NBS_ATOMS atoms --------------------------------------------
 // Such a build is bound by the latency of nine short launches and of the wait for the extents (51 us of GPU time for
-// 4096 atoms of which 38 in kernels; 28 us for 108).  One workgroup of 1024 threads does the same with its counters in
+// 4096 atoms, of which 38 in kernels; 29 us here, and 11 us for 108 atoms).  One workgroup of 1024 threads does the same with its counters in
 // LDS: extents, grid, counts, prefix sum, image numbers dealt to their bins, and every record written once, to its final
 // place (an image's place in its bin is the number of larger image numbers there).  The images of an atom are found per
-// axis when the lattice is diagonal and an axis has at most three images and kept in three
-// registers per atom, else one by one.  What the grid turned out to be goes to the host while the rest runs; a box or image count
+// axis when the lattice is diagonal and an axis has at most three images, else one by one.  What the grid turned out to be goes to the host while the rest runs; a box or image count
 // beyond the LDS empties the lists and is reported, and the host then takes the general route.
 constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 11264, NBS_IMAGES = 15360;
 constexpr int NBS_AXIS = 254;                     // bins per axis: a bin is a byte, 255 marks an image outside the box
-constexpr int NBS_PER = NBS_ATOMS / NBS_THREADS;  // atoms per thread
 constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_IMAGES * 6;
+
+constexpr int NBS_ATOM_BITS = 12, NBS_TRIPLES = 256;
+static_assert(NBS_ATOMS <= 1 << NBS_ATOM_BITS, "an atom's number fits below the image's");
+
+template <typename T>
+__device__ __forceinline__ unsigned image_triple(const Grid<T>& g, int im)
+{
+    const int k = im % g.img_dim[2], ij = im / g.img_dim[2];
+    return (unsigned)(ij / g.img_dim[1]) | (unsigned)(ij % g.img_dim[1]) << 10 | (unsigned)k << 20;
+}
 
 // posted to the host: [0] 1 if the lists are complete, [1..3] the box, [4..5] the largest |coordinate| kept (a double)
 constexpr int NBS_WORDS = 6;
@@ -455,68 +463,66 @@ __global__ void __launch_bounds__(NBS_THREADS)
 small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restrict__ x, GridDyn<T>* __restrict__ gd,
                   int* __restrict__ offsets, T* __restrict__ s_rec, const int* __restrict__ types, int* __restrict__ ilist,
                   int* __restrict__ types_out, int* __restrict__ incoming, int mark_types, int separable, int cap0, int cap1,
-                  int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq)
+                  int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq,
+                  unsigned* __restrict__ axis_images)
 {
     extern __shared__ __align__(16) unsigned char sh_small[];
     int* const cnt = (int*)sh_small;                             // per bin: count, then end of the bin's records
     int* const num = cnt + NBS_BINS;                             // image numbers, by bin
     unsigned short* const bin_of_num = (unsigned short*)(num + NBS_IMAGES);
-    __shared__ T sh_ext[NBS_THREADS / 64][12];
+    static_assert(NBS_LDS >= 12 * NBS_THREADS * sizeof(double), "the extremes pass through the counters' LDS");
     __shared__ T ext[12];
     __shared__ GridDyn<T> dyn;
     __shared__ int sh_ok[3], sh_scan[NBS_THREADS / 64], sh_bad;
+    __shared__ unsigned sh_triple[NBS_TRIPLES];                  // image number -> (i, j, k), 10 bits each
     const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int N = g_in.N;
     if (tid == 0) sh_bad = 0;
     __syncthreads();
 
     // 1. coordinates, extents
-    T c[NBS_PER][3], v[12];
+    T v[12];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         v[a] = (T)INT_MAX; v[3 + a] = (T)INT_MIN;       // structure.h:1018-1022
         v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
     }
+#pragma unroll 1
+    for (int p = tid; p < N; p += NBS_THREADS) {
+        T c[3], w[6];
+        atom_extremes<T>(g_in, coords, p, c, w);
+        if (ilist) { ilist[p] = p; types_out[p] = types[p]; }      // neighborList.h:548-553
+        if (incoming) incoming[p] = 0;                             // counted up by the list kernel
 #pragma unroll
-    for (int u = 0; u < NBS_PER; u++) {
-        const int p = u * NBS_THREADS + tid;
-        c[u][0] = c[u][1] = c[u][2] = (T)0;
-        if (p < N) {
-            T w[6];
-            atom_extremes<T>(g_in, coords, p, c[u], w);
-            if (ilist) { ilist[p] = p; types_out[p] = types[p]; }      // neighborList.h:548-553
-            if (incoming) incoming[p] = 0;                             // counted up by the list kernel
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                x[(size_t)p * 3 + a] = c[u][a];
-                if (!(fabs((double)c[u][a]) < 1.0e30)) sh_bad = 1;     // the comparisons below pass a NaN by
-                v[a] = w[a] < v[a] ? w[a] : v[a];
-                v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
-                v[6 + a] = c[u][a] < v[6 + a] ? c[u][a] : v[6 + a];
-                v[9 + a] = c[u][a] > v[9 + a] ? c[u][a] : v[9 + a];
-            }
+        for (int a = 0; a < 3; a++) {
+            x[(size_t)p * 3 + a] = c[a];
+            if (!(fabs((double)c[a]) < 1.0e30)) sh_bad = 1;        // the comparisons below pass a NaN by
+            v[a] = w[a] < v[a] ? w[a] : v[a];
+            v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
+            v[6 + a] = c[a] < v[6 + a] ? c[a] : v[6 + a];
+            v[9 + a] = c[a] > v[9 + a] ? c[a] : v[9 + a];
         }
     }
+    // each extreme is taken over the threads' values by one wavefront: twelve reductions by shuffles in every
+    // wavefront would be a chain of 72
+    T* const sh_v = (T*)sh_small;                                // [12][NBS_THREADS], before the counters
 #pragma unroll
-    for (int q = 0; q < 12; q++) {
-        const bool is_min = (q % 6) < 3;
-        T r = v[q];
+    for (int q = 0; q < 12; q++) sh_v[q * NBS_THREADS + tid] = v[q];
+    __syncthreads();
+    if (wv < 12) {
+        const bool is_min = (wv % 6) < 3;
+        T o[NBS_THREADS / 64];
+#pragma unroll
+        for (int w = 0; w < NBS_THREADS / 64; w++) o[w] = sh_v[wv * NBS_THREADS + w * 64 + lane];
+        T r = o[0];
+#pragma unroll
+        for (int w = 1; w < NBS_THREADS / 64; w++) r = is_min ? (o[w] < r ? o[w] : r) : (o[w] > r ? o[w] : r);
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
-            const T o = __shfl_xor(r, off, 64);
-            r = is_min ? (o < r ? o : r) : (o > r ? o : r);
+            const T t = __shfl_xor(r, off, 64);
+            r = is_min ? (t < r ? t : r) : (t > r ? t : r);
         }
-        if (lane == 0) sh_ext[wv][q] = r;
-    }
-    __syncthreads();
-    if (tid < 12) {
-        const bool is_min = (tid % 6) < 3;
-        T r = sh_ext[0][tid];
-        for (int w = 1; w < NBS_THREADS / 64; w++) {
-            const T o = sh_ext[w][tid];
-            r = is_min ? (o < r ? o : r) : (o > r ? o : r);
-        }
-        ext[tid] = r;
+        if (lane == 0) ext[wv] = r;
     }
     __syncthreads();
     if (tid < 3) sh_ok[tid] = grid_axis<T>(g_in, ext, &dyn, tid, tid == 0 ? cap0 : tid == 1 ? cap1 : cap2, big_bound) ? 1 : 0;
@@ -526,85 +532,119 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     const int nregion = ok ? (int)nregion_ll : 0;
     const Grid<T> g = with_dyn<T>(g_in, &dyn);
 
-    // 2. counts
-    // separable: an axis' images inside the box, 10 bits each (image index, bin), and how many above bit 30
-    unsigned pk[NBS_PER][3];
     for (int i = tid; i < nregion; i += NBS_THREADS) cnt[i] = 0;
+    if (tid < min(g.nimg, NBS_TRIPLES)) sh_triple[tid] = image_triple(g, tid);
     __syncthreads();
-    if (ok && separable) {
-#pragma unroll
-        for (int u = 0; u < NBS_PER; u++) {
-            const bool have = u * NBS_THREADS + tid < N;
-#pragma unroll
-            for (int a = 0; a < 3; a++) {
-                unsigned w = 0, n = 0;
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    // (the other axes' indices only add zeros: their lattice components along this axis vanish)
-                    const T ci = add_rn(c[u][a], mul_rn(g.b[a][a], (T)(g.img_lo[a] + i)));
-                    if (have && i < g.img_dim[a] && !(ci < g.keep_lo[a] || ci > g.keep_hi[a])) {
-                        const int b = bin_of(ci, g.mn[a], g.bin_size) - g.rlo[a];
-                        if (b >= 0 && b < g.rdim[a]) { w |= ((unsigned)i << 8 | (unsigned)b) << (10 * n); n++; }
-                    }
-                }
-                pk[u][a] = w | n << 30;
+
+    // 2. counts, 3. prefix sum, 4. image numbers to their bins.  One copy of the code that enumerates the images serves
+    // both passes: it runs once or a few times per call, so fetching instructions is a good part of what it costs.
+    int total = 0;
+#pragma unroll 1
+    for (int pass = 0; pass < 2 && ok; pass++) {
+        auto image = [&](int im, int p, int b) __attribute__((always_inline)) {
+            const int pos = atomicAdd(&cnt[b], 1);
+            if (pass) {
+                num[pos] = im << NBS_ATOM_BITS | p;              // ordered as the supercell index im * N + p
+                bin_of_num[pos] = (unsigned short)b;
             }
-        }
-    }
-    // calls f(image number, bin) on every image of the thread's atoms that lies in the box; a thread walks its own
-    // images only, so a wavefront takes as many trips as its atom with the most (eight next to a corner of the cell)
-    auto images = [&](auto&& f) __attribute__((always_inline)) {
-        if (separable) {
+        };
+        // the bin along axis a of the image that is i cells along it, or -1 outside the box (separable: the other axes'
+        // indices only add zeros, their lattice components along this axis vanish)
+        auto along = [&](T ca, int a, int i) __attribute__((always_inline)) -> int {
+            const T ci = add_rn(ca, mul_rn(g.b[a][a], (T)(g.img_lo[a] + i)));
+            if (ci < g.keep_lo[a] || ci > g.keep_hi[a]) return -1;
+            const int b = bin_of(ci, g.mn[a], g.bin_size) - g.rlo[a];
+            return b < g.rdim[a] ? b : -1;
+        };
+        if (separable && N * g.img_dim[0] * g.img_dim[1] <= 2 * NBS_THREADS) {
+            // few atoms: a thread takes the images in one column of cells of an atom
+#pragma unroll 1
+            for (int w = tid; w < N * g.img_dim[0] * g.img_dim[1]; w += NBS_THREADS) {
+                const int ij = w / N, p = w - ij * N, i = ij / g.img_dim[1], j = ij - i * g.img_dim[1];
+                const T cx = x[(size_t)p * 3], cy = x[(size_t)p * 3 + 1], cz = x[(size_t)p * 3 + 2];
+                const int bx = along(cx, 0, i), by = along(cy, 1, j);
+                if (bx < 0 || by < 0) continue;
+#pragma unroll 1
+                for (int k = 0; k < g.img_dim[2]; k++) {
+                    const int bz = along(cz, 2, k);
+                    if (bz >= 0) image(ij * g.img_dim[2] + k, p, (bx * g.rdim[1] + by) * g.rdim[2] + bz);
+                }
+            }
+        } else if (separable) {
+#pragma unroll 1
+            for (int p = tid; p < N; p += NBS_THREADS) {
+                // an axis' images inside the box, 10 bits each (image index, bin), and how many above bit 30
+                unsigned pk[3];
+                if (pass == 0) {
 #pragma unroll
-            for (int u = 0; u < NBS_PER; u++) {
-                if (u * NBS_THREADS >= N) break;                                  // uniform
-                const unsigned n0 = pk[u][0] >> 30, n1 = pk[u][1] >> 30, n2 = pk[u][2] >> 30, n = n0 * n1 * n2;
-                unsigned w0 = pk[u][0], w1 = pk[u][1], w2 = pk[u][2], j = 0, k = 0;
+                    for (int a = 0; a < 3; a++) {
+                        const T ca = x[(size_t)p * 3 + a];
+                        unsigned w = 0, n = 0;
+#pragma unroll 1
+                        for (int i = 0; i < g.img_dim[a]; i++) {
+                            const int b = along(ca, a, i);
+                            if (b >= 0) { w |= ((unsigned)i << 8 | (unsigned)b) << (10 * n); n++; }
+                        }
+                        pk[a] = w | n << 30;
+                        axis_images[p * 3 + a] = pk[a];
+                    }
+                } else {
+#pragma unroll
+                    for (int a = 0; a < 3; a++) pk[a] = axis_images[p * 3 + a];
+                }
+                // a thread walks its own images only: a wavefront takes as many trips as its atom with the most (eight
+                // next to a corner of the cell)
+                const unsigned n1 = pk[1] >> 30, n2 = pk[2] >> 30, n = (pk[0] >> 30) * n1 * n2;
+                unsigned w0 = pk[0], w1 = pk[1], w2 = pk[2], j = 0, k = 0;
+#pragma unroll 1
                 for (unsigned q = 0; q < n; q++) {
                     const int bin = (int)(((w0 & 0xffu) * g.rdim[1] + (w1 & 0xffu)) * g.rdim[2] + (w2 & 0xffu));
                     const int im = (int)((((w0 >> 8) & 3u) * g.img_dim[1] + ((w1 >> 8) & 3u)) * g.img_dim[2] + ((w2 >> 8) & 3u));
-                    f(im * N + u * NBS_THREADS + tid, bin);
+                    image(im, p, bin);
                     w2 >>= 10;
                     if (++k == n2) {
-                        k = 0; w2 = pk[u][2];
+                        k = 0; w2 = pk[2];
                         w1 >>= 10;
-                        if (++j == n1) { j = 0; w1 = pk[u][1]; w0 >>= 10; }
+                        if (++j == n1) { j = 0; w1 = pk[1]; w0 >>= 10; }
                     }
                 }
             }
         } else {
+#pragma unroll 1
             for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
                 const int m = w / N, p = w - m * N;
                 const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
                 const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
                 T ci[3];
                 const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
-                if (b >= 0) f(w, b);
+                if (b >= 0) image(m, p, b);
             }
         }
-    };
-    if (ok) images([&](int, int b) __attribute__((always_inline)) { atomicAdd(&cnt[b], 1); });
-    __syncthreads();
+        __syncthreads();
+        if (pass) break;                                         // cnt[b] is now where bin b ends, and bin b + 1 begins
 
-    // 3. prefix sum in place: a thread takes consecutive bins
-    const int per = (nregion + NBS_THREADS - 1) / NBS_THREADS;
-    const int b0 = min(tid * per, nregion), b1 = min(b0 + per, nregion);
-    int mine = 0;
-    for (int b = b0; b < b1; b++) mine += cnt[b];
-    const int incl = wave_inclusive_scan(mine);
-    if (lane == 63) sh_scan[wv] = incl;
-    __syncthreads();
-    int run = incl - mine, total = 0;
-    for (int w = 0; w < NBS_THREADS / 64; w++) {
-        if (w < wv) run += sh_scan[w];
-        total += sh_scan[w];
-    }
-    ok = ok && total <= NBS_IMAGES;                              // uniform
-    for (int b = b0; b < b1; b++) {
-        const int n = cnt[b];
-        cnt[b] = run;
-        if (ok) offsets[b] = run;
-        run += n;
+        // prefix sum in place: a thread takes consecutive bins
+        const int per = (nregion + NBS_THREADS - 1) / NBS_THREADS;
+        const int b0 = min(tid * per, nregion), b1 = min(b0 + per, nregion);
+        int mine = 0;
+        for (int b = b0; b < b1; b++) mine += cnt[b];
+        const int incl = wave_inclusive_scan(mine);
+        if (lane == 63) sh_scan[wv] = incl;
+        __syncthreads();
+        int run = incl - mine;
+        for (int w = 0; w < NBS_THREADS / 64; w++) {
+            const int t = sh_scan[w];
+            run += w < wv ? t : 0;
+            total += t;
+        }
+        ok = total <= NBS_IMAGES;                                // uniform
+        for (int b = b0; b < b1; b++) {
+            const int n = cnt[b];
+            cnt[b] = run;
+            if (ok) offsets[b] = run;
+            run += n;
+        }
+        __syncthreads();
     }
     if (tid == 0) {
         if (!ok) {
@@ -624,32 +664,24 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         }
     }
     if (!ok) return;
-    __syncthreads();
 
-    // 4. image numbers to their bins; afterwards cnt[b] is where bin b ends, and bin b + 1 begins
-    images([&](int m, int b) __attribute__((always_inline)) {
-        const int pos = atomicAdd(&cnt[b], 1);
-        num[pos] = m;
-        bin_of_num[pos] = (unsigned short)b;
-    });
-    __syncthreads();
-
-    // 5. records in descending image number within a bin (head insertion, binLinkedList.h:833)
+    // 5. records in descending image number within a bin (head insertion, binLinkedList.h:833), as binsort_kernel leaves
+    // them.  Shifts and a table stand in for the five integer divisions a record would take.
     const int central = ((-g.img_lo[0]) * g.img_dim[1] + (-g.img_lo[1])) * g.img_dim[2] + (-g.img_lo[2]);
+#pragma unroll 1
     for (int e = tid; e < total; e += NBS_THREADS) {
         const int b = bin_of_num[e], m = num[e];
+        const int im = m >> NBS_ATOM_BITS, p = m & ((1 << NBS_ATOM_BITS) - 1);
+        const unsigned t = im < NBS_TRIPLES ? sh_triple[im] : image_triple(g, im);
+        const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
         const int beg = b > 0 ? cnt[b - 1] : 0, end = cnt[b];
         int place = beg;
         for (int q = beg; q < end; q++) place += num[q] > m ? 1 : 0;
-        const int im = m / N, p = m - im * N;
-        const int k = im % g.img_dim[2], ij = im / g.img_dim[2];
-        const int i = ij / g.img_dim[1], j = ij % g.img_dim[1];
         T ci[3];
 #pragma unroll
         for (int a = 0; a < 3; a++)
-            ci[a] = image_coord(x[(size_t)p * 3 + a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + i, g.img_lo[1] + j,
-                                g.img_lo[2] + k);
-        // as binsort_kernel leaves it
+            ci[a] = image_coord(xp[a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + (int)(t & 1023u),
+                                g.img_lo[1] + (int)((t >> 10) & 1023u), g.img_lo[2] + (int)(t >> 20));
         entry_store<T>(s_rec + (size_t)place * 4, ci[0], ci[1], ci[2],
                        mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
     }
@@ -1638,10 +1670,11 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     g.inv_side = 1.0f / (float)(2 * g.ext_bins + 1);
     g.inv_bin = 1.0f / (float)g.bin_size;
 
-    // workspace A: x[N*3] | partial[nblocks*12] | ext[12]
+    // workspace A: x[N*3] | partial[nblocks*12] | ext[12] | (compact lists: xs[N*3] | inv[N]) | axis_images[N*3]
     const int nblocks = ceil_div(N, NBL_BLOCK);
     void* wsA = nullptr;
-    size_t bytesA = ((size_t)N * 3 * (co ? 2 : 1) + (size_t)nblocks * 12 + 16) * sizeof(T) + (co ? (size_t)N * sizeof(int) : 0);
+    const size_t axis_off = (((size_t)N * 3 * (co ? 2 : 1) + (size_t)nblocks * 12 + 16) * sizeof(T) + (co ? (size_t)N * sizeof(int) : 0) + 7) / 8 * 8;
+    size_t bytesA = axis_off + (N <= NBS_ATOMS ? (size_t)N * 3 * sizeof(unsigned) : 0);
     int rc = ws_get(WS_NBL_A, bytesA, &wsA);
     if (rc) return rc;
     T* x = (T*)wsA;
@@ -1649,6 +1682,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     T* ext_dev = partial + (size_t)nblocks * 12;
     T* xs = ext_dev + 16;                               // coordinates in processing order (compact lists)
     int* inv = (int*)(xs + (size_t)N * 3);              // ... and the inverse of the order
+    unsigned* axis_images = (unsigned*)((char*)wsA + axis_off);     // small_bins_kernel
     void* flags = nullptr;
     rc = ws_get(WS_FLAGS, 64, &flags);
     if (rc) return rc;
@@ -1775,7 +1809,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             hipLaunchKernelGGL(small_bins_kernel<T>, dim3(1), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x, gd, offsets,
                                (T*)wsC0, types, want_rows ? ilist : (int*)nullptr, types_out, incoming, co ? 1 : 0,
                                separable ? 1 : 0, cap[0], cap[1], cap[2], bound_of_coords, sync_free ? 1 : 0, status,
-                               posted ? post_slot : nullptr, post.seq);
+                               posted ? post_slot : nullptr, post.seq, axis_images);
             prof_end(stream);
             if (hipGetLastError() != hipSuccess) rc = A2P_ERR_HIP;
         }
