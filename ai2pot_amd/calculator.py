@@ -97,9 +97,11 @@ class NepCalculator:
             raise ValueError("path must be auto, gather or segments")
         if path == "gather" and not can_gather:
             raise ValueError("the gather path does not cover this model shape / list options")
-        # "auto": the gather kernels give every atom a thread and want tens of thousands of them; small
-        # systems stay with the lane-group kernel of the segment path
-        self.path = "gather" if (can_gather and (path == "gather" or (path == "auto" and self.n >= 32768))) else "segments"
+        # "auto": the gather kernels give every atom a thread and want tens of thousands of them; smaller systems take
+        # the segment path, whose kernel gives every atom a wavefront.  A step with rebuild, segments / gather:
+        # fp32 24,000 atoms 170 / 181 us, 32,000 202 / 188; fp64 16,384 203 / 234, 24,000 261 / 247
+        most = 28672 if f32 else 20480
+        self.path = "gather" if (can_gather and (path == "gather" or (path == "auto" and self.n >= most))) else "segments"
         self.padded = bool(padded) or self.path != "gather"
         self.input_order = int(reorder_every) == 0
         self.reorder_every = max(1, int(reorder_every))

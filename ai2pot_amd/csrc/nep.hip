@@ -439,6 +439,14 @@ int launch(const NepArgs<T>& a, size_t lds, hipStream_t stream)
     return A2P_OK;
 }
 
+// Atoms of a batch up to which a wavefront per atom beats the staged kernel's thread per atom, where both have the shape.
+// A wavefront per atom costs more instructions in all, but its chain is short and a few thousand atoms fill the chip; a
+// thread per atom takes the same time from one atom to as many as there are lanes.  Measured (6 radial, l_max 4, 60
+// neighbours; wavefront / staged, whole operator): fp32 8,000 atoms 69 / 166 us, 32,000 145 / 179, 45,000 188 / 193,
+// 64,000 244 / 218; fp64 8,000 98 / 227, 24,000 203 / 238, 32,000 257 / 242.
+template <typename T>
+constexpr long long wave_most() { return sizeof(T) == 4 ? 40960 : 28672; }
+
 template <typename T>
 int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coeffs, const T* w0,
             const T* b0, const T* w1, const T* bias, const T* q_scaler, double rr, double ra, int B,
@@ -490,10 +498,11 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     size_t lds_staged = 0;
     const bool staged = !(mb4 || mb5) && nep_staged_supported<T>(a, &lds_staged);
     if (staged) a.nblocks = nep_staged_nblocks(P);
-    size_t lds_group = 0;
-    // fewer staged workgroups than half the compute units: the system is small, spread it wider
-    const bool group = staged && (long long)B * nep_staged_nblocks(P) < 128 && nep_group_supported<T>(a, &lds_group);
-    if (group) a.nblocks = nep_group_nblocks(P);
+    // the wavefront-per-atom kernel: every shape it has in batches up to wave_most, beyond it those the staged kernel does
+    // not have
+    size_t lds_wave = 0;
+    const bool wave = !(mb4 || mb5) && ((long long)B * P < wave_most<T>() || !staged) && nep_wave_supported<T>(a, &lds_wave);
+    if (wave) a.nblocks = nep_wave_nblocks(P, B);
 
     void* ws = nullptr;
     int rc = ws_get(WS_FLAGS, 64, &ws);
@@ -506,8 +515,8 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     a.force = force;
     const size_t force_bytes = (size_t)B * (P + nghost) * 3 * sizeof(T);
 
-    if (group) {
-        return nep_group_run<T>(a, lds_group, etot, virial, stream);     // includes the energy / virial sums
+    if (wave) {
+        return nep_wave_run<T>(a, lds_wave, etot, virial, stream);       // includes the energy / virial sums
     } else if (staged) {
         return nep_staged_run<T>(a, lds_staged, etot, virial, stream);
     } else {

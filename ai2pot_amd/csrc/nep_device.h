@@ -214,15 +214,13 @@ __device__ __forceinline__ void blm_dir_derivs(T x, T y, T z, T wx, T wy, T wz, 
 // whether it applies; nep_staged_run() performs forces' zero-fill, pair counting, the kernel and
 // the pair reduction, whose launch also sums the workgroup partial sums of a.partial (a.nblocks
 // is set by staged_nblocks()) into etot and virial.
-// The same model shape with 8 lanes per atom (nep_group.hip): an atom's latency is an eighth of
-// the staged kernel's and a workgroup holds 32 atoms, which is what a small system needs to
-// occupy the device; per atom it executes more instructions, so large systems stay with the
-// staged kernel.
+// A wavefront per atom (nep_wave.hip), for systems too small to give every lane of the chip an atom; also l_max 3, and
+// any number of species whose tables fit the LDS.
 template <typename T>
-bool nep_group_supported(const nepdev::NepArgs<T>& a, size_t* lds_bytes);
-int nep_group_nblocks(int P);
+bool nep_wave_supported(const nepdev::NepArgs<T>& a, size_t* lds_bytes);
+int nep_wave_nblocks(int P, int B);
 template <typename T>
-int nep_group_run(const nepdev::NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream);
+int nep_wave_run(const nepdev::NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream);
 
 template <typename T>
 bool nep_staged_supported(const nepdev::NepArgs<T>& a, size_t* lds_bytes);

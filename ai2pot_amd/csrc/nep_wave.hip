@@ -1,0 +1,580 @@
+// NEP energy / force / virial, one wavefront per atom, for the common model shapes (chebyshev_size 8, n_radial 4 or 6,
+// n_angular 4, l_max 3 or 4) on lists in the padded layout, up to some tens of thousands of atoms.
+//
+// What bounds such systems is how much of an atom's work is a serial chain and how many chains are in flight: a thread
+// per atom leaves most of the chip empty, and eight lanes per atom still ran 6 neighbours one after the other and left
+// half of the compute units without a workgroup at 4096 atoms.  Here every step has its own division over the 64 lanes:
+//   * a row is read once, lane = slot, 128 slots at a time; pairs inside the angular cutoff are compacted to the front of
+//     the wavefront's tile in LDS, pairs between the cutoffs to its back (ballots); a pair claims its place in its
+//     target's reduction segment with one integer atomic (a2p::PairCsr);
+//   * radial functions and radial forces: lane = neighbour (47 of 64 lanes at the benchmark's density);
+//   * angular moments and forces: lane = (neighbour, angular channel), 16 neighbours at a time; a lane holds the 24
+//     moments of its channel, summed over the neighbours with four cross-lane additions;
+//   * hidden layer: lane = neuron, then lane = (descriptor, half of the neurons) for dE/dq.
+// About 1900 vector instructions per atom (6 radial, l_max 4, 48 + 12 neighbours), bound by their issue once every SIMD
+// holds two wavefronts and more.  The model's tables lie in LDS once per workgroup of four wavefronts, which walk through the structure's atoms with a stride.
+//
+// Measured, fp32, 6 radial functions, l_max 4, against eight lanes per atom (up to 8192 atoms) or a thread per atom:
+// 108 atoms 32 -> 16 us, 4096 39 -> 33, 20011 with skin lists 135 -> 92; of the first two some 10 us are the first fetch
+// of the code.  One loop for both passes over the pairs, which halves the code and keeps what the first pass computed, was
+// slower (39 and 109 us): it does not fit the 128 registers that four wavefronts per SIMD leave.  The lanes' virial sums
+// in LDS instead of registers: 37 and 117 us, one workgroup per compute unit fewer.
+//
+// Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
+#include "a2p_common.h"
+#include "nep_device.h"
+
+#include <type_traits>
+
+namespace a2p {
+using namespace nepdev;
+namespace {
+
+constexpr int NW_THREADS = 256, NW_WAVES = NW_THREADS / 64;
+constexpr int NW_CAP = 128;                  // slots of a row per tile
+constexpr int KC = 8, NAC = 4;
+constexpr int WROW = 28;                     // row of w0 in LDS: 16-byte reads by 8 lanes with consecutive rows touch
+                                             // each bank once
+constexpr int CPAD = 4;                      // values behind the coefficients of a species pair (bank spread)
+
+// ---- cross-lane sums -----------------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ int dpp_move(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) { return __int_as_float(dpp_move<CTRL>(__float_as_int(v))); }
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = dpp_move<CTRL>((int)(b & 0xffffffffll));
+    const int hi = dpp_move<CTRL>((int)(b >> 32));
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+// v[lane] + v[lane ^ 16] and v[lane] + v[lane ^ 32]: the swap of a value with its copy leaves one half's rows in the
+// first and the other half's in the second
+template <int ROWS>
+__device__ __forceinline__ void swap_rows(unsigned v, unsigned& a, unsigned& b)
+{
+    const auto r = ROWS == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
+                              : __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0]; b = r[1];
+}
+template <int ROWS>
+__device__ __forceinline__ float add_rows(float v)
+{
+    unsigned a, b;
+    swap_rows<ROWS>(__float_as_uint(v), a, b);
+    return __uint_as_float(a) + __uint_as_float(b);
+}
+template <int ROWS>
+__device__ __forceinline__ double add_rows(double v)
+{
+    const unsigned long long w = (unsigned long long)__double_as_longlong(v);
+    unsigned al, bl, ah, bh;
+    swap_rows<ROWS>((unsigned)w, al, bl);
+    swap_rows<ROWS>((unsigned)(w >> 32), ah, bh);
+    return __longlong_as_double((long long)((unsigned long long)ah << 32 | al)) +
+           __longlong_as_double((long long)((unsigned long long)bh << 32 | bl));
+}
+template <typename T>
+__device__ __forceinline__ T quad_sum(T v)          // the four lanes of a quad
+{
+    v += dpp_move<0xB1>(v);    // quad_perm [1,0,3,2]
+    v += dpp_move<0x4E>(v);    // quad_perm [2,3,0,1]
+    return v;
+}
+template <typename T>
+__device__ __forceinline__ T sum_over_quads(T v)    // the sixteen lanes with the same place in their quad
+{
+    v += dpp_move<0x124>(v);   // row_ror:4
+    v += dpp_move<0x128>(v);   // row_ror:8
+    v = add_rows<16>(v);
+    return add_rows<32>(v);
+}
+template <typename T>
+__device__ __forceinline__ T all_sum(T v) { return sum_over_quads(quad_sum(v)); }
+
+// ---- LDS -----------------------------------------------------------------------------------------
+__device__ __forceinline__ void lds_load4(const float* p, float (&o)[4])
+{
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    o[0] = v.x; o[1] = v.y; o[2] = v.z; o[3] = v.w;
+}
+__device__ __forceinline__ void lds_load4(const double* p, double (&o)[4])
+{
+    const double2 v0 = *reinterpret_cast<const double2*>(p);
+    const double2 v1 = *reinterpret_cast<const double2*>(p + 2);
+    o[0] = v0.x; o[1] = v0.y; o[2] = v1.x; o[3] = v1.y;
+}
+// tile entries: [x y z species]
+__device__ __forceinline__ void ent_store(float* p, float x, float y, float z, int w)
+{
+    *reinterpret_cast<float4*>(p) = make_float4(x, y, z, __int_as_float(w));
+}
+__device__ __forceinline__ void ent_load(const float* p, float& x, float& y, float& z, int& w)
+{
+    const float4 v = *reinterpret_cast<const float4*>(p);
+    x = v.x; y = v.y; z = v.z; w = __float_as_int(v.w);
+}
+__device__ __forceinline__ void ent_store(double* p, double x, double y, double z, int w)
+{
+    *reinterpret_cast<double2*>(p) = make_double2(x, y);
+    *reinterpret_cast<double2*>(p + 2) = make_double2(z, __longlong_as_double((long long)w));
+}
+__device__ __forceinline__ void ent_load(const double* p, double& x, double& y, double& z, int& w)
+{
+    const double2 v0 = *reinterpret_cast<const double2*>(p);
+    const double2 v1 = *reinterpret_cast<const double2*>(p + 2);
+    x = v0.x; y = v0.y; z = v1.x; w = (int)__double_as_longlong(v1.y);
+}
+
+template <typename T>
+struct WaveLds {
+    T *w0, *coef, *b0, *w1, *qs;     // model tables, shared by the workgroup
+    double* red;
+    T *ent, *ang, *q, *dq, *sde, *cc;       // of the wavefront: tile, angular forces of its front, read-out scratch
+    int* pos;
+};
+
+template <typename T>
+__host__ __device__ __forceinline__ size_t wave_lds_layout(int nt, int H, int nb, int wave, unsigned char* base,
+                                                           WaveLds<T>& L)
+{
+    size_t off = 0;
+    auto take = [&](size_t n, size_t size) {
+        unsigned char* p = base + off;
+        off += (n * size + 15) / 16 * 16;
+        return p;
+    };
+    L.w0 = (T*)take((size_t)nt * H * WROW, sizeof(T));
+    L.coef = (T*)take((size_t)nt * nt * (nb * KC + CPAD), sizeof(T));
+    L.b0 = (T*)take((size_t)nt * H, sizeof(T));
+    L.w1 = (T*)take((size_t)nt * H, sizeof(T));
+    L.qs = (T*)take(WROW, sizeof(T));
+    L.red = (double*)take(NW_WAVES * 10, sizeof(double));
+    const size_t shared = off;
+    L.ent = (T*)take(NW_CAP * 4, sizeof(T));
+    L.ang = (T*)take(NW_CAP * 3, sizeof(T));
+    L.pos = (int*)take(NW_CAP, sizeof(int));
+    L.q = (T*)take(WROW, sizeof(T));
+    L.dq = (T*)take(WROW, sizeof(T));
+    L.sde = (T*)take(H, sizeof(T));
+    L.cc = (T*)take(nt * KC, sizeof(T));
+    const size_t own = off - shared;
+    const size_t shift = own * wave;
+    L.ent = (T*)((unsigned char*)L.ent + shift); L.ang = (T*)((unsigned char*)L.ang + shift);
+    L.pos = (int*)((unsigned char*)L.pos + shift); L.q = (T*)((unsigned char*)L.q + shift);
+    L.dq = (T*)((unsigned char*)L.dq + shift); L.sde = (T*)((unsigned char*)L.sde + shift);
+    L.cc = (T*)((unsigned char*)L.cc + shift);
+    return shared + own * NW_WAVES;
+}
+
+struct SegArgs {
+    int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
+    int cap;       // capacity of a segment
+    int spare;     // entry that takes what overflows a segment
+};
+
+// Slots [128 t, 128 t + 128) of a row into the wavefront's tile; nA / nR: entries at its front / back.
+template <typename T>
+__device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& seg, T* __restrict__ seg_g,
+                                          const WaveLds<T>& L, int t, int lane, size_t row, int b, int NF, int nn, T rr,
+                                          T ra, bool claim, int& nA, int& nR)
+{
+    const int* types = a.btypes + (size_t)b * NF;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    nA = 0; nR = 0;
+    int nj[2], tj[2];
+    T x[2], y[2], z[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {                      // both halves of the tile in flight
+        const int slot = t * NW_CAP + h * 64 + lane;
+        nj[h] = -1;
+        x[h] = y[h] = z[h] = (T)0;
+        if (slot < nn) {
+            const size_t pr = row * a.U + slot;
+            nj[h] = a.bfirstneigh[pr];
+            const T* p = a.brcs + pr * 3;
+            x[h] = p[0]; y[h] = p[1]; z[h] = p[2];
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int slot = t * NW_CAP + h * 64 + lane;
+        const bool bad = slot < nn && (unsigned)nj[h] >= (unsigned)NF;
+        if (bad) atomicOr(a.status, ST_BAD_NEIGHBOR);
+        tj[h] = -1;
+        if (slot < nn && !bad) tj[h] = types[nj[h]];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (t * NW_CAP + h * 64 >= nn) break;          // uniform
+        const int slot = t * NW_CAP + h * 64 + lane;
+        const bool valid = slot < nn && (unsigned)nj[h] < (unsigned)NF;
+        if (valid && (unsigned)tj[h] >= (unsigned)a.ntypes) { atomicOr(a.status, ST_BAD_TYPE); tj[h] = 0; }
+        const T r = sqrt_t(x[h] * x[h] + y[h] * y[h] + z[h] * z[h]);
+        const bool inA = valid && r <= ra && r <= rr;   // nepBasis.h:106, 135: beyond the radial cutoff a neighbour is skipped
+        const bool inR = valid && !inA && r <= rr;
+        int pos = 0;
+        // A pair beyond the cutoffs (a list with a skin) needs no place in this call; when the places are kept with
+        // the list it has one all the same and stores a zero.
+        if (valid && claim && seg.cursor && (inA || inR || a.brank)) {
+            const size_t pr = row * a.U + slot;
+            const int tg = b * NF + nj[h];
+            int rk;
+            if (a.brank && a.ranks_valid) {
+                rk = a.brank[pr];
+            } else {
+                rk = atomicAdd(&seg.cursor[tg], 1);
+                if (a.brank) a.brank[pr] = rk;
+            }
+            pos = (unsigned)rk < (unsigned)seg.cap ? tg * seg.cap + rk : seg.spare;
+            if ((unsigned)rk >= (unsigned)seg.cap) atomicOr(a.status, ST_SEG_OVERFLOW);
+            if (!(inA || inR)) {
+                T* dst = seg_g + (size_t)pos * 3;
+                dst[0] = (T)0; dst[1] = (T)0; dst[2] = (T)0;
+            }
+        }
+        const unsigned long long mA = __ballot(inA), mR = __ballot(inR);
+        if (inA || inR) {
+            const int k = inA ? nA + __popcll(mA & lt) : NW_CAP - 1 - (nR + __popcll(mR & lt));
+            ent_store(L.ent + k * 4, x[h], y[h], z[h], tj[h]);
+            L.pos[k] = pos;
+        }
+        nA += __popcll(mA);
+        nR += __popcll(mR);
+    }
+    __builtin_amdgcn_wave_barrier();
+}
+
+template <typename T, int NR, int LC>
+__global__ void __launch_bounds__(NW_THREADS, sizeof(T) == 4 ? 4 : 2)
+nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
+{
+    constexpr int NLM = LC * LC + 2 * LC, NB = NR + NAC, D = NR + NAC * LC, CROW = NB * KC + CPAD;
+    static_assert(D <= WROW, "descriptor count exceeds the padded row");
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = blockIdx.y, H = a.H, nt = a.ntypes, NF = a.P + a.nghost;
+    WaveLds<T> L;
+    wave_lds_layout<T>(nt, H, NB, wave, smem_raw, L);
+
+    for (int i = tid; i < nt * H * WROW; i += NW_THREADS) {
+        const int r = i / WROW, j = i - r * WROW;
+        L.w0[i] = j < D ? a.w0[(size_t)r * D + j] : (T)0;
+    }
+    for (int i = tid; i < nt * nt * NB * KC; i += NW_THREADS) {
+        const int p = i / (NB * KC);
+        L.coef[p * CROW + (i - p * NB * KC)] = a.coeffs[i];
+    }
+    for (int i = tid; i < nt * H; i += NW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
+    if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / a.q_scaler[tid] : (T)0;
+    __syncthreads();
+
+    const int inum = a.binum[b];
+    const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
+    const bool derivs = a.force != nullptr || a.want_virial;
+    const int quad = lane >> 2, chan = lane & 3;       // neighbour within a round of 16, angular channel
+    double e_sum = 0.0, v_sum[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) v_sum[i] = 0.0;
+
+    for (int ii = blockIdx.x * NW_WAVES + wave; ii < inum; ii += gridDim.x * NW_WAVES) {
+        const size_t row = (size_t)b * a.P + ii;
+        int center = a.bilist[row], nn = a.bnumneigh[row];
+        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
+        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
+        int ti = a.btypes[(size_t)b * NF + center];
+        if ((unsigned)ti >= (unsigned)nt) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
+        const int ntiles = (nn + NW_CAP - 1) / NW_CAP;
+        const T* const cti = L.coef + (size_t)ti * nt * CROW;
+
+        // ---- radial sums, angular moments ------------------------------------------------------------
+        T S[NLM], q[NR];
+#pragma unroll
+        for (int m = 0; m < NLM; m++) S[m] = (T)0;
+#pragma unroll
+        for (int n = 0; n < NR; n++) q[n] = (T)0;
+        int nA = 0, nR = 0;
+        for (int t = 0; t < ntiles; t++) {
+            // (a row of several tiles is read again for the forces, and its pairs claim their places then)
+            load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, ntiles == 1, nA, nR);
+            for (int e = lane; e < nA + nR; e += 64) {
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + (e < nA ? e : NW_CAP - 1 - (e - nA)) * 4, x, y, z, tj);
+                T f[KC], df[KC];
+                radial_basis<T, KC, false>(sqrt_t(x * x + y * y + z * z), rr_inv, KC, f, df);
+                const T* c = cti + tj * CROW;
+#pragma unroll
+                for (int n = 0; n < NR; n++) {
+                    T c0[4], c1[4];
+                    lds_load4(c + n * KC, c0);
+                    lds_load4(c + n * KC + 4, c1);
+#pragma unroll
+                    for (int k = 0; k < 4; k++) q[n] += c0[k] * f[k];
+#pragma unroll
+                    for (int k = 0; k < 4; k++) q[n] += c1[k] * f[4 + k];
+                }
+            }
+            for (int e0 = 0; e0 < nA; e0 += 16) {
+                const int e = e0 + quad;
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                T f[KC], df[KC];
+                radial_basis<T, KC, false>(r, ra_inv, KC, f, df);
+                T c0[4], c1[4], g = (T)0;
+                lds_load4(cti + tj * CROW + (NR + chan) * KC, c0);
+                lds_load4(cti + tj * CROW + (NR + chan) * KC + 4, c1);
+#pragma unroll
+                for (int k = 0; k < 4; k++) g += c0[k] * f[k];
+#pragma unroll
+                for (int k = 0; k < 4; k++) g += c1[k] * f[4 + k];
+                if (e >= nA) g = (T)0;
+                T bl[NLM];
+                blm_values<T, LC>(x * rinv, y * rinv, z * rinv, bl);
+#pragma unroll
+                for (int m = 0; m < NLM; m++) S[m] += g * bl[m];
+            }
+            __builtin_amdgcn_wave_barrier();          // the tile is overwritten by the next one
+        }
+#pragma unroll
+        for (int n = 0; n < NR; n++) q[n] = all_sum(q[n]);
+#pragma unroll
+        for (int m = 0; m < NLM; m++) S[m] = sum_over_quads(S[m]);
+
+        // ---- descriptors: the radial ones in every lane, the angular ones of a channel in its lanes -----------
+#pragma unroll
+        for (int n = 0; n < NR; n++)
+            if (lane == n) L.q[n] = q[n];
+        // q_{n,l} = sum_m w_m C_lm S^2  (nepBasis.h:174-190)
+#pragma unroll
+        for (int l = 1; l <= LC; l++) {
+            T acc = (T)0;
+#pragma unroll
+            for (int mp = 0; mp < 2 * l + 1; mp++) {
+                const int m = l * l - 1 + mp;
+                acc += (T)(mp == 0 ? 1.0 : 2.0) * (T)kC3B[m] * S[m] * S[m];
+            }
+            if (lane < NAC) L.q[NR + chan * LC + (l - 1)] = acc;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (lane < D) {
+            const T v = L.q[lane];
+            if (a.desc) a.desc[row * D + lane] = v;
+            L.q[lane] = v * L.qs[lane];
+        } else if (lane < WROW) {
+            L.q[lane] = (T)0;
+        }
+        __builtin_amdgcn_wave_barrier();
+
+        // ---- hidden layer (nep.h:415-447): lane = neuron -------------------------------------------------
+        T e_site = (T)0;
+        for (int p = lane; p < H; p += 64) {
+            const T* wrow = L.w0 + (size_t)(ti * H + p) * WROW;
+            T h = L.b0[ti * H + p];
+#pragma unroll
+            for (int j = 0; j < D; j += 4) {
+                T w[4], v[4];
+                lds_load4(wrow + j, w);
+                lds_load4(L.q + j, v);
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    if (j + i < D) h += w[i] * v[i];
+            }
+            const T th = tanh_t(h), w1p = L.w1[ti * H + p];
+            e_site += w1p * th;
+            L.sde[p] = w1p * ((T)1 - th * th);
+        }
+        e_site = all_sum(e_site) + a.bias[ti];
+        e_sum += (double)e_site;
+        if (!derivs) { __builtin_amdgcn_wave_barrier(); continue; }
+        __builtin_amdgcn_wave_barrier();
+        {
+            // dE/dq: lane = (descriptor, half of the neurons); the halves meet in lanes 0 .. D-1
+            const int half = lane >> 5, d = lane & 31;
+            T acc = (T)0;
+            if (d < D) {
+                const T* col = L.w0 + (size_t)ti * H * WROW + d;
+                const int mid = (H + 1) / 2, p1 = half ? H : mid;
+#pragma unroll 5
+                for (int p = half ? mid : 0; p < p1; p++) acc += L.sde[p] * col[(size_t)p * WROW];
+            }
+            acc = add_rows<32>(acc);
+            if (lane < D) L.dq[lane] = acc * L.qs[lane];
+        }
+        __builtin_amdgcn_wave_barrier();
+
+        // ---- dE/dS (nep.h:450-466), overwriting S; radial coefficients contracted with dE/dq ---------------
+#pragma unroll
+        for (int l = 1; l <= LC; l++) {
+            const T dl = L.dq[NR + chan * LC + (l - 1)];
+#pragma unroll
+            for (int mp = 0; mp < 2 * l + 1; mp++) {
+                const int m = l * l - 1 + mp;
+                S[m] *= dl * (T)(mp == 0 ? 2.0 : 4.0) * (T)kC3B[m];
+            }
+        }
+        for (int i = lane; i < nt * KC; i += 64) {
+            const T* c = cti + (i >> 3) * CROW + (i & 7);
+            T v = (T)0;
+#pragma unroll
+            for (int n = 0; n < NR; n++) v += L.dq[n] * c[n * KC];
+            L.cc[i] = v;
+        }
+        __builtin_amdgcn_wave_barrier();
+
+        // ---- pair derivatives ------------------------------------------------------------------------------
+        T fx = (T)0, fy = (T)0, fz = (T)0, vir[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) vir[i] = (T)0;
+        for (int t = 0; t < ntiles; t++) {
+            if (ntiles > 1) load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, true, nA, nR);
+            for (int e0 = 0; e0 < nA; e0 += 16) {
+                const int e = e0 + quad;
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
+                T f[KC], df[KC];
+                radial_basis<T, KC, true>(r, ra_inv, KC, f, df);
+                T c0[4], c1[4], g = (T)0, dg = (T)0;
+                lds_load4(cti + tj * CROW + (NR + chan) * KC, c0);
+                lds_load4(cti + tj * CROW + (NR + chan) * KC + 4, c1);
+#pragma unroll
+                for (int k = 0; k < 4; k++) { g += c0[k] * f[k]; dg += c0[k] * df[k]; }
+#pragma unroll
+                for (int k = 0; k < 4; k++) { g += c1[k] * f[4 + k]; dg += c1[k] * df[4 + k]; }
+                T bl[NLM];
+                blm_values<T, LC>(ux, uy, uz, bl);
+                T srad = (T)0;
+#pragma unroll
+                for (int l = 1; l <= LC; l++) {
+                    T sl = (T)0;
+#pragma unroll
+                    for (int mp = 0; mp < 2 * l + 1; mp++) sl += S[l * l - 1 + mp] * bl[l * l - 1 + mp];
+                    srad += (dg - (T)l * rinv * g) * sl;
+                }
+                T wx = (T)0, wy = (T)0, wz = (T)0;
+                blm_grad_dot<T, LC>(ux, uy, uz, S, wx, wy, wz);
+                const T gr = g * rinv;
+                const T gx = quad_sum(srad * ux + wx * gr), gy = quad_sum(srad * uy + wy * gr),
+                        gz = quad_sum(srad * uz + wz * gr);
+                if (e < nA && chan == 0) { L.ang[e * 3] = gx; L.ang[e * 3 + 1] = gy; L.ang[e * 3 + 2] = gz; }
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int e = lane; e < nA + nR; e += 64) {
+                const int k = e < nA ? e : NW_CAP - 1 - (e - nA);
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + k * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z);
+                T f[KC], df[KC];
+                radial_basis<T, KC, true>(r, rr_inv, KC, f, df);
+                T c0[4], c1[4], sr = (T)0;
+                lds_load4(L.cc + tj * KC, c0);
+                lds_load4(L.cc + tj * KC + 4, c1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) sr += c0[i] * df[i];
+#pragma unroll
+                for (int i = 0; i < 4; i++) sr += c1[i] * df[4 + i];
+                sr /= r;
+                T gx = sr * x, gy = sr * y, gz = sr * z;
+                if (e < nA) { gx += L.ang[e * 3]; gy += L.ang[e * 3 + 1]; gz += L.ang[e * 3 + 2]; }
+                if (seg_g) {
+                    T* dst = seg_g + (size_t)L.pos[k] * 3;
+                    dst[0] = gx; dst[1] = gy; dst[2] = gz;
+                }
+                fx += gx; fy += gy; fz += gz;
+                vir[0] -= gx * x; vir[1] -= gx * y; vir[2] -= gx * z;
+                vir[3] -= gy * x; vir[4] -= gy * y; vir[5] -= gy * z;
+                vir[6] -= gz * x; vir[7] -= gz * y; vir[8] -= gz * z;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int i = 0; i < 9; i++) v_sum[i] += (double)vir[i];
+        if (a.force) {
+            fx = all_sum(fx); fy = all_sum(fy); fz = all_sum(fz);
+            if (lane < 3) a.force[((size_t)b * NF + center) * 3 + lane] = lane == 0 ? fx : lane == 1 ? fy : fz;
+        }
+    }
+
+    // ---- workgroup partial sums of energy and virial (fp64) ---------------------------------
+    if (lane == 0) L.red[wave * 10] = e_sum;
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        const double v = all_sum(v_sum[i]);
+        if (lane == 0) L.red[wave * 10 + 1 + i] = v;
+    }
+    __syncthreads();
+    if (tid < 10) {
+        double v = 0.0;
+        for (int w = 0; w < NW_WAVES; w++) v += L.red[w * 10 + tid];
+        a.partial[((size_t)b * a.nblocks + blockIdx.x) * 10 + tid] = v;
+    }
+}
+
+template <typename T, int NR, int LC>
+int launch_wave(const NepArgs<T>& a, size_t lds, const PairCsr& csr, hipStream_t stream)
+{
+    SegArgs seg{csr.cursor, csr.seg_cap, csr.n * csr.seg_cap};
+    auto kern = nep_wave_kernel<T, NR, LC>;
+    if (lds > 48 * 1024)
+        A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    prof_begin("nep_wave_kernel", stream);
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(NW_THREADS), lds, stream, a, seg, (T*)csr.seg_g);
+    prof_end(stream);
+    A2P_HIP_CHECK(hipGetLastError());
+    return A2P_OK;
+}
+
+}  // namespace
+
+// Workgroups per structure: an atom per wavefront until the batch has some 1024 workgroups (four per compute unit), from
+// there on several, so that the tables are staged once for all of them.
+int nep_wave_nblocks(int P, int B)
+{
+    return std::max(1, std::min(ceil_div(P, NW_WAVES), 1024 / std::max(B, 1)));
+}
+
+template <typename T>
+bool nep_wave_supported(const NepArgs<T>& a, size_t* lds_bytes)
+{
+    if (!(a.K == KC && (a.n_r == 4 || a.n_r == 6) && a.n_a == NAC && (a.l_max == 3 || a.l_max == 4))) return false;
+    WaveLds<T> unused;
+    *lds_bytes = wave_lds_layout<T>(a.ntypes, a.H, a.n_r + NAC, 0, nullptr, unused);
+    return *lds_bytes <= 150 * 1024;
+}
+
+template <typename T>
+int nep_wave_run(const NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream)
+{
+    PairCsr csr{};
+    int rc;
+    if (a.force) {
+        rc = pair_fixed_begin<T>(&csr, a.B, a.P, a.U, a.nghost, stream, a.force,
+                                 (size_t)a.B * (a.P + a.nghost) * 3 * sizeof(T), a.bincoming,
+                                 a.bincoming != nullptr && a.ranks_valid != 0);
+        if (rc) return rc;
+    }
+    if (a.n_r == 4) rc = a.l_max == 3 ? launch_wave<T, 4, 3>(a, lds_bytes, csr, stream) : launch_wave<T, 4, 4>(a, lds_bytes, csr, stream);
+    else rc = a.l_max == 3 ? launch_wave<T, 6, 3>(a, lds_bytes, csr, stream) : launch_wave<T, 6, 4>(a, lds_bytes, csr, stream);
+    if (rc) return rc;
+    if (a.force) return pair_csr_finish<T>(a.force, csr, stream, etot, virial, a.partial, a.B, a.nblocks);
+    return finish_energy_virial<T>(etot, virial, a.partial, a.B, a.nblocks, stream);
+}
+
+template bool nep_wave_supported<float>(const NepArgs<float>&, size_t*);
+template bool nep_wave_supported<double>(const NepArgs<double>&, size_t*);
+template int nep_wave_run<float>(const NepArgs<float>&, size_t, float*, float*, hipStream_t);
+template int nep_wave_run<double>(const NepArgs<double>&, size_t, double*, double*, hipStream_t);
+
+}  // namespace a2p
