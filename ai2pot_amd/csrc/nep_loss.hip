@@ -22,12 +22,14 @@
 //              Q_n(j) = (u.w) sum_lm tau Y_lm(j);  dPhi/dc[ti,tj,n_r+n,k] = sum_j fa_k(r_j) P_n(j) + fa'_k(r_j) Q_n(j)
 // with Ydot_lm = (1/r) (w . grad b_lm(u) - l b_lm(u) (u.w)).
 //
-// One workgroup of 128 threads per centre atom, neighbours in chunks of 32 with a per-neighbour
+// The common model shapes take nep_loss_wave.hip.  Any other: one workgroup of 128 threads per centre atom, neighbours in
+// chunks of 32 with a per-neighbour
 // table in LDS; every sum runs in a fixed order (no atomics).  Per-atom gradient rows (the
 // blocks of the centre's species only) are summed per structure in atom order by a second kernel.
 #include "a2p_common.h"
 #include "loss_kernels.h"
 #include "nep_device.h"
+#include "nep_loss.h"
 
 namespace a2p {
 using namespace nepdev;
@@ -37,22 +39,6 @@ constexpr int LNT = 128;     // threads per atom
 constexpr int LNC = 32;      // neighbours per chunk
 constexpr int LKMAX = 16;
 constexpr int LNLM = 24;
-
-template <typename T>
-struct NepLossArgs {
-    int K, n_r, n_a, l_max, H, ntypes, D;
-    const T *coeffs, *w0, *b0, *w1, *q_scaler;
-    T rr, ra;
-    int B, P, U;
-    const int *binum, *bilist, *bnumneigh, *bfirstneigh;
-    const T* brcs;
-    const int* btypes;
-    const T *cE, *dFs, *dVs;
-    T* gpart;          // [B, P, nrow]
-    int nrow;          // ntypes*(n_r+n_a)*K + H*D + 2H + 1
-    int E;             // table entries per neighbour
-    int* status;
-};
 
 template <typename T>
 struct LossLds {
@@ -85,8 +71,6 @@ __host__ __device__ inline size_t loss_lds_layout(const NepLossArgs<T>& a, unsig
     off += LNC * sizeof(int);
     return off;
 }
-
-__device__ __forceinline__ int l_of_lm(int m) { return m < 3 ? 1 : m < 8 ? 2 : m < 15 ? 3 : 4; }
 
 // Table of neighbours [c0, c0+nc): per neighbour  f[K] f'[K] (radial cutoff; zero outside) |
 // fa[K] fa'[K] (angular cutoff; zero outside) | Y[24] | Ydot[24] | u.w
@@ -427,7 +411,9 @@ int nep_loss(double e_w, double f_w, double v_w, const T* e_dft, const T* f_dft,
     a.B = B; a.P = P; a.U = U;
     a.binum = binum; a.bilist = bilist; a.bnumneigh = bnumneigh; a.bfirstneigh = bfirstneigh;
     a.brcs = brcs; a.btypes = btypes;
-    a.nrow = ntypes * (n_r + n_a) * K + H * a.D + 2 * H + 1;
+    size_t lds_wave = 0;
+    const bool wave = nep_loss_wave_supported<T>(a, &lds_wave);
+    a.nrow = wave ? nep_loss_wave_row<T>(a) : ntypes * (n_r + n_a) * K + H * a.D + 2 * H + 1;
     a.E = 4 * K + 2 * LNLM + 1;
     if ((a.E & 1) == 0) a.E++;
     const bool want_grad = dcoeffs || dw0 || db0 || dw1 || dbias;
@@ -453,6 +439,7 @@ int nep_loss(double e_w, double f_w, double v_w, const T* e_dft, const T* f_dft,
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
     a.cE = cE; a.dFs = dFs; a.dVs = dVs;
+    if (wave) return nep_loss_wave_run<T>(a, lds_wave, dcoeffs, dw0, db0, dw1, dbias, stream);
     LossLds<T> unused;
     const size_t lds = loss_lds_layout<T>(a, nullptr, unused);
     A2P_REQUIRE(lds <= 150 * 1024, A2P_ERR_INVALID, "nep loss: model too large for LDS (%zu bytes)", lds);

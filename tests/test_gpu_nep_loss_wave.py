@@ -1,0 +1,48 @@
+"""The wavefront-per-atom gradient kernel of the NEP loss at the edges of its tiles (64 slots of a row, 32 pairs inside the
+angular cutoff, 16 columns of a matrix instruction), against the kernel for any shape: the same model with one more basis
+function, whose coefficients are zero, takes that kernel and has the same gradients in its other entries."""
+import numpy as np
+import pytest
+
+from ai2pot_amd import synth
+from test_gpu_nep_loss import GRADS, close, gpu_loss
+
+pytestmark = pytest.mark.gpu
+ROWS = [0, 1, 16, 17, 63, 64, 65, 129, 200]
+INNER = [0, 1, 15, 16, 17, 32, 33, 64, 65]
+
+
+@pytest.mark.parametrize("np_dtype,n_r,l_max,ntypes,H", [(np.float64, 6, 4, 3, 50), (np.float64, 4, 3, 1, 30),
+                                                         (np.float64, 6, 3, 5, 65), (np.float32, 6, 4, 3, 50),
+                                                         (np.float32, 4, 3, 2, 30), (np.float32, 4, 4, 17, 4)])
+def test_tile_edges(np_dtype, n_r, l_max, ntypes, H):
+    rng = np.random.default_rng(7)
+    P, U = len(ROWS) * len(INNER), 200
+    rows = np.repeat(ROWS, len(INNER))
+    nb = dict(binum=np.array([P, P - 5, 1], np.int32), bilist=np.tile(rng.permutation(P), (3, 1)).astype(np.int32),
+              bnumneigh=np.tile(rows, (3, 1)).astype(np.int32),
+              bfirstneigh=rng.integers(0, P, (3, P, U)).astype(np.int32), brcs=np.zeros((3, P, U, 3), np_dtype),
+              btypes=rng.integers(0, ntypes, (3, P)).astype(np.int32), nghost=0)
+    u = rng.normal(size=(3, P, U, 3))
+    # the first slots of a row, in random order, are inside the angular cutoff of 4, as many as its quota; the last of the
+    # others lie beyond the radial one
+    place = np.stack([[np.concatenate([rng.permutation(n), np.arange(n, U)]) for n in rows] for _ in range(3)])
+    inner = place < np.tile(INNER, len(ROWS))[None, :, None]
+    r = np.where(inner, rng.uniform(2.0, 3.99, inner.shape), rng.uniform(4.01, 7.4, inner.shape))
+    nb["brcs"][:] = u * (r / np.linalg.norm(u, axis=3))[..., None]
+
+    m = synth.nep_model(ntypes=ntypes, n_radial_basis=n_r, l_max=l_max, num_neurons=H, sigma=0.12)
+    m["type_map"] = np.arange(1, ntypes + 1, dtype=np.int32)
+    m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    wide = dict(m, chebyshev_size=9)
+    c = m["coeffs"].reshape(-1, 8)
+    wide["coeffs"] = np.concatenate([c, np.zeros((len(c), 1))], axis=1).ravel()
+    labels = dict(energy=rng.normal(-5.0, 2.0, 3), force=rng.normal(size=(3, P, 3)), virial=rng.normal(size=(3, 9)))
+    got = gpu_loss(m, nb, labels, (0.9, 1.3, 0.4), np_dtype)
+    want = gpu_loss(wide, nb, labels, (0.9, 1.3, 0.4), np_dtype)
+    want["dcoeffs"] = want["dcoeffs"].reshape(3, -1, 9)[..., :8].reshape(3, -1)
+    # both kernels add some 80 rows of up to 200 terms, in different orders: at most 300 roundings of the largest partial
+    # sum, itself a few times the result
+    tol = 1e-12 if np_dtype == np.float64 else 300 * 2.0**-24 * 4
+    for k in GRADS:
+        assert close(got[k], want[k], tol), (k, np.abs(got[k] - want[k]).max() / np.abs(want[k]).max())
