@@ -334,7 +334,7 @@ struct BasisFunction : public torch::autograd::Function<BasisFunction> {
     }
 };
 
-// X^T X [n, n] and X^T y [n] of a tall matrix X [N, n]: the rows are cut into up to 64 blocks whose products run
+// (More columns than a2p_normal_equations_* takes.)  X^T X [n, n] and X^T y [n] of a tall matrix X [N, n]: the rows are cut into up to 64 blocks whose products run
 // as one batched GEMM and are added afterwards (a single GEMM with n of about a hundred and N in the tens of
 // thousands occupies one tile of the chip: 0.66 ms against 0.03 ms for 24576 x 95 in fp64)
 std::pair<at::Tensor, at::Tensor> gram(const at::Tensor& X, const at::Tensor& y)
@@ -350,7 +350,7 @@ std::pair<at::Tensor, at::Tensor> gram(const at::Tensor& X, const at::Tensor& y)
 }
 
 // normal equations of the linear parameters (linear_mtp_gram_and_cross.h:446-575): components by the
-// library, Gram products by torch's BLAS
+// library, Gram products by a2p_normal_equations_*, or by torch's BLAS for wide systems
 variable_list lin_matrix_lin_vector(double e_w, double f_w, double v_w, const at::Tensor& e_dft,
                                     const at::Tensor& f_dft, const at::Tensor& v_dft, int64_t K, double scaling,
                                     const at::Tensor& coeffs, int64_t n_moms, const at::Tensor& basic,
@@ -363,7 +363,7 @@ variable_list lin_matrix_lin_vector(double e_w, double f_w, double v_w, const at
     TORCH_CHECK(nghost == 0, "LinMatrixLinVectorOp requires nghost == 0: the reference's force components have "
                              "natoms_pad rows");
     auto opt = brcs.options();
-    at::Tensor lin0 = at::zeros({mapping.numel()}, opt), bias0 = at::zeros({type_map.numel()}, opt);
+    at::Tensor lin0 = at::empty({mapping.numel()}, opt), bias0 = at::empty({type_map.numel()}, opt);      // not read
     MtpCtx c = check_mtp(K, coeffs, lin0, bias0, n_moms, basic, times, mapping, nmus, binum, bilist, bnumneigh,
                          bfirstneigh, brcs, btypes, type_map, nghost, q_scaler);
     check_device_float(brcs, e_dft, "betot_dft");
@@ -395,6 +395,24 @@ variable_list lin_matrix_lin_vector(double e_w, double f_w, double v_w, const at
         return rc;
     };
     run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
+    if (n <= 575) {
+        // (wider systems keep a matrix product busy by themselves)
+        at::Tensor A = at::empty({n, n}, opt), b = at::empty({n}, opt);
+        const long long rows[3] = {B, (long long)B * P * 3, (long long)B * 9};
+        const double w[3] = {e_w, f_w, v_w};
+        int rc;
+        if (brcs.scalar_type() == at::kDouble) {
+            const double* X[3] = {ec.data_ptr<double>(), fc.data_ptr<double>(), vc.data_ptr<double>()};
+            const double* y[3] = {e_dft.data_ptr<double>(), f_dft.data_ptr<double>(), v_dft.data_ptr<double>()};
+            rc = a2p_normal_equations_f64((int)n, rows, w, X, y, A.data_ptr<double>(), b.data_ptr<double>(), st);
+        } else {
+            const float* X[3] = {ec.data_ptr<float>(), fc.data_ptr<float>(), vc.data_ptr<float>()};
+            const float* y[3] = {e_dft.data_ptr<float>(), f_dft.data_ptr<float>(), v_dft.data_ptr<float>()};
+            rc = a2p_normal_equations_f32((int)n, rows, w, X, y, A.data_ptr<float>(), b.data_ptr<float>(), st);
+        }
+        check_rc(rc);
+        return {A, b};
+    }
     auto ge = gram(ec, e_dft.reshape({B})), gf = gram(fc, f_dft.reshape({-1})), gv = gram(vc, v_dft.reshape({-1}));
     at::Tensor A = e_w * ge.first + f_w * gf.first + v_w * gv.first;
     at::Tensor b = e_w * ge.second + f_w * gf.second + v_w * gv.second;

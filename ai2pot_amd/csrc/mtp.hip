@@ -1100,11 +1100,13 @@ comp_rows_kernel(int B, int P, int U, int ntypes, const int* __restrict__ binum,
     nnc[row] = nn;
 }
 
-// the pairs that name each atom: counted, then listed (comp_incoming_fill), then put in order (comp_incoming_sort)
+// The pairs that name each atom.  Each atom has room for `cap` of them (the row length of the list: enough for every list
+// built with one cutoff), so one pass lists them; when an atom is named more often (spill[0] counts what found no room)
+// the pass is repeated for counts only and then into segments of the right lengths (seg).
 __global__ void __launch_bounds__(256)
 comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int* __restrict__ pair_off,
-                     const int* __restrict__ bfirstneigh, int* __restrict__ cnt, const int* __restrict__ ioff,
-                     int* __restrict__ inc)
+                     const int* __restrict__ bfirstneigh, int* __restrict__ cnt, const int* __restrict__ seg, int cap,
+                     int* __restrict__ inc, int* __restrict__ spill)
 {
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
     if (q >= (long long)B * P * U) return;
@@ -1114,74 +1116,123 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
     if ((unsigned)nj >= (unsigned)P) return;             // flagged by the components kernel's table
     const int tg = (row / P) * P + nj;
     const int place = atomicAdd(cnt + tg, 1);
-    if (inc) inc[ioff[tg] + place] = pair_off[row] + j;
+    if (!inc) return;
+    if (seg) inc[seg[tg] + place] = pair_off[row] + j;
+    else if (place < cap) inc[(size_t)tg * cap + place] = pair_off[row] + j;
+    else atomicAdd(spill, 1);
 }
 
-__global__ void __launch_bounds__(256)
-comp_incoming_sort_kernel(int n, const int* __restrict__ ioff, int* __restrict__ inc)
-{
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t >= n) return;
-    int* v = inc + ioff[t];
-    const int m = ioff[t + 1] - ioff[t];
-    for (int i = 1; i < m; i++) {
-        const int x = v[i];
-        int k = i - 1;
-        while (k >= 0 && v[k] > x) { v[k + 1] = v[k]; k--; }
-        v[k + 1] = x;
-    }
-}
+// Force column of every atom: its own row's sum minus the pairs that name it, in the order of their numbers.  The pairs
+// arrive in any order: a workgroup (one wavefront) ranks those of its atom in LDS, up to COMP_SORT of them; a longer list
+// is walked from each number to the next larger one.  Columns from S on (species counts) are zero.
+// Bound by the reads of the pair derivatives; sorting the lists by insertion, one thread per atom, used to take as long as
+// they do (95 us beside 98 us at 64 structures of 128 atoms).
+constexpr int COMP_SORT = 256;
 
-// force column of every atom: its own row's sum minus the pairs that name it, in the order of the sorted list
 template <typename T>
 __global__ void __launch_bounds__(64)
-comp_force_kernel(int S, int n, const int* __restrict__ row_of1, const int* __restrict__ ioff,
-                  const int* __restrict__ inc, const T* __restrict__ pb, const T* __restrict__ rowpart,
-                  T* __restrict__ fcomp)
+comp_force_kernel(int S, int n, int cap, const int* __restrict__ row_of1, const int* __restrict__ cnt,
+                  const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ pb,
+                  const T* __restrict__ rowpart, T* __restrict__ fcomp)
 {
-    const int t = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x;
-    if (s >= S) return;
-    T f[3] = {(T)0, (T)0, (T)0};
+    __shared__ int list[COMP_SORT], order[COMP_SORT];
+    const int t = blockIdx.x, lane = threadIdx.x, col = blockIdx.y * 64 + lane, s = min(col, S - 1);
+    const int* v = inc + (seg ? (size_t)seg[t] : (size_t)t * cap);
+    const int m = seg ? seg[t + 1] - seg[t] : min(cnt[t], cap);
     const int r1 = row_of1[t];
+    const bool ranked = m <= COMP_SORT;
+    if (ranked) {
+        for (int k = lane; k < m; k += 64) list[k] = v[k];
+        __syncthreads();
+        for (int k = lane; k < m; k += 64) {
+            const int x = list[k];
+            int r = 0;
+            for (int i = 0; i < m; i++) r += list[i] < x;
+            order[r] = x;
+        }
+        __syncthreads();
+    }
+    T f[3] = {(T)0, (T)0, (T)0};
     if (r1 > 0) {
         const T* o = rowpart + (size_t)(r1 - 1) * 12 * S + s;
 #pragma unroll
         for (int i = 0; i < 3; i++) f[i] = o[(size_t)i * S];
     }
-    for (int k = ioff[t]; k < ioff[t + 1]; k++) {
-        const T* g = pb + (size_t)inc[k] * 3 * S + s;
-        f[0] -= g[0]; f[1] -= g[S]; f[2] -= g[2 * S];
-    }
+    if (ranked) {
+        for (int k0 = 0; k0 < m; k0 += 4) {              // twelve loads in flight
+            T g[4][3];
 #pragma unroll
-    for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + s] = f[i];
+            for (int u = 0; u < 4; u++) {
+                const T* src = pb + (size_t)order[min(k0 + u, m - 1)] * 3 * S + s;
+#pragma unroll
+                for (int i = 0; i < 3; i++) g[u][i] = src[(size_t)i * S];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (k0 + u < m)
+#pragma unroll
+                    for (int i = 0; i < 3; i++) f[i] -= g[u][i];
+        }
+    } else {
+        int last = -1;
+        for (int k = 0; k < m; k++) {
+            int next = 0x7fffffff;
+            for (int i = lane; i < m; i += 64) {
+                const int x = v[i];
+                if (x > last && x < next) next = x;
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) next = min(next, __shfl_xor(next, off, 64));
+            last = next;
+            const T* g = pb + (size_t)next * 3 * S + s;
+#pragma unroll
+            for (int i = 0; i < 3; i++) f[i] -= g[(size_t)i * S];
+        }
+    }
+    if (col < n)
+#pragma unroll
+        for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + col] = col < S ? f[i] : (T)0;
 }
 
-// energy and virial columns per structure: sums over the rows in row order, in two steps (blocks of COMP_ROWS rows,
-// then the blocks); part[B][nblocks][10][S]
-constexpr int COMP_ROWS = 32;
+// Energy and virial columns per structure: sums over the rows in row order, in two steps (blocks of COMP_ROWS rows, then
+// the blocks); part[B][nblocks][10][n].  Column S + t counts the rows whose centre has species t; its virial is zero.
+// The first step reads 80 bytes per row and column: short blocks (8 rows: 25 -> 8 us against 32 at 64 x 128 rows) keep
+// enough wavefronts in flight.
+constexpr int COMP_ROWS = 8;
 
 template <typename T>
 __global__ void __launch_bounds__(64)
-comp_structure_blocks_kernel(int S, int P, int nblocks, const int* __restrict__ binum, const T* __restrict__ desc,
+comp_structure_blocks_kernel(int S, int n, int P, int nblocks, const int* __restrict__ binum,
+                             const int* __restrict__ bilist, const int* __restrict__ btypes, const T* __restrict__ desc,
                              const T* __restrict__ rowpart, T* __restrict__ part)
 {
     const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x, blk = blockIdx.z;
-    if (s >= S) return;
+    if (s >= n) return;
     T e = (T)0, v[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) v[i] = (T)0;
-    const int i1 = min(binum[b], (blk + 1) * COMP_ROWS);
-    for (int ii = blk * COMP_ROWS; ii < i1; ii++) {
-        const size_t row = (size_t)b * P + ii;
-        e += desc[row * S + s];
-        const T* o = rowpart + row * 12 * S + s;
+    const int i0 = blk * COMP_ROWS, i1 = min(binum[b], i0 + COMP_ROWS);
+    if (s < S) {
+#pragma unroll 4
+        for (int ii = i0; ii < i1; ii++) {
+            const size_t row = (size_t)b * P + ii;
+            e += desc[row * S + s];
+            const T* o = rowpart + row * 12 * S + s;
 #pragma unroll
-        for (int i = 0; i < 9; i++) v[i] += o[(size_t)(3 + i) * S];
+            for (int i = 0; i < 9; i++) v[i] += o[(size_t)(3 + i) * S];
+        }
+    } else {
+        int c[COMP_ROWS];
+#pragma unroll
+        for (int u = 0; u < COMP_ROWS; u++) c[u] = i0 + u < i1 ? bilist[(size_t)b * P + i0 + u] : -1;
+#pragma unroll
+        for (int u = 0; u < COMP_ROWS; u++)
+            if ((unsigned)c[u] < (unsigned)P && btypes[(size_t)b * P + c[u]] == s - S) e += (T)1;
     }
-    T* o = part + ((size_t)b * nblocks + blk) * 10 * S + s;
+    T* o = part + ((size_t)b * nblocks + blk) * 10 * n + s;
     o[0] = e;
 #pragma unroll
-    for (int i = 0; i < 9; i++) o[(size_t)(1 + i) * S] = v[i];
+    for (int i = 0; i < 9; i++) o[(size_t)(1 + i) * n] = v[i];
 }
 
 template <typename T>
@@ -1190,16 +1241,16 @@ comp_structure_kernel(int n, int S, int nblocks, const T* __restrict__ q_scaler,
                       T* __restrict__ ecomp, T* __restrict__ vcomp)
 {
     const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x;
-    if (s >= S) return;
+    if (s >= n) return;
     T acc[10];
 #pragma unroll
     for (int i = 0; i < 10; i++) acc[i] = (T)0;
     for (int blk = 0; blk < nblocks; blk++) {
-        const T* o = part + ((size_t)b * nblocks + blk) * 10 * S + s;
+        const T* o = part + ((size_t)b * nblocks + blk) * 10 * n + s;
 #pragma unroll
-        for (int i = 0; i < 10; i++) acc[i] += o[(size_t)i * S];
+        for (int i = 0; i < 10; i++) acc[i] += o[(size_t)i * n];
     }
-    ecomp[(size_t)b * n + s] = acc[0] / q_scaler[s];
+    ecomp[(size_t)b * n + s] = s < S ? acc[0] / q_scaler[s] : acc[0];
 #pragma unroll
     for (int i = 0; i < 9; i++) vcomp[((size_t)b * 9 + i) * n + s] = acc[1 + i];
 }
@@ -2101,18 +2152,24 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
 {
     const int B = a.B, P = a.P, U = a.U;
     const int rows = B * P;
-    // integer scratch: nnc[rows+1] | pair_off[rows+1] | cnt[rows+1] | ioff[rows+1] | row_of1[rows] | scan tmp
+    // integer scratch: nnc[rows+1] | pair_off[rows+1] | spill | cnt[rows+1] | row_of1[rows] | seg[rows+1] | scan tmp
     const int ntmp = scan_tmp_ints(rows + 1);
     void* wsI = nullptr;
-    int rc = ws_get(WS_CSR, ((size_t)(rows + 1) * 4 + rows + ntmp) * sizeof(int), &wsI);
+    int rc = ws_get(WS_CSR, ((size_t)(rows + 1) * 4 + 1 + rows + ntmp) * sizeof(int), &wsI);
     if (rc) return rc;
     int* nnc = (int*)wsI;
     int* pair_off = nnc + rows + 1;
-    int* cnt = pair_off + rows + 1;
-    int* ioff = cnt + rows + 1;
-    int* row_of1 = ioff + rows + 1;
-    int* tmp = row_of1 + rows;
-    rc = fill_zero2(cnt, (size_t)(rows + 1) * sizeof(int), row_of1, (size_t)rows * sizeof(int), stream);
+    int* spill = pair_off + rows + 1;        // (behind the number of pairs: read back together)
+    int* cnt = spill + 1;
+    int* row_of1 = cnt + rows + 1;
+    int* seg = row_of1 + rows;
+    int* tmp = seg + rows + 1;
+    // the list of the pairs that name each atom has a place of its own: it is filled before the number of pairs is known
+    void* wsL = nullptr;
+    rc = ws_get(WS_NBL_A, (size_t)rows * U * sizeof(int), &wsL);
+    if (rc) return rc;
+    int* inc = (int*)wsL;
+    rc = fill_zero(spill, (size_t)(2 * rows + 2) * sizeof(int), stream);       // spill, cnt, row_of1
     if (rc) return rc;
     prof_begin("mtp_components_lists", stream);
     hipLaunchKernelGGL(comp_rows_kernel, dim3(ceil_div(rows + 1, 256)), dim3(256), 0, stream, B, P, U, a.ntypes, a.binum,
@@ -2120,34 +2177,38 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
     prof_end(stream);
     rc = exclusive_scan_i32(nnc, pair_off, rows + 1, tmp, stream);
     if (rc) return rc;
-    int npairs = 0;                         // sizes the pair buffer: one read-back per call
-    rc = read_back(pair_off + rows, 1, &npairs, stream);
+    const long long nslots = (long long)rows * U;
+    prof_begin("mtp_components_lists", stream);
+    hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U, (const int*)nnc,
+                       (const int*)pair_off, a.bfirstneigh, cnt, (const int*)nullptr, U, inc, spill);
+    prof_end(stream);
+    int found[2] = {0, 0};                  // the first sizes the pair buffer: one read-back per call
+    rc = read_back(pair_off + rows, 2, found, stream);
     if (rc) return rc;
-    if (npairs < 0) npairs = 0;
-    // pair derivatives | row sums | scalar moments | list of the pairs that name each atom
+    A2P_HIP_CHECK(hipGetLastError());
+    const int npairs = std::max(found[0], 0);
+    const int* in_seg = nullptr;
+    if (found[1] > 0) {                     // an atom is named by more pairs than a row has room for
+        rc = exclusive_scan_i32(cnt, seg, rows + 1, tmp, stream);
+        if (rc) return rc;
+        rc = fill_zero(cnt, (size_t)(rows + 1) * sizeof(int), stream);
+        if (rc) return rc;
+        rc = ws_get(WS_NBL_A, (size_t)std::max(npairs, 1) * sizeof(int), &wsL);
+        if (rc) return rc;
+        inc = (int*)wsL;
+        hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U,
+                           (const int*)nnc, (const int*)pair_off, a.bfirstneigh, cnt, (const int*)seg, U, inc, spill);
+        A2P_HIP_CHECK(hipGetLastError());
+        in_seg = seg;
+    }
+    // pair derivatives | row sums | scalar moments
     const size_t n_pb = (size_t)std::max(npairs, 1) * 3 * S, n_rp = (size_t)rows * 12 * S, n_desc = (size_t)rows * S;
     void* wsT = nullptr;
-    rc = ws_get(WS_MTP, (n_pb + n_rp + n_desc) * sizeof(T) + ((size_t)npairs + 1) * sizeof(int), &wsT);
+    rc = ws_get(WS_MTP, (n_pb + n_rp + n_desc) * sizeof(T), &wsT);
     if (rc) return rc;
     T* pb = (T*)wsT;
     T* rowpart = pb + n_pb;
     T* desc = rowpart + n_rp;
-    int* inc = (int*)(desc + n_desc);
-    const long long nslots = (long long)rows * U;
-    prof_begin("mtp_components_lists", stream);
-    hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U, (const int*)nnc,
-                       (const int*)pair_off, a.bfirstneigh, cnt, (const int*)nullptr, (int*)nullptr);
-    prof_end(stream);
-    rc = exclusive_scan_i32(cnt, ioff, rows + 1, tmp, stream);
-    if (rc) return rc;
-    rc = fill_zero(cnt, (size_t)(rows + 1) * sizeof(int), stream);
-    if (rc) return rc;
-    prof_begin("mtp_components_lists", stream);
-    hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U, (const int*)nnc,
-                       (const int*)pair_off, a.bfirstneigh, cnt, (const int*)ioff, inc);
-    hipLaunchKernelGGL(comp_incoming_sort_kernel, dim3(ceil_div(rows, 256)), dim3(256), 0, stream, rows, (const int*)ioff,
-                       inc);
-    prof_end(stream);
 
     CompArgs<T> c;
     c.pb = pb; c.pair_off = pair_off; c.nnc = nnc; c.desc = desc; c.rowpart = rowpart;
@@ -2183,15 +2244,15 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         prof_end(stream);
     }
     prof_begin("mtp_components_sums", stream);
-    hipLaunchKernelGGL(comp_force_kernel<T>, dim3(rows, ceil_div(S, 64)), dim3(64), 0, stream, S, n, (const int*)row_of1,
-                       (const int*)ioff, (const int*)inc, (const T*)pb, (const T*)rowpart, fcomp);
+    hipLaunchKernelGGL(comp_force_kernel<T>, dim3(rows, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, (const int*)row_of1,
+                       (const int*)cnt, in_seg, (const int*)inc, (const T*)pb, (const T*)rowpart, fcomp);
     const int nblocks = ceil_div(P, COMP_ROWS);
     void* wsP = nullptr;
-    rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * S * sizeof(T), &wsP);
+    rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * n * sizeof(T), &wsP);
     if (rc) return rc;
-    hipLaunchKernelGGL(comp_structure_blocks_kernel<T>, dim3(B, ceil_div(S, 64), nblocks), dim3(64), 0, stream, S, P,
-                       nblocks, a.binum, (const T*)desc, (const T*)rowpart, (T*)wsP);
-    hipLaunchKernelGGL(comp_structure_kernel<T>, dim3(B, ceil_div(S, 64)), dim3(64), 0, stream, n, S, nblocks, a.q_scaler,
+    hipLaunchKernelGGL(comp_structure_blocks_kernel<T>, dim3(B, ceil_div(n, 64), nblocks), dim3(64), 0, stream, S, n, P,
+                       nblocks, a.binum, a.bilist, a.btypes, (const T*)desc, (const T*)rowpart, (T*)wsP);
+    hipLaunchKernelGGL(comp_structure_kernel<T>, dim3(B, ceil_div(n, 64)), dim3(64), 0, stream, n, S, nblocks, a.q_scaler,
                        (const T*)wsP, ecomp, vcomp);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
@@ -2217,6 +2278,15 @@ int mtp_lin_components(void* handle, int K, double scaling, const T* coeffs, int
     A2P_REQUIRE(ntypes >= 1 && B >= 0 && P >= 0, A2P_ERR_INVALID, "mtp components: bad shape");
     const int S = plan->d.n_scalar, n = S + ntypes;
     if (B == 0 || P == 0) return A2P_OK;
+    if (components_route() == 1 && !plan->xbatches.empty()) {
+        MtpArgs<T> a;
+        rc = fill_args(a, plan, K, scaling, coeffs, (const T*)nullptr, (const T*)nullptr, nmus, ntypes, q_scaler, rmax,
+                       rmin, B, P, U, 0, binum, bilist, bnumneigh, bfirstneigh, brcs, btypes, false);
+        if (rc) return rc;
+        A2P_REQUIRE(q_scaler, A2P_ERR_INVALID, "mtp components: null q_scaler");
+        a.E = table_entries<T>(a.p, K, false);
+        return mtp_lin_components_nodes<T>(plan, a, S, n, ecomp, fcomp, vcomp, stream);
+    }
     rc = fill_zero(ecomp, (size_t)B * n * sizeof(T), stream);
     if (rc) return rc;
     rc = fill_zero(fcomp, (size_t)B * P * 3 * n * sizeof(T), stream);
@@ -2233,18 +2303,6 @@ int mtp_lin_components(void* handle, int K, double scaling, const T* coeffs, int
     hipLaunchKernelGGL(species_count_kernel, dim3(ceil_div(B * P, 256)), dim3(256), 0, stream, B, P, ntypes, binum, bilist,
                        btypes, counts);
     A2P_HIP_CHECK(hipGetLastError());
-    if (components_route() == 1 && !plan->xbatches.empty()) {
-        MtpArgs<T> a;
-        rc = fill_args(a, plan, K, scaling, coeffs, (const T*)nullptr, (const T*)nullptr, nmus, ntypes, q_scaler, rmax,
-                       rmin, B, P, U, 0, binum, bilist, bnumneigh, bfirstneigh, brcs, btypes, false);
-        if (rc) return rc;
-        A2P_REQUIRE(q_scaler, A2P_ERR_INVALID, "mtp components: null q_scaler");
-        a.E = table_entries<T>(a.p, K, false);
-        hipLaunchKernelGGL(lin_components_init_kernel<T>, dim3(ceil_div(B * ntypes, 256)), dim3(256), 0, stream,
-                           (T*)nullptr, S, ecomp, B, ntypes, (const int*)counts);
-        A2P_HIP_CHECK(hipGetLastError());
-        return mtp_lin_components_nodes<T>(plan, a, S, n, ecomp, fcomp, vcomp, stream);
-    }
     // one E/F/V pass per scalar moment with a one-hot read-out
     // workspace: eye[S*S] | zero bias[ntypes] | etot[B] | force[B*P*3] | virial[B*9]
     const size_t nT = (size_t)S * S + ntypes + B + (size_t)B * P * 3 + (size_t)B * 9;

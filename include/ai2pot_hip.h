@@ -532,7 +532,10 @@ int a2p_zbl_esites_f32(double zbl_rmax, double zbl_rmin, const float* zbl_cks, c
  * moment s over q_scaler[s]; column n_scalar + t: the species count in the energy, zero elsewhere).
  * The normal equations of the reference,
  *   lin_matrix = sum_b e_w E_b^T E_b + f_w F_b^T F_b + v_w V_b^T V_b,   lin_vector = the same against the residuals,
- * are plain GEMMs over these arrays and are left to the caller's BLAS (the bind library uses torch's).
+ * are a2p_normal_equations_* over these arrays: A = sum_k w_k X_k^T X_k [n, n] and b = sum_k w_k X_k^T y_k [n] for three
+ * row-major matrices X_k[rows_k, n] with y_k[rows_k] (rows, weights, X and y are HOST arrays of three, X_k and y_k device
+ * pointers), sums in the precision of X inside blocks of rows and in double over the blocks; n up to 575 (beyond that a
+ * matrix product fills the chip by itself and is left to the caller's BLAS).
  * nghost is 0, as the reference's force_components has natoms_pad rows.
  * All columns come from one pass over the atoms: the adjoint of column s is non-zero on the ancestors of scalar
  * moment s only, so the adjoints of all columns together are one gather about as long as an ordinary adjoint sweep
@@ -557,6 +560,10 @@ int a2p_mtp_lin_components_f32(void* plan, int chebyshev_size, double scaling, c
                                const int* bfirstneigh, const float* brcs, const int* btypes, float* ecomp,
                                float* fcomp, float* vcomp, void* stream);
 int a2p_mtp_components_route(int route);
+int a2p_normal_equations_f64(int n, const long long* rows, const double* weights, const double* const* X,
+                             const double* const* y, double* A, double* b, void* stream);
+int a2p_normal_equations_f32(int n, const long long* rows, const double* weights, const float* const* X,
+                             const float* const* y, float* A, float* b, void* stream);
 int a2p_mtp_schmidt_orth_f64(int ntypes, int nmus, int chebyshev_size, const double* coeffs, double* orth_coeffs,
                              void* stream);
 int a2p_mtp_schmidt_orth_f32(int ntypes, int nmus, int chebyshev_size, const float* coeffs, float* orth_coeffs,
