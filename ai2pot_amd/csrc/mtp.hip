@@ -50,7 +50,7 @@ __host__ __device__ inline bool mtp_gred_in_moments(bool loss, int n_moms)
 // thread has finished reading it.
 // The adjoints live in this region too, behind the partial sums (mtp_adjoint_offset): they are needed from the end of
 // the forward sweep to the last pass over the neighbours, which is when the neighbour table is not.  That pass needs
-// the adjoints of the basic moments only: the energy / force / virial kernel gathers them into its dense array, the
+// the adjoints of the basic moments only: the energy / force / virial kernel moves them to its polynomials, the
 // loss kernel copies them behind the region first.
 __host__ __device__ inline int mtp_adjoint_offset(int max_level_slots)
 {
@@ -73,8 +73,8 @@ __host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_
     if (keep) return a + n_moms;
     return a > b ? a : b;
 }
-// the dense adjoint array of the pair-derivative pass takes the place of the moments when it fits
-__host__ __device__ inline bool mtp_dense_in_moments(int nq, int nmp, int n_moms) { return nq * nmp <= n_moms; }
+// the coefficients of the pair-derivative pass's polynomials take the place of the moments when they fit
+__host__ __device__ inline bool mtp_polys_in_moments(int ncoef, int n_moms) { return ncoef <= n_moms; }
 constexpr int MTP_NGMAX = 16;     // most thread groups that share the basic moments of a chunk
 constexpr int MTP_KMAX = 16;      // radial basis size limit
 constexpr int MTP_NMUS_MAX = 8;   // radial function count limit
@@ -349,50 +349,69 @@ __device__ __forceinline__ T block_sum(T v, T* scratch, int tid)
     return t;
 }
 
-// Pair derivatives of one neighbour by a walk over the monomial rows (mtp_plan.h): the lane owns the
-// neighbour whose table row is `t`, takes rows h, h + ng, ... and returns its share of
-//   gs = sum_i adj_i m_i (g' - k g / r),   w = sum_i adj_i g grad_u m_i,
-// with  c_q = sum_mu AD[q][mu] g_mu  and  d_q = sum_mu AD[q][mu] g'_mu  formed once per monomial:
-//   gs += m_q (d_q - k_q c_q / r),  w_x += c_q a x^(a-1) y^b z^c,  w_y += c_q b x^a y^(b-1) z^c,
-//   w_z += c_q c x^a y^b z^(c-1).
-template <typename T, int NMP>
-__device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __restrict__ AD, const int* __restrict__ rows,
-                                          int nrows, int h, int ng, int kmax, int nmus, int OX, int OY, int OZ, int OG,
-                                          int ODG, T rinv, T& gs, T& wx, T& wy, T& wz)
+// The adjoints of the basic moments as coefficients of the row polynomials (mtp_plan.h).  Ends without a barrier.
+template <typename T, int NT>
+__device__ __forceinline__ void scatter_polys(const MtpPlanDevice& p, T* __restrict__ dst, const T* __restrict__ src, int tid)
 {
-    T g[NMP], dg[NMP];
-#pragma unroll
-    for (int mu = 0; mu < NMP; mu++) {
-        g[mu] = mu < nmus ? t[OG + mu] : (T)0;
-        dg[mu] = mu < nmus ? t[ODG + mu] : (T)0;
+    if (p.poly_unique && p.ncoef_poly == p.n_basic) {        // the usual case: a permutation
+        for (int i = tid; i < p.n_basic; i += NT) dst[p.poly_pos[i]] = src[i];
+        return;
     }
+    for (int e = tid; e < p.ncoef_poly; e += NT) {
+        const int one = p.poly_src[e];
+        T v = (T)0;
+        if (one >= 0) v = src[one];
+        else if (one == -2)
+            for (int q = p.poly_off[e]; q < p.poly_off[e + 1]; q++) v += src[p.poly_items[q]];
+        dst[e] = v;
+    }
+}
+
+// Pair derivatives of one neighbour by a walk over the monomial rows (mtp_plan.h): the lane owns the
+// neighbour whose table row is `t`, takes every ng-th row and returns its share of
+//   gs = sum_i adj_i m_i (g' - k g / r),   w = sum_i adj_i g grad_u m_i.
+// A row (a, b) and a radial function mu make a polynomial in z, P(z) = sum_c adj z^c over the basic moments
+// (mu, a, b, c), whose value and derivative come from one Horner walk: two FMAs per basic moment and neighbour.  With
+// s1 = sum_mu g P, s2 = sum_mu g P', sd = sum_mu g' P (and z P' = sum_c c adj z^c) the row adds
+//   gs += x^a y^b (sd - ((a + b) s1 + z s2) / r),  w_x += a x^(a-1) y^b s1,  w_y += b x^a y^(b-1) s1,  w_z += x^a y^b s2.
+// What bounds it: the vector ALUs' issue and the LDS reads of the coefficients (uniform over a group's lanes).  A walk
+// over all monomials with every mu (a dense array of adjoints, 2 nmus + 12 operations per monomial) took @@.
+template <typename T>
+__device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __restrict__ coef, const int* __restrict__ rows,
+                                          const int* __restrict__ polys, int nrows, int h, int ng, int OX, int OY, int OZ,
+                                          int OG, int ODG, T rinv, T& gs, T& wx, T& wy, T& wz)
+{
     const T z = t[OZ + 1];
-    for (int r = h; r < nrows; r += ng) {
+    // the rows are sorted by length: groups take them in alternating direction, which evens out their shares
+    for (int pass = 0, r = h; r < nrows; pass++, r = pass * ng + (pass & 1 ? ng - 1 - h : h)) {
         const int rw = rows[r];
         const int ea = rw & 255, eb = (rw >> 8) & 255;
-        const int len = kmax - ea - eb + 1;
+        const int s_end = rows[r + 1] >> 16;
+        T s1 = (T)0, s2 = (T)0, sd = (T)0;
+        for (int s = rw >> 16; s < s_end; s++) {
+            const int pw = polys[s];
+            const T g = t[OG + (pw & 15)], dg = t[ODG + (pw & 15)];
+            const T* c = coef + (pw >> 12);                  // highest power first
+            int len = (pw >> 4) & 255;
+            T v = (T)0, d = (T)0;
+            if (len & 1) v = *c++;
+            for (len >>= 1; len > 0; len--, c += 2) {
+                const T c0 = c[0], c1 = c[1];
+                d = d * z + v;
+                v = v * z + c0;
+                d = d * z + v;
+                v = v * z + c1;
+            }
+            s1 += g * v;
+            s2 += g * d;
+            sd += dg * v;
+        }
         const T xa = t[OX + ea], yb = t[OY + eb];
         const T xy = xa * yb;
-        const T Wx = (T)ea * t[OX + max(ea - 1, 0)] * yb;
-        const T Wy = (T)eb * xa * t[OY + max(eb - 1, 0)];
-        const T* ad = AD + (size_t)(rw >> 16) * NMP;
-        T zc = (T)1, zcm = (T)0, kf = (T)(ea + eb), cf = (T)0;
-        for (int c = 0; c < len; c++) {
-            T cq = (T)0, dq = (T)0;
-#pragma unroll
-            for (int mu = 0; mu < NMP; mu++) {
-                const T v = ad[mu];
-                cq += v * g[mu];
-                dq += v * dg[mu];
-            }
-            gs += xy * zc * (dq - kf * cq * rinv);
-            const T cz = cq * zc;
-            wx += cz * Wx;
-            wy += cz * Wy;
-            wz += cq * cf * zcm * xy;
-            zcm = zc; zc *= z; kf += (T)1; cf += (T)1;
-            ad += NMP;
-        }
+        gs += xy * (sd - ((T)(ea + eb) * s1 + z * s2) * rinv);
+        wx += (T)ea * t[OX + max(ea - 1, 0)] * yb * s1;
+        wy += (T)eb * xa * t[OY + max(eb - 1, 0)] * s1;
+        wz += xy * s2;
     }
 }
 
@@ -462,9 +481,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
     for (int i = lane; i < n_basic; i += NT)
         bas[i] = (unsigned)p.basic[i * 4] | ((unsigned)p.basic[i * 4 + 1] << 8) |
                  ((unsigned)p.basic[i * 4 + 2] << 16) | ((unsigned)p.basic[i * 4 + 3] << 24);
-    int* rws = (int*)(bas + n_basic);        // monomial rows of the pair-derivative walk
+    int* rws = (int*)(bas + n_basic);        // monomial rows and polynomials of the pair-derivative walk
     if (!LOSS) {
-        for (int i = lane; i < p.nrows; i += NT) rws[i] = p.rows[i];
+        for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
+        for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
     }
     for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
     for (int i = lane; i < n_moms; i += NT) {
@@ -586,23 +606,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
 
     if (!LOSS) {
         // ---- pair derivatives ------------------------------------------------------------------
-        // The adjoints of the basic moments, gathered by monomial (mtp_plan.h); the moments are dead
-        T* AD = mtp_dense_in_moments(p.nq, p.nmp, n_moms) ? M : nnb + (a.H > 0 ? p.n_scalar + a.H : 0);
-        __syncthreads();
-        if (p.dense_unique) {
-            for (int e = lane; e < p.nq * p.nmp; e += NT) AD[e] = (T)0;
-            __syncthreads();
-            for (int i = lane; i < n_basic; i += NT) AD[p.dense_pos[i]] = A[i];
-        } else {
-            for (int e = lane; e < p.nq * p.nmp; e += NT) {
-                const int src = p.dense_src[e];
-                T v = (T)0;
-                if (src >= 0) v = A[src];
-                else if (src == -2)
-                    for (int q = p.dense_off[e]; q < p.dense_off[e + 1]; q++) v += A[p.dense_items[q]];
-                AD[e] = v;
-            }
-        }
+        // The adjoints of the basic moments as polynomial coefficients; the moments are dead
+        T* AD = mtp_polys_in_moments(p.ncoef_poly, n_moms) ? M : nnb + (a.H > 0 ? p.n_scalar + a.H : 0);
+        scatter_polys<T, NT>(p, AD, A, lane);
         // The row is cut into equal chunks of at most MTP_NC neighbours; within a chunk of nc
         // neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one
         // per monomial row) share the rows, so a short chunk still keeps the workgroup busy.
@@ -627,12 +633,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
             if (h < ng) {
                 const T* t = tab + j * E;
                 ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
-                switch (p.nmp) {
-                case 2: pair_walk<T, 2>(t, AD, rws, p.nrows, h, ng, kmax, nmus, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz); break;
-                case 4: pair_walk<T, 4>(t, AD, rws, p.nrows, h, ng, kmax, nmus, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz); break;
-                case 6: pair_walk<T, 6>(t, AD, rws, p.nrows, h, ng, kmax, nmus, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz); break;
-                default: pair_walk<T, 8>(t, AD, rws, p.nrows, h, ng, kmax, nmus, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz); break;
-                }
+                pair_walk<T>(t, AD, rws, rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
             }
             __syncthreads();            // every thread has read its table row: the group sums take its place
             // group sums in the order h = 0 .. ng-1
@@ -1453,35 +1454,54 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     for (int m = nmus - 1; m >= 0; m--) mu_begin[m] = std::min(mu_begin[m], mu_begin[m + 1]);
     mu_begin[0] = 0;
 
-    // monomial rows and the dense adjoint map of the pair-derivative pass (mtp_plan.h)
-    const int nmp = (nmus + 1) / 2 * 2;
-    std::vector<int> row_base((kmax + 1) * (kmax + 1), -1), rows;
-    int nq = 0;
-    for (int a = 0; a <= kmax; a++)
-        for (int b = 0; a + b <= kmax; b++) {
-            row_base[a * (kmax + 1) + b] = nq;
-            rows.push_back(a | (b << 8) | (nq << 16));
-            nq += kmax - a - b + 1;
-        }
-    A2P_REQUIRE(nq < 32768, A2P_ERR_INVALID, "mtp plan: too many monomials");
-    std::stable_sort(rows.begin(), rows.end(), [&](int x, int y) {
-        return (x & 255) + ((x >> 8) & 255) < (y & 255) + ((y >> 8) & 255);     // longest rows first
-    });
-    std::vector<std::vector<int>> dense_lists((size_t)nq * nmp);
+    // monomial rows, their polynomials and the places of the basic moments among the coefficients (mtp_plan.h)
+    std::vector<int> degree((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);      // highest c + 1 of (a, b, mu), 0: none
     for (int i = 0; i < n_basic; i++) {
         const int* q = basic + i * 4;
-        dense_lists[(size_t)(row_base[q[1] * (kmax + 1) + q[2]] + q[3]) * nmp + q[0]].push_back(i);
+        int& l = degree[((size_t)q[1] * (kmax + 1) + q[2]) * nmus + q[0]];
+        l = std::max(l, q[3] + 1);
     }
-    std::vector<int> dense_src((size_t)nq * nmp), dense_off((size_t)nq * nmp + 1, 0), dense_items, dense_pos(n_basic);
-    int dense_unique = 1;
-    for (size_t e = 0; e < dense_lists.size(); e++) {
-        dense_src[e] = dense_lists[e].empty() ? -1 : (dense_lists[e].size() == 1 ? dense_lists[e][0] : -2);
-        dense_off[e] = (int)dense_items.size();
-        if (dense_lists[e].size() > 1) dense_unique = 0;
-        for (int i : dense_lists[e]) dense_pos[i] = (int)e;
-        dense_items.insert(dense_items.end(), dense_lists[e].begin(), dense_lists[e].end());
+    std::vector<std::pair<int, int>> row_ab;
+    auto row_size = [&](const std::pair<int, int>& r) {
+        int n = 0;
+        for (int m = 0; m < nmus; m++) n += degree[((size_t)r.first * (kmax + 1) + r.second) * nmus + m];
+        return n;
+    };
+    for (int a = 0; a <= kmax; a++)
+        for (int b = 0; a + b <= kmax; b++)
+            if (row_size({a, b})) row_ab.push_back({a, b});
+    std::stable_sort(row_ab.begin(), row_ab.end(), [&](const std::pair<int, int>& x, const std::pair<int, int>& y) {
+        return row_size(x) > row_size(y);                                       // longest rows first
+    });
+    std::vector<int> rows, polys, poly_off((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);
+    int n_poly_coef = 0;
+    for (const auto& r : row_ab) {
+        rows.push_back(r.first | (r.second << 8) | ((int)polys.size() << 16));
+        for (int m = 0; m < nmus; m++) {
+            const size_t e = ((size_t)r.first * (kmax + 1) + r.second) * nmus + m;
+            if (!degree[e]) continue;
+            poly_off[e] = n_poly_coef;
+            polys.push_back(m | (degree[e] << 4) | (n_poly_coef << 12));
+            n_poly_coef += degree[e];
+        }
     }
-    dense_off[dense_lists.size()] = (int)dense_items.size();
+    rows.push_back((int)polys.size() << 16);
+    std::vector<std::vector<int>> poly_lists(n_poly_coef);
+    std::vector<int> poly_src(n_poly_coef), poly_items_off((size_t)n_poly_coef + 1, 0), poly_items, poly_pos(n_basic);
+    int poly_unique = 1;
+    for (int i = 0; i < n_basic; i++) {
+        const int* q = basic + i * 4;
+        const size_t e = ((size_t)q[1] * (kmax + 1) + q[2]) * nmus + q[0];
+        poly_pos[i] = poly_off[e] + degree[e] - 1 - q[3];
+        poly_lists[poly_pos[i]].push_back(i);
+    }
+    for (int e = 0; e < n_poly_coef; e++) {
+        poly_src[e] = poly_lists[e].empty() ? -1 : (poly_lists[e].size() == 1 ? poly_lists[e][0] : -2);
+        poly_items_off[e] = (int)poly_items.size();
+        if (poly_lists[e].size() > 1) poly_unique = 0;
+        poly_items.insert(poly_items.end(), poly_lists[e].begin(), poly_lists[e].end());
+    }
+    poly_items_off[n_poly_coef] = (int)poly_items.size();
 
     // nodes (scalar moment, ancestor) and their reverse gather (mtp_plan.h), for batches of scalar moments whose node
     // adjoints fit MTP_NODE_CAP entries of LDS
@@ -1620,10 +1640,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const size_t o_rh = add(R.gdepth.data(), sizeof(int) * R.gdepth.size());
     const size_t o_rt = add(R.terms.data(), sizeof(int2) * R.terms.size());
     const size_t o_rows = add(rows.data(), sizeof(int) * rows.size());
-    const size_t o_dsrc = add(dense_src.data(), sizeof(int) * dense_src.size());
-    const size_t o_doff = add(dense_off.data(), sizeof(int) * dense_off.size());
-    const size_t o_dit = add(dense_items.data(), sizeof(int) * dense_items.size());
-    const size_t o_dpos = add(dense_pos.data(), sizeof(int) * dense_pos.size());
+    const size_t o_poly = add(polys.data(), sizeof(int) * polys.size());
+    const size_t o_psrc = add(poly_src.data(), sizeof(int) * poly_src.size());
+    const size_t o_poff = add(poly_items_off.data(), sizeof(int) * poly_items_off.size());
+    const size_t o_pit = add(poly_items.data(), sizeof(int) * poly_items.size());
+    const size_t o_ppos = add(poly_pos.data(), sizeof(int) * poly_pos.size());
     struct XOff { size_t root, seed, level, multi, src, rem, gbase, gdepth, terms, bbase, bdepth, bsteps, brem, bwords; };
     std::vector<XOff> xoffs;
     for (const XHost& h : xhosts) {
@@ -1668,10 +1689,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.r_gbase = (const int*)(base + o_rg); d.r_gdepth = (const int*)(base + o_rh);
     d.r_terms = (const int2*)(base + o_rt);
     d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
-    d.nq = nq; d.nmp = nmp; d.nrows = (int)rows.size();
-    d.rows = (const int*)(base + o_rows); d.dense_src = (const int*)(base + o_dsrc);
-    d.dense_off = (const int*)(base + o_doff); d.dense_items = (const int*)(base + o_dit);
-    d.dense_pos = (const int*)(base + o_dpos); d.dense_unique = dense_unique;
+    d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
+    d.rows = (const int*)(base + o_rows); d.polys = (const int*)(base + o_poly);
+    d.poly_src = (const int*)(base + o_psrc); d.poly_off = (const int*)(base + o_poff);
+    d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
+    d.poly_unique = poly_unique;
     d.x_nodes = 0; d.x_slots = 0;                // set per batch by the components call (MtpPlan::xbatches)
     for (size_t i = 0; i < xhosts.size(); i++) {
         const XOff& o = xoffs[i];
@@ -1723,7 +1745,7 @@ size_t lds_bytes(const MtpPlanDevice& p, int E, bool loss, int ntypes, int K, in
     // loss mode: P, Q, the neighbour types and the per-atom coefficient-gradient block
     if (loss) n += 2 * (size_t)MTP_NC * p.nmus + MTP_NC + (size_t)ntypes * p.nmus * K;
     if (H > 0) n += (size_t)p.n_scalar + (loss ? 5 : 1) * (size_t)H;     // network inputs and per-neuron values
-    if (!loss && !mtp_dense_in_moments(p.nq, p.nmp, p.n_moms)) n += (size_t)p.nq * p.nmp;
+    if (!loss && !mtp_polys_in_moments(p.ncoef_poly, p.n_moms)) n += (size_t)p.ncoef_poly;
     return n * sizeof(T) + 64;      // the packed basic-moment table (4 n_basic bytes) follows
 }
 
@@ -1772,8 +1794,8 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
     const bool wide = a.p.n_moms >= (LOSS ? 300 : 1000);   // enough work per atom to keep 256 threads busy
     auto lds_for = [&](int nc, size_t* main, bool keep = false) {
         *main = (lds_bytes<T>(a.p, a.E, LOSS, a.ntypes, a.K, a.H, nc, wide ? 256 : 64, keep) + 15) / 16 * 16;
-        // the packed basic-moment table; energy / force / virial kernel: + the monomial rows
-        return *main + (LOSS ? (size_t)a.p.n_basic : (size_t)a.p.n_basic + a.p.nrows) * sizeof(unsigned);
+        // the packed basic-moment table; energy / force / virial kernel: + the monomial rows and polynomials
+        return *main + ((size_t)a.p.n_basic + (LOSS ? 0 : a.p.nrows + 1 + a.p.npoly)) * sizeof(unsigned);
     };
     size_t lds_main = 0;
     int nc_cap = MTP_NC;

@@ -58,18 +58,17 @@ struct MtpPlanDevice {
     const int* r_gdepth;       // [n_rslots/64]
     const int2* r_terms;
     int max_level_slots;       // most slots of any level (forward or reverse)
-    // Monomial walk of the pair-derivative pass.  The monomials x^a y^b z^c, a + b + c <= kmax, are numbered
-    // q = row_base(a, b) + c; the adjoints of the basic moments are gathered into a dense array
-    // AD[q][nmp] (mu fastest, nmp = nmus rounded up to even, zero where no basic moment has that
-    // (mu, a, b, c)), so that a lane that owns one neighbour can walk a row (a, b), c = 0 .. kmax-a-b,
-    // with z^c by recurrence and the adjoints as uniform reads.
-    int nq, nmp, nrows;
-    const int* rows;           // [nrows] a | b << 8 | row_base << 16, longest rows first
-    const int* dense_pos;      // [n_basic] entry of each basic moment
-    int dense_unique;          // no two basic moments share an entry (the usual case: a plain scatter fills AD)
-    const int* dense_src;      // [nq*nmp] basic moment behind the entry, -1 none, -2 several (dense_off/items)
-    const int* dense_off;      // [nq*nmp+1]
-    const int* dense_items;    // [n_basic] basic moments ordered by dense entry
+    // Polynomials of the passes that own a neighbour per lane.  The basic moments (mu, a, b, c) with the same row (a, b) and
+    // the same mu are the coefficients of a polynomial in z; its coefficients lie together, highest power first, up to
+    // the highest power in the tables (powers the tables leave out: zero).
+    int nrows, npoly, ncoef_poly;
+    const int* rows;           // [nrows + 1] a | b << 8 | first polynomial << 16, longest rows first
+    const int* polys;          // [npoly] mu | length << 4 | first coefficient << 12
+    const int* poly_pos;       // [n_basic] coefficient of each basic moment
+    int poly_unique;           // no two basic moments share a coefficient (the usual case: a plain scatter fills them)
+    const int* poly_src;       // [ncoef_poly] basic moment behind the coefficient, -1 none, -2 several (poly_off / items)
+    const int* poly_off;       // [ncoef_poly+1]
+    const int* poly_items;     // [n_basic] basic moments ordered by coefficient
     // The one-hot adjoints of all scalar moments at once (linear-solver components).  A node (s, m) is moment m as an
     // ancestor of scalar moment s: mapping[s] itself, or a factor of a product among its ancestors.  The adjoint
     // sweeps of all read-outs e_s together are one reverse gather over the nodes, laid out like the reverse gather
