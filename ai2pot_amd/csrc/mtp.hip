@@ -51,7 +51,7 @@ __host__ __device__ inline bool mtp_gred_in_moments(bool loss, int n_moms)
 // The adjoints live in this region too, behind the partial sums (mtp_adjoint_offset): they are needed from the end of
 // the forward sweep to the last pass over the neighbours, which is when the neighbour table is not.  That pass needs
 // the adjoints of the basic moments only: the energy / force / virial kernel moves them to its polynomials, the
-// loss kernel copies them behind the region first.
+// loss kernel moves them behind the region first.
 __host__ __device__ inline int mtp_adjoint_offset(int max_level_slots)
 {
     return ((max_level_slots > 8 ? max_level_slots : 8) + 1) & ~1;     // at least the scratch of a block sum
@@ -375,7 +375,8 @@ __device__ __forceinline__ void scatter_polys(const MtpPlanDevice& p, T* __restr
 // s1 = sum_mu g P, s2 = sum_mu g P', sd = sum_mu g' P (and z P' = sum_c c adj z^c) the row adds
 //   gs += x^a y^b (sd - ((a + b) s1 + z s2) / r),  w_x += a x^(a-1) y^b s1,  w_y += b x^a y^(b-1) s1,  w_z += x^a y^b s2.
 // What bounds it: the vector ALUs' issue and the LDS reads of the coefficients (uniform over a group's lanes).  A walk
-// over all monomials with every mu (a dense array of adjoints, 2 nmus + 12 operations per monomial) took @@.
+// over all monomials with every mu (a dense array of adjoints, 2 nmus + 12 operations per monomial) took
+// 356 instead of 334 us for the whole kernel at level 20, 8192 atoms, and 125 instead of 118 us at level 16.
 template <typename T>
 __device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __restrict__ coef, const int* __restrict__ rows,
                                           const int* __restrict__ polys, int nrows, int h, int ng, int OX, int OY, int OZ,
@@ -415,6 +416,48 @@ __device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __re
     }
 }
 
+// The polynomials of a neighbour for the loss gradient: every ng-th one of a radial function's from the s-th on.  With
+// A = sum adj m, B = sum (cE adj + mixed) m over the basic moments of mu and k m = u . grad m (m is homogeneous),
+//   P_mu = B + (w - (w . u) u) . grad A / r,   Q_mu = (w . u) A.
+// Three FMAs per basic moment and neighbour; forming each monomial with its gradient from the table of powers instead
+// took about thirty operations and nine LDS reads (263 -> 252 us for the kernel, level 16, 64 structures of 128 atoms).
+template <typename T>
+__device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __restrict__ Ac, const T* __restrict__ Bc,
+                                          const int* __restrict__ polys, int& s, int end, int ng, int OX, int OY, int OZ,
+                                          int OU, int OW, T cE, bool no_tan, T& P, T& Q)
+{
+    P = Q = (T)0;
+    if (s >= end) return;
+    const T z = t[OZ + 1], rinv = t[OU + 3];
+    const T wu = no_tan ? (T)0 : t[OW + 3];
+    const T vx = no_tan ? (T)0 : (t[OW + 0] - wu * t[OU + 0]) * rinv;
+    const T vy = no_tan ? (T)0 : (t[OW + 1] - wu * t[OU + 1]) * rinv;
+    const T vz = no_tan ? (T)0 : (t[OW + 2] - wu * t[OU + 2]) * rinv;
+    for (; s < end; s += ng) {
+        const int pw = polys[s];
+        const int ea = pw & 31, eb = (pw >> 5) & 31;
+        int len = (pw >> 10) & 31;
+        const T* ca = Ac + (pw >> 15);
+        const T* cb = Bc + (pw >> 15);
+        const T xa = t[OX + ea], yb = t[OY + eb], xm = t[OX + max(ea - 1, 0)], ym = t[OY + max(eb - 1, 0)];
+        T va = (T)0, da = (T)0, vb = (T)0;
+        if (len & 1) { va = *ca++; vb = *cb++; }
+        for (len >>= 1; len > 0; len--, ca += 2, cb += 2) {
+            const T a0 = ca[0], a1 = ca[1], b0 = cb[0], b1 = cb[1];
+            da = da * z + va;
+            va = va * z + a0;
+            vb = vb * z + b0;
+            da = da * z + va;
+            va = va * z + a1;
+            vb = vb * z + b1;
+        }
+        const T xy = xa * yb;
+        P += xy * (cE * va + vb) + va * (vx * ((T)ea * xm * yb) + vy * ((T)eb * xa * ym)) + da * (vz * xy);
+        Q += xy * va;
+    }
+    Q *= wu;
+}
+
 // NT threads per centre atom: 64 for small tables, 256 when there is enough work per atom
 // (four workgroups of 256 threads fit the LDS of a CU at the larger levels: keep the registers to match)
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
@@ -451,11 +494,11 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
     const bool share = mtp_gred_in_moments(LOSS, n_moms);
     // energy / force / virial kernel: the group sums are written over the table once it has been read
     T* gred = LOSS ? (share ? M : tab + MTP_NC * E) : tab;
-    // loss mode, behind the region: adjoints and mixed adjoints of the basic moments (copies for the last pass) |
+    // loss mode, behind the region: adjoints and mixed adjoints of the basic moments (as coefficients of the polynomials) |
     // P[nc][nmus] | Q[nc][nmus] | ...
     T* Ab = tab + mtp_table_region(MTP_NC, E, LOSS, n_moms, p.max_level_slots, NT, keep);
-    T* Bb = Ab + n_basic;
-    T* pq = LOSS ? Bb + n_basic : Ab;
+    T* Bb = Ab + p.ncoef_poly;
+    T* pq = LOSS ? Bb + p.ncoef_poly : Ab;
 
     if (ii >= a.binum[b]) {                  // padded row: contributes nothing
         if (!LOSS && a.partial && lane < 10) a.partial[row * 10 + lane] = 0.0;
@@ -485,6 +528,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
     if (!LOSS) {
         for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
         for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
+    } else {
+        for (int i = lane; i < p.npoly; i += NT) rws[i] = p.polys_mu[i];
+        for (int i = lane; i <= nmus; i += NT) rws[p.npoly + i] = p.polys_end[i];
     }
     for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
     for (int i = lane; i < n_moms; i += NT) {
@@ -699,7 +745,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
         // linearMtpLoss.h:417-434; the reference's network backward has no such term (Bm stays zero)
         if (!no_tan && (a.H == 0 || a.nn_exact)) sweep_reverse<T, true, NT>(p, M, Bm, A, Tg, lane);
         // the last pass needs the adjoints of the basic moments while the table is back in its region
-        for (int i = lane; i < n_basic; i += NT) { Ab[i] = A[i]; Bb[i] = Bm[i]; }
+        scatter_polys<T, NT>(p, Ab, A, lane);
+        scatter_polys<T, NT>(p, Bb, Bm, lane);
         T* grow = a.gpart + row * a.ngrad;
         for (int q = lane; q < a.ngrad; q += NT) grow[q] = (T)0;
         __syncthreads();         // other threads overwrite some of these entries below
@@ -747,29 +794,13 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
             __syncthreads();
             build_table<T, true, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
             __syncthreads();
-            // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out
+            // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  The groups take the polynomials in
+            // turn, on from one mu to the next.  (All of a thread's sums kept to the end, with one round of group sums: 100
+            // registers instead of 70, so five wavefronts per SIMD instead of six, and the kernel 263 -> 320 us.)
+            int s = h < ng ? h : p.npoly;
             for (int mu = 0; mu < nmus; mu++) {
-                T Pv = (T)0, Qv = (T)0;
-                if (h < ng) {
-                    const T* t = tab + j * E;
-                    const T rinv = t[OU + 3], wu = t[OW + 3];
-                    for (int i = p.mu_begin[mu] + h; i < p.mu_begin[mu + 1]; i += ng) {
-                        const unsigned bw = bas[i];
-                        const int ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
-                        const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
-                        const T m = xa * yb * zc;
-                        const T adj = Ab[i];
-                        if (no_tan) {                 // w = 0: only the energy term is left
-                            Pv += cE * adj * m;
-                            continue;
-                        }
-                        const T gm = (T)ea * t[OX + max(ea - 1, 0)] * yb * zc * t[OW + 0] +
-                                     (T)eb * xa * t[OY + max(eb - 1, 0)] * zc * t[OW + 1] +
-                                     (T)ec * xa * yb * t[OZ + max(ec - 1, 0)] * t[OW + 2];
-                        Pv += (cE * adj + Bb[i]) * m + adj * rinv * (gm - (T)(ea + eb + ec) * m * wu);
-                        Qv += adj * m * wu;
-                    }
-                }
+                T Pv, Qv;
+                loss_walk<T>(tab + j * E, Ab, Bb, rws, s, rws[p.npoly + mu + 1], ng, OX, OY, OZ, OU, OW, cE, no_tan, Pv, Qv);
                 {
                     T* gr = gred + lane * 2;
                     gr[0] = Pv; gr[1] = Qv;
@@ -1449,11 +1480,6 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const Ell F = build_ell(fl, f_by), R = build_ell(rl, r_by);
     A2P_REQUIRE(!F.too_long && !R.too_long, A2P_ERR_INVALID,
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
-    std::vector<int> mu_begin(nmus + 1, n_basic);
-    for (int i = n_basic - 1; i >= 0; i--) mu_begin[basic[i * 4]] = i;
-    for (int m = nmus - 1; m >= 0; m--) mu_begin[m] = std::min(mu_begin[m], mu_begin[m + 1]);
-    mu_begin[0] = 0;
-
     // monomial rows, their polynomials and the places of the basic moments among the coefficients (mtp_plan.h)
     std::vector<int> degree((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);      // highest c + 1 of (a, b, mu), 0: none
     for (int i = 0; i < n_basic; i++) {
@@ -1486,6 +1512,14 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         }
     }
     rows.push_back((int)polys.size() << 16);
+    std::vector<int> polys_mu, polys_end(nmus + 1, 0);            // by mu, for the loss gradient
+    for (int m = 0; m < nmus; m++) {
+        for (const auto& r : row_ab) {
+            const size_t e = ((size_t)r.first * (kmax + 1) + r.second) * nmus + m;
+            if (degree[e]) polys_mu.push_back(r.first | (r.second << 5) | (degree[e] << 10) | (poly_off[e] << 15));
+        }
+        polys_end[m + 1] = (int)polys_mu.size();
+    }
     std::vector<std::vector<int>> poly_lists(n_poly_coef);
     std::vector<int> poly_src(n_poly_coef), poly_items_off((size_t)n_poly_coef + 1, 0), poly_items, poly_pos(n_basic);
     int poly_unique = 1;
@@ -1621,7 +1655,6 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         return off;
     };
     const size_t o_basic = add(basic, sizeof(int) * 4 * n_basic);
-    const size_t o_mu = add(mu_begin.data(), sizeof(int) * mu_begin.size());
     const size_t o_map = add(mapping, sizeof(int) * n_scalar);
     const size_t o_fl = add(F.level.data(), sizeof(int) * F.level.size());
     const size_t o_fe = add(F.lend.data(), sizeof(int) * F.lend.size());
@@ -1641,6 +1674,8 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const size_t o_rt = add(R.terms.data(), sizeof(int2) * R.terms.size());
     const size_t o_rows = add(rows.data(), sizeof(int) * rows.size());
     const size_t o_poly = add(polys.data(), sizeof(int) * polys.size());
+    const size_t o_pmu = add(polys_mu.data(), sizeof(int) * polys_mu.size());
+    const size_t o_pend = add(polys_end.data(), sizeof(int) * polys_end.size());
     const size_t o_psrc = add(poly_src.data(), sizeof(int) * poly_src.size());
     const size_t o_poff = add(poly_items_off.data(), sizeof(int) * poly_items_off.size());
     const size_t o_pit = add(poly_items.data(), sizeof(int) * poly_items.size());
@@ -1676,7 +1711,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     MtpPlanDevice& d = plan->d;
     d.n_moms = n_moms; d.n_basic = n_basic; d.n_times = n_times; d.n_scalar = n_scalar;
     d.nmus = nmus; d.kmax = kmax; d.n_levels = n_levels;
-    d.basic = (const int*)(base + o_basic); d.mu_begin = (const int*)(base + o_mu);
+    d.basic = (const int*)(base + o_basic);
     d.mapping = (const int*)(base + o_map);
     d.f_level = (const int*)(base + o_fl); d.f_lend = (const int*)(base + o_fe);
     d.f_multi = (const int*)(base + o_fx);
@@ -1691,6 +1726,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
     d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
     d.rows = (const int*)(base + o_rows); d.polys = (const int*)(base + o_poly);
+    d.polys_mu = (const int*)(base + o_pmu); d.polys_end = (const int*)(base + o_pend);
     d.poly_src = (const int*)(base + o_psrc); d.poly_off = (const int*)(base + o_poff);
     d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
     d.poly_unique = poly_unique;
@@ -1740,7 +1776,7 @@ size_t lds_bytes(const MtpPlanDevice& p, int E, bool loss, int ntypes, int K, in
 {
     // the neighbour table and the group sums double as the sweeps' partial-sum arrays
     const size_t tabs = (size_t)mtp_table_region(MTP_NC, E, loss, p.n_moms, p.max_level_slots, nt, keep);
-    size_t n = (size_t)p.n_moms * (loss ? 2 : 1) + tabs + (loss ? 2 * (size_t)p.n_basic : 0) +
+    size_t n = (size_t)p.n_moms * (loss ? 2 : 1) + tabs + (loss ? 2 * (size_t)p.ncoef_poly : 0) +
                (size_t)ntypes * p.nmus * K;   // + the coefficient copy
     // loss mode: P, Q, the neighbour types and the per-atom coefficient-gradient block
     if (loss) n += 2 * (size_t)MTP_NC * p.nmus + MTP_NC + (size_t)ntypes * p.nmus * K;
@@ -1794,8 +1830,8 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
     const bool wide = a.p.n_moms >= (LOSS ? 300 : 1000);   // enough work per atom to keep 256 threads busy
     auto lds_for = [&](int nc, size_t* main, bool keep = false) {
         *main = (lds_bytes<T>(a.p, a.E, LOSS, a.ntypes, a.K, a.H, nc, wide ? 256 : 64, keep) + 15) / 16 * 16;
-        // the packed basic-moment table; energy / force / virial kernel: + the monomial rows and polynomials
-        return *main + ((size_t)a.p.n_basic + (LOSS ? 0 : a.p.nrows + 1 + a.p.npoly)) * sizeof(unsigned);
+        // the packed basic-moment table and the polynomials, with the monomial rows or the run of every mu
+        return *main + ((size_t)a.p.n_basic + a.p.npoly + 1 + (LOSS ? a.p.nmus : a.p.nrows)) * sizeof(unsigned);
     };
     size_t lds_main = 0;
     int nc_cap = MTP_NC;

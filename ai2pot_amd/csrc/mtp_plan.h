@@ -28,7 +28,6 @@ struct MtpPlanDevice {
     int n_levels;              // number of product levels (>= 0)
     // device arrays
     const int* basic;          // [n_basic*4]  (mu, a, b, c)
-    const int* mu_begin;       // [nmus+1]     basics are grouped by mu: run of each mu
     const int* mapping;        // [n_scalar]
     // forward gather.  A slot holds up to MTP_SLOT_CAP terms of one destination moment; a longer
     // list is cut into consecutive slots (pieces), so that no lane walks a long list alone; the pieces of a
@@ -64,6 +63,8 @@ struct MtpPlanDevice {
     int nrows, npoly, ncoef_poly;
     const int* rows;           // [nrows + 1] a | b << 8 | first polynomial << 16, longest rows first
     const int* polys;          // [npoly] mu | length << 4 | first coefficient << 12
+    const int* polys_mu;       // [npoly] the same by mu: a | b << 5 | length << 10 | first coefficient << 15
+    const int* polys_end;      // [nmus + 1] run of each mu in polys_mu
     const int* poly_pos;       // [n_basic] coefficient of each basic moment
     int poly_unique;           // no two basic moments share a coefficient (the usual case: a plain scatter fills them)
     const int* poly_src;       // [ncoef_poly] basic moment behind the coefficient, -1 none, -2 several (poly_off / items)
