@@ -23,6 +23,7 @@
 #include "a2p_common.h"
 #include "mtp_plan.h"
 #include "loss_kernels.h"
+#include "wave_ops.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -84,7 +85,7 @@ template <typename T>
 struct MtpArgs {
     MtpPlanDevice p;
     int K, ntypes;
-    T scaling, rmax, rmin;
+    T scaling, rmax, rmin, inv_span;     // inv_span = 1 / (rmax - rmin)
     const T *coeffs, *lin, *bias, *q_scaler;
     int B, P, U, nghost;
     const int *binum, *bilist, *bnumneigh, *bfirstneigh;
@@ -134,12 +135,18 @@ __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 // Per-neighbour table for neighbours [c0, c0+nc) of the row.
 // Layout per neighbour (E entries of T): ux^0..kmax | uy^.. | uz^.. | g[nmus] | dg[nmus] |
 // ux uy uz 1/r | (loss mode) wx wy wz w.u | f[K] | df[K]
-// The work is spread over nc * (nmus + 3) tasks: task (role, j) computes for neighbour j either
-// one radial function g_role(r) with its derivative (role < nmus; coefficients from the LDS copy
-// `cf` of the centre species' block) or the powers of one unit-vector component (role - nmus),
-// so the table costs one Chebyshev recurrence of latency instead of nmus of them on nc lanes.
+// PASS says what the pass that follows reads: TAB_MOMENTS powers, g, dg; TAB_TANGENTS also w; TAB_GRADIENT powers, w, f, df.
+// The threads form groups of nc, a neighbour to a thread.  Groups share the radial functions, two to a Chebyshev
+// recurrence (coefficients from the LDS copy `cf` of the centre species' block); more than two where the workgroup has no
+// room for their groups beside those of the powers, of w and of f.  What bounds it is the issue of fp64 instructions, so a
+// group for every function, which would be no faster, is no gain.
+// (One task per radial function and per axis, with every value in every pass, took 333 instead of 324 us for the whole
+// kernel at level 20, 8192 atoms, 118 instead of 111 at level 16, 64 structures of 128 atoms, and 252 instead of 244 for
+// the loss gradient there; early claims and row-swap sums at the end included.)
 // Lanes j < nc also return the neighbour's index, validity and displacement.
-template <typename T, bool LOSS, int NT>
+enum TablePass { TAB_MOMENTS, TAB_TANGENTS, TAB_GRADIENT };
+
+template <typename T, TablePass PASS, int NT>
 __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T* cf, int lane, int nc, int c0,
                                             const T* rcs, const int* first, const int* types, int center,
                                             int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true)
@@ -158,68 +165,86 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
         *nj_out = nj;
         *valid_out = !(sqrt_t(x * x + y * y + z * z) > a.rmax);      // mtpBasis.h:457, linearMtp.h:316
     }
-    const int ntask = fill ? nc * (nmus + 3) : 0;          // fill = false: the table is in place, only the lanes' own
-    for (int task = lane; task < ntask; task += NT) {      // neighbours are returned
+    if (!fill) return;                      // the table is in place, only the lanes' own neighbours are returned
+    // groups [0, nrad) radial functions, then powers, then w, then f
+    constexpr int OTHERS = PASS == TAB_MOMENTS ? 1 : (PASS == TAB_TANGENTS ? 2 : 3);
+    int share = 0, nrad = 0;
+    if (PASS != TAB_GRADIENT) {
+        nrad = max(1, min((nmus + 1) / 2, NT / nc - OTHERS));
+        share = ((nmus + nrad - 1) / nrad + 1) & ~1;
+        nrad = (nmus + share - 1) / share;
+    }
+    const int ntask = nc * (nrad + OTHERS);
+    for (int task = lane; task < ntask; task += NT) {
         const int role = task / nc, j = task - role * nc;
         const int jj = c0 + j;
         const T x = rcs[jj * 3 + 0], y = rcs[jj * 3 + 1], z = rcs[jj * 3 + 2];
         const T r = sqrt_t(x * x + y * y + z * z);
         T* t = tab + j * a.E;
-        // radial functions, basis.h:154-196, 351-381, 620-637
-        const T span = a.rmax - a.rmin;
-        const T xx = ((T)2 * r - (a.rmax + a.rmin)) / span;
-        const T dxx = (T)2 / span;
-        const T u = (r - a.rmin) / span;
-        T s = (T)0, ds = (T)0;
-        if (!(r > a.rmax) && r >= a.rmin && r < a.rmax) {
-            s = u * u * u * ((T)-6 * u * u + (T)15 * u - (T)10) + (T)1;
-            ds = (T)1 / span * ((T)-30 * u * u * u * u + (T)60 * u * u * u - (T)30 * u * u);
+        if (role == nrad) {                                            // powers of the unit vector
+            const T rinv = (T)1 / r;
+            const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
+            T px = (T)1, py = (T)1, pz = (T)1;
+            for (int k = 0; k <= kmax; k++) {
+                t[k] = px; t[kmax + 1 + k] = py; t[2 * (kmax + 1) + k] = pz;
+                px *= ux; py *= uy; pz *= uz;
+            }
+            t[OU + 0] = ux; t[OU + 1] = uy; t[OU + 2] = uz; t[OU + 3] = rinv;
+            continue;
         }
         int nj = first[jj];
         if ((unsigned)nj >= (unsigned)NF) nj = center;
-        if (role < nmus || (LOSS && role == nmus + 1)) {
-            int tj = types[nj];
-            if ((unsigned)tj >= (unsigned)a.ntypes) tj = 0;
-            const T* c = cf + (tj * nmus + (role < nmus ? role : 0)) * K;
-            T g = (T)0, dg = (T)0;
+        if (PASS != TAB_MOMENTS && role == nrad + 1) {
+            // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386)
+            const T* fc = a.dFs + ((size_t)b * a.P + center) * 3;
+            const T* fn = a.dFs + ((size_t)b * a.P + nj) * 3;
+            const T* dv = a.dVs + (size_t)b * 9;
+            T w[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++)
+                w[q] = fc[q] - fn[q] - (dv[q * 3 + 0] * x + dv[q * 3 + 1] * y + dv[q * 3 + 2] * z);
+            t[OW + 0] = w[0]; t[OW + 1] = w[1]; t[OW + 2] = w[2];
+            t[OW + 3] = (w[0] * x + w[1] * y + w[2] * z) / r;
+            continue;
+        }
+        // radial functions, basis.h:154-196, 351-381, 620-637
+        const T xx = ((T)2 * r - (a.rmax + a.rmin)) * a.inv_span, x2 = (T)2 * xx;
+        const T u = (r - a.rmin) * a.inv_span;
+        T s = (T)0, ds = (T)0;
+        if (!(r > a.rmax) && r >= a.rmin && r < a.rmax) {
+            s = a.scaling * (u * u * u * ((T)-6 * u * u + (T)15 * u - (T)10) + (T)1);
+            ds = a.scaling * a.inv_span * ((T)-30 * u * u * u * u + (T)60 * u * u * u - (T)30 * u * u);
+        }
+        const T sx = s * (T)2 * a.inv_span;
+        if (PASS == TAB_GRADIENT) {
             T t0 = (T)1, t1 = xx, d0 = (T)0, d1 = (T)1;
             for (int k = 0; k < K; k++) {
-                T tv, dv;
-                if (k == 0) { tv = t0; dv = d0; }
-                else if (k == 1) { tv = t1; dv = d1; }
-                else {
-                    tv = (T)2 * xx * t1 - t0;
-                    dv = (T)2 * t1 + (T)2 * xx * d1 - d0;
-                    t0 = t1; t1 = tv; d0 = d1; d1 = dv;
-                }
-                const T f = a.scaling * s * tv;
-                const T df = a.scaling * (ds * tv + s * dv * dxx);
-                if (role < nmus) { g += c[k] * f; dg += c[k] * df; }
-                else { t[OF + k] = f; t[ODF + k] = df; }
+                t[OF + k] = s * t0;
+                t[ODF + k] = ds * t0 + sx * d0;
+                const T tv = x2 * t1 - t0, dv = (T)2 * t1 + x2 * d1 - d0;
+                t0 = t1; t1 = tv; d0 = d1; d1 = dv;
             }
-            if (role < nmus) { t[OG + role] = g; t[ODG + role] = dg; }
+            continue;
         }
-        if (role >= nmus) {
-            const int ax = role - nmus;
-            const T rinv = (T)1 / r;
-            const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
-            const T uc = ax == 0 ? ux : (ax == 1 ? uy : uz);
-            T pw = (T)1;
-            T* tp = t + ax * (kmax + 1);
-            for (int k = 0; k <= kmax; k++) { tp[k] = pw; pw *= uc; }
-            if (ax == 0) { t[OU + 0] = ux; t[OU + 1] = uy; t[OU + 2] = uz; t[OU + 3] = rinv; }
-            if (LOSS && ax == 2) {
-                // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386)
-                const T* fc = a.dFs + ((size_t)b * a.P + center) * 3;
-                const T* fn = a.dFs + ((size_t)b * a.P + nj) * 3;
-                const T* dv = a.dVs + (size_t)b * 9;
-                T w[3];
-#pragma unroll
-                for (int q = 0; q < 3; q++)
-                    w[q] = fc[q] - fn[q] - (dv[q * 3 + 0] * x + dv[q * 3 + 1] * y + dv[q * 3 + 2] * z);
-                t[OW + 0] = w[0]; t[OW + 1] = w[1]; t[OW + 2] = w[2];
-                t[OW + 3] = w[0] * ux + w[1] * uy + w[2] * uz;
+        int tj = types[nj];
+        if ((unsigned)tj >= (unsigned)a.ntypes) tj = 0;
+        const int m1 = min(nmus, (role + 1) * share);
+        for (int mu = role * share; mu < m1; mu += 2) {
+            const int two = mu + 1 < m1;
+            const T* ca = cf + (tj * nmus + mu) * K;
+            const T* cb = ca + two * K;
+            T t0 = (T)1, t1 = xx, d0 = (T)0, d1 = (T)1;
+            T ga = (T)0, gb = (T)0, ha = (T)0, hb = (T)0;
+#pragma unroll 4
+            for (int k = 0; k < K; k++) {
+                const T c0k = ca[k], c1k = cb[k];
+                ga += c0k * t0; ha += c0k * d0;
+                gb += c1k * t0; hb += c1k * d0;
+                const T tv = x2 * t1 - t0, dv = (T)2 * t1 + x2 * d1 - d0;
+                t0 = t1; t1 = tv; d0 = d1; d1 = dv;
             }
+            t[OG + mu] = s * ga; t[ODG + mu] = ds * ga + sx * ha;
+            if (two) { t[OG + mu + 1] = s * gb; t[ODG + mu + 1] = ds * gb + sx * hb; }
         }
     }
 }
@@ -338,7 +363,7 @@ __device__ __forceinline__ void sweep_reverse(const MtpPlanDevice& p, const T* M
 template <typename T, int NT>
 __device__ __forceinline__ T block_sum(T v, T* scratch, int tid)
 {
-    v = wave_sum(v);
+    v = wave::all_sum(v);
     if (NT == 64) return v;
     __syncthreads();
     if ((tid & 63) == 0) scratch[tid >> 6] = v;
@@ -522,8 +547,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
     // (mu, a, b, c) of every basic moment, one byte each, behind everything else in LDS
     unsigned* bas = (unsigned*)(smem_raw + a.lds_basic_off);
     for (int i = lane; i < n_basic; i += NT)
-        bas[i] = (unsigned)p.basic[i * 4] | ((unsigned)p.basic[i * 4 + 1] << 8) |
-                 ((unsigned)p.basic[i * 4 + 2] << 16) | ((unsigned)p.basic[i * 4 + 3] << 24);
+        bas[i] = p.basic[i];
     int* rws = (int*)(bas + n_basic);        // monomial rows and polynomials of the pair-derivative walk
     if (!LOSS) {
         for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
@@ -544,7 +568,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
     for (int c0 = 0; c0 < nn; c0 += chunk) {
         const int nc = min(chunk, nn - c0);
         int nj; bool valid; T d[3];
-        build_table<T, LOSS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+        build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
         __syncthreads();
         for (int i = lane; i < n_basic; i += NT) {
             const unsigned bw = bas[i];
@@ -606,8 +630,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
                 acc += w0[(size_t)n * S + k] * qv[k];
                 if (LOSS) tac += w0[(size_t)n * S + k] * Tg[p.mapping[k]] / a.q_scaler[k];
             }
-            acc = wave_sum(acc);
-            if (LOSS) tac = wave_sum(tac);
+            acc = wave::all_sum(acc);
+            if (LOSS) tac = wave::all_sum(tac);
             if ((lane & 63) == 0) {
                 hv[n] = acc;
                 if (LOSS) n_tau[n] = tac;
@@ -671,9 +695,14 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
             int nj; bool valid; T d[3] = {(T)0, (T)0, (T)0};
             __syncthreads();
             // (a row of one chunk finds the table of the first pass still in place when the adjoints lie behind it)
-            build_table<T, false, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
+            build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
                                       !(keep && nchunks == 1));
             __syncthreads();
+            // the pair claims an entry of its target's segment (zeros too: the count of a segment is the number of pairs
+            // naming the target); claimed here, so that the walk covers the answer's way
+            const int tg = b * NF + nj;
+            int rk = 0;
+            if (a.seg_cursor && lane < nc) rk = atomicAdd(&a.seg_cursor[tg], 1);
             T gs = (T)0, wx = (T)0, wy = (T)0, wz = (T)0;
             T ux = (T)0, uy = (T)0, uz = (T)0, rinv = (T)0;
             if (h < ng) {
@@ -699,11 +728,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
                 T gy = gs * uy + wy * rinv;
                 T gz = gs * uz + wz * rinv;
                 if (!valid) { gx = (T)0; gy = (T)0; gz = (T)0; }
-                if (a.seg_cursor && j < nc) {
-                    // the pair claims an entry of its target's segment (zeros too: the count of a segment
-                    // is the number of pairs naming the target)
-                    const int tg = b * NF + nj;
-                    const int rk = atomicAdd(&a.seg_cursor[tg], 1);
+                if (a.seg_cursor) {
                     T* dst = a.seg_g + (size_t)(rk < a.seg_cap ? tg * a.seg_cap + rk : a.seg_spare) * 3;
                     if (rk >= a.seg_cap) atomicOr(a.status, ST_SEG_OVERFLOW);
                     dst[0] = gx; dst[1] = gy; dst[2] = gz;
@@ -721,11 +746,11 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
         // only the threads of group 0 (inside wave 0) hold force and virial terms: the other wavefronts are done
         const double e_atom = (double)block_sum<T, NT>(e_part, gred, lane);
         if (lane >= 64) return;
-        fx = wave_sum(fx); fy = wave_sum(fy); fz = wave_sum(fz);
+        fx = wave::all_sum(fx); fy = wave::all_sum(fy); fz = wave::all_sum(fz);
         double out[10];
         out[0] = e_atom + (seeded ? 0.0 : (double)a.bias[ti]);
 #pragma unroll
-        for (int q = 0; q < 9; q++) out[1 + q] = (double)wave_sum(vir[q]);
+        for (int q = 0; q < 9; q++) out[1 + q] = (double)wave::all_sum(vir[q]);
         if (lane == 0) {
             if (!SEED || a.force) {
                 T* fo = a.force + ((size_t)b * NF + center) * 3;
@@ -792,7 +817,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const Mtp
             const int h = lane / nc, j = lane - h * nc;
             int nj; bool valid; T d[3];
             __syncthreads();
-            build_table<T, true, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+            build_table<T, TAB_GRADIENT, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
             __syncthreads();
             // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  The groups take the polynomials in
             // turn, on from one mu to the next.  (All of a thread's sums kept to the end, with one round of group sums: 100
@@ -968,8 +993,7 @@ __global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, 
     const int* first = a.bfirstneigh + row * a.U;
     const T* rcs = a.brcs + row * a.U * 3;
     for (int i = lane; i < n_basic; i += NT)
-        bas[i] = (unsigned)p.basic[i * 4] | ((unsigned)p.basic[i * 4 + 1] << 8) |
-                 ((unsigned)p.basic[i * 4 + 2] << 16) | ((unsigned)p.basic[i * 4 + 3] << 24);
+        bas[i] = p.basic[i];
     for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
     for (int i = lane; i < n_moms; i += NT) M[i] = (T)0;
     for (int i = lane; i <= p.x_nodes; i += NT) X[i] = (T)0;
@@ -982,7 +1006,7 @@ __global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, 
     for (int c0 = 0; c0 < nn; c0 += chunk) {
         const int nc = min(chunk, nn - c0);
         int nj; bool valid; T d[3];
-        build_table<T, false, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+        build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
         __syncthreads();
         for (int i = lane; i < n_basic; i += NT) {
             const unsigned bw = bas[i];
@@ -1022,7 +1046,7 @@ __global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, 
         if (nchunks > 1) {                                  // (a single chunk's table is still in place)
             int nj; bool valid; T d[3];
             __syncthreads();
-            build_table<T, false, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+            build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
             __syncthreads();
         }
         for (int j = wv; j < nc; j += NT / 64) {
@@ -1654,7 +1678,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         total += (bytes + 15) / 16 * 16;
         return off;
     };
-    const size_t o_basic = add(basic, sizeof(int) * 4 * n_basic);
+    std::vector<unsigned> basic_words(n_basic);
+    for (int i = 0; i < n_basic; i++)
+        basic_words[i] = (unsigned)basic[i * 4] | ((unsigned)basic[i * 4 + 1] << 8) | ((unsigned)basic[i * 4 + 2] << 16) |
+                         ((unsigned)basic[i * 4 + 3] << 24);
+    const size_t o_basic = add(basic_words.data(), sizeof(unsigned) * n_basic);
     const size_t o_map = add(mapping, sizeof(int) * n_scalar);
     const size_t o_fl = add(F.level.data(), sizeof(int) * F.level.size());
     const size_t o_fe = add(F.lend.data(), sizeof(int) * F.lend.size());
@@ -1711,7 +1739,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     MtpPlanDevice& d = plan->d;
     d.n_moms = n_moms; d.n_basic = n_basic; d.n_times = n_times; d.n_scalar = n_scalar;
     d.nmus = nmus; d.kmax = kmax; d.n_levels = n_levels;
-    d.basic = (const int*)(base + o_basic);
+    d.basic = (const unsigned*)(base + o_basic);
     d.mapping = (const int*)(base + o_map);
     d.f_level = (const int*)(base + o_fl); d.f_lend = (const int*)(base + o_fe);
     d.f_multi = (const int*)(base + o_fx);
@@ -1801,6 +1829,7 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     A2P_REQUIRE((long long)B * P * U < (1ll << 31), A2P_ERR_INVALID, "mtp: batch too large");
     a.p = plan->d;
     a.K = K; a.ntypes = ntypes; a.scaling = (T)scaling; a.rmax = (T)rmax; a.rmin = (T)rmin;
+    a.inv_span = (T)1 / (a.rmax - a.rmin);
     a.coeffs = coeffs; a.lin = lin; a.bias = bias; a.q_scaler = q_scaler;
     a.B = B; a.P = P; a.U = U; a.nghost = nghost;
     a.binum = binum; a.bilist = bilist; a.bnumneigh = bnumneigh; a.bfirstneigh = bfirstneigh;

@@ -27,7 +27,7 @@ struct MtpPlanDevice {
     int n_moms, n_basic, n_times, n_scalar, nmus, kmax;
     int n_levels;              // number of product levels (>= 0)
     // device arrays
-    const int* basic;          // [n_basic*4]  (mu, a, b, c)
+    const unsigned* basic;     // [n_basic]    mu | a << 8 | b << 16 | c << 24
     const int* mapping;        // [n_scalar]
     // forward gather.  A slot holds up to MTP_SLOT_CAP terms of one destination moment; a longer
     // list is cut into consecutive slots (pieces), so that no lane walks a long list alone; the pieces of a
