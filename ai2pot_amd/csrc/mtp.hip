@@ -208,8 +208,11 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
             continue;
         }
         // radial functions, basis.h:154-196, 351-381, 620-637
-        const T xx = ((T)2 * r - (a.rmax + a.rmin)) * a.inv_span, x2 = (T)2 * xx;
-        const T u = (r - a.rmin) * a.inv_span;
+        // quotients by the span: a product and one correction step, which restores the last bit
+        const T span = a.rmax - a.rmin;
+        auto over_span = [&](T v) { const T q = v * a.inv_span; return fma(fma(-q, span, v), a.inv_span, q); };
+        const T xx = over_span((T)2 * r - (a.rmax + a.rmin)), x2 = (T)2 * xx;
+        const T u = over_span(r - a.rmin);
         T s = (T)0, ds = (T)0;
         if (!(r > a.rmax) && r >= a.rmin && r < a.rmax) {
             s = a.scaling * (u * u * u * ((T)-6 * u * u + (T)15 * u - (T)10) + (T)1);
@@ -959,10 +962,31 @@ struct CompArgs {
     T* desc;                // [rows, n_scalar] scalar moments
     T* rowpart;             // [rows, 12, n_scalar] per row and column: sum of the pair derivatives (3), virial (9)
     int nc_cap, lds_basic_off;
+    int node_region;        // entries of the node adjoints' place (even)
+    int batch;              // neighbours whose D vectors are formed together (even)
+    int d_over_nodes;       // all groups of pieces are worked on at once, so the D vectors take the place of the node adjoints
 };
 
+// six values from an even entry of LDS: 16-byte reads (8-byte in single precision)
+__device__ __forceinline__ void load6(const double* p, double (&o)[6])
+{
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const double2 v = *reinterpret_cast<const double2*>(p + 2 * q);
+        o[2 * q] = v.x; o[2 * q + 1] = v.y;
+    }
+}
+__device__ __forceinline__ void load6(const float* p, float (&o)[6])
+{
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const float2 v = *reinterpret_cast<const float2*>(p + 2 * q);
+        o[2 * q] = v.x; o[2 * q + 1] = v.y;
+    }
+}
+
 template <typename T, int NT>
-__global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, const CompArgs<T> c)
+__global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> a, const CompArgs<T> c)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const MtpPlanDevice& p = a.p;
@@ -975,8 +999,8 @@ __global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, 
     const int S = p.n_scalar;
     // moments | node adjoints (+ the zero entry) | coefficients | neighbour table
     T* M = (T*)smem_raw;
-    T* X = M + n_moms;
-    T* cf = X + ((p.x_nodes + 2) & ~1);
+    T* X = M + ((n_moms + 1) & ~1);
+    T* cf = X + c.node_region;
     T* tab = cf + a.ntypes * nmus * K;
     unsigned* bas = (unsigned*)(smem_raw + c.lds_basic_off);
     const int nn = c.nnc[row];
@@ -1033,100 +1057,130 @@ __global__ void __launch_bounds__(NT) mtp_components_kernel(const MtpArgs<T> a, 
         sweep_reverse<T, false, NT>(px, M, X, (const T*)nullptr, (const T*)nullptr, lane);
     }
 
-    // Pair derivatives.  A wavefront takes a neighbour j: its lanes first form, for every basic moment, the vector
+    // Pair derivatives, four or eight neighbours at a time.  A wavefront forms, for one of them and every basic moment, the vector
     //   D_b = d(g_mu x^a y^b z^c)/dr_j = m (g' - k g / r) u + g / r grad_u m
-    // from the neighbour's table row into the wavefront's own LDS buffer; then a lane owns a column and sums
-    // adj * D_b over the column's basic ancestors (three reads and three FMAs per ancestor).  The own-row sums of the
-    // columns (force of the centre, virial) are kept per lane and added over the wavefronts at the end.
+    // in LDS; then a lane owns a piece of a column's list of basic ancestors and sums adj * D_b over it for
+    // pairs of neighbours (three 16-byte reads and six FMAs per ancestor).  The lane keeps its words and their adjoints in registers over
+    // the whole row, and sums the column's force of the centre and virial as it goes.  Up to four groups of 64 pieces are
+    // worked on at once; fewer groups share out the neighbours.
+    // What bounds it: the LDS reads of D and the latency of their chains.  With a wavefront per neighbour for every
+    // group, words and adjoints fetched again for each neighbour and the row sums read back from memory at the end, the
+    // kernel took 494 instead of 374 us at level 16, 64 structures of 128 atoms (442 with neighbours one by one and 8-byte
+    // reads, 438 with the lists ordered, 384 with pairs of neighbours and 16-byte reads, 374 with eight at a time).
     const int ngroups = p.x_slots >> 6;
-    const int l64 = lane & 63, wv = lane >> 6;
-    T* D = tab + (size_t)c.nc_cap * E + (size_t)wv * n_basic * 3;
-    for (int c0 = 0; c0 < nn; c0 += chunk) {
-        const int nc = min(chunk, nn - c0);
-        if (nchunks > 1) {                                  // (a single chunk's table is still in place)
-            int nj; bool valid; T d[3];
-            __syncthreads();
-            build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
-            __syncthreads();
-        }
-        for (int j = wv; j < nc; j += NT / 64) {
-            const T* t = tab + j * E;
-            const T ux = t[OU + 0], uy = t[OU + 1], uz = t[OU + 2], rinv = t[OU + 3];
-            __builtin_amdgcn_wave_barrier();               // the last neighbour's sums have read D
-            for (int i = l64; i < n_basic; i += 64) {
-                const unsigned bw = bas[i];
-                const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
-                const T gm = t[OG + mu], dg = t[ODG + mu];
-                const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
-                const T gs = xa * yb * zc * (dg - (T)(ea + eb + ec) * gm * rinv);
-                const T gr = gm * rinv;
-                D[i * 3 + 0] = gs * ux + gr * ((T)ea * t[OX + max(ea - 1, 0)] * yb * zc);
-                D[i * 3 + 1] = gs * uy + gr * ((T)eb * xa * t[OY + max(eb - 1, 0)] * zc);
-                D[i * 3 + 2] = gs * uz + gr * ((T)ec * xa * yb * t[OZ + max(ec - 1, 0)]);
+    const int l64 = lane & 63, wv = __builtin_amdgcn_readfirstlane(lane >> 6);
+    constexpr int NW = NT / 64;
+    const int plen = n_basic * 6 + 6;                      // D of a pair of neighbours; the last six: their displacements
+    T* D = c.d_over_nodes ? X : (T*)smem_raw + (((tab - (T*)smem_raw) + (size_t)c.nc_cap * E + 1) & ~(size_t)1);
+    const int at_once = min(ngroups, NW), shares = NW / at_once;
+    const int batch = c.batch;
+    for (int g0 = 0; g0 < ngroups; g0 += NW) {
+        const int g = g0 + wv % at_once, share = wv / at_once;
+        const bool works = share < shares && g < ngroups;   // uniform over the wavefront
+        const int depth = works ? p.x_bdepth[g] : 0, steps = works ? p.x_bsteps[g] : 0;
+        int off[MTP_SLOT_CAP], col = -1, rem = 0;
+        T adj[MTP_SLOT_CAP];
+        if (works) {
+            const int* wp = p.x_bwords + p.x_bbase[g] + l64;
+            col = p.x_seed[g * 64 + l64];
+            rem = p.x_brem[g * 64 + l64];
+#pragma unroll
+            for (int k = 0; k < MTP_SLOT_CAP; k++) off[k] = k < depth ? wp[k * 64] : 0;
+#pragma unroll
+            for (int k = 0; k < MTP_SLOT_CAP; k++) {
+                adj[k] = k < depth ? X[(unsigned)off[k] & 0xffffu] : (T)0;
+                off[k] = ((unsigned)off[k] >> 16) * 6;
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            for (int g = 0; g < ngroups; g++) {
-                const int depth = p.x_bdepth[g], steps = p.x_bsteps[g];
-                const int* wp = p.x_bwords + p.x_bbase[g] + l64;
-                const int col = p.x_seed[g * 64 + l64];
-                T gx = (T)0, gy = (T)0, gz = (T)0;
-                // all words of the slot (at most MTP_SLOT_CAP; the depth is a multiple of four and shared by the
-                // wavefront) are requested before the first is used
-                int w[MTP_SLOT_CAP];
+        }
+        T all[12];                                         // force of the centre (3), virial (9)
 #pragma unroll
-                for (int k = 0; k < MTP_SLOT_CAP; k += 4)
-                    if (k < depth) {
-#pragma unroll
-                        for (int u = 0; u < 4; u++) w[k + u] = wp[(k + u) * 64];
+        for (int i = 0; i < 12; i++) all[i] = (T)0;
+        for (int c0 = 0; c0 < nn; c0 += chunk) {
+            const int nc = min(chunk, nn - c0);
+            __syncthreads();                               // the adjoints, or the last batch of D, have been read
+            if (nchunks > 1) {                             // (a single chunk's table is still in place)
+                int nj; bool valid; T d[3];
+                build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+                __syncthreads();
+            }
+            for (int j0 = 0; j0 < nc; j0 += batch) {
+                if (j0) __syncthreads();
+                for (int jb = wv; jb < min(batch, nc - j0); jb += NW) {
+                    const int j = j0 + jb;
+                    const T* t = tab + j * E;
+                    T* Dw = D + (jb >> 1) * plen + (jb & 1) * 3;
+                    const T ux = t[OU + 0], uy = t[OU + 1], uz = t[OU + 2], rinv = t[OU + 3];
+                    for (int i = l64; i < n_basic; i += 64) {
+                        const unsigned bw = bas[i];
+                        const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
+                        const T gm = t[OG + mu], dg = t[ODG + mu];
+                        const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
+                        const T gs = xa * yb * zc * (dg - (T)(ea + eb + ec) * gm * rinv);
+                        const T gr = gm * rinv;
+                        Dw[i * 6 + 0] = gs * ux + gr * ((T)ea * t[OX + max(ea - 1, 0)] * yb * zc);
+                        Dw[i * 6 + 1] = gs * uy + gr * ((T)eb * xa * t[OY + max(eb - 1, 0)] * zc);
+                        Dw[i * 6 + 2] = gs * uz + gr * ((T)ec * xa * yb * t[OZ + max(ec - 1, 0)]);
                     }
+                    if (l64 < 3) Dw[n_basic * 6 + l64] = rcs[(c0 + j) * 3 + l64];
+                }
+                __syncthreads();
+                if (!works) continue;
+                for (int jp = share * 2; jp < min(batch, nc - j0); jp += shares * 2) {
+                    const T* Dp = D + (jp >> 1) * plen;
+                    T gr[6];
 #pragma unroll
-                for (int k = 0; k < MTP_SLOT_CAP; k += 4)
-                    if (k < depth) {
+                    for (int q = 0; q < 6; q++) gr[q] = (T)0;
 #pragma unroll
-                        for (int u = k; u < k + 4; u++) {
-                            const T adj = X[(unsigned)w[u] & 0xffffu];
-                            const T* dv = D + ((unsigned)w[u] >> 16) * 3;
-                            gx += adj * dv[0]; gy += adj * dv[1]; gz += adj * dv[2];
+                    for (int k = 0; k < MTP_SLOT_CAP; k += 2)
+                        if (k < depth) {
+#pragma unroll
+                            for (int u = k; u < k + 2; u++) {
+                                T dv[6];
+                                load6(Dp + off[u], dv);
+#pragma unroll
+                                for (int q = 0; q < 6; q++) gr[q] += adj[u] * dv[q];
+                            }
+                        }
+                    if (steps) {                            // a long list's pieces sit in neighbouring lanes
+#pragma unroll
+                        for (int q = 0; q < 6; q++) gr[q] = piece_sum(gr[q], rem, steps);
+                    }
+                    T* dst = c.pb + ((size_t)(c.pair_off[row] + c0 + j0 + jp) * 3) * S + col;
+#pragma unroll
+                    for (int o = 0; o < 2; o++) {
+                        if (j0 + jp + o >= nc) continue;    // (the other half of D is not of this row)
+                        const T* dj = Dp + n_basic * 6 + o * 3;
+#pragma unroll
+                        for (int q = 0; q < 3; q++) {
+                            all[q] += gr[o * 3 + q];
+#pragma unroll
+                            for (int i = 0; i < 3; i++) all[3 + q * 3 + i] -= gr[o * 3 + q] * dj[i];
+                            if (col >= 0) dst[(size_t)(o * 3 + q) * S] = gr[o * 3 + q];
                         }
                     }
-                if (steps) {                                // a long list's pieces sit in neighbouring lanes
-                    const int rem = p.x_brem[g * 64 + l64];
-                    gx = piece_sum(gx, rem, steps); gy = piece_sum(gy, rem, steps); gz = piece_sum(gz, rem, steps);
-                }
-                if (col >= 0) {
-                    T* dst = c.pb + ((size_t)(c.pair_off[row] + c0 + j) * 3) * S + col;
-                    dst[0] = gx;
-                    dst[S] = gy;
-                    dst[2 * S] = gz;
                 }
             }
         }
-    }
-    // own-row sums of every column (force of the centre, virial), in neighbour order, from the pair derivatives this
-    // workgroup has just written: rowpart[row][12][S]
-    __syncthreads();
-    for (int q = lane; q < S; q += NT) {
-        if (p.x_root[q] < 0) continue;                      // a column of another launch
-        T f[3] = {(T)0, (T)0, (T)0}, v[9];
+        // the shares of a group: four values of the others at a time through LDS
+        if (shares > 1) {
 #pragma unroll
-        for (int i = 0; i < 9; i++) v[i] = (T)0;
-        const T* g = c.pb + (size_t)c.pair_off[row] * 3 * S + q;
-        for (int j = 0; j < nn; j++) {
-            const T gx = g[0], gy = g[S], gz = g[2 * S];
-            const T dx = rcs[j * 3], dy = rcs[j * 3 + 1], dz = rcs[j * 3 + 2];
-            f[0] += gx; f[1] += gy; f[2] += gz;
-            v[0] -= gx * dx; v[1] -= gx * dy; v[2] -= gx * dz;
-            v[3] -= gy * dx; v[4] -= gy * dy; v[5] -= gy * dz;
-            v[6] -= gz * dx; v[7] -= gz * dy; v[8] -= gz * dz;
-            g += 3 * (size_t)S;
+            for (int q0 = 0; q0 < 12; q0 += 4) {
+                __syncthreads();
+                if (works && share > 0)
+#pragma unroll
+                    for (int q = 0; q < 4; q++) D[((wv - at_once) * 4 + q) * 64 + l64] = all[q0 + q];
+                __syncthreads();
+                if (share == 0)
+                    for (int o = wv; o < (shares - 1) * at_once; o += at_once)
+#pragma unroll
+                        for (int q = 0; q < 4; q++) all[q0 + q] += D[(o * 4 + q) * 64 + l64];
+            }
         }
-        T* o = c.rowpart + row * 12 * S + q;
+        if (works && share == 0 && col >= 0) {
+            T* o = c.rowpart + row * 12 * S + col;
 #pragma unroll
-        for (int i = 0; i < 3; i++) o[(size_t)i * S] = f[i];
-#pragma unroll
-        for (int i = 0; i < 9; i++) o[(size_t)(3 + i) * S] = v[i];
+            for (int q = 0; q < 12; q++) o[(size_t)q * S] = all[q];
+        }
     }
 }
 
@@ -1376,6 +1430,58 @@ __global__ void schmidt_orth_kernel(T* __restrict__ out, const T* __restrict__ i
 // ---- plan construction ---------------------------------------------------------------------------
 std::mutex g_plan_mutex;
 std::set<MtpPlan*> g_plans;
+
+// Order in which 16 lanes read their vectors D_b (pairs of neighbours: three 16-byte reads 48 bytes apart): lists[q] are
+// the words (node | basic << 16) of lane q, at most `depth` of them; out[k * stride + q] is the lane's word of step k, or
+// a word of the node `zero_node` where it has none.  16 lanes read from the 64 banks at a time, and lanes that name basic
+// moments of the same remainder mod 16 wait for each other unless they name the same one.  Greedy: the lanes with the
+// fewest steps to spare choose first, each the moment whose banks are least taken; the best of a few orders of the lanes
+// is kept.  (Longest waits summed over the steps at level 16: 167 as the lists come, 112 ordered, as many as steps.)
+void spread_over_banks(const std::vector<std::vector<int>>& lists, int depth, int zero_node, int* out, int stride)
+{
+    const int n = (int)lists.size();
+    long long best_cost = -1;
+    std::vector<int> best;
+    unsigned seed = 1;
+    for (int attempt = 0; attempt < 4; attempt++) {
+        std::vector<std::vector<int>> left = lists;
+        std::vector<int> words((size_t)depth * n, -1);
+        long long cost = 0;
+        for (int k = 0; k < depth; k++) {
+            std::vector<std::pair<int, int>> order;                       // (steps to spare, tie break and lane)
+            for (int q = 0; q < n; q++) {
+                seed = seed * 1664525u + 1013904223u;
+                order.push_back({depth - k - (int)left[q].size(), (int)(seed >> 20) * n + q});
+            }
+            std::sort(order.begin(), order.end());
+            std::vector<int> taken[16];
+            int most = 0, any = 0;
+            for (const auto& o : order) {
+                const int q = o.second % n;
+                int pick = -1, load = 1 << 30;
+                for (int i = 0; i < (int)left[q].size(); i++) {
+                    const int b = left[q][i] >> 16;
+                    const auto& t = taken[b % 16];
+                    const int l = std::find(t.begin(), t.end(), b) != t.end() ? 0 : (int)t.size() + 1;
+                    if (l < load) { load = l; pick = i; }
+                }
+                if (pick < 0 || (o.first > 0 && load > 1 && load > most)) continue;      // waits for a later step
+                const int w = left[q][pick];
+                left[q].erase(left[q].begin() + pick);
+                words[(size_t)k * n + q] = w;
+                any = w >> 16;
+                if (load > 0) taken[(w >> 16) % 16].push_back(w >> 16);
+                most = std::max(most, (int)taken[(w >> 16) % 16].size());
+            }
+            cost += std::max(most, 1);
+            for (int q = 0; q < n; q++)
+                if (words[(size_t)k * n + q] < 0) words[(size_t)k * n + q] = zero_node | (any << 16);
+        }
+        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = words; }
+    }
+    for (int k = 0; k < depth; k++)
+        for (int q = 0; q < n; q++) out[(size_t)k * stride + q] = best[(size_t)k * n + q];
+}
 
 int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const int* times, int n_scalar,
                 const int* mapping, MtpPlan** out)
@@ -1656,10 +1762,16 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 h.bdepth.push_back(depth);
                 h.bsteps.push_back(steps);
                 h.bwords.resize(h.bwords.size() + (size_t)depth * 64, h.nodes);       // node `nodes` (a zero), basic moment 0
+                for (int half = 0; half < 64; half += 16) {
+                    std::vector<std::vector<int>> lists(16);
+                    for (int q = 0; q < 16; q++) {
+                        const Piece& pc = pieces[g0 + half + q];
+                        if (pc.n) lists[q].assign(seed_basic[pc.s].begin() + pc.t0, seed_basic[pc.s].begin() + pc.t0 + pc.n);
+                    }
+                    spread_over_banks(lists, depth, h.nodes, &h.bwords[h.bbase.back() + half], 64);
+                }
                 for (size_t q = g0; q < g0 + 64; q++) {
                     const Piece& pc = pieces[q];
-                    for (int k = 0; k < pc.n; k++)
-                        h.bwords[h.bbase.back() + (size_t)k * 64 + (q - g0)] = seed_basic[pc.s][pc.t0 + k];
                     h.seed.push_back(pc.s >= 0 && pc.t0 == 0 ? pc.s : -1);
                     h.brem.push_back(pc.rem);
                 }
@@ -2306,17 +2418,23 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         p.x_level = xb.level; p.x_multi = xb.multi; p.x_src = xb.src; p.x_rem = xb.rem;
         p.x_gbase = xb.gbase; p.x_gdepth = xb.gdepth; p.x_terms = xb.terms;
         p.x_bbase = xb.bbase; p.x_bdepth = xb.bdepth; p.x_bsteps = xb.bsteps; p.x_brem = xb.brem; p.x_bwords = xb.bwords;
-        // LDS: moments | node adjoints | coefficients | table of nc rows | 3 n_basic values per wavefront; then the
-        // packed basic moments.  Workgroups per CU count first, then the longest table that still allows them.
+        // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 256
+        // values each); then the packed basic moments.  With at most four groups of pieces the adjoints are in registers
+        // when the first D is formed, and D takes their place (level 16: 36 instead of 46 KB).
+        // Workgroups per CU count first, then the longest table that still allows them.
+        c.batch = p.x_slots <= 128 ? 8 : 4;         // a pair of neighbours for every wavefront that shares a group
+        const int d_vals = std::max(c.batch * (3 * p.n_basic + 3), 768);
+        c.d_over_nodes = p.x_slots <= 4 * 64;
+        c.node_region = (std::max(p.x_nodes + 1, c.d_over_nodes ? d_vals : 0) + 1) & ~1;
         auto lds_for = [&](int nc, size_t* main) {
-            const size_t vals = (size_t)p.n_moms + ((p.x_nodes + 2) & ~1) + (size_t)a.ntypes * p.nmus * a.K +
-                                (size_t)nc * a.E + (size_t)4 * p.n_basic * 3;
+            const size_t vals = (size_t)((p.n_moms + 1) & ~1) + c.node_region + (size_t)a.ntypes * p.nmus * a.K +
+                                (size_t)nc * a.E + (c.d_over_nodes ? 0 : d_vals + 1);
             *main = (vals * sizeof(T) + 15) / 16 * 16;
             return *main + (size_t)p.n_basic * sizeof(unsigned);
         };
         auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
         size_t m = 0;
-        const size_t want = std::min<size_t>(per_cu(lds_for(MTP_NC_MIN, &m)), 8);
+        const size_t want = std::min<size_t>(per_cu(lds_for(MTP_NC_MIN, &m)), 4);
         A2P_REQUIRE(want >= 1, A2P_ERR_INVALID, "mtp components: %d moments need %zu bytes of LDS per atom", p.n_moms,
                     lds_for(MTP_NC_MIN, &m));
         int nc_cap = MTP_NC_MIN;

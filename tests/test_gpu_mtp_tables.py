@@ -1,0 +1,71 @@
+"""The passes over the neighbours of the moment tensor potentials where their layouts can go wrong: basic moments whose
+powers of z have gaps or occur twice, and linear-solver components for one to four groups of columns and for rows with
+few neighbours (pairs of neighbours that have no second one)."""
+import numpy as np
+import pytest
+
+from ai2pot_amd import synth
+from test_gpu_mtp import close, gpu_efv, gpu_loss, loss_inputs, model_to_device, structure
+from conftest import to_device
+
+pytestmark = pytest.mark.gpu
+
+# (mu, a, b, c): z^0 and z^2 of a row without z^1, a row without its constant, and the same moment twice
+GAPS = [(0, 0, 0, 0), (0, 0, 0, 2), (0, 1, 0, 1), (0, 1, 1, 3), (1, 0, 0, 1), (1, 0, 2, 0)]
+TWICE = GAPS[:4] + [(0, 0, 0, 2)] + GAPS[4:] + [(1, 0, 2, 0)]
+
+
+def tables(basic):
+    nb = len(basic)
+    times = [(0, 1, 2, nb), (2, 3, 1, nb), (4, 5, 1, nb + 1), (nb, nb + 1, 3, nb + 2), (nb - 1, nb - 1, 1, nb + 2)]
+    mapping = [0, 1, nb - 1, nb, nb + 2]
+    return dict(alpha_moments_count=nb + 3, alpha_index_basic=np.array(basic, np.int32),
+                alpha_index_times=np.array(times, np.int32), alpha_moment_mapping=np.array(mapping, np.int32),
+                nmus=2)
+
+
+@pytest.mark.parametrize("basic", [GAPS, TWICE], ids=["gaps", "twice"])
+def test_irregular_basic_moments(oracle, basic):
+    """Energies, forces, virials and loss gradients against the oracle: fp64, 1e-10 as for the shipped tables."""
+    nt = 2
+    nb = synth.pack_batch([structure(oracle, n, (8.5, 9.0, 9.5), nt, 21 + n, 5.0) for n in (40, 23)])
+    m = synth.mtp_model(tables(basic), nt, 6, 5.0, 1.5, 3200)
+    m["q_scaler"] = np.linspace(0.8, 1.3, m["q_scaler"].size)
+    for got, ref in zip(gpu_efv(m, nb), oracle.mtp_efv(m, nb)):
+        assert close(got, ref)
+    B, P = nb["bilist"].shape
+    labels = dict(energy=synth.rng_normal(1, B, -4 * 40, 3), force=synth.rng_normal(2, B * P * 3).reshape(B, P, 3),
+                  virial=synth.rng_normal(3, B * 9, 0, 0.5).reshape(B, 9))
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w), oracle.mtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dlinear", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
+@pytest.mark.parametrize("level", [8, 14, 16, 18])                # 1, 1, 2 and 4 groups of 64 pieces
+@pytest.mark.parametrize("U", [1, 2, 3, 9, None])
+def test_components_by_group_and_row_length(oracle, level, U):
+    """All columns from one pass against a pass per column, fp64 1e-10."""
+    from ai2pot_amd import _lib, ops
+    import torch
+    m, nb, _ = loss_inputs(oracle, level, 2, sizes=(20, 13))
+    if U is not None:
+        nb = dict(nb)
+        nb["bnumneigh"] = np.minimum(nb["bnumneigh"], U)
+        nb["bnumneigh"][0, 3] = 0
+    md = model_to_device(m, torch.float64)
+    d = to_device(nb, torch.float64)
+    args = (m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+            md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], d["binum"], d["bilist"], d["bnumneigh"],
+            d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"])
+    L = _lib.lib()
+    before = L.a2p_mtp_components_route(1)
+    try:
+        one = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+        L.a2p_mtp_components_route(0)
+        per_column = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+    finally:
+        L.a2p_mtp_components_route(before)
+    for a, b in zip(one, per_column):
+        assert np.abs(b).max() > 0
+        assert close(a, b)
