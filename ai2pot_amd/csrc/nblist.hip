@@ -143,28 +143,32 @@ __device__ __forceinline__ void atom_extremes(const Grid<T>& g, const T* __restr
     }
 }
 
+// Four workgroups per CU: beyond that a thread takes several atoms before the sums across lanes, which are what the
+// kernel waits for, and the kernel behind it has fewer values to compare
+// (1,048,576 atoms, fp32: 19.1 -> 10.9 and 13.5 -> 4.6 us with 1024 instead of 4096 workgroups).
+constexpr int MINMAX_BLOCKS = 1024;
+
 template <typename T>
 __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coords, T* __restrict__ x,
                                      T* __restrict__ partial)
 {
     __shared__ T sh[NBL_BLOCK / 64][12];
-    const int p = blockIdx.x * NBL_BLOCK + threadIdx.x;
     T v[12];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         v[a] = (T)INT_MAX; v[3 + a] = (T)INT_MIN;       // structure.h:1018-1022
         v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
     }
-    if (p < g.N) {
+    for (int p = blockIdx.x * NBL_BLOCK + threadIdx.x; p < g.N; p += gridDim.x * NBL_BLOCK) {
         T c[3], w[6];
         atom_extremes<T>(g, coords, p, c, w);
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             x[(size_t)p * 3 + a] = c[a];
-            v[a] = w[a];
-            v[3 + a] = w[3 + a];
-            v[6 + a] = c[a];
-            v[9 + a] = c[a];
+            v[a] = w[a] < v[a] ? w[a] : v[a];
+            v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
+            v[6 + a] = c[a] < v[6 + a] ? c[a] : v[6 + a];
+            v[9 + a] = c[a] > v[9 + a] ? c[a] : v[9 + a];
         }
     }
 #pragma unroll
@@ -1830,11 +1834,12 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     dim3 image_grid;
     if (!small) {
     prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(nblocks), dim3(NBL_BLOCK), 0, stream, g, coords, x,
+    const int mm_blocks = std::min(nblocks, MINMAX_BLOCKS);
+    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(mm_blocks), dim3(NBL_BLOCK), 0, stream, g, coords, x,
                        partial);
     prof_end(stream);
     prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(12 * 64), 0, stream, partial, nblocks, ext_dev);
+    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(12 * 64), 0, stream, partial, mm_blocks, ext_dev);
     prof_end(stream);
     if (sync_free) {
         for (int a = 0; a < 3; a++) {
