@@ -956,7 +956,8 @@ column_store_kernel(T* __restrict__ dst, const T* __restrict__ src, long long n,
 // latter in the fixed order of a sorted list) and per structure.
 template <typename T>
 struct CompArgs {
-    T* pb;                  // [pairs, 3, n_scalar]
+    T* pb;                  // [pairs of the structures from b0 on, 3, n_scalar]
+    int b0;                 // first structure of the launch
     const int* pair_off;    // [rows + 1] first pair of each row
     const int* nnc;         // [rows] checked neighbour count of each row (0 for rows that are not evaluated)
     T* desc;                // [rows, n_scalar] scalar moments
@@ -991,7 +992,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const MtpPlanDevice& p = a.p;
     const int lane = threadIdx.x;
-    const int ii = blockIdx.x, b = blockIdx.y;
+    const int ii = blockIdx.x, b = blockIdx.y + c.b0;
     const int NF = a.P;
     const size_t row = (size_t)b * a.P + ii;
     const int n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, kmax = p.kmax, K = a.K, E = a.E;
@@ -1009,6 +1010,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
         for (int q = lane; q < 12 * S; q += NT) c.rowpart[row * 12 * S + q] = (T)0;
         return;
     }
+    const int pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
     int center = a.bilist[row];
     if ((unsigned)center >= (unsigned)NF) center = 0;
     const int* types = a.btypes + (size_t)b * NF;
@@ -1145,7 +1147,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
 #pragma unroll
                         for (int q = 0; q < 6; q++) gr[q] = piece_sum(gr[q], rem, steps);
                     }
-                    T* dst = c.pb + ((size_t)(c.pair_off[row] + c0 + j0 + jp) * 3) * S + col;
+                    T* dst = c.pb + ((size_t)(pair0 + c0 + j0 + jp) * 3) * S + col;
 #pragma unroll
                     for (int o = 0; o < 2; o++) {
                         if (j0 + jp + o >= nc) continue;    // (the other half of D is not of this row)
@@ -1241,15 +1243,15 @@ constexpr int COMP_SORT = 256;
 
 template <typename T>
 __global__ void __launch_bounds__(64)
-comp_force_kernel(int S, int n, int cap, const int* __restrict__ row_of1, const int* __restrict__ cnt,
+comp_force_kernel(int S, int n, int cap, int row0, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
                   const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ pb,
                   const T* __restrict__ rowpart, T* __restrict__ fcomp)
 {
     __shared__ int list[COMP_SORT], order[COMP_SORT];
-    const int t = blockIdx.x, lane = threadIdx.x, col = blockIdx.y * 64 + lane, s = min(col, S - 1);
+    const int t = blockIdx.x + row0, lane = threadIdx.x, col = blockIdx.y * 64 + lane, s = min(col, S - 1);
     const int* v = inc + (seg ? (size_t)seg[t] : (size_t)t * cap);
     const int m = seg ? seg[t + 1] - seg[t] : min(cnt[t], cap);
-    const int r1 = row_of1[t];
+    const int r1 = row_of1[t], base = pair_off[row0];    // pb holds the pairs from row0 on
     const bool ranked = m <= COMP_SORT;
     if (ranked) {
         for (int k = lane; k < m; k += 64) list[k] = v[k];
@@ -1273,7 +1275,7 @@ comp_force_kernel(int S, int n, int cap, const int* __restrict__ row_of1, const 
             T g[4][3];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const T* src = pb + (size_t)order[min(k0 + u, m - 1)] * 3 * S + s;
+                const T* src = pb + (size_t)(order[min(k0 + u, m - 1)] - base) * 3 * S + s;
 #pragma unroll
                 for (int i = 0; i < 3; i++) g[u][i] = src[(size_t)i * S];
             }
@@ -1294,7 +1296,7 @@ comp_force_kernel(int S, int n, int cap, const int* __restrict__ row_of1, const 
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) next = min(next, __shfl_xor(next, off, 64));
             last = next;
-            const T* g = pb + (size_t)next * 3 * S + s;
+            const T* g = pb + (size_t)(next - base) * 3 * S + s;
 #pragma unroll
             for (int i = 0; i < 3; i++) f[i] -= g[(size_t)i * S];
         }
@@ -2412,45 +2414,58 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
     CompArgs<T> c;
     c.pb = pb; c.pair_off = pair_off; c.nnc = nnc; c.desc = desc; c.rowpart = rowpart;
     auto kern = mtp_components_kernel<T, 256>;
-    for (const MtpXBatch& xb : plan->xbatches) {
-        MtpPlanDevice& p = a.p;
-        p.x_nodes = xb.nodes; p.x_slots = xb.slots; p.x_root = xb.root; p.x_seed = xb.seed;
-        p.x_level = xb.level; p.x_multi = xb.multi; p.x_src = xb.src; p.x_rem = xb.rem;
-        p.x_gbase = xb.gbase; p.x_gdepth = xb.gdepth; p.x_terms = xb.terms;
-        p.x_bbase = xb.bbase; p.x_bdepth = xb.bdepth; p.x_bsteps = xb.bsteps; p.x_brem = xb.brem; p.x_bwords = xb.bwords;
-        // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 256
-        // values each); then the packed basic moments.  With at most four groups of pieces the adjoints are in registers
-        // when the first D is formed, and D takes their place (level 16: 36 instead of 46 KB).
-        // Workgroups per CU count first, then the longest table that still allows them.
-        c.batch = p.x_slots <= 128 ? 8 : 4;         // a pair of neighbours for every wavefront that shares a group
-        const int d_vals = std::max(c.batch * (3 * p.n_basic + 3), 768);
-        c.d_over_nodes = p.x_slots <= 4 * 64;
-        c.node_region = (std::max(p.x_nodes + 1, c.d_over_nodes ? d_vals : 0) + 1) & ~1;
-        auto lds_for = [&](int nc, size_t* main) {
-            const size_t vals = (size_t)((p.n_moms + 1) & ~1) + c.node_region + (size_t)a.ntypes * p.nmus * a.K +
-                                (size_t)nc * a.E + (c.d_over_nodes ? 0 : d_vals + 1);
-            *main = (vals * sizeof(T) + 15) / 16 * 16;
-            return *main + (size_t)p.n_basic * sizeof(unsigned);
-        };
-        auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
-        size_t m = 0;
-        const size_t want = std::min<size_t>(per_cu(lds_for(MTP_NC_MIN, &m)), 4);
-        A2P_REQUIRE(want >= 1, A2P_ERR_INVALID, "mtp components: %d moments need %zu bytes of LDS per atom", p.n_moms,
-                    lds_for(MTP_NC_MIN, &m));
-        int nc_cap = MTP_NC_MIN;
-        for (int nc : {MTP_NC_MAX, 40, 32, 24, 20, MTP_NC_MIN})
-            if (per_cu(lds_for(nc, &m)) >= want) { nc_cap = nc; break; }
-        const size_t lds = lds_for(nc_cap, &m);
-        c.nc_cap = nc_cap; c.lds_basic_off = (int)m;
-        if (lds > 48 * 1024)
-            A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        prof_begin("mtp_components_kernel", stream);
-        hipLaunchKernelGGL(kern, dim3(P, B), dim3(256), lds, stream, a, c);
+    // The pair derivatives are written once and read once: structures are taken in chunks whose derivatives fit the
+    // memory-side cache (256 MB) with what is read beside them, as long as a chunk fills the chip twice.  Level 16, 64
+    // structures of 128 atoms, 390 MB: kernel + sums 370 + 124 us in one piece, 391 + 83 in two, 411 + 88 in four.
+    const long long pair_bytes = (long long)npairs * 3 * S * (long long)sizeof(T);
+    const int parts = (int)std::min<long long>(ceil_div(pair_bytes, 200ll << 20), std::max(1, rows / 2048));
+    const int per = ceil_div(B, std::max(parts, 1));
+    for (int b0 = 0; b0 < B; b0 += per) {
+        const int nb = std::min(per, B - b0);
+        c.b0 = b0;
+        for (const MtpXBatch& xb : plan->xbatches) {
+            MtpPlanDevice& p = a.p;
+            p.x_nodes = xb.nodes; p.x_slots = xb.slots; p.x_root = xb.root; p.x_seed = xb.seed;
+            p.x_level = xb.level; p.x_multi = xb.multi; p.x_src = xb.src; p.x_rem = xb.rem;
+            p.x_gbase = xb.gbase; p.x_gdepth = xb.gdepth; p.x_terms = xb.terms;
+            p.x_bbase = xb.bbase; p.x_bdepth = xb.bdepth; p.x_bsteps = xb.bsteps; p.x_brem = xb.brem; p.x_bwords = xb.bwords;
+            // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 256
+            // values each); then the packed basic moments.  With at most four groups of pieces the adjoints are in registers
+            // when the first D is formed, and D takes their place (level 16: 36 instead of 46 KB).
+            // Workgroups per CU count first, then the longest table that still allows them.
+            c.batch = p.x_slots <= 128 ? 8 : 4;         // a pair of neighbours for every wavefront that shares a group
+            const int d_vals = std::max(c.batch * (3 * p.n_basic + 3), 768);
+            c.d_over_nodes = p.x_slots <= 4 * 64;
+            c.node_region = (std::max(p.x_nodes + 1, c.d_over_nodes ? d_vals : 0) + 1) & ~1;
+            auto lds_for = [&](int nc, size_t* main) {
+                const size_t vals = (size_t)((p.n_moms + 1) & ~1) + c.node_region + (size_t)a.ntypes * p.nmus * a.K +
+                                    (size_t)nc * a.E + (c.d_over_nodes ? 0 : d_vals + 1);
+                *main = (vals * sizeof(T) + 15) / 16 * 16;
+                return *main + (size_t)p.n_basic * sizeof(unsigned);
+            };
+            auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
+            size_t m = 0;
+            const size_t want = std::min<size_t>(per_cu(lds_for(MTP_NC_MIN, &m)), 4);
+            A2P_REQUIRE(want >= 1, A2P_ERR_INVALID, "mtp components: %d moments need %zu bytes of LDS per atom", p.n_moms,
+                        lds_for(MTP_NC_MIN, &m));
+            int nc_cap = MTP_NC_MIN;
+            for (int nc : {MTP_NC_MAX, 40, 32, 24, 20, MTP_NC_MIN})
+                if (per_cu(lds_for(nc, &m)) >= want) { nc_cap = nc; break; }
+            const size_t lds = lds_for(nc_cap, &m);
+            c.nc_cap = nc_cap; c.lds_basic_off = (int)m;
+            if (lds > 48 * 1024)
+                A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            prof_begin("mtp_components_kernel", stream);
+            hipLaunchKernelGGL(kern, dim3(P, nb), dim3(256), lds, stream, a, c);
+            prof_end(stream);
+        }
+        prof_begin("mtp_components_sums", stream);
+        hipLaunchKernelGGL(comp_force_kernel<T>, dim3(nb * P, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, b0 * P,
+                           (const int*)pair_off, (const int*)row_of1,
+                           (const int*)cnt, in_seg, (const int*)inc, (const T*)pb, (const T*)rowpart, fcomp);
         prof_end(stream);
     }
     prof_begin("mtp_components_sums", stream);
-    hipLaunchKernelGGL(comp_force_kernel<T>, dim3(rows, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, (const int*)row_of1,
-                       (const int*)cnt, in_seg, (const int*)inc, (const T*)pb, (const T*)rowpart, fcomp);
     const int nblocks = ceil_div(P, COMP_ROWS);
     void* wsP = nullptr;
     rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * n * sizeof(T), &wsP);

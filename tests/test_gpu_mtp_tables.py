@@ -69,3 +69,27 @@ def test_components_by_group_and_row_length(oracle, level, U):
     for a, b in zip(one, per_column):
         assert np.abs(b).max() > 0
         assert close(a, b)
+
+
+def test_components_in_chunks_of_structures(oracle):
+    """Enough pair derivatives (level 16: 92 columns, more than 200 MB) that the structures are taken in chunks, the last
+    one shorter: every structure equal to the call with that structure alone, bit for bit, in force columns too."""
+    from ai2pot_amd import ops
+    import torch
+    m, nb, _ = loss_inputs(oracle, 16, 2, sizes=(48,))
+    md = model_to_device(m, torch.float64)
+    d = to_device(nb, torch.float64)
+    n, B = int(nb["binum"][0]), 91
+    keys = ("binum", "bilist", "bnumneigh", "bfirstneigh", "brcs", "btypes")
+    assert nb["bnumneigh"].sum() * B * 3 * m["q_scaler"].size * 8 > (200 << 20) and n * B >= 4096
+
+    def components(t):
+        return ops.mtp_lin_components(
+            m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+            md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], t["binum"], t["bilist"], t["bnumneigh"],
+            t["bfirstneigh"], t["brcs"], t["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"])
+
+    batch = {k: d[k].expand(B, *d[k].shape[1:]).contiguous() for k in keys}
+    alone = components(d)
+    for whole, one in zip(components(batch), alone):
+        assert torch.equal(whole, one.expand_as(whole))
