@@ -486,12 +486,12 @@ __device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __re
     Q *= wu;
 }
 
-// NT threads per centre atom: 64 for small tables, 256 when there is enough work per atom
-// (four workgroups of 256 threads fit the LDS of a CU at the larger levels: keep the registers to match)
+// NT threads per centre atom: 64 or 256 (wide_atoms).  Five workgroups of 256 threads fit the LDS of a CU at level 20 and
+// the registers are kept to match (four: 321 us instead of 303 at 8192 atoms; six spill: 361).
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
 // (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.
 template <typename T, bool LOSS, int NT, bool SEED = false>
-__global__ void __launch_bounds__(NT, (!LOSS ? 4 : 1)) mtp_atom_kernel(const MtpArgs<T> a)
+__global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_atom_kernel(const MtpArgs<T> a)
 {
     const bool seeded = (SEED || LOSS) && a.row_seed != nullptr;
     const bool no_tan = LOSS && a.no_tangent != 0;      // uniform over the launch
@@ -1437,52 +1437,45 @@ std::set<MtpPlan*> g_plans;
 // the words (node | basic << 16) of lane q, at most `depth` of them; out[k * stride + q] is the lane's word of step k, or
 // a word of the node `zero_node` where it has none.  16 lanes read from the 64 banks at a time, and lanes that name basic
 // moments of the same remainder mod 16 wait for each other unless they name the same one.  Greedy: the lanes with the
-// fewest steps to spare choose first, each the moment whose banks are least taken; the best of a few orders of the lanes
-// is kept.  (Longest waits summed over the steps at level 16: 167 as the lists come, 112 ordered, as many as steps.)
+// fewest steps to spare choose first, each the moment whose banks are least taken.  (Longest waits summed over the steps
+// at level 16: 185 as the lists come, 114 ordered; there are 112 steps.)
 void spread_over_banks(const std::vector<std::vector<int>>& lists, int depth, int zero_node, int* out, int stride)
 {
-    const int n = (int)lists.size();
-    long long best_cost = -1;
-    std::vector<int> best;
-    unsigned seed = 1;
-    for (int attempt = 0; attempt < 4; attempt++) {
-        std::vector<std::vector<int>> left = lists;
-        std::vector<int> words((size_t)depth * n, -1);
-        long long cost = 0;
-        for (int k = 0; k < depth; k++) {
-            std::vector<std::pair<int, int>> order;                       // (steps to spare, tie break and lane)
-            for (int q = 0; q < n; q++) {
-                seed = seed * 1664525u + 1013904223u;
-                order.push_back({depth - k - (int)left[q].size(), (int)(seed >> 20) * n + q});
-            }
-            std::sort(order.begin(), order.end());
-            std::vector<int> taken[16];
-            int most = 0, any = 0;
-            for (const auto& o : order) {
-                const int q = o.second % n;
-                int pick = -1, load = 1 << 30;
-                for (int i = 0; i < (int)left[q].size(); i++) {
-                    const int b = left[q][i] >> 16;
-                    const auto& t = taken[b % 16];
-                    const int l = std::find(t.begin(), t.end(), b) != t.end() ? 0 : (int)t.size() + 1;
-                    if (l < load) { load = l; pick = i; }
-                }
-                if (pick < 0 || (o.first > 0 && load > 1 && load > most)) continue;      // waits for a later step
-                const int w = left[q][pick];
-                left[q].erase(left[q].begin() + pick);
-                words[(size_t)k * n + q] = w;
-                any = w >> 16;
-                if (load > 0) taken[(w >> 16) % 16].push_back(w >> 16);
-                most = std::max(most, (int)taken[(w >> 16) % 16].size());
-            }
-            cost += std::max(most, 1);
-            for (int q = 0; q < n; q++)
-                if (words[(size_t)k * n + q] < 0) words[(size_t)k * n + q] = zero_node | (any << 16);
-        }
-        if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = words; }
+    constexpr int LANES = 16;
+    int left[LANES][MTP_SLOT_CAP], count[LANES];
+    for (int q = 0; q < LANES; q++) {
+        count[q] = (int)lists[q].size();
+        std::copy(lists[q].begin(), lists[q].end(), left[q]);
     }
-    for (int k = 0; k < depth; k++)
-        for (int q = 0; q < n; q++) out[(size_t)k * stride + q] = best[(size_t)k * n + q];
+    for (int k = 0; k < depth; k++) {
+        int order[LANES];                               // lanes by the steps they have to spare
+        for (int q = 0; q < LANES; q++) {
+            int at = q;
+            for (; at > 0 && count[order[at - 1]] < count[q]; at--) order[at] = order[at - 1];
+            order[at] = q;
+        }
+        int taken[LANES][LANES], ntaken[LANES] = {0}, most = 0, any = 0;
+        bool waits[LANES] = {false};
+        for (int o = 0; o < LANES; o++) {
+            const int q = order[o];
+            int pick = -1, load = 1 << 30;
+            for (int i = 0; i < count[q] && load > 0; i++) {
+                const int b = left[q][i] >> 16, bank = b % LANES;
+                const bool same = std::find(taken[bank], taken[bank] + ntaken[bank], b) != taken[bank] + ntaken[bank];
+                const int l = same ? 0 : ntaken[bank] + 1;
+                if (l < load) { load = l; pick = i; }
+            }
+            if (pick < 0 || (depth - k > count[q] && load > 1 && load > most)) { waits[q] = true; continue; }
+            const int w = left[q][pick], bank = (w >> 16) % LANES;
+            left[q][pick] = left[q][--count[q]];
+            out[(size_t)k * stride + q] = w;
+            any = w >> 16;
+            if (load > 0) taken[bank][ntaken[bank]++] = w >> 16;
+            most = std::max(most, ntaken[bank]);
+        }
+        for (int q = 0; q < LANES; q++)
+            if (waits[q]) out[(size_t)k * stride + q] = zero_node | (any << 16);
+    }
 }
 
 int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const int* times, int n_scalar,
@@ -1963,6 +1956,22 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
 
 int g_keep_table = 1;      // (measurement switch: AI2POT_MTP_KEEP_TABLE=0)
 
+// 256 threads per atom or 64: a rule on the tables alone, so that a structure's results do not depend on the batch it is
+// in (the sums over neighbours are grouped by the threads).  Kernel times in us, 64 / 256 threads, fp64, energy / force /
+// virial (8,000 atoms; 250 atoms) and loss gradient (8,000; 250):
+//   level 8 (18 moments)   44 / 106   15.5 / 16.3   132 / 172   36 / 38
+//   level 10 (41)          49 / 113   19.0 / 17.5   185 / 188   39 / 41
+//   level 12 (84)          56 / 121   19.0 / 17.5   203 / 200   42 / 43
+//   level 14 (174)         82 / 130   28 / 19       301 / 249   53 / 47
+//   level 16 (350)        109 / 148   35 / 20       (loss: 256 threads before)
+//   level 18 (718)        194 / 183
+// With a network the loss gradient has a weight per neuron and scalar moment besides (64 x 125 atoms; 2 x 60; 30 neurons):
+//   level 8  221 / 211 (10 neurons: 170 / 186)   46 / 40      level 10  273 / 230   51 / 44      level 12  304 / 247   56 / 46
+inline bool wide_atoms(int n_moms, bool loss, bool network)
+{
+    return n_moms >= (loss ? (network ? 40 : 150) : 600);
+}
+
 template <typename T, bool LOSS, bool SEED = false>
 int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
 {
@@ -1970,7 +1979,7 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         static const char* e = getenv("AI2POT_MTP_KEEP_TABLE");
         if (e) g_keep_table = e[0] != '0';
     }
-    const bool wide = a.p.n_moms >= (LOSS ? 300 : 1000);   // enough work per atom to keep 256 threads busy
+    const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0);
     auto lds_for = [&](int nc, size_t* main, bool keep = false) {
         *main = (lds_bytes<T>(a.p, a.E, LOSS, a.ntypes, a.K, a.H, nc, wide ? 256 : 64, keep) + 15) / 16 * 16;
         // the packed basic-moment table and the polynomials, with the monomial rows or the run of every mu
@@ -1982,13 +1991,13 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
     // Rows of the neighbour table (energy / force / virial kernel; the loss kernels keep MTP_NC): the kernel waits on
     // dependent LDS reads and barriers, so workgroups per CU count first (level 16: 12 -> 16 workgroups, 0.136 -> 0.122 ms
     // although rows of more than 20 neighbours then take two chunks), and among the tables that allow as many
-    // workgroups as the registers do (four waves per SIMD), or as the shortest table does, the longest is taken
+    // workgroups as the registers do (four or five waves per SIMD), or as the shortest table does, the longest is taken
     // (level 20: a row of 35 neighbours in one chunk instead of two, 0.45 -> 0.41 ms).
     if (!LOSS) {
         // LDS is handed out in pieces of 1280 bytes on this chip
         auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
         size_t m = 0;
-        const size_t by_registers = wide ? 4 : 16;
+        const size_t by_registers = wide ? 5 : 16;
         const size_t want = std::min(by_registers, per_cu(lds_for(MTP_NC_MIN, &m)));
         for (int nc : {MTP_NC_MAX, 40, 32, 24, 20, MTP_NC_MIN}) {
             const size_t l = lds_for(nc, &m);
