@@ -633,7 +633,7 @@ def run_nep_train(args):
 
 def run_mtp_solver(args):
     """The normal equations of the linear parameters (LinMatrixLinVectorOp) on configuration 4's structures, level
-    16: the components of all 92 scalar moments from one pass over the atoms, plus three Gram products by the BLAS."""
+    16: the components of all 92 scalar moments from one pass over the atoms, plus the three Gram products."""
     import torch
     from ai2pot_amd import _lib, ops, synth
     dev = torch.device("cuda:0")
