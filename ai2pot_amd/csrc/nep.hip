@@ -443,7 +443,9 @@ int launch(const NepArgs<T>& a, size_t lds, hipStream_t stream)
 // A wavefront per atom costs more instructions in all, but its chain is short and a few thousand atoms fill the chip; a
 // thread per atom takes the same time from one atom to as many as there are lanes.  Measured (6 radial, l_max 4, 60
 // neighbours; wavefront / staged, whole operator): fp32 8,000 atoms 69 / 166 us, 32,000 145 / 179, 45,000 188 / 193,
-// 64,000 244 / 218; fp64 8,000 98 / 227, 24,000 203 / 238, 32,000 257 / 242.
+// 64,000 244 / 218; fp64 8,000 98 / 227, 24,000 203 / 238, 32,000 257 / 242.  The thread's chain grows with the row, the
+// wavefront's work hardly does up to 64 neighbours, so the line moves with the length of the rows, which the host does not
+// know: 16 neighbours 22,000 atoms (fp64 17,000), 24: 28,000 (20,000), 36: 36,000 (28,000), 52: 42,000 (32,000).
 template <typename T>
 constexpr long long wave_most() { return sizeof(T) == 4 ? 40960 : 28672; }
 
