@@ -446,7 +446,7 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
 // axis when the lattice is diagonal and an axis has at most three images, else one by one.  What the grid turned out to be goes to the host while the rest runs; a box or image count
 // beyond the LDS empties the lists and is reported, and the host then takes the general route.
 constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 11264, NBS_IMAGES = 15360;
-constexpr int NBS_AXIS = 254;                     // bins per axis: a bin is a byte, 255 marks an image outside the box
+constexpr int NBS_AXIS = 256;                     // bins per axis: a bin is a byte
 constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_IMAGES * 6;
 
 constexpr int NBS_ATOM_BITS = 12, NBS_TRIPLES = 256;
@@ -1747,6 +1747,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             images *= std::min((double)g.img_dim[a], n * (double)g.bin_size / len);
         }
         small = small && bins < NBS_BINS && (!separable || images <= NBS_IMAGES);
+        // without a read-back the box may grow to its bound: every box within it has to keep its bins a byte wide
+        for (int a = 0; a < 3 && sync_free; a++) small = small && cap[a] <= NBS_AXIS;
     }
     // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
     // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;

@@ -77,3 +77,38 @@ def test_atoms_outside_the_cell(oracle, dt):
         pass
     args = (lat, ty, (f * L).astype(dt), 5.0, 120)
     assert_same(gpu_list(*args), oracle.nblist(*args))            # still usable
+
+
+def sync_free_builds(oracle, lat, ty, xs, rcut, umax, pbc=(True, True, True)):
+    """A synchronised build of xs[0], then builds of the others that do not read the extents back: each against the
+    oracle, with nothing flagged."""
+    import torch
+    from ai2pot_amd import _lib, nblist
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    lib = _lib.lib()
+    for k, x in enumerate(xs):
+        before = lib.a2p_nblist_sync_free(1 if k else 0)
+        try:
+            out = nblist.find_info4mlff_device(lat, d(ty), d(x), rcut, umax, True, pbc, False, check=False)
+            _lib.check_status(torch.cuda.current_stream().cuda_stream)
+        finally:
+            lib.a2p_nblist_sync_free(before)
+        got = tuple(o.cpu().numpy() if hasattr(o, "cpu") else o for o in out)
+        assert_same(got, oracle.nblist(lat, ty, x, rcut, umax, pbc=pbc))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("beyond", [24, 30])
+def test_wire_whose_box_grows_past_a_byte(oracle, dt, beyond):
+    """A wire of 220 bins with one atom `beyond` bins outside it in the synchronised build and up to 21 bins further out
+    afterwards (within the eighth that the box may grow by): boxes of up to 280 bins along the axis."""
+    n, bin_size = 900, 2.5
+    lat = np.diag([220 * bin_size, 2.4, 2.4]).astype(dt)
+    x = np.stack([np.sort(synth.rng_uniform(5, n)) * lat[0, 0], *(2.4 * synth.rng_uniform(6, 2 * n).reshape(2, n))], 1)
+    ty = synth.rng_randint(7, n, 2)
+    xs = []
+    for more in (0, 2, 12, 21):
+        y = x.copy()
+        y[n // 2, 0] = (220 + beyond + more) * bin_size
+        xs.append(y.astype(dt))
+    sync_free_builds(oracle, lat, ty, xs, 2 * bin_size, 60, pbc=(True, False, False))
