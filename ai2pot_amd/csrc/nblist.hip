@@ -443,9 +443,12 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
 // 4096 atoms, of which 38 in kernels; 29 us here, and 11 us for 108 atoms).  One workgroup of 1024 threads does the same with its counters in
 // LDS: extents, grid, counts, prefix sum, image numbers dealt to their bins, and every record written once, to its final
 // place (an image's place in its bin is the number of larger image numbers there).  The images of an atom are found per
-// axis when the lattice is diagonal and an axis has at most three images, else one by one.  What the grid turned out to be goes to the host while the rest runs; a box or image count
-// beyond the LDS empties the lists and is reported, and the host then takes the general route.
-constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 11264, NBS_IMAGES = 15360;
+// axis when the lattice is diagonal and an axis has at most three images, else one by one.  Images beyond the LDS (atoms
+// crowded into a corner of the cell are within reach of eight cells each) pass through global memory instead.  What the
+// grid turned out to be goes to the host while the rest runs; a box beyond the LDS empties the lists and is reported, and
+// the host then takes the general route.
+// (bins: a cube of 21, grown by the two that a build without a read-back allows for)
+constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 12288, NBS_IMAGES = 15360;
 constexpr int NBS_AXIS = 256;                     // bins per axis: a bin is a byte
 constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_IMAGES * 6;
 
@@ -468,7 +471,7 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
                   int* __restrict__ offsets, T* __restrict__ s_rec, const int* __restrict__ types, int* __restrict__ ilist,
                   int* __restrict__ types_out, int* __restrict__ incoming, int mark_types, int separable, int cap0, int cap1,
                   int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq,
-                  unsigned* __restrict__ axis_images)
+                  unsigned* __restrict__ axis_images, int* __restrict__ spare, int spare_images)
 {
     extern __shared__ __align__(16) unsigned char sh_small[];
     int* const cnt = (int*)sh_small;                             // per bin: count, then end of the bin's records
@@ -543,13 +546,15 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     // 2. counts, 3. prefix sum, 4. image numbers to their bins.  One copy of the code that enumerates the images serves
     // both passes: it runs once or a few times per call, so fetching instructions is a good part of what it costs.
     int total = 0;
+    bool in_lds = true;                                          // uniform
 #pragma unroll 1
     for (int pass = 0; pass < 2 && ok; pass++) {
         auto image = [&](int im, int p, int b) __attribute__((always_inline)) {
             const int pos = atomicAdd(&cnt[b], 1);
             if (pass) {
-                num[pos] = im << NBS_ATOM_BITS | p;              // ordered as the supercell index im * N + p
-                bin_of_num[pos] = (unsigned short)b;
+                const int m = im << NBS_ATOM_BITS | p;           // ordered as the supercell index im * N + p
+                if (in_lds) { num[pos] = m; bin_of_num[pos] = (unsigned short)b; }
+                else { spare[pos] = m; spare[spare_images + pos] = b; }
             }
         };
         // the bin along axis a of the image that is i cells along it, or -1 outside the box (separable: the other axes'
@@ -641,7 +646,8 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
             run += w < wv ? t : 0;
             total += t;
         }
-        ok = total <= NBS_IMAGES;                                // uniform
+        in_lds = total <= NBS_IMAGES;
+        ok = in_lds || total <= spare_images;                    // uniform
         for (int b = b0; b < b1; b++) {
             const int n = cnt[b];
             cnt[b] = run;
@@ -672,23 +678,27 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     // 5. records in descending image number within a bin (head insertion, binLinkedList.h:833), as binsort_kernel leaves
     // them.  Shifts and a table stand in for the five integer divisions a record would take.
     const int central = ((-g.img_lo[0]) * g.img_dim[1] + (-g.img_lo[1])) * g.img_dim[2] + (-g.img_lo[2]);
+    auto records = [&](const auto* numbers, const auto* bins) __attribute__((always_inline)) {
 #pragma unroll 1
-    for (int e = tid; e < total; e += NBS_THREADS) {
-        const int b = bin_of_num[e], m = num[e];
-        const int im = m >> NBS_ATOM_BITS, p = m & ((1 << NBS_ATOM_BITS) - 1);
-        const unsigned t = im < NBS_TRIPLES ? sh_triple[im] : image_triple(g, im);
-        const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
-        const int beg = b > 0 ? cnt[b - 1] : 0, end = cnt[b];
-        int place = beg;
-        for (int q = beg; q < end; q++) place += num[q] > m ? 1 : 0;
-        T ci[3];
+        for (int e = tid; e < total; e += NBS_THREADS) {
+            const int b = bins[e], m = numbers[e];
+            const int im = m >> NBS_ATOM_BITS, p = m & ((1 << NBS_ATOM_BITS) - 1);
+            const unsigned t = im < NBS_TRIPLES ? sh_triple[im] : image_triple(g, im);
+            const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+            const int beg = b > 0 ? cnt[b - 1] : 0, end = cnt[b];
+            int place = beg;
+            for (int q = beg; q < end; q++) place += numbers[q] > m ? 1 : 0;
+            T ci[3];
 #pragma unroll
-        for (int a = 0; a < 3; a++)
-            ci[a] = image_coord(xp[a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + (int)(t & 1023u),
-                                g.img_lo[1] + (int)((t >> 10) & 1023u), g.img_lo[2] + (int)(t >> 20));
-        entry_store<T>(s_rec + (size_t)place * 4, ci[0], ci[1], ci[2],
-                       mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
-    }
+            for (int a = 0; a < 3; a++)
+                ci[a] = image_coord(xp[a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + (int)(t & 1023u),
+                                    g.img_lo[1] + (int)((t >> 10) & 1023u), g.img_lo[2] + (int)(t >> 20));
+            entry_store<T>(s_rec + (size_t)place * 4, ci[0], ci[1], ci[2],
+                           mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
+        }
+    };
+    if (in_lds) records(num, bin_of_num);
+    else records(spare, spare + spare_images);
 }
 
 // ---- processing order of the compact lists: atoms along a Morton curve through the bins ----------
@@ -1747,8 +1757,10 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             images *= std::min((double)g.img_dim[a], n * (double)g.bin_size / len);
         }
         small = small && bins < NBS_BINS && (!separable || images <= NBS_IMAGES);
-        // without a read-back the box may grow to its bound: every box within it has to keep its bins a byte wide
+        // without a read-back the box may grow to its bound: every box within it has to keep its bins a byte wide and
+        // its counters in LDS
         for (int a = 0; a < 3 && sync_free; a++) small = small && cap[a] <= NBS_AXIS;
+        if (sync_free) small = small && (long long)cap[0] * cap[1] * cap[2] < NBS_BINS;
     }
     // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
     // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;
@@ -1791,18 +1803,22 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     GridDyn<T>* gd = nullptr;
     int* offsets = nullptr;
     long long total = 0;
+    int spare_images = 0;                               // images the one-workgroup binning has room for in global memory
     if (small) {
         posted = !sync_free;
         void* wsG = nullptr;
         rc = ws_get(WS_GRID, 256, &wsG);
-        if (rc == A2P_OK) rc = ws_get(WS_NBL_B, (NBS_BINS + 1) * sizeof(int), (void**)&offsets);
+        // one by one there are at most NBS_IMAGES images; told by axis, every one of them may be in reach
+        spare_images = separable && (long long)N * g.nimg > NBS_IMAGES ? N * g.nimg : 0;
+        if (rc == A2P_OK)
+            rc = ws_get(WS_NBL_B, ((size_t)NBS_BINS + 1 + 2 * (size_t)spare_images) * sizeof(int), (void**)&offsets);
         gd = (GridDyn<T>*)wsG;
-        total = NBS_IMAGES;
+        total = std::max(NBS_IMAGES, spare_images);
     }
 
     if (small && rc == A2P_OK) {
         void* wsC0 = nullptr;
-        rc = ws_get(WS_MISC, (size_t)NBS_IMAGES * 4 * sizeof(T) + 256 + sort_bytes, &wsC0);
+        rc = ws_get(WS_MISC, (size_t)total * 4 * sizeof(T) + 256 + sort_bytes, &wsC0);
         static std::atomic<unsigned long long> lds_set{0};          // devices on which the kernel may use its LDS
         if (rc == A2P_OK && (device > 63 || !(lds_set.load() & (1ull << device)))) {
             if (hipFuncSetAttribute((const void*)small_bins_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -1815,7 +1831,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             hipLaunchKernelGGL(small_bins_kernel<T>, dim3(1), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x, gd, offsets,
                                (T*)wsC0, types, want_rows ? ilist : (int*)nullptr, types_out, incoming, co ? 1 : 0,
                                separable ? 1 : 0, cap[0], cap[1], cap[2], bound_of_coords, sync_free ? 1 : 0, status,
-                               posted ? post_slot : nullptr, post.seq, axis_images);
+                               posted ? post_slot : nullptr, post.seq, axis_images, offsets + NBS_BINS + 1, spare_images);
             prof_end(stream);
             if (hipGetLastError() != hipSuccess) rc = A2P_ERR_HIP;
         }

@@ -112,3 +112,51 @@ def test_wire_whose_box_grows_past_a_byte(oracle, dt, beyond):
         y[n // 2, 0] = (220 + beyond + more) * bin_size
         xs.append(y.astype(dt))
     sync_free_builds(oracle, lat, ty, xs, 2 * bin_size, 60, pbc=(True, False, False))
+
+
+def growing_boxes(n, outside):
+    """Cell, cutoff and positions whose boxes grow within the eighth: 16 bins along an axis, and an atom outside the cell."""
+    L, f = jittered(n, n, density=0.045, shape=(1.0, 1.0, 1.0))
+    bin_size = L[0] / 15.9
+    x = f * L
+    far = np.argmax(x.sum(1))
+    x[far] = L + outside * bin_size
+    spread = x.copy()
+    spread[far] += 1.9 * bin_size
+    # crowded around the origin, where eight cells meet and every atom has eight images in reach
+    corner = np.where(x < 0.5 * L, 0.45 * x, L - 0.45 * (L - x))
+    return L, 2.0 * bin_size, [x, 0.999 * x, spread, corner, x]
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [2300, 4096])
+@pytest.mark.parametrize("outside", [-1.1, 0.9])
+def test_sync_free_box_grown_by_an_eighth(oracle, dt, n, outside):
+    """Atoms that spread or crowd together within the box of the synchronised build and its eighth: boxes of more bins, and
+    more images, than one workgroup holds in LDS are binned all the same."""
+    L, rcut, xs = growing_boxes(n, outside)
+    sync_free_builds(oracle, np.diag(L).astype(dt), synth.rng_randint(n, n, 2), [x.astype(dt) for x in xs], rcut, 1200)
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_more_images_than_lds(oracle, dt):
+    """The same crowd of 4096 atoms (26,000 images) in synchronised builds: plain, sorted and in compact lists' records."""
+    import torch
+    from ai2pot_amd.calculator import NepCalculator
+    L, rcut, xs = growing_boxes(4096, -1.1)
+    lat, ty, x = np.diag(L).astype(dt), synth.rng_randint(9, 4096, 2), xs[3].astype(dt)
+    for sort in (False, True):
+        assert_same(gpu_list(lat, ty, x, rcut, 600, sort=sort), oracle.nblist(lat, ty, x, rcut, 600, sort=sort))
+    m = synth.nep_model(rmax_radial=rcut, rmax_angular=0.7 * rcut)
+    kw = dict(umax=400, dtype=torch.float32 if dt == np.float32 else torch.float64)
+    if dt == np.float32:
+        gather = NepCalculator(m, 4096, lat, ty, path="gather", **kw)
+        rows = NepCalculator(m, 4096, lat, ty, path="segments", **kw)
+        d = torch.from_numpy(x).to("cuda:0")
+        e, f, v = gather.step(d)
+        gather.check()
+        e0, f0, v0 = rows.step(d)
+        rows.check()
+        # 400 terms a row, of either sign: two summation orders in single precision
+        for a, b in ((e, e0), (f, f0), (v, v0)):
+            assert (a - b).abs().max() <= 1e-5 * b.abs().max()
