@@ -1750,6 +1750,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     if (small) {
         double bins = 1, images = N;
         for (int a = 0; a < 3; a++) {
+            small = small && g.img_dim[a] <= 1024;      // image_triple has ten bits for an axis
             const double len = std::fabs((double)g.b[0][a]) + std::fabs((double)g.b[1][a]) + std::fabs((double)g.b[2][a]);
             const double n = std::ceil(len / (double)g.bin_size) + 2 + 2 * g.ext_bins;
             small = small && n <= NBS_AXIS;

@@ -160,3 +160,16 @@ def test_more_images_than_lds(oracle, dt):
         # 400 terms a row, of either sign: two summation orders in single precision
         for a, b in ((e, e0), (f, f0), (v, v0)):
             assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("axis", [0, 1, 2])
+@pytest.mark.parametrize("spacing", [0.005, 0.0059])
+def test_more_than_a_thousand_images_along_an_axis(oracle, dt, axis, spacing):
+    """One atom in a cell far shorter than the cutoff: 1201 and 1019 images along the axis, ten bits' worth on either side."""
+    lat = np.diag([20.0, 18.0, 22.0])
+    lat[axis, axis] = spacing
+    x = np.array([[0.1, 0.2, 0.3]])
+    pbc = [a == axis for a in range(3)]
+    args = (lat.astype(dt), np.zeros(1, np.int32), x.astype(dt), 3.0, 1300)
+    assert_same(gpu_list(*args, pbc=pbc), oracle.nblist(*args, pbc=pbc))
