@@ -281,10 +281,12 @@ inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tenso
         total += n;
     }
     const int np = (int)shape.size();
-    // a backward pass that is itself differentiated (in grad_output) goes through operators autograd knows
-    if (B == 0 || (at::GradMode::is_enabled() && gl.requires_grad())) {
+    // a backward pass that is itself differentiated (in grad_output, either way) or mapped over a batch of gradients, whose
+    // tensors wrap others and have no storage of their own, goes through operators that know of it
+    if (B == 0 || !gl.has_storage() || gl._fw_grad(/*level=*/0).defined() ||
+        (at::GradMode::is_enabled() && gl.requires_grad())) {
         for (int64_t i = 0, beg = 0; i < np; beg += numel[i] * B, i++)
-            out[first + i] = torch::matmul(gl, flat.narrow(0, beg, numel[i] * B).view({B, (int64_t)numel[i]})).view(shape[i]);
+            out[first + i] = torch::matmul(gl, flat.narrow(0, beg, numel[i] * B).view({B, (int64_t)numel[i]})).reshape(shape[i]);
         return;
     }
     DeviceGuard guard(flat);

@@ -90,3 +90,34 @@ def test_bad_index_is_raised_by_the_call_itself(oracle):
         with pytest.raises(RuntimeError, match="neighbour index"):
             call(bad)
         assert torch.equal(call()[0].detach(), want)            # nothing is left behind for the next call
+
+
+def test_gradients_of_a_batch_of_weights(oracle):
+    """is_grads_batched hands the backward pass one wrapped tensor for all weight vectors: the Jacobian of the
+    per-structure losses in one pass, and any other batch of weights."""
+    import torch
+    call, par, nb = _loss(oracle, torch.float64)
+    one = [torch.autograd.grad(call()[0][k], par) for k in range(3)]
+    w = torch.tensor([[1.0, 0.0, 0.0], [0.0, 1.0, 0.0], [0.0, 0.0, 1.0], [0.3, -1.1, 0.7]], dtype=torch.float64, device="cuda:0")
+    got = torch.autograd.grad(call()[0], par, w, is_grads_batched=True)
+    for i, g in enumerate(got):
+        assert g.shape == (4,) + tuple(par[i].shape)
+        want = torch.einsum("kb,b...->k...", w, torch.stack([o[i] for o in one]))
+        # a product of three terms in another order
+        assert torch.allclose(g, want, rtol=1e-13, atol=1e-15 * float(want.abs().max()))
+
+
+def test_forward_derivative_of_the_gradient(oracle):
+    """A weight vector with a tangent: the gradients carry the tangent's own gradients (they are linear in the weights)."""
+    import torch
+    import torch.autograd.forward_ad as fwad
+    call, par, nb = _loss(oracle, torch.float64)
+    w, t = (torch.tensor(v, dtype=torch.float64, device="cuda:0") for v in ([0.3, -1.1, 0.7], [1.5, 0.2, -0.4]))
+    want, want_t = (torch.autograd.grad(call()[0], par, v) for v in (w, t))
+    with fwad.dual_level():
+        got = [fwad.unpack_dual(g) for g in torch.autograd.grad(call()[0], par, fwad.make_dual(w, t))]
+        got = [(g.primal.clone(), None if g.tangent is None else g.tangent.clone()) for g in got]
+    for (p, d), a, b in zip(got, want, want_t):
+        assert d is not None
+        assert torch.allclose(p, a, rtol=1e-13, atol=1e-15 * float(a.abs().max()))
+        assert torch.allclose(d, b, rtol=1e-13, atol=1e-15 * float(b.abs().max()))
