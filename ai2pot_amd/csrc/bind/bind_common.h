@@ -272,13 +272,11 @@ inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tenso
     const at::Tensor gl = grad_output.defined() ? grad_output.contiguous() : at::zeros({B}, flat.options());
     std::vector<std::vector<int64_t>> shape;
     std::vector<long long> numel;
-    long long total = 0;
     for (size_t i = 0; i < shapes.size(); i += 1 + shapes[i]) {
         shape.emplace_back(shapes.begin() + i + 1, shapes.begin() + i + 1 + shapes[i]);
         long long n = 1;
         for (int64_t d : shape.back()) n *= d;
         numel.push_back(n);
-        total += n;
     }
     const int np = (int)shape.size();
     // a backward pass that is itself differentiated (in grad_output, either way) or mapped over a batch of gradients, whose
@@ -290,20 +288,27 @@ inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tenso
         return;
     }
     DeviceGuard guard(flat);
-    const at::Tensor sums = at::empty({(int64_t)total}, flat.options());
+    for (int i = 0; i < np; i++) out[first + i] = at::empty(shape[i], flat.options());
     void* st = current_stream(flat);
     int rc;
     if (flat.scalar_type() == at::kDouble) {
         std::vector<const double*> parts;
-        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) parts.push_back(flat.data_ptr<double>() + beg);
-        rc = a2p_weighted_rows_f64((int)B, gl.data_ptr<double>(), np, parts.data(), numel.data(), sums.data_ptr<double>(), st);
+        std::vector<double*> outs;
+        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) {
+            parts.push_back(flat.data_ptr<double>() + beg);
+            outs.push_back(out[first + i].data_ptr<double>());
+        }
+        rc = a2p_weighted_rows_split_f64((int)B, gl.data_ptr<double>(), np, parts.data(), numel.data(), outs.data(), st);
     } else {
         std::vector<const float*> parts;
-        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) parts.push_back(flat.data_ptr<float>() + beg);
-        rc = a2p_weighted_rows_f32((int)B, gl.data_ptr<float>(), np, parts.data(), numel.data(), sums.data_ptr<float>(), st);
+        std::vector<float*> outs;
+        for (long long i = 0, beg = 0; i < np; beg += numel[i] * B, i++) {
+            parts.push_back(flat.data_ptr<float>() + beg);
+            outs.push_back(out[first + i].data_ptr<float>());
+        }
+        rc = a2p_weighted_rows_split_f32((int)B, gl.data_ptr<float>(), np, parts.data(), numel.data(), outs.data(), st);
     }
     check_rc(rc);
-    for (int64_t i = 0, beg = 0; i < np; beg += numel[i], i++) out[first + i] = piece(sums, beg, shape[i]);
 }
 
 // Labels of a loss operator with the ZBL pair repulsion taken out.  The correction does not depend

@@ -479,23 +479,25 @@ constexpr int WR_PARTS = 8;
 template <typename T>
 struct WeightedRows {
     const T* part[WR_PARTS];
-    long long beg[WR_PARTS + 1];       // first element of each part in out
+    T* out[WR_PARTS];
+    long long beg[WR_PARTS + 1];       // where each part begins among the elements of all
     int nparts;
 };
 template <typename T>
 __global__ void __launch_bounds__(256)
-weighted_rows_kernel(int B, const T* __restrict__ w, const WeightedRows<T> a, T* __restrict__ out)
+weighted_rows_kernel(int B, const T* __restrict__ w, const WeightedRows<T> a)
 {
     __shared__ double red[4][64];
     const int lane = threadIdx.x & 63, run = threadIdx.x >> 6;
     const long long e = (long long)blockIdx.x * 64 + lane, total = a.beg[a.nparts];
     double acc = 0.0;
+    T* dst = a.out[0] + e;
     if (e < total) {
         const T* src = a.part[0];
         long long beg = 0, n = a.beg[1];
 #pragma unroll
         for (int p = 1; p < WR_PARTS; p++)
-            if (p < a.nparts && e >= a.beg[p]) { src = a.part[p]; beg = a.beg[p]; n = a.beg[p + 1] - beg; }
+            if (p < a.nparts && e >= a.beg[p]) { src = a.part[p]; beg = a.beg[p]; n = a.beg[p + 1] - beg; dst = a.out[p] + (e - beg); }
         src += e - beg;
         const int len = (B + 3) / 4, b1 = min(B, (run + 1) * len);
         for (int b0 = run * len; b0 < b1; b0 += 8) {
@@ -509,31 +511,44 @@ weighted_rows_kernel(int B, const T* __restrict__ w, const WeightedRows<T> a, T*
     }
     red[run][lane] = acc;
     __syncthreads();
-    if (run == 0 && e < total) out[e] = (T)(((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
+    if (run == 0 && e < total) *dst = (T)(((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
 }
 
 template <typename T>
-int weighted_rows(int B, const T* w, int nparts, const T* const* parts, const long long* sizes, T* out, hipStream_t stream)
+int weighted_rows(int B, const T* w, int nparts, const T* const* parts, const long long* sizes, T* const* outs,
+                  hipStream_t stream)
 {
-    A2P_REQUIRE(B >= 1 && nparts >= 1 && nparts <= WR_PARTS && w && parts && sizes && out, A2P_ERR_INVALID,
+    A2P_REQUIRE(B >= 1 && nparts >= 1 && nparts <= WR_PARTS && w && parts && sizes && outs, A2P_ERR_INVALID,
                 "weighted_rows: need a batch, 1 to %d parts and non-null pointers", WR_PARTS);
     WeightedRows<T> a;
     a.nparts = nparts;
     a.beg[0] = 0;
     for (int p = 0; p < WR_PARTS; p++) {
         const bool have = p < nparts;
-        A2P_REQUIRE(!have || (parts[p] && sizes[p] >= 0), A2P_ERR_INVALID, "weighted_rows: part %d", p);
+        A2P_REQUIRE(!have || (parts[p] && sizes[p] >= 0 && (outs[p] || sizes[p] == 0)), A2P_ERR_INVALID, "weighted_rows: part %d", p);
         a.part[p] = have ? parts[p] : nullptr;
+        a.out[p] = have ? outs[p] : nullptr;
         a.beg[p + 1] = a.beg[p] + (have ? sizes[p] : 0);
     }
     const long long total = a.beg[nparts];
     if (total == 0) return A2P_OK;
     A2P_REQUIRE(total < (1ll << 36), A2P_ERR_INVALID, "weighted_rows: too many elements");
     prof_begin("weighted_rows", stream);
-    hipLaunchKernelGGL(weighted_rows_kernel<T>, dim3(ceil_div(total, 64)), dim3(256), 0, stream, B, w, a, out);
+    hipLaunchKernelGGL(weighted_rows_kernel<T>, dim3(ceil_div(total, 64)), dim3(256), 0, stream, B, w, a);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
+}
+
+// the results behind one another
+template <typename T>
+int weighted_rows_joined(int B, const T* w, int nparts, const T* const* parts, const long long* sizes, T* out, hipStream_t stream)
+{
+    A2P_REQUIRE(nparts >= 1 && nparts <= WR_PARTS && sizes && out, A2P_ERR_INVALID,
+                "weighted_rows: need 1 to %d parts and non-null pointers", WR_PARTS);
+    T* outs[WR_PARTS];
+    for (int p = 0; p < nparts; p++) { outs[p] = out; out += std::max(sizes[p], 0ll); }
+    return weighted_rows<T>(B, w, nparts, parts, sizes, outs, stream);
 }
 
 }  // namespace a2p
@@ -543,13 +558,25 @@ extern "C" {
 int a2p_weighted_rows_f32(int batch, const float* w, int nparts, const float* const* parts, const long long* sizes,
                           float* out, void* stream)
 {
-    return a2p::weighted_rows<float>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+    return a2p::weighted_rows_joined<float>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+}
+
+int a2p_weighted_rows_split_f32(int batch, const float* w, int nparts, const float* const* parts, const long long* sizes,
+                                float* const* outs, void* stream)
+{
+    return a2p::weighted_rows<float>(batch, w, nparts, parts, sizes, outs, (hipStream_t)stream);
 }
 
 int a2p_weighted_rows_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
                           double* out, void* stream)
 {
-    return a2p::weighted_rows<double>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+    return a2p::weighted_rows_joined<double>(batch, w, nparts, parts, sizes, out, (hipStream_t)stream);
+}
+
+int a2p_weighted_rows_split_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
+                                double* const* outs, void* stream)
+{
+    return a2p::weighted_rows<double>(batch, w, nparts, parts, sizes, outs, (hipStream_t)stream);
 }
 
 const char* a2p_last_error(void) { return a2p::last_error(); }

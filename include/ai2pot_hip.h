@@ -68,6 +68,11 @@ int a2p_weighted_rows_f32(int batch, const float* w, int nparts, const float* co
                           float* out, void* stream);
 int a2p_weighted_rows_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
                           double* out, void* stream);
+/* the same with a device pointer for each part's result (`outs`, a host array) */
+int a2p_weighted_rows_split_f32(int batch, const float* w, int nparts, const float* const* parts, const long long* sizes,
+                                float* const* outs, void* stream);
+int a2p_weighted_rows_split_f64(int batch, const double* w, int nparts, const double* const* parts, const long long* sizes,
+                                double* const* outs, void* stream);
 
 /* Per-kernel timing for benchmarks (no counterpart in the reference, which leaves timing to
  * commented-out std::chrono calls, interface/lammps/AI2POT/pair_ai2pot.cpp:392-442).  While

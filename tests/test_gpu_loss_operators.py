@@ -36,6 +36,13 @@ def test_weighted_rows(dtype, B, sizes):
     eps = np.finfo(dtype).eps
     bound = torch.cat([(w.double().abs()[:, None] * p.double().abs()).sum(0) for p in parts]) * B * 2.3e-16 + want.abs() * eps
     assert bool(((out[:-1].double() - want).abs() <= bound).all()) and float(out[-1]) == 7.0
+    # results in places of their own: the same bits, and nothing beside them
+    outs = [torch.full((n + 1,), 7.0, device="cuda:0", dtype=dt) for n in sizes]
+    fn = L.a2p_weighted_rows_split_f32 if dtype == "float32" else L.a2p_weighted_rows_split_f64
+    dst = (ctypes.c_void_p * len(sizes))(*[o.data_ptr() for o in outs])
+    _lib.check(fn(ctypes.c_int(B), ctypes.c_void_p(w.data_ptr()), ctypes.c_int(len(sizes)), ptr, num, dst,
+                  ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert torch.equal(torch.cat([o[:-1] for o in outs]), out[:-1]) and all(float(o[-1]) == 7.0 for o in outs)
 
 
 def _loss(oracle, dtype):
@@ -121,3 +128,14 @@ def test_forward_derivative_of_the_gradient(oracle):
         assert d is not None
         assert torch.allclose(p, a, rtol=1e-13, atol=1e-15 * float(a.abs().max()))
         assert torch.allclose(d, b, rtol=1e-13, atol=1e-15 * float(b.abs().max()))
+
+
+def test_gradients_are_tensors_of_their_own(oracle):
+    """Each gradient has its own storage, no larger than it is: kept or saved alone it keeps nothing else."""
+    import torch
+    call, par, nb = _loss(oracle, torch.float64)
+    grads = torch.autograd.grad(call()[0].sum(), par)
+    assert len({g.untyped_storage().data_ptr() for g in grads}) == len(grads)
+    for g, p in zip(grads, par):
+        assert g.shape == p.shape and g.is_contiguous() and g.data_ptr() % 256 == 0
+        assert g.untyped_storage().nbytes() == g.numel() * g.element_size()
