@@ -97,6 +97,14 @@ __device__ __forceinline__ void read_back_store(int* slot, int seq, const int* w
 // Called where every check of the call's inputs has been queued: posts the status word if the calling thread asked
 // for it (a2p_status_early).
 int status_post_early(hipStream_t stream);
+// The same for a call whose own check is all that is asked for: its kernel stores a non-zero value to the word of pinned
+// memory that early_word gives (null: nothing was asked for, or no slot is free; the latter is *no_slot), and
+// early_word_post, behind that kernel, ends the report.  The shared status word is left alone.  early_word_known reports
+// what the host found by itself, early_word_drop gives the word back when the kernel was not launched.
+int* early_word(hipStream_t stream, bool* no_slot);
+int early_word_post(hipStream_t stream);
+void early_word_known(int word);
+void early_word_drop();
 
 inline int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 

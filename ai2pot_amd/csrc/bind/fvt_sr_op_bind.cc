@@ -208,7 +208,8 @@ TORCH_LIBRARY(fvt, m)
                           "brcs must match bdei_drij in dtype and device");
               check_device_int(dei, bnumneigh, "bnumneigh");
               TORCH_CHECK(bnumneigh.numel() == dei.size(0) * dei.size(1), "bnumneigh must have shape [B, nlocal]");
-              // the kernel reports a row that is too long; with validation off its status word is left alone
+              // the kernel reports a row that is too long to this call alone: the device's status word, which may hold what
+              // an earlier call without validation found, is neither read nor cleared
               const char* too_long = "a neighbour count exceeds umax_num_neighs";
               const bool any = bnumneigh.numel() > 0;
               if (any && !validate_flag()) TORCH_CHECK(bnumneigh.max().item<int>() <= umax, too_long);

@@ -279,8 +279,46 @@ int read_back(const void* device_src, int nwords, void* host_dst, hipStream_t st
 // of the call runs: see a2p_status_early.
 namespace {
 thread_local bool g_early_asked = false, g_early_posted = false;
+thread_local bool g_early_own = false;     // the posted word is the call's own (early_word), not the shared status word
+thread_local int g_early_known = 0;        // ... and its value, where there is no slot to wait for
 thread_local ReadBack g_early;
+
+__global__ void early_word_kernel(int* slot, int seq)
+{
+    if (threadIdx.x == 0) __hip_atomic_store(slot, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 }  // namespace
+
+int* early_word(hipStream_t stream, bool* no_slot)
+{
+    *no_slot = false;
+    if (!g_early_asked || g_early_posted) return nullptr;
+    int* const slot = read_back_take(1, stream, &g_early);
+    *no_slot = slot == nullptr;
+    if (!slot) return nullptr;
+    __atomic_store_n(slot + 1, 0, __ATOMIC_RELAXED);
+    return slot + 1;
+}
+
+int early_word_post(hipStream_t stream)
+{
+    // (kernels of a stream run in order, and what the one before stored to host memory is there when it has ended)
+    hipLaunchKernelGGL(early_word_kernel, dim3(1), dim3(64), 0, stream, g_rb_page + g_early.slot * RB_WORDS, g_early.seq);
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess) read_back_drop(g_early);
+    A2P_HIP_CHECK(err);
+    g_early_posted = g_early_own = true;
+    return A2P_OK;
+}
+
+void early_word_known(int word)
+{
+    g_early_known = word;
+    g_early.slot = -1;
+    g_early_posted = g_early_own = true;
+}
+
+void early_word_drop() { read_back_drop(g_early); }
 
 int status_post_early(hipStream_t stream)
 {
@@ -658,8 +696,8 @@ void a2p_status_early(int on)
 {
     if (a2p::g_early_posted) {          // left over from a call that failed: its slot is free once the word has arrived
         int word;
-        (void)a2p::read_back_wait(a2p::g_early, &word);
-        a2p::g_early_posted = false;
+        if (!a2p::g_early_own || a2p::g_early.slot >= 0) (void)a2p::read_back_wait(a2p::g_early, &word);
+        a2p::g_early_posted = a2p::g_early_own = false;
     }
     a2p::g_early_asked = on != 0;
 }
@@ -670,11 +708,16 @@ int a2p_check_status_early(void* stream_)
         a2p::g_early_asked = false;
         return a2p_check_status(stream_);
     }
-    int host = 0;
-    const int rc = a2p::read_back_wait(a2p::g_early, &host);
-    a2p::g_early_asked = a2p::g_early_posted = false;
+    const bool own = a2p::g_early_own;
+    int host = a2p::g_early_known;
+    const int rc = own && a2p::g_early.slot < 0 ? A2P_OK : a2p::read_back_wait(a2p::g_early, &host);
+    a2p::g_early_asked = a2p::g_early_posted = a2p::g_early_own = false;
     if (rc) return rc;
     if (host == 0) return A2P_OK;
+    if (own) {
+        a2p::set_error("a neighbour count exceeds umax_num_neigh_atoms");
+        return A2P_ERR_OVERFLOW;
+    }
     return a2p_check_status(stream_);   // behind the whole call: the word is cleared with nothing of the call to come
 }
 

@@ -13,6 +13,7 @@
 #include "a2p_common.h"
 
 #include <mutex>
+#include <vector>
 
 namespace a2p {
 namespace {
@@ -48,16 +49,17 @@ force_bwd_kernel(T* __restrict__ gout, const T* __restrict__ gF, int B, int P, i
     }
 }
 
-// one wavefront per row -> 9 partial sums per row (fp64), reduced by finish_partials
+// one wavefront per row -> 9 partial sums per row (fp64), reduced by finish_partials; too_long (a word of host memory)
+// is set when a row claims more than U neighbours
 template <typename T>
 __global__ void __launch_bounds__(256)
 virial_rows_kernel(double* __restrict__ partial, const T* __restrict__ g, const T* __restrict__ r, int B,
-                   int P, int U, const int* __restrict__ bnumneigh, int* __restrict__ status)
+                   int P, int U, const int* __restrict__ bnumneigh, int* too_long)
 {
     const int row = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (row >= B * P) return;
     const int nn = min(bnumneigh[row], U);
-    if (status && lane == 0 && bnumneigh[row] > U) atomicOr(status, ST_NEIGH_OVERFLOW);
+    if (too_long && lane == 0 && bnumneigh[row] > U) __hip_atomic_store(too_long, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const T* gr = g + (size_t)row * U * 3;
     const T* rr = r + (size_t)row * U * 3;
     double v[9];
@@ -150,18 +152,26 @@ int virial_fwd(int B, int P, int U, const int* bnumneigh, const T* rcs, const T*
     if (B == 0) return A2P_OK;
     if (P == 0) return fill_zero(virial, (size_t)B * 9 * sizeof(T), stream);
     void* ws = nullptr;
-    rc = ws_get(WS_FLAGS, 64, &ws);
-    if (rc) return rc;
-    int* const status = (int*)ws;
     rc = ws_get(WS_PARTIAL, (size_t)B * P * 9 * sizeof(double), &ws);
     if (rc) return rc;
+    bool no_slot = false;
+    int* const too_long = early_word(stream, &no_slot);
     prof_begin("fvt_virial_rows", stream);
     hipLaunchKernelGGL(virial_rows_kernel<T>, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
-                       (double*)ws, dei, rcs, B, P, U, bnumneigh, status);
+                       (double*)ws, dei, rcs, B, P, U, bnumneigh, too_long);
     prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
-    rc = status_post_early(stream);
-    if (rc) return rc;
+    const hipError_t err = hipGetLastError();
+    if (err != hipSuccess && too_long) early_word_drop();
+    A2P_HIP_CHECK(err);
+    if (too_long) {
+        rc = early_word_post(stream);
+        if (rc) return rc;
+    } else if (no_slot) {                    // more calls waiting than there are slots
+        std::vector<int> nn((size_t)B * P);
+        A2P_HIP_CHECK(hipMemcpyAsync(nn.data(), bnumneigh, nn.size() * sizeof(int), hipMemcpyDeviceToHost, stream));
+        A2P_HIP_CHECK(hipStreamSynchronize(stream));
+        early_word_known(*std::max_element(nn.begin(), nn.end()) > U ? 1 : 0);
+    }
     return finish_partials<T>(virial, (const double*)ws, B, P, 9, 9, 9, stream);
 }
 

@@ -56,7 +56,9 @@ int a2p_check_status(void* stream);
 /* The same for the loss entry points, whose first kernels make every check: a2p_status_early(1) before such a call
  * sends the status word to the host behind those kernels, and a2p_check_status_early after it waits for that word
  * only, while the gradient kernels of the call may still run (a raised bit is then confirmed by a2p_check_status behind
- * the whole call).  Per host thread, for one call; after a call of another kind it is a2p_check_status. */
+ * the whole call).  After a2p_fvt_virial_fwd_* it is that call's own check (A2P_OK, or A2P_ERR_OVERFLOW for a row of more
+ * than umax neighbours), and the status word stays as it was.  Per host thread, for one call; after a call of another kind
+ * it is a2p_check_status. */
 void a2p_status_early(int on);
 int a2p_check_status_early(void* stream);
 

@@ -112,3 +112,43 @@ def test_errors():
         ops.ForceSrOp(dev(binum), dev(bilist), dev(nn), dev(fn), 4, U + 1, dev(dei))
     with pytest.raises(RuntimeError):
         ops.VirialSrOp(dev(nn), dev(rcs).float(), U, dev(dei))
+
+
+def test_virial_reports_its_own_rows_only():
+    """A row that is too long raises in the call that was given it.  What an earlier call without validation left in the
+    device's status word is not this operator's: it neither raises for it nor takes it away."""
+    import os
+    import torch
+    libdir = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ai2pot_amd", "_lib")
+    torch.ops.load_library(os.path.join(libdir, "libfvt_sr_op_bind.so"))
+    fvt = torch.ops.fvt
+    binum, bilist, nn, fn, dei, rcs = random_case()
+    U = fn.shape[2]
+    bad, longer = fn.copy(), nn.copy()
+    bad[:, :, 0], longer[1, 2] = 999, U + 1
+    good = lambda: fvt.VirialSrOp(dev(nn), dev(rcs), U, dev(dei))[0]
+    force = lambda f: fvt.ForceSrOp(dev(binum), dev(bilist), dev(nn), dev(f), 4, U, dev(dei))[0]
+    want = good()
+    for pending in (False, True):
+        if pending:
+            fvt.set_validate(False)
+            try:
+                force(bad)                                      # leaves its finding for whoever asks
+            finally:
+                fvt.set_validate(True)
+        assert torch.equal(good(), want)
+        with pytest.raises(RuntimeError, match="neighbour count exceeds"):
+            fvt.VirialSrOp(dev(longer), dev(rcs), U, dev(dei))
+        assert torch.equal(good(), want)
+        if pending:
+            with pytest.raises(RuntimeError, match="neighbour index"):
+                fvt.check_status(want)
+        fvt.check_status(want)
+    fvt.set_validate(False)
+    try:
+        with pytest.raises(RuntimeError, match="neighbour count exceeds"):
+            fvt.VirialSrOp(dev(longer), dev(rcs), U, dev(dei))
+        assert torch.equal(good(), want)
+    finally:
+        fvt.set_validate(True)
+    fvt.check_status(want)
