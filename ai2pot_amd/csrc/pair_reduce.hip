@@ -3,10 +3,11 @@
 // neighbour is j  on top of the sum over its own row that the producing kernel stored.
 //
 // Steps (all on `stream`):
-//   1. clear  : a cursor per target, the overflow count (and the caller's force array)
+//   1. clear  : a cursor and the heads of sixteen chains per target (and the caller's force array)
 //   2. claim  : every pair takes an entry of its target's segment (a returning integer atomic; the order inside a
 //               segment is therefore arbitrary) and leaves its number there.  Segments hold as many pairs as a row: a
-//               list built with one cutoff never needs more, and what does not fit goes to one list for all targets
+//               list built with one cutoff never needs more.  What does not fit (half lists, ghosts that collect the pairs
+//               of several rows) is chained behind the target, its pairs dealt to the sixteen chains in turn
 //   3. reduce : per target, order-independent sum over the pairs named: every term is converted to 64-bit fixed
 //               point against the segment's largest magnitude, integers are added (exact,
 //               associative), the total is converted back.  The result is identical for
@@ -127,13 +128,19 @@ __global__ void scan_apply(const int* __restrict__ in, int* __restrict__ out,
     }
 }
 
+// Chains of a target that is named by more pairs than a row holds: one for each lane that sums it, so that a chain's
+// dependent loads are a sixteenth of what ran over.  Force of 50,000 rows of 32 neighbours, fp64, whole operator: 231 us
+// where every segment fits, 328 where an eighth of the atoms collects all pairs (7/8 of them chained), 10 ms where one atom
+// collects the pairs of 6,250 rows.
+constexpr int SPILL_CHAINS = 16;
+
 // Claims of step 2, one wavefront per row.  With OWN the wavefront also sums the row itself and stores it as the force
 // on the row's centre (a centre has one row).
 template <typename T, bool OWN>
 __global__ void __launch_bounds__(256)
 claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum, const int* __restrict__ bilist,
              const int* __restrict__ bnumneigh, const int* __restrict__ bfirstneigh, const T* __restrict__ pair_g,
-             int* __restrict__ cursor, int* __restrict__ seg, int2* __restrict__ spill, int* __restrict__ nspill,
+             int* __restrict__ cursor, int* __restrict__ seg, int* __restrict__ heads, int* __restrict__ next,
              T* __restrict__ force, int* __restrict__ status)
 {
     const int row = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
@@ -157,8 +164,9 @@ claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum
         }
         const int t = b * NF + j;
         const int k = atomicAdd(&cursor[t], 1);
-        if (k < cap) seg[(size_t)t * cap + k] = row * U + s;
-        else spill[atomicAdd(nspill, 1)] = make_int2(t, row * U + s);      // at most one entry per pair
+        const int pair = row * U + s;
+        if (k < cap) seg[(size_t)t * cap + k] = pair;
+        else next[pair] = atomicExch(&heads[(size_t)t * SPILL_CHAINS + (k - cap) % SPILL_CHAINS], pair + 1);   // 0 ends a chain
     }
     if (OWN) {
         sx = wave_sum(sx); sy = wave_sum(sy); sz = wave_sum(sz);
@@ -179,7 +187,7 @@ claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum
 template <typename T, bool NAMED>
 __global__ void __launch_bounds__(256)
 reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __restrict__ counts, int NT, int seg_cap,
-              const int* __restrict__ seg_pair, const int2* __restrict__ spill, const int* __restrict__ nspill,
+              const int* __restrict__ seg_pair, const int* __restrict__ heads, const int* __restrict__ next,
               int reduce_blocks, T* __restrict__ etot, T* __restrict__ virial, const double* __restrict__ partial,
               int nblocks)
 {
@@ -199,15 +207,12 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __r
     auto entry = [&](int e) __attribute__((always_inline)) -> const T* {
         return seg_g + (NAMED ? (size_t)seg_pair[beg + e] : beg + e) * 3;
     };
-    // calls f on every entry beyond the four in registers: the rest of the segment, then the target's pairs among
-    // those that did not fit (a scan of the whole list; no list built with one cutoff gets here)
+    // calls f on every entry beyond the four in registers: the rest of the segment, then this lane's chain of those that
+    // did not fit
     auto others = [&](auto&& f) __attribute__((always_inline)) {
         for (int e = sub + 64; e < cnt; e += 16) f(entry(e));
-        if (NAMED && all > seg_cap) {
-            const int n = *nspill;
-            for (int i = sub; i < n; i += 16)
-                if (spill[i].x == t) f(seg_g + (size_t)spill[i].y * 3);
-        }
+        if (NAMED && all > seg_cap)
+            for (int e = heads[(size_t)t * SPILL_CHAINS + sub]; e > 0; e = next[e - 1]) f(seg_g + (size_t)(e - 1) * 3);
     };
     T gx[4], gy[4], gz[4];
 #pragma unroll
@@ -399,7 +404,7 @@ int pair_csr_finish(T* force, const PairCsr& csr, hipStream_t stream, T* etot, T
     prof_begin("reduce_sum", stream);
     hipLaunchKernelGGL((reduce_kernel<T, false>), dim3(reduce_blocks + ev_blocks), dim3(256), 0, stream,
                        force, (const T*)csr.seg_g, (const int*)csr.cursor, csr.n, csr.seg_cap, (const int*)nullptr,
-                       (const int2*)nullptr, (const int*)nullptr, reduce_blocks, etot, virial, partial, nblocks);
+                       (const int*)nullptr, (const int*)nullptr, reduce_blocks, etot, virial, partial, nblocks);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
@@ -414,25 +419,26 @@ int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, cons
     A2P_REQUIRE(NT < (1ll << 31) - 1 && rows * U < (1ll << 31), A2P_ERR_INVALID,
                 "pair_reduce: batch too large for 32-bit pair indexing");
     const int n = (int)NT;
-    // workspace: cursor[n] | nspill[1] | seg[n*U] | spill[rows*U] (8 bytes each)
-    const size_t head = (((size_t)n + 1) * sizeof(int) + 255) / 256 * 256;
+    // workspace: cursor[n] | heads[n*16] | seg[n*U] | next[rows*U] (by pair)
+    const size_t clear_bytes = (size_t)n * (1 + SPILL_CHAINS) * sizeof(int);
+    const size_t head = (clear_bytes + 255) / 256 * 256;
     const size_t seg_bytes = ((size_t)n * U * sizeof(int) + 255) / 256 * 256;
     void* ws = nullptr;
-    int rc = ws_get(WS_CSR, head + seg_bytes + (size_t)rows * U * sizeof(int2), &ws);
+    int rc = ws_get(WS_CSR, head + seg_bytes + (size_t)rows * U * sizeof(int), &ws);
     if (rc) return rc;
     int* cursor = (int*)ws;
-    int* nspill = cursor + n;
+    int* heads = cursor + n;
     int* seg = (int*)((char*)ws + head);
-    int2* spill = (int2*)((char*)ws + head + seg_bytes);
+    int* next = (int*)((char*)ws + head + seg_bytes);
     rc = ws_get(WS_FLAGS, 64, &ws);
     if (rc) return rc;
     // own: the rows' own sums are formed here, and atoms without a row start from zero
-    rc = fill_zero2(cursor, ((size_t)n + 1) * sizeof(int), own ? (void*)force : nullptr, own ? (size_t)n * 3 * sizeof(T) : 0,
+    rc = fill_zero2(cursor, clear_bytes, own ? (void*)force : nullptr, own ? (size_t)n * 3 * sizeof(T) : 0,
                     stream);
     if (rc) return rc;
     prof_begin("reduce_claim", stream);
     hipLaunchKernelGGL((own ? claim_kernel<T, true> : claim_kernel<T, false>), dim3(ceil_div(rows * 64, 256)), dim3(256), 0,
-                       stream, B, P, U, NF, U, binum, bilist, bnumneigh, bfirstneigh, pair_g, cursor, seg, spill, nspill,
+                       stream, B, P, U, NF, U, binum, bilist, bnumneigh, bfirstneigh, pair_g, cursor, seg, heads, next,
                        force, (int*)ws);
     prof_end(stream);
     rc = status_post_early(stream);
@@ -440,7 +446,7 @@ int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, cons
     const int reduce_blocks = ceil_div((long long)n * 16, 256);
     prof_begin("reduce_sum", stream);
     hipLaunchKernelGGL((reduce_kernel<T, true>), dim3(reduce_blocks), dim3(256), 0, stream, force, pair_g,
-                       (const int*)cursor, n, U, (const int*)seg, (const int2*)spill, (const int*)nspill, reduce_blocks,
+                       (const int*)cursor, n, U, (const int*)seg, (const int*)heads, (const int*)next, reduce_blocks,
                        (T*)nullptr, (T*)nullptr, (const double*)nullptr, 0);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
