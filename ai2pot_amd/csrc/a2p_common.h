@@ -59,10 +59,10 @@ int ws_drop(int slot); // synchronises the device and frees one buffer of the cu
 size_t ws_bytes();     // held on the current device
 int ws_release();      // synchronises the device, frees the current device's buffers
 
-// Host memory for arrays that are copied from or to the device, pinned (and reused) while the library's share of
-// pinned memory lasts, ordinary otherwise; given back with host_free from any thread.
-void* host_alloc(size_t bytes, bool* pinned);
-void host_free(void* p);
+// Pinned host memory for one call's copies from or to the device, or null beyond the library's share of it; given back,
+// from any thread, when nothing queued reads or writes it any more.
+void* pinned_take(size_t bytes);
+void pinned_give(void* p);
 
 // Device status word bits written by kernels when inputs violate the contract.
 enum StatusBits {

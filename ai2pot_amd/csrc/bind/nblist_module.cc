@@ -3,8 +3,8 @@
 //       -> (inum, ilist, numneigh, firstneigh, rcs, types, nghost)
 // (source/nblist/bind/nblist_bind.cc:35-207): same positional signature, same type checks
 // (TypeError), NumPy arrays in and out, float32 / float64 selected by the dtype of coords.
-// The list is built on the current HIP device by libai2pot_hip.so (a2p_nblist_host_*); the arrays
-// returned share one block of host memory, owned by the last of them.  Unlike the reference, more than `umax` neighbours raises
+// The list is built on the current HIP device by libai2pot_hip.so (a2p_nblist_host_into_*); the arrays
+// returned are ordinary NumPy arrays.  Unlike the reference, more than `umax` neighbours raises
 // RuntimeError instead of overrunning the output arrays.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
@@ -22,51 +22,34 @@ PyObject* fail(PyObject* exc, const std::string& msg)
     return nullptr;
 }
 
-void free_block(PyObject* capsule)
-{
-    a2p_host_lists_free(PyCapsule_GetPointer(capsule, "a2p_host_lists"));
-}
-
-// An array over part of the block, which lives as long as any of its arrays.
-PyObject* array_over(PyObject* owner, int nd, npy_intp* dims, int type, void* data)
-{
-    PyObject* a = PyArray_SimpleNewFromData(nd, dims, type, data);
-    if (!a) return nullptr;
-    Py_INCREF(owner);
-    if (PyArray_SetBaseObject((PyArrayObject*)a, owner) != 0) {
-        Py_DECREF(a);
-        return nullptr;
-    }
-    return a;
-}
-
 PyObject* run(PyArrayObject* lattice, PyArrayObject* types, PyArrayObject* coords, double rcut, int umax,
               bool is_cart, const int* pbc, bool sort, int npy_float)
 {
     const int n = (int)PyArray_DIM(coords, 0);
     if (n <= 0) return fail(PyExc_RuntimeError, "the structure has no atoms");
-    a2p_host_lists out;
-    const int rc = npy_float == NPY_FLOAT32
-        ? a2p_nblist_host_f32((const float*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
-                              (const float*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, &out)
-        : a2p_nblist_host_f64((const double*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
-                              (const double*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, &out);
-    if (rc != A2P_OK) return fail(PyExc_RuntimeError, std::string("libai2pot_hip: ") + a2p_last_error());
-    PyObject* owner = PyCapsule_New(out.block, "a2p_host_lists", free_block);
-    if (!owner) {
-        a2p_host_lists_free(out.block);
-        return nullptr;
-    }
     npy_intp d1[1] = {n}, d2[2] = {n, umax}, d3[3] = {n, umax, 3};
-    PyObject* ilist = array_over(owner, 1, d1, NPY_INT32, out.ilist);
-    PyObject* nn = array_over(owner, 1, d1, NPY_INT32, out.numneigh);
-    PyObject* first = array_over(owner, 2, d2, NPY_INT32, out.firstneigh);
-    PyObject* rcs = array_over(owner, 3, d3, npy_float, out.rcs);
-    PyObject* tout = array_over(owner, 1, d1, NPY_INT32, out.types);
-    Py_DECREF(owner);
-    if (!(ilist && nn && first && rcs && tout)) {
+    PyObject* ilist = PyArray_SimpleNew(1, d1, NPY_INT32);
+    PyObject* nn = PyArray_SimpleNew(1, d1, NPY_INT32);
+    PyObject* first = PyArray_SimpleNew(2, d2, NPY_INT32);
+    PyObject* rcs = PyArray_SimpleNew(3, d3, npy_float);
+    PyObject* tout = PyArray_SimpleNew(1, d1, NPY_INT32);
+    auto drop = [&]() -> PyObject* {
         Py_XDECREF(ilist); Py_XDECREF(nn); Py_XDECREF(first); Py_XDECREF(rcs); Py_XDECREF(tout);
         return nullptr;
+    };
+    if (!(ilist && nn && first && rcs && tout)) return drop();
+    auto data = [](PyObject* a) { return PyArray_DATA((PyArrayObject*)a); };
+    int most = 0;
+    const int rc = npy_float == NPY_FLOAT32
+        ? a2p_nblist_host_into_f32((const float*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
+                                   (const float*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, (int*)data(ilist),
+                                   (int*)data(nn), (int*)data(first), (float*)data(rcs), (int*)data(tout), &most)
+        : a2p_nblist_host_into_f64((const double*)PyArray_DATA(lattice), (const int*)PyArray_DATA(types),
+                                   (const double*)PyArray_DATA(coords), n, rcut, umax, is_cart, pbc, sort, (int*)data(ilist),
+                                   (int*)data(nn), (int*)data(first), (double*)data(rcs), (int*)data(tout), &most);
+    if (rc != A2P_OK) {
+        drop();
+        return fail(PyExc_RuntimeError, std::string("libai2pot_hip: ") + a2p_last_error());
     }
     return Py_BuildValue("(iNNNNNi)", n, ilist, nn, first, rcs, tout, 0);
 }

@@ -24,75 +24,64 @@ void set_error(const char* fmt, ...)
 
 const char* last_error() { return g_err.c_str(); }
 
-// ---- host blocks ---------------------------------------------------------------------------------------
+// ---- pinned blocks -------------------------------------------------------------------------------------
 // Copies from pageable memory are staged by the runtime (90 KB took 36 us down and up to 100 us up, 9 us from pinned
-// memory) and pinning costs more than a small list: blocks are pinned once and kept.  The library holds at most
-// kPinnedMost bytes pinned, in use and idle together; a larger share, or a block above kPinnedBlock, is ordinary memory.
+// memory) and pinning costs more than a small list: blocks are pinned once and kept.  A block belongs to one call, which
+// gives it back with nothing queued that reads or writes it.  The library holds at most kPinnedMost bytes, in use and idle
+// together, and no block above kPinnedBlock.
 namespace {
 constexpr size_t kPinnedMost = (size_t)256 << 20, kPinnedBlock = (size_t)64 << 20, kPinnedStep = 64 << 10;
-struct HostBlock {
+struct PinnedBlock {
     char* ptr;
     size_t bytes;
     bool idle;
 };
-std::mutex g_host_mutex;
-std::vector<HostBlock> g_host_blocks;      // the pinned ones
-size_t g_host_pinned = 0;
+std::mutex g_pinned_mutex;
+std::vector<PinnedBlock> g_pinned_blocks;
+size_t g_pinned_bytes = 0;
 
 // frees idle blocks until `want` more bytes fit the share (all of them with want = kPinnedMost)
-void host_trim(size_t want)
+void pinned_trim(size_t want)
 {
-    for (size_t i = 0; i < g_host_blocks.size() && g_host_pinned + want > kPinnedMost;) {
-        if (!g_host_blocks[i].idle) { i++; continue; }
-        (void)hipHostFree(g_host_blocks[i].ptr);
-        g_host_pinned -= g_host_blocks[i].bytes;
-        g_host_blocks.erase(g_host_blocks.begin() + i);
+    for (size_t i = 0; i < g_pinned_blocks.size() && g_pinned_bytes + want > kPinnedMost;) {
+        if (!g_pinned_blocks[i].idle) { i++; continue; }
+        (void)hipHostFree(g_pinned_blocks[i].ptr);
+        g_pinned_bytes -= g_pinned_blocks[i].bytes;
+        g_pinned_blocks.erase(g_pinned_blocks.begin() + i);
     }
 }
 }  // namespace
 
-void* host_alloc(size_t bytes, bool* pinned)
+void* pinned_take(size_t bytes)
 {
-    *pinned = false;
-    if (bytes <= kPinnedBlock) {
-        std::lock_guard<std::mutex> lock(g_host_mutex);
-        HostBlock* best = nullptr;
-        for (HostBlock& b : g_host_blocks)
-            if (b.idle && b.bytes >= bytes && b.bytes <= 2 * bytes + kPinnedStep && (!best || b.bytes < best->bytes)) best = &b;
-        if (best) {
-            // its last owner may have queued a copy that still reads it
-            if (hipDeviceSynchronize() == hipSuccess) {
-                best->idle = false;
-                *pinned = true;
-                return best->ptr;
-            }
-            return nullptr;
-        }
-        const size_t want = (bytes + kPinnedStep - 1) / kPinnedStep * kPinnedStep;
-        if (g_host_pinned + want > kPinnedMost) host_trim(want);
-        if (g_host_pinned + want <= kPinnedMost) {
-            void* p = nullptr;
-            if (hipHostMalloc(&p, want, hipHostMallocPortable) == hipSuccess && p) {
-                g_host_blocks.push_back({(char*)p, want, false});
-                g_host_pinned += want;
-                *pinned = true;
-                return p;
-            }
-            (void)hipGetLastError();
-        }
+    if (bytes > kPinnedBlock) return nullptr;
+    std::lock_guard<std::mutex> lock(g_pinned_mutex);
+    PinnedBlock* best = nullptr;
+    for (PinnedBlock& b : g_pinned_blocks)
+        if (b.idle && b.bytes >= bytes && b.bytes <= 2 * bytes + kPinnedStep && (!best || b.bytes < best->bytes)) best = &b;
+    if (best) {
+        best->idle = false;
+        return best->ptr;
     }
-    return malloc(bytes ? bytes : 1);
+    const size_t want = (bytes + kPinnedStep - 1) / kPinnedStep * kPinnedStep;
+    if (g_pinned_bytes + want > kPinnedMost) pinned_trim(want);
+    if (g_pinned_bytes + want > kPinnedMost) return nullptr;
+    void* p = nullptr;
+    if (hipHostMalloc(&p, want, hipHostMallocPortable) != hipSuccess || !p) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    g_pinned_blocks.push_back({(char*)p, want, false});
+    g_pinned_bytes += want;
+    return p;
 }
 
-void host_free(void* p)
+void pinned_give(void* p)
 {
     if (!p) return;
-    {
-        std::lock_guard<std::mutex> lock(g_host_mutex);
-        for (HostBlock& b : g_host_blocks)
-            if (b.ptr == (char*)p) { b.idle = true; return; }
-    }
-    free(p);
+    std::lock_guard<std::mutex> lock(g_pinned_mutex);
+    for (PinnedBlock& b : g_pinned_blocks)
+        if (b.ptr == (char*)p) { b.idle = true; return; }
 }
 
 namespace {
@@ -165,8 +154,8 @@ int ws_release()
     A2P_HIP_CHECK(hipGetDevice(&dev));
     A2P_HIP_CHECK(hipDeviceSynchronize());          // no kernel of any stream still uses the buffers
     {
-        std::lock_guard<std::mutex> host_lock(g_host_mutex);
-        host_trim(kPinnedMost);
+        std::lock_guard<std::mutex> pinned_lock(g_pinned_mutex);
+        pinned_trim(kPinnedMost);
     }
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     if ((int)g_ws.size() <= dev) return A2P_OK;

@@ -2113,67 +2113,108 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     return A2P_OK;
 }
 
-// The list as host arrays in one block.  Inputs go through a pinned block that the first kernels read across the bus
-// (each value once), outputs are built on the device and come back as one copy.  108 atoms, fp32, umax 200: bound by the
-// latency of the build's launches: 211 -> 111 us with this in place of an allocation and a pageable copy per array
-// (1000 atoms 417 -> 168 us).
+// Host arrays of a list, the caller's own.
+template <typename T>
+struct HostLists {
+    int *ilist, *numneigh, *firstneigh;
+    T* rcs;
+    int* types;
+};
+
+// The list with host arrays in and out.  Inputs go through a pinned block that the first kernels read across the bus (each
+// value once); outputs are built on the device, come back as one copy into another pinned block and go from there to the
+// caller's arrays, which stay ordinary memory: a copy that the caller queues from a pinned array would still read it when
+// the caller already writes to it.  Both blocks are the call's own until it returns.
 template <typename T>
 int nblist_host(const T* lattice, const int* types, const T* coords, int N, double rcut, int umax, int is_cart,
-                const int* pbc, int sort, a2p_host_lists* out)
+                const int* pbc, int sort, const HostLists<T>& out, int* max_numneigh)
 {
-    A2P_REQUIRE(out, A2P_ERR_INVALID, "nblist: null output");
-    *out = a2p_host_lists{};
     A2P_REQUIRE(types && coords && N > 0 && umax > 0, A2P_ERR_INVALID, "nblist: null host pointer or empty structure");
+    A2P_REQUIRE(out.ilist && out.numneigh && out.firstneigh && out.rcs && out.types && max_numneigh, A2P_ERR_INVALID,
+                "nblist: null output");
     const size_t n_rcs = (size_t)N * umax * 3 * sizeof(T), n_first = (size_t)N * umax * sizeof(int), n_i = (size_t)N * sizeof(int);
     const size_t bytes = n_rcs + n_first + 3 * n_i;
     void* dev = nullptr;
     int rc = ws_get(WS_HOST_LISTS, bytes, &dev);
     if (rc) return rc;
-    bool in_pinned = false, out_pinned = false;
     const size_t n_x = (size_t)N * 3 * sizeof(T);
-    char* in = (char*)host_alloc(n_x + n_i, &in_pinned);
-    char* block = (char*)host_alloc(bytes, &out_pinned);
+    char* in = (char*)pinned_take(n_x + n_i);
+    char* block = (char*)pinned_take(bytes);
     char* in_dev = in;
     void* in_buf = nullptr;
-    auto fail = [&](int code) { host_free(in); host_free(block); if (in_buf) (void)hipFree(in_buf); return code; };
-    if (!in || !block) {
-        set_error("nblist: no host memory for %zu bytes of lists", bytes);
-        return fail(A2P_ERR_HIP);
-    }
-    memcpy(in, coords, n_x);
-    memcpy(in + n_x, types, n_i);
+    auto done = [&](int code) {                         // (an early return leaves nothing queued that reads the blocks)
+        if (code != A2P_OK) (void)hipStreamSynchronize(nullptr);
+        pinned_give(in);
+        pinned_give(block);
+        if (in_buf) (void)hipFree(in_buf);
+        return code;
+    };
     hipError_t err = hipSuccess;
-    if (!in_pinned) {
+    if (in) {
+        memcpy(in, coords, n_x);
+        memcpy(in + n_x, types, n_i);
+    } else {
         err = hipMalloc(&in_buf, n_x + n_i);
-        if (err == hipSuccess) err = hipMemcpy(in_buf, in, n_x + n_i, hipMemcpyHostToDevice);
         in_dev = (char*)in_buf;
+        if (err == hipSuccess) err = hipMemcpy(in_dev, coords, n_x, hipMemcpyHostToDevice);
+        if (err == hipSuccess) err = hipMemcpy(in_dev + n_x, types, n_i, hipMemcpyHostToDevice);
     }
-    if (err != hipSuccess) { set_error("nblist: copy to the device failed: %s", hipGetErrorString(err)); return fail(A2P_ERR_HIP); }
+    if (err != hipSuccess) { set_error("nblist: copy to the device failed: %s", hipGetErrorString(err)); return done(A2P_ERR_HIP); }
     T* const d_rcs = (T*)dev;
     int* const d_first = (int*)((char*)dev + n_rcs);
     int* const d_i = (int*)((char*)dev + n_rcs + n_first);
     rc = nblist_build<T>(lattice, (const int*)(in_dev + n_x), (const T*)in_dev, N, rcut, umax, is_cart, pbc, sort, d_i, d_i + N,
                          d_first, d_rcs, d_i + 2 * (size_t)N, nullptr, nullptr);
-    if (rc) return fail(rc);
-    err = hipMemcpyAsync(block, dev, bytes, hipMemcpyDeviceToHost, nullptr);
-    if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
-    if (err != hipSuccess) { set_error("nblist: copy from the device failed: %s", hipGetErrorString(err)); return fail(A2P_ERR_HIP); }
-    out->block = block;
-    out->rcs = block;
-    out->firstneigh = (int*)(block + n_rcs);
-    out->ilist = (int*)(block + n_rcs + n_first);
-    out->numneigh = out->ilist + N;
-    out->types = out->ilist + 2 * (size_t)N;
-    for (int i = 0; i < N; i++) out->max_numneigh = std::max(out->max_numneigh, out->numneigh[i]);
-    if (out->max_numneigh > umax) {
-        void* flags = nullptr;
-        if (ws_get(WS_FLAGS, 64, &flags) == A2P_OK) (void)fill_zero(flags, sizeof(int), nullptr);
-        set_error("nblist: an atom has %d neighbours, more than umax_num_neigh_atoms = %d", out->max_numneigh, umax);
-        *out = a2p_host_lists{};
-        return fail(A2P_ERR_OVERFLOW);
+    if (rc) return done(rc);
+    if (block) {
+        err = hipMemcpyAsync(block, dev, bytes, hipMemcpyDeviceToHost, nullptr);
+        if (err == hipSuccess) err = hipStreamSynchronize(nullptr);
     }
-    host_free(in);
-    if (in_buf) (void)hipFree(in_buf);
+    const struct { void* to; size_t from, n; } piece[5] = {
+        {out.numneigh, n_rcs + n_first + n_i, n_i}, {out.rcs, 0, n_rcs}, {out.firstneigh, n_rcs, n_first},
+        {out.ilist, n_rcs + n_first, n_i}, {out.types, n_rcs + n_first + 2 * n_i, n_i}};
+    *max_numneigh = 0;
+    for (const auto& p : piece) {
+        if (err != hipSuccess) break;
+        if (block) memcpy(p.to, block + p.from, p.n);
+        else err = hipMemcpy(p.to, (const char*)dev + p.from, p.n, hipMemcpyDeviceToHost);
+        if (&p != &piece[0] || err != hipSuccess) continue;
+        for (int i = 0; i < N; i++) *max_numneigh = std::max(*max_numneigh, out.numneigh[i]);
+        if (*max_numneigh > umax) {
+            void* flags = nullptr;
+            if (ws_get(WS_FLAGS, 64, &flags) == A2P_OK) (void)fill_zero(flags, sizeof(int), nullptr);
+            set_error("nblist: an atom has %d neighbours, more than umax_num_neigh_atoms = %d", *max_numneigh, umax);
+            return done(A2P_ERR_OVERFLOW);
+        }
+    }
+    if (err != hipSuccess) { set_error("nblist: copy from the device failed: %s", hipGetErrorString(err)); return done(A2P_ERR_HIP); }
+    return done(A2P_OK);
+}
+
+// The same with the arrays in one block of the library's making.
+template <typename T>
+int nblist_host_block(const T* lattice, const int* types, const T* coords, int N, double rcut, int umax, int is_cart,
+                      const int* pbc, int sort, a2p_host_lists* out)
+{
+    A2P_REQUIRE(out, A2P_ERR_INVALID, "nblist: null output");
+    *out = a2p_host_lists{};
+    A2P_REQUIRE(N > 0 && umax > 0, A2P_ERR_INVALID, "nblist: null host pointer or empty structure");
+    const size_t row = (size_t)N * umax;
+    char* const block = (char*)malloc(row * (3 * sizeof(T) + sizeof(int)) + (size_t)N * 3 * sizeof(int));
+    A2P_REQUIRE(block, A2P_ERR_HIP, "nblist: no host memory for the lists");
+    int* const first = (int*)(block + row * 3 * sizeof(T));
+    const HostLists<T> lists{first + row, first + row + N, first, (T*)block, first + row + 2 * (size_t)N};
+    const int rc = nblist_host<T>(lattice, types, coords, N, rcut, umax, is_cart, pbc, sort, lists, &out->max_numneigh);
+    if (rc) {
+        free(block);
+        *out = a2p_host_lists{};
+        return rc;
+    }
+    out->block = out->rcs = block;
+    out->firstneigh = first;
+    out->ilist = lists.ilist;
+    out->numneigh = lists.numneigh;
+    out->types = lists.types;
     return A2P_OK;
 }
 
@@ -2185,16 +2226,32 @@ extern "C" {
 int a2p_nblist_host_f32(const float* lattice, const int* types, const float* coords, int natoms, double rcut, int umax,
                         int is_cart, const int* pbc, int sort, a2p_host_lists* out)
 {
-    return a2p::nblist_host<float>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort, out);
+    return a2p::nblist_host_block<float>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort, out);
+}
+
+int a2p_nblist_host_into_f32(const float* lattice, const int* types, const float* coords, int natoms, double rcut, int umax,
+                             int is_cart, const int* pbc, int sort, int* ilist, int* numneigh, int* firstneigh, float* rcs,
+                             int* types_out, int* max_numneigh)
+{
+    return a2p::nblist_host<float>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort,
+                                {ilist, numneigh, firstneigh, rcs, types_out}, max_numneigh);
 }
 
 int a2p_nblist_host_f64(const double* lattice, const int* types, const double* coords, int natoms, double rcut, int umax,
                         int is_cart, const int* pbc, int sort, a2p_host_lists* out)
 {
-    return a2p::nblist_host<double>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort, out);
+    return a2p::nblist_host_block<double>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort, out);
 }
 
-void a2p_host_lists_free(void* block) { a2p::host_free(block); }
+int a2p_nblist_host_into_f64(const double* lattice, const int* types, const double* coords, int natoms, double rcut, int umax,
+                             int is_cart, const int* pbc, int sort, int* ilist, int* numneigh, int* firstneigh, double* rcs,
+                             int* types_out, int* max_numneigh)
+{
+    return a2p::nblist_host<double>(lattice, types, coords, natoms, rcut, umax, is_cart, pbc, sort,
+                                {ilist, numneigh, firstneigh, rcs, types_out}, max_numneigh);
+}
+
+void a2p_host_lists_free(void* block) { free(block); }
 
 int a2p_nblist_sync_free(int on)
 {

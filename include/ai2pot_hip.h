@@ -198,8 +198,9 @@ int a2p_nblist_build_f64(const double* lattice, const int* types, const double* 
 
 /* The list with host arrays in and out, as nblist.find_info4mlff has them (source/nblist/bind/nblist_bind.cc:35-189):
  * types int32[natoms] and coords [natoms, 3] are host pointers; the results lie in one host block that the caller hands
- * back to a2p_host_lists_free (any thread; the library keeps pinned blocks for later calls, at most 256 MiB in all).
- * Runs on the null stream and waits for it.  A neighbour count above umax is A2P_ERR_OVERFLOW, and nothing is returned. */
+ * back to a2p_host_lists_free (any thread).  Runs on the null stream and waits for it.  A neighbour count above umax is
+ * A2P_ERR_OVERFLOW, and nothing is returned.  The library passes inputs and results through pinned blocks that it keeps for
+ * later calls, at most 256 MiB in all (a2p_workspace_release frees them). */
 typedef struct {
     void* block;          /* owns the five arrays */
     void* rcs;            /* [natoms, umax, 3] of the type of coords */
@@ -211,6 +212,14 @@ int a2p_nblist_host_f32(const float* lattice, const int* types, const float* coo
 int a2p_nblist_host_f64(const double* lattice, const int* types, const double* coords, int natoms, double rcut, int umax,
                         int is_cart, const int* pbc, int sort, a2p_host_lists* out);
 void a2p_host_lists_free(void* block);
+/* The same into the caller's host arrays; *max_numneigh receives the largest neighbour count, and above umax the arrays
+ * hold nothing of use. */
+int a2p_nblist_host_into_f32(const float* lattice, const int* types, const float* coords, int natoms, double rcut, int umax,
+                             int is_cart, const int* pbc, int sort, int* ilist, int* numneigh, int* firstneigh, float* rcs,
+                             int* types_out, int* max_numneigh);
+int a2p_nblist_host_into_f64(const double* lattice, const int* types, const double* coords, int natoms, double rcut, int umax,
+                             int is_cart, const int* pbc, int sort, int* ilist, int* numneigh, int* firstneigh, double* rcs,
+                             int* types_out, int* max_numneigh);
 
 /* Rebuild into buffers that already hold a list.  Same arguments and results as
  * a2p_nblist_build_*, for a caller that keeps its list buffers between steps (molecular

@@ -1,6 +1,6 @@
-"""The CPython module's lists: five arrays over one host block that the library pins and reuses (csrc/common.hip,
-host_alloc).  Lists that are kept stay what they were while others are built and dropped, also past the library's share
-of pinned memory."""
+"""The CPython module's lists: ordinary arrays, filled through pinned blocks that the library reuses (csrc/common.hip,
+pinned_take).  Lists that are kept stay what they were while others are built and dropped, also past the size of the
+pinned blocks; each array is memory of its own."""
 import os
 import sys
 
@@ -18,7 +18,7 @@ def test_kept_lists_stay(oracle):
     if LIBDIR not in sys.path:
         sys.path.append(LIBDIR)
     import nblist
-    n, umax = 60, 20000                               # 19 MB and 34 MB a list: more than 256 MiB are alive at the end
+    n, umax = 60, 20000                               # 19 MB and 34 MB a list
     kept = []
     for k in range(12):
         dt = (np.float32, np.float64)[k % 2]
@@ -35,8 +35,35 @@ def test_kept_lists_stay(oracle):
         want = oracle.nblist(args[0], args[1], args[2], 4.0, umax, sort=args[7])
         if isinstance(out, tuple):
             assert_same(out, want)
-        else:                                         # one array holds the block on its own
+        else:                                         # one array kept alone
             assert np.array_equal(out.view(np.uint8), want[4].view(np.uint8))
     with pytest.raises(RuntimeError):
         nblist.find_info4mlff(*args[:4], 3, *args[5:])
     assert_same(nblist.find_info4mlff(*args), want)   # nothing is left behind by the failed call
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_arrays_are_ordinary_memory(oracle, dt):
+    """A non-blocking copy of an array to the device has read it when it returns, as of any array that is not pinned: what
+    the caller writes into the array afterwards is not what arrives, however long the queue ahead of the copy.  No array
+    keeps another's memory."""
+    import torch
+    if LIBDIR not in sys.path:
+        sys.path.append(LIBDIR)
+    import nblist
+    lat, pos = synth.random_packed(300, [19.0, 18.0, 17.5], 2.0, 11)
+    ty = synth.rng_randint(5, 300, 3)
+    args = (lat.astype(dt), ty, pos.astype(dt), 5.0, 200, True, [True, True, True], False)
+    out = nblist.find_info4mlff(*args)
+    want = oracle.nblist(args[0], ty, args[2], 5.0, 200)
+    assert_same(out, want)
+    queue = torch.zeros(1 << 26, device="cuda:0")
+    for a in out[1:6]:
+        assert a.flags.owndata and not torch.from_numpy(a).is_pinned()
+    for _ in range(200):                              # about 20 ms
+        queue.add_(1.0)
+    up = [torch.from_numpy(a).to("cuda:0", non_blocking=True) for a in out[1:6]]
+    for a in out[1:6]:
+        a[...] = 77
+    for g, w in zip(up, want[1:6]):
+        assert np.array_equal(g.cpu().numpy(), w)
