@@ -61,6 +61,7 @@ int ws_release();      // synchronises the device, frees the current device's bu
 
 // Pinned host memory for one call's copies from or to the device, or null beyond the library's share of it; given back,
 // from any thread, when nothing queued reads or writes it any more.
+constexpr size_t PINNED_BLOCK = (size_t)64 << 20;      // the largest
 void* pinned_take(size_t bytes);
 void pinned_give(void* p);
 

@@ -28,9 +28,9 @@ const char* last_error() { return g_err.c_str(); }
 // Copies from pageable memory are staged by the runtime (90 KB took 36 us down and up to 100 us up, 9 us from pinned
 // memory) and pinning costs more than a small list: blocks are pinned once and kept.  A block belongs to one call, which
 // gives it back with nothing queued that reads or writes it.  The library holds at most kPinnedMost bytes, in use and idle
-// together, and no block above kPinnedBlock.
+// together, and no block above PINNED_BLOCK.
 namespace {
-constexpr size_t kPinnedMost = (size_t)256 << 20, kPinnedBlock = (size_t)64 << 20, kPinnedStep = 64 << 10;
+constexpr size_t kPinnedMost = (size_t)256 << 20, kPinnedStep = 64 << 10;
 struct PinnedBlock {
     char* ptr;
     size_t bytes;
@@ -54,7 +54,7 @@ void pinned_trim(size_t want)
 
 void* pinned_take(size_t bytes)
 {
-    if (bytes > kPinnedBlock) return nullptr;
+    if (bytes > PINNED_BLOCK) return nullptr;
     std::lock_guard<std::mutex> lock(g_pinned_mutex);
     PinnedBlock* best = nullptr;
     for (PinnedBlock& b : g_pinned_blocks)

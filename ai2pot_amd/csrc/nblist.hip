@@ -2134,8 +2134,14 @@ int nblist_host(const T* lattice, const int* types, const T* coords, int N, doub
                 "nblist: null output");
     const size_t n_rcs = (size_t)N * umax * 3 * sizeof(T), n_first = (size_t)N * umax * sizeof(int), n_i = (size_t)N * sizeof(int);
     const size_t bytes = n_rcs + n_first + 3 * n_i;
-    void* dev = nullptr;
-    int rc = ws_get(WS_HOST_LISTS, bytes, &dev);
+    // on the device in the workspace up to the size of a pinned block, beyond that in memory of the call's own
+    void *dev = nullptr, *own = nullptr;
+    int rc = A2P_OK;
+    if (bytes <= PINNED_BLOCK) rc = ws_get(WS_HOST_LISTS, bytes, &dev);
+    else {
+        A2P_HIP_CHECK(hipMalloc(&own, bytes));
+        dev = own;
+    }
     if (rc) return rc;
     const size_t n_x = (size_t)N * 3 * sizeof(T);
     char* in = (char*)pinned_take(n_x + n_i);
@@ -2147,6 +2153,7 @@ int nblist_host(const T* lattice, const int* types, const T* coords, int N, doub
         pinned_give(in);
         pinned_give(block);
         if (in_buf) (void)hipFree(in_buf);
+        if (own) (void)hipFree(own);
         return code;
     };
     hipError_t err = hipSuccess;

@@ -67,3 +67,24 @@ def test_arrays_are_ordinary_memory(oracle, dt):
         a[...] = 77
     for g, w in zip(up, want[1:6]):
         assert np.array_equal(g.cpu().numpy(), w)
+
+
+def test_a_large_list_is_not_kept_on_the_device(oracle):
+    """Lists beyond the size of a pinned block (64 MiB) take no part of the workspace, which would hold the largest of them
+    for good."""
+    from ai2pot_amd import _lib
+    import ctypes
+    if LIBDIR not in sys.path:
+        sys.path.append(LIBDIR)
+    import nblist
+    L = _lib.lib()
+    L.a2p_workspace_bytes.restype = ctypes.c_size_t
+    lat, pos = synth.random_packed(300, [19.0, 18.0, 17.5], 2.0, 11)
+    ty = synth.rng_randint(5, 300, 3)
+    args = lambda umax: (lat, ty, pos, 5.0, umax, True, [True, True, True], False)
+    small = nblist.find_info4mlff(*args(200))
+    before = L.a2p_workspace_bytes()
+    out = nblist.find_info4mlff(*args(9000))          # 76 MB
+    assert L.a2p_workspace_bytes() - before < 16 << 20
+    assert_same(out, oracle.nblist(lat, ty, pos, 5.0, 9000))
+    assert all(np.array_equal(a, b) for a, b in zip(small[1:6], nblist.find_info4mlff(*args(200))[1:6]))
