@@ -212,6 +212,14 @@ inline at::Tensor zbl_esites(double zbl_rmax, double zbl_rmin, const at::Tensor&
     return out;
 }
 
+// Whether the numbers in a tensor's memory are all there is to it: no gradient is recorded for it and it carries no tangent
+// (a backward pass may itself be differentiated, either way), and it is no wrapper over a batch of tensors, which has no
+// memory.  Others go through operators that autograd knows.
+inline bool only_numbers(const at::Tensor& t)
+{
+    return t.has_storage() && !t._fw_grad(/*level=*/0).defined() && !(at::GradMode::is_enabled() && t.requires_grad());
+}
+
 // What the loss functions of the three families share around their library call.
 
 // Tensor over elements [beg, beg + numel(shape)) of a one-dimensional one, without the view relation to it: an
@@ -279,10 +287,7 @@ inline void grad_products(torch::autograd::AutogradContext* ctx, const at::Tenso
         numel.push_back(n);
     }
     const int np = (int)shape.size();
-    // a backward pass that is itself differentiated (in grad_output, either way) or mapped over a batch of gradients, whose
-    // tensors wrap others and have no storage of their own, goes through operators that know of it
-    if (B == 0 || !gl.has_storage() || gl._fw_grad(/*level=*/0).defined() ||
-        (at::GradMode::is_enabled() && gl.requires_grad())) {
+    if (B == 0 || !only_numbers(gl)) {
         for (int64_t i = 0, beg = 0; i < np; beg += numel[i] * B, i++)
             out[first + i] = torch::matmul(gl, flat.narrow(0, beg, numel[i] * B).view({B, (int64_t)numel[i]})).reshape(shape[i]);
         return;

@@ -334,9 +334,10 @@ struct BasisFunction : public torch::autograd::Function<BasisFunction> {
     }
 };
 
-// (More columns than a2p_normal_equations_* takes.)  X^T X [n, n] and X^T y [n] of a tall matrix X [N, n]: the rows are cut into up to 64 blocks whose products run
-// as one batched GEMM and are added afterwards (a single GEMM with n of about a hundred and N in the tens of
-// thousands occupies one tile of the chip: 0.66 ms against 0.03 ms for 24576 x 95 in fp64)
+// (More columns than a2p_normal_equations_* takes, or labels that want a gradient.)  X^T X [n, n] and X^T y [n] of a tall
+// matrix X [N, n]: the rows are cut into up to 64 blocks whose products run as one batched GEMM and are added afterwards
+// (a single GEMM with n of about a hundred and N in the tens of thousands occupies one tile of the chip: 0.66 ms against
+// 0.03 ms for 24576 x 95 in fp64)
 std::pair<at::Tensor, at::Tensor> gram(const at::Tensor& X, const at::Tensor& y)
 {
     const int64_t N = X.size(0), n = X.size(1);
@@ -395,8 +396,8 @@ variable_list lin_matrix_lin_vector(double e_w, double f_w, double v_w, const at
         return rc;
     };
     run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
-    if (n <= 575) {
-        // (wider systems keep a matrix product busy by themselves)
+    // (wider systems keep a matrix product busy by themselves)
+    if (n <= 575 && only_numbers(e_dft) && only_numbers(f_dft) && only_numbers(v_dft)) {
         at::Tensor A = at::empty({n, n}, opt), b = at::empty({n}, opt);
         const long long rows[3] = {B, (long long)B * P * 3, (long long)B * 9};
         const double w[3] = {e_w, f_w, v_w};

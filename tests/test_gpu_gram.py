@@ -3,11 +3,13 @@ around the 16 columns of a tile and the 24 tiles of a workgroup, and at row coun
 force components of a list that names an atom by more pairs than a row has room for, and by more than the 256 that are
 ranked in LDS (csrc/mtp.hip comp_force_kernel), against one pass per column."""
 import ctypes as c
+import os
 
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
+LIBDIR = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "ai2pot_amd", "_lib")
 
 
 @pytest.mark.parametrize("dtype", ["float64", "float32"])
@@ -74,3 +76,37 @@ def test_an_atom_named_by_many_pairs(oracle, named):
         L.a2p_pair_segment_capacity(cap)
     for a, b, c_ in zip(one, per_column, again):
         assert np.abs(b).max() > 0 and close(a, b) and np.array_equal(a, c_)
+
+
+def _solver(oracle, dtype):
+    import torch
+    from conftest import to_device
+    from test_gpu_mtp import loss_inputs, model_to_device
+    torch.ops.load_library(os.path.join(LIBDIR, "libmtpr_bind.so"))
+    m, nb, lab = loss_inputs(oracle, 10, 2, sizes=(17, 12, 23))
+    md, d = model_to_device(m, dtype), to_device(nb, dtype)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0", dtype)
+    labels = [t(lab[k]) for k in ("energy", "force", "virial")]
+    z = torch.zeros(0, dtype=dtype, device="cuda:0")
+    args = (m["chebyshev_size"], m["scaling"], md["coeffs"], md["linear_coeffs"], md["type_bias"], m["alpha_moments_count"],
+            md["alpha_index_basic"], md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], d["binum"], d["bilist"],
+            d["bnumneigh"], d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], 0, m["rmax"], m["rmin"], md["q_scaler"],
+            0.0, 0.0, z, z)
+    return labels, args
+
+
+def test_labels_that_want_a_gradient(oracle):
+    """lin_vector is linear in the labels: u . lin_vector is their product with its gradient, and the numbers are those of
+    labels that want none."""
+    import torch
+    labels, args = _solver(oracle, torch.float64)
+    op = torch.ops.mtpr.LinMatrixLinVectorOp
+    A0, b0 = op(1.0, 0.7, 0.3, *labels, *args)
+    leaves = [l.clone().requires_grad_(True) for l in labels]
+    A, b = op(1.0, 0.7, 0.3, *leaves, *args)
+    assert torch.allclose(A, A0, rtol=1e-11, atol=1e-13 * float(A0.abs().max()))
+    assert torch.allclose(b, b0, rtol=1e-11, atol=1e-13 * float(b0.abs().max()))
+    u = torch.linspace(-1.0, 1.3, b.numel(), dtype=torch.float64, device="cuda:0")
+    grads = torch.autograd.grad((u * b).sum(), leaves)
+    total = sum((g * l).sum() for g, l in zip(grads, labels))
+    assert abs(float(total - (u * b0).sum())) <= 1e-11 * float((u * b0).abs().sum())
