@@ -910,7 +910,8 @@ def mtp_lin_components(chebyshev_size, scaling, coeffs, alpha_moments_count, alp
 
 
 def _gram(X, y):
-    """X^T X [n, n] and X^T y [n] of a tall matrix X [N, n].  The rows are cut into up to 64 blocks whose products run as
+    """(For labels that want a gradient, or more columns than the library's kernel takes.)
+    X^T X [n, n] and X^T y [n] of a tall matrix X [N, n].  The rows are cut into up to 64 blocks whose products run as
     one batched GEMM and are added afterwards: a single GEMM with n of about a hundred and N in the tens of thousands
     occupies one tile of the chip (0.66 ms against 0.03 ms for 24576 x 95 in fp64)."""
     N, n = X.shape
@@ -922,6 +923,30 @@ def _gram(X, y):
     if head < N:
         G = G + X[head:].t() @ R[head:]
     return G[:, :n], G[:, n]
+
+
+_NORMAL_EQUATIONS_MOST = 575         # columns, a2p_normal_equations_*
+
+
+def _only_numbers(t):
+    """Whether a kernel may read the tensor in place of what autograd knows of it."""
+    import torch.autograd.forward_ad as fwad
+    return not (torch._C._functorch.is_functorch_wrapped_tensor(t) or (torch.is_grad_enabled() and t.requires_grad) or
+                fwad.unpack_dual(t).tangent is not None)
+
+
+def _normal_equations(weights, X, y):
+    """[sum_k w_k X_k^T X_k, sum_k w_k X_k^T y_k] for three matrices [rows_k, n] by the library."""
+    n, dtype, device = X[0].shape[1], X[0].dtype, X[0].device
+    A = torch.empty((n, n), dtype=dtype, device=device)
+    b = torch.empty((n,), dtype=dtype, device=device)
+    L = _lib.lib()
+    fn = L.a2p_normal_equations_f32 if dtype == torch.float32 else L.a2p_normal_equations_f64
+    three = lambda ts: (_c.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    with torch.cuda.device(device):
+        _lib.check(fn(_c.c_int(n), (_c.c_longlong * 3)(*[t.shape[0] for t in X]), (_c.c_double * 3)(*map(float, weights)),
+                      three(X), three(y), _ptr(A), _ptr(b), _stream(device)))
+    return [A, b]
 
 
 def LinMatrixLinVectorOp(e_weight, f_weight, v_weight, betot_dft, bforce_dft, bvirial_dft, chebyshev_size, scaling,
@@ -951,6 +976,9 @@ def LinMatrixLinVectorOp(e_weight, f_weight, v_weight, betot_dft, bforce_dft, bv
         _req(t.numel() == numel, "%s has %d elements, expected %d" % (name, t.numel(), numel))
     F = fcomp.reshape(B * P * 3, n)          # rows of padded atoms are zero
     V = vcomp.reshape(B * 9, n)
+    labels = (betot_dft, bforce_dft, bvirial_dft)
+    if n <= _NORMAL_EQUATIONS_MOST and all(_only_numbers(t) for t in labels):
+        return _normal_equations((e_weight, f_weight, v_weight), (ecomp, F, V), labels)
     (ae, be), (af, bf), (av, bv) = (_gram(ecomp, betot_dft.reshape(B)), _gram(F, bforce_dft.reshape(-1)),
                                     _gram(V, bvirial_dft.reshape(-1)))
     lin_matrix = e_weight * ae + f_weight * af + v_weight * av

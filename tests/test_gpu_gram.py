@@ -95,12 +95,25 @@ def _solver(oracle, dtype):
     return labels, args
 
 
-def test_labels_that_want_a_gradient(oracle):
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+def test_one_answer_from_both_entry_points(oracle, dtype):
+    """The operator of the bind library and the Python one are the same calls: the same bits."""
+    import torch
+    from ai2pot_amd import ops
+    labels, args = _solver(oracle, getattr(torch, dtype))
+    for a, b in zip(torch.ops.mtpr.LinMatrixLinVectorOp(1.0, 0.7, 0.3, *labels, *args),
+                    ops.LinMatrixLinVectorOp(1.0, 0.7, 0.3, *labels, *args)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("entry", ["bind", "python"])
+def test_labels_that_want_a_gradient(oracle, entry):
     """lin_vector is linear in the labels: u . lin_vector is their product with its gradient, and the numbers are those of
     labels that want none."""
     import torch
     labels, args = _solver(oracle, torch.float64)
-    op = torch.ops.mtpr.LinMatrixLinVectorOp
+    from ai2pot_amd import ops
+    op = torch.ops.mtpr.LinMatrixLinVectorOp if entry == "bind" else ops.LinMatrixLinVectorOp
     A0, b0 = op(1.0, 0.7, 0.3, *labels, *args)
     leaves = [l.clone().requires_grad_(True) for l in labels]
     A, b = op(1.0, 0.7, 0.3, *leaves, *args)
@@ -110,3 +123,9 @@ def test_labels_that_want_a_gradient(oracle):
     grads = torch.autograd.grad((u * b).sum(), leaves)
     total = sum((g * l).sum() for g, l in zip(grads, labels))
     assert abs(float(total - (u * b0).sum())) <= 1e-11 * float((u * b0).abs().sum())
+    if entry == "bind":
+        return                                               # (registered operators have no batching rule)
+    # and a batch of labels, mapped over
+    A2, b2 = torch.func.vmap(lambda *l: tuple(op(1.0, 0.7, 0.3, *l, *args)))(*[torch.stack([l, 2.0 * l]) for l in labels])
+    assert torch.allclose(A2[1], A0, rtol=1e-11, atol=1e-13 * float(A0.abs().max()))
+    assert torch.allclose(b2, torch.stack([b0, 2.0 * b0]), rtol=1e-11, atol=2e-13 * float(b0.abs().max()))
