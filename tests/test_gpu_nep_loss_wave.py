@@ -1,21 +1,20 @@
 """The wavefront-per-atom gradient kernel of the NEP loss at the edges of its tiles (64 slots of a row, 32 pairs inside the
 angular cutoff, 16 columns of a matrix instruction), against the kernel for any shape: the same model with one more basis
-function, whose coefficients are zero, takes that kernel and has the same gradients in its other entries."""
+function, whose coefficients are zero, takes that kernel and has the same gradients in its other entries; and against
+central differences of the oracle's loss."""
 import numpy as np
 import pytest
 
 from ai2pot_amd import synth
-from test_gpu_nep_loss import GRADS, close, gpu_loss
+from test_gpu_nep_loss import GRADS, PARAMS, close, gpu_loss
 
 pytestmark = pytest.mark.gpu
 ROWS = [0, 1, 16, 17, 63, 64, 65, 129, 200]
 INNER = [0, 1, 15, 16, 17, 32, 33, 64, 65]
 
 
-@pytest.mark.parametrize("np_dtype,n_r,l_max,ntypes,H", [(np.float64, 6, 4, 3, 50), (np.float64, 4, 3, 1, 30),
-                                                         (np.float64, 6, 3, 5, 65), (np.float32, 6, 4, 3, 50),
-                                                         (np.float32, 4, 3, 2, 30), (np.float32, 4, 4, 17, 4)])
-def test_tile_edges(np_dtype, n_r, l_max, ntypes, H):
+def edges(np_dtype, n_r, l_max, ntypes, H):
+    """Model, batch and labels whose rows and angular neighbours lie at the tiles' edges."""
     rng = np.random.default_rng(7)
     P, U = len(ROWS) * len(INNER), 200
     rows = np.repeat(ROWS, len(INNER))
@@ -34,10 +33,18 @@ def test_tile_edges(np_dtype, n_r, l_max, ntypes, H):
     m = synth.nep_model(ntypes=ntypes, n_radial_basis=n_r, l_max=l_max, num_neurons=H, sigma=0.12)
     m["type_map"] = np.arange(1, ntypes + 1, dtype=np.int32)
     m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    labels = dict(energy=rng.normal(-5.0, 2.0, 3), force=rng.normal(size=(3, P, 3)), virial=rng.normal(size=(3, 9)))
+    return m, nb, labels
+
+
+@pytest.mark.parametrize("np_dtype,n_r,l_max,ntypes,H", [(np.float64, 6, 4, 3, 50), (np.float64, 4, 3, 1, 30),
+                                                         (np.float64, 6, 3, 5, 65), (np.float32, 6, 4, 3, 50),
+                                                         (np.float32, 4, 3, 2, 30), (np.float32, 4, 4, 17, 4)])
+def test_tile_edges(np_dtype, n_r, l_max, ntypes, H):
+    m, nb, labels = edges(np_dtype, n_r, l_max, ntypes, H)
     wide = dict(m, chebyshev_size=9)
     c = m["coeffs"].reshape(-1, 8)
     wide["coeffs"] = np.concatenate([c, np.zeros((len(c), 1))], axis=1).ravel()
-    labels = dict(energy=rng.normal(-5.0, 2.0, 3), force=rng.normal(size=(3, P, 3)), virial=rng.normal(size=(3, 9)))
     got = gpu_loss(m, nb, labels, (0.9, 1.3, 0.4), np_dtype)
     want = gpu_loss(wide, nb, labels, (0.9, 1.3, 0.4), np_dtype)
     want["dcoeffs"] = want["dcoeffs"].reshape(3, -1, 9)[..., :8].reshape(3, -1)
@@ -46,3 +53,21 @@ def test_tile_edges(np_dtype, n_r, l_max, ntypes, H):
     tol = 1e-12 if np_dtype == np.float64 else 300 * 2.0**-24 * 4
     for k in GRADS:
         assert close(got[k], want[k], tol), (k, np.abs(got[k] - want[k]).max() / np.abs(want[k]).max())
+
+
+@pytest.mark.parametrize("n_r,l_max,ntypes,H", [(6, 4, 3, 50), (4, 3, 1, 30), (6, 3, 2, 65), (4, 4, 3, 4)])
+def test_tile_edges_against_the_oracle(oracle, n_r, l_max, ntypes, H):
+    """Loss, and its derivative along a direction in one group of parameters at a time, by central differences of the
+    oracle's own loss."""
+    m, nb, labels = edges(np.float64, n_r, l_max, ntypes, H)
+    w, h = (0.9, 1.3, 0.4), 1e-6
+    got = gpu_loss(m, nb, labels, w)
+    bloss = oracle.nep_loss(m, nb, w, labels)[0]
+    assert close(got["bloss"], bloss)
+    for i, (gk, pk) in enumerate(zip(GRADS, PARAMS)):
+        d = synth.rng_normal(500 + i, np.size(m[pk])).reshape(np.shape(m[pk]))
+        an, fd = got[gk] @ np.ravel(d), oracle.nep_loss_dirderiv(m, nb, w, labels, {pk: d}, h=h)
+        # the difference's own errors: two losses with some hundred roundings of their terms over 2 h, and the third
+        # derivative over 6 h**-2
+        size = np.abs(got[gk]) @ np.abs(np.ravel(d))
+        assert np.all(np.abs(an - fd) <= 100 * 2.3e-16 * bloss / h + 1e-7 * size), (pk, an, fd)
