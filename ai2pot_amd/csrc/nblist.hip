@@ -548,13 +548,12 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     int total = 0;
     bool in_lds = true;                                          // uniform
 #pragma unroll 1
-    for (int pass = 0; pass < 2 && ok; pass++) {
+    for (int pass = 0; pass < 2 && ok && in_lds; pass++) {
         auto image = [&](int im, int p, int b) __attribute__((always_inline)) {
             const int pos = atomicAdd(&cnt[b], 1);
             if (pass) {
-                const int m = im << NBS_ATOM_BITS | p;           // ordered as the supercell index im * N + p
-                if (in_lds) { num[pos] = m; bin_of_num[pos] = (unsigned short)b; }
-                else { spare[pos] = m; spare[spare_images + pos] = b; }
+                num[pos] = im << NBS_ATOM_BITS | p;              // ordered as the supercell index im * N + p
+                bin_of_num[pos] = (unsigned short)b;
             }
         };
         // the bin along axis a of the image that is i cells along it, or -1 outside the box (separable: the other axes'
@@ -697,8 +696,26 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
                            mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
         }
     };
-    if (in_lds) records(num, bin_of_num);
-    else records(spare, spare + spare_images);
+    if (__builtin_expect(in_lds, 1)) {
+        records(num, bin_of_num);
+        return;
+    }
+    // more images than LDS: their numbers go through global memory (code of its own, so that the common case fetches none
+    // of it: 77.9 -> 77.6 us a step at 4096 atoms)
+#pragma unroll 1
+    for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
+        const int m = w / N, p = w - m * N;
+        const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
+        const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+        T ci[3];
+        const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
+        if (b < 0) continue;
+        const int pos = atomicAdd(&cnt[b], 1);
+        spare[pos] = m << NBS_ATOM_BITS | p;
+        spare[spare_images + pos] = b;
+    }
+    __syncthreads();
+    records(spare, spare + spare_images);
 }
 
 // ---- processing order of the compact lists: atoms along a Morton curve through the bins ----------
