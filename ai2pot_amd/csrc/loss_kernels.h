@@ -25,8 +25,9 @@ loss_forward_kernel(int P, const int* __restrict__ binum, const int* __restrict_
     for (int q = threadIdx.x; q < P * 3; q += 256) dFs[(size_t)b * P * 3 + q] = (T)0;
     __syncthreads();
     double fl = 0.0;
-    for (int ii = threadIdx.x; ii < inum; ii += 256) {
+    for (int ii = threadIdx.x; ii < min(inum, P); ii += 256) {
         const int c = bilist[(size_t)b * P + ii];
+        if ((unsigned)c >= (unsigned)P) continue;      // (reported by the kernels before)
         for (int q = 0; q < 3; q++) {
             const T dlt = force[((size_t)b * P + c) * 3 + q] - f_dft[((size_t)b * P + c) * 3 + q];
             fl += (double)dlt * (double)dlt;

@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
     }
     __syncthreads();
 
-    const int inum = a.binum[b];
+    const int inum = min(a.binum[b], a.P);
     const T cE = a.cE[b], rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
     const int* types = a.btypes + (size_t)b * a.P;
     const T* dv = a.dVs + (size_t)b * 9;
@@ -423,7 +423,7 @@ nep_loss_wave_reduce_kernel(const NepLossArgs<T> a, int sum_blocks, T* __restric
     const int e = min(job * 64 + lane, ncl + 2 * H - 1);         // element of a row
     const int p0 = (job - sum_blocks) * 64 + wave * 16, p = min(p0 + c16, H - 1);
     const int d1 = min(16 + c16, D - 1);
-    const int inum = a.binum[b];
+    const int inum = min(a.binum[b], a.P);
     const T* const rows = a.gpart + (size_t)b * a.P * a.nrow;
     T acc = (T)0;
     typename Acc<T>::type o[2];

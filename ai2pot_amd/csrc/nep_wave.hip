@@ -183,7 +183,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
     if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / a.q_scaler[tid] : (T)0;
     __syncthreads();
 
-    const int inum = a.binum[b];
+    const int inum = min(a.binum[b], a.P);            // (the loop below strides over the rows: none beyond the last)
     const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
     const bool derivs = a.force != nullptr || a.want_virial;
     const int quad = lane >> 2, chan = lane & 3;       // neighbour within a round of 16, angular channel

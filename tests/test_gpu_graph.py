@@ -1,6 +1,6 @@
 """HIP-graph replay of the energy / force / virial operators: every replay is checked against the
 eager result on the same inputs, with eager work and synchronisations between the replays and the
-inputs rewritten in place, for the NEP kernels (8 lanes per atom and a thread per atom) and the MTP."""
+inputs rewritten in place, for the NEP kernels (a wavefront per atom and a thread per atom) and the MTP."""
 import numpy as np
 import pytest
 
@@ -28,7 +28,7 @@ def replay_matches_eager(op, args, brcs, n_out):
     assert not torch.equal(got[0], torch.zeros_like(got[0]))
 
 
-@pytest.mark.parametrize("reps", [4, 21])
+@pytest.mark.parametrize("reps", [4, 22])
 def test_nep_graph(oracle, reps):
     import torch
     from ai2pot_amd import ops

@@ -99,11 +99,11 @@ def test_batch_padding_permuted_ilist(oracle):
     check(run_gpu(m, nb, np.float32), oracle.nep_efv(m, nb, np.float32), np.float32)
 
 
-@pytest.mark.parametrize("reps", [4, 21])
+@pytest.mark.parametrize("reps", [4, 22])
 def test_angular_cutoff_beyond_radial(oracle, reps):
     """A neighbour beyond the radial cutoff is skipped altogether, also when it lies inside a larger
-    angular cutoff (nepBasis.h:106, 135).  256 atoms take the kernel with 8 lanes per atom, 37044
-    atoms the one with a thread per atom."""
+    angular cutoff (nepBasis.h:106, 135).  256 atoms take the kernel with a wavefront per atom, 42592 atoms
+    the one with a thread per atom."""
     lat, pos = synth.fcc_cell(reps, 4.6, 0.15, 61)
     ty = synth.rng_randint(62, pos.shape[0], 3)
     nb = synth.pack_batch([oracle.nblist(lat, ty, pos, 6.0, 100)])
@@ -113,11 +113,11 @@ def test_angular_cutoff_beyond_radial(oracle, reps):
         check(run_gpu(m, nbt, dt), oracle.nep_efv(m, nbt, dt), dt)
 
 
-@pytest.mark.parametrize("reps", [4, 21])
+@pytest.mark.parametrize("reps", [4, 22])
 def test_reference_default_model(oracle, reps):
     """The hyperparameters ai2pot/models/nep/nep.py:32-46 defaults to (n_radial_basis 4, 30 neurons)
-    take the same fast kernels as the benchmark model (n_radial_basis 6): 256 atoms the one with
-    8 lanes per atom, 37044 atoms the staging + model pair."""
+    take the same fast kernels as the benchmark model (n_radial_basis 6): 256 atoms the one with a
+    wavefront per atom, 42592 atoms the staging + model pair."""
     lat, pos = synth.fcc_cell(reps, 4.6, 0.15, 63)
     ty = synth.rng_randint(64, pos.shape[0], 2)
     nb = synth.pack_batch([oracle.nblist(lat, ty, pos, 6.0, 100)])

@@ -67,3 +67,27 @@ def test_tile_edges(oracle, np_dtype, n_r, l_max, ntypes, H, nghost, skin):
         got = [t.cpu().numpy().reshape(o.shape) for t, o in zip((e, f, v), out)]
         check(got, ref, np_dtype)
         assert skin or all(np.array_equal(g, o) for g, o in zip(got, out))
+
+
+@pytest.mark.parametrize("np_dtype", [np.float64, np.float32])
+def test_no_row_beyond_the_last(oracle, np_dtype):
+    """A row count beyond the padded length counts the rows there are (the operators of the bind library take it unread),
+    with a workgroup for every four of them and with fewer."""
+    import torch
+    from ai2pot_amd import ops
+    nb = _lists(np_dtype, 3, 0, 0.0)
+    m = synth.nep_model(sigma=0.12)
+    m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    P = nb["bilist"].shape[1]
+    dtype = torch.float32 if np_dtype == np.float32 else torch.float64
+    md = _model_to_device(m, dtype)
+    for copies in (1, 300):                          # (18 and 3 workgroups of four rows for 72)
+        d = to_device({k: np.repeat(v[:1], copies, axis=0) if isinstance(v, np.ndarray) else v for k, v in nb.items()}, dtype)
+        out = []
+        for rows in (P, P + 100000):
+            r = ops.nepToEFVOp(m["chebyshev_size"], m["n_radial_basis"], m["n_angular_basis"], m["l_max"], md["coeffs"],
+                               md["w0"], md["b0"], md["w1"], md["type_bias"], torch.full_like(d["binum"], rows), d["bilist"],
+                               d["bnumneigh"], d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], 0, m["rmax_radial"],
+                               m["rmax_angular"], md["q_scaler"], 0.0, 0.0, None, None, validate=False)
+            out.append([t.cpu() for t in r])
+        assert all(torch.equal(a, b) for a, b in zip(*out))
