@@ -16,7 +16,7 @@
 //               of the largest term, i.e. below the rounding error of a floating sum.
 // Three short launches, bound by their latency for systems of a few thousand atoms (counting, a prefix sum in three
 // launches and a copy of the derivatives in place of the claim took ten).  Force and virial of 4 x 1000 atoms with their
-// gradients, fp64: 65 us of kernels, of which claim 10.9 and reduce 5.6, in a call of 105 to 122 us (202 with the ten).
+// gradients, fp64: 65 us of kernels, of which claim 10.9 and reduce 5.6, in a call of 123 us on average (202 with the ten).
 // No floating-point atomics are used.
 #include "a2p_common.h"
 
