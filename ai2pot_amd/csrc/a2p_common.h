@@ -49,11 +49,12 @@ enum WsSlot {
     WS_GRID,           // neighbor-list: the bin grid derived on the device (builds without read-back)
     WS_NEP_CLAIMS,     // NEP on compact lists: counters of claimed places and spare rows; zero between calls
     WS_HOST_LISTS,     // neighbour lists on their way to host arrays
+    WS_CURSORS,        // pair reduction: cursors and chain heads of the targets; zero between calls
     WS_NSLOTS
 };
 // Returns a device pointer valid until the next ws_get on the same slot with a larger size.
 // Growth synchronises the device (hipFree); steady-state calls do not allocate.
-// WS_FLAGS and WS_NEP_CLAIMS are zero-filled when they are allocated; their users leave them zero.
+// WS_FLAGS, WS_NEP_CLAIMS and WS_CURSORS are zero-filled when they are allocated; their users leave them zero.
 int ws_get(int slot, size_t bytes, void** out);
 int ws_drop(int slot); // synchronises the device and frees one buffer of the current device (its contents are suspect)
 size_t ws_bytes();     // held on the current device
@@ -98,6 +99,15 @@ __device__ __forceinline__ void read_back_store(int* slot, int seq, const int* w
 // Called where every check of the call's inputs has been queued: posts the status word if the calling thread asked
 // for it (a2p_status_early).
 int status_post_early(hipStream_t stream);
+// The same for a kernel that is launched at that point anyway and posts the word itself (read_back_store of *flags, by one
+// lane): slot is null when nothing was asked for or no slot is free.  early_posted tells whether the kernel was launched.
+struct EarlyPost {
+    int* slot;
+    int seq;
+    const int* flags;
+};
+int early_take(hipStream_t stream, EarlyPost* post);
+void early_posted(const EarlyPost& post, bool launched);
 // The same for a call whose own check is all that is asked for: its kernel stores a non-zero value to the word of pinned
 // memory that early_word gives (null: nothing was asked for, or no slot is free; the latter is *no_slot), and
 // early_word_post, behind that kernel, ends the report.  The shared status word is left alone.  early_word_known reports
@@ -184,29 +194,40 @@ int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, cons
 int pair_segment_capacity(int U);
 // pair_fixed_begin: every target owns a segment of fixed capacity seg_cap (umax by default)
 // (a cutoff-built list sends an atom no more pairs than its own row could hold); the producer
-// claims  rank = atomicAdd(&cursor[t], 1),  stores at  pos = t*seg_cap + rank  when rank < seg_cap
-// and otherwise raises ST_SEG_OVERFLOW and stores at the spare entry n*seg_cap.
+// claims  rank = pair_claim(&cursor[t]),  stores at  pos = t*seg_cap + rank  when rank < seg_cap
+// and otherwise raises ST_SEG_OVERFLOW and stores at the spare entry n*seg_cap.  Where it stores an atom's own sum to
+// `force` it calls pair_mark_own on the atom's cursor when `mark` is set: the reduction then takes every other atom's own
+// sum for zero, so that `force` needs no clearing, and leaves the cursors zero for the next call.
+constexpr int PAIR_OWN = (int)0x80000000;          // counts stay below 2^31
+__device__ __forceinline__ int pair_claim(int* cursor) { return atomicAdd(cursor, 1) & ~PAIR_OWN; }
+__device__ __forceinline__ void pair_mark_own(int* cursor) { atomicOr(cursor, PAIR_OWN); }
 struct PairCsr {
-    int* cursor;
-    void* seg_g;
-    int n;          // B * (P + nghost) targets
-    int seg_cap;
+    int* cursor = nullptr;
+    void* seg_g = nullptr;
+    int n = 0;          // B * (P + nghost) targets
+    int seg_cap = 0;
+    int mark = 0;
+    PairCsr() = default;
+    PairCsr(const PairCsr&) = delete;
+    PairCsr& operator=(const PairCsr&) = delete;
+    ~PairCsr() { if (mark) (void)ws_drop(WS_CURSORS); }     // begun and not finished (a launch failed): not known to be zero
 };
 template <typename T>
-int pair_fixed_begin(PairCsr* csr, int B, int P, int U, int nghost, hipStream_t stream, void* also_zero = nullptr,
-                     size_t also_bytes = 0, int* cursor_ext = nullptr, bool cursor_final = false);
+int pair_fixed_begin(PairCsr* csr, int B, int P, int U, int nghost, hipStream_t stream, T* force, int* cursor_ext = nullptr,
+                     bool cursor_final = false);
 // cursor_ext (optional): the caller's array takes the place of the cursors, so that the counts
 // survive the call; cursor_final: it already holds the final counts (every pair's place is known
-// from an earlier call), so it is neither zeroed nor written.
+// from an earlier call), so it is neither zeroed nor written.  Nothing is marked then: `force` is cleared by a launch.
 
 // rank[B, P, U] = index of pair (row, slot) among the pairs naming the same neighbour (-1 for an
 // index out of range), incoming[B, P+nghost] = number of pairs naming each atom.
 int pair_ranks(int B, int P, int U, int nghost, const int* binum, const int* bnumneigh, const int* bfirstneigh,
                int* rank, int* incoming, hipStream_t stream);
+// Posts the status word if the calling thread asked for it (status_post_early).
 // With etot or virial given, the same launch also sums the energy / virial partials
 // (finish_energy_virial's work, in workgroups of its own behind those of the segments).
 template <typename T>
-int pair_csr_finish(T* force, const PairCsr& csr, hipStream_t stream, T* etot = nullptr, T* virial = nullptr,
+int pair_csr_finish(T* force, PairCsr& csr, hipStream_t stream, T* etot = nullptr, T* virial = nullptr,
                     const double* partial = nullptr, int B = 0, int nblocks = 0);
 
 // out[b*out_stride + c] = sum over blocks of partial[(b*nblocks + block)*src_stride + c], c < ncomp,

@@ -119,11 +119,11 @@ struct EarlyStatus {
 // A list that names an atom more often than a row is long (half lists, ghosts collecting the pairs of
 // several rows) overflows the fixed reduction segments of the fast kernels: the status says so and
 // the call is repeated once with segments sized for the list at hand.
-// early: a loss call, whose status is final before its gradient kernels run; the host then goes on (to the backward
-// call, as a rule) while they do.
+// early: the status is final before the call's last kernels (the reduction of the forces, the gradients of a loss), and the
+// host goes on while they run; a call without such a point is waited for as a whole.
 template <class Call>
 inline void run_checked(const at::Tensor& brcs, const at::Tensor& binum, const at::Tensor& bnumneigh,
-                        const at::Tensor& bfirstneigh, int nghost, Call&& call, bool early = false)
+                        const at::Tensor& bfirstneigh, int nghost, Call&& call, bool early = true)
 {
     EarlyStatus status(early && validate_flag());
     check_rc(call());

@@ -137,7 +137,7 @@ struct LossFunction : public torch::autograd::Function<LossFunction> {
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
         save_grad_rows(ctx, need, rows, {&coeffs, &lin, &bias});
         if (with_virial) return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1}), piece(rmse, 2, {1})};
         return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1})};
@@ -395,7 +395,7 @@ variable_list lin_matrix_lin_vector(double e_w, double f_w, double v_w, const at
         }
         return rc;
     };
-    run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
+    run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, false);
     // (wider systems keep a matrix product busy by themselves)
     if (n <= 575 && only_numbers(e_dft) && only_numbers(f_dft) && only_numbers(v_dft)) {
         at::Tensor A = at::empty({n, n}, opt), b = at::empty({n}, opt);

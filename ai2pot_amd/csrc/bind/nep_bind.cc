@@ -210,7 +210,7 @@ struct NepLossFunction : public torch::autograd::Function<NepLossFunction> {
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
         save_grad_rows(ctx, need, rows, {&coeffs, &w0, &b0, &w1, &bias});
         if (with_virial) return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1}), piece(rmse, 2, {1})};
         return {bloss, piece(rmse, 0, {1}), piece(rmse, 1, {1})};

@@ -262,7 +262,7 @@ struct NNLossFunction : public torch::autograd::Function<NNLossFunction> {
             }
             return rc;
         };
-        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call, true);
+        run_checked(brcs, binum, bnumneigh, bfirstneigh, 0, call);
         save_grad_rows(ctx, need, rows, {&coeffs, &w0, &w1, &bias});
         return {bloss};
     }

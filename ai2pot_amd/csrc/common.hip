@@ -114,7 +114,10 @@ int ws_get(int slot, size_t bytes, void** out)
         size_t want = bytes + bytes / 8 + 256;      // head-room so small growth does not realloc
         A2P_HIP_CHECK(hipMalloc(&b.ptr, want));
         b.bytes = want;
-        if (slot == WS_FLAGS || slot == WS_NEP_CLAIMS) A2P_HIP_CHECK(hipMemset(b.ptr, 0, want));
+        if (slot == WS_FLAGS || slot == WS_NEP_CLAIMS || slot == WS_CURSORS) {
+            A2P_HIP_CHECK(hipMemset(b.ptr, 0, want));
+            A2P_HIP_CHECK(hipStreamSynchronize(nullptr));      // callers' streams need not wait for the null stream
+        }
     }
     *out = b.ptr;
     return A2P_OK;
@@ -308,6 +311,28 @@ void early_word_known(int word)
 }
 
 void early_word_drop() { read_back_drop(g_early); }
+
+int early_take(hipStream_t stream, EarlyPost* post)
+{
+    *post = EarlyPost{nullptr, 0, nullptr};
+    if (!g_early_asked || g_early_posted) return A2P_OK;
+    void* flags = nullptr;
+    const int rc = ws_get(WS_FLAGS, 64, &flags);
+    if (rc) return rc;
+    post->flags = (const int*)flags;
+    post->slot = read_back_take(1, stream, &g_early);
+    post->seq = g_early.seq;
+    g_early.src = flags;                 // more waiters than slots: read_back_wait copies instead
+    if (!post->slot) g_early_posted = true;
+    return A2P_OK;
+}
+
+void early_posted(const EarlyPost& post, bool launched)
+{
+    if (!post.slot) return;
+    if (launched) g_early_posted = true;
+    else read_back_drop(g_early);
+}
 
 int status_post_early(hipStream_t stream)
 {

@@ -96,6 +96,7 @@ struct MtpArgs {
     T* seg_g;          // the entries, and the entry that takes what overflows a segment;
     int seg_spare;     // seg_cursor is null when no forces are wanted
     int seg_cap;       // capacity of a segment
+    int seg_mark;      // own sums are marked in the cursors
     double* partial;   // [B, P, 10]  energy + virial per atom
     int* status;
     int E;             // table entries per neighbour
@@ -705,7 +706,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
             // naming the target); claimed here, so that the walk covers the answer's way
             const int tg = b * NF + nj;
             int rk = 0;
-            if (a.seg_cursor && lane < nc) rk = atomicAdd(&a.seg_cursor[tg], 1);
+            if (a.seg_cursor && lane < nc) rk = pair_claim(&a.seg_cursor[tg]);
             T gs = (T)0, wx = (T)0, wy = (T)0, wz = (T)0;
             T ux = (T)0, uy = (T)0, uz = (T)0, rinv = (T)0;
             if (h < ng) {
@@ -758,6 +759,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
             if (!SEED || a.force) {
                 T* fo = a.force + ((size_t)b * NF + center) * 3;
                 fo[0] = fx; fo[1] = fy; fo[2] = fz;
+                if (a.seg_mark) pair_mark_own(&a.seg_cursor[b * NF + center]);
             }
             if (!SEED || a.partial) {
 #pragma unroll
@@ -1942,7 +1944,8 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.binum = binum; a.bilist = bilist; a.bnumneigh = bnumneigh; a.bfirstneigh = bfirstneigh;
     a.brcs = brcs; a.btypes = btypes;
     a.cE = nullptr; a.dFs = nullptr; a.dVs = nullptr; a.gpart = nullptr; a.ngrad = 0;
-    a.force = nullptr; a.seg_cursor = nullptr; a.seg_g = nullptr; a.seg_spare = 0; a.seg_cap = 0; a.partial = nullptr;
+    a.force = nullptr; a.seg_cursor = nullptr; a.seg_g = nullptr; a.seg_spare = 0; a.seg_cap = 0; a.seg_mark = 0;
+    a.partial = nullptr;
     a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0;
     a.nn_exact = 1;
     a.row_seed = nullptr; a.pair_out = nullptr;
@@ -2080,14 +2083,15 @@ int mtp_efv(void* handle, int K, double scaling, const T* coeffs, const T* lin, 
         if (rc) return rc;
         a.force = (T*)ws;
     }
-    PairCsr csr{};
-    if (force) {       // the force array is zeroed with the cursors (the reference zeroes on entry, linearMtp.h:228-230)
-        rc = pair_fixed_begin<T>(&csr, B, P, U, nghost, stream, a.force, force_bytes);
+    PairCsr csr;
+    if (force) {       // (atoms without a row start from zero, linearMtp.h:228-230)
+        rc = pair_fixed_begin<T>(&csr, B, P, U, nghost, stream, a.force);
         if (rc) return rc;
         a.seg_cursor = csr.cursor;
         a.seg_g = (T*)csr.seg_g;
         a.seg_spare = csr.n * csr.seg_cap;
         a.seg_cap = csr.seg_cap;
+        a.seg_mark = csr.mark;
     } else {
         rc = fill_zero(a.force, force_bytes, stream);
         if (rc) return rc;

@@ -166,7 +166,7 @@ __device__ __forceinline__ void staged_load(const NepArgs<T>& a, const SegArgs& 
             if (a.brank && a.ranks_valid) {
                 rk = pos[it];
             } else {
-                rk = atomicAdd(&seg.cursor[t], 1);
+                rk = pair_claim(&seg.cursor[t]);
                 if (a.brank) {                         // recorded for the later calls on the same list
                     const int e = it * SB + tid;
                     a.brank[(rowbase + e / SCH) * a.U + c0 + e % SCH] = rk;
@@ -362,7 +362,7 @@ nep_stage_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g, T
 
 template <typename T, int NTC, int NR>
 __global__ void __launch_bounds__(FB, (sizeof(T) == 4 ? 2 : 1))
-nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, const T* __restrict__ ang_xyz,
+nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, int* __restrict__ own_mark, const T* __restrict__ ang_xyz,
                   const unsigned* __restrict__ typew, const T* __restrict__ radial, const int* __restrict__ counts)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -653,6 +653,7 @@ nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, const T*
         if (active && a.force) {
             T* fo = a.force + ((size_t)b * NF + center) * 3;
             fo[0] = fx; fo[1] = fy; fo[2] = fz;
+            if (own_mark) pair_mark_own(&own_mark[b * NF + center]);
         }
     }
 
@@ -709,7 +710,8 @@ int launch_staged(const NepArgs<T>& a, size_t lds, const PairCsr& csr, hipStream
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)lds));
     prof_begin("nep_staged_kernel", stream);
-    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(FB), lds, stream, a, (T*)csr.seg_g, seg.spare, (const T*)ang_xyz,
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(FB), lds, stream, a, (T*)csr.seg_g, seg.spare,
+                       csr.mark ? csr.cursor : (int*)nullptr, (const T*)ang_xyz,
                        (const unsigned*)typew, (const T*)radial, (const int*)counts);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
@@ -735,11 +737,10 @@ bool nep_staged_supported(const NepArgs<T>& a, size_t* lds_bytes)
 template <typename T>
 int nep_staged_run(const NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream)
 {
-    PairCsr csr{};
+    PairCsr csr;
     int rc;
     if (a.force) {
-        rc = pair_fixed_begin<T>(&csr, a.B, a.P, a.U, a.nghost, stream, a.force,
-                                 (size_t)a.B * (a.P + a.nghost) * 3 * sizeof(T), a.bincoming,
+        rc = pair_fixed_begin<T>(&csr, a.B, a.P, a.U, a.nghost, stream, a.force, a.bincoming,
                                  a.bincoming != nullptr && a.ranks_valid != 0);
         if (rc) return rc;
     }

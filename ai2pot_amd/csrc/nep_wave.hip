@@ -84,6 +84,7 @@ struct SegArgs {
     int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
     int cap;       // capacity of a segment
     int spare;     // entry that takes what overflows a segment
+    int mark;      // own sums are marked in the cursors (PairCsr)
 };
 
 // Slots [128 t, 128 t + 128) of a row into the wavefront's tile; nA / nR: entries at its front / back.
@@ -136,7 +137,7 @@ __device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& se
             if (a.brank && a.ranks_valid) {
                 rk = a.brank[pr];
             } else {
-                rk = atomicAdd(&seg.cursor[tg], 1);
+                rk = pair_claim(&seg.cursor[tg]);
                 if (a.brank) a.brank[pr] = rk;
             }
             pos = (unsigned)rk < (unsigned)seg.cap ? tg * seg.cap + rk : seg.spare;
@@ -412,6 +413,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
         if (a.force) {
             fx = all_sum(fx); fy = all_sum(fy); fz = all_sum(fz);
             if (lane < 3) a.force[((size_t)b * NF + center) * 3 + lane] = lane == 0 ? fx : lane == 1 ? fy : fz;
+            if (seg.mark && lane == 3) pair_mark_own(&seg.cursor[b * NF + center]);
         }
     }
 
@@ -433,7 +435,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
 template <typename T, int NR, int LC>
 int launch_wave(const NepArgs<T>& a, size_t lds, const PairCsr& csr, hipStream_t stream)
 {
-    SegArgs seg{csr.cursor, csr.seg_cap, csr.n * csr.seg_cap};
+    SegArgs seg{csr.cursor, csr.seg_cap, csr.n * csr.seg_cap, csr.mark};
     auto kern = nep_wave_kernel<T, NR, LC>;
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -465,11 +467,10 @@ bool nep_wave_supported(const NepArgs<T>& a, size_t* lds_bytes)
 template <typename T>
 int nep_wave_run(const NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream)
 {
-    PairCsr csr{};
+    PairCsr csr;
     int rc;
     if (a.force) {
-        rc = pair_fixed_begin<T>(&csr, a.B, a.P, a.U, a.nghost, stream, a.force,
-                                 (size_t)a.B * (a.P + a.nghost) * 3 * sizeof(T), a.bincoming,
+        rc = pair_fixed_begin<T>(&csr, a.B, a.P, a.U, a.nghost, stream, a.force, a.bincoming,
                                  a.bincoming != nullptr && a.ranks_valid != 0);
         if (rc) return rc;
     }

@@ -3,20 +3,23 @@
 // neighbour is j  on top of the sum over its own row that the producing kernel stored.
 //
 // Steps (all on `stream`):
-//   1. clear  : a cursor and the heads of sixteen chains per target (and the caller's force array)
-//   2. claim  : every pair takes an entry of its target's segment (a returning integer atomic; the order inside a
+//   1. claim  : every pair takes an entry of its target's segment (a returning integer atomic; the order inside a
 //               segment is therefore arbitrary) and leaves its number there.  Segments hold as many pairs as a row: a
 //               list built with one cutoff never needs more.  What does not fit (half lists, ghosts that collect the pairs
 //               of several rows) is chained behind the target, its pairs dealt to the sixteen chains in turn
-//   3. reduce : per target, order-independent sum over the pairs named: every term is converted to 64-bit fixed
+//   2. reduce : per target, order-independent sum over the pairs named: every term is converted to 64-bit fixed
 //               point against the segment's largest magnitude, integers are added (exact,
 //               associative), the total is converted back.  The result is identical for
 //               any arrival order, so the output is bit-reproducible run to run; the
 //               conversion error per term is below 2^-37 (fp32 inputs) / 2^-52 (fp64 inputs)
 //               of the largest term, i.e. below the rounding error of a floating sum.
-// Three short launches, bound by their latency for systems of a few thousand atoms (counting, a prefix sum in three
-// launches and a copy of the derivatives in place of the claim took ten).  Force and virial of 4 x 1000 atoms with their
-// gradients, fp64: 65 us of kernels, of which claim 10.9 and reduce 5.6, in a call of 123 us on average (202 with the ten).
+// The cursors and chain heads are zero between calls: step 2 clears what step 1 wrote.  Step 1 also marks in its cursor
+// an atom whose own sum it stored, so the output needs no clearing either.  With the status word leaving by step 2 as well
+// (instead of a kernel behind it), an energy / force call of 216 atoms takes 32.2 instead of 37.8 us (level-10 MTP), of
+// 20,011 atoms and their ghosts 102.8 instead of 113 (NEP).
+// Two short launches, bound by their latency for systems of a few thousand atoms.  Force and virial of 4 x 1000 atoms with
+// their gradients, fp64: 59 us of kernels, of which claim 10.8 and reduce 5.5 (65 with a launch that cleared and one that
+// sent the status).
 // No floating-point atomics are used.
 #include "a2p_common.h"
 
@@ -134,7 +137,7 @@ __global__ void scan_apply(const int* __restrict__ in, int* __restrict__ out,
 // collects the pairs of 6,250 rows.
 constexpr int SPILL_CHAINS = 16;
 
-// Claims of step 2, one wavefront per row.  With OWN the wavefront also sums the row itself and stores it as the force
+// Claims of step 1, one wavefront per row.  With OWN the wavefront also sums the row itself and stores it as the force
 // on the row's centre (a centre has one row).
 template <typename T, bool OWN>
 __global__ void __launch_bounds__(256)
@@ -163,7 +166,7 @@ claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum
             continue;
         }
         const int t = b * NF + j;
-        const int k = atomicAdd(&cursor[t], 1);
+        const int k = pair_claim(&cursor[t]);
         const int pair = row * U + s;
         if (k < cap) seg[(size_t)t * cap + k] = pair;
         else next[pair] = atomicExch(&heads[(size_t)t * SPILL_CHAINS + (k - cap) % SPILL_CHAINS], pair + 1);   // 0 ends a chain
@@ -176,21 +179,29 @@ claim_kernel(int B, int P, int U, int NF, int cap, const int* __restrict__ binum
         } else if (lane == 0) {
             T* f = force + ((size_t)b * NF + c) * 3;
             f[0] = sx; f[1] = sy; f[2] = sz;
+            pair_mark_own(&cursor[b * NF + c]);
         }
     }
 }
 
 // 16 lanes per target atom.  Workgroups from `reduce_blocks` on sum the energy / virial partials
 // instead (one component of one structure each), which saves small systems a launch.
+// With `clear` the cursors (and the heads of the chains in use) are left zero; with `marked` an atom without its producer's
+// mark has no own sum in `force` yet.  The status word leaves with the first workgroup when it was asked for: every check of the
+// producers is behind this launch, so a caller that waits for it waits for no launch of its own, nor for the sums.
 // NAMED: the segments hold the numbers of the pairs (claim_kernel), otherwise the derivatives themselves.
 // The first four entries of every lane stay in registers between the two passes (largest magnitude, then the sum).
 template <typename T, bool NAMED>
 __global__ void __launch_bounds__(256)
-reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __restrict__ counts, int NT, int seg_cap,
-              const int* __restrict__ seg_pair, const int* __restrict__ heads, const int* __restrict__ next,
-              int reduce_blocks, T* __restrict__ etot, T* __restrict__ virial, const double* __restrict__ partial,
+reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restrict__ counts, int clear, int marked, int NT, int seg_cap,
+              const int* __restrict__ seg_pair, int* __restrict__ heads, const int* __restrict__ next,
+              const EarlyPost post, int reduce_blocks, T* __restrict__ etot, T* __restrict__ virial, const double* __restrict__ partial,
               int nblocks)
 {
+    if (post.slot && blockIdx.x == 0 && threadIdx.x == 0) {
+        const int word = *post.flags;
+        read_back_store(post.slot, post.seq, &word, 1);
+    }
     if ((int)blockIdx.x >= reduce_blocks) {
         __shared__ double sh[256];
         const int id = (int)blockIdx.x - reduce_blocks;
@@ -200,7 +211,15 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __r
     const int t = (int)(blockIdx.x * 16u + (threadIdx.x >> 4));       // 256 threads
     const int sub = threadIdx.x & 15;
     // target t owns entries [t*seg_cap, (t+1)*seg_cap); uniform over the 16 lanes of a target
-    const int all = t < NT ? counts[t] : 0;
+    int all = t < NT ? counts[t] : 0;
+    T* const fo = force + (size_t)t * 3;
+    bool own = true;
+    if (clear) {
+        own = !marked || all < 0;
+        if (all != 0 && sub == 0) counts[t] = 0;         // the lanes of a target read it in one instruction
+        all &= ~PAIR_OWN;
+        if (!own && all == 0 && t < NT && sub == 0) fo[0] = fo[1] = fo[2] = (T)0;
+    }
     const int cnt = min(all, seg_cap);
     if (all == 0) return;
     const size_t beg = (size_t)t * seg_cap;
@@ -224,7 +243,6 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __r
             gx[k] = g[0]; gy[k] = g[1]; gz[k] = g[2];
         }
     }
-    T* const fo = force + (size_t)t * 3;
     if constexpr (sizeof(T) == 4) {
         // fp32 segments: every value is rounded to a multiple of 2^q, q chosen from the segment's
         // largest magnitude and its length so that any partial sum of the rounded values fits the
@@ -272,10 +290,10 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __r
         if (sub == 0) {
             if (!finite) {
                 fo[0] = fo[1] = fo[2] = (T)NAN;
-            } else if (any) {
-                fo[0] = (T)((double)fo[0] - s0);
-                fo[1] = (T)((double)fo[1] - s1);
-                fo[2] = (T)((double)fo[2] - s2);
+            } else if (any || !own) {
+                fo[0] = (T)((own ? (double)fo[0] : 0.0) - s0);
+                fo[1] = (T)((own ? (double)fo[1] : 0.0) - s1);
+                fo[2] = (T)((own ? (double)fo[2] : 0.0) - s2);
             }
         }
     } else {
@@ -317,12 +335,15 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, const int* __r
             if (!finite) {
                 fo[0] = fo[1] = fo[2] = (T)NAN;
             } else if (m > 0.0) {
-                fo[0] = (T)((double)fo[0] - (double)s0 / scale);
-                fo[1] = (T)((double)fo[1] - (double)s1 / scale);
-                fo[2] = (T)((double)fo[2] - (double)s2 / scale);
+                fo[0] = (T)((own ? (double)fo[0] : 0.0) - (double)s0 / scale);
+                fo[1] = (T)((own ? (double)fo[1] : 0.0) - (double)s1 / scale);
+                fo[2] = (T)((own ? (double)fo[2] : 0.0) - (double)s2 / scale);
+            } else if (!own) {
+                fo[0] = fo[1] = fo[2] = (T)0;
             }
         }
     }
+    if (NAMED && clear && all > seg_cap) heads[(size_t)t * SPILL_CHAINS + sub] = 0;     // each lane its own chain's
 }
 
 }  // namespace
@@ -351,28 +372,32 @@ static thread_local int g_seg_capacity = 0;
 int pair_segment_capacity(int U) { return g_seg_capacity > U ? g_seg_capacity : U; }
 
 template <typename T>
-int pair_fixed_begin(PairCsr* csr, int B, int P, int U_rows, int nghost, hipStream_t stream, void* also_zero,
-                     size_t also_bytes, int* cursor_ext, bool cursor_final)
+int pair_fixed_begin(PairCsr* csr, int B, int P, int U_rows, int nghost, hipStream_t stream, T* force, int* cursor_ext,
+                     bool cursor_final)
 {
     const int U = pair_segment_capacity(U_rows);
     const long long NT = (long long)B * (P + nghost);
     A2P_REQUIRE(NT * U + 1 < (1ll << 31), A2P_ERR_INVALID,
                 "pair_reduce: (natoms_pad + nghost) * segment capacity exceeds 32-bit pair indexing");
     const int n = (int)NT;
-    // workspace: cursor[n] | seg_g[(n*U + 1) * 3]   (the last entry takes what overflows)
-    size_t bytes = (((size_t)n * sizeof(int) + 255) / 256) * 256;
-    size_t seg_bytes = ((size_t)n * U + 1) * 3 * sizeof(T);
+    // seg_g[(n*U + 1) * 3]: the last entry takes what overflows
     void* ws = nullptr;
-    int rc = ws_get(WS_CSR, bytes + seg_bytes, &ws);
+    int rc = ws_get(WS_CSR, ((size_t)n * U + 1) * 3 * sizeof(T), &ws);
     if (rc) return rc;
     csr->n = n;
     csr->seg_cap = U;
+    csr->seg_g = ws;
+    if (cursor_ext) {                                    // the caller keeps the counts
+        csr->cursor = cursor_ext;
+        const size_t force_bytes = (size_t)n * 3 * sizeof(T);
+        if (cursor_final) return fill_zero(force, force_bytes, stream);      // ... and every pair's place is known
+        return fill_zero2(cursor_ext, (size_t)n * sizeof(int), force, force_bytes, stream);
+    }
+    rc = ws_get(WS_CURSORS, (size_t)n * sizeof(int), &ws);
+    if (rc) return rc;
     csr->cursor = (int*)ws;
-    csr->seg_g = (void*)((char*)ws + bytes);
-    if (cursor_ext) csr->cursor = cursor_ext;            // the caller keeps the counts
-    if (cursor_ext && cursor_final)                      // ... and they are final: every pair's place is known
-        return fill_zero(also_zero, also_bytes, stream);
-    return fill_zero2(csr->cursor, (size_t)n * sizeof(int), also_zero, also_bytes, stream);
+    csr->mark = 1;
+    return A2P_OK;
 }
 
 int pair_ranks(int B, int P, int U, int nghost, const int* binum, const int* bnumneigh, const int* bfirstneigh,
@@ -396,17 +421,23 @@ int pair_ranks(int B, int P, int U, int nghost, const int* binum, const int* bnu
 }
 
 template <typename T>
-int pair_csr_finish(T* force, const PairCsr& csr, hipStream_t stream, T* etot, T* virial, const double* partial,
+int pair_csr_finish(T* force, PairCsr& csr, hipStream_t stream, T* etot, T* virial, const double* partial,
                     int B, int nblocks)
 {
+    EarlyPost post;
+    const int rc = early_take(stream, &post);
+    if (rc) return rc;
     const int reduce_blocks = ceil_div((long long)csr.n * 16, 256);
     const int ev_blocks = (etot || virial) ? 10 * B : 0;
     prof_begin("reduce_sum", stream);
     hipLaunchKernelGGL((reduce_kernel<T, false>), dim3(reduce_blocks + ev_blocks), dim3(256), 0, stream,
-                       force, (const T*)csr.seg_g, (const int*)csr.cursor, csr.n, csr.seg_cap, (const int*)nullptr,
-                       (const int*)nullptr, (const int*)nullptr, reduce_blocks, etot, virial, partial, nblocks);
+                       force, (const T*)csr.seg_g, csr.cursor, csr.mark, csr.mark, csr.n, csr.seg_cap, (const int*)nullptr,
+                       (int*)nullptr, (const int*)nullptr, post, reduce_blocks, etot, virial, partial, nblocks);
     prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
+    const hipError_t err = hipGetLastError();
+    early_posted(post, err == hipSuccess);
+    A2P_HIP_CHECK(err);
+    csr.mark = 0;                                        // the cursors are zero again behind this launch
     return A2P_OK;
 }
 
@@ -419,44 +450,47 @@ int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, cons
     A2P_REQUIRE(NT < (1ll << 31) - 1 && rows * U < (1ll << 31), A2P_ERR_INVALID,
                 "pair_reduce: batch too large for 32-bit pair indexing");
     const int n = (int)NT;
-    // workspace: cursor[n] | heads[n*16] | seg[n*U] | next[rows*U] (by pair)
-    const size_t clear_bytes = (size_t)n * (1 + SPILL_CHAINS) * sizeof(int);
-    const size_t head = (clear_bytes + 255) / 256 * 256;
+    // workspace: seg[n*U] | next[rows*U] (by pair), and cursor[n] | heads[n*16]
     const size_t seg_bytes = ((size_t)n * U * sizeof(int) + 255) / 256 * 256;
-    void* ws = nullptr;
-    int rc = ws_get(WS_CSR, head + seg_bytes + (size_t)rows * U * sizeof(int), &ws);
+    void *ws = nullptr, *cursors = nullptr;
+    int rc = ws_get(WS_CSR, seg_bytes + (size_t)rows * U * sizeof(int), &ws);
     if (rc) return rc;
-    int* cursor = (int*)ws;
-    int* heads = cursor + n;
-    int* seg = (int*)((char*)ws + head);
-    int* next = (int*)((char*)ws + head + seg_bytes);
+    int* seg = (int*)ws;
+    int* next = (int*)((char*)ws + seg_bytes);
     rc = ws_get(WS_FLAGS, 64, &ws);
     if (rc) return rc;
-    // own: the rows' own sums are formed here, and atoms without a row start from zero
-    rc = fill_zero2(cursor, clear_bytes, own ? (void*)force : nullptr, own ? (size_t)n * 3 * sizeof(T) : 0,
-                    stream);
+    rc = ws_get(WS_CURSORS, (size_t)n * (1 + SPILL_CHAINS) * sizeof(int), &cursors);
     if (rc) return rc;
+    PairCsr csr;                                         // (gives the cursors up when a launch fails)
+    csr.cursor = (int*)cursors;
+    csr.mark = 1;
+    int* const cursor = csr.cursor;
+    int* const heads = cursor + n;
     prof_begin("reduce_claim", stream);
     hipLaunchKernelGGL((own ? claim_kernel<T, true> : claim_kernel<T, false>), dim3(ceil_div(rows * 64, 256)), dim3(256), 0,
                        stream, B, P, U, NF, U, binum, bilist, bnumneigh, bfirstneigh, pair_g, cursor, seg, heads, next,
                        force, (int*)ws);
     prof_end(stream);
-    rc = status_post_early(stream);
+    EarlyPost post;
+    rc = early_take(stream, &post);
     if (rc) return rc;
     const int reduce_blocks = ceil_div((long long)n * 16, 256);
     prof_begin("reduce_sum", stream);
     hipLaunchKernelGGL((reduce_kernel<T, true>), dim3(reduce_blocks), dim3(256), 0, stream, force, pair_g,
-                       (const int*)cursor, n, U, (const int*)seg, (const int*)heads, (const int*)next, reduce_blocks,
+                       cursor, 1, own ? 1 : 0, n, U, (const int*)seg, heads, (const int*)next, post, reduce_blocks,
                        (T*)nullptr, (T*)nullptr, (const double*)nullptr, 0);
     prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
+    const hipError_t err = hipGetLastError();
+    early_posted(post, err == hipSuccess);
+    A2P_HIP_CHECK(err);
+    csr.mark = 0;
     return A2P_OK;
 }
 
-template int pair_fixed_begin<float>(PairCsr*, int, int, int, int, hipStream_t, void*, size_t, int*, bool);
-template int pair_fixed_begin<double>(PairCsr*, int, int, int, int, hipStream_t, void*, size_t, int*, bool);
-template int pair_csr_finish<float>(float*, const PairCsr&, hipStream_t, float*, float*, const double*, int, int);
-template int pair_csr_finish<double>(double*, const PairCsr&, hipStream_t, double*, double*, const double*, int, int);
+template int pair_fixed_begin<float>(PairCsr*, int, int, int, int, hipStream_t, float*, int*, bool);
+template int pair_fixed_begin<double>(PairCsr*, int, int, int, int, hipStream_t, double*, int*, bool);
+template int pair_csr_finish<float>(float*, PairCsr&, hipStream_t, float*, float*, const double*, int, int);
+template int pair_csr_finish<double>(double*, PairCsr&, hipStream_t, double*, double*, const double*, int, int);
 template int pair_reduce<float>(float*, const float*, int, int, int, int, const int*, const int*, const int*, const int*,
                                 bool, hipStream_t);
 template int pair_reduce<double>(double*, const double*, int, int, int, int, const int*, const int*, const int*,

@@ -53,9 +53,9 @@ unsigned long long a2p_workspace_generation(void);
  * Synchronises `stream`.  Returns A2P_OK, A2P_ERR_INPUT, A2P_ERR_OVERFLOW, A2P_ERR_SEGMENT or A2P_ERR_GRID.  The reference has no such check: it asserts or overflows
  * (source/nblist/include/neighborList.h:550, commented-out assert). */
 int a2p_check_status(void* stream);
-/* The same for the loss entry points, whose first kernels make every check: a2p_status_early(1) before such a call
+/* The same for the energy / force / virial and the loss entry points, whose first kernels make every check: a2p_status_early(1) before such a call
  * sends the status word to the host behind those kernels, and a2p_check_status_early after it waits for that word
- * only, while the gradient kernels of the call may still run (a raised bit is then confirmed by a2p_check_status behind
+ * only, while the last kernels of the call may still run (a raised bit is then confirmed by a2p_check_status behind
  * the whole call).  After a2p_fvt_virial_fwd_* it is that call's own check (A2P_OK, or A2P_ERR_OVERFLOW for a row of more
  * than umax neighbours), and the status word stays as it was.  Per host thread, for one call; after a call of another kind
  * it is a2p_check_status. */
