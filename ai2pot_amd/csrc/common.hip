@@ -499,7 +499,7 @@ int finish_partials(T* out, const double* partial, int B, int nblocks, int ncomp
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
 }
-// Energy (component 0) and virial (components 1-9) of partial[.., 10] in one launch; either output
+// Energy (component 0) and virial (components 1-9) of ev_partial's array in one launch; either output
 // may be null.  Same summation per component as finish_partials.
 template <typename T>
 __global__ void finish_ev_kernel(T* etot, T* virial, const double* partial, int nblocks)

@@ -97,7 +97,7 @@ struct MtpArgs {
     int seg_spare;     // seg_cursor is null when no forces are wanted
     int seg_cap;       // capacity of a segment
     int seg_mark;      // own sums are marked in the cursors
-    double* partial;   // [B, P, 10]  energy + virial per atom
+    double* partial;   // energy and virial per atom (ev_partial, a block per row)
     int* status;
     int E;             // table entries per neighbour
     // loss gradient mode
@@ -530,7 +530,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
     T* pq = LOSS ? Bb + p.ncoef_poly : Ab;
 
     if (ii >= a.binum[b]) {                  // padded row: contributes nothing
-        if (!LOSS && a.partial && lane < 10) a.partial[row * 10 + lane] = 0.0;
+        if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
         if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
         if (!LOSS && a.desc)
             for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
@@ -763,7 +763,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
             }
             if (!SEED || a.partial) {
 #pragma unroll
-                for (int q = 0; q < 10; q++) a.partial[row * 10 + q] = out[q];
+                for (int q = 0; q < 10; q++) a.partial[ev_partial(a.P, b, ii, q)] = out[q];
             }
         }
         return;

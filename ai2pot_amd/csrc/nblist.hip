@@ -111,9 +111,9 @@ __device__ __forceinline__ int bin_of(T c, T mn, T bin_size)      // binLinkedLi
 }
 
 // ---- 1. coordinates and extents --------------------------------------------------------------
-// Cartesian coordinates of atom p, and the extremes of its images (v[0..2] minima, v[3..5] maxima).
+// Cartesian coordinates of atom p
 template <typename T>
-__device__ __forceinline__ void atom_extremes(const Grid<T>& g, const T* __restrict__ coords, int p, T (&c)[3], T (&v)[6])
+__device__ __forceinline__ void cart_coords(const Grid<T>& g, const T* __restrict__ coords, int p, T (&c)[3])
 {
     if (g.is_cart) {
 #pragma unroll
@@ -124,56 +124,55 @@ __device__ __forceinline__ void atom_extremes(const Grid<T>& g, const T* __restr
         for (int a = 0; a < 3; a++)
             c[a] = add_rn(add_rn(mul_rn(f0, g.b[0][a]), mul_rn(f1, g.b[1][a])), mul_rn(f2, g.b[2][a]));
     }
-    // Extremes over the atom's images (structure.h:1018-1052 takes them over the whole supercell).  Rounded
-    // multiplication and addition are monotone in each operand, so image_coord is monotone in each image
-    // index, rising or falling with the sign of the lattice component: the extremes sit at the ends of
-    // the index ranges, and two images per axis give the same values as the loop over all of them.
+}
+
+// Extremes along axis a over the images of atoms whose coordinates lie between c_lo and c_hi, both of them some atom's
+// (structure.h:1018-1052 takes them over the whole supercell).  Rounded multiplication and addition are monotone in each
+// operand, so image_coord rises with the atom's coordinate and is monotone in each image index, rising or falling with the
+// sign of the lattice component: the extremes sit at the ends of the index ranges and at the extreme atoms, and two images
+// give the same values as the loop over all of them.
+template <typename T>
+__device__ __forceinline__ void image_extremes(const Grid<T>& g, int a, T c_lo, T c_hi, T& v_lo, T& v_hi)
+{
+    int lo[3], hi[3];
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        int lo[3], hi[3];
-#pragma unroll
-        for (int w = 0; w < 3; w++) {
-            const int first = g.img_lo[w], last = g.img_lo[w] + g.img_dim[w] - 1;
-            const bool rising = g.b[w][a] >= (T)0;
-            lo[w] = rising ? first : last;
-            hi[w] = rising ? last : first;
-        }
-        v[a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], lo[0], lo[1], lo[2]);
-        v[3 + a] = image_coord(c[a], g.b[0][a], g.b[1][a], g.b[2][a], hi[0], hi[1], hi[2]);
+    for (int w = 0; w < 3; w++) {
+        const int first = g.img_lo[w], last = g.img_lo[w] + g.img_dim[w] - 1;
+        const bool rising = g.b[w][a] >= (T)0;
+        lo[w] = rising ? first : last;
+        hi[w] = rising ? last : first;
     }
+    v_lo = image_coord(c_lo, g.b[0][a], g.b[1][a], g.b[2][a], lo[0], lo[1], lo[2]);
+    v_hi = image_coord(c_hi, g.b[0][a], g.b[1][a], g.b[2][a], hi[0], hi[1], hi[2]);
 }
 
 // Four workgroups per CU: beyond that a thread takes several atoms before the sums across lanes, which are what the
 // kernel waits for, and the kernel behind it has fewer values to compare
-// (1,048,576 atoms, fp32: 19.1 -> 10.9 and 13.5 -> 4.6 us with 1024 instead of 4096 workgroups).
+// (1,048,576 atoms, fp32: 19.1 -> 10.9 and 13.5 -> 4.6 us with 1024 instead of 4096 workgroups; 7.3 and 4.5 since the images'
+// extremes are taken from the atoms' and Cartesian coordinates are not copied).
 constexpr int MINMAX_BLOCKS = 1024;
 
 template <typename T>
 __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coords, T* __restrict__ x,
                                      T* __restrict__ partial)
 {
-    __shared__ T sh[NBL_BLOCK / 64][12];
-    T v[12];
+    __shared__ T sh[NBL_BLOCK / 64][6];
+    T v[6];                                             // minima and maxima of the atoms (a NaN is passed by)
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        v[a] = (T)INT_MAX; v[3 + a] = (T)INT_MIN;       // structure.h:1018-1022
-        v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
-    }
+    for (int a = 0; a < 3; a++) { v[a] = (T)INFINITY; v[3 + a] = (T)-INFINITY; }
     for (int p = blockIdx.x * NBL_BLOCK + threadIdx.x; p < g.N; p += gridDim.x * NBL_BLOCK) {
-        T c[3], w[6];
-        atom_extremes<T>(g, coords, p, c, w);
+        T c[3];
+        cart_coords<T>(g, coords, p, c);
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            x[(size_t)p * 3 + a] = c[a];
-            v[a] = w[a] < v[a] ? w[a] : v[a];
-            v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
-            v[6 + a] = c[a] < v[6 + a] ? c[a] : v[6 + a];
-            v[9 + a] = c[a] > v[9 + a] ? c[a] : v[9 + a];
+            if (x) x[(size_t)p * 3 + a] = c[a];
+            v[a] = c[a] < v[a] ? c[a] : v[a];
+            v[3 + a] = c[a] > v[3 + a] ? c[a] : v[3 + a];
         }
     }
 #pragma unroll
-    for (int q = 0; q < 12; q++) {
-        const bool is_min = (q % 6) < 3;
+    for (int q = 0; q < 6; q++) {
+        const bool is_min = q < 3;
         T r = v[q];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) {
@@ -183,30 +182,44 @@ __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coor
         if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = r;
     }
     __syncthreads();
-    if (threadIdx.x < 12) {
+    if (threadIdx.x < 6) {
         const int q = threadIdx.x;
-        const bool is_min = (q % 6) < 3;
+        const bool is_min = q < 3;
         T r = sh[0][q];
         for (int w = 1; w < NBL_BLOCK / 64; w++) {
             T o = sh[w][q];
             r = is_min ? (o < r ? o : r) : (o > r ? o : r);
         }
-        partial[(size_t)blockIdx.x * 12 + q] = r;
+        partial[(size_t)blockIdx.x * 6 + q] = r;
     }
 }
 
-// 12 wavefronts, one per extent (minima of the image coordinates, their maxima, minima and maxima
-// of the centre atoms, three axes each)
+// The twelve extents of axis a from the atoms' (out[6 + a], out[9 + a]): over the images, and both from INT_MAX down and
+// from INT_MIN up (structure.h:1018-1022).
 template <typename T>
-__global__ void minmax_finish_kernel(const T* __restrict__ partial, int nblocks, T* __restrict__ out)
+__device__ __forceinline__ void extents_of_axis(const Grid<T>& g, int a, T* out)
 {
+    T lo = out[6 + a], hi = out[9 + a], first, last;
+    image_extremes<T>(g, a, lo, hi, first, last);
+    out[a] = first < (T)INT_MAX ? first : (T)INT_MAX;
+    out[3 + a] = last > (T)INT_MIN ? last : (T)INT_MIN;
+    out[6 + a] = lo < (T)INT_MAX ? lo : (T)INT_MAX;
+    out[9 + a] = hi > (T)INT_MIN ? hi : (T)INT_MIN;
+}
+
+// 6 wavefronts, one per extreme of the atoms, then the extents (minima of the image coordinates, their maxima, minima and
+// maxima of the centre atoms, three axes each)
+template <typename T>
+__global__ void minmax_finish_kernel(const Grid<T> g, const T* __restrict__ partial, int nblocks, T* __restrict__ out)
+{
+    __shared__ T ext[12];
     const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool is_min = (q % 6) < 3;
-    T r = is_min ? (T)INT_MAX : (T)INT_MIN;
+    const bool is_min = q < 3;
+    T r = is_min ? (T)INFINITY : (T)-INFINITY;
     for (int k0 = lane; k0 < nblocks; k0 += 64 * 8) {
         T o[8];                                    // eight loads in flight
 #pragma unroll
-        for (int u = 0; u < 8; u++) o[u] = partial[(size_t)min(k0 + 64 * u, nblocks - 1) * 12 + q];
+        for (int u = 0; u < 8; u++) o[u] = partial[(size_t)min(k0 + 64 * u, nblocks - 1) * 6 + q];
 #pragma unroll
         for (int u = 0; u < 8; u++) r = is_min ? (o[u] < r ? o[u] : r) : (o[u] > r ? o[u] : r);
     }
@@ -215,7 +228,11 @@ __global__ void minmax_finish_kernel(const T* __restrict__ partial, int nblocks,
         const T o = __shfl_xor(r, off, 64);
         r = is_min ? (o < r ? o : r) : (o > r ? o : r);
     }
-    if (lane == 0) out[q] = r;
+    if (lane == 0) ext[6 + q] = r;
+    __syncthreads();
+    if (threadIdx.x < 3) extents_of_axis<T>(g, (int)threadIdx.x, ext);
+    __syncthreads();
+    if (threadIdx.x < 12) out[threadIdx.x] = ext[threadIdx.x];
 }
 
 // ---- 1b. bin grid from the extents, on the device (builds that do not read the extents back) ----------
@@ -438,19 +455,26 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
     }
 }
 
-// ---- 1-5 in one workgroup: structures of up to NBS_ATOMS atoms --------------------------------------------
+// ---- 1-5 in one launch: structures of up to NBS_ATOMS atoms ------------------------------------------------
 // Such a build is bound by the latency of nine short launches and of the wait for the extents (51 us of GPU time for
-// 4096 atoms, of which 38 in kernels; 31 us here, 36 when another kernel has just written the coordinates, and 12 us for
-// 108 atoms).  One workgroup of 1024 threads does the same with its counters in LDS: extents, grid, counts, prefix sum, image numbers dealt to their bins, and every record written once, to its final
-// place (an image's place in its bin is the number of larger image numbers there).  The images of an atom are found per
-// axis when the lattice is diagonal and an axis has at most three images, else one by one.  Images beyond the LDS (atoms
-// crowded into a corner of the cell are within reach of eight cells each) pass through global memory instead.  What the
-// grid turned out to be goes to the host while the rest runs; a box beyond the LDS empties the lists and is reported, and
-// the host then takes the general route.
+// 4096 atoms, of which 38 in kernels).  Here every workgroup finds the extents and the grid for itself (the atoms are
+// few) and bins one slab of the box, a plane of bins across x or a few, with its counters in LDS: the images in its slab
+// are listed and dealt to their bins, those in the slabs before it are only counted, which says where its records begin,
+// and every record is written once, to its final place (an image's place in its bin is the number of larger image numbers
+// there).  No workgroup waits for another.  4096 atoms take 14.5 us (one workgroup for the whole box: 31), of which extents
+// and grid 5, finding the images 4, dealing them 3.
+// Told axis by axis (diagonal lattice, at most three images an axis), an image is placed by comparisons with the edges of
+// the box and of the slab; the exactly rounded division decides next to an edge only, and for the bins of the slab's own.
+// Other lattices are tried image by image.  Images of a slab beyond its LDS (atoms crowded into a corner of the cell are
+// within reach of eight cells each) pass through global memory instead.  What the grid turned out to be goes to the host
+// while the rest runs; a box beyond the LDS empties the lists and is reported, and the host then takes the general route.
 // (bins: a cube of 21, grown by the two that a build without a read-back allows for)
 constexpr int NBS_THREADS = 1024, NBS_ATOMS = 4096, NBS_BINS = 12288, NBS_IMAGES = 15360;
-constexpr int NBS_AXIS = 256;                     // bins per axis: a bin is a byte
-constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_IMAGES * 6;
+constexpr int NBS_AXIS = 256;                     // bins per axis
+constexpr int NBS_SLABS = 32;                     // workgroups: a plane of bins each for boxes of up to 32
+constexpr int NBS_CAP = 8192;                     // images of a slab in LDS
+constexpr int NBS_WORK = 3 * NBS_ATOMS;           // (atom, image along x) in a slab
+constexpr size_t NBS_LDS = (size_t)NBS_BINS * 4 + (size_t)NBS_CAP * 10 + (size_t)NBS_WORK * 2;
 
 constexpr int NBS_ATOM_BITS = 12, NBS_TRIPLES = 256;
 static_assert(NBS_ATOMS <= 1 << NBS_ATOM_BITS, "an atom's number fits below the image's");
@@ -471,53 +495,59 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
                   int* __restrict__ offsets, T* __restrict__ s_rec, const int* __restrict__ types, int* __restrict__ ilist,
                   int* __restrict__ types_out, int* __restrict__ incoming, int mark_types, int separable, int cap0, int cap1,
                   int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq,
-                  unsigned* __restrict__ axis_images, int* __restrict__ spare, int spare_images)
+                  int* __restrict__ spare, int spare_images)
 {
     extern __shared__ __align__(16) unsigned char sh_small[];
     int* const cnt = (int*)sh_small;                             // per bin: count, then end of the bin's records
-    int* const num = cnt + NBS_BINS;                             // image numbers, by bin
-    unsigned short* const bin_of_num = (unsigned short*)(num + NBS_IMAGES);
-    static_assert(NBS_LDS >= 12 * NBS_THREADS * sizeof(double), "the extremes pass through the counters' LDS");
+    int* const found = cnt + NBS_BINS;                           // image numbers, as they were found
+    int* const num = found + NBS_CAP;                            // ... and by bin
+    unsigned short* const bin_of_found = (unsigned short*)(num + NBS_CAP);
+    unsigned short* const work = bin_of_found + NBS_CAP;         // atom | image along x << 12
+    static_assert(NBS_LDS >= 6 * NBS_THREADS * sizeof(double), "the extremes pass through the counters' LDS");
     __shared__ T ext[12];
     __shared__ GridDyn<T> dyn;
-    __shared__ int sh_ok[3], sh_scan[NBS_THREADS / 64], sh_bad;
+    __shared__ int sh_ok[3], sh_scan[3][NBS_THREADS / 64], sh_bad, sh_found, sh_work;
     __shared__ unsigned sh_triple[NBS_TRIPLES];                  // image number -> (i, j, k), 10 bits each
     const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int N = g_in.N;
-    if (tid == 0) sh_bad = 0;
+    if (tid == 0) { sh_bad = 0; sh_found = 0; sh_work = 0; }
     __syncthreads();
 
-    // 1. coordinates, extents
-    T v[12];
+    // 1. coordinates, extents (image_extremes: those of the atoms are enough)
+    constexpr int PER = NBS_ATOMS / NBS_THREADS;
+    const int chunk = (N + (int)gridDim.x - 1) / (int)gridDim.x;          // the atoms whose outputs this workgroup writes
+    const int own0 = chunk * (int)blockIdx.x, own1 = min(own0 + chunk, N);
+    T lo[3], hi[3];
+    bool bad = false;
 #pragma unroll
-    for (int a = 0; a < 3; a++) {
-        v[a] = (T)INT_MAX; v[3 + a] = (T)INT_MIN;       // structure.h:1018-1022
-        v[6 + a] = (T)INT_MAX; v[9 + a] = (T)INT_MIN;
-    }
-#pragma unroll 1
-    for (int p = tid; p < N; p += NBS_THREADS) {
-        T c[3], w[6];
-        atom_extremes<T>(g_in, coords, p, c, w);
-        if (ilist) { ilist[p] = p; types_out[p] = types[p]; }      // neighborList.h:548-553
-        if (incoming) incoming[p] = 0;                             // counted up by the list kernel
+    for (int a = 0; a < 3; a++) { lo[a] = (T)INFINITY; hi[a] = (T)-INFINITY; }
+#pragma unroll
+    for (int r = 0; r < PER; r++) {
+        const int p = tid + r * NBS_THREADS;
+        if (p >= N) break;
+        T c[3];
+        cart_coords<T>(g_in, coords, p, c);
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            x[(size_t)p * 3 + a] = c[a];
-            if (!(fabs((double)c[a]) < 1.0e30)) sh_bad = 1;        // the comparisons below pass a NaN by
-            v[a] = w[a] < v[a] ? w[a] : v[a];
-            v[3 + a] = w[3 + a] > v[3 + a] ? w[3 + a] : v[3 + a];
-            v[6 + a] = c[a] < v[6 + a] ? c[a] : v[6 + a];
-            v[9 + a] = c[a] > v[9 + a] ? c[a] : v[9 + a];
+            bad = bad || !(fabs((double)c[a]) < 1.0e30);           // the comparisons below pass a NaN by
+            lo[a] = c[a] < lo[a] ? c[a] : lo[a];
+            hi[a] = c[a] > hi[a] ? c[a] : hi[a];
+        }
+        if (p >= own0 && p < own1) {
+            if (x) { x[(size_t)p * 3] = c[0]; x[(size_t)p * 3 + 1] = c[1]; x[(size_t)p * 3 + 2] = c[2]; }
+            if (ilist) { ilist[p] = p; types_out[p] = types[p]; }  // neighborList.h:548-553
+            if (incoming) incoming[p] = 0;                         // counted up by the list kernel
         }
     }
-    // each extreme is taken over the threads' values by one wavefront: twelve reductions by shuffles in every
-    // wavefront would be a chain of 72
-    T* const sh_v = (T*)sh_small;                                // [12][NBS_THREADS], before the counters
+    if (bad) sh_bad = 1;
+    // each extreme is taken over the threads' values by one wavefront: six reductions by shuffles in every
+    // wavefront would be a chain of 36
+    T* const sh_v = (T*)sh_small;                                // [6][NBS_THREADS], before the counters
 #pragma unroll
-    for (int q = 0; q < 12; q++) sh_v[q * NBS_THREADS + tid] = v[q];
+    for (int a = 0; a < 3; a++) { sh_v[a * NBS_THREADS + tid] = lo[a]; sh_v[(3 + a) * NBS_THREADS + tid] = hi[a]; }
     __syncthreads();
-    if (wv < 12) {
-        const bool is_min = (wv % 6) < 3;
+    if (wv < 6) {
+        const bool is_min = wv < 3;
         T o[NBS_THREADS / 64];
 #pragma unroll
         for (int w = 0; w < NBS_THREADS / 64; w++) o[w] = sh_v[wv * NBS_THREADS + w * 64 + lane];
@@ -529,139 +559,179 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
             const T t = __shfl_xor(r, off, 64);
             r = is_min ? (t < r ? t : r) : (t > r ? t : r);
         }
-        if (lane == 0) ext[wv] = r;
+        if (lane == 0) ext[6 + wv] = r;
     }
     __syncthreads();
-    if (tid < 3) sh_ok[tid] = grid_axis<T>(g_in, ext, &dyn, tid, tid == 0 ? cap0 : tid == 1 ? cap1 : cap2, big_bound) ? 1 : 0;
+    if (tid < 3) {
+        extents_of_axis<T>(g_in, tid, ext);
+        sh_ok[tid] = grid_axis<T>(g_in, ext, &dyn, tid, tid == 0 ? cap0 : tid == 1 ? cap1 : cap2, big_bound) ? 1 : 0;
+    }
     __syncthreads();
     const long long nregion_ll = (long long)max(dyn.rdim[0], 0) * max(dyn.rdim[1], 0) * max(dyn.rdim[2], 0);
-    bool ok = !sh_bad && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform
-    const int nregion = ok ? (int)nregion_ll : 0;
+    bool ok = !sh_bad && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform, alike in all workgroups
     const Grid<T> g = with_dyn<T>(g_in, &dyn);
+    const int nx = ok ? g.rdim[0] : 0, plane = ok ? g.rdim[1] * g.rdim[2] : 0;
+    const int planes = (nx + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int x0 = min(planes * (int)blockIdx.x, nx), x1 = min(x0 + planes, nx);
+    if (blockIdx.x > 0 && x0 >= x1) return;                      // no slab; the first workgroup reports
+    const int nbins = (x1 - x0) * plane;
 
-    for (int i = tid; i < nregion; i += NBS_THREADS) cnt[i] = 0;
+    for (int i = tid; i < nbins; i += NBS_THREADS) cnt[i] = 0;
     if (tid < min(g.nimg, NBS_TRIPLES)) sh_triple[tid] = image_triple(g, tid);
     __syncthreads();
 
-    // 2. counts, 3. prefix sum, 4. image numbers to their bins.  One copy of the code that enumerates the images serves
-    // both passes: it runs once or a few times per call, so fetching instructions is a good part of what it costs.
-    int total = 0;
-    bool in_lds = true;                                          // uniform
-#pragma unroll 1
-    for (int pass = 0; pass < 2 && ok && in_lds; pass++) {
-        auto image = [&](int im, int p, int b) __attribute__((always_inline)) {
-            const int pos = atomicAdd(&cnt[b], 1);
-            if (pass) {
-                num[pos] = im << NBS_ATOM_BITS | p;              // ordered as the supercell index im * N + p
-                bin_of_num[pos] = (unsigned short)b;
-            }
-        };
-        // the bin along axis a of the image that is i cells along it, or -1 outside the box (separable: the other axes'
-        // indices only add zeros, their lattice components along this axis vanish)
-        auto along = [&](T ca, int a, int i) __attribute__((always_inline)) -> int {
-            const T ci = add_rn(ca, mul_rn(g.b[a][a], (T)(g.img_lo[a] + i)));
-            if (ci < g.keep_lo[a] || ci > g.keep_hi[a]) return -1;
-            const int b = bin_of(ci, g.mn[a], g.bin_size) - g.rlo[a];
-            return b < g.rdim[a] ? b : -1;
-        };
-        if (separable && N * g.img_dim[0] * g.img_dim[1] <= 2 * NBS_THREADS) {
-            // few atoms: a thread takes the images in one column of cells of an atom
-#pragma unroll 1
-            for (int w = tid; w < N * g.img_dim[0] * g.img_dim[1]; w += NBS_THREADS) {
-                const int ij = w / N, p = w - ij * N, i = ij / g.img_dim[1], j = ij - i * g.img_dim[1];
-                const T cx = x[(size_t)p * 3], cy = x[(size_t)p * 3 + 1], cz = x[(size_t)p * 3 + 2];
-                const int bx = along(cx, 0, i), by = along(cy, 1, j);
-                if (bx < 0 || by < 0) continue;
-#pragma unroll 1
-                for (int k = 0; k < g.img_dim[2]; k++) {
-                    const int bz = along(cz, 2, k);
-                    if (bz >= 0) image(ij * g.img_dim[2] + k, p, (bx * g.rdim[1] + by) * g.rdim[2] + bz);
-                }
-            }
-        } else if (separable) {
-#pragma unroll 1
-            for (int p = tid; p < N; p += NBS_THREADS) {
-                // an axis' images inside the box, 10 bits each (image index, bin), and how many above bit 30
-                unsigned pk[3];
-                if (pass == 0) {
+    // 2. images: found (in the slab), before it, in the box
+    int before = 0, all = 0;
+    auto image = [&](int im, int p, int b) __attribute__((always_inline)) {      // bin b of the slab
+        atomicAdd(&cnt[b], 1);
+        const int k = atomicAdd(&sh_found, 1);
+        if (k < NBS_CAP) {
+            found[k] = im << NBS_ATOM_BITS | p;                  // ordered as the supercell index im * N + p
+            bin_of_found[k] = (unsigned short)b;
+        }
+    };
+    if (ok && separable) {
+        // An image at distance v from the middle of the kept interval is outside the box for sure when |v| > reach, inside
+        // when |v| < inner, and likewise before the slab when v < from, behind it when v > to.  The margins are that of
+        // keep_lo, a hundred times the rounding of the binning, and of this arithmetic.
+        T shift[3][3], reach[3], inner[3], from, to;
 #pragma unroll
-                    for (int a = 0; a < 3; a++) {
-                        const T ca = x[(size_t)p * 3 + a];
-                        unsigned w = 0, n = 0;
-#pragma unroll 1
-                        for (int i = 0; i < g.img_dim[a]; i++) {
-                            const int b = along(ca, a, i);
-                            if (b >= 0) { w |= ((unsigned)i << 8 | (unsigned)b) << (10 * n); n++; }
-                        }
-                        pk[a] = w | n << 30;
-                        axis_images[p * 3 + a] = pk[a];
-                    }
-                } else {
+        for (int a = 0; a < 3; a++) {
+            const double lo_edge = (double)g.mn[a] + (double)g.rlo[a] * (double)g.bin_size;
+            const double margin = lo_edge - (double)g.keep_lo[a];
+            const double mid = 0.5 * ((double)g.keep_lo[a] + (double)g.keep_hi[a]);
+            reach[a] = (T)((double)g.keep_hi[a] - mid);
+            inner[a] = (T)((double)g.keep_hi[a] - mid - 2.0 * margin);
+            if (a == 0) {
+                from = (T)(lo_edge + (double)x0 * (double)g.bin_size - margin - mid);
+                to = (T)(lo_edge + (double)x1 * (double)g.bin_size + margin - mid);
+            }
 #pragma unroll
-                    for (int a = 0; a < 3; a++) pk[a] = axis_images[p * 3 + a];
-                }
-                // a thread walks its own images only: a wavefront takes as many trips as its atom with the most (eight
-                // next to a corner of the cell)
-                const unsigned n1 = pk[1] >> 30, n2 = pk[2] >> 30, n = (pk[0] >> 30) * n1 * n2;
-                unsigned w0 = pk[0], w1 = pk[1], w2 = pk[2], j = 0, k = 0;
+            for (int i = 0; i < 3; i++)
+                shift[a][i] = i < g.img_dim[a] ? (T)((double)g.b[a][a] * (double)(g.img_lo[a] + i) - mid) : (T)4.0e30;
+        }
+        // the coordinate along axis a of the image that is i cells along it (the other axes' indices only add zeros, their
+        // lattice components along this axis vanish), its bin, and whether it is inside, exactly
+        auto at = [&](T ca, int a, int i) __attribute__((always_inline)) -> T {
+            return add_rn(ca, mul_rn(g.b[a][a], (T)(g.img_lo[a] + i)));
+        };
+        auto bin = [&](T ci, int a) __attribute__((always_inline)) -> int { return bin_of(ci, g.mn[a], g.bin_size) - g.rlo[a]; };
+        auto inside = [&](T ci, int a) __attribute__((always_inline)) -> bool {
+            if (ci < g.keep_lo[a] || ci > g.keep_hi[a]) return false;
+            const int b = bin(ci, a);
+            return b >= 0 && b < g.rdim[a];
+        };
+        T ahead_c[3];
+        if (tid < N) cart_coords<T>(g, coords, tid, ahead_c);
 #pragma unroll 1
-                for (unsigned q = 0; q < n; q++) {
-                    const int bin = (int)(((w0 & 0xffu) * g.rdim[1] + (w1 & 0xffu)) * g.rdim[2] + (w2 & 0xffu));
-                    const int im = (int)((((w0 >> 8) & 3u) * g.img_dim[1] + ((w1 >> 8) & 3u)) * g.img_dim[2] + ((w2 >> 8) & 3u));
-                    image(im, p, bin);
-                    w2 >>= 10;
-                    if (++k == n2) {
-                        k = 0; w2 = pk[2];
-                        w1 >>= 10;
-                        if (++j == n1) { j = 0; w1 = pk[1]; w0 >>= 10; }
+        for (int p = tid, next = tid; p < N; p = next) {
+            T c[3];
+#pragma unroll
+            for (int a = 0; a < 3; a++) c[a] = ahead_c[a];
+            next += NBS_THREADS;
+            if (next < N) cart_coords<T>(g, coords, next, ahead_c);        // on its way while this one is placed
+            int n[3], sure[3], ahead = 0, upto = 0;
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                n[a] = sure[a] = 0;
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    const T v = c[a] + shift[a][i], d = v < (T)0 ? -v : v;
+                    n[a] += d <= reach[a] ? 1 : 0;
+                    sure[a] += d < inner[a] ? 1 : 0;
+                    if (a == 0) {
+                        ahead += d < inner[a] && v < from ? 1 : 0;
+                        upto += d <= reach[a] && v <= to ? 1 : 0;
                     }
                 }
-            }
-        } else {
+                if (a > 0 && n[a] != sure[a]) {
+                    n[a] = 0;
 #pragma unroll 1
-            for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
-                const int m = w / N, p = w - m * N;
-                const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
-                const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
-                T ci[3];
-                const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
-                if (b >= 0) image(m, p, b);
+                    for (int i = 0; i < g.img_dim[a]; i++) n[a] += inside(at(c[a], a, i), a) ? 1 : 0;
+                }
+            }
+            const int n12 = n[1] * n[2];
+            if ((n[0] != sure[0] || upto != ahead) && n12 > 0) {           // next to an edge of the box, or in the slab
+                n[0] = ahead = 0;
+#pragma unroll 1
+                for (int i = 0; i < g.img_dim[0]; i++) {
+                    const T ci = at(c[0], 0, i);
+                    if (!inside(ci, 0)) continue;
+                    n[0]++;
+                    const int b = bin(ci, 0);
+                    if (b < x0) ahead++;
+                    else if (b < x1) work[atomicAdd(&sh_work, 1)] = (unsigned short)(p | i << NBS_ATOM_BITS);
+                }
+            }
+            all += n[0] * n12;
+            before += ahead * n12;
+        }
+        __syncthreads();
+        // the slab's own, all lanes busy
+        const int nwork = sh_work;
+#pragma unroll 1
+        for (int w = tid; w < nwork * g.img_dim[1]; w += NBS_THREADS) {
+            const int j = w / nwork, pi = work[w - j * nwork], p = pi & ((1 << NBS_ATOM_BITS) - 1), i = pi >> NBS_ATOM_BITS;
+            T c[3];
+            cart_coords<T>(g, coords, p, c);
+            const T cy = at(c[1], 1, j);
+            if (!inside(cy, 1)) continue;
+            const int bxy = (bin(at(c[0], 0, i), 0) - x0) * g.rdim[1] + bin(cy, 1);
+#pragma unroll 1
+            for (int k = 0; k < g.img_dim[2]; k++) {
+                const T cz = at(c[2], 2, k);
+                if (inside(cz, 2)) image((i * g.img_dim[1] + j) * g.img_dim[2] + k, p, bxy * g.rdim[2] + bin(cz, 2));
             }
         }
-        __syncthreads();
-        if (pass) break;                                         // cnt[b] is now where bin b ends, and bin b + 1 begins
-
-        // prefix sum in place: a thread takes consecutive bins
-        const int per = (nregion + NBS_THREADS - 1) / NBS_THREADS;
-        const int b0 = min(tid * per, nregion), b1 = min(b0 + per, nregion);
-        int mine = 0;
-        for (int b = b0; b < b1; b++) mine += cnt[b];
-        const int incl = wave_inclusive_scan(mine);
-        if (lane == 63) sh_scan[wv] = incl;
-        __syncthreads();
-        int run = incl - mine;
-        for (int w = 0; w < NBS_THREADS / 64; w++) {
-            const int t = sh_scan[w];
-            run += w < wv ? t : 0;
-            total += t;
+    } else if (ok) {
+#pragma unroll 1
+        for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
+            const int m = w / N, p = w - m * N;
+            const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
+            T xp[3], ci[3];
+            cart_coords<T>(g, coords, p, xp);
+            const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
+            if (b < 0) continue;
+            all++;
+            if (b < x0 * plane) before++;
+            else if (b < x1 * plane) image(m, p, b - x0 * plane);
         }
-        in_lds = total <= NBS_IMAGES;
-        ok = in_lds || total <= spare_images;                    // uniform
-        for (int b = b0; b < b1; b++) {
-            const int n = cnt[b];
-            cnt[b] = run;
-            if (ok) offsets[b] = run;
-            run += n;
-        }
-        __syncthreads();
     }
-    if (tid == 0) {
+    before = wave_sum(before);
+    all = wave_sum(all);
+    if (lane == 0) { sh_scan[1][wv] = before; sh_scan[2][wv] = all; }
+    __syncthreads();
+
+    // 3. prefix sum in place: a thread takes consecutive bins
+    const int per = (nbins + NBS_THREADS - 1) / NBS_THREADS;
+    const int b0 = min(tid * per, nbins), b1 = min(b0 + per, nbins);
+    int mine = 0;
+    for (int b = b0; b < b1; b++) mine += cnt[b];
+    const int incl = wave_inclusive_scan(mine);
+    if (lane == 63) sh_scan[0][wv] = incl;
+    __syncthreads();
+    int run = incl - mine, own = 0, base = 0, total = 0;
+    for (int w = 0; w < NBS_THREADS / 64; w++) {
+        const int t = sh_scan[0][w];
+        run += w < wv ? t : 0;
+        own += t;
+        base += sh_scan[1][w];
+        total += sh_scan[2][w];
+    }
+    ok = ok && total <= spare_images;                            // (the room for records)
+    for (int b = b0; b < b1; b++) {
+        const int n = cnt[b];
+        cnt[b] = run;
+        if (ok) offsets[x0 * plane + b] = base + run;
+        run += n;
+    }
+    if (tid == 0 && blockIdx.x == 0) {
         if (!ok) {
             for (int a = 0; a < 3; a++) { dyn.rdim[a] = 0; dyn.keep_lo[a] = (T)1; dyn.keep_hi[a] = (T)-1; }
             if (raise) atomicOr(status, ST_GRID_BOUND);
         }
-        dyn.nregion = ok ? nregion : 0;
-        if (ok) offsets[nregion] = total;
+        dyn.nregion = ok ? nx * plane : 0;
+        if (ok) offsets[nx * plane] = total;
         double big = 0;
         for (int a = 0; a < 3; a++) big = fmax(big, fmax(fabs((double)dyn.keep_lo[a]), fabs((double)dyn.keep_hi[a])));
         *gd = dyn;
@@ -673,21 +743,22 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         }
     }
     if (!ok) return;
+    __syncthreads();
 
-    // 5. records in descending image number within a bin (head insertion, binLinkedList.h:833), as binsort_kernel leaves
-    // them.  Shifts and a table stand in for the five integer divisions a record would take.
+    // 4. image numbers to their bins, 5. records in descending image number within a bin (head insertion,
+    // binLinkedList.h:833), as binsort_kernel leaves them.  A table stands in for the integer divisions a record would take.
     const int central = ((-g.img_lo[0]) * g.img_dim[1] + (-g.img_lo[1])) * g.img_dim[2] + (-g.img_lo[2]);
-    auto records = [&](const auto* numbers, const auto* bins) __attribute__((always_inline)) {
+    auto records = [&](const auto* numbers, const auto* bins, const auto* by_bin) __attribute__((always_inline)) {
 #pragma unroll 1
-        for (int e = tid; e < total; e += NBS_THREADS) {
+        for (int e = tid; e < own; e += NBS_THREADS) {
             const int b = bins[e], m = numbers[e];
             const int im = m >> NBS_ATOM_BITS, p = m & ((1 << NBS_ATOM_BITS) - 1);
             const unsigned t = im < NBS_TRIPLES ? sh_triple[im] : image_triple(g, im);
-            const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+            T xp[3], ci[3];
+            cart_coords<T>(g, coords, p, xp);
             const int beg = b > 0 ? cnt[b - 1] : 0, end = cnt[b];
-            int place = beg;
-            for (int q = beg; q < end; q++) place += numbers[q] > m ? 1 : 0;
-            T ci[3];
+            int place = base + beg;
+            for (int q = beg; q < end; q++) place += by_bin[q] > m ? 1 : 0;
 #pragma unroll
             for (int a = 0; a < 3; a++)
                 ci[a] = image_coord(xp[a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + (int)(t & 1023u),
@@ -696,26 +767,29 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
                            mark_types ? p | ((types[p] & 15) << CL_TYPE_SHIFT) | (im != central ? CL_IMAGE_BIT : 0) : p);
         }
     };
-    if (__builtin_expect(in_lds, 1)) {
-        records(num, bin_of_num);
+    if (__builtin_expect(own <= NBS_CAP, 1)) {
+        for (int e = tid; e < own; e += NBS_THREADS) num[atomicAdd(&cnt[bin_of_found[e]], 1)] = found[e];
+        __syncthreads();                                         // cnt[b] is now where bin b ends, and bin b + 1 begins
+        records(found, bin_of_found, num);
         return;
     }
-    // more images than LDS: their numbers go through global memory (code of its own, so that the common case fetches none
-    // of it: 77.9 -> 77.6 us a step at 4096 atoms)
+    // more images than LDS: their numbers go through global memory, to places of this slab's own
+    int* const by_bin = spare + base;
+    int* const bins = spare + spare_images + base;
 #pragma unroll 1
     for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
         const int m = w / N, p = w - m * N;
         const int k = m % g.img_dim[2], ij = m / g.img_dim[2];
-        const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
-        T ci[3];
-        const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
-        if (b < 0) continue;
+        T xp[3], ci[3];
+        cart_coords<T>(g, coords, p, xp);
+        const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci) - x0 * plane;
+        if (b < 0 || b >= nbins) continue;
         const int pos = atomicAdd(&cnt[b], 1);
-        spare[pos] = m << NBS_ATOM_BITS | p;
-        spare[spare_images + pos] = b;
+        by_bin[pos] = m << NBS_ATOM_BITS | p;
+        bins[pos] = b;
     }
     __syncthreads();
-    records(spare, spare + spare_images);
+    records(by_bin, bins, by_bin);
 }
 
 // ---- processing order of the compact lists: atoms along a Morton curve through the bins ----------
@@ -1632,7 +1706,7 @@ struct GridBound {
     double lattice[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, rcut = 0;
     int rdim[3] = {0, 0, 0};
     double big = 0;    // largest |coordinate| of the box kept by that build
-    bool large = false;    // the box did not fit one workgroup (small_bins_kernel)
+    bool large = false;    // the box did not fit small_bins_kernel
 };
 // a few structures per host thread (two calculators used in turn keep both of their bounds), oldest replaced first
 constexpr size_t kMaxBounds = 8;
@@ -1701,19 +1775,18 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     g.inv_side = 1.0f / (float)(2 * g.ext_bins + 1);
     g.inv_bin = 1.0f / (float)g.bin_size;
 
-    // workspace A: x[N*3] | partial[nblocks*12] | ext[12] | (compact lists: xs[N*3] | inv[N]) | axis_images[N*3]
+    // workspace A: x[N*3] | partial[nblocks*6] | ext[12] | (compact lists: xs[N*3] | inv[N])
     const int nblocks = ceil_div(N, NBL_BLOCK);
     void* wsA = nullptr;
-    const size_t axis_off = (((size_t)N * 3 * (co ? 2 : 1) + (size_t)nblocks * 12 + 16) * sizeof(T) + (co ? (size_t)N * sizeof(int) : 0) + 7) / 8 * 8;
-    size_t bytesA = axis_off + (N <= NBS_ATOMS ? (size_t)N * 3 * sizeof(unsigned) : 0);
+    const size_t bytesA = ((size_t)N * 3 * (co ? 2 : 1) + (size_t)nblocks * 6 + 16) * sizeof(T) + (co ? (size_t)N * sizeof(int) : 0);
     int rc = ws_get(WS_NBL_A, bytesA, &wsA);
     if (rc) return rc;
-    T* x = (T*)wsA;
-    T* partial = x + (size_t)N * 3;
-    T* ext_dev = partial + (size_t)nblocks * 12;
+    T* const x_out = is_cart ? nullptr : (T*)wsA;       // Cartesian coordinates are read where they are
+    const T* const x = is_cart ? coords : (const T*)wsA;
+    T* partial = (T*)wsA + (size_t)N * 3;
+    T* ext_dev = partial + (size_t)nblocks * 6;
     T* xs = ext_dev + 16;                               // coordinates in processing order (compact lists)
     int* inv = (int*)(xs + (size_t)N * 3);              // ... and the inverse of the order
-    unsigned* axis_images = (unsigned*)((char*)wsA + axis_off);     // small_bins_kernel
     void* flags = nullptr;
     rc = ws_get(WS_FLAGS, 64, &flags);
     if (rc) return rc;
@@ -1757,7 +1830,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         big_coord = bound->big + (double)(grow + 2) * (double)g.bin_size;   // the box cannot have moved further
     }
 
-    // One workgroup bins the whole structure (small_bins_kernel) when its images can be told axis by axis or are few, and
+    // One launch bins the whole structure (small_bins_kernel) when its images can be told axis by axis or are few, and
     // the box expected of atoms inside the cell, a bin to spare on each side, fits its LDS.
     bool diagonal = true;
     for (int i = 0; i < 3; i++)
@@ -1821,17 +1894,17 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     GridDyn<T>* gd = nullptr;
     int* offsets = nullptr;
     long long total = 0;
-    int spare_images = 0;                               // images the one-workgroup binning has room for in global memory
+    int spare_images = 0;                               // images the binning in one launch has room for
     if (small) {
         posted = !sync_free;
         void* wsG = nullptr;
         rc = ws_get(WS_GRID, 256, &wsG);
         // one by one there are at most NBS_IMAGES images; told by axis, every one of them may be in reach
-        spare_images = separable && (long long)N * g.nimg > NBS_IMAGES ? N * g.nimg : 0;
+        spare_images = std::max(NBS_IMAGES, N * g.nimg);
         if (rc == A2P_OK)
             rc = ws_get(WS_NBL_B, ((size_t)NBS_BINS + 1 + 2 * (size_t)spare_images) * sizeof(int), (void**)&offsets);
         gd = (GridDyn<T>*)wsG;
-        total = std::max(NBS_IMAGES, spare_images);
+        total = spare_images;
     }
 
     if (small && rc == A2P_OK) {
@@ -1846,10 +1919,10 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         if (rc == A2P_OK) {
             const double bound_of_coords = sync_free ? big_coord : 1.0e30;
             prof_begin("nbl_small_bins", stream);
-            hipLaunchKernelGGL(small_bins_kernel<T>, dim3(1), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x, gd, offsets,
+            hipLaunchKernelGGL(small_bins_kernel<T>, dim3(NBS_SLABS), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x_out, gd, offsets,
                                (T*)wsC0, types, want_rows ? ilist : (int*)nullptr, types_out, incoming, co ? 1 : 0,
                                separable ? 1 : 0, cap[0], cap[1], cap[2], bound_of_coords, sync_free ? 1 : 0, status,
-                               posted ? post_slot : nullptr, post.seq, axis_images, offsets + NBS_BINS + 1, spare_images);
+                               posted ? post_slot : nullptr, post.seq, offsets + NBS_BINS + 1, spare_images);
             prof_end(stream);
             if (hipGetLastError() != hipSuccess) rc = A2P_ERR_HIP;
         }
@@ -1871,11 +1944,11 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     if (!small) {
     prof_begin("nbl_coords_minmax", stream);
     const int mm_blocks = std::min(nblocks, MINMAX_BLOCKS);
-    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(mm_blocks), dim3(NBL_BLOCK), 0, stream, g, coords, x,
+    hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(mm_blocks), dim3(NBL_BLOCK), 0, stream, g, coords, x_out,
                        partial);
     prof_end(stream);
     prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(12 * 64), 0, stream, partial, mm_blocks, ext_dev);
+    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(6 * 64), 0, stream, g, (const T*)partial, mm_blocks, ext_dev);
     prof_end(stream);
     if (sync_free) {
         for (int a = 0; a < 3; a++) {

@@ -411,7 +411,7 @@ nep_efv_kernel(const NepArgs<T> a)
     if (tid < 10) {
         double v = 0.0;
         for (int w = 0; w < NEP_BLOCK / 64; w++) v += s_red[w * 10 + tid];
-        a.partial[((size_t)b * a.nblocks + blockIdx.x) * 10 + tid] = v;
+        a.partial[ev_partial(a.nblocks, b, blockIdx.x, tid)] = v;
     }
 }
 

@@ -57,7 +57,7 @@ struct GatherArgs {
     int* incoming;        // [natoms] places claimed so far
     double overflow_limit; // largest magnitude a spare row accepts per value (sums of umax values must fit)
     T* force;             // [natoms][3] or null
-    double* partial;      // [nblocks][10]: energy and virial, each workgroup's share
+    double* partial;      // energy and virial, each workgroup's share (ev_partial)
     int* status;
     int want_virial;
 };
@@ -791,7 +791,7 @@ nep_adjoint_kernel(const GatherArgs<T> a)
         if (tid < nv) {
             double v = 0.0;
             for (int w = 0; w < CB / 64; w++) v += L.red[w * 10 + tid];
-            a.partial[(size_t)blk * 10 + tid] = v;
+            a.partial[ev_partial(gridDim.x, 0, blk, tid)] = v;
         }
     }
 }
@@ -899,9 +899,10 @@ nep_gather_kernel(const GatherArgs<T> a)
         }
         __syncthreads();
         if (tid < 9) {
-            double v = a.partial[(size_t)blk * 10 + 1 + tid];      // the adjoint kernel's share
+            double& share = a.partial[ev_partial(gridDim.x, 0, blk, 1 + tid)];
+            double v = share;                                      // the adjoint kernel's share
             for (int w = 0; w < CB / 64; w++) v += L.red[w * 9 + tid];
-            a.partial[(size_t)blk * 10 + 1 + tid] = v;
+            share = v;
         }
     }
 }

@@ -36,7 +36,7 @@ struct NepArgs {
     T* force;        // [B, P+nghost, 3] or null
     T* pair_g;       // [B*P, U, 3] or null (needed when force != null)
     T* desc;         // [B, P, D] or null
-    double* partial; // [B, nblocks, 10]
+    double* partial; // energy and virial per workgroup (ev_partial)
     int* status;
     int want_virial;
     int w_in_lds;    // network weights staged in LDS (else read from global memory)

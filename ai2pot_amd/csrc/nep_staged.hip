@@ -673,7 +673,7 @@ nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, int* __r
     if (tid < 10) {
         double v = 0.0;
         for (int w = 0; w < FB / 64; w++) v += s_red[w * 10 + tid];
-        a.partial[((size_t)b * a.nblocks + blockIdx.x) * 10 + tid] = v;
+        a.partial[ev_partial(a.nblocks, b, blockIdx.x, tid)] = v;
     }
 }
 

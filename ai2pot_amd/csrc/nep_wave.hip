@@ -428,7 +428,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
     if (tid < 10) {
         double v = 0.0;
         for (int w = 0; w < NW_WAVES; w++) v += L.red[w * 10 + tid];
-        a.partial[((size_t)b * a.nblocks + blockIdx.x) * 10 + tid] = v;
+        a.partial[ev_partial(a.nblocks, b, blockIdx.x, tid)] = v;
     }
 }
 

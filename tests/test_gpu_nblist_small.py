@@ -1,4 +1,4 @@
-"""Lists of structures whose binning one workgroup does (csrc/nblist.hip, small_bins_kernel): atom counts around its
+"""Lists of structures whose binning one launch does (csrc/nblist.hip, small_bins_kernel): atom counts around its
 threads and its limit, cells told axis by axis and cells whose images are tried one by one, open boundaries, and boxes
 that do not fit (atoms far outside the cell), where the build starts over on the general route."""
 import numpy as np
@@ -133,7 +133,7 @@ def growing_boxes(n, outside):
 @pytest.mark.parametrize("outside", [-1.1, 0.9])
 def test_sync_free_box_grown_by_an_eighth(oracle, dt, n, outside):
     """Atoms that spread or crowd together within the box of the synchronised build and its eighth: boxes of more bins, and
-    more images, than one workgroup holds in LDS are binned all the same."""
+    more images, than the one launch holds in LDS are binned all the same."""
     L, rcut, xs = growing_boxes(n, outside)
     sync_free_builds(oracle, np.diag(L).astype(dt), synth.rng_randint(n, n, 2), [x.astype(dt) for x in xs], rcut, 1200)
 
@@ -160,6 +160,20 @@ def test_more_images_than_lds(oracle, dt):
         # 400 terms a row, of either sign: two summation orders in single precision
         for a, b in ((e, e0), (f, f0), (v, v0)):
             assert (a - b).abs().max() <= 1e-5 * b.abs().max()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("tilt", [0.0, 0.1])
+def test_one_plane_of_bins_with_more_images_than_lds(oracle, dt, tilt):
+    """2400 atoms in one plane across x, around the corner of the other two axes: 9600 images for one workgroup; in a tilted
+    cell the images are tried one by one (1600 atoms with nine images each stay below the limit of that way)."""
+    n = 2400 if tilt == 0.0 else 1600
+    u = synth.rng_uniform(11, 3 * n).reshape(n, 3)
+    lat = np.diag([6.0, 30.0, 30.0])
+    lat[2, 1] = tilt * 30.0
+    x = np.stack([2.8 + 0.4 * u[:, 0], (9.0 * u[:, 1] - 4.5) % 30.0, (9.0 * u[:, 2] - 4.5) % 30.0], 1)
+    ty = synth.rng_randint(12, n, 2)
+    sync_free_builds(oracle, lat.astype(dt), ty, [x.astype(dt)] * 2, 5.0, n, pbc=(False, True, True))
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
