@@ -199,7 +199,9 @@ int pair_segment_capacity(int U);
 // `force` it calls pair_mark_own on the atom's cursor when `mark` is set: the reduction then takes every other atom's own
 // sum for zero, so that `force` needs no clearing, and leaves the cursors zero for the next call.
 constexpr int PAIR_OWN = (int)0x80000000;          // counts stay below 2^31
-__device__ __forceinline__ int pair_claim(int* cursor) { return atomicAdd(cursor, 1) & ~PAIR_OWN; }
+__device__ __forceinline__ int pair_claim_raw(int* cursor) { return atomicAdd(cursor, 1); }
+__device__ __forceinline__ int pair_rank(int raw) { return raw & ~PAIR_OWN; }       // (where the rank is used: it waits for the claim)
+__device__ __forceinline__ int pair_claim(int* cursor) { return pair_rank(pair_claim_raw(cursor)); }
 __device__ __forceinline__ void pair_mark_own(int* cursor) { atomicOr(cursor, PAIR_OWN); }
 struct PairCsr {
     int* cursor = nullptr;

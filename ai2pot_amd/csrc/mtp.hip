@@ -106,7 +106,11 @@ struct MtpArgs {
     const T* dVs;      // [B, 9]     2 v_w / (9N) (V - V_dft)
     T* gpart;          // [B, P, ngrad] per-atom gradient rows (ngrad = ncoef + n_scalar + ntypes)
     int ngrad;
+    // Places in LDS, in entries (AtomLds), and in a row of the neighbour table: worked out once for the launch.
+    int at_Tg, at_cf, at_tab, at_A, at_Bm, at_gred, at_Ab, at_Bb, at_pq, at_polys, at_net;
+    int OY, OZ, OG, ODG, OU, OW, OF, ODF;
     int lds_basic_off;  // byte offset of the packed basic-moment table in LDS
+    int mom_groups;     // thread groups that share a row's neighbours in the sums of the basic moments (basic_sums), or 0
     int nc_cap;         // rows of the LDS neighbour table: a row is processed in chunks of at most nc_cap
     int keep_table;     // energy / force / virial kernel: the adjoints lie behind the table (mtp_table_region)
     // site-energy / descriptor mode (linearMtp.h:514-611, 821-890)
@@ -127,6 +131,31 @@ struct MtpArgs {
     T* pair_out;       // [B, P, U, 3] derivative of the row's weighted moments along each pair vector, or null
 };
 
+// The kernels' arguments are some eighty scalars, and the plan names two dozen arrays: held in registers from the first
+// use to the last they do not fit, and what did not (some 150 values) moved between lanes of vector registers all the time:
+// 300 instead of 281 us for the energies and forces of level 20, 8192 atoms, 238 instead of 222 for the loss gradient of
+// level 16, 64 structures of 128 atoms.  Each phase takes the arguments from the segment they were passed in anew (scalar loads; the empty
+// statement keeps the compiler from carrying an earlier phase's values over).
+#define A2P_CONSTANT __attribute__((address_space(4)))
+template <typename S>
+__device__ __forceinline__ const A2P_CONSTANT S& again(const A2P_CONSTANT S* args)
+{
+    asm volatile("" : "+s"(args));
+    return *args;
+}
+template <typename T>
+__device__ __forceinline__ const A2P_CONSTANT MtpArgs<T>* kernel_args()
+{
+    return (const A2P_CONSTANT MtpArgs<T>*)__builtin_amdgcn_kernarg_segment_ptr();      // the first parameter
+}
+// A plan array that a wavefront reads uniformly: by scalar loads.
+template <typename S>
+__device__ __forceinline__ const A2P_CONSTANT S* uniform_array(const S* p) { return (const A2P_CONSTANT S*)(uintptr_t)p; }
+
+// a / b for small integers, 0 <= a < 2^20, b > 0 (the exact quotient is at least 0.5 / b away from the next integer, the
+// rounding here below 2^-22 of it)
+__device__ __forceinline__ int small_div(int a, int b) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b)); }
+
 __device__ __forceinline__ float tanh_t(float x) { return tanhf(x); }
 __device__ __forceinline__ double tanh_t(double x) { return tanh(x); }
 
@@ -135,7 +164,7 @@ __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 
 // Per-neighbour table for neighbours [c0, c0+nc) of the row.
 // Layout per neighbour (E entries of T): ux^0..kmax | uy^.. | uz^.. | g[nmus] | dg[nmus] |
-// ux uy uz 1/r | (loss mode) wx wy wz w.u | f[K] | df[K]
+// ux uy uz 1/r | (loss mode) vx vy vz w.u | f[K] | df[K]
 // PASS says what the pass that follows reads: TAB_MOMENTS powers, g, dg; TAB_TANGENTS also w; TAB_GRADIENT powers, w, f, df.
 // The threads form groups of nc, a neighbour to a thread.  Groups share the radial functions, two to a Chebyshev
 // recurrence (coefficients from the LDS copy `cf` of the centre species' block); more than two where the workgroup has no
@@ -147,13 +176,13 @@ __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 // Lanes j < nc also return the neighbour's index, validity and displacement.
 enum TablePass { TAB_MOMENTS, TAB_TANGENTS, TAB_GRADIENT };
 
-template <typename T, TablePass PASS, int NT>
-__device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T* cf, int lane, int nc, int c0,
+template <typename T, TablePass PASS, int NT, typename Args>
+__device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int lane, int nc, int c0,
                                             const T* rcs, const int* first, const int* types, int center,
                                             int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true)
 {
     const int kmax = a.p.kmax, nmus = a.p.nmus, K = a.K;
-    const int OG = 3 * (kmax + 1), ODG = OG + nmus, OU = ODG + nmus, OW = OU + 4, OF = OW + 4, ODF = OF + K;
+    const int OG = a.OG, ODG = a.ODG, OU = a.OU, OW = a.OW, OF = a.OF, ODF = a.ODF;
     *valid_out = false;
     *nj_out = center;
     if (lane < nc) {
@@ -171,13 +200,13 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
     constexpr int OTHERS = PASS == TAB_MOMENTS ? 1 : (PASS == TAB_TANGENTS ? 2 : 3);
     int share = 0, nrad = 0;
     if (PASS != TAB_GRADIENT) {
-        nrad = max(1, min((nmus + 1) / 2, NT / nc - OTHERS));
-        share = ((nmus + nrad - 1) / nrad + 1) & ~1;
-        nrad = (nmus + share - 1) / share;
+        nrad = max(1, min((nmus + 1) / 2, __builtin_amdgcn_readfirstlane(small_div(NT, nc)) - OTHERS));
+        share = (__builtin_amdgcn_readfirstlane(small_div(nmus + nrad - 1, nrad)) + 1) & ~1;
+        nrad = __builtin_amdgcn_readfirstlane(small_div(nmus + share - 1, share));
     }
     const int ntask = nc * (nrad + OTHERS);
     for (int task = lane; task < ntask; task += NT) {
-        const int role = task / nc, j = task - role * nc;
+        const int role = small_div(task, nc), j = task - role * nc;
         const int jj = c0 + j;
         const T x = rcs[jj * 3 + 0], y = rcs[jj * 3 + 1], z = rcs[jj * 3 + 2];
         const T r = sqrt_t(x * x + y * y + z * z);
@@ -196,7 +225,8 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
         int nj = first[jj];
         if ((unsigned)nj >= (unsigned)NF) nj = center;
         if (PASS != TAB_MOMENTS && role == nrad + 1) {
-            // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386)
+            // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386), kept as w . u and
+            // v = (w - (w . u) u) / r: the monomials are homogeneous, k m = u . grad m, so D_w m = (w . u) m' + v . grad m
             const T* fc = a.dFs + ((size_t)b * a.P + center) * 3;
             const T* fn = a.dFs + ((size_t)b * a.P + nj) * 3;
             const T* dv = a.dVs + (size_t)b * 9;
@@ -204,8 +234,11 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
 #pragma unroll
             for (int q = 0; q < 3; q++)
                 w[q] = fc[q] - fn[q] - (dv[q * 3 + 0] * x + dv[q * 3 + 1] * y + dv[q * 3 + 2] * z);
-            t[OW + 0] = w[0]; t[OW + 1] = w[1]; t[OW + 2] = w[2];
-            t[OW + 3] = (w[0] * x + w[1] * y + w[2] * z) / r;
+            const T rinv = (T)1 / r, wu = (w[0] * x + w[1] * y + w[2] * z) * rinv;
+            t[OW + 0] = (w[0] - wu * (x * rinv)) * rinv;
+            t[OW + 1] = (w[1] - wu * (y * rinv)) * rinv;
+            t[OW + 2] = (w[2] - wu * (z * rinv)) * rinv;
+            t[OW + 3] = wu;
             continue;
         }
         // radial functions, basis.h:154-196, 351-381, 620-637
@@ -253,15 +286,99 @@ __device__ __forceinline__ void build_table(const MtpArgs<T>& a, T* tab, const T
     }
 }
 
-// Sum over the pieces of a list (mtp_plan.h): the pieces sit in neighbouring lanes of one wavefront, `rem` is the
-// number of pieces behind the lane's own in its list; after `steps` doubling steps the lane of a list's first piece
-// holds the list's sum (pieces in a fixed tree order).  All 64 lanes take part.
+// Basic moments of the polynomial (mu, a, b, z^0 .. z^(len-1)) that the thread owns (mtp_plan.h: polys_len), over every
+// ng-th neighbour of a chunk from the h-th on: four LDS reads per polynomial and neighbour and two operations per moment;
+// a thread per basic moment takes four reads and three operations each (tangents: eleven reads and twenty operations; the
+// loss gradient of level 16, 64 structures of 128 atoms, ~ 10 of 230 us longer; energies and forces within 1 %).
+// With TANGENT also D_w M = sum (w . u) g' m + g v . grad m.  `top` is the length of the wavefront's longest polynomial;
+// what a shorter one sums up beyond its length is not used.
+// (A copy of the loop for every second length: one for all, ended by a test behind each power, becomes selects.)
+constexpr int MTP_POLY_MAX = 10;       // longest polynomial (levels up to 22)
+template <typename T, bool TANGENT, int N>
+__device__ __forceinline__ void basic_loop(const T* tab, int E, int nc, int h, int ng, int mu, int ea, int eb, int OX, int OY,
+                                           int OZ, int OG, int ODG, int OW, T (&acc)[MTP_POLY_MAX],
+                                           T (&tacc)[TANGENT ? MTP_POLY_MAX : 1])
+{
+#pragma unroll 1
+    for (int j = h; j < nc; j += ng) {
+        const T* t = tab + j * E;
+        const T xa = t[OX + ea], yb = t[OY + eb], z = t[OZ + 1], g = t[OG + mu];
+        const T ab = xa * yb;
+        T p = g * ab;
+        if (!TANGENT) {
+#pragma unroll
+            for (int c = 0; c < N; c++) {
+                acc[c] += p;
+                if (c + 1 < N) p *= z;
+            }
+        } else {
+            const T q = t[OW + 3] * t[ODG + mu] * ab +
+                        g * (((T)ea * t[OX + max(ea - 1, 0)] * yb) * t[OW + 0] + ((T)eb * xa * t[OY + max(eb - 1, 0)]) * t[OW + 1]);
+            const T pv = p * t[OW + 2];
+            T zc = (T)1, dz = (T)0;                              // z^c and its derivative
+#pragma unroll
+            for (int c = 0; c < N; c++) {
+                acc[c] += p * zc;
+                tacc[c] += q * zc + pv * dz;
+                dz = dz * z + zc;
+                zc *= z;
+            }
+        }
+    }
+}
+template <typename T, bool TANGENT>
+__device__ __forceinline__ void basic_sums(const T* tab, int E, int nc, int h, int ng, unsigned word, int top, int OX, int OY,
+                                           int OZ, int OG, int ODG, int OW, T (&acc)[MTP_POLY_MAX],
+                                           T (&tacc)[TANGENT ? MTP_POLY_MAX : 1])
+{
+    const int mu = word & 7, ea = (word >> 3) & 31, eb = (word >> 8) & 31;
+#pragma unroll
+    for (int c = 0; c < MTP_POLY_MAX; c++) {
+        acc[c] = (T)0;
+        if (TANGENT) tacc[c] = (T)0;
+    }
+    if (h >= ng) nc = 0;
+    if (top <= 2) basic_loop<T, TANGENT, 2>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
+    else if (top <= 4) basic_loop<T, TANGENT, 4>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
+    else if (top <= 6) basic_loop<T, TANGENT, 6>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
+    else if (top <= 8) basic_loop<T, TANGENT, 8>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
+    else basic_loop<T, TANGENT, 10>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
+}
+
+// A thread's sums to its group's coefficients in `part` [ng][ncoef] (highest power first), and a coefficient's sum over the
+// groups, in their order.
+template <typename T>
+__device__ __forceinline__ void basic_part(T* part, const T (&acc)[MTP_POLY_MAX], int h, int ng, unsigned word, int ncoef)
+{
+    const int len = (word >> 13) & 63;
+    T* const mine = part + h * ncoef + (word >> 19) + (len - 1);
+    if (h < ng) {
+#pragma unroll
+        for (int c = 0; c < MTP_POLY_MAX; c++)
+            if (c < len) mine[-c] = acc[c];
+    }
+}
+template <typename T>
+__device__ __forceinline__ T group_sum(const T* src, int ng, int ncoef)
+{
+    T v = src[0];
+    for (int k = 1; k < ng; k++) v += src[k * ncoef];
+    return v;
+}
+
+// Sum over the pieces of a list (mtp_plan.h: MtpStream): `rem` is the number of pieces behind the lane's own in its list;
+// after `steps` doubling steps the lane of a list's first piece holds the list's sum (pieces in a fixed tree order).  Within
+// a row of sixteen lanes by data-parallel moves, which bring a zero from beyond the row.  All 64 lanes take part.
 template <typename T>
 __device__ __forceinline__ T piece_sum(T v, int rem, int steps)
 {
-    for (int k = 0; k < steps; k++) {
-        const int d = 1 << k;
-        const T o = __shfl_down(v, d, 64);
+    T o = wave::dpp_move<0x101>(v);                   // row_shl:1
+    v += rem >= 1 ? o : (T)0;
+    if (steps > 1) { o = wave::dpp_move<0x102>(v); v += rem >= 2 ? o : (T)0; }
+    if (steps > 2) { o = wave::dpp_move<0x104>(v); v += rem >= 4 ? o : (T)0; }
+    if (steps > 3) { o = wave::dpp_move<0x108>(v); v += rem >= 8 ? o : (T)0; }
+    for (int d = 16; d < 1 << steps; d <<= 1) {
+        o = __shfl_down(v, d, 64);
         v += rem >= d ? o : (T)0;
     }
     return v;
@@ -275,41 +392,74 @@ __device__ __forceinline__ T plan_entry(const T* base, unsigned off)
     return *(const T*)((const char*)base + (sizeof(T) == 8 ? off : off >> 1));
 }
 
-// forward products: M[dst] = sum mult M[m0] M[m1]; with TANGENT also the product rule on Tg.
-template <typename T, bool TANGENT, int NT>
-__device__ __forceinline__ void sweep_forward(const MtpPlanDevice& p, T* M, T* Tg, int tid)
+// A gather (mtp_plan.h: MtpStream): terms(words) for a step's terms of the thread's slot and done(slot, rem, steps) behind the
+// last of a group; a barrier behind every level.  What bounds it is the number of instructions a wavefront issues one after
+// the other, so the plan holds everything in the order of use; the words of the next two steps are on their way meanwhile,
+// also across a barrier (the plan does not depend on the moments).  Looking up each group's place, depth and moment when
+// its turn comes took 280 instead of 260 us for the whole kernel at level 20, 8192 atoms, 217 instead of 203 for the loss
+// gradient and 193 instead of 176 for the columns of the linear solver (level 16, 64 structures of 128 atoms).
+template <typename Stream, typename Terms, typename Done>
+__device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& done)
 {
-    for (int l = 0; l < p.n_levels; l++) {
-        const int s0 = p.f_level[l], s1 = p.f_level[l + 1];     // whole groups of 64 slots: every lane of a wave walks one
-        for (int s = s0 + tid; s < s1; s += NT) {
-            const int grp = __builtin_amdgcn_readfirstlane(s >> 6);     // the wavefront's group: scalar loads below
-            const int steps = p.f_multi[grp];                // of the group: only groups with cut lists pay for the sums
-            const int depth = p.f_gdepth[grp];               // shared by the 64 lanes of the group, a multiple of MTP_DEPTH_STEP
-            const int2* tp = p.f_terms + p.f_gbase[grp] + (s & 63);
-            const int dst = p.f_dst[s];                      // requested with the two words above
-            const int rem = steps ? p.f_rem[s] : 0;
-            T acc = (T)0, tacc = (T)0;
-            // all the slot's words (at most MTP_SLOT_CAP, the depth is shared by the wavefront) are requested
-            // before the first is used: one trip to memory per slot
-            int2 w[MTP_SLOT_CAP];
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const A2P_CONSTANT int* const head = uniform_array((const int*)g.head) + wave * 4;
+    const int first = head[0], n = head[1];
+    for (int k = head[3]; k > 0; k--) __syncthreads();
+    if (n == 0) return;
+    const A2P_CONSTANT int* ctrl = uniform_array(g.ctrl) + first;
+    const int* sp = g.slots + (size_t)head[2] * 64 + lane;
+    const int2* tp = g.words + (size_t)first * (MTP_DEPTH_STEP * 64) + lane;
+    int2 a[MTP_DEPTH_STEP], b[MTP_DEPTH_STEP];
+    int slot = sp[0], next_slot = sp[64];              // (each array ends with two steps' worth of padding)
 #pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k += MTP_DEPTH_STEP)
-                if (k < depth) {
+    for (int u = 0; u < MTP_DEPTH_STEP; u++) a[u] = tp[u * 64];
 #pragma unroll
-                    for (int u = 0; u < MTP_DEPTH_STEP; u++) w[k + u] = tp[(k + u) * 64];
-                }
+    for (int u = 0; u < MTP_DEPTH_STEP; u++) b[u] = tp[(MTP_DEPTH_STEP + u) * 64];
+    auto step = [&](int2 (&w)[MTP_DEPTH_STEP], int i) __attribute__((always_inline)) {
+        const int c = ctrl[i];
+        terms(w);
 #pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k += MTP_DEPTH_STEP)
-                if (k < depth) {
+        for (int u = 0; u < MTP_DEPTH_STEP; u++) w[u] = tp[(2 * MTP_DEPTH_STEP + u) * 64];
+        tp += MTP_DEPTH_STEP * 64;
+        if (c) {
+            done((slot & 0xffff) - 1, slot >> 16, (c >> 1) & 7);
+            slot = next_slot;
+            sp += 64;
+            next_slot = sp[64];
+            for (int k = c >> 4; k > 0; k--) __syncthreads();
+        }
+    };
+#pragma unroll 1
+    for (int i = 0; i < n; i += 2) {
+        step(a, i);
+        if (i + 1 == n) break;
+        step(b, i + 1);
+    }
+}
+
+// forward products: M[dst] = sum mult M[m0] M[m1]; with TANGENT also the product rule on Tg.
+template <typename T, bool TANGENT, typename Stream>
+__device__ __forceinline__ void sweep_forward(Stream& g, T* M, T* Tg, int tid)
+{
+    T acc = (T)0, tacc = (T)0;
+    walk(g, tid,
+        [&](const int2 (&w)[MTP_DEPTH_STEP]) __attribute__((always_inline)) {
+            constexpr int C = MTP_DEPTH_STEP;
+            T v0[C], v1[C], t0[C], t1[C];
 #pragma unroll
-                    for (int u = k; u < k + MTP_DEPTH_STEP; u++) {
-                        const unsigned m0 = (unsigned)w[u].x & 0xffffu, m1 = (unsigned)w[u].x >> 16;
-                        const T mult = (T)w[u].y;
-                        const T v0 = plan_entry(M, m0), v1 = plan_entry(M, m1);
-                        acc += mult * v0 * v1;
-                        if (TANGENT) tacc += plan_entry(Tg, m0) * mult * v1 + plan_entry(Tg, m1) * mult * v0;
-                    }
-                }
+            for (int u = 0; u < C; u++) {
+                const unsigned m0 = (unsigned)w[u].x & 0xffffu, m1 = (unsigned)w[u].x >> 16;
+                v0[u] = plan_entry(M, m0); v1[u] = plan_entry(M, m1);
+                if (TANGENT) { t0[u] = plan_entry(Tg, m0); t1[u] = plan_entry(Tg, m1); }
+            }
+#pragma unroll
+            for (int u = 0; u < C; u++) {
+                const T mult = (T)w[u].y;
+                acc += mult * v0[u] * v1[u];
+                if (TANGENT) tacc += t0[u] * mult * v1[u] + t1[u] * mult * v0[u];
+            }
+        },
+        [&](int dst, int rem, int steps) __attribute__((always_inline)) {
             if (steps) {
                 acc = piece_sum(acc, rem, steps);
                 if (TANGENT) tacc = piece_sum(tacc, rem, steps);
@@ -318,49 +468,37 @@ __device__ __forceinline__ void sweep_forward(const MtpPlanDevice& p, T* M, T* T
                 M[dst] = acc;
                 if (TANGENT) Tg[dst] = tacc;
             }
-        }
-        __syncthreads();
-    }
+            acc = tacc = (T)0;
+        });
 }
 
 // reverse gather: X[m] += sum mult (X[dst] M[other] (+ A[dst] Tg[other] when MIXED))
-template <typename T, bool MIXED, int NT>
-__device__ __forceinline__ void sweep_reverse(const MtpPlanDevice& p, const T* M, T* X, const T* A,
-                                              const T* Tg, int tid)
+template <typename T, bool MIXED, typename Stream>
+__device__ __forceinline__ void sweep_reverse(Stream& g, const T* M, T* X, const T* A, const T* Tg, int tid)
 {
-    for (int l = p.n_levels - 1; l >= 0; l--) {
-        const int s0 = p.r_level[l], s1 = p.r_level[l + 1];
-        for (int s = s0 + tid; s < s1; s += NT) {
-            const int grp = __builtin_amdgcn_readfirstlane(s >> 6);
-            const int steps = p.r_multi[grp];
-            const int depth = p.r_gdepth[grp];
-            const int2* tp = p.r_terms + p.r_gbase[grp] + (s & 63);
-            const int src = p.r_src[s];
-            const int rem = steps ? p.r_rem[s] : 0;
-            T acc = (T)0;
-            int2 w[MTP_SLOT_CAP];
+    T acc = (T)0;
+    walk(g, tid,
+        [&](const int2 (&w)[MTP_DEPTH_STEP]) __attribute__((always_inline)) {
+            constexpr int C = MTP_DEPTH_STEP;
+            T v0[C], v1[C], t0[C], t1[C];
 #pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k += MTP_DEPTH_STEP)
-                if (k < depth) {
+            for (int u = 0; u < C; u++) {
+                const unsigned dst = (unsigned)w[u].x & 0xffffu, other = (unsigned)w[u].x >> 16;
+                v0[u] = plan_entry(X, dst); v1[u] = plan_entry(M, other);
+                if (MIXED) { t0[u] = plan_entry(A, dst); t1[u] = plan_entry(Tg, other); }
+            }
 #pragma unroll
-                    for (int u = 0; u < MTP_DEPTH_STEP; u++) w[k + u] = tp[(k + u) * 64];
-                }
-#pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k += MTP_DEPTH_STEP)
-                if (k < depth) {
-#pragma unroll
-                    for (int u = k; u < k + MTP_DEPTH_STEP; u++) {
-                        const unsigned dst = (unsigned)w[u].x & 0xffffu, other = (unsigned)w[u].x >> 16;
-                        const T mult = (T)w[u].y;
-                        acc += plan_entry(X, dst) * mult * plan_entry(M, other);
-                        if (MIXED) acc += mult * plan_entry(A, dst) * plan_entry(Tg, other);
-                    }
-                }
+            for (int u = 0; u < C; u++) {
+                const T mult = (T)w[u].y;
+                acc += v0[u] * mult * v1[u];
+                if (MIXED) acc += mult * t0[u] * t1[u];
+            }
+        },
+        [&](int src, int rem, int steps) __attribute__((always_inline)) {
             if (steps) acc = piece_sum(acc, rem, steps);
             if (src >= 0) X[src] += acc;
-        }
-        __syncthreads();
-    }
+            acc = (T)0;
+        });
 }
 
 // sum over the NT threads of a workgroup in a fixed order (wave sums, then wave 0 .. last)
@@ -379,8 +517,8 @@ __device__ __forceinline__ T block_sum(T v, T* scratch, int tid)
 }
 
 // The adjoints of the basic moments as coefficients of the row polynomials (mtp_plan.h).  Ends without a barrier.
-template <typename T, int NT>
-__device__ __forceinline__ void scatter_polys(const MtpPlanDevice& p, T* __restrict__ dst, const T* __restrict__ src, int tid)
+template <typename T, int NT, typename Plan>
+__device__ __forceinline__ void scatter_polys(Plan& p, T* __restrict__ dst, const T* __restrict__ src, int tid)
 {
     if (p.poly_unique && p.ncoef_poly == p.n_basic) {        // the usual case: a permutation
         for (int i = tid; i < p.n_basic; i += NT) dst[p.poly_pos[i]] = src[i];
@@ -453,15 +591,13 @@ __device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __re
 template <typename T>
 __device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __restrict__ Ac, const T* __restrict__ Bc,
                                           const int* __restrict__ polys, int& s, int end, int ng, int OX, int OY, int OZ,
-                                          int OU, int OW, T cE, bool no_tan, T& P, T& Q)
+                                          int OW, T cE, bool no_tan, T& P, T& Q)
 {
     P = Q = (T)0;
     if (s >= end) return;
-    const T z = t[OZ + 1], rinv = t[OU + 3];
+    const T z = t[OZ + 1];
     const T wu = no_tan ? (T)0 : t[OW + 3];
-    const T vx = no_tan ? (T)0 : (t[OW + 0] - wu * t[OU + 0]) * rinv;
-    const T vy = no_tan ? (T)0 : (t[OW + 1] - wu * t[OU + 1]) * rinv;
-    const T vz = no_tan ? (T)0 : (t[OW + 2] - wu * t[OU + 2]) * rinv;
+    const T vx = no_tan ? (T)0 : t[OW + 0], vy = no_tan ? (T)0 : t[OW + 1], vz = no_tan ? (T)0 : t[OW + 2];
     for (; s < end; s += ng) {
         const int pw = polys[s];
         const int ea = pw & 31, eb = (pw >> 5) & 31;
@@ -487,97 +623,163 @@ __device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __re
     Q *= wu;
 }
 
+// The workgroup's LDS: moments | (loss mode: their tangents) | coefficients of the centre species | region of the neighbour
+// table | ...
+template <typename T, bool LOSS, int NT>
+struct AtomLds {
+    T *M, *Tg, *cf, *tab, *A, *Bm, *gred, *Ab, *Bb, *pq, *polys, *net;
+    unsigned* bas;
+    int* rws;
+    bool keep;
+    template <typename Args>
+    __device__ __forceinline__ AtomLds(Args& a, unsigned char* smem)
+    {
+        M = (T*)smem;
+        Tg = M + a.at_Tg;
+        cf = M + a.at_cf;                       // [ntypes][nmus][K]
+        tab = M + a.at_tab;
+        // the adjoints (loss mode: and the mixed adjoints) share the table's region, or lie behind the table (keep)
+        keep = !LOSS && a.keep_table != 0;      // uniform over the launch
+        A = M + a.at_A;
+        Bm = M + a.at_Bm;
+        gred = M + a.at_gred;                   // partial sums of the thread groups
+        // loss mode: adjoints and mixed adjoints of the basic moments (as coefficients of the polynomials) | P[nc][nmus] |
+        // Q[nc][nmus] | ...
+        Ab = M + a.at_Ab;
+        Bb = M + a.at_Bb;
+        pq = M + a.at_pq;
+        polys = M + a.at_polys;                 // energy / force / virial: coefficients of the polynomials
+        net = M + a.at_net;                     // network inputs and per-neuron values
+        // behind everything else: (mu, a, b, c) of every basic moment, one byte each, or its place among the coefficients
+        // (mom_groups); monomial rows and polynomials of the pair-derivative walk
+        bas = (unsigned*)(smem + a.lds_basic_off);
+        rws = (int*)(bas + a.p.n_basic);
+    }
+};
+
+// What a phase of the atom kernel works with, under the names of the formulas.
+#define MTP_PHASE                                                                                                          \
+    [[maybe_unused]] auto& a = again(kernel_args<T>());                                                                    \
+    [[maybe_unused]] auto& p = a.p;                                                                                        \
+    [[maybe_unused]] const bool seeded = (SEED || LOSS) && a.row_seed != nullptr;                                          \
+    [[maybe_unused]] const bool no_tan = LOSS && a.no_tangent != 0;                 /* uniform over the launch */          \
+    [[maybe_unused]] const AtomLds<T, LOSS, NT> L(a, smem_raw);                                                            \
+    [[maybe_unused]] T *const M = L.M, *const Tg = L.Tg, *const cf = L.cf, *const tab = L.tab, *const A = L.A, *const Bm = L.Bm; \
+    [[maybe_unused]] const int NF = a.P + a.nghost, n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, kmax = p.kmax,  \
+                               K = a.K, E = a.E, MTP_NC = a.nc_cap;                                                        \
+    [[maybe_unused]] const int OX = 0, OY = a.OY, OZ = a.OZ, OG = a.OG, ODG = a.ODG, OU = a.OU, OW = a.OW, OF = a.OF, ODF = a.ODF; \
+    [[maybe_unused]] const size_t row = (size_t)b * a.P + ii;                                                              \
+    [[maybe_unused]] const int* const first = a.bfirstneigh + row * a.U;                                                   \
+    [[maybe_unused]] const T* const rcs = a.brcs + row * a.U * 3;                                                          \
+    [[maybe_unused]] const int* const types = a.btypes + (size_t)b * NF
+
 // NT threads per centre atom: 64 or 256 (wide_atoms).  Five workgroups of 256 threads fit the LDS of a CU at level 20 and
 // the registers are kept to match (four: 321 us instead of 303 at 8192 atoms; six spill: 361).
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
 // (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.
 template <typename T, bool LOSS, int NT, bool SEED = false>
-__global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_atom_kernel(const MtpArgs<T> a)
+__global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) == 8 ? 6 : 1)) mtp_atom_kernel(const MtpArgs<T>)
 {
-    const bool seeded = (SEED || LOSS) && a.row_seed != nullptr;
-    const bool no_tan = LOSS && a.no_tangent != 0;      // uniform over the launch
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const MtpPlanDevice& p = a.p;
     const int lane = threadIdx.x;     // thread in the workgroup
     const int ii = blockIdx.x, b = blockIdx.y;
-    const int NF = a.P + a.nghost;
-    const size_t row = (size_t)b * a.P + ii;
-    const int n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, kmax = p.kmax, K = a.K, E = a.E;
-    const int OX = 0, OY = kmax + 1, OZ = 2 * (kmax + 1), OG = 3 * (kmax + 1), ODG = OG + nmus,
-              OU = ODG + nmus, OW = OU + 4, OF = OW + 4, ODF = OF + K;
-    const int ncoef = a.ntypes * a.ntypes * nmus * K;
+    int center, nn, ti;
+    int mgroups, mh, mtop = 0;        // sums of the basic moments: groups, the thread's group, the longest polynomial
+    unsigned pword = 0;               // ... and the thread's polynomial
+    {
+        MTP_PHASE;
+        if (ii >= a.binum[b]) {                  // padded row: contributes nothing
+            if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
+            if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
+            if (!LOSS && a.desc)
+                for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
+            if (LOSS)
+                for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
+            return;
+        }
+        center = __builtin_amdgcn_readfirstlane(a.bilist[row]);
+        nn = __builtin_amdgcn_readfirstlane(a.bnumneigh[row]);
+        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
+        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
+        ti = __builtin_amdgcn_readfirstlane(types[center]);
+        if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
 
-    const int MTP_NC = a.nc_cap;
-    // moments | (loss mode: their tangents) | coefficients | region of the neighbour table
-    T* M = (T*)smem_raw;
-    T* Tg = M + n_moms;
-    T* cf = Tg + (LOSS ? n_moms : 0);        // coefficients of the centre species: [ntypes][nmus][K]
-    T* tab = cf + a.ntypes * nmus * K;
-    // the adjoints (loss mode: and the mixed adjoints) share the table's region, behind the sweeps' partial sums
-    const bool keep = !LOSS && a.keep_table != 0;       // uniform over the launch
-    T* A = tab + (keep ? mtp_table_entries(MTP_NC, E, LOSS, n_moms, NT) : mtp_adjoint_offset((LOSS ? 2 : 1) * p.max_level_slots));
-    T* Bm = A + n_moms;
-    // [256/32][32][4] partial sums of the thread groups.  They are needed only in the last pass over the
-    // neighbours, when the moments (and, in loss mode, their tangents) are dead: a long enough moment
-    // vector lends them its place
-    const bool share = mtp_gred_in_moments(LOSS, n_moms);
-    // energy / force / virial kernel: the group sums are written over the table once it has been read
-    T* gred = LOSS ? (share ? M : tab + MTP_NC * E) : tab;
-    // loss mode, behind the region: adjoints and mixed adjoints of the basic moments (as coefficients of the polynomials) |
-    // P[nc][nmus] | Q[nc][nmus] | ...
-    T* Ab = tab + mtp_table_region(MTP_NC, E, LOSS, n_moms, p.max_level_slots, NT, keep);
-    T* Bb = Ab + p.ncoef_poly;
-    T* pq = LOSS ? Bb + p.ncoef_poly : Ab;
+        mgroups = a.mom_groups;       // uniform over the launch
+        const unsigned* const bsrc = mgroups ? (const unsigned*)p.poly_pos : p.basic;
+        for (int i = lane; i < n_basic; i += NT) L.bas[i] = bsrc[i];
+        mh = mgroups;
+        if (mgroups) {
+            mh = small_div(lane, p.npoly);
+            if (mh < mgroups) pword = p.polys_len[lane - mh * p.npoly];
+            const int len = (pword >> 13) & 63;
+#pragma unroll
+            for (int c = 0; c < MTP_POLY_MAX; c++)
+                if (__any(len > c)) mtop = c + 1;
+        }
+        int* const rws = L.rws;
+        if (!LOSS) {
+            for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
+            for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
+        } else {
+            for (int i = lane; i < p.npoly; i += NT) rws[i] = p.polys_mu[i];
+            for (int i = lane; i <= nmus; i += NT) rws[p.npoly + i] = p.polys_end[i];
+        }
+        for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
+        for (int i = lane; i < n_moms; i += NT) {
+            M[i] = (T)0;
+            if (LOSS) Tg[i] = (T)0;
+        }
+        __syncthreads();
+    }
 
-    if (ii >= a.binum[b]) {                  // padded row: contributes nothing
-        if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
-        if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
-        if (!LOSS && a.desc)
-            for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
-        if (LOSS)
-            for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
-        return;
+    // The row is cut into equal chunks of at most nc_cap neighbours.
+    int nchunks, csize;
+    {
+        MTP_PHASE;
+        nchunks = __builtin_amdgcn_readfirstlane(small_div(nn + MTP_NC - 1, MTP_NC));
+        csize = nchunks > 1 ? __builtin_amdgcn_readfirstlane(small_div(nn + nchunks - 1, nchunks)) : max(nn, 1);
     }
-    int center = a.bilist[row];
-    int nn = a.bnumneigh[row];
-    if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
-    if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-    const int* types = a.btypes + (size_t)b * NF;
-    int ti = types[center];
-    if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
-    const int* first = a.bfirstneigh + row * a.U;
-    const T* rcs = a.brcs + row * a.U * 3;
-
-    // (mu, a, b, c) of every basic moment, one byte each, behind everything else in LDS
-    unsigned* bas = (unsigned*)(smem_raw + a.lds_basic_off);
-    for (int i = lane; i < n_basic; i += NT)
-        bas[i] = p.basic[i];
-    int* rws = (int*)(bas + n_basic);        // monomial rows and polynomials of the pair-derivative walk
-    if (!LOSS) {
-        for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
-        for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
-    } else {
-        for (int i = lane; i < p.npoly; i += NT) rws[i] = p.polys_mu[i];
-        for (int i = lane; i <= nmus; i += NT) rws[p.npoly + i] = p.polys_end[i];
-    }
-    for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
-    for (int i = lane; i < n_moms; i += NT) {
-        M[i] = (T)0;
-        if (LOSS) Tg[i] = (T)0;
-    }
-    __syncthreads();
 
     // ---- basic moments (and their tangents) --------------------------------------------------
-    const int chunk = nn > 0 ? (nn + (nn + MTP_NC - 1) / MTP_NC - 1) / ((nn + MTP_NC - 1) / MTP_NC) : 1;
-    for (int c0 = 0; c0 < nn; c0 += chunk) {
-        const int nc = min(chunk, nn - c0);
-        int nj; bool valid; T d[3];
-        build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
-        __syncthreads();
+    for (int c0 = 0; c0 < nn; c0 += csize) {
+        const int nc = min(csize, nn - c0);
+        {
+            MTP_PHASE;
+            int nj; bool valid; T d[3];
+            build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+            __syncthreads();
+        }
+        MTP_PHASE;
+        if (mgroups) {
+            // the groups' sums pass through the table's place, or through the adjoints' when the table stays
+            T* const part = L.keep ? A : tab;
+            T macc[MTP_POLY_MAX];
+            if (LOSS && !no_tan) {
+                T mtan[LOSS ? MTP_POLY_MAX : 1];
+                basic_sums<T, LOSS>(tab, E, nc, mh, mgroups, pword, mtop, OX, OY, OZ, OG, ODG, OW, macc, mtan);
+                if constexpr (LOSS) {
+                    __syncthreads();
+                    basic_part<T>(part + mgroups * p.ncoef_poly, mtan, mh, mgroups, pword, p.ncoef_poly);
+                }
+            } else {
+                T none[1];
+                basic_sums<T, false>(tab, E, nc, mh, mgroups, pword, mtop, OX, OY, OZ, OG, ODG, OW, macc, none);
+                if (!L.keep) __syncthreads();
+            }
+            basic_part<T>(part, macc, mh, mgroups, pword, p.ncoef_poly);
+            __syncthreads();
+            for (int i = lane; i < n_basic; i += NT) {
+                const int pos = L.bas[i];
+                M[i] += group_sum<T>(part + pos, mgroups, p.ncoef_poly);
+                if (LOSS && !no_tan) Tg[i] += group_sum<T>(part + mgroups * p.ncoef_poly + pos, mgroups, p.ncoef_poly);
+            }
+            __syncthreads();
+            continue;
+        }
+        // (tables beyond the fields of polys_len)
         for (int i = lane; i < n_basic; i += NT) {
-            const unsigned bw = bas[i];
+            const unsigned bw = L.bas[i];
             const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
-            const T kk = (T)(ea + eb + ec);
             T acc = (T)0, tacc = (T)0;
             for (int j = 0; j < nc; j++) {
                 const T* t = tab + j * E;
@@ -586,11 +788,11 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
                 const T m = xa * yb * zc;
                 acc += g * m;
                 if (LOSS && !no_tan) {
-                    const T dg = t[ODG + mu], rinv = t[OU + 3], wu = t[OW + 3];
+                    const T dg = t[ODG + mu], wu = t[OW + 3];
                     const T gm = (T)ea * t[OX + max(ea - 1, 0)] * yb * zc * t[OW + 0] +
                                  (T)eb * xa * t[OY + max(eb - 1, 0)] * zc * t[OW + 1] +
                                  (T)ec * xa * yb * t[OZ + max(ec - 1, 0)] * t[OW + 2];
-                    tacc += wu * m * (dg - kk * g * rinv) + g * rinv * gm;
+                    tacc += wu * m * dg + g * gm;
                 }
             }
             M[i] += acc;
@@ -600,141 +802,155 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
     }
 
     // ---- products, energy, adjoint ------------------------------------------------------------
-    if (LOSS && !no_tan) sweep_forward<T, LOSS, NT>(p, M, Tg, lane);
-    else sweep_forward<T, false, NT>(p, M, Tg, lane);
-    for (int i = lane; i < n_moms; i += NT) {    // the table is dead: its place now holds the adjoints
-        A[i] = (T)0;
-        if (LOSS) Bm[i] = (T)0;
+    {
+        MTP_PHASE;
+        if (LOSS && !no_tan) sweep_forward<T, LOSS>(p.fwd[NT / 256], M, Tg, lane);
+        else sweep_forward<T, false>(p.fwd[NT / 256], M, Tg, lane);
     }
-    __syncthreads();
     T e_part = (T)0;
-    // network buffers (H > 0): inputs q[S]; per neuron w1 tanh', and in loss mode tanh, tanh', tanh'', tau
-    T* nnb = LOSS ? pq + 2 * MTP_NC * nmus + MTP_NC + a.ntypes * nmus * K : pq;
-    if (a.H > 0) {
-        // one tanh layer of the centre's species on the shifted, scaled scalar moments; the
-        // adjoint is seeded with dE_i/dM_k = sum_p w1_p tanh'(h_p) w0_pk / q_scaler_k
-        // (nnMtp.h:470-507).  Loss mode also needs the derivative of that seed along the tangent:
-        // tau_p = sum_k w0_pk Tg_k / q_scaler_k is the tangent of h_p, and the adjoint of
-        // D_w E = sum_p w1_p tanh'(h_p) tau_p  w.r.t. M_k is  sum_p w1_p tanh''(h_p) tau_p w0_pk / q_scaler_k,
-        // the seed of the mixed sweep (nnMtpLoss.h:216-610 computes the same quantities atom by atom).
-        const int S = p.n_scalar, H = a.H;
-        T* qv = nnb;                          // [S] network inputs
-        T* hv = nnb + S;                      // [H] pre-activations, then w1 * tanh'
-        T* n_th = hv + H;                     // loss mode: tanh, tanh', tanh'', tau   [H] each
-        T* n_d1 = n_th + H;
-        T* n_d2 = n_d1 + H;
-        T* n_tau = n_d2 + H;
-        const T* w0 = a.w0 + (size_t)ti * H * S;
-        const T* w1 = a.w1 + (size_t)ti * H;
-        for (int s = lane; s < S; s += NT) qv[s] = (M[p.mapping[s]] - a.q_shift[s]) / a.q_scaler[s];
-        __syncthreads();
-        for (int n = lane >> 6; n < H; n += NT / 64) {          // one wave per neuron
-            T acc = (T)0, tac = (T)0;
-            for (int k = lane & 63; k < S; k += 64) {
-                acc += w0[(size_t)n * S + k] * qv[k];
-                if (LOSS) tac += w0[(size_t)n * S + k] * Tg[p.mapping[k]] / a.q_scaler[k];
-            }
-            acc = wave::all_sum(acc);
-            if (LOSS) tac = wave::all_sum(tac);
-            if ((lane & 63) == 0) {
-                hv[n] = acc;
-                if (LOSS) n_tau[n] = tac;
-            }
+    {
+        MTP_PHASE;
+        for (int i = lane; i < n_moms; i += NT) {    // the table is dead: its place now holds the adjoints
+            A[i] = (T)0;
+            if (LOSS) Bm[i] = (T)0;
         }
         __syncthreads();
-        for (int n = lane; n < H; n += NT) {
-            const T th = tanh_t(hv[n]);
-            const T d1 = (T)1 - th * th;
-            e_part += w1[n] * th;
-            hv[n] = w1[n] * d1;
-            if (LOSS) { n_th[n] = th; n_d1[n] = d1; n_d2[n] = (T)-2 * th * d1; }
+        // network buffers (H > 0): inputs q[S]; per neuron w1 tanh', and in loss mode tanh, tanh', tanh'', tau
+        T* nnb = L.net;
+        if (a.H > 0) {
+            // one tanh layer of the centre's species on the shifted, scaled scalar moments; the
+            // adjoint is seeded with dE_i/dM_k = sum_p w1_p tanh'(h_p) w0_pk / q_scaler_k
+            // (nnMtp.h:470-507).  Loss mode also needs the derivative of that seed along the tangent:
+            // tau_p = sum_k w0_pk Tg_k / q_scaler_k is the tangent of h_p, and the adjoint of
+            // D_w E = sum_p w1_p tanh'(h_p) tau_p  w.r.t. M_k is  sum_p w1_p tanh''(h_p) tau_p w0_pk / q_scaler_k,
+            // the seed of the mixed sweep (nnMtpLoss.h:216-610 computes the same quantities atom by atom).
+            const int S = p.n_scalar, H = a.H;
+            T* qv = nnb;                          // [S] network inputs
+            T* hv = nnb + S;                      // [H] pre-activations, then w1 * tanh'
+            T* n_th = hv + H;                     // loss mode: tanh, tanh', tanh'', tau   [H] each
+            T* n_d1 = n_th + H;
+            T* n_d2 = n_d1 + H;
+            T* n_tau = n_d2 + H;
+            const T* w0 = a.w0 + (size_t)ti * H * S;
+            const T* w1 = a.w1 + (size_t)ti * H;
+            for (int s = lane; s < S; s += NT) qv[s] = (M[p.mapping[s]] - a.q_shift[s]) / a.q_scaler[s];
+            __syncthreads();
+            for (int n = lane >> 6; n < H; n += NT / 64) {          // one wave per neuron
+                T acc = (T)0, tac = (T)0;
+                for (int k = lane & 63; k < S; k += 64) {
+                    acc += w0[(size_t)n * S + k] * qv[k];
+                    if (LOSS) tac += w0[(size_t)n * S + k] * Tg[p.mapping[k]] / a.q_scaler[k];
+                }
+                acc = wave::all_sum(acc);
+                if (LOSS) tac = wave::all_sum(tac);
+                if ((lane & 63) == 0) {
+                    hv[n] = acc;
+                    if (LOSS) n_tau[n] = tac;
+                }
+            }
+            __syncthreads();
+            for (int n = lane; n < H; n += NT) {
+                const T th = tanh_t(hv[n]);
+                const T d1 = (T)1 - th * th;
+                e_part += w1[n] * th;
+                hv[n] = w1[n] * d1;
+                if (LOSS) { n_th[n] = th; n_d1[n] = d1; n_d2[n] = (T)-2 * th * d1; }
+            }
+            __syncthreads();
+            for (int k = lane; k < S; k += NT) {
+                T acc = (T)0, bac = (T)0;
+                for (int n = 0; n < H; n++) {
+                    const T w = w0[(size_t)n * S + k];
+                    acc += hv[n] * w;
+                    if (LOSS) bac += w1[n] * n_d2[n] * n_tau[n] * w;
+                }
+                A[p.mapping[k]] = acc / a.q_scaler[k];
+                if (LOSS && a.nn_exact) Bm[p.mapping[k]] = bac / a.q_scaler[k];
+            }
+        } else if (seeded) {
+            for (int s = lane; s < p.n_scalar; s += NT) A[p.mapping[s]] = a.row_seed[row * p.n_scalar + s];
+        } else {
+            for (int s = lane; s < p.n_scalar; s += NT) {
+                e_part += a.lin[s] * M[p.mapping[s]] / a.q_scaler[s];
+                A[p.mapping[s]] = a.lin[s] / a.q_scaler[s];
+            }
+        }
+        if (!LOSS && (a.e_sites || a.desc)) {
+            if (a.desc)                                          // linearMtp.h:884-885: unscaled scalar moments
+                for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = M[p.mapping[s]];
+            const T e_row = block_sum<T, NT>(e_part, tab, lane) + a.bias[ti];      // the table is idle between the sweeps
+            if (a.e_sites && lane == 0) a.e_sites[row] = e_row;  // linearMtp.h:594-599
+            if (a.energy_only) return;
         }
         __syncthreads();
-        for (int k = lane; k < S; k += NT) {
-            T acc = (T)0, bac = (T)0;
-            for (int n = 0; n < H; n++) {
-                const T w = w0[(size_t)n * S + k];
-                acc += hv[n] * w;
-                if (LOSS) bac += w1[n] * n_d2[n] * n_tau[n] * w;
-            }
-            A[p.mapping[k]] = acc / a.q_scaler[k];
-            if (LOSS && a.nn_exact) Bm[p.mapping[k]] = bac / a.q_scaler[k];
-        }
-    } else if (seeded) {
-        for (int s = lane; s < p.n_scalar; s += NT) A[p.mapping[s]] = a.row_seed[row * p.n_scalar + s];
-    } else {
-        for (int s = lane; s < p.n_scalar; s += NT) {
-            e_part += a.lin[s] * M[p.mapping[s]] / a.q_scaler[s];
-            A[p.mapping[s]] = a.lin[s] / a.q_scaler[s];
-        }
     }
-    if (!LOSS && (a.e_sites || a.desc)) {
-        if (a.desc)                                          // linearMtp.h:884-885: unscaled scalar moments
-            for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = M[p.mapping[s]];
-        const T e_row = block_sum<T, NT>(e_part, tab, lane) + a.bias[ti];      // the table is idle between the sweeps
-        if (a.e_sites && lane == 0) a.e_sites[row] = e_row;  // linearMtp.h:594-599
-        if (a.energy_only) return;
+    {
+        MTP_PHASE;
+        sweep_reverse<T, false>(p.rev[NT / 256], M, A, (const T*)nullptr, (const T*)nullptr, lane);
     }
-    __syncthreads();
-    sweep_reverse<T, false, NT>(p, M, A, nullptr, nullptr, lane);
 
     if (!LOSS) {
         // ---- pair derivatives ------------------------------------------------------------------
         // The adjoints of the basic moments as polynomial coefficients; the moments are dead
-        T* AD = mtp_polys_in_moments(p.ncoef_poly, n_moms) ? M : nnb + (a.H > 0 ? p.n_scalar + a.H : 0);
-        scatter_polys<T, NT>(p, AD, A, lane);
-        // The row is cut into equal chunks of at most MTP_NC neighbours; within a chunk of nc
-        // neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one
+        // Within a chunk of nc neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one
         // per monomial row) share the rows, so a short chunk still keeps the workgroup busy.
+        {
+            MTP_PHASE;
+            scatter_polys<T, NT>(p, L.polys, A, lane);
+        }
         T fx = (T)0, fy = (T)0, fz = (T)0;
         T vir[9];
 #pragma unroll
         for (int q = 0; q < 9; q++) vir[q] = (T)0;
-        const int nchunks = (nn + MTP_NC - 1) / MTP_NC;
-        const int csize = nchunks > 0 ? (nn + nchunks - 1) / nchunks : 1;
         for (int c0 = 0; c0 < nn; c0 += csize) {
             const int nc = min(csize, nn - c0);
-            const int ng = min(NT / nc, p.nrows);
-            const int h = lane / nc, j = lane - h * nc;
             int nj; bool valid; T d[3] = {(T)0, (T)0, (T)0};
             __syncthreads();
             // (a row of one chunk finds the table of the first pass still in place when the adjoints lie behind it)
-            build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
-                                      !(keep && nchunks == 1));
-            __syncthreads();
-            // the pair claims an entry of its target's segment (zeros too: the count of a segment is the number of pairs
-            // naming the target); claimed here, so that the walk covers the answer's way
-            const int tg = b * NF + nj;
-            int rk = 0;
-            if (a.seg_cursor && lane < nc) rk = pair_claim(&a.seg_cursor[tg]);
+            {
+                MTP_PHASE;
+                build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
+                                          !(L.keep && nchunks == 1));
+                __syncthreads();
+            }
             T gs = (T)0, wx = (T)0, wy = (T)0, wz = (T)0;
             T ux = (T)0, uy = (T)0, uz = (T)0, rinv = (T)0;
-            if (h < ng) {
-                const T* t = tab + j * E;
-                ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
-                pair_walk<T>(t, AD, rws, rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
+            // the pair claims an entry of its target's segment (zeros too: the count of a segment is the number of pairs
+            // naming the target); claimed here, so that the walk covers the answer's way
+            int rk = 0, ng, h, j;
+            {
+                MTP_PHASE;
+                ng = min(small_div(NT, nc), p.nrows);
+                h = small_div(lane, nc); j = lane - h * nc;
+                if (a.seg_cursor && lane < nc) rk = pair_claim_raw(&a.seg_cursor[b * NF + nj]);
+                if (h < ng) {
+                    const T* t = tab + j * E;
+                    ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
+                    pair_walk<T>(t, L.polys, L.rws, L.rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
+                }
             }
             __syncthreads();            // every thread has read its table row: the group sums take its place
+            MTP_PHASE;
             // group sums in the order h = 0 .. ng-1
             {
-                T* gr = gred + lane * 4;
+                T* gr = L.gred + lane * 4;
                 gr[0] = gs; gr[1] = wx; gr[2] = wy; gr[3] = wz;
             }
             __syncthreads();
             if (h == 0) {
                 for (int hh = 1; hh < ng; hh++) {
-                    const T* gr = gred + (hh * nc + j) * 4;
+                    const T* gr = L.gred + (hh * nc + j) * 4;
                     gs += gr[0]; wx += gr[1]; wy += gr[2]; wz += gr[3];
                 }
-            }
-            if (h == 0) {
                 T gx = gs * ux + wx * rinv;
                 T gy = gs * uy + wy * rinv;
                 T gz = gs * uz + wz * rinv;
                 if (!valid) { gx = (T)0; gy = (T)0; gz = (T)0; }
                 if (a.seg_cursor) {
-                    T* dst = a.seg_g + (size_t)(rk < a.seg_cap ? tg * a.seg_cap + rk : a.seg_spare) * 3;
-                    if (rk >= a.seg_cap) atomicOr(a.status, ST_SEG_OVERFLOW);
+                    rk = pair_rank(rk);
+                    const bool fits = (unsigned)rk < (unsigned)a.seg_cap;
+                    T* dst = a.seg_g + (size_t)(fits ? (b * NF + nj) * a.seg_cap + rk : a.seg_spare) * 3;
+                    if (!fits) atomicOr(a.status, ST_SEG_OVERFLOW);
                     dst[0] = gx; dst[1] = gy; dst[2] = gz;
                 }
                 if (SEED && a.pair_out) {         // padded layout of brcs; entries beyond the row stay zero
@@ -747,8 +963,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
                 vir[6] -= gz * d[0]; vir[7] -= gz * d[1]; vir[8] -= gz * d[2];
             }
         }
+        MTP_PHASE;
         // only the threads of group 0 (inside wave 0) hold force and virial terms: the other wavefronts are done
-        const double e_atom = (double)block_sum<T, NT>(e_part, gred, lane);
+        const double e_atom = (double)block_sum<T, NT>(e_part, L.gred, lane);
         if (lane >= 64) return;
         fx = wave::all_sum(fx); fy = wave::all_sum(fy); fz = wave::all_sum(fz);
         double out[10];
@@ -771,86 +988,102 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
 
     // ---- loss gradient ------------------------------------------------------------------------
     if (LOSS) {
-        const T cE = seeded ? (T)1 : (a.cE_per_atom ? a.cE[row] : a.cE[b]);
-        // linearMtpLoss.h:417-434; the reference's network backward has no such term (Bm stays zero)
-        if (!no_tan && (a.H == 0 || a.nn_exact)) sweep_reverse<T, true, NT>(p, M, Bm, A, Tg, lane);
-        // the last pass needs the adjoints of the basic moments while the table is back in its region
-        scatter_polys<T, NT>(p, Ab, A, lane);
-        scatter_polys<T, NT>(p, Bb, Bm, lane);
-        T* grow = a.gpart + row * a.ngrad;
-        for (int q = lane; q < a.ngrad; q += NT) grow[q] = (T)0;
-        __syncthreads();         // other threads overwrite some of these entries below
-        // everything but the coefficient block is written now: the pass over the neighbours below does
-        // not read the moments or their tangents, and the group sums may take their place
-        if (a.H > 0) {
-            // compact row of the centre species: coefficient block | w0[H, S] | w1[H] | bias
-            const int S = p.n_scalar, H = a.H, nblk = a.ntypes * nmus * K;
-            const T* qv = nnb;
-            const T* n_th = nnb + S + H;
-            const T* n_d1 = n_th + H;
-            const T* n_d2 = n_d1 + H;
-            const T* n_tau = n_d2 + H;
-            const T* w1 = a.w1 + (size_t)ti * H;
-            const T* w0 = a.w0 + (size_t)ti * H * S;
-            for (int q = lane; q < H * S; q += NT) {
-                const int n = q / S, k = q - n * S;
-                const T tk = Tg[p.mapping[k]] / a.q_scaler[k];
-                if (a.nn_exact)
-                    grow[nblk + q] = w1[n] * ((cE * n_d1[n] + n_d2[n] * n_tau[n]) * qv[k] + n_d1[n] * tk);
-                else        // nnMtpLoss.h:560-585: only the k' = k term of tau
-                    grow[nblk + q] = w1[n] * (cE * n_d1[n] * qv[k] + tk * (n_d1[n] + n_d2[n] * w0[q] * qv[k]));
-            }
-            for (int n = lane; n < H; n += NT) grow[nblk + H * S + n] = cE * n_th[n] + n_d1[n] * n_tau[n];
-            if (lane == 0) grow[nblk + H * S + H] = cE;
-        } else if (!seeded) {
-            // linear coefficients and bias: linearMtpLoss.h:539-554
-            for (int s = lane; s < p.n_scalar; s += NT)
-                grow[ncoef + s] = (cE * M[p.mapping[s]] + Tg[p.mapping[s]]) / a.q_scaler[s];
-            if (lane == 0) grow[ncoef + p.n_scalar + ti] = cE;
+        T cE;
+        {
+            MTP_PHASE;
+            cE = seeded ? (T)1 : (a.cE_per_atom ? a.cE[row] : a.cE[b]);
+            // linearMtpLoss.h:417-434; the reference's network backward has no such term (Bm stays zero)
+            if (!no_tan && (a.H == 0 || a.nn_exact)) sweep_reverse<T, true>(p.rev[NT / 256], M, Bm, A, Tg, lane);
         }
-        T* Pm = pq;
-        T* Qm = pq + MTP_NC * nmus;
-        int* tjs = (int*)(pq + 2 * MTP_NC * nmus);
-        T* gacc = pq + 2 * MTP_NC * nmus + MTP_NC;          // [ntypes][nmus][K] for this centre type
-        for (int q = lane; q < a.ntypes * nmus * K; q += NT) gacc[q] = (T)0;
-        const int nchunks = (nn + MTP_NC - 1) / MTP_NC;
-        const int csize = nchunks > 0 ? (nn + nchunks - 1) / nchunks : 1;
+        {
+            MTP_PHASE;
+            // the last pass needs the adjoints of the basic moments while the table is back in its region
+            scatter_polys<T, NT>(p, L.Ab, A, lane);
+            scatter_polys<T, NT>(p, L.Bb, Bm, lane);
+            const int ncoef = a.ntypes * a.ntypes * nmus * K;
+            T* grow = a.gpart + row * a.ngrad;
+            for (int q = lane; q < a.ngrad; q += NT) grow[q] = (T)0;
+            __syncthreads();         // other threads overwrite some of these entries below
+            // everything but the coefficient block is written now: the pass over the neighbours below does
+            // not read the moments or their tangents, and the group sums may take their place
+            if (a.H > 0) {
+                // compact row of the centre species: coefficient block | w0[H, S] | w1[H] | bias
+                const int S = p.n_scalar, H = a.H, nblk = a.ntypes * nmus * K;
+                const T* qv = L.net;
+                const T* n_th = qv + S + H;
+                const T* n_d1 = n_th + H;
+                const T* n_d2 = n_d1 + H;
+                const T* n_tau = n_d2 + H;
+                const T* w1 = a.w1 + (size_t)ti * H;
+                const T* w0 = a.w0 + (size_t)ti * H * S;
+                for (int q = lane; q < H * S; q += NT) {
+                    const int n = q / S, k = q - n * S;
+                    const T tk = Tg[p.mapping[k]] / a.q_scaler[k];
+                    if (a.nn_exact)
+                        grow[nblk + q] = w1[n] * ((cE * n_d1[n] + n_d2[n] * n_tau[n]) * qv[k] + n_d1[n] * tk);
+                    else        // nnMtpLoss.h:560-585: only the k' = k term of tau
+                        grow[nblk + q] = w1[n] * (cE * n_d1[n] * qv[k] + tk * (n_d1[n] + n_d2[n] * w0[q] * qv[k]));
+                }
+                for (int n = lane; n < H; n += NT) grow[nblk + H * S + n] = cE * n_th[n] + n_d1[n] * n_tau[n];
+                if (lane == 0) grow[nblk + H * S + H] = cE;
+            } else if (!seeded) {
+                // linear coefficients and bias: linearMtpLoss.h:539-554
+                for (int s = lane; s < p.n_scalar; s += NT)
+                    grow[ncoef + s] = (cE * M[p.mapping[s]] + Tg[p.mapping[s]]) / a.q_scaler[s];
+                if (lane == 0) grow[ncoef + p.n_scalar + ti] = cE;
+            }
+            T* gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;          // [ntypes][nmus][K] for this centre type
+            for (int q = lane; q < a.ntypes * nmus * K; q += NT) gacc[q] = (T)0;
+        }
         for (int c0 = 0; c0 < nn; c0 += csize) {
             // equal chunks and as many thread groups per chunk as fit, as in the pair-derivative pass
             const int nc = min(csize, nn - c0);
-            const int ng = min(NT / nc, MTP_NGMAX);
-            const int h = lane / nc, j = lane - h * nc;
+            const int ng = min(small_div(NT, nc), MTP_NGMAX);
+            const int h = small_div(lane, nc), j = lane - h * nc;
             int nj; bool valid; T d[3];
             __syncthreads();
-            build_table<T, TAB_GRADIENT, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
-            __syncthreads();
-            // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  The groups take the polynomials in
-            // turn, on from one mu to the next.  (All of a thread's sums kept to the end, with one round of group sums: 100
-            // registers instead of 70, so five wavefronts per SIMD instead of six, and the kernel 263 -> 320 us.)
-            int s = h < ng ? h : p.npoly;
-            for (int mu = 0; mu < nmus; mu++) {
-                T Pv, Qv;
-                loss_walk<T>(tab + j * E, Ab, Bb, rws, s, rws[p.npoly + mu + 1], ng, OX, OY, OZ, OU, OW, cE, no_tan, Pv, Qv);
-                {
-                    T* gr = gred + lane * 2;
-                    gr[0] = Pv; gr[1] = Qv;
-                }
-                __syncthreads();
-                if (h == 0) {
-                    for (int hh = 1; hh < ng; hh++) {
-                        const T* gr = gred + (hh * nc + j) * 2;
-                        Pv += gr[0]; Qv += gr[1];
-                    }
-                    Pm[j * nmus + mu] = Pv; Qm[j * nmus + mu] = Qv;
-                }
+            {
+                MTP_PHASE;
+                build_table<T, TAB_GRADIENT, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
                 __syncthreads();
             }
+            {
+                MTP_PHASE;
+                // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  The groups take the polynomials in
+                // turn, on from one mu to the next.  (All of a thread's sums kept to the end, with one round of group sums:
+                // 100 registers instead of 70, so five wavefronts per SIMD instead of six, and the kernel 263 -> 320 us.)
+                T* const Pm = L.pq;
+                T* const Qm = L.pq + MTP_NC * nmus;
+                int s = h < ng ? h : p.npoly;
+                for (int mu = 0; mu < nmus; mu++) {
+                    T Pv, Qv;
+                    loss_walk<T>(tab + j * E, L.Ab, L.Bb, L.rws, s, L.rws[p.npoly + mu + 1], ng, OX, OY, OZ, OW, cE, no_tan, Pv, Qv);
+                    {
+                        T* gr = L.gred + lane * 2;
+                        gr[0] = Pv; gr[1] = Qv;
+                    }
+                    __syncthreads();
+                    if (h == 0) {
+                        for (int hh = 1; hh < ng; hh++) {
+                            const T* gr = L.gred + (hh * nc + j) * 2;
+                            Pv += gr[0]; Qv += gr[1];
+                        }
+                        Pm[j * nmus + mu] = Pv; Qm[j * nmus + mu] = Qv;
+                    }
+                    __syncthreads();
+                }
+            }
+            MTP_PHASE;
+            const T* const Pm = L.pq;
+            const T* const Qm = L.pq + MTP_NC * nmus;
+            int* const tjs = (int*)(L.pq + 2 * MTP_NC * nmus);
+            T* const gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;
             // tj of each neighbour of the chunk, for the accumulation below
             if (h == 0) tjs[j] = valid ? types[nj] : -1;
             __syncthreads();
             // lanes <- (mu, k): sequential over neighbours keeps the sum order fixed
             for (int q = lane; q < nmus * K; q += NT) {
-                const int mu = q / K, k = q - mu * K;
+                const int mu = small_div(q, K), k = q - mu * K;
                 for (int jn = 0; jn < nc; jn++) {
                     const int tj = tjs[jn];
                     if (tj < 0) continue;
@@ -860,14 +1093,13 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : 1)) mtp_ato
             }
         }
         __syncthreads();
-        if (a.H > 0) {
-            for (int q = lane; q < a.ntypes * nmus * K; q += NT) grow[q] = gacc[q];
-            return;
-        }
-        for (int q = lane; q < a.ntypes * nmus * K; q += NT)
-            grow[(size_t)ti * a.ntypes * nmus * K + q] = gacc[q];
+        MTP_PHASE;
+        const T* const gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;
+        T* const grow = a.gpart + row * a.ngrad + (a.H > 0 ? 0 : (size_t)ti * a.ntypes * nmus * K);
+        for (int q = lane; q < a.ntypes * nmus * K; q += NT) grow[q] = gacc[q];
     }
 }
+#undef MTP_PHASE
 
 // out[b, q] = sum over atoms ii < binum[b] of gpart[b, ii, q], in atom order
 template <typename T>
@@ -1048,18 +1280,13 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
         }
         __syncthreads();
     }
-    sweep_forward<T, false, NT>(p, M, (T*)nullptr, lane);
+    sweep_forward<T, false>(p.fwd[NT / 256], M, (T*)nullptr, lane);
     for (int s = lane; s < S; s += NT) {
         c.desc[row * S + s] = M[p.mapping[s]];
         if (p.x_root[s] >= 0) X[p.x_root[s]] = (T)1 / a.q_scaler[s];       // (the columns of this launch)
     }
     __syncthreads();
-    {
-        MtpPlanDevice px = p;              // the reverse gather over the nodes
-        px.r_level = p.x_level; px.r_multi = p.x_multi; px.r_src = p.x_src; px.r_rem = p.x_rem;
-        px.r_gbase = p.x_gbase; px.r_gdepth = p.x_gdepth; px.r_terms = p.x_terms;
-        sweep_reverse<T, false, NT>(px, M, X, (const T*)nullptr, (const T*)nullptr, lane);
-    }
+    sweep_reverse<T, false>(p.x, M, X, (const T*)nullptr, (const T*)nullptr, lane);
 
     // Pair derivatives, four or eight neighbours at a time.  A wavefront forms, for one of them and every basic moment, the vector
     //   D_b = d(g_mu x^a y^b z^c)/dr_j = m (g' - k g / r) u + g / r grad_u m
@@ -1525,16 +1752,15 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     A2P_REQUIRE(n_moms < 8192, A2P_ERR_INVALID, "mtp plan: more than 8191 moments");    // 16-bit byte offsets
     // Interleaved gather lists (see mtp_plan.h).  `lists[m]` holds the packed terms of moment m.
     struct Ell {
-        std::vector<int> level, lend, multi, slot, lead, gbase, gdepth;   // multi: doubling steps; lead: pieces behind
+        std::vector<int> level, slot, lead;                // lead: pieces behind
+        std::vector<int4> group;                           // first term, depth, doubling steps
         std::vector<int2> terms;
-        int max_slots = 0;
         bool too_long = false;
     };
     auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level) {
         Ell e;
         for (const auto& members : by_level) {
-            const int first_slot = (int)e.slot.size();
-            e.level.push_back(first_slot);
+            e.level.push_back((int)e.slot.size());
             std::vector<int> ms = members;
             std::stable_sort(ms.begin(), ms.end(),
                              [&](int x, int y) { return lists[x].size() > lists[y].size(); });
@@ -1542,18 +1768,17 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             // adjacent and stay inside one group of 64 slots (one wavefront adds them up with shuffles)
             struct Piece { int m, t0, n, rem; };
             std::vector<Piece> pieces;
-            int most = 1;
             for (int m : ms) {
                 const int n = (int)lists[m].size();
                 const int np = (n + MTP_SLOT_CAP - 1) / MTP_SLOT_CAP;
                 if (np > 64) { e.too_long = true; continue; }
-                most = std::max(most, np);
+                if ((int)(pieces.size() % 16) + np > 16)                  // a row of sixteen lanes, or from its beginning on
+                    while (pieces.size() % 16) pieces.push_back({-1, 0, 0, 0});
                 if ((int)(pieces.size() % 64) + np > 64)
                     while (pieces.size() % 64) pieces.push_back({-1, 0, 0, 0});
                 for (int q = 0; q < np; q++)
                     pieces.push_back({m, q * MTP_SLOT_CAP, std::min(MTP_SLOT_CAP, n - q * MTP_SLOT_CAP), np - 1 - q});
             }
-            (void)most;
             for (size_t g0 = 0; g0 < pieces.size(); g0 += 64) {
                 const size_t g1 = std::min(pieces.size(), g0 + 64);
                 int depth = 0, longest = 1;
@@ -1563,29 +1788,58 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 }
                 int steps = 0;                      // doubling steps that add up the pieces of this group's lists
                 while ((1 << steps) < longest) steps++;
-                e.multi.push_back(steps);
                 depth = (depth + MTP_DEPTH_STEP - 1) / MTP_DEPTH_STEP * MTP_DEPTH_STEP;    // the sweeps fetch that many terms at a time
-                e.gbase.push_back((int)e.terms.size());
-                e.gdepth.push_back(depth);
+                e.group.push_back(make_int4((int)e.terms.size(), depth, steps, 0));
                 e.terms.resize(e.terms.size() + (size_t)depth * 64, make_int2(0, 0));
                 for (size_t q = g0; q < g1; q++) {
                     const Piece& pc = pieces[q];
                     for (int k = 0; k < pc.n; k++)
-                        e.terms[e.gbase.back() + (size_t)k * 64 + (q - g0)] = lists[pc.m][pc.t0 + k];
-                    e.slot.push_back(pc.t0 == 0 ? pc.m : -1);      // the first piece of a list names the moment
+                        e.terms[e.group.back().x + (size_t)k * 64 + (q - g0)] = lists[pc.m][pc.t0 + k];
+                    e.slot.push_back(pc.n > 0 && pc.t0 == 0 ? pc.m : -1);      // the first piece of a list names the moment
                     e.lead.push_back(pc.rem);
                 }
             }
-            e.lend.push_back((int)e.slot.size());
-            e.max_slots = std::max(e.max_slots, (int)e.slot.size() - first_slot);
             while (e.slot.size() % 64) { e.slot.push_back(-1); e.lead.push_back(0); }
         }
         e.level.push_back((int)e.slot.size());
-        e.lend.push_back((int)e.slot.size());
-        if (e.terms.empty()) e.terms.push_back(make_int2(0, 0));
-        if (e.gbase.empty()) { e.gbase.push_back(0); e.gdepth.push_back(0); e.multi.push_back(0); }
-        if (e.slot.empty()) { e.slot.push_back(-1); e.lead.push_back(0); }
         return e;
+    };
+    struct Stream {
+        std::vector<int4> head;
+        std::vector<int> ctrl, slots;
+        std::vector<int2> words;
+    };
+    auto build_stream = [](const Ell& e, bool up, int waves) {
+        Stream st;
+        const int levels = (int)e.level.size() - 1;
+        std::vector<std::vector<std::pair<int, int>>> seq(waves);        // (step of the level order, group) of each wavefront
+        for (int q = 0; q < levels; q++) {
+            const int l = up ? q : levels - 1 - q;
+            std::vector<int> load(waves, 0);
+            for (int g = e.level[l] / 64; g < e.level[l + 1] / 64; g++) {
+                const int w = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+                load[w] += e.group[g].y + 4;
+                seq[w].push_back({q, g});
+            }
+        }
+        for (int w = 0; w < waves; w++) {
+            const int first = (int)st.ctrl.size(), row = (int)st.slots.size() / 64;
+            for (size_t i = 0; i < seq[w].size(); i++) {
+                const int q = seq[w][i].first, g = seq[w][i].second;
+                const int barriers = (i + 1 < seq[w].size() ? seq[w][i + 1].first : levels) - q;
+                const int4 info = e.group[g];
+                st.words.insert(st.words.end(), e.terms.begin() + info.x, e.terms.begin() + info.x + (size_t)info.y * 64);
+                for (int k = MTP_DEPTH_STEP; k < info.y; k += MTP_DEPTH_STEP) st.ctrl.push_back(0);
+                st.ctrl.push_back(1 | info.z << 1 | barriers << 4);
+                for (int q64 = 0; q64 < 64; q64++)
+                    st.slots.push_back((e.slot[g * 64 + q64] + 1) | e.lead[g * 64 + q64] << 16);
+            }
+            st.head.push_back(make_int4(first, (int)st.ctrl.size() - first, row, seq[w].empty() ? levels : seq[w][0].first));
+        }
+        st.words.resize(st.words.size() + 2 * MTP_DEPTH_STEP * 64, make_int2(0, 0));     // requested ahead
+        st.ctrl.resize(st.ctrl.size() + 2, 0);
+        st.slots.resize(st.slots.size() + 2 * 64, 0);
+        return st;
     };
     // forward: terms per destination in file order; level l >= 1 at index l - 1
     std::vector<std::vector<int2>> fl(n_moms), rl(n_moms);
@@ -1647,6 +1901,16 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         }
         polys_end[m + 1] = (int)polys_mu.size();
     }
+    std::vector<unsigned> polys_len;                              // longest first, for the sums of the basic moments
+    bool polys_fit = nmus <= 8 && n_poly_coef < (1 << 13);
+    for (size_t r = 0; r < row_ab.size(); r++)
+        for (int q = rows[r] >> 16; q < rows[r + 1] >> 16; q++) {
+            const int mu = polys[q] & 15, len = (polys[q] >> 4) & 255, beg = polys[q] >> 12;
+            polys_fit = polys_fit && len <= MTP_POLY_MAX && row_ab[r].first < 32 && row_ab[r].second < 32;
+            polys_len.push_back((unsigned)mu | (unsigned)row_ab[r].first << 3 | (unsigned)row_ab[r].second << 8 |
+                                (unsigned)len << 13 | (unsigned)beg << 19);
+        }
+    std::stable_sort(polys_len.begin(), polys_len.end(), [](unsigned x, unsigned y) { return (x >> 13 & 63) > (y >> 13 & 63); });
     std::vector<std::vector<int>> poly_lists(n_poly_coef);
     std::vector<int> poly_src(n_poly_coef), poly_items_off((size_t)n_poly_coef + 1, 0), poly_items, poly_pos(n_basic);
     int poly_unique = 1;
@@ -1668,7 +1932,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     // adjoints fit MTP_NODE_CAP entries of LDS
     struct XHost {
         std::vector<int> root, seed, brem, bsteps, bbase, bdepth, bwords;
-        Ell ell;
+        Stream stream;
         int nodes = 0;
     };
     std::vector<XHost> xhosts;
@@ -1729,8 +1993,9 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 for (int m : anc) node_of[m] = -1;
             }
             if (xl.empty()) xl.emplace_back();
-            h.ell = build_ell(xl, x_by);
-            A2P_REQUIRE(!h.ell.too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
+            const Ell ell = build_ell(xl, x_by);
+            h.stream = build_stream(ell, false, 4);
+            A2P_REQUIRE(!ell.too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
                         64 * MTP_SLOT_CAP);
             std::vector<int> by_len = seeds;
             std::stable_sort(by_len.begin(), by_len.end(),
@@ -1740,6 +2005,8 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             for (int s : by_len) {
                 const int len = (int)seed_basic[s].size();
                 const int np = std::max(1, (len + MTP_SLOT_CAP - 1) / MTP_SLOT_CAP);      // <= 64: n_basic < 64 * cap
+                if ((int)(pieces.size() % 16) + np > 16)                                  // as in the gathers (piece_sum)
+                    while (pieces.size() % 16) pieces.push_back({-1, 0, 0, 0});
                 if ((int)(pieces.size() % 64) + np > 64)
                     while (pieces.size() % 64) pieces.push_back({-1, 0, 0, 0});
                 for (int q = 0; q < np; q++)
@@ -1793,22 +2060,19 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                          ((unsigned)basic[i * 4 + 3] << 24);
     const size_t o_basic = add(basic_words.data(), sizeof(unsigned) * n_basic);
     const size_t o_map = add(mapping, sizeof(int) * n_scalar);
-    const size_t o_fl = add(F.level.data(), sizeof(int) * F.level.size());
-    const size_t o_fe = add(F.lend.data(), sizeof(int) * F.lend.size());
-    const size_t o_fx = add(F.multi.data(), sizeof(int) * F.multi.size());
-    const size_t o_fd = add(F.slot.data(), sizeof(int) * F.slot.size());
-    const size_t o_fc = add(F.lead.data(), sizeof(int) * F.lead.size());
-    const size_t o_fg = add(F.gbase.data(), sizeof(int) * F.gbase.size());
-    const size_t o_fh = add(F.gdepth.data(), sizeof(int) * F.gdepth.size());
-    const size_t o_ft = add(F.terms.data(), sizeof(int2) * F.terms.size());
-    const size_t o_rl = add(R.level.data(), sizeof(int) * R.level.size());
-    const size_t o_re = add(R.lend.data(), sizeof(int) * R.lend.size());
-    const size_t o_rx = add(R.multi.data(), sizeof(int) * R.multi.size());
-    const size_t o_rs = add(R.slot.data(), sizeof(int) * R.slot.size());
-    const size_t o_rc = add(R.lead.data(), sizeof(int) * R.lead.size());
-    const size_t o_rg = add(R.gbase.data(), sizeof(int) * R.gbase.size());
-    const size_t o_rh = add(R.gdepth.data(), sizeof(int) * R.gdepth.size());
-    const size_t o_rt = add(R.terms.data(), sizeof(int2) * R.terms.size());
+    struct StreamOff { size_t head, ctrl, slots, words; };
+    auto add_stream = [&](const Stream& st) {
+        return StreamOff{add(st.head.data(), sizeof(int4) * st.head.size()), add(st.ctrl.data(), sizeof(int) * st.ctrl.size()),
+                         add(st.slots.data(), sizeof(int) * st.slots.size()), add(st.words.data(), sizeof(int2) * st.words.size())};
+    };
+    Stream fs[2], rs[2];
+    StreamOff o_f[2], o_r[2];
+    for (int i = 0; i < 2; i++) {
+        fs[i] = build_stream(F, true, i ? 4 : 1);
+        rs[i] = build_stream(R, false, i ? 4 : 1);
+        o_f[i] = add_stream(fs[i]);
+        o_r[i] = add_stream(rs[i]);
+    }
     const size_t o_rows = add(rows.data(), sizeof(int) * rows.size());
     const size_t o_poly = add(polys.data(), sizeof(int) * polys.size());
     const size_t o_pmu = add(polys_mu.data(), sizeof(int) * polys_mu.size());
@@ -1817,19 +2081,14 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const size_t o_poff = add(poly_items_off.data(), sizeof(int) * poly_items_off.size());
     const size_t o_pit = add(poly_items.data(), sizeof(int) * poly_items.size());
     const size_t o_ppos = add(poly_pos.data(), sizeof(int) * poly_pos.size());
-    struct XOff { size_t root, seed, level, multi, src, rem, gbase, gdepth, terms, bbase, bdepth, bsteps, brem, bwords; };
+    const size_t o_plen = add(polys_len.data(), sizeof(unsigned) * polys_len.size());
+    struct XOff { size_t root, seed, bbase, bdepth, bsteps, brem, bwords; StreamOff x; };
     std::vector<XOff> xoffs;
     for (const XHost& h : xhosts) {
         XOff o;
         o.root = add(h.root.data(), sizeof(int) * h.root.size());
         o.seed = add(h.seed.data(), sizeof(int) * h.seed.size());
-        o.level = add(h.ell.level.data(), sizeof(int) * h.ell.level.size());
-        o.multi = add(h.ell.multi.data(), sizeof(int) * h.ell.multi.size());
-        o.src = add(h.ell.slot.data(), sizeof(int) * h.ell.slot.size());
-        o.rem = add(h.ell.lead.data(), sizeof(int) * h.ell.lead.size());
-        o.gbase = add(h.ell.gbase.data(), sizeof(int) * h.ell.gbase.size());
-        o.gdepth = add(h.ell.gdepth.data(), sizeof(int) * h.ell.gdepth.size());
-        o.terms = add(h.ell.terms.data(), sizeof(int2) * h.ell.terms.size());
+        o.x = add_stream(h.stream);
         o.bbase = add(h.bbase.data(), sizeof(int) * h.bbase.size());
         o.bdepth = add(h.bdepth.data(), sizeof(int) * h.bdepth.size());
         o.bsteps = add(h.bsteps.data(), sizeof(int) * h.bsteps.size());
@@ -1850,22 +2109,18 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.nmus = nmus; d.kmax = kmax; d.n_levels = n_levels;
     d.basic = (const unsigned*)(base + o_basic);
     d.mapping = (const int*)(base + o_map);
-    d.f_level = (const int*)(base + o_fl); d.f_lend = (const int*)(base + o_fe);
-    d.f_multi = (const int*)(base + o_fx);
-    d.f_dst = (const int*)(base + o_fd); d.f_rem = (const int*)(base + o_fc);
-    d.f_gbase = (const int*)(base + o_fg); d.f_gdepth = (const int*)(base + o_fh);
-    d.f_terms = (const int2*)(base + o_ft);
-    d.r_level = (const int*)(base + o_rl); d.r_lend = (const int*)(base + o_re);
-    d.r_multi = (const int*)(base + o_rx);
-    d.r_src = (const int*)(base + o_rs); d.r_rem = (const int*)(base + o_rc);
-    d.r_gbase = (const int*)(base + o_rg); d.r_gdepth = (const int*)(base + o_rh);
-    d.r_terms = (const int2*)(base + o_rt);
+    auto stream_at = [&](const StreamOff& o) {
+        return MtpStream{(const int4*)(base + o.head), (const int*)(base + o.ctrl), (const int*)(base + o.slots), (const int2*)(base + o.words)};
+    };
+    for (int i = 0; i < 2; i++) { d.fwd[i] = stream_at(o_f[i]); d.rev[i] = stream_at(o_r[i]); }
+    d.x = MtpStream{nullptr, nullptr, nullptr, nullptr};
     d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
     d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
     d.rows = (const int*)(base + o_rows); d.polys = (const int*)(base + o_poly);
     d.polys_mu = (const int*)(base + o_pmu); d.polys_end = (const int*)(base + o_pend);
     d.poly_src = (const int*)(base + o_psrc); d.poly_off = (const int*)(base + o_poff);
     d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
+    d.polys_len = polys_fit ? (const unsigned*)(base + o_plen) : nullptr;
     d.poly_unique = poly_unique;
     d.x_nodes = 0; d.x_slots = 0;                // set per batch by the components call (MtpPlan::xbatches)
     for (size_t i = 0; i < xhosts.size(); i++) {
@@ -1873,10 +2128,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         MtpXBatch xb;
         xb.nodes = xhosts[i].nodes; xb.slots = (int)xhosts[i].seed.size();
         xb.root = (const int*)(base + o.root); xb.seed = (const int*)(base + o.seed);
-        xb.level = (const int*)(base + o.level); xb.multi = (const int*)(base + o.multi);
-        xb.src = (const int*)(base + o.src); xb.rem = (const int*)(base + o.rem);
-        xb.gbase = (const int*)(base + o.gbase); xb.gdepth = (const int*)(base + o.gdepth);
-        xb.terms = (const int2*)(base + o.terms);
+        xb.x = stream_at(o.x);
         xb.bbase = (const int*)(base + o.bbase); xb.bdepth = (const int*)(base + o.bdepth);
         xb.bsteps = (const int*)(base + o.bsteps); xb.brem = (const int*)(base + o.brem);
         xb.bwords = (const int*)(base + o.bwords);
@@ -1949,6 +2201,8 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0;
     a.nn_exact = 1;
     a.row_seed = nullptr; a.pair_out = nullptr;
+    a.OY = a.p.kmax + 1; a.OZ = 2 * a.OY; a.OG = 3 * a.OY; a.ODG = a.OG + nmus; a.OU = a.ODG + nmus; a.OW = a.OU + 4;
+    a.OF = a.OW + 4; a.ODF = a.OF + K;
     a.H = 0; a.w0 = nullptr; a.w1 = nullptr; a.q_shift = nullptr;
     void* ws = nullptr;
     int rc = ws_get(WS_FLAGS, 64, &ws);
@@ -2018,8 +2272,35 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
             }
         const_cast<MtpArgs<T>&>(a).keep_table = keep;
     }
-    const_cast<MtpArgs<T>&>(a).lds_basic_off = (int)lds_main;
-    const_cast<MtpArgs<T>&>(a).nc_cap = nc_cap;
+    {
+        MtpArgs<T>& w = const_cast<MtpArgs<T>&>(a);
+        const MtpPlanDevice& p = a.p;
+        const int nt = wide ? 256 : 64;
+        const bool keep = !LOSS && w.keep_table != 0;
+        w.lds_basic_off = (int)lds_main;
+        w.nc_cap = nc_cap;
+        // moments | (loss mode: their tangents) | coefficients | region of the neighbour table | ...
+        w.at_Tg = p.n_moms;
+        w.at_cf = w.at_Tg + (LOSS ? p.n_moms : 0);
+        w.at_tab = w.at_cf + a.ntypes * p.nmus * a.K;
+        // the adjoints share the table's region, behind the sweeps' partial sums, or lie behind the table
+        w.at_A = w.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt)
+                                  : mtp_adjoint_offset((LOSS ? 2 : 1) * p.max_level_slots));
+        w.at_Bm = w.at_A + p.n_moms;
+        // Partial sums of the thread groups, needed only in the last pass over the neighbours, when the moments (and, in
+        // loss mode, their tangents) are dead: a long enough moment vector lends them its place.  Energy / force / virial
+        // kernel: they are written over the table once it has been read.
+        w.at_gred = !LOSS ? w.at_tab : mtp_gred_in_moments(LOSS, p.n_moms) ? 0 : w.at_tab + nc_cap * a.E;
+        w.at_Ab = w.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, p.max_level_slots, nt, keep);
+        w.at_Bb = w.at_Ab + p.ncoef_poly;
+        w.at_pq = LOSS ? w.at_Bb + p.ncoef_poly : w.at_Ab;
+        w.at_net = w.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);
+        w.at_polys = mtp_polys_in_moments(p.ncoef_poly, p.n_moms) ? 0 : w.at_pq + (a.H > 0 ? p.n_scalar + a.H : 0);
+    }
+    // as many groups of a thread per polynomial as the workgroup has, and as the place of their sums holds
+    const int room = !LOSS && a.keep_table ? a.p.n_moms : mtp_table_entries(nc_cap, a.E, LOSS, a.p.n_moms, wide ? 256 : 64);
+    const_cast<MtpArgs<T>&>(a).mom_groups =
+        a.p.polys_len ? std::min((wide ? 256 : 64) / std::max(a.p.npoly, 1), room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1)) : 0;
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
     auto kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
@@ -2439,8 +2720,7 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         for (const MtpXBatch& xb : plan->xbatches) {
             MtpPlanDevice& p = a.p;
             p.x_nodes = xb.nodes; p.x_slots = xb.slots; p.x_root = xb.root; p.x_seed = xb.seed;
-            p.x_level = xb.level; p.x_multi = xb.multi; p.x_src = xb.src; p.x_rem = xb.rem;
-            p.x_gbase = xb.gbase; p.x_gdepth = xb.gdepth; p.x_terms = xb.terms;
+            p.x = xb.x;
             p.x_bbase = xb.bbase; p.x_bdepth = xb.bdepth; p.x_bsteps = xb.bsteps; p.x_brem = xb.brem; p.x_bwords = xb.bwords;
             // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 256
             // values each); then the packed basic moments.  With at most four groups of pieces the adjoints are in registers

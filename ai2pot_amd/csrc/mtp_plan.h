@@ -19,8 +19,25 @@
 namespace a2p {
 
 constexpr int MTP_SLOT_CAP = 16;
-// The sweeps fetch the words of a slot MTP_DEPTH_STEP at a time; the depth of a group of slots is a multiple of it.
-constexpr int MTP_DEPTH_STEP = 2;
+// Terms of a slot to a step of the sweeps.
+constexpr int MTP_DEPTH_STEP = 4;
+
+// A gather as the wavefronts of a workgroup walk it.  `lists[m]` holds the terms of moment m.  A slot holds up to
+// MTP_SLOT_CAP of them; a longer list is cut into consecutive slots (pieces), so that no lane walks a long list alone.  Slots
+// are grouped 64 at a time, one to a lane; the pieces of a list lie in one group, a list of up to sixteen within a row of
+// sixteen lanes and a longer one from the beginning of a row on, and the wavefront adds their sums (four doubling steps
+// within a row, two across).  Lists are sorted by length, so only a level's first groups hold cut ones.  The words of a
+// group are padded with zero terms to its depth (a multiple of MTP_DEPTH_STEP); a word packs x = 8 m0 | 8 m1 << 16 (byte
+// offsets into an array of doubles), y = multiplicity.
+// The groups of a level are dealt to the wavefronts, the deepest first and to the one with the least to do, and everything a
+// wavefront needs lies in the order in which it needs it: MTP_DEPTH_STEP x 64 words to a step, a control word for each step,
+// and a row of 64 slot words for each group.
+struct MtpStream {
+    const int4* head;          // [wavefronts] first step, steps, first row of slots, barriers before the first step
+    const int* ctrl;           // 0, or behind the last step of a group: 1 | doubling steps << 1 | barriers to pass << 4
+    const int* slots;          // moment + 1 in the first piece of a list (0 elsewhere) | pieces of the list behind this one << 16
+    const int2* words;
+};
 
 struct MtpPlanDevice {
     // sizes
@@ -29,33 +46,9 @@ struct MtpPlanDevice {
     // device arrays
     const unsigned* basic;     // [n_basic]    mu | a << 8 | b << 16 | c << 24
     const int* mapping;        // [n_scalar]
-    // forward gather.  A slot holds up to MTP_SLOT_CAP terms of one destination moment; a longer
-    // list is cut into consecutive slots (pieces), so that no lane walks a long list alone; the pieces of a
-    // list lie in one group of 64 slots and the wavefront that walks the group adds their partial sums with
-    // shuffles (f_multi[group] doubling steps: lists are sorted by length, so only a level's first groups hold cut lists).  Slots are grouped 64 at a time; level l covers slots
-    // [f_level[l], f_level[l+1]) (whole groups; [f_level[l], f_lend[l]) without the padding slots).  The terms of a group are stored
-    // interleaved and padded with zero terms to the group's depth (a multiple of MTP_DEPTH_STEP): term k of slot s is
-    // f_terms[f_gbase[s >> 6] + k * 64 + (s & 63)], k < f_gdepth[s >> 6], so the 64 lanes that walk
-    // a group read consecutive words and share the trip count.  A term packs x = 8 m0 | 8 m1 << 16 (byte offsets
-    // into an array of doubles), y = multiplicity.
-    const int* f_level;        // [n_levels+1]
-    const int* f_lend;         // [n_levels+1]
-    const int* f_multi;        // [n_fslots/64] doubling steps that add up the pieces of the group's longest list (0: none is cut)
-    const int* f_dst;          // [n_fslots]   destination in the first piece of a list (-1 elsewhere and in padding)
-    const int* f_rem;          // [n_fslots]   pieces of the same list behind this one
-    const int* f_gbase;        // [n_fslots/64]
-    const int* f_gdepth;       // [n_fslots/64]
-    const int2* f_terms;
-    // reverse gather, same layout: sources by level (index l = level of the SOURCE moment),
-    // processed from the last level to level 0; a term packs x = 8 dst | 8 other << 16, y = mult
-    const int* r_level;        // [n_levels+1]
-    const int* r_lend;         // [n_levels+1]
-    const int* r_multi;        // [n_rslots/64]
-    const int* r_src;          // [n_rslots]
-    const int* r_rem;          // [n_rslots]
-    const int* r_gbase;        // [n_rslots/64]
-    const int* r_gdepth;       // [n_rslots/64]
-    const int2* r_terms;
+    // forward gather (terms of a product: its factors) and reverse gather (terms of a factor: x = 8 dst | 8 other << 16;
+    // sources by level, from the last level to level 0), for workgroups of one wavefront and of four
+    MtpStream fwd[2], rev[2];
     int max_level_slots;       // most slots of any level (forward or reverse)
     // Polynomials of the passes that own a neighbour per lane.  The basic moments (mu, a, b, c) with the same row (a, b) and
     // the same mu are the coefficients of a polynomial in z; its coefficients lie together, highest power first, up to
@@ -66,6 +59,8 @@ struct MtpPlanDevice {
     const int* polys_mu;       // [npoly] the same by mu: a | b << 5 | length << 10 | first coefficient << 15
     const int* polys_end;      // [nmus + 1] run of each mu in polys_mu
     const int* poly_pos;       // [n_basic] coefficient of each basic moment
+    const unsigned* polys_len; // [npoly] the same, longest first: mu | a << 3 | b << 8 | length << 13 | first coefficient << 19
+                               // (null: one of them does not fit its field)
     int poly_unique;           // no two basic moments share a coefficient (the usual case: a plain scatter fills them)
     const int* poly_src;       // [ncoef_poly] basic moment behind the coefficient, -1 none, -2 several (poly_off / items)
     const int* poly_off;       // [ncoef_poly+1]
@@ -73,10 +68,10 @@ struct MtpPlanDevice {
     // The one-hot adjoints of all scalar moments at once (linear-solver components).  A node (s, m) is moment m as an
     // ancestor of scalar moment s: mapping[s] itself, or a factor of a product among its ancestors.  The adjoint
     // sweeps of all read-outs e_s together are one reverse gather over the nodes, laid out like the reverse gather
-    // above (a term packs x = 8 node(dst) | 8 other << 16 with `other` a moment, y = mult; x_src names the node).
+    // above (a term packs x = 8 node(dst) | 8 other << 16 with `other` a moment, y = mult).
     // The basic ancestors of a scalar moment form a list of words node | basic << 16; lists are sorted by length, cut into
     // pieces of at most MTP_SLOT_CAP words, and dealt to slots, 64 slots a group, the pieces of a list in neighbouring
-    // slots of one group (the wavefront adds their sums with shuffles, x_bsteps doubling steps).  A group's words are
+    // slots as in the gathers (the wavefront adds their sums, x_bsteps doubling steps).  A group's words are
     // stored interleaved and padded to the group's depth with node x_nodes, whose adjoint is always zero: word k of
     // slot q is x_bwords[x_bbase[q >> 6] + k * 64 + (q & 63)].
     // The scalar moments are dealt to batches whose nodes fit the kernel's LDS budget (MtpPlan::xbatches); the fields
@@ -85,13 +80,7 @@ struct MtpPlanDevice {
     const int* x_root;         // [n_scalar] node (s, mapping[s])
     const int* x_seed;         // [x_slots]  scalar moment, in the slot of its list's first piece; -1 elsewhere
     const int* x_brem;         // [x_slots]  pieces of the same list behind this one
-    const int* x_level;        // [n_levels+1]
-    const int* x_multi;        // [n_xslots/64]
-    const int* x_src;          // [n_xslots]
-    const int* x_rem;          // [n_xslots]
-    const int* x_gbase;        // [n_xslots/64]
-    const int* x_gdepth;       // [n_xslots/64]
-    const int2* x_terms;
+    MtpStream x;               // the reverse gather over the nodes, for four wavefronts (a slot word names the node)
     const int* x_bbase;        // [x_slots/64]
     const int* x_bdepth;       // [x_slots/64]
     const int* x_bsteps;       // [x_slots/64]
@@ -101,8 +90,8 @@ struct MtpPlanDevice {
 // one batch of scalar moments of the components kernel: the x_ fields of MtpPlanDevice
 struct MtpXBatch {
     int nodes, slots;
-    const int *root, *seed, *level, *multi, *src, *rem, *gbase, *gdepth;
-    const int2* terms;
+    const int *root, *seed;
+    MtpStream x;
     const int *bbase, *bdepth, *bsteps, *brem, *bwords;
 };
 

@@ -1,5 +1,5 @@
 """The passes over the neighbours of the moment tensor potentials where their layouts can go wrong: basic moments whose
-powers of z have gaps or occur twice, and linear-solver components for one to four groups of columns and for rows with
+powers of z have gaps, occur twice or are high, or that make many polynomials, and linear-solver components for one to four groups of columns and for rows with
 few neighbours (pairs of neighbours that have no second one)."""
 import numpy as np
 import pytest
@@ -13,6 +13,9 @@ pytestmark = pytest.mark.gpu
 # (mu, a, b, c): z^0 and z^2 of a row without z^1, a row without its constant, and the same moment twice
 GAPS = [(0, 0, 0, 0), (0, 0, 0, 2), (0, 1, 0, 1), (0, 1, 1, 3), (1, 0, 0, 1), (1, 0, 2, 0)]
 TWICE = GAPS[:4] + [(0, 0, 0, 2)] + GAPS[4:] + [(1, 0, 2, 0)]
+# a polynomial in z longer than a thread's sums, and more polynomials than a wavefront has lanes
+LONG = GAPS + [(1, 0, 0, 11)]
+MANY = [(mu, a, b, 0) for mu in (0, 1) for a in range(8) for b in range(8 - a)]
 
 
 def tables(basic):
@@ -24,7 +27,7 @@ def tables(basic):
                 nmus=2)
 
 
-@pytest.mark.parametrize("basic", [GAPS, TWICE], ids=["gaps", "twice"])
+@pytest.mark.parametrize("basic", [GAPS, TWICE, LONG, MANY], ids=["gaps", "twice", "long", "many"])
 def test_irregular_basic_moments(oracle, basic):
     """Energies, forces, virials and loss gradients against the oracle: fp64, 1e-10 as for the shipped tables."""
     nt = 2
