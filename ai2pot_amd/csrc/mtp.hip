@@ -58,7 +58,8 @@ __host__ __device__ inline int mtp_adjoint_offset(int max_level_slots)
     return ((max_level_slots > 8 ? max_level_slots : 8) + 1) & ~1;     // at least the scratch of a block sum
 }
 // keep (energy / force / virial kernel, when the LDS allows it without costing a workgroup per CU): the adjoints lie
-// behind the table instead of inside it, so that a row of one chunk finds its table still in place in the last pass.
+// behind the table instead of inside it, so that a row of one chunk finds its table still in place in the last pass; keep
+// is the number of entries there (0: inside).
 __host__ __device__ inline int mtp_table_entries(int nc, int E, bool loss, int n_moms, int nt)
 {
     int a = loss ? nc * E + (mtp_gred_in_moments(loss, n_moms) ? 0 : (256 / 32) * 32 * 4) : nc * E;
@@ -66,12 +67,12 @@ __host__ __device__ inline int mtp_table_entries(int nc, int E, bool loss, int n
     return (a + 1) & ~1;
 }
 __host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_moms, int max_level_slots, int nt,
-                                                bool keep = false)
+                                                int keep = 0)
 {
     const int a = mtp_table_entries(nc, E, loss, n_moms, nt);
     // loss mode: two partial-sum arrays, then the adjoints and the mixed adjoints
     const int b = loss ? mtp_adjoint_offset(2 * max_level_slots) + 2 * n_moms : mtp_adjoint_offset(max_level_slots) + n_moms;
-    if (keep) return a + n_moms;
+    if (keep) return a + keep;
     return a > b ? a : b;
 }
 // the coefficients of the pair-derivative pass's polynomials take the place of the moments when they fit
@@ -109,7 +110,9 @@ struct MtpArgs {
     // Places in LDS, in entries (AtomLds), and in a row of the neighbour table: worked out once for the launch.
     int at_Tg, at_cf, at_tab, at_A, at_Bm, at_gred, at_Ab, at_Bb, at_pq, at_polys, at_net;
     int OY, OZ, OG, ODG, OU, OW, OF, ODF;
+    int z_powers;       // the table holds the powers of z (else z alone, and OZ + 1 is its place)
     int lds_basic_off;  // byte offset of the packed basic-moment table in LDS
+    int grad_parts;     // loss gradient: parts of a chunk's neighbours that are summed at the same time
     int mom_groups;     // thread groups that share a row's neighbours in the sums of the basic moments (basic_sums), or 0
     int nc_cap;         // rows of the LDS neighbour table: a row is processed in chunks of at most nc_cap
     int keep_table;     // energy / force / virial kernel: the adjoints lie behind the table (mtp_table_region)
@@ -163,7 +166,7 @@ __device__ __forceinline__ float sqrt_t(float x) { return sqrtf(x); }
 __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 
 // Per-neighbour table for neighbours [c0, c0+nc) of the row.
-// Layout per neighbour (E entries of T): ux^0..kmax | uy^.. | uz^.. | g[nmus] | dg[nmus] |
+// Layout per neighbour (E entries of T): ux^0..kmax | uy^.. | (z_powers) uz^.. | g[nmus] | dg[nmus] |
 // ux uy uz 1/r | (loss mode) vx vy vz w.u | f[K] | df[K]
 // PASS says what the pass that follows reads: TAB_MOMENTS powers, g, dg; TAB_TANGENTS also w; TAB_GRADIENT powers, w, f, df.
 // The threads form groups of nc, a neighbour to a thread.  Groups share the radial functions, two to a Chebyshev
@@ -215,9 +218,16 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             const T rinv = (T)1 / r;
             const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
             T px = (T)1, py = (T)1, pz = (T)1;
-            for (int k = 0; k <= kmax; k++) {
-                t[k] = px; t[kmax + 1 + k] = py; t[2 * (kmax + 1) + k] = pz;
-                px *= ux; py *= uy; pz *= uz;
+            if (a.z_powers) {
+                for (int k = 0; k <= kmax; k++) {
+                    t[k] = px; t[kmax + 1 + k] = py; t[2 * (kmax + 1) + k] = pz;
+                    px *= ux; py *= uy; pz *= uz;
+                }
+            } else {
+                for (int k = 0; k <= kmax; k++) {
+                    t[k] = px; t[kmax + 1 + k] = py;
+                    px *= ux; py *= uy;
+                }
             }
             t[OU + 0] = ux; t[OU + 1] = uy; t[OU + 2] = uz; t[OU + 3] = rinv;
             continue;
@@ -350,8 +360,8 @@ __device__ __forceinline__ void basic_sums(const T* tab, int E, int nc, int h, i
 template <typename T>
 __device__ __forceinline__ void basic_part(T* part, const T (&acc)[MTP_POLY_MAX], int h, int ng, unsigned word, int ncoef)
 {
-    const int len = (word >> 13) & 63;
-    T* const mine = part + h * ncoef + (word >> 19) + (len - 1);
+    const int len = (word >> 13) & 31;
+    T* const mine = part + h * ncoef + (word >> 18) + (len - 1);
     if (h < ng) {
 #pragma unroll
         for (int c = 0; c < MTP_POLY_MAX; c++)
@@ -583,6 +593,49 @@ __device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __re
     }
 }
 
+// The same sums polynomial by polynomial, longest first (mtp_plan.h: polys_len): every ng-th one, so that the lanes of a
+// wavefront walk polynomials of about the same length.  With V, D the value and derivative in z the polynomial adds
+//   gs += x^a y^b g' V,  w_x += a x^(a-1) y^b g V,  w_y += b x^a y^(b-1) g V,  w_z += x^a y^b g D
+// and the monomials are homogeneous, k m = u . grad m, so -(u . w) / r completes gs at the end.  What bounds it is the chain
+// of LDS reads and operations of a polynomial: its word is read while the one before is worked on, and its values in one go.
+// (Row by row, the radial functions of a row together, the whole kernel took 102 us instead of 98 for 64 x 128 atoms at level
+// 16, 260 instead of 255 for 8192 atoms at level 20 and 17.6 instead of 16.6 for 216 at level 10.)
+template <typename T>
+__device__ __forceinline__ void poly_walk(const T* __restrict__ t, const T* __restrict__ coef, const unsigned* __restrict__ words,
+                                          int npoly, int h, int ng, int OX, int OY, int OZ, int OG, int ODG, T ux, T uy, T uz,
+                                          T rinv, T& gs, T& wx, T& wy, T& wz)
+{
+    const T z = t[OZ + 1];
+    unsigned next = words[h];
+#pragma unroll 1
+    for (int s = h; s < npoly;) {
+        const unsigned pw = next;
+        s += ng;
+        if (s < npoly) next = words[s];
+        const int mu = pw & 7, ea = (pw >> 3) & 31, eb = (pw >> 8) & 31;
+        int len = (pw >> 13) & 31;
+        const T* c = coef + (pw >> 18);                          // highest power first
+        const T g = t[OG + mu], dg = t[ODG + mu], xa = t[OX + ea], yb = t[OY + eb], xm = t[OX + max(ea - 1, 0)],
+                ym = t[OY + max(eb - 1, 0)];
+        T v = (T)0, d = (T)0;
+        if (len & 1) v = *c++;
+#pragma unroll 1
+        for (len >>= 1; len > 0; len--, c += 2) {
+            const T c0 = c[0], c1 = c[1];
+            d = d * z + v;
+            v = v * z + c0;
+            d = d * z + v;
+            v = v * z + c1;
+        }
+        const T xy = xa * yb, gv = g * v;
+        gs += xy * dg * v;
+        wx += (T)ea * xm * yb * gv;
+        wy += (T)eb * xa * ym * gv;
+        wz += xy * g * d;
+    }
+    gs -= (ux * wx + uy * wy + uz * wz) * rinv;
+}
+
 // The polynomials of a neighbour for the loss gradient: every ng-th one of a radial function's from the s-th on.  With
 // A = sum adj m, B = sum (cE adj + mixed) m over the basic moments of mu and k m = u . grad m (m is homogeneous),
 //   P_mu = B + (w - (w . u) u) . grad A / r,   Q_mu = (w . u) A.
@@ -711,13 +764,15 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         if (mgroups) {
             mh = small_div(lane, p.npoly);
             if (mh < mgroups) pword = p.polys_len[lane - mh * p.npoly];
-            const int len = (pword >> 13) & 63;
+            const int len = (pword >> 13) & 31;
 #pragma unroll
             for (int c = 0; c < MTP_POLY_MAX; c++)
                 if (__any(len > c)) mtop = c + 1;
         }
         int* const rws = L.rws;
-        if (!LOSS) {
+        if (!LOSS && p.polys_len) {
+            for (int i = lane; i < p.npoly; i += NT) rws[i] = (int)p.polys_len[i];
+        } else if (!LOSS) {
             for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
             for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
         } else {
@@ -835,17 +890,28 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             const T* w1 = a.w1 + (size_t)ti * H;
             for (int s = lane; s < S; s += NT) qv[s] = (M[p.mapping[s]] - a.q_shift[s]) / a.q_scaler[s];
             __syncthreads();
-            for (int n = lane >> 6; n < H; n += NT / 64) {          // one wave per neuron
-                T acc = (T)0, tac = (T)0;
+            // a wavefront takes four neurons at a time, so that their weights' ways and their sums overlap
+            for (int n0 = (lane >> 6) * 4; n0 < H; n0 += NT / 64 * 4) {
+                T acc[4], tac[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) acc[u] = tac[u] = (T)0;
                 for (int k = lane & 63; k < S; k += 64) {
-                    acc += w0[(size_t)n * S + k] * qv[k];
-                    if (LOSS) tac += w0[(size_t)n * S + k] * Tg[p.mapping[k]] / a.q_scaler[k];
+                    const T q = qv[k], t = LOSS ? Tg[p.mapping[k]] / a.q_scaler[k] : (T)0;
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const T w = w0[(size_t)min(n0 + u, H - 1) * S + k];
+                        acc[u] += w * q;
+                        if (LOSS) tac[u] += w * t;
+                    }
                 }
-                acc = wave::all_sum(acc);
-                if (LOSS) tac = wave::all_sum(tac);
-                if ((lane & 63) == 0) {
-                    hv[n] = acc;
-                    if (LOSS) n_tau[n] = tac;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    acc[u] = wave::all_sum(acc[u]);
+                    if (LOSS) tac[u] = wave::all_sum(tac[u]);
+                    if ((lane & 63) == u && n0 + u < H) {
+                        hv[n0 + u] = acc[u];
+                        if (LOSS) n_tau[n0 + u] = tac[u];
+                    }
                 }
             }
             __syncthreads();
@@ -859,6 +925,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             __syncthreads();
             for (int k = lane; k < S; k += NT) {
                 T acc = (T)0, bac = (T)0;
+#pragma unroll 4
                 for (int n = 0; n < H; n++) {
                     const T w = w0[(size_t)n * S + k];
                     acc += hv[n] * w;
@@ -920,13 +987,16 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             int rk = 0, ng, h, j;
             {
                 MTP_PHASE;
-                ng = min(small_div(NT, nc), p.nrows);
+                ng = min(small_div(NT, nc), p.polys_len ? p.npoly : p.nrows);
                 h = small_div(lane, nc); j = lane - h * nc;
                 if (a.seg_cursor && lane < nc) rk = pair_claim_raw(&a.seg_cursor[b * NF + nj]);
                 if (h < ng) {
                     const T* t = tab + j * E;
                     ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
-                    pair_walk<T>(t, L.polys, L.rws, L.rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
+                    if (p.polys_len)
+                        poly_walk<T>(t, L.polys, (const unsigned*)L.rws, p.npoly, h, ng, OX, OY, OZ, OG, ODG, ux, uy, uz, rinv, gs, wx, wy, wz);
+                    else
+                        pair_walk<T>(t, L.polys, L.rws, L.rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
                 }
             }
             __syncthreads();            // every thread has read its table row: the group sums take its place
@@ -1078,17 +1148,42 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             const T* const Qm = L.pq + MTP_NC * nmus;
             int* const tjs = (int*)(L.pq + 2 * MTP_NC * nmus);
             T* const gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;
+            // The coefficient gradient: thread <- (part of the neighbours, mu, k), the parts' sums by species in the place of
+            // the group sums.  (A thread per (mu, k) took 8.2 of the 77 thousand cycles an atom takes at level 16, this 3.3.)
+            const int n1 = nmus * K, n2 = a.ntypes * n1;
+            if (a.grad_parts > 1) {
+                T* const part = L.gred;
+                const int parts = a.grad_parts;
+                for (int q = lane; q < parts * n2; q += NT) part[q] = (T)0;
+                // tj of each neighbour of the chunk
+                if (h == 0) tjs[j] = valid ? types[nj] : -1;
+                __syncthreads();
+                const int pt = small_div(lane, n1), q = lane - pt * n1;
+                if (pt < parts) {
+                    const int mu = small_div(q, K), k = q - mu * K;
+                    T* const mine = part + pt * n2 + q;
+                    for (int jn = pt; jn < nc; jn += parts) {
+                        const int tj = tjs[jn];
+                        const T* t = tab + jn * E;
+                        const T g = t[OF + k] * Pm[jn * nmus + mu] + t[ODF + k] * Qm[jn * nmus + mu];
+                        if (tj >= 0) mine[tj * n1] += g;
+                    }
+                }
+                __syncthreads();
+                for (int e = lane; e < n2; e += NT) gacc[e] += group_sum<T>(part + e, parts, n2);
+                continue;
+            }
             // tj of each neighbour of the chunk, for the accumulation below
             if (h == 0) tjs[j] = valid ? types[nj] : -1;
             __syncthreads();
             // lanes <- (mu, k): sequential over neighbours keeps the sum order fixed
-            for (int q = lane; q < nmus * K; q += NT) {
+            for (int q = lane; q < n1; q += NT) {
                 const int mu = small_div(q, K), k = q - mu * K;
                 for (int jn = 0; jn < nc; jn++) {
                     const int tj = tjs[jn];
                     if (tj < 0) continue;
                     const T* t = tab + jn * E;
-                    gacc[tj * nmus * K + q] += t[OF + k] * Pm[jn * nmus + mu] + t[ODF + k] * Qm[jn * nmus + mu];
+                    gacc[tj * n1 + q] += t[OF + k] * Pm[jn * nmus + mu] + t[ODF + k] * Qm[jn * nmus + mu];
                 }
             }
         }
@@ -1902,15 +1997,16 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         polys_end[m + 1] = (int)polys_mu.size();
     }
     std::vector<unsigned> polys_len;                              // longest first, for the sums of the basic moments
-    bool polys_fit = nmus <= 8 && n_poly_coef < (1 << 13);
+    const bool polys_fit = n_poly_coef < (1 << 14);               // (kmax <= 24, nmus <= 8)
+    int poly_top = 0;
     for (size_t r = 0; r < row_ab.size(); r++)
         for (int q = rows[r] >> 16; q < rows[r + 1] >> 16; q++) {
             const int mu = polys[q] & 15, len = (polys[q] >> 4) & 255, beg = polys[q] >> 12;
-            polys_fit = polys_fit && len <= MTP_POLY_MAX && row_ab[r].first < 32 && row_ab[r].second < 32;
+            poly_top = std::max(poly_top, len);
             polys_len.push_back((unsigned)mu | (unsigned)row_ab[r].first << 3 | (unsigned)row_ab[r].second << 8 |
-                                (unsigned)len << 13 | (unsigned)beg << 19);
+                                (unsigned)len << 13 | (unsigned)beg << 18);
         }
-    std::stable_sort(polys_len.begin(), polys_len.end(), [](unsigned x, unsigned y) { return (x >> 13 & 63) > (y >> 13 & 63); });
+    std::stable_sort(polys_len.begin(), polys_len.end(), [](unsigned x, unsigned y) { return (x >> 13 & 31) > (y >> 13 & 31); });
     std::vector<std::vector<int>> poly_lists(n_poly_coef);
     std::vector<int> poly_src(n_poly_coef), poly_items_off((size_t)n_poly_coef + 1, 0), poly_items, poly_pos(n_basic);
     int poly_unique = 1;
@@ -2121,6 +2217,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.poly_src = (const int*)(base + o_psrc); d.poly_off = (const int*)(base + o_poff);
     d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
     d.polys_len = polys_fit ? (const unsigned*)(base + o_plen) : nullptr;
+    d.poly_top = poly_top;
     d.poly_unique = poly_unique;
     d.x_nodes = 0; d.x_slots = 0;                // set per batch by the components call (MtpPlan::xbatches)
     for (size_t i = 0; i < xhosts.size(); i++) {
@@ -2150,18 +2247,39 @@ int plan_check(void* handle, MtpPlan** out)
     return A2P_OK;
 }
 
-template <typename T>
-int table_entries(const MtpPlanDevice& p, int K, bool loss)
+// 256 threads per atom or 64 (the rule is at its definition)
+bool wide_atoms(int n_moms, bool loss, bool network);
+
+// Whether the atom kernel sums the basic moments by polynomials (basic_sums): each has a thread, and the sums of a group
+// of threads fit the place of the shortest table.  Otherwise each moment is formed by itself, from powers of z.
+bool poly_sums(const MtpPlanDevice& p, bool loss, bool network)
 {
-    int E = 3 * (p.kmax + 1) + 2 * p.nmus + 4;
-    if (loss) E += 4 + 2 * K;
-    if ((E & 1) == 0) E++;            // odd stride: neighbours land in different LDS banks
-    return E;
+    return p.polys_len && p.poly_top <= MTP_POLY_MAX && p.npoly <= (wide_atoms(p.n_moms, loss, network) ? 256 : 64) &&
+           (loss ? 2 : 1) * p.ncoef_poly <= MTP_NC_MIN * (2 * (p.kmax + 1) + 2 * p.nmus + 4);
+}
+
+// The entries of a row of the neighbour table.
+template <typename T>
+void table_layout(MtpArgs<T>& a, bool loss, bool z_powers)
+{
+    const MtpPlanDevice& p = a.p;
+    a.z_powers = z_powers ? 1 : 0;
+    a.OY = p.kmax + 1;
+    a.OG = (z_powers ? 3 : 2) * (p.kmax + 1);
+    a.ODG = a.OG + p.nmus; a.OU = a.ODG + p.nmus; a.OW = a.OU + 4; a.OF = a.OW + 4; a.ODF = a.OF + a.K;
+    a.OZ = z_powers ? 2 * (p.kmax + 1) : a.OU + 1;
+    a.E = a.OU + 4 + (loss ? 4 + 2 * a.K : 0);
+    if ((a.E & 1) == 0) a.E++;        // odd stride: neighbours land in different LDS banks
+}
+template <typename T>
+void table_layout(MtpArgs<T>& a, bool loss)
+{
+    table_layout(a, loss, !poly_sums(a.p, loss, a.H > 0));
 }
 
 template <typename T>
 size_t lds_bytes(const MtpPlanDevice& p, int E, bool loss, int ntypes, int K, int H, int MTP_NC, int nt,
-                 bool keep = false)
+                 int keep = 0)
 {
     // the neighbour table and the group sums double as the sweeps' partial-sum arrays
     const size_t tabs = (size_t)mtp_table_region(MTP_NC, E, loss, p.n_moms, p.max_level_slots, nt, keep);
@@ -2201,8 +2319,6 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0;
     a.nn_exact = 1;
     a.row_seed = nullptr; a.pair_out = nullptr;
-    a.OY = a.p.kmax + 1; a.OZ = 2 * a.OY; a.OG = 3 * a.OY; a.ODG = a.OG + nmus; a.OU = a.ODG + nmus; a.OW = a.OU + 4;
-    a.OF = a.OW + 4; a.ODF = a.OF + K;
     a.H = 0; a.w0 = nullptr; a.w1 = nullptr; a.q_shift = nullptr;
     void* ws = nullptr;
     int rc = ws_get(WS_FLAGS, 64, &ws);
@@ -2224,7 +2340,7 @@ int g_keep_table = 1;      // (measurement switch: AI2POT_MTP_KEEP_TABLE=0)
 //   level 18 (718)        194 / 183
 // With a network the loss gradient has a weight per neuron and scalar moment besides (64 x 125 atoms; 2 x 60; 30 neurons):
 //   level 8  221 / 211 (10 neurons: 170 / 186)   46 / 40      level 10  273 / 230   51 / 44      level 12  304 / 247   56 / 46
-inline bool wide_atoms(int n_moms, bool loss, bool network)
+bool wide_atoms(int n_moms, bool loss, bool network)
 {
     return n_moms >= (loss ? (network ? 40 : 150) : 600);
 }
@@ -2237,7 +2353,9 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         if (e) g_keep_table = e[0] != '0';
     }
     const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0);
-    auto lds_for = [&](int nc, size_t* main, bool keep = false) {
+    const int groups = a.z_powers ? 0 : (wide ? 256 : 64) / std::max(a.p.npoly, 1);      // of a thread per polynomial
+    const int kept_adjoints = std::max(a.p.n_moms, groups * a.p.ncoef_poly);
+    auto lds_for = [&](int nc, size_t* main, int keep = 0) {
         *main = (lds_bytes<T>(a.p, a.E, LOSS, a.ntypes, a.K, a.H, nc, wide ? 256 : 64, keep) + 15) / 16 * 16;
         // the packed basic-moment table and the polynomials, with the monomial rows or the run of every mu
         return *main + ((size_t)a.p.n_basic + a.p.npoly + 1 + (LOSS ? a.p.nmus : a.p.nrows)) * sizeof(unsigned);
@@ -2267,7 +2385,7 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         int keep = 0;
         if (!a.e_sites && !a.desc && !a.energy_only && g_keep_table)
             for (int nc : {MTP_NC_MAX, 40, 32}) {
-                const size_t l = lds_for(nc, &m, true);
+                const size_t l = lds_for(nc, &m, kept_adjoints);
                 if (per_cu(l) >= want) { keep = 1; nc_cap = nc; lds = l; lds_main = m; break; }
             }
         const_cast<MtpArgs<T>&>(a).keep_table = keep;
@@ -2276,7 +2394,7 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         MtpArgs<T>& w = const_cast<MtpArgs<T>&>(a);
         const MtpPlanDevice& p = a.p;
         const int nt = wide ? 256 : 64;
-        const bool keep = !LOSS && w.keep_table != 0;
+        const int keep = !LOSS && w.keep_table != 0 ? kept_adjoints : 0;
         w.lds_basic_off = (int)lds_main;
         w.nc_cap = nc_cap;
         // moments | (loss mode: their tangents) | coefficients | region of the neighbour table | ...
@@ -2297,10 +2415,14 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         w.at_net = w.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);
         w.at_polys = mtp_polys_in_moments(p.ncoef_poly, p.n_moms) ? 0 : w.at_pq + (a.H > 0 ? p.n_scalar + a.H : 0);
     }
+    if (LOSS) {
+        // the group sums' place: the moments and their tangents, or 1024 entries behind the table
+        const int n1 = a.p.nmus * a.K, place = mtp_gred_in_moments(true, a.p.n_moms) ? 2 * a.p.n_moms : 1024;
+        const_cast<MtpArgs<T>&>(a).grad_parts = std::max(1, std::min((wide ? 256 : 64) / n1, place / (a.ntypes * n1)));
+    }
     // as many groups of a thread per polynomial as the workgroup has, and as the place of their sums holds
-    const int room = !LOSS && a.keep_table ? a.p.n_moms : mtp_table_entries(nc_cap, a.E, LOSS, a.p.n_moms, wide ? 256 : 64);
-    const_cast<MtpArgs<T>&>(a).mom_groups =
-        a.p.polys_len ? std::min((wide ? 256 : 64) / std::max(a.p.npoly, 1), room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1)) : 0;
+    const int room = !LOSS && a.keep_table ? kept_adjoints : mtp_table_entries(nc_cap, a.E, LOSS, a.p.n_moms, wide ? 256 : 64);
+    const_cast<MtpArgs<T>&>(a).mom_groups = std::min(groups, room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1));
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
     auto kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
@@ -2352,7 +2474,7 @@ int mtp_efv(void* handle, int K, double scaling, const T* coeffs, const T* lin, 
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
     a.e_sites = e_sites;
-    a.E = table_entries<T>(a.p, K, false);
+    table_layout(a, false);
     void* ws = nullptr;
     rc = ws_get(WS_PARTIAL, (size_t)B * P * 10 * sizeof(double), &ws);
     if (rc) return rc;
@@ -2428,7 +2550,7 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
-    a.E = table_entries<T>(a.p, K, true);
+    table_layout(a, true);
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
@@ -2493,7 +2615,7 @@ int nnmtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft,
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
-    a.E = table_entries<T>(a.p, K, true);
+    table_layout(a, true);
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = nrow;
     a.nn_exact = exact ? 1 : 0;
     rc = launch_atoms<T, true>(a, stream);
@@ -2524,7 +2646,7 @@ int mtp_esites(void* handle, int K, double scaling, const T* coeffs, const T* li
     rc = set_net(a, net);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
-    a.E = table_entries<T>(a.p, K, false);
+    table_layout(a, false);
     a.e_sites = e_sites; a.desc = desc; a.energy_only = 1;
     return launch_atoms<T, false>(a, stream);
 }
@@ -2559,7 +2681,7 @@ int mtp_esites_bwd(void* handle, int K, double scaling, const T* coeffs, const T
     T* gpart = (T*)ws + nzero;
     rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
     if (rc) return rc;
-    a.E = table_entries<T>(a.p, K, true);
+    table_layout(a, true);
     a.cE = gout; a.cE_per_atom = 1; a.no_tangent = 1; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
@@ -2597,7 +2719,7 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         rc = fill_zero(drcs, (size_t)B * P * U * 3 * sizeof(T), stream);
         if (rc) return rc;
         MtpArgs<T> e = a;
-        e.E = table_entries<T>(e.p, K, false);
+        table_layout(e, false);
         e.pair_out = drcs;
         rc = launch_atoms<T, false, true>(e, stream);
         if (rc) return rc;
@@ -2615,7 +2737,7 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
         if (rc) return rc;
         MtpArgs<T> g = a;
-        g.E = table_entries<T>(g.p, K, true);
+        table_layout(g, true);
         g.dFs = dFs; g.dVs = dVs; g.gpart = gpart; g.ngrad = ncoef; g.no_tangent = 1;
         rc = launch_atoms<T, true>(g, stream);
         if (rc) return rc;
@@ -2797,7 +2919,7 @@ int mtp_lin_components(void* handle, int K, double scaling, const T* coeffs, int
                        rmin, B, P, U, 0, binum, bilist, bnumneigh, bfirstneigh, brcs, btypes, false);
         if (rc) return rc;
         A2P_REQUIRE(q_scaler, A2P_ERR_INVALID, "mtp components: null q_scaler");
-        a.E = table_entries<T>(a.p, K, false);
+        table_layout(a, false, true);     // (the kernel forms derivatives of each basic moment)
         return mtp_lin_components_nodes<T>(plan, a, S, n, ecomp, fcomp, vcomp, stream);
     }
     rc = fill_zero(ecomp, (size_t)B * n * sizeof(T), stream);
@@ -2891,7 +3013,7 @@ int nnmtp_esites_bwd(void* handle, int K, const MtpNet<T>& net, const T* coeffs,
     T* gpart = (T*)ws + nzero;
     rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
     if (rc) return rc;
-    a.E = table_entries<T>(a.p, K, true);
+    table_layout(a, true);
     a.cE = gout; a.cE_per_atom = 1; a.no_tangent = 1; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = nrow;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;

@@ -59,8 +59,9 @@ struct MtpPlanDevice {
     const int* polys_mu;       // [npoly] the same by mu: a | b << 5 | length << 10 | first coefficient << 15
     const int* polys_end;      // [nmus + 1] run of each mu in polys_mu
     const int* poly_pos;       // [n_basic] coefficient of each basic moment
-    const unsigned* polys_len; // [npoly] the same, longest first: mu | a << 3 | b << 8 | length << 13 | first coefficient << 19
-                               // (null: one of them does not fit its field)
+    const unsigned* polys_len; // [npoly] the same, longest first: mu | a << 3 | b << 8 | length << 13 | first coefficient << 18
+                               // (null: a coefficient does not fit its field)
+    int poly_top;              // length of the longest
     int poly_unique;           // no two basic moments share a coefficient (the usual case: a plain scatter fills them)
     const int* poly_src;       // [ncoef_poly] basic moment behind the coefficient, -1 none, -2 several (poly_off / items)
     const int* poly_off;       // [ncoef_poly+1]
