@@ -100,34 +100,6 @@ __device__ __forceinline__ void ld4_stream(const double* p, double (&o)[4])
 __device__ __forceinline__ int entry_bits(float w) { return __float_as_int(w); }
 __device__ __forceinline__ int entry_bits(double w) { return (int)__double_as_longlong(w); }
 
-// nep_device.h's radial_basis (f_k = 1/2 (T_k(x)+1) fc(r), basis.h:137-158, 300-332, 519-530) for all KC functions
-template <typename T, bool DER>
-__device__ __forceinline__ void radial_functions(T r, T rc_inv, T (&f)[KC], T (&df)[KC])
-{
-    const T t = r * rc_inv;
-    const T xr = t - (T)1;
-    const T x = (T)2 * xr * xr - (T)1, x2 = x + x;
-    T sn, cs;
-    sincospi_t(t, &sn, &cs);
-    const T fc = (T)0.5 * ((T)1 + cs), hfc = (T)0.5 * fc;
-    const T dfc = (T)(-0.5 * 3.14159265358979323846) * sn * rc_inv, hdfc = (T)0.5 * dfc;
-    const T w = hfc * ((T)4 * rc_inv * xr);                  // 1/2 fc dx/dr
-    T t0 = (T)1, t1 = x, d0 = (T)0, d1 = (T)1;
-    f[0] = fc; f[1] = hfc * x + hfc;
-    if (DER) { df[0] = dfc; df[1] = hdfc * x + hdfc + w; }
-#pragma unroll
-    for (int k = 2; k < KC; k++) {
-        const T tv = x2 * t1 - t0;
-        f[k] = hfc * tv + hfc;
-        if (DER) {
-            const T dv = (T)2 * t1 + (x2 * d1 - d0);
-            df[k] = (hdfc * tv + hdfc) + w * dv;
-            d0 = d1; d1 = dv;
-        }
-        t0 = t1; t1 = tv;
-    }
-}
-
 // sum_k a_k f_k'(r) without the functions themselves:
 //   1/2 fc' (sum a_k T_k + sum a_k) + 1/2 fc x' sum a_k T_k'
 template <typename T>
@@ -136,10 +108,10 @@ __device__ __forceinline__ T radial_derivative_dot(T r, T rc_inv, const T (&a)[K
     const T t = r * rc_inv;
     const T xr = t - (T)1;
     const T x = (T)2 * xr * xr - (T)1, x2 = x + x;
-    T sn, cs;
-    sincospi_t(t, &sn, &cs);
-    const T hfc = (T)0.25 * ((T)1 + cs);
-    const T hdfc = (T)(-0.25 * 3.14159265358979323846) * sn * rc_inv;
+    T cs, sn;
+    cos_sin_pi(t, cs, sn);
+    const T hfc = (T)0.25 * cs + (T)0.25;
+    const T hdfc = (T)(-0.25 * 3.14159265358979323846) * rc_inv * sn;
     T t0 = (T)1, t1 = x, d0 = (T)0, d1 = (T)1;
     T s0 = a[0] + a[1], st = a[0] + a[1] * x, sd = a[1];
 #pragma unroll
@@ -540,14 +512,14 @@ nep_adjoint_kernel(const GatherArgs<T> a)
         const T r = sqrt_t(x * x + y * y + z * z);
         const T rinv = (T)1 / r;
         T f[KC], df[KC];
-        radial_functions<T, false>(r, rr_inv, f, df);
+        radial_basis<T, KC, false>(r, rr_inv, KC, f, df);
 #pragma unroll
         for (int t = 0; t < NTC; t++) {
             const T mt = (valid && tj == t) ? (T)1 : (T)0;
 #pragma unroll
             for (int k = 0; k < KC; k++) F[t][k] += mt * f[k];
         }
-        radial_functions<T, false>(r, ra_inv, f, df);
+        radial_basis<T, KC, false>(r, ra_inv, KC, f, df);
         const T* c = L.coef + ((ti * nt + tj) * NB + NR) * KC;
         T bl[NLM];
         blm_values<T, LC>(x * rinv, y * rinv, z * rinv, bl);
@@ -571,7 +543,7 @@ nep_adjoint_kernel(const GatherArgs<T> a)
         const int tj = min((bits >> CL_TYPE_SHIFT) & 15, nt - 1);
         const T r = sqrt_t(x * x + y * y + z * z);
         T f[KC], df[KC];
-        radial_functions<T, false>(r, rr_inv, f, df);
+        radial_basis<T, KC, false>(r, rr_inv, KC, f, df);
 #pragma unroll
         for (int t = 0; t < NTC; t++) {
             const T mt = (valid && tj == t) ? (T)1 : (T)0;
@@ -716,7 +688,7 @@ nep_adjoint_kernel(const GatherArgs<T> a)
                 for (int k = 0; k < KC; k++) ck[k] = L.acc[(tj * KC + k) * CB + tid];
                 srad = radial_derivative_dot<T>(r, rr_inv, ck);
             }
-            radial_functions<T, true>(r, ra_inv, f, df);
+            radial_basis<T, KC, true>(r, ra_inv, KC, f, df);
             const T* ci = L.coef + ((ti * nt + tj) * NB + NR) * KC;
             T A[NLM], Ad[NLM];
 #pragma unroll

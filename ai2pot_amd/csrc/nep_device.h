@@ -50,8 +50,42 @@ struct NepArgs {
     int mb4 = 0, mb5 = 0;   // extension (generic kernel only): four- / five-body invariant per angular channel
 };
 
-__device__ __forceinline__ void sincospi_t(float x, float* s, float* c) { sincospif(x, s, c); }
-__device__ __forceinline__ void sincospi_t(double x, double* s, double* c) { sincospi(x, s, c); }
+// sin(pi u / 2) on [-1, 1]: u + u p(u^2), p + 1 the polynomial of least relative error (5e-9; 2.6e-19) for sin(pi sqrt(y) / 2) / sqrt(y)
+__device__ __forceinline__ float quarter_sine(float u)
+{
+    const float y = u * u;
+    float p = 0.000151485130733f;
+    p = p * y - 0.0046737666124f;
+    p = p * y + 0.0796896789478f;
+    p = p * y - 0.6459637106f;
+    p = p * y + 0.57079631845f;
+    return u * p + u;
+}
+__device__ __forceinline__ double quarter_sine(double u)
+{
+    const double y = u * u;
+    double p = 5.8706109783952470938e-12;
+    p = p * y - 6.684321720453320249e-10;
+    p = p * y + 5.6921348727149338656e-8;
+    p = p * y - 3.5988430072086468421e-6;
+    p = p * y + 0.00016044118470682204322;
+    p = p * y - 0.0046817541353026425916;
+    p = p * y + 0.079692626246165435628;
+    p = p * y - 0.64596409750624619109;
+    p = p * y + 0.5707963267948966188;
+    return u * p + u;
+}
+// cos(pi t) and sin(pi t) for t in [0, 1] (a dummy neighbour's larger t is taken for 1).  The library's pair reduces any
+// argument first: 660 instead of 631 us for the adjoint kernel of 1,048,576 atoms, 96 instead of 90 for a wavefront per atom at
+// 20,011; forces against fp64 differ by 4.7e-7 with either.
+template <typename T>
+__device__ __forceinline__ void cos_sin_pi(T t, T& c, T& s)
+{
+    t = min(t, (T)1);
+    const T m = min(t, (T)1 - t);
+    c = quarter_sine((T)1 - (t + t));
+    s = quarter_sine(m + m);
+}
 __device__ __forceinline__ float tanh_t(float x) { return tanhf(x); }
 __device__ __forceinline__ double tanh_t(double x) { return tanh(x); }
 __device__ __forceinline__ float sqrt_t(float x) { return sqrtf(x); }
@@ -64,26 +98,23 @@ __device__ __forceinline__ void radial_basis(T r, T rc_inv, int K, T (&f)[KC], T
 {
     const T t = r * rc_inv;
     const T xr = t - (T)1;
-    const T x = (T)2 * xr * xr - (T)1;
-    const T dxdr = (T)4 * rc_inv * xr;
-    T sn, cs;
-    sincospi_t(t, &sn, &cs);
-    const T fc = (T)0.5 * ((T)1 + cs);
-    const T dfc = (T)(-0.5 * 3.14159265358979323846) * sn * rc_inv;
+    const T x = (T)2 * xr * xr - (T)1, x2 = x + x;
+    T cs, sn;
+    cos_sin_pi(t, cs, sn);
+    const T h = (T)0.25 * cs + (T)0.25;                                           // 1/2 fc
+    const T dh = (T)(-0.25 * 3.14159265358979323846) * rc_inv * sn;               // 1/2 fc'
+    const T w = h * ((T)4 * rc_inv * xr);                                         // 1/2 fc dx/dr
     T t0 = (T)1, t1 = x, d0 = (T)0, d1 = (T)1;
 #pragma unroll
     for (int k = 0; k < KC; k++) {
-        T tv, dv;
-        if (k == 0) { tv = t0; dv = d0; }
-        else if (k == 1) { tv = t1; dv = d1; }
-        else {
-            tv = (T)2 * x * t1 - t0;
-            dv = (T)2 * t1 + (T)2 * x * d1 - d0;
+        T tv = k == 0 ? t0 : t1, dv = k == 0 ? d0 : d1;
+        if (k >= 2) {
+            tv = x2 * t1 - t0;
+            dv = (T)2 * t1 + (x2 * d1 - d0);
             t0 = t1; t1 = tv; d0 = d1; d1 = dv;
         }
-        const T v = (T)0.5 * (tv + (T)1);
-        f[k] = (k < K) ? fc * v : (T)0;
-        if (DER) df[k] = (k < K) ? dfc * v + fc * (T)0.5 * dv * dxdr : (T)0;
+        f[k] = (k < K) ? (k == 0 ? h + h : h * tv + h) : (T)0;
+        if (DER) df[k] = (k < K) ? (k == 0 ? dh + dh : (dh * tv + dh) + w * dv) : (T)0;
     }
 }
 
