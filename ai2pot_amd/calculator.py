@@ -98,9 +98,10 @@ class NepCalculator:
         if path == "gather" and not can_gather:
             raise ValueError("the gather path does not cover this model shape / list options")
         # "auto": the gather kernels give every atom a thread and want tens of thousands of them; smaller systems take
-        # the segment path, whose kernel gives every atom a wavefront.  A step with rebuild, segments / gather:
-        # fp32 24,000 atoms 170 / 181 us, 32,000 202 / 188; fp64 16,384 203 / 234, 24,000 261 / 247
-        most = 28672 if f32 else 20480
+        # the segment path, whose kernel has four atoms to a wavefront.  A step with rebuild, segments / gather, 16, 36 and
+        # 72 neighbours: fp32 56,000 atoms 152 / 163, 175 / 190, 233 / 242 us, 80,000 196 / 197, 235 / 233, 321 / 305;
+        # fp64 28,000 178 / 187, 211 / 228, 252 / 290, 40,000 226 / 196, 272 / 239, 328 / 313
+        most = 65536 if f32 else 30720
         self.path = "gather" if (can_gather and (path == "gather" or (path == "auto" and self.n >= most))) else "segments"
         self.padded = bool(padded) or self.path != "gather"
         self.input_order = int(reorder_every) == 0

@@ -187,6 +187,22 @@ template <typename T>
 int pair_reduce(T* force, const T* pair_g, int B, int P, int U, int nghost, const int* binum, const int* bilist,
                 const int* bnumneigh, const int* bfirstneigh, bool own, hipStream_t stream);
 
+// A kernel's argument block, taken anew from the segment it was passed in: a kernel of many phases holds each value in a
+// register from its first to its last use otherwise, and what does not fit moves between lanes of vector registers.  S is the
+// kernel's first parameter; the empty statement keeps the compiler from carrying an earlier phase's values over.
+#define A2P_CONSTANT __attribute__((address_space(4)))
+template <typename S>
+__device__ __forceinline__ const A2P_CONSTANT S& again(const A2P_CONSTANT S* args)
+{
+    asm volatile("" : "+s"(args));
+    return *args;
+}
+template <typename S>
+__device__ __forceinline__ const A2P_CONSTANT S* kernel_args() { return (const A2P_CONSTANT S*)__builtin_amdgcn_kernarg_segment_ptr(); }
+// An array that a wavefront reads uniformly: by scalar loads.
+template <typename S>
+__device__ __forceinline__ const A2P_CONSTANT S* uniform_array(const S* p) { return (const A2P_CONSTANT S*)(uintptr_t)p; }
+
 // The same reduction for a producer that stores each pair derivative straight into its target's segment, without the
 // intermediate [row, slot, 3] array (pair_fixed_begin, the producer, pair_csr_finish).
 // Capacity of the fixed reduction segments: umax unless the calling thread asked for more with

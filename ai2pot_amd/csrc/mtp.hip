@@ -134,27 +134,6 @@ struct MtpArgs {
     T* pair_out;       // [B, P, U, 3] derivative of the row's weighted moments along each pair vector, or null
 };
 
-// The kernels' arguments are some eighty scalars, and the plan names two dozen arrays: held in registers from the first
-// use to the last they do not fit, and what did not (some 150 values) moved between lanes of vector registers all the time:
-// 300 instead of 281 us for the energies and forces of level 20, 8192 atoms, 238 instead of 222 for the loss gradient of
-// level 16, 64 structures of 128 atoms.  Each phase takes the arguments from the segment they were passed in anew (scalar loads; the empty
-// statement keeps the compiler from carrying an earlier phase's values over).
-#define A2P_CONSTANT __attribute__((address_space(4)))
-template <typename S>
-__device__ __forceinline__ const A2P_CONSTANT S& again(const A2P_CONSTANT S* args)
-{
-    asm volatile("" : "+s"(args));
-    return *args;
-}
-template <typename T>
-__device__ __forceinline__ const A2P_CONSTANT MtpArgs<T>* kernel_args()
-{
-    return (const A2P_CONSTANT MtpArgs<T>*)__builtin_amdgcn_kernarg_segment_ptr();      // the first parameter
-}
-// A plan array that a wavefront reads uniformly: by scalar loads.
-template <typename S>
-__device__ __forceinline__ const A2P_CONSTANT S* uniform_array(const S* p) { return (const A2P_CONSTANT S*)(uintptr_t)p; }
-
 // a / b for small integers, 0 <= a < 2^20, b > 0 (the exact quotient is at least 0.5 / b away from the next integer, the
 // rounding here below 2^-22 of it)
 __device__ __forceinline__ int small_div(int a, int b) { return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b)); }
@@ -711,8 +690,12 @@ struct AtomLds {
 };
 
 // What a phase of the atom kernel works with, under the names of the formulas.
+// The kernels' arguments are some eighty scalars, and the plan names two dozen arrays: held in registers from the first
+// use to the last they do not fit, and what did not (some 150 values) moved between lanes of vector registers all the time:
+// 300 instead of 281 us for the energies and forces of level 20, 8192 atoms, 238 instead of 222 for the loss gradient of
+// level 16, 64 structures of 128 atoms.  Each phase takes the arguments from the segment they were passed in anew (scalar loads).
 #define MTP_PHASE                                                                                                          \
-    [[maybe_unused]] auto& a = again(kernel_args<T>());                                                                    \
+    [[maybe_unused]] auto& a = again(kernel_args<MtpArgs<T>>());                                                                \
     [[maybe_unused]] auto& p = a.p;                                                                                        \
     [[maybe_unused]] const bool seeded = (SEED || LOSS) && a.row_seed != nullptr;                                          \
     [[maybe_unused]] const bool no_tan = LOSS && a.no_tangent != 0;                 /* uniform over the launch */          \

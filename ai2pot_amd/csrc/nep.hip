@@ -439,15 +439,14 @@ int launch(const NepArgs<T>& a, size_t lds, hipStream_t stream)
     return A2P_OK;
 }
 
-// Atoms of a batch up to which a wavefront per atom beats the staged kernel's thread per atom, where both have the shape.
-// A wavefront per atom costs more instructions in all, but its chain is short and a few thousand atoms fill the chip; a
-// thread per atom takes the same time from one atom to as many as there are lanes.  Measured (6 radial, l_max 4, 60
-// neighbours; wavefront / staged, whole operator): fp32 8,000 atoms 69 / 166 us, 32,000 145 / 179, 45,000 188 / 193,
-// 64,000 244 / 218; fp64 8,000 98 / 227, 24,000 203 / 238, 32,000 257 / 242.  The thread's chain grows with the row, the
-// wavefront's work hardly does up to 64 neighbours, so the line moves with the length of the rows, which the host does not
-// know: 16 neighbours 22,000 atoms (fp64 17,000), 24: 28,000 (20,000), 36: 36,000 (28,000), 52: 42,000 (32,000).
+// Atoms of a batch up to which four atoms per wavefront beat the staged kernel's thread per atom, where both have the shape.
+// Whole operator, 6 radial, l_max 4, us (wavefront / staged).  fp32, 16, 36 and 72 neighbours: 40,000 atoms 72 / 162, 85 / 161,
+// 121 / 189; 100,000 138 / 139, 172 / 261, 259 / 432; 200,000 267 / 263, 339 / 514, 489 / 836: always the wavefront (the staged
+// kernel keeps the networks too large for its LDS, some 1300 neurons).  fp64, which holds a wavefront per SIMD: 40,000
+// 161 / 146, 194 / 214, 245 / 347; 60,000 225 / 157, 277 / 264, 350 / 426; 100,000 372 / 258, 458 / 447, 563 / 713.  The line
+// moves with the length of the rows, which the host does not know.
 template <typename T>
-constexpr long long wave_most() { return sizeof(T) == 4 ? 40960 : 28672; }
+constexpr long long wave_most() { return sizeof(T) == 4 ? 1ll << 62 : 49152; }
 
 template <typename T>
 int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coeffs, const T* w0,
@@ -500,11 +499,9 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     size_t lds_staged = 0;
     const bool staged = !(mb4 || mb5) && nep_staged_supported<T>(a, &lds_staged);
     if (staged) a.nblocks = nep_staged_nblocks(P);
-    // the wavefront-per-atom kernel: every shape it has in batches up to wave_most, beyond it those the staged kernel does
-    // not have
-    size_t lds_wave = 0;
-    const bool wave = !(mb4 || mb5) && ((long long)B * P < wave_most<T>() || !staged) && nep_wave_supported<T>(a, &lds_wave);
-    if (wave) a.nblocks = nep_wave_nblocks(P, B);
+    // four atoms per wavefront: every shape it has in batches up to wave_most, beyond it those the staged kernel does not have
+    const bool wave = !(mb4 || mb5) && ((long long)B * P < wave_most<T>() || !staged) && nep_wave_supported<T>(a);
+    if (wave) a.nblocks = nep_wave_nblocks<T>(a);
 
     void* ws = nullptr;
     int rc = ws_get(WS_FLAGS, 64, &ws);
@@ -518,7 +515,7 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     const size_t force_bytes = (size_t)B * (P + nghost) * 3 * sizeof(T);
 
     if (wave) {
-        return nep_wave_run<T>(a, lds_wave, etot, virial, stream);       // includes the energy / virial sums
+        return nep_wave_run<T>(a, etot, virial, stream);       // includes the energy / virial sums
     } else if (staged) {
         return nep_staged_run<T>(a, lds_staged, etot, virial, stream);
     } else {

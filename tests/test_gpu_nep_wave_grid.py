@@ -1,0 +1,58 @@
+"""The NEP kernel with four atoms per wavefront over the sizes of its launches: wavefronts of a workgroup, workgroups of a
+compute unit and rows of a wavefront change with the number of rows."""
+import numpy as np
+import pytest
+
+from ai2pot_amd import synth
+from test_gpu_nep import run_gpu
+
+pytestmark = pytest.mark.gpu
+ROWS, U = 71, 72
+
+
+def _block(np_dtype, ntypes):
+    rng = np.random.default_rng(11)
+    n = rng.integers(0, U + 1, ROWS).astype(np.int32)
+    u = rng.normal(size=(ROWS, U, 3))
+    u /= np.linalg.norm(u, axis=2, keepdims=True)
+    r = np.where(rng.random((ROWS, U)) < 0.35, rng.uniform(2.0, 3.99, (ROWS, U)), rng.uniform(4.01, 7.5, (ROWS, U)))
+    return dict(n=n, first=rng.integers(0, ROWS, (ROWS, U)).astype(np.int32), rcs=(u * r[..., None]).astype(np_dtype),
+                types=rng.integers(0, ntypes, ROWS).astype(np.int32))
+
+
+def _copies(blk, copies, batch):
+    """`copies` of the block as one structure, the last without its last row; `batch` such structures."""
+    first = (blk["first"][None] + ROWS * np.arange(copies, dtype=np.int32)[:, None, None]).reshape(-1, U)
+    one = dict(bilist=np.arange(ROWS * copies, dtype=np.int32), bnumneigh=np.tile(blk["n"], copies), bfirstneigh=first,
+               brcs=np.tile(blk["rcs"], (copies, 1, 1)), btypes=np.tile(blk["types"], copies))
+    nb = {k: np.array(np.broadcast_to(v, (batch,) + v.shape)) for k, v in one.items()}
+    return dict(nb, binum=np.full(batch, ROWS * copies - 1, np.int32), nghost=0)
+
+
+# fp32 at three species: up to 4096 rows four wavefronts, up to 8192 two workgroups of four, beyond it twelve wavefronts, beyond
+# 12288 several times four rows each; fp64 holds four wavefronts throughout.  One species: several workgroups of any size.
+@pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("ntypes,copies,batch", [(3, 1, 1), (3, 57, 1), (3, 58, 1), (3, 115, 1), (3, 116, 1), (3, 180, 1), (3, 600, 1),
+                                                 (3, 1, 61), (3, 3, 61), (1, 180, 1), (5, 60, 3)])
+def test_every_launch_gives_the_same(np_dtype, ntypes, copies, batch):
+    blk = _block(np_dtype, ntypes)
+    m = synth.nep_model(ntypes=ntypes, num_neurons=30, type_map=(1, 2, 3, 4, 5), sigma=0.12)
+    m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    e2, f2, _ = run_gpu(m, _copies(blk, 2, 1), np_dtype)               # (a launch of nine workgroups' worth at most)
+    e3, _, v3 = run_gpu(m, _copies(blk, 3, 1), np_dtype)
+    _, _, v2 = run_gpu(m, _copies(blk, 2, 1), np_dtype)
+    e, f, v = run_gpu(m, _copies(blk, copies, batch), np_dtype)
+    # An atom's sums run over up to 72 pairs in another order when its lane or chunk is another; a pair's force is a sum over the
+    # 24 x 4 moments: 100 roundings of the largest term, with room for the cancellation of pairs of a dozen times the sum.
+    eps = np.finfo(np_dtype).eps
+    inner = f2.reshape(2, ROWS, 3)[0]
+    tol = 1200 * eps * np.abs(inner).max()
+    f = f.reshape(batch, copies, ROWS, 3)
+    if copies > 1:
+        assert np.abs(f[:, :-1] - inner).max() <= tol
+    assert np.abs(f[:, -1] - f2.reshape(2, ROWS, 3)[1]).max() <= tol
+    # energies and virials: those of two blocks and so many times those of one more
+    per_e, per_v = e3 - e2, v3 - v2
+    scale = max(copies, 3) * eps * 1200
+    assert np.abs(e - (e2 + (copies - 2) * per_e)).max() <= scale * np.abs(e3).max()
+    assert np.abs(v - (v2 + (copies - 2) * per_v)).max() <= scale * np.abs(v3).max()
