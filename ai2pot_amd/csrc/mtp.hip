@@ -1279,6 +1279,11 @@ struct CompArgs {
     int batch;              // neighbours whose D vectors are formed together (even)
     int d_over_nodes;       // all groups of pieces are worked on at once, so the D vectors take the place of the node adjoints
 };
+template <typename T>
+struct CompKernelArgs {
+    MtpArgs<T> mtp;
+    CompArgs<T> comp;
+};
 
 // six values from an even entry of LDS: 16-byte reads (8-byte in single precision)
 __device__ __forceinline__ void load6(const double* p, double (&o)[6])
@@ -1298,50 +1303,63 @@ __device__ __forceinline__ void load6(const float* p, float (&o)[6])
     }
 }
 
+// Arguments anew in each phase, as in mtp_atom_kernel: 173 instead of 178 us for 32 structures of 128 atoms at level 16; with two
+// places of D to a register, where sixteen of them and their adjoints had not fitted, 170.  (The basic moments by polynomials, as there:
+// 173.  The pair derivatives as products of 16 x 16 tiles on the matrix cores, tiles without entries left out: 272; the fp64
+// products take 41 us of that, the operands' chain of table, vector and gather the rest.)
+#define COMP_PHASE                                                                                                         \
+    [[maybe_unused]] auto& K_ = again(kernel_args<CompKernelArgs<T>>());                                                   \
+    [[maybe_unused]] auto& a = K_.mtp;                                                                                     \
+    [[maybe_unused]] auto& c = K_.comp;                                                                                    \
+    [[maybe_unused]] auto& p = a.p;                                                                                        \
+    [[maybe_unused]] const int NF = a.P, n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, K = a.K, E = a.E,          \
+                               S = p.n_scalar;                                                                             \
+    [[maybe_unused]] const int OX = 0, OY = a.OY, OZ = a.OZ, OG = a.OG, ODG = a.ODG, OU = a.OU;                            \
+    /* moments | node adjoints (+ the zero entry) | coefficients | neighbour table */                                      \
+    [[maybe_unused]] T* const M = (T*)smem_raw;                                                                            \
+    [[maybe_unused]] T* const X = M + ((n_moms + 1) & ~1);                                                                 \
+    [[maybe_unused]] T* const cf = X + c.node_region;                                                                      \
+    [[maybe_unused]] T* const tab = cf + a.ntypes * nmus * K;                                                              \
+    [[maybe_unused]] unsigned* const bas = (unsigned*)(smem_raw + c.lds_basic_off);                                        \
+    [[maybe_unused]] const size_t row = (size_t)b * a.P + ii;                                                              \
+    [[maybe_unused]] const int* const first = a.bfirstneigh + row * a.U;                                                   \
+    [[maybe_unused]] const T* const rcs = a.brcs + row * a.U * 3;                                                          \
+    [[maybe_unused]] const int* const types = a.btypes + (size_t)b * NF
+
 template <typename T, int NT>
-__global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> a, const CompArgs<T> c)
+__global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelArgs<T>)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const MtpPlanDevice& p = a.p;
     const int lane = threadIdx.x;
-    const int ii = blockIdx.x, b = blockIdx.y + c.b0;
-    const int NF = a.P;
-    const size_t row = (size_t)b * a.P + ii;
-    const int n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, kmax = p.kmax, K = a.K, E = a.E;
-    const int OX = 0, OY = kmax + 1, OZ = 2 * (kmax + 1), OG = 3 * (kmax + 1), ODG = OG + nmus, OU = ODG + nmus;
-    const int S = p.n_scalar;
-    // moments | node adjoints (+ the zero entry) | coefficients | neighbour table
-    T* M = (T*)smem_raw;
-    T* X = M + ((n_moms + 1) & ~1);
-    T* cf = X + c.node_region;
-    T* tab = cf + a.ntypes * nmus * K;
-    unsigned* bas = (unsigned*)(smem_raw + c.lds_basic_off);
-    const int nn = c.nnc[row];
-    if (ii >= a.binum[b] || nn == 0) {                       // padded or refused row (k_rows flags the reasons)
-        for (int s = lane; s < S; s += NT) c.desc[row * S + s] = (T)0;
-        for (int q = lane; q < 12 * S; q += NT) c.rowpart[row * 12 * S + q] = (T)0;
-        return;
+    const int ii = blockIdx.x, b = blockIdx.y + kernel_args<CompKernelArgs<T>>()->comp.b0;
+    int nn, pair0, center, ti;
+    {
+        COMP_PHASE;
+        nn = c.nnc[row];
+        if (ii >= a.binum[b] || nn == 0) {                       // padded or refused row (k_rows flags the reasons)
+            for (int s = lane; s < S; s += NT) c.desc[row * S + s] = (T)0;
+            for (int q = lane; q < 12 * S; q += NT) c.rowpart[row * 12 * S + q] = (T)0;
+            return;
+        }
+        pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
+        center = a.bilist[row];
+        if ((unsigned)center >= (unsigned)NF) center = 0;
+        ti = types[center];
+        if ((unsigned)ti >= (unsigned)a.ntypes) ti = 0;
+        for (int i = lane; i < n_basic; i += NT)
+            bas[i] = p.basic[i];
+        for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
+        for (int i = lane; i < n_moms; i += NT) M[i] = (T)0;
+        for (int i = lane; i <= p.x_nodes; i += NT) X[i] = (T)0;
     }
-    const int pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
-    int center = a.bilist[row];
-    if ((unsigned)center >= (unsigned)NF) center = 0;
-    const int* types = a.btypes + (size_t)b * NF;
-    int ti = types[center];
-    if ((unsigned)ti >= (unsigned)a.ntypes) ti = 0;
-    const int* first = a.bfirstneigh + row * a.U;
-    const T* rcs = a.brcs + row * a.U * 3;
-    for (int i = lane; i < n_basic; i += NT)
-        bas[i] = p.basic[i];
-    for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
-    for (int i = lane; i < n_moms; i += NT) M[i] = (T)0;
-    for (int i = lane; i <= p.x_nodes; i += NT) X[i] = (T)0;
     __syncthreads();
 
     // basic moments (as in mtp_atom_kernel)
-    const int MTP_NC = c.nc_cap;
+    const int MTP_NC = kernel_args<CompKernelArgs<T>>()->comp.nc_cap;
     const int nchunks = (nn + MTP_NC - 1) / MTP_NC;
     const int chunk = nchunks > 0 ? (nn + nchunks - 1) / nchunks : 1;
     for (int c0 = 0; c0 < nn; c0 += chunk) {
+        COMP_PHASE;
         const int nc = min(chunk, nn - c0);
         int nj; bool valid; T d[3];
         build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
@@ -1358,13 +1376,19 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
         }
         __syncthreads();
     }
-    sweep_forward<T, false>(p.fwd[NT / 256], M, (T*)nullptr, lane);
-    for (int s = lane; s < S; s += NT) {
-        c.desc[row * S + s] = M[p.mapping[s]];
-        if (p.x_root[s] >= 0) X[p.x_root[s]] = (T)1 / a.q_scaler[s];       // (the columns of this launch)
+    {
+        COMP_PHASE;
+        sweep_forward<T, false>(p.fwd[NT / 256], M, (T*)nullptr, lane);
     }
-    __syncthreads();
-    sweep_reverse<T, false>(p.x, M, X, (const T*)nullptr, (const T*)nullptr, lane);
+    {
+        COMP_PHASE;
+        for (int s = lane; s < S; s += NT) {
+            c.desc[row * S + s] = M[p.mapping[s]];
+            if (p.x_root[s] >= 0) X[p.x_root[s]] = (T)1 / a.q_scaler[s];       // (the columns of this launch)
+        }
+        __syncthreads();
+        sweep_reverse<T, false>(p.x, M, X, (const T*)nullptr, (const T*)nullptr, lane);
+    }
 
     // Pair derivatives, four or eight neighbours at a time.  A wavefront forms, for one of them and every basic moment, the vector
     //   D_b = d(g_mu x^a y^b z^c)/dr_j = m (g' - k g / r) u + g / r grad_u m
@@ -1376,30 +1400,39 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
     // group, words and adjoints fetched again for each neighbour and the row sums read back from memory at the end, the
     // kernel took 494 instead of 374 us at level 16, 64 structures of 128 atoms (442 with neighbours one by one and 8-byte
     // reads, 438 with the lists ordered, 384 with pairs of neighbours and 16-byte reads, 374 with eight at a time).
-    const int ngroups = p.x_slots >> 6;
     const int l64 = lane & 63, wv = __builtin_amdgcn_readfirstlane(lane >> 6);
     constexpr int NW = NT / 64;
-    const int plen = n_basic * 6 + 6;                      // D of a pair of neighbours; the last six: their displacements
-    T* D = c.d_over_nodes ? X : (T*)smem_raw + (((tab - (T*)smem_raw) + (size_t)c.nc_cap * E + 1) & ~(size_t)1);
-    const int at_once = min(ngroups, NW), shares = NW / at_once;
-    const int batch = c.batch;
+    int ngroups, at_once, shares, batch, plen;                 // plen: D of a pair of neighbours; the last six their displacements
+    T* D;
+    {
+        COMP_PHASE;
+        ngroups = p.x_slots >> 6;
+        at_once = min(ngroups, NW); shares = NW / at_once;
+        batch = c.batch;
+        plen = n_basic * 6 + 6;
+        D = c.d_over_nodes ? X : (T*)smem_raw + (((tab - (T*)smem_raw) + (size_t)c.nc_cap * E + 1) & ~(size_t)1);
+    }
     for (int g0 = 0; g0 < ngroups; g0 += NW) {
         const int g = g0 + wv % at_once, share = wv / at_once;
         const bool works = share < shares && g < ngroups;   // uniform over the wavefront
-        const int depth = works ? p.x_bdepth[g] : 0, steps = works ? p.x_bsteps[g] : 0;
-        int off[MTP_SLOT_CAP], col = -1, rem = 0;
+        int depth = 0, steps = 0;
+        int off[MTP_SLOT_CAP / 2], col = -1, rem = 0;         // (two places of D to a register, 16 bits each)
         T adj[MTP_SLOT_CAP];
         if (works) {
+            COMP_PHASE;
+            depth = uniform_array(p.x_bdepth)[g];
+            steps = uniform_array(p.x_bsteps)[g];
             const int* wp = p.x_bwords + p.x_bbase[g] + l64;
             col = p.x_seed[g * 64 + l64];
             rem = p.x_brem[g * 64 + l64];
+            int w[MTP_SLOT_CAP];
 #pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k++) off[k] = k < depth ? wp[k * 64] : 0;
+            for (int k = 0; k < MTP_SLOT_CAP; k++) w[k] = k < depth ? wp[k * 64] : 0;
 #pragma unroll
-            for (int k = 0; k < MTP_SLOT_CAP; k++) {
-                adj[k] = k < depth ? X[(unsigned)off[k] & 0xffffu] : (T)0;
-                off[k] = ((unsigned)off[k] >> 16) * 6;
-            }
+            for (int k = 0; k < MTP_SLOT_CAP; k++) adj[k] = k < depth ? X[(unsigned)w[k] & 0xffffu] : (T)0;
+#pragma unroll
+            for (int k = 0; k < MTP_SLOT_CAP; k += 2)
+                off[k / 2] = (int)(((unsigned)w[k] >> 16) * 6 | ((unsigned)w[k + 1] >> 16) * 6 << 16);
         }
         T all[12];                                         // force of the centre (3), virial (9)
 #pragma unroll
@@ -1408,6 +1441,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
             const int nc = min(chunk, nn - c0);
             __syncthreads();                               // the adjoints, or the last batch of D, have been read
             if (nchunks > 1) {                             // (a single chunk's table is still in place)
+                COMP_PHASE;
                 int nj; bool valid; T d[3];
                 build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
                 __syncthreads();
@@ -1415,6 +1449,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
             for (int j0 = 0; j0 < nc; j0 += batch) {
                 if (j0) __syncthreads();
                 for (int jb = wv; jb < min(batch, nc - j0); jb += NW) {
+                    COMP_PHASE;
                     const int j = j0 + jb;
                     const T* t = tab + j * E;
                     T* Dw = D + (jb >> 1) * plen + (jb & 1) * 3;
@@ -1435,6 +1470,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
                 __syncthreads();
                 if (!works) continue;
                 for (int jp = share * 2; jp < min(batch, nc - j0); jp += shares * 2) {
+                    COMP_PHASE;
                     const T* Dp = D + (jp >> 1) * plen;
                     T gr[6];
 #pragma unroll
@@ -1445,7 +1481,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
 #pragma unroll
                             for (int u = k; u < k + 2; u++) {
                                 T dv[6];
-                                load6(Dp + off[u], dv);
+                                load6(Dp + ((unsigned)off[u / 2] >> (u & 1) * 16 & 0xffffu), dv);
 #pragma unroll
                                 for (int q = 0; q < 6; q++) gr[q] += adj[u] * dv[q];
                             }
@@ -1486,12 +1522,14 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const MtpArgs<T> 
             }
         }
         if (works && share == 0 && col >= 0) {
+            COMP_PHASE;
             T* o = c.rowpart + row * 12 * S + col;
 #pragma unroll
             for (int q = 0; q < 12; q++) o[(size_t)q * S] = all[q];
         }
     }
 }
+#undef COMP_PHASE
 
 // rows that the components kernel evaluates, with the checks of mtp_atom_kernel; row_of1[b, atom] = 1 + the row whose
 // centre the atom is
@@ -2854,7 +2892,7 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
             if (lds > 48 * 1024)
                 A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             prof_begin("mtp_components_kernel", stream);
-            hipLaunchKernelGGL(kern, dim3(P, nb), dim3(256), lds, stream, a, c);
+            hipLaunchKernelGGL(kern, dim3(P, nb), dim3(256), lds, stream, CompKernelArgs<T>{a, c});
             prof_end(stream);
         }
         prof_begin("mtp_components_sums", stream);
