@@ -439,14 +439,22 @@ int launch(const NepArgs<T>& a, size_t lds, hipStream_t stream)
     return A2P_OK;
 }
 
-// Atoms of a batch up to which four atoms per wavefront beat the staged kernel's thread per atom, where both have the shape.
-// Whole operator, 6 radial, l_max 4, us (wavefront / staged).  fp32, 16, 36 and 72 neighbours: 40,000 atoms 72 / 162, 85 / 161,
-// 121 / 189; 100,000 138 / 139, 172 / 261, 259 / 432; 200,000 267 / 263, 339 / 514, 489 / 836: always the wavefront (the staged
+// Atoms of a batch up to which four atoms per wavefront (nep_quad.hip) beat the staged kernel's thread per atom, where both have the shape.
+// Whole operator, 6 radial, l_max 4, us (four per wavefront / staged).  fp32, 16, 36 and 72 neighbours: 40,000 atoms 72 / 162, 85 / 161,
+// 121 / 189; 100,000 138 / 139, 172 / 261, 259 / 432; 200,000 267 / 263, 339 / 514, 489 / 836: always the former (the staged
 // kernel keeps the networks too large for its LDS, some 1300 neurons).  fp64, which holds a wavefront per SIMD: 40,000
 // 161 / 146, 194 / 214, 245 / 347; 60,000 225 / 157, 277 / 264, 350 / 426; 100,000 372 / 258, 458 / 447, 563 / 713.  The line
 // moves with the length of the rows, which the host does not know.
 template <typename T>
-constexpr long long wave_most() { return sizeof(T) == 4 ? 1ll << 62 : 49152; }
+constexpr long long quad_most() { return sizeof(T) == 4 ? 1ll << 62 : 49152; }
+
+// Atoms up to which a wavefront per atom beats four atoms per wavefront: its chain is a third shorter, and it repeats most of its
+// instructions for every atom, which costs nothing while a SIMD holds one to three wavefronts (fp32; fp64: one, by registers).
+// Kernel, 16 and 72 neighbours, us (one / four): fp32 108 atoms 12.1 / 16.0 and 16.0 / 23.0, 2000 15.1 / 16.4 and 23.5 / 27.4,
+// 3000 17.9 / 17.1 and 25.9 / 27.1, 4096 24.3 / 17.3 and 34.4 / 27.3; fp64 1000 16.8 / 20.5 and 22.9 / 34.1, 1500 29.7 / 20.6
+// and 37.9 / 35.4.
+template <typename T>
+constexpr long long wave_most() { return sizeof(T) == 4 ? 2560 : 1024; }
 
 template <typename T>
 int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coeffs, const T* w0,
@@ -499,9 +507,13 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     size_t lds_staged = 0;
     const bool staged = !(mb4 || mb5) && nep_staged_supported<T>(a, &lds_staged);
     if (staged) a.nblocks = nep_staged_nblocks(P);
-    // four atoms per wavefront: every shape it has in batches up to wave_most, beyond it those the staged kernel does not have
-    const bool wave = !(mb4 || mb5) && ((long long)B * P < wave_most<T>() || !staged) && nep_wave_supported<T>(a);
-    if (wave) a.nblocks = nep_wave_nblocks<T>(a);
+    // four atoms per wavefront: every shape it has in batches up to quad_most, beyond it those the staged kernel does not have
+    const bool quad = !(mb4 || mb5) && ((long long)B * P < quad_most<T>() || !staged) && nep_quad_supported<T>(a);
+    if (quad) a.nblocks = nep_quad_nblocks<T>(a);
+    // a wavefront per atom: the same shapes in batches up to wave_most
+    size_t lds_wave = 0;
+    const bool wave = !(mb4 || mb5) && ((long long)B * P < wave_most<T>() || (!quad && !staged)) && nep_wave_supported<T>(a, &lds_wave);
+    if (wave) a.nblocks = nep_wave_nblocks(P, B);
 
     void* ws = nullptr;
     int rc = ws_get(WS_FLAGS, 64, &ws);
@@ -515,7 +527,9 @@ int nep_efv(int K, int n_r, int n_a, int l_max, int H, int ntypes, const T* coef
     const size_t force_bytes = (size_t)B * (P + nghost) * 3 * sizeof(T);
 
     if (wave) {
-        return nep_wave_run<T>(a, etot, virial, stream);       // includes the energy / virial sums
+        return nep_wave_run<T>(a, lds_wave, etot, virial, stream);       // includes the energy / virial sums
+    } else if (quad) {
+        return nep_quad_run<T>(a, etot, virial, stream);
     } else if (staged) {
         return nep_staged_run<T>(a, lds_staged, etot, virial, stream);
     } else {

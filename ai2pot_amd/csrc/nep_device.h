@@ -245,13 +245,19 @@ __device__ __forceinline__ void blm_dir_derivs(T x, T y, T z, T wx, T wy, T wz, 
 // whether it applies; nep_staged_run() performs forces' zero-fill, pair counting, the kernel and
 // the pair reduction, whose launch also sums the workgroup partial sums of a.partial (a.nblocks
 // is set by staged_nblocks()) into etot and virial.
-// Four atoms per wavefront (nep_wave.hip); also l_max 3, and any number of species whose tables fit the LDS.
+// Four atoms per wavefront (nep_quad.hip); also l_max 3, and any number of species whose tables fit the LDS.
 template <typename T>
-bool nep_wave_supported(const nepdev::NepArgs<T>& a);
+bool nep_quad_supported(const nepdev::NepArgs<T>& a);
 template <typename T>
-int nep_wave_nblocks(const nepdev::NepArgs<T>& a);
+int nep_quad_nblocks(const nepdev::NepArgs<T>& a);
 template <typename T>
-int nep_wave_run(const nepdev::NepArgs<T>& a, T* etot, T* virial, hipStream_t stream);
+int nep_quad_run(const nepdev::NepArgs<T>& a, T* etot, T* virial, hipStream_t stream);
+// A wavefront per atom (nep_wave.hip), the same shapes, for batches too small to give every SIMD a few wavefronts.
+template <typename T>
+bool nep_wave_supported(const nepdev::NepArgs<T>& a, size_t* lds_bytes);
+int nep_wave_nblocks(int P, int B);
+template <typename T>
+int nep_wave_run(const nepdev::NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream);
 
 template <typename T>
 bool nep_staged_supported(const nepdev::NepArgs<T>& a, size_t* lds_bytes);

@@ -1,27 +1,21 @@
-// NEP energy / force / virial, four atoms per wavefront, for the common model shapes (chebyshev_size 8, n_radial 4 or 6,
-// n_angular 4, l_max 3 or 4) on lists in the padded layout.
+// NEP energy / force / virial, one wavefront per atom, for the common model shapes (chebyshev_size 8, n_radial 4 or 6,
+// n_angular 4, l_max 3 or 4) on lists in the padded layout, for systems of up to some thousand atoms.
 //
-// What bounds it is the issue of vector instructions once a SIMD holds three wavefronts, and an atom's chain of dependent steps
-// before that.  A wavefront per atom (1900 instructions an atom) repeated radial functions and b_lm in every channel's lanes,
-// summed 24 moments over the wavefront, and left lanes idle wherever an atom has fewer than 64 of something.  Here sixteen
-// lanes are an atom's, four atoms share an instruction (3600 for the four), and every step has its own division:
-//   * slots of the row: lane = slot, two in flight per lane; radial sums on the way; pairs inside the angular cutoff are
-//     compacted to the front of the atom's entries in LDS, pairs between the cutoffs to their back;
-//   * angular pairs of all four atoms, 64 at a time: lane = pair, so that each radial function and b_lm is evaluated once; rows
-//     [g | b_lm] in LDS turn them over to
-//   * moments: lane = (atom, channel, quarter of the moments), which runs through the atom's pairs: no sums across lanes;
-//   * hidden layer: lane = neuron, then lane = descriptor for dE/dq;
-//   * angular forces: lane = pair again, from the moments' adjoints contracted over the channels; radial forces: lane = entry.
-// A pair claims its place in its target's reduction segment with one integer atomic (a2p::PairCsr), issued as soon as the
-// pairs are known and waited for behind the read-out (the atomics of all rows take some 5 us at 4096 atoms).  The model's
-// tables lie in LDS once per workgroup.
-// Registers decide how many wavefronts a SIMD holds: each phase takes arguments, LDS addresses and the lane's place anew.  With
-// 60 values spilled for three wavefronts the kernel took 89 us at 20,011 atoms, with two 72, so 58.
+// What bounds such systems is the serial chain of an atom and the first fetch of the code: every SIMD holds three wavefronts at
+// most.  Here every step has its own division over the 64 lanes:
+//   * a row is read once, lane = slot, 128 slots at a time; pairs inside the angular cutoff are compacted to the front of
+//     the wavefront's tile in LDS, pairs between the cutoffs to its back (ballots); a pair claims its place in its
+//     target's reduction segment with one integer atomic (a2p::PairCsr);
+//   * radial functions and radial forces: lane = neighbour (47 of 64 lanes at the benchmark's density);
+//   * angular moments and forces: lane = (neighbour, angular channel), 16 neighbours at a time; a lane holds the 24
+//     moments of its channel, summed over the neighbours with four cross-lane additions;
+//   * hidden layer: lane = neuron, then lane = (descriptor, half of the neurons) for dE/dq.
+// About 1900 vector instructions per atom (6 radial, l_max 4, 48 + 12 neighbours); nep_quad.hip shares most of them between four
+// atoms and takes over where their issue counts.  The model's tables lie in LDS once per workgroup of four wavefronts.
 //
-// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms 34 -> 22 us, 20,011 with
-// skin lists 94 -> 57, 64 structures of 128 atoms 43 -> 25.  Of the 43 thousand cycles of a wavefront at 4096 atoms the tables
-// take 6.4, slots 7, angular pairs and moments 6, read-out 10, angular forces 2.2, radial forces 4.6.  Taken back: two neurons a
-// lane at a time (8 values spilled: 61 us), the neurons of dE/dq by fours (57 -> 58).
+// Measured, fp32, 6 radial functions, l_max 4, 40 neurons, one species: 108 atoms with 72 neighbours 19.6 -> 16.0 us, 1000 22.3 ->
+// 18.3 (fp64 22.7 -> 19.9, 26.4 -> 22.9), by first slots and tables all on their way at the start (0.8 us) and by as many
+// registers as it asks for (with the 128 of four wavefronts per SIMD 42 values are spilled).
 //
 // Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
 #include "a2p_common.h"
@@ -35,75 +29,53 @@ using namespace nepdev;
 using namespace wave;
 namespace {
 
-template <typename T>
-constexpr int wave_cap() { return sizeof(T) == 4 ? 12 : 4; }     // wavefronts of a compute unit: three (fp64: one) per SIMD by registers
-constexpr int NW_ATOMS = 4, NW_LANES = 64 / NW_ATOMS;      // atoms of a wavefront, lanes of an atom
+constexpr int NW_THREADS = 256, NW_WAVES = NW_THREADS / 64;
 constexpr int NW_CAP = 128;                  // slots of a row per tile
-constexpr int NW_TRIPS = NW_CAP / NW_LANES;
 constexpr int KC = 8, NAC = 4;
-constexpr int WROW = 24;                     // row of w0 in LDS: 16-byte reads by 8 lanes with consecutive rows touch
+constexpr int WROW = 28;                     // row of w0 in LDS: 16-byte reads by 8 lanes with consecutive rows touch
                                              // each bank once
 constexpr int CPAD = 4;                      // values behind the coefficients of a species pair (bank spread)
 
-// Shape of the angular part: a lane holds MG moments of a channel, four lanes a channel's (l_max 4: 24, l_max 3: 15 + 1).
-template <int LC>
-struct Angular {
-    static constexpr int NLM = LC * LC + 2 * LC, MG = (NLM + 3) / 4;
-    static constexpr int ROW = NAC + 4 * MG;               // of a pair: g of the channels, b_lm
-    static constexpr int XYZ = 64 * ROW / (3 * NW_ATOMS);  // angular pairs of an atom whose vectors wait there for their turn
-    static constexpr int SCH = 4 * MG, SAT = NAC * SCH + 4;        // moments of a channel, of an atom (banks of the four atoms apart)
-};
-
-// Where things lie in LDS, in bytes: the model's tables of the workgroup (w0 first), behind them `own` bytes for each wavefront.
-struct WaveAt {
-    int coef, b0, w1, qs, cw, bias, shared;        // (cw: w_m C_lm of the 24 moments)
-    int own, rows, ang, mom, cc, q, dq, sde;       // of a wavefront, whose entries come first; mom .. sde in the place of rows
-};
-template <typename T, int LC>
-WaveAt wave_at(int nt, int H, int nb)
-{
-    typedef Angular<LC> A;
-    static_assert(64 * A::ROW * sizeof(T) >= 64 * 10 * sizeof(double), "room for the sums at the end");
-    WaveAt at;
-    size_t off = 0;
-    auto take = [&](size_t n, size_t size) { const int at = (int)off; off += (n * size + 15) / 16 * 16; return at; };
-    take((size_t)nt * H * WROW, sizeof(T));
-    at.coef = take((size_t)nt * nt * (nb * KC + CPAD), sizeof(T));
-    at.b0 = take((size_t)nt * H, sizeof(T));
-    at.w1 = take((size_t)nt * H, sizeof(T));
-    at.qs = take(WROW, sizeof(T));
-    at.cw = take(4 * A::MG, sizeof(T));
-    at.bias = take((size_t)nt, sizeof(T));
-    at.shared = (int)std::min(off, (size_t)1 << 20);      // (beyond the LDS in any case)
-    off = 0;
-    take(NW_ATOMS * NW_CAP, sizeof(int2));
-    at.rows = at.mom = take(NW_ATOMS * A::SAT, sizeof(T));
-    at.cc = take((size_t)NW_ATOMS * nt * KC, sizeof(T));
-    at.q = take(NW_ATOMS * WROW, sizeof(T));
-    at.dq = take(NW_ATOMS * WROW, sizeof(T));
-    at.sde = take((size_t)NW_ATOMS * ((H + 3) / 4 * 4), sizeof(T));
-    off = std::max(off, at.rows + 64 * A::ROW * sizeof(T));
-    at.ang = take(64 * 3, sizeof(T));
-    at.own = (int)std::min(off, (size_t)1 << 20);
-    return at;
-}
 template <typename T>
 struct WaveLds {
-    T *w0, *coef, *b0, *w1, *qs, *cw, *bias;
-    int2* ent;                       // pairs of the four atoms' tiles (neighbour, later its place; slot | species << 16)
-    T *rows, *ang;                   // angular pairs for the moments; their forces
-    T *mom, *cc;                     // moments' adjoints; radial coefficients contracted with dE/dq
-    T *q, *dq, *sde;                 // of the read-out
-    template <typename At>
-    __device__ __forceinline__ WaveLds(const At& at, unsigned char* base, int wave)
-    {
-        w0 = (T*)base; coef = (T*)(base + at.coef); b0 = (T*)(base + at.b0); w1 = (T*)(base + at.w1); qs = (T*)(base + at.qs);
-        cw = (T*)(base + at.cw); bias = (T*)(base + at.bias);
-        unsigned char* const mine = base + at.shared + at.own * wave;
-        ent = (int2*)mine; rows = (T*)(mine + at.rows); ang = (T*)(mine + at.ang); mom = (T*)(mine + at.mom); cc = (T*)(mine + at.cc);
-        q = (T*)(mine + at.q); dq = (T*)(mine + at.dq); sde = (T*)(mine + at.sde);
-    }
+    T *w0, *coef, *b0, *w1, *qs;     // model tables, shared by the workgroup
+    double* red;
+    T *ent, *ang, *q, *dq, *sde, *cc;       // of the wavefront: tile, angular forces of its front, read-out scratch
+    int* pos;
 };
+
+template <typename T>
+__host__ __device__ __forceinline__ size_t wave_lds_layout(int nt, int H, int nb, int wave, unsigned char* base,
+                                                           WaveLds<T>& L)
+{
+    size_t off = 0;
+    auto take = [&](size_t n, size_t size) {
+        unsigned char* p = base + off;
+        off += (n * size + 15) / 16 * 16;
+        return p;
+    };
+    L.w0 = (T*)take((size_t)nt * H * WROW, sizeof(T));
+    L.coef = (T*)take((size_t)nt * nt * (nb * KC + CPAD), sizeof(T));
+    L.b0 = (T*)take((size_t)nt * H, sizeof(T));
+    L.w1 = (T*)take((size_t)nt * H, sizeof(T));
+    L.qs = (T*)take(WROW, sizeof(T));
+    L.red = (double*)take(NW_WAVES * 10, sizeof(double));
+    const size_t shared = off;
+    L.ent = (T*)take(NW_CAP * 4, sizeof(T));
+    L.ang = (T*)take(NW_CAP * 3, sizeof(T));
+    L.pos = (int*)take(NW_CAP, sizeof(int));
+    L.q = (T*)take(WROW, sizeof(T));
+    L.dq = (T*)take(WROW, sizeof(T));
+    L.sde = (T*)take(H, sizeof(T));
+    L.cc = (T*)take(nt * KC, sizeof(T));
+    const size_t own = off - shared;
+    const size_t shift = own * wave;
+    L.ent = (T*)((unsigned char*)L.ent + shift); L.ang = (T*)((unsigned char*)L.ang + shift);
+    L.pos = (int*)((unsigned char*)L.pos + shift); L.q = (T*)((unsigned char*)L.q + shift);
+    L.dq = (T*)((unsigned char*)L.dq + shift); L.sde = (T*)((unsigned char*)L.sde + shift);
+    L.cc = (T*)((unsigned char*)L.cc + shift);
+    return shared + own * NW_WAVES;
+}
 
 struct SegArgs {
     int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
@@ -112,688 +84,395 @@ struct SegArgs {
     int mark;      // own sums are marked in the cursors (PairCsr)
 };
 
-// N values (N even) behind an address aligned to two of them
-template <typename T, int N>
-__device__ __forceinline__ void lds_load_even(const T* p, T (&o)[N])
+// Slots [128 t, 128 t + 128) of a row, of which `room` are read: lane = slot, both halves in flight.
+template <typename T>
+struct Slots {
+    int nj[2];
+    T x[2], y[2], z[2];
+};
+template <typename T>
+__device__ __forceinline__ void load_slots(const NepArgs<T>& a, int t, int lane, size_t row, int room, Slots<T>& o)
 {
-    typedef T Two __attribute__((ext_vector_type(2)));
 #pragma unroll
-    for (int i = 0; i < N; i += 2) {
-        const Two v = *reinterpret_cast<const Two*>(p + i);
-        o[i] = v.x; o[i + 1] = v.y;
+    for (int h = 0; h < 2; h++) {
+        const int slot = t * NW_CAP + h * 64 + lane;
+        o.nj[h] = -1;
+        o.x[h] = o.y[h] = o.z[h] = (T)0;
+        if (slot < room) {
+            const size_t pr = row * a.U + slot;
+            o.nj[h] = a.bfirstneigh[pr];
+            const T* p = a.brcs + pr * 3;
+            o.x[h] = p[0]; o.y[h] = p[1]; o.z[h] = p[2];
+        }
     }
 }
-
-// r and 1 / r from r^2: the estimate of 1 / r and a Newton step for each, a third of the operations of square root and
-// division.  r^2 = 0 gives NaN, as 0 / 0 does; MIN keeps it from that.
-template <bool MIN>
-__device__ __forceinline__ float length(float d2, float& rinv)
+// They into the wavefront's tile; nA / nR: entries at its front / back.
+template <typename T>
+__device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& seg, T* __restrict__ seg_g,
+                                          const WaveLds<T>& L, int t, int lane, size_t row, int b, int NF, int nn, T rr,
+                                          T ra, bool claim, const Slots<T>& in, int& nA, int& nR)
 {
-    if (MIN) d2 = d2 < 1e-30f ? 1e-30f : d2;                    // (NaN stays)
-    const float y = __builtin_amdgcn_rsqf(d2), r0 = d2 * y;
-    const float r = r0 + (d2 - r0 * r0) * (0.5f * y);
-    rinv = y + y * (1.0f - r * y);
-    return r;
-}
-template <bool MIN>
-__device__ __forceinline__ double length(double d2, double& rinv)
-{
-    const double r = sqrt(d2);
-    rinv = 1.0 / r;
-    return r;
-}
-
-// What a lane of the wavefront wrote to LDS is read by the others behind this.
-__device__ __forceinline__ void wave_sync()
-{
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    const int* types = a.btypes + (size_t)b * NF;
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    nA = 0; nR = 0;
+    const int (&nj)[2] = in.nj;
+    const T (&x)[2] = in.x, (&y)[2] = in.y, (&z)[2] = in.z;
+    int tj[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int slot = t * NW_CAP + h * 64 + lane;
+        const bool bad = slot < nn && (unsigned)nj[h] >= (unsigned)NF;
+        if (bad) atomicOr(a.status, ST_BAD_NEIGHBOR);
+        tj[h] = -1;
+        if (slot < nn && !bad) tj[h] = types[nj[h]];
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        if (t * NW_CAP + h * 64 >= nn) break;          // uniform
+        const int slot = t * NW_CAP + h * 64 + lane;
+        const bool valid = slot < nn && (unsigned)nj[h] < (unsigned)NF;
+        if (valid && (unsigned)tj[h] >= (unsigned)a.ntypes) { atomicOr(a.status, ST_BAD_TYPE); tj[h] = 0; }
+        const T r = sqrt_t(x[h] * x[h] + y[h] * y[h] + z[h] * z[h]);
+        const bool inA = valid && r <= ra && r <= rr;   // nepBasis.h:106, 135: beyond the radial cutoff a neighbour is skipped
+        const bool inR = valid && !inA && r <= rr;
+        int pos = 0;
+        // A pair beyond the cutoffs (a list with a skin) needs no place in this call; when the places are kept with
+        // the list it has one all the same and stores a zero.
+        if (valid && claim && seg.cursor && (inA || inR || a.brank)) {
+            const size_t pr = row * a.U + slot;
+            const int tg = b * NF + nj[h];
+            int rk;
+            if (a.brank && a.ranks_valid) {
+                rk = a.brank[pr];
+            } else {
+                rk = pair_claim(&seg.cursor[tg]);
+                if (a.brank) a.brank[pr] = rk;
+            }
+            pos = (unsigned)rk < (unsigned)seg.cap ? tg * seg.cap + rk : seg.spare;
+            if ((unsigned)rk >= (unsigned)seg.cap) atomicOr(a.status, ST_SEG_OVERFLOW);
+            if (!(inA || inR)) {
+                T* dst = seg_g + (size_t)pos * 3;
+                dst[0] = (T)0; dst[1] = (T)0; dst[2] = (T)0;
+            }
+        }
+        const unsigned long long mA = __ballot(inA), mR = __ballot(inR);
+        if (inA || inR) {
+            const int k = inA ? nA + __popcll(mA & lt) : NW_CAP - 1 - (nR + __popcll(mR & lt));
+            ent_store(L.ent + k * 4, x[h], y[h], z[h], tj[h]);
+            L.pos[k] = pos;
+        }
+        nA += __popcll(mA);
+        nR += __popcll(mR);
+    }
     __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-__device__ __forceinline__ int of_atom(int v, int g) { return __builtin_amdgcn_readlane(v, g * NW_LANES); }
-__device__ __forceinline__ int most_of_atoms(int v) { return max(max(of_atom(v, 0), of_atom(v, 1)), max(of_atom(v, 2), of_atom(v, 3))); }
-__device__ __forceinline__ int pick(int g, int v0, int v1, int v2, int v3) { return g < 2 ? (g == 0 ? v0 : v1) : (g == 2 ? v2 : v3); }
-
-template <typename T>
-__device__ __forceinline__ T row_sum(T v)          // the sixteen lanes of a row
-{
-    v += dpp_move<0x128>(v);                       // row_ror: 8, 4, 2, 1
-    v += dpp_move<0x124>(v);
-    v += dpp_move<0x122>(v);
-    return v + dpp_move<0x121>(v);
-}
-
-template <typename T>
-struct WaveArgs {
-    NepArgs<T> nep;
-    SegArgs seg;
-    T* seg_g;
-    WaveAt at;
-};
-// The lane's place, found anew by each phase as well (again() of a2p_common.h): what the phases derive from it does not fit the registers
-// of three wavefronts per SIMD either.
-__device__ __forceinline__ int lane_again()
-{
-    int lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-    asm volatile("" : "+v"(lane));
-    return lane;
-}
-#define NW_PHASE                                                                                                            \
-    [[maybe_unused]] auto& K_ = again(kernel_args<WaveArgs<T>>());                                                          \
-    [[maybe_unused]] auto& a = K_.nep;                                                                                      \
-    [[maybe_unused]] auto& seg = K_.seg;                                                                                    \
-    [[maybe_unused]] const WaveLds<T> L(K_.at, smem_raw, wave);                                                         \
-    [[maybe_unused]] const int H = a.H, nt = a.ntypes, U = a.U, NF = a.P + a.nghost;                                    \
-    [[maybe_unused]] const int lane = lane_again();                                                                     \
-    [[maybe_unused]] const int g = lane / NW_LANES, s = lane % NW_LANES;       /* atom of the wavefront, lane of the atom */\
-    [[maybe_unused]] const int chan = s & 3, mg = s >> 2;                      /* angular channel, MG of its moments */ \
-    [[maybe_unused]] int2* const ent = L.ent + g * NW_CAP
 
 template <typename T, int NR, int LC>
-__global__ void __launch_bounds__(64 * wave_cap<T>(), sizeof(T) == 4 ? 3 : 1)
-nep_wave_kernel(const WaveArgs<T>)
+__global__ void __launch_bounds__(NW_THREADS, 1)
+nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
 {
-    typedef Angular<LC> A;
-    constexpr int NLM = A::NLM, MG = A::MG, XYZ = A::XYZ, NB = NR + NAC, D = NR + NAC * LC, CROW = NB * KC + CPAD;
-    static_assert(D <= WROW && D <= 16 + 8, "descriptor count exceeds the padded row or the lanes of dE/dq");
+    constexpr int NLM = LC * LC + 2 * LC, NB = NR + NAC, D = NR + NAC * LC, CROW = NB * KC + CPAD;
+    static_assert(D <= WROW, "descriptor count exceeds the padded row");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.y;
-    int inum;
-    bool derivs, claims;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int b = blockIdx.y, H = a.H, nt = a.ntypes, NF = a.P + a.nghost;
+    WaveLds<T> L;
+    wave_lds_layout<T>(nt, H, NB, wave, smem_raw, L);
+
+    // What the wavefront's first atom begins with, on its way while the tables are: the atom, its number of neighbours, its
+    // first 128 slots (whether they hold a neighbour or not).
+    const int first = blockIdx.x * NW_WAVES + wave;
+    const size_t row1 = (size_t)b * a.P + min(first, a.P - 1);
+    const int center1 = a.bilist[row1], nn1 = a.bnumneigh[row1];
+    Slots<T> slots;
+    load_slots<T>(a, 0, lane, row1, a.U, slots);
     {
-        NW_PHASE;
-        inum = min(a.binum[b], a.P);                  // (the loop below strides over the rows: none beyond the last)
-        derivs = a.force != nullptr || a.want_virial;
-        claims = derivs && seg.cursor;
+        // The model's tables: the first values of every thread are all on their way before one is stored.
+        constexpr int W0 = sizeof(T) == 4 ? 16 : 8, C0 = 4;
+        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
+        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
+        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
+        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
+#pragma unroll
+        for (int u = 0; u < C0; u++) { const int i = tid + u * NW_THREADS; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
+#pragma unroll
+        for (int u = 0; u < W0; u++) { const int i = tid + u * NW_THREADS; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
+        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
+        if (tid < D) qs = a.q_scaler[tid];
+#pragma unroll
+        for (int u = 0; u < C0; u++) { const int i = tid + u * NW_THREADS; if (i < nc) put_coef(i, c0[u]); }
+#pragma unroll
+        for (int u = 0; u < W0; u++) { const int i = tid + u * NW_THREADS; if (i < nw0) put_w0(i, w0[u]); }
+        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
+        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
+        for (int i = tid + C0 * NW_THREADS; i < nc; i += NW_THREADS) put_coef(i, a.coeffs[i]);
+        for (int i = tid + W0 * NW_THREADS; i < nw0; i += NW_THREADS) put_w0(i, a.w0[i]);
+        for (int i = tid + NW_THREADS; i < nh; i += NW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
     }
+    __syncthreads();
+
+    const int inum = min(a.binum[b], a.P);            // (the loop below strides over the rows: none beyond the last)
+    const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
+    const bool derivs = a.force != nullptr || a.want_virial;
+    const int quad = lane >> 2, chan = lane & 3;       // neighbour within a round of 16, angular channel
     double e_sum = 0.0, v_sum[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) v_sum[i] = 0.0;
 
-    // What the next four rows begin with, on its way while the rows before are worked on: the atom, its number of neighbours,
-    // the first 2 * STEP slots (whether they hold a neighbour or not).
-    constexpr int V = 2, STEP = V * NW_LANES;              // slots of a lane in flight, of an atom per trip
-    int center1, nn1, nj[V], nj1[V];
-    T x[V], y[V], z[V], x1[V], y1[V], z1[V];
-    auto load = [&](int base, int room, int slot0, int (&n)[V], T (&px)[V], T (&py)[V], T (&pz)[V]) __attribute__((always_inline)) {
-        NW_PHASE;
-#pragma unroll
-        for (int v = 0; v < V; v++) {
-            const int slot = slot0 + v * NW_LANES + s;
-            n[v] = -1; px[v] = py[v] = pz[v] = (T)0;
-            if (slot < room) {
-                n[v] = a.bfirstneigh[base + slot];
-                const T* p = a.brcs + (size_t)(base + slot) * 3;
-                px[v] = p[0]; py[v] = p[1]; pz[v] = p[2];
-            }
-        }
-    };
-    auto begin = [&](int i0) __attribute__((always_inline)) {
-        NW_PHASE;
-        const int row = b * a.P + min(i0 + g, a.P - 1);
-        center1 = a.bilist[row];
-        nn1 = a.bnumneigh[row];
-        load(row * U, U, 0, nj, x, y, z);
-        load(row * U, U, STEP, nj1, x1, y1, z1);
-    };
-    const int nwaves = blockDim.x >> 6, first = NW_ATOMS * (wave * gridDim.x + blockIdx.x), stride = NW_ATOMS * nwaves * gridDim.x;
-    begin(first);
-    {
-        // The model's tables: the first values of every thread are all on their way before one is stored.
-        NW_PHASE;
-        const int tid = threadIdx.x, nthreads = blockDim.x;
-        constexpr int W0 = 16, C0 = 4;
-        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
-        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1, bias = (T)0;
-        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
-        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
-        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
-        if (tid < nt) bias = a.bias[tid];
-        if (tid < D) qs = a.q_scaler[tid];
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; if (i < nc) put_coef(i, c0[u]); }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; if (i < nw0) put_w0(i, w0[u]); }
-        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
-        if (tid < nt) L.bias[tid] = bias;
-        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
-        if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)kC3B[tid] : (T)0;
-        for (int i = tid + C0 * nthreads; i < nc; i += nthreads) put_coef(i, a.coeffs[i]);
-        for (int i = tid + W0 * nthreads; i < nw0; i += nthreads) put_w0(i, a.w0[i]);
-        for (int i = tid + nthreads; i < nh; i += nthreads) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
-        for (int i = tid + nthreads; i < nt; i += nthreads) L.bias[i] = a.bias[i];
-    }
-    __syncthreads();
+    for (int ii = first; ii < inum; ii += gridDim.x * NW_WAVES) {
+        const size_t row = (size_t)b * a.P + ii;
+        int center = ii == first ? center1 : a.bilist[row], nn = ii == first ? nn1 : a.bnumneigh[row];
+        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
+        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
+        int ti = a.btypes[(size_t)b * NF + center];
+        if ((unsigned)ti >= (unsigned)nt) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
+        const int ntiles = (nn + NW_CAP - 1) / NW_CAP;
+        const T* const cti = L.coef + (size_t)ti * nt * CROW;
 
-    for (int i0 = first; i0 < inum; i0 += stride) {
-        int center = center1, nn = nn1, ti, base0;
-        {
-            NW_PHASE;
-            const bool act = i0 + g < inum;
-            base0 = (b * a.P + min(i0 + g, a.P - 1)) * U;                    // first pair of the row (pairs: below 2^31)
-            if (!act) { center = 0; nn = 0; }
-            if (nn > U) { if (s == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = U; }
-            if ((unsigned)center >= (unsigned)NF) { if (s == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-            ti = a.btypes[(size_t)b * NF + center];
-            if ((unsigned)ti >= (unsigned)nt) { if (s == 0 && act) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
-        }
-        const int ntiles = max(1, (most_of_atoms(nn) + NW_CAP - 1) / NW_CAP);
-        const int ti0 = of_atom(ti, 0), ti1 = of_atom(ti, 1), ti2 = of_atom(ti, 2), ti3 = of_atom(ti, 3);
-
-        T S[MG], q[NR];
+        // ---- radial sums, angular moments ------------------------------------------------------------
+        T S[NLM], q[NR];
 #pragma unroll
-        for (int m = 0; m < MG; m++) S[m] = (T)0;
+        for (int m = 0; m < NLM; m++) S[m] = (T)0;
 #pragma unroll
         for (int n = 0; n < NR; n++) q[n] = (T)0;
-        T fx = (T)0, fy = (T)0, fz = (T)0;
-
-        // Tile by tile for the sums (mom), behind the last one the read-out, from the last one on tile by tile for the
-        // forces (frc).  Rows of one tile, nearly all, are passed once.
-        for (int jt = 0; jt < (derivs ? 2 * ntiles - 1 : ntiles); jt++) {
-            const int t = jt < ntiles ? jt : jt - ntiles;
-            const bool mom = jt < ntiles, frc = derivs && jt >= ntiles - 1;
-            const bool claim = frc && claims;
-            const int base = base0 + t * NW_CAP;
-            const int tn = min(max(nn - t * NW_CAP, 0), NW_CAP);
-
-            // ---- slots of the tile: radial sums; pairs inside the angular cutoff to the front of the atom's entries, pairs
-            // between the cutoffs to their back
-            int nA = 0, nR = 0;
-            {
-                NW_PHASE;
-                T* const seg_g = K_.seg_g;
-                const T* const cti = L.coef + ti * nt * CROW;
-                const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr;
-                const int* const types = a.btypes + (size_t)b * NF;
-                const unsigned below = (1u << s) - 1u;
-                const int room = min(U - t * NW_CAP, NW_CAP);
-                if (jt > 0) {
-                    load(base, room, 0, nj, x, y, z);
-                    load(base, room, STEP, nj1, x1, y1, z1);
-                }
-                auto species = [&](int nj) __attribute__((always_inline)) { return (unsigned)nj < (unsigned)NF ? types[nj] : 0; };
-                const int trips = (most_of_atoms(tn) + STEP - 1) / STEP;
-                int tj[V], tj1[V];
+        int nA = 0, nR = 0;
+        for (int t = 0; t < ntiles; t++) {
+            // (a row of several tiles is read again for the forces, and its pairs claim their places then)
+            if (t > 0 || ii != first) load_slots<T>(a, t, lane, row, nn, slots);
+            load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, ntiles == 1, slots, nA, nR);
+            for (int e = lane; e < nA + nR; e += 64) {
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + (e < nA ? e : NW_CAP - 1 - (e - nA)) * 4, x, y, z, tj);
+                T f[KC], df[KC];
+                radial_basis<T, KC, false>(sqrt_t(x * x + y * y + z * z), rr_inv, KC, f, df);
+                const T* c = cti + tj * CROW;
 #pragma unroll
-                for (int v = 0; v < V; v++) tj[v] = species(nj[v]);
-#pragma unroll 1
-                for (int k = 0; k < trips; k++) {
-                    const int slot0 = k * STEP + s;
-                    int nj2[V];
-                    T x2[V], y2[V], z2[V];
-                    load(base, tn, (k + 2) * STEP, nj2, x2, y2, z2);
+                for (int n = 0; n < NR; n++) {
+                    T c0[4], c1[4];
+                    lds_load4(c + n * KC, c0);
+                    lds_load4(c + n * KC + 4, c1);
 #pragma unroll
-                    for (int v = 0; v < V; v++) tj1[v] = species(nj1[v]);
-                    bool valid[V], inA[V], inR[V];
-                    T r[V];
+                    for (int k = 0; k < 4; k++) q[n] += c0[k] * f[k];
 #pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        valid[v] = slot0 + v * NW_LANES < tn;
-                        if (valid[v] && (unsigned)nj[v] >= (unsigned)NF) { atomicOr(a.status, ST_BAD_NEIGHBOR); valid[v] = false; }
-                        if (valid[v] && (unsigned)tj[v] >= (unsigned)nt) { atomicOr(a.status, ST_BAD_TYPE); tj[v] = 0; }
-                        T unused;
-                        r[v] = length<true>(x[v] * x[v] + y[v] * y[v] + z[v] * z[v], unused);
-                        inA[v] = valid[v] && r[v] <= ra && r[v] <= rr;   // nepBasis.h:106, 135: beyond the radial cutoff a neighbour is skipped
-                        inR[v] = valid[v] && !inA[v] && r[v] <= rr;
-                    }
-                    if (mom) {
-                        T f[V][KC], df[KC];
-#pragma unroll
-                        for (int v = 0; v < V; v++) {
-                            radial_basis<T, KC, false>(r[v], rr_inv, KC, f[v], df);
-#pragma unroll
-                            for (int i = 0; i < KC; i++) f[v][i] = inA[v] || inR[v] ? f[v][i] : (T)0;
-                        }
-#pragma unroll
-                        for (int n = 0; n < NR; n++) {
-#pragma unroll
-                            for (int v = 0; v < V; v++) {
-                                T c0[4], c1[4];
-                                lds_load4(cti + tj[v] * CROW + n * KC, c0);
-                                lds_load4(cti + tj[v] * CROW + n * KC + 4, c1);
-                                T u = (T)0;
-#pragma unroll
-                                for (int i = 0; i < 4; i++) u += c0[i] * f[v][i];
-#pragma unroll
-                                for (int i = 0; i < 4; i++) u += c1[i] * f[v][4 + i];
-                                q[n] += u;
-                            }
-                        }
-                    }
-#pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        const int slot = slot0 + v * NW_LANES;
-                        // A pair beyond the cutoffs (a list with a skin) needs no place in this call; when the places are
-                        // kept with the list it has one all the same and stores a zero.
-                        if (claim && a.brank && valid[v] && !inA[v] && !inR[v]) {
-                            const int tg = b * NF + nj[v];
-                            int rk;
-                            if (a.ranks_valid) rk = a.brank[base + slot];
-                            else a.brank[base + slot] = rk = pair_claim(&seg.cursor[tg]);
-                            if ((unsigned)rk >= (unsigned)seg.cap) atomicOr(a.status, ST_SEG_OVERFLOW);
-                            T* dst = seg_g + (size_t)((unsigned)rk < (unsigned)seg.cap ? tg * seg.cap + rk : seg.spare) * 3;
-                            dst[0] = (T)0; dst[1] = (T)0; dst[2] = (T)0;
-                        }
-                        const unsigned long long bA = __ballot(inA[v]), bR = __ballot(inR[v]);
-                        const unsigned mA = (unsigned)(bA >> (g * NW_LANES)) & 0xffffu, mR = (unsigned)(bR >> (g * NW_LANES)) & 0xffffu;
-                        if (mom && inA[v]) {                       // (behind the read-out its results lie there)
-                            const int k = nA + __popc(mA & below);
-                            if (k < XYZ) {
-                                T* const p = L.rows + (g * XYZ + k) * 3;
-                                p[0] = x[v]; p[1] = y[v]; p[2] = z[v];
-                            }
-                        }
-                        if (inA[v] || inR[v])
-                            ent[inA[v] ? nA + __popc(mA & below) : NW_CAP - 1 - (nR + __popc(mR & below))] = make_int2(nj[v], slot | tj[v] << 16);
-                        nA += __popc(mA);
-                        nR += __popc(mR);
-                    }
-#pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        nj[v] = nj1[v]; x[v] = x1[v]; y[v] = y1[v]; z[v] = z1[v]; tj[v] = tj1[v];
-                        nj1[v] = nj2[v]; x1[v] = x2[v]; y1[v] = y2[v]; z1[v] = z2[v];
-                    }
+                    for (int k = 0; k < 4; k++) q[n] += c1[k] * f[4 + k];
                 }
             }
-            wave_sync();
-            const int n_own = nA + nR, n_most = most_of_atoms(n_own);
-            auto entry = [&](int e) __attribute__((always_inline)) { return e < nA ? e : NW_CAP - 1 - (e - nA); };
+            for (int e0 = 0; e0 < nA; e0 += 16) {
+                const int e = e0 + quad;
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                T f[KC], df[KC];
+                radial_basis<T, KC, false>(r, ra_inv, KC, f, df);
+                T c0[4], c1[4], g = (T)0;
+                lds_load4(cti + tj * CROW + (NR + chan) * KC, c0);
+                lds_load4(cti + tj * CROW + (NR + chan) * KC + 4, c1);
+#pragma unroll
+                for (int k = 0; k < 4; k++) g += c0[k] * f[k];
+#pragma unroll
+                for (int k = 0; k < 4; k++) g += c1[k] * f[4 + k];
+                if (e >= nA) g = (T)0;
+                T bl[NLM];
+                blm_values<T, LC>(x * rinv, y * rinv, z * rinv, bl);
+#pragma unroll
+                for (int m = 0; m < NLM; m++) S[m] += g * bl[m];
+            }
+            __builtin_amdgcn_wave_barrier();          // the tile is overwritten by the next one
+        }
+#pragma unroll
+        for (int n = 0; n < NR; n++) q[n] = all_sum(q[n]);
+#pragma unroll
+        for (int m = 0; m < NLM; m++) S[m] = sum_over_quads(S[m]);
 
-            // ---- angular pairs, 64 at a time over the four atoms
-            const int n0 = of_atom(nA, 0), n1 = of_atom(nA, 1), n2 = of_atom(nA, 2), n3 = of_atom(nA, 3);
-            const int o1 = n0, o2 = n0 + n1, o3 = o2 + n2, total = o3 + n3;
-            const int nch = max(1, (total + 63) / 64);
-            const bool xyz_held = mom && max(max(n0, n1), max(n2, n3)) <= XYZ;
-            int rk[NW_TRIPS];
-            for (int it = 0; it < nch + (mom && frc ? nch - 1 : 0); it++) {
-                const int c0 = (it < nch ? it : it - nch) * 64;
-                const int p = c0 + lane_again();
-                // -- lane = pair: direction, radial functions, b_lm
-                const int pg = (p >= o1) + (p >= o2) + (p >= o3);
-                const bool on = p < total;
-                T ux = (T)0, uy = (T)0, uz = (T)0, rinv = (T)0, ga[NAC], dg[NAC];
+        // ---- descriptors: the radial ones in every lane, the angular ones of a channel in its lanes -----------
 #pragma unroll
-                for (int c = 0; c < NAC; c++) ga[c] = dg[c] = (T)0;
-                if (on) {
-                    NW_PHASE;
-                    const int row0 = b * a.P + i0;
-                    const T ra_inv = (T)1 / a.ra;
-                    const int w = L.ent[pg * NW_CAP + (p - pick(pg, 0, o1, o2, o3))].y;
-                    T x, y, z;
-                    if (it == 0 && xyz_held) {
-                        const T* const xp = L.rows + (pg * XYZ + (p - pick(pg, 0, o1, o2, o3))) * 3;
-                        x = xp[0]; y = xp[1]; z = xp[2];
-                    } else {
-                        const T* const xp = a.brcs + (size_t)((row0 + pg) * U + t * NW_CAP + (w & 0xffff)) * 3;
-                        x = xp[0]; y = xp[1]; z = xp[2];
-                    }
-                    const T r = length<false>(x * x + y * y + z * z, rinv);
-                    ux = x * rinv; uy = y * rinv; uz = z * rinv;
-                    T f[KC], df[KC];
-                    radial_basis<T, KC, true>(r, ra_inv, KC, f, df);
-                    const T* c = L.coef + (size_t)(pick(pg, ti0, ti1, ti2, ti3) * nt + (w >> 16)) * CROW + NR * KC;
+        for (int n = 0; n < NR; n++)
+            if (lane == n) L.q[n] = q[n];
+        // q_{n,l} = sum_m w_m C_lm S^2  (nepBasis.h:174-190)
 #pragma unroll
-                    for (int n = 0; n < NAC; n++) {
-                        T v0[4], v1[4];
-                        lds_load4(c + n * KC, v0);
-                        lds_load4(c + n * KC + 4, v1);
+        for (int l = 1; l <= LC; l++) {
+            T acc = (T)0;
 #pragma unroll
-                        for (int i = 0; i < 4; i++) { ga[n] += v0[i] * f[i]; dg[n] += v0[i] * df[i]; }
-#pragma unroll
-                        for (int i = 0; i < 4; i++) { ga[n] += v1[i] * f[4 + i]; dg[n] += v1[i] * df[4 + i]; }
-                    }
-                }
-                if (claim && it == (mom ? nch - 1 : 0)) {
-                    // -- the pairs claim their places; the answers are stored when the forces' turn comes (the loads above
-                    // would wait for them)
-                    NW_PHASE;
-#pragma unroll
-                    for (int k = 0; k < NW_TRIPS; k++) {
-                        const int e = k * NW_LANES + s;
-                        rk[k] = 0;
-                        if (k * NW_LANES < n_most && e < n_own) {
-                            const int2 w = ent[entry(e)];
-                            if (a.brank && a.ranks_valid) rk[k] = a.brank[base + (w.y & 0xffff)];
-                            else rk[k] = pair_claim_raw(&seg.cursor[b * NF + w.x]);
-                        }
-                    }
-                }
-                if (mom && it < nch) {
-                    NW_PHASE;
-                    // -- moments: lane = (atom, channel, MG of the moments), the atom's pairs one after the other
-                    wave_sync();
-                    if (on) {
-                        T bl[NLM];
-                        blm_values<T, LC>(ux, uy, uz, bl);
-                        T* const rw = L.rows + lane * A::ROW;
-                        lds_store4(rw, ga[0], ga[1], ga[2], ga[3]);
-#pragma unroll
-                        for (int m = 0; m < 4 * MG; m += 4)
-                            lds_store4(rw + NAC + m, bl[m], bl[m + 1], bl[m + 2], m + 3 < NLM ? bl[m + 3 < NLM ? m + 3 : 0] : (T)0);
-                    }
-                    wave_sync();
-                    const int o_own = pick(g, 0, o1, o2, o3), lo = max(o_own, c0) - c0, n = max(min(o_own + nA, c0 + 64) - c0 - lo, 0), trips = most_of_atoms(n);
-                    if (n > 0) {
-                        const T* const rw = L.rows + lo * A::ROW;
-                        for (int k0 = 0; k0 < trips; k0 += 4) {
-                            T gc[4], bm[4][MG];
-#pragma unroll
-                            for (int u = 0; u < 4; u++) {
-                                const T* const r = rw + min(k0 + u, n - 1) * A::ROW;
-                                gc[u] = r[chan];
-                                lds_load_even(r + NAC + mg * MG, bm[u]);
-                            }
-#pragma unroll
-                            for (int u = 0; u < 4; u++) gc[u] = k0 + u < n ? gc[u] : (T)0;
-#pragma unroll
-                            for (int m = 0; m < MG; m++)
-                                S[m] += (gc[0] * bm[0][m] + gc[1] * bm[1][m]) + (gc[2] * bm[2][m] + gc[3] * bm[3][m]);
-                        }
-                    }
-                    wave_sync();
-                }
-                if (mom && jt == ntiles - 1 && it == nch - 1) {
-                    NW_PHASE;
-                    // ---- descriptors.  q_{n,l} = sum_m w_m C_lm S^2  (nepBasis.h:174-190)
-                    T cw[MG];
-                    lds_load_even(L.cw + mg * MG, cw);
-                    const bool act = i0 + g < inum;
-                    const T* const cti = L.coef + ti * nt * CROW;
-                    T* const mo = L.mom + g * A::SAT + chan * A::SCH;
-#pragma unroll
-                    for (int m = 0; m < MG; m++) mo[mg * MG + m] = cw[m] * S[m] * S[m];
-#pragma unroll
-                    for (int n = 0; n < NR; n++) q[n] = row_sum(q[n]);
-                    wave_sync();
-                    T* const Q = L.q + g * WROW;
-                    T qr = (T)0;
-#pragma unroll
-                    for (int n = 0; n < NR; n++) qr = s == n ? q[n] : qr;
-                    if (s < NR) Q[s] = qr;
-                    if (mg < LC) {
-                        const int l = mg + 1;
-                        T acc = (T)0;
-#pragma unroll
-                        for (int i = 0; i < 2 * LC + 1; i++)
-                            if (i < 2 * l + 1) acc += mo[l * l - 1 + i];
-                        Q[NR + chan * LC + mg] = acc;
-                    }
-                    wave_sync();
-#pragma unroll
-                    for (int d0 = 0; d0 < WROW; d0 += NW_LANES) {
-                        const int d = d0 + s;
-                        if (d < D) {
-                            const T v = Q[d];
-                            if (a.desc && act) a.desc[((size_t)b * a.P + i0 + g) * D + d] = v;
-                            Q[d] = v * L.qs[d];
-                        } else if (d < WROW) {
-                            Q[d] = (T)0;
-                        }
-                    }
-                    wave_sync();
+            for (int mp = 0; mp < 2 * l + 1; mp++) {
+                const int m = l * l - 1 + mp;
+                acc += (T)(mp == 0 ? 1.0 : 2.0) * (T)kC3B[m] * S[m] * S[m];
+            }
+            if (lane < NAC) L.q[NR + chan * LC + (l - 1)] = acc;
+        }
+        __builtin_amdgcn_wave_barrier();
+        if (lane < D) {
+            const T v = L.q[lane];
+            if (a.desc) a.desc[row * D + lane] = v;
+            L.q[lane] = v * L.qs[lane];
+        } else if (lane < WROW) {
+            L.q[lane] = (T)0;
+        }
+        __builtin_amdgcn_wave_barrier();
 
-                    // ---- hidden layer (nep.h:415-447): lane = neuron -------------------------------------------------
-                    T qv[(D + 3) / 4 * 4], e_site = (T)0;
+        // ---- hidden layer (nep.h:415-447): lane = neuron -------------------------------------------------
+        T e_site = (T)0;
+        for (int p = lane; p < H; p += 64) {
+            const T* wrow = L.w0 + (size_t)(ti * H + p) * WROW;
+            T h = L.b0[ti * H + p];
 #pragma unroll
-                    for (int j = 0; j < D; j += 4) {
-                        T v[4];
-                        lds_load4(Q + j, v);
+            for (int j = 0; j < D; j += 4) {
+                T w[4], v[4];
+                lds_load4(wrow + j, w);
+                lds_load4(L.q + j, v);
 #pragma unroll
-                        for (int i = 0; i < 4; i++) qv[j + i] = v[i];
-                    }
-                    T* const sde = L.sde + g * ((H + 3) / 4 * 4);
-#pragma unroll 1
-                    for (int n = s; n < H; n += NW_LANES) {
-                        const T* wrow = L.w0 + (size_t)(ti * H + n) * WROW;
-                        T h = L.b0[ti * H + n];
-#pragma unroll
-                        for (int j = 0; j < D; j += 4) {
-                            T w[4];
-                            lds_load4(wrow + j, w);
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                if (j + i < D) h += w[i] * qv[j + i];
-                        }
-                        const T th = tanh_t(h), w1p = L.w1[ti * H + n];
-                        e_site += w1p * th;
-                        sde[n] = w1p * ((T)1 - th * th);
-                    }
-                    e_site = row_sum(e_site);
-                    if (act && s == 0) e_sum += (double)e_site + (double)L.bias[ti];         // (rounded to fp32 the bias shifts every atom alike)
-                    if (derivs) {
-                        wave_sync();
-                        // dE/dq: lane = descriptor; of those from the sixteenth on a lane takes half of the neurons
-                        T* const DQ = L.dq + g * WROW;
-                        const T* col = L.w0 + (size_t)ti * H * WROW;
-                        T acc = (T)0, acc1 = (T)0, acc2 = (T)0;
-                        const int half = H >> 1, d2 = NW_LANES + (s & 7), h2 = s < 8 ? 0 : half;
+                for (int i = 0; i < 4; i++)
+                    if (j + i < D) h += w[i] * v[i];
+            }
+            const T th = tanh_t(h), w1p = L.w1[ti * H + p];
+            e_site += w1p * th;
+            L.sde[p] = w1p * ((T)1 - th * th);
+        }
+        e_site = all_sum(e_site) + a.bias[ti];
+        e_sum += (double)e_site;
+        if (!derivs) { __builtin_amdgcn_wave_barrier(); continue; }
+        __builtin_amdgcn_wave_barrier();
+        {
+            // dE/dq: lane = (descriptor, half of the neurons); the halves meet in lanes 0 .. D-1
+            const int half = lane >> 5, d = lane & 31;
+            T acc = (T)0;
+            if (d < D) {
+                const T* col = L.w0 + (size_t)ti * H * WROW + d;
+                const int mid = (H + 1) / 2, p1 = half ? H : mid;
 #pragma unroll 5
-                        for (int n = 0; n < half; n++) {
-                            acc += sde[n] * col[n * WROW + s];
-                            acc1 += sde[half + n] * col[(half + n) * WROW + s];
-                            if (D > NW_LANES) acc2 += sde[h2 + n] * col[(h2 + n) * WROW + d2];
-                        }
-                        if (H & 1) {
-                            acc += sde[H - 1] * col[(H - 1) * WROW + s];
-                            if (D > NW_LANES && s < 8) acc2 += sde[H - 1] * col[(H - 1) * WROW + d2];
-                        }
-                        if (D > NW_LANES) {
-                            acc2 += dpp_move<0x128>(acc2);
-                            if (s < 8) DQ[d2] = acc2 * L.qs[d2];
-                        }
-                        DQ[s] = (acc + acc1) * L.qs[s];
-                        wave_sync();
-                        // ---- dE/dS (nep.h:450-466); radial coefficients contracted with dE/dq
-#pragma unroll
-                        for (int m = 0; m < MG; m++) {
-                            const int lm = mg * MG + m;
-                            const int l1 = lm < 3 ? 0 : lm < 8 ? 1 : lm < 15 ? 2 : 3;
-                            mo[lm] = S[m] * DQ[NR + chan * LC + min(l1, LC - 1)] * ((T)2 * cw[m]);
-                        }
-                        for (int i = s; i < nt * KC; i += NW_LANES) {
-                            const T* c = cti + (i >> 3) * CROW + (i & 7);
-                            T v = (T)0;
-#pragma unroll
-                            for (int n = 0; n < NR; n++) v += DQ[n] * c[n * KC];
-                            L.cc[g * nt * KC + i] = v;
-                        }
-                    }
-                    wave_sync();
-                }
-                if (!frc || (mom && it < nch - 1)) continue;
+                for (int p = half ? mid : 0; p < p1; p++) acc += L.sde[p] * col[(size_t)p * WROW];
+            }
+            acc = add_rows<32>(acc);
+            if (lane < D) L.dq[lane] = acc * L.qs[lane];
+        }
+        __builtin_amdgcn_wave_barrier();
 
-                // ---- pair derivatives ------------------------------------------------------------------------------
-                if (claim && it == (mom ? nch - 1 : 0)) {
-                    NW_PHASE;
+        // ---- dE/dS (nep.h:450-466), overwriting S; radial coefficients contracted with dE/dq ---------------
 #pragma unroll
-                    for (int k = 0; k < NW_TRIPS; k++) {
-                        const int e = k * NW_LANES + s;
-                        if (k * NW_LANES < n_most && e < n_own) {
-                            int2* const w = &ent[entry(e)];
-                            const int tg = b * NF + w->x, r = pair_rank(rk[k]);
-                            if (a.brank && !a.ranks_valid) a.brank[base + (w->y & 0xffff)] = r;
-                            const bool fits = (unsigned)r < (unsigned)seg.cap;
-                            if (!fits) atomicOr(a.status, ST_SEG_OVERFLOW);
-                            w->x = fits ? tg * seg.cap + r : seg.spare;
-                        }
-                    }
-                }
-                // -- lane = pair: F = g' T u + (w - (w . u) u) / r with the moments' adjoints s, T = s . b and w = s . grad b
-                if (on) {
-                    NW_PHASE;
-                    const T* mo = L.mom + pg * A::SAT;
-                    T bl[NLM];                                    // (again: held over the read-out they would cost a wavefront per SIMD)
-                    asm volatile("" : "+v"(ux), "+v"(uy), "+v"(uz));
-                    blm_values<T, LC>(ux, uy, uz, bl);
-                    T P[NLM], srad = (T)0;
+        for (int l = 1; l <= LC; l++) {
+            const T dl = L.dq[NR + chan * LC + (l - 1)];
 #pragma unroll
-                    for (int m = 0; m < NLM; m++) P[m] = (T)0;
-#pragma unroll
-                    for (int c = 0; c < NAC; c++) {
-                        T tc = (T)0;
-#pragma unroll
-                        for (int m = 0; m < 4 * MG; m += 4) {
-                            T v[4];
-                            lds_load4(mo + c * A::SCH + m, v);
-#pragma unroll
-                            for (int i = 0; i < 4; i++)
-                                if (m + i < NLM) { P[m + i] += ga[c] * v[i]; tc += v[i] * bl[m + i]; }
-                        }
-                        srad += dg[c] * tc;
-                    }
-                    T wx = (T)0, wy = (T)0, wz = (T)0;
-                    blm_grad_dot<T, LC>(ux, uy, uz, P, wx, wy, wz);
-                    const T along = srad - (wx * ux + wy * uy + wz * uz) * rinv;
-                    T* const rw = L.ang + lane * 3;
-                    rw[0] = along * ux + wx * rinv;
-                    rw[1] = along * uy + wy * rinv;
-                    rw[2] = along * uz + wz * rinv;
-                }
-                wave_sync();
-                // -- lane = neighbour of the atom: the radial part, the pair's force; behind the last angular pairs also the
-                // pairs between the cutoffs
-                const bool tail = it == nch - 1;
-                NW_PHASE;
-                const int o_own = pick(g, 0, o1, o2, o3);
-                const T rr_inv = (T)1 / a.rr;
-                const int f0 = min(max(c0 - o_own, 0), nA), f1 = min(max(c0 + 64 - o_own, 0), nA);
-                const int nf = f1 - f0, nr = tail ? nR : 0, trips = (most_of_atoms(nf + nr) + 2 * NW_LANES - 1) / (2 * NW_LANES);
-                T* const seg_g = K_.seg_g;
-                auto fetch = [&](int k, int2& w, T& x, T& y, T& z) __attribute__((always_inline)) {
-                    w = make_int2(0, 0); x = (T)1; y = z = (T)0;
-                    if (k < nf + nr) {
-                        w = ent[k < nf ? f0 + k : NW_CAP - 1 - (k - nf)];
-                        const T* xp = a.brcs + (size_t)(base + (w.y & 0xffff)) * 3;
-                        x = xp[0]; y = xp[1]; z = xp[2];
-                    }
-                };
-                T vir[9];
-#pragma unroll
-                for (int i = 0; i < 9; i++) vir[i] = (T)0;
-                int2 w1[V];
-                T xn[V], yn[V], zn[V];
-#pragma unroll
-                for (int v = 0; v < V; v++) fetch(v * NW_LANES + s, w1[v], xn[v], yn[v], zn[v]);
-#pragma unroll 1
-                for (int k0 = 0; k0 < trips; k0++) {
-                    const int k = k0 * STEP + s;
-                    int2 w[V];
-                    T px[V], py[V], pz[V], gx[V], gy[V], gz[V];
-#pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        w[v] = w1[v]; px[v] = xn[v]; py[v] = yn[v]; pz[v] = zn[v];
-                        fetch(k + STEP + v * NW_LANES, w1[v], xn[v], yn[v], zn[v]);
-                    }
-#pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        T ri;
-                        const T r = length<false>(px[v] * px[v] + py[v] * py[v] + pz[v] * pz[v], ri);
-                        T f[KC], df[KC];
-                        radial_basis<T, KC, true>(r, rr_inv, KC, f, df);
-                        T v0[4], v1[4], sr = (T)0;
-                        const T* cc = L.cc + (g * nt + (w[v].y >> 16)) * KC;
-                        lds_load4(cc, v0);
-                        lds_load4(cc + 4, v1);
-#pragma unroll
-                        for (int i = 0; i < 4; i++) sr += v0[i] * df[i];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) sr += v1[i] * df[4 + i];
-                        sr *= ri;
-                        gx[v] = sr * px[v]; gy[v] = sr * py[v]; gz[v] = sr * pz[v];
-                    }
-#pragma unroll
-                    for (int v = 0; v < V; v++) {
-                        const int kv = k + v * NW_LANES;
-                        if (kv < nf + nr) {
-                            if (kv < nf) {
-                                const T* rw = L.ang + (o_own + f0 + kv - c0) * 3;
-                                gx[v] += rw[0]; gy[v] += rw[1]; gz[v] += rw[2];
-                            }
-                            if (seg_g) {
-                                T* dst = seg_g + (size_t)w[v].x * 3;
-                                dst[0] = gx[v]; dst[1] = gy[v]; dst[2] = gz[v];
-                            }
-                        } else {
-                            gx[v] = gy[v] = gz[v] = (T)0;
-                        }
-                    }
-                    static_assert(V == 2, "sums two by two: as many roundings as over 64 lanes");
-                    fx += gx[0] + gx[1]; fy += gy[0] + gy[1]; fz += gz[0] + gz[1];
-                    vir[0] -= gx[0] * px[0] + gx[1] * px[1]; vir[1] -= gx[0] * py[0] + gx[1] * py[1]; vir[2] -= gx[0] * pz[0] + gx[1] * pz[1];
-                    vir[3] -= gy[0] * px[0] + gy[1] * px[1]; vir[4] -= gy[0] * py[0] + gy[1] * py[1]; vir[5] -= gy[0] * pz[0] + gy[1] * pz[1];
-                    vir[6] -= gz[0] * px[0] + gz[1] * px[1]; vir[7] -= gz[0] * py[0] + gz[1] * py[1]; vir[8] -= gz[0] * pz[0] + gz[1] * pz[1];
-                }
-#pragma unroll
-                for (int i = 0; i < 9; i++) v_sum[i] += (double)vir[i];
-                wave_sync();
+            for (int mp = 0; mp < 2 * l + 1; mp++) {
+                const int m = l * l - 1 + mp;
+                S[m] *= dl * (T)(mp == 0 ? 2.0 : 4.0) * (T)kC3B[m];
             }
         }
-        NW_PHASE;
-        if (a.force) {
-            fx = row_sum(fx); fy = row_sum(fy); fz = row_sum(fz);
-            const bool act = i0 + g < inum;
-            if (act && s < 3) a.force[((size_t)b * NF + center) * 3 + s] = s == 0 ? fx : s == 1 ? fy : fz;
-            if (act && seg.mark && s == 3) pair_mark_own(&seg.cursor[b * NF + center]);
+        for (int i = lane; i < nt * KC; i += 64) {
+            const T* c = cti + (i >> 3) * CROW + (i & 7);
+            T v = (T)0;
+#pragma unroll
+            for (int n = 0; n < NR; n++) v += L.dq[n] * c[n * KC];
+            L.cc[i] = v;
         }
-        begin(i0 + stride);
+        __builtin_amdgcn_wave_barrier();
+
+        // ---- pair derivatives ------------------------------------------------------------------------------
+        T fx = (T)0, fy = (T)0, fz = (T)0, vir[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) vir[i] = (T)0;
+        for (int t = 0; t < ntiles; t++) {
+            if (ntiles > 1) {
+                load_slots<T>(a, t, lane, row, nn, slots);
+                load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, true, slots, nA, nR);
+            }
+            for (int e0 = 0; e0 < nA; e0 += 16) {
+                const int e = e0 + quad;
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
+                T f[KC], df[KC];
+                radial_basis<T, KC, true>(r, ra_inv, KC, f, df);
+                T c0[4], c1[4], g = (T)0, dg = (T)0;
+                lds_load4(cti + tj * CROW + (NR + chan) * KC, c0);
+                lds_load4(cti + tj * CROW + (NR + chan) * KC + 4, c1);
+#pragma unroll
+                for (int k = 0; k < 4; k++) { g += c0[k] * f[k]; dg += c0[k] * df[k]; }
+#pragma unroll
+                for (int k = 0; k < 4; k++) { g += c1[k] * f[4 + k]; dg += c1[k] * df[4 + k]; }
+                T bl[NLM];
+                blm_values<T, LC>(ux, uy, uz, bl);
+                T srad = (T)0;
+#pragma unroll
+                for (int l = 1; l <= LC; l++) {
+                    T sl = (T)0;
+#pragma unroll
+                    for (int mp = 0; mp < 2 * l + 1; mp++) sl += S[l * l - 1 + mp] * bl[l * l - 1 + mp];
+                    srad += (dg - (T)l * rinv * g) * sl;
+                }
+                T wx = (T)0, wy = (T)0, wz = (T)0;
+                blm_grad_dot<T, LC>(ux, uy, uz, S, wx, wy, wz);
+                const T gr = g * rinv;
+                const T gx = quad_sum(srad * ux + wx * gr), gy = quad_sum(srad * uy + wy * gr),
+                        gz = quad_sum(srad * uz + wz * gr);
+                if (e < nA && chan == 0) { L.ang[e * 3] = gx; L.ang[e * 3 + 1] = gy; L.ang[e * 3 + 2] = gz; }
+            }
+            __builtin_amdgcn_wave_barrier();
+            for (int e = lane; e < nA + nR; e += 64) {
+                const int k = e < nA ? e : NW_CAP - 1 - (e - nA);
+                T x, y, z;
+                int tj;
+                ent_load(L.ent + k * 4, x, y, z, tj);
+                const T r = sqrt_t(x * x + y * y + z * z);
+                T f[KC], df[KC];
+                radial_basis<T, KC, true>(r, rr_inv, KC, f, df);
+                T c0[4], c1[4], sr = (T)0;
+                lds_load4(L.cc + tj * KC, c0);
+                lds_load4(L.cc + tj * KC + 4, c1);
+#pragma unroll
+                for (int i = 0; i < 4; i++) sr += c0[i] * df[i];
+#pragma unroll
+                for (int i = 0; i < 4; i++) sr += c1[i] * df[4 + i];
+                sr /= r;
+                T gx = sr * x, gy = sr * y, gz = sr * z;
+                if (e < nA) { gx += L.ang[e * 3]; gy += L.ang[e * 3 + 1]; gz += L.ang[e * 3 + 2]; }
+                if (seg_g) {
+                    T* dst = seg_g + (size_t)L.pos[k] * 3;
+                    dst[0] = gx; dst[1] = gy; dst[2] = gz;
+                }
+                fx += gx; fy += gy; fz += gz;
+                vir[0] -= gx * x; vir[1] -= gx * y; vir[2] -= gx * z;
+                vir[3] -= gy * x; vir[4] -= gy * y; vir[5] -= gy * z;
+                vir[6] -= gz * x; vir[7] -= gz * y; vir[8] -= gz * z;
+            }
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int i = 0; i < 9; i++) v_sum[i] += (double)vir[i];
+        if (a.force) {
+            fx = all_sum(fx); fy = all_sum(fy); fz = all_sum(fz);
+            if (lane < 3) a.force[((size_t)b * NF + center) * 3 + lane] = lane == 0 ? fx : lane == 1 ? fy : fz;
+            if (seg.mark && lane == 3) pair_mark_own(&seg.cursor[b * NF + center]);
+        }
     }
 
-    // ---- workgroup partial sums of energy and virial (fp64): 16 threads to a sum, lanes 4 k .. 4 k + 3 of every wavefront
-    // to the k-th
-    {
-        NW_PHASE;
-        double* const mine = (double*)L.rows;              // (of the wavefront; the read-out's scratch is no longer in use)
-        mine[lane] = e_sum;
+    // ---- workgroup partial sums of energy and virial (fp64) ---------------------------------
+    if (lane == 0) L.red[wave * 10] = e_sum;
 #pragma unroll
-        for (int i = 0; i < 9; i++) mine[(1 + i) * 64 + lane] = v_sum[i];
+    for (int i = 0; i < 9; i++) {
+        const double v = all_sum(v_sum[i]);
+        if (lane == 0) L.red[wave * 10 + 1 + i] = v;
     }
     __syncthreads();
-    NW_PHASE;
-    for (int c = threadIdx.x >> 4; c < 10; c += nwaves * 4) {
+    if (tid < 10) {
         double v = 0.0;
-        for (int w = 0; w < nwaves; w++) {
-            const double* theirs = (const double*)((const unsigned char*)L.rows + (w - wave) * K_.at.own) + c * 64 + s * 4;
-#pragma unroll
-            for (int i = 0; i < 4; i++) v += theirs[i];
-        }
-        v = row_sum(v);
-        if (s == 0) a.partial[ev_partial(a.nblocks, b, blockIdx.x, c)] = v;
+        for (int w = 0; w < NW_WAVES; w++) v += L.red[w * 10 + tid];
+        a.partial[ev_partial(a.nblocks, b, blockIdx.x, tid)] = v;
     }
-}
-#undef NW_PHASE
-
-// Wavefronts of a workgroup, workgroups of a structure.  A workgroup to a compute unit, which shares the model's tables, or two
-// where they have room; as many rows for each wavefront as it takes with the most wavefronts a compute unit holds, and then no
-// more wavefronts than that takes (four stage the tables faster than one).
-struct WaveShape { int waves, nblocks; size_t lds; WaveAt at; };
-template <typename T>
-WaveShape wave_shape(const NepArgs<T>& a)
-{
-    const WaveAt at = a.l_max == 3 ? wave_at<T, 3>(a.ntypes, a.H, a.n_r + NAC) : wave_at<T, 4>(a.ntypes, a.H, a.n_r + NAC);
-    const int most = std::min(wave_cap<T>(), (160 * 1024 - std::min(at.shared, 160 * 1024)) / at.own);
-    if (most < 1) return {0, 0, 0, at};
-    const int per = std::max(1, ceil_div(a.P, NW_ATOMS));                    // sets of four rows of a structure
-    const long long sets = (long long)a.B * per;
-    int waves = std::min(most, (int)std::min<long long>((sets + 256 * 4 - 1) / (256 * 4) * 4, wave_cap<T>())), held = 1;
-    if (waves == 8 && 2 * (at.shared + 4 * at.own) <= 160 * 1024) { waves = 4; held = 2; }
-    const int nblocks = std::min(ceil_div(per, waves), std::max(1, held * 256 / std::max(a.B, 1)));
-    return {waves, nblocks, (size_t)at.shared + (size_t)waves * at.own, at};
 }
 
 template <typename T, int NR, int LC>
-int launch_wave(const NepArgs<T>& a, const PairCsr& csr, hipStream_t stream)
+int launch_wave(const NepArgs<T>& a, size_t lds, const PairCsr& csr, hipStream_t stream)
 {
     SegArgs seg{csr.cursor, csr.seg_cap, csr.n * csr.seg_cap, csr.mark};
     auto kern = nep_wave_kernel<T, NR, LC>;
-    const WaveShape w = wave_shape<T>(a);
-    if (w.lds > 48 * 1024)
-        A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)w.lds));
+    if (lds > 48 * 1024)
+        A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     prof_begin("nep_wave_kernel", stream);
-    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at});
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(NW_THREADS), lds, stream, a, seg, (T*)csr.seg_g);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
@@ -801,20 +480,24 @@ int launch_wave(const NepArgs<T>& a, const PairCsr& csr, hipStream_t stream)
 
 }  // namespace
 
-template <typename T>
-int nep_wave_nblocks(const NepArgs<T>& a)
+// Workgroups per structure: an atom per wavefront until the batch has some 1024 workgroups (four per compute unit), from
+// there on several, so that the tables are staged once for all of them.
+int nep_wave_nblocks(int P, int B)
 {
-    return wave_shape<T>(a).nblocks;
+    return std::max(1, std::min(ceil_div(P, NW_WAVES), 1024 / std::max(B, 1)));
 }
 
 template <typename T>
-bool nep_wave_supported(const NepArgs<T>& a)
+bool nep_wave_supported(const NepArgs<T>& a, size_t* lds_bytes)
 {
-    return a.K == KC && (a.n_r == 4 || a.n_r == 6) && a.n_a == NAC && (a.l_max == 3 || a.l_max == 4) && wave_shape<T>(a).waves > 0;
+    if (!(a.K == KC && (a.n_r == 4 || a.n_r == 6) && a.n_a == NAC && (a.l_max == 3 || a.l_max == 4))) return false;
+    WaveLds<T> unused;
+    *lds_bytes = wave_lds_layout<T>(a.ntypes, a.H, a.n_r + NAC, 0, nullptr, unused);
+    return *lds_bytes <= 150 * 1024;
 }
 
 template <typename T>
-int nep_wave_run(const NepArgs<T>& a, T* etot, T* virial, hipStream_t stream)
+int nep_wave_run(const NepArgs<T>& a, size_t lds_bytes, T* etot, T* virial, hipStream_t stream)
 {
     PairCsr csr;
     int rc;
@@ -823,18 +506,16 @@ int nep_wave_run(const NepArgs<T>& a, T* etot, T* virial, hipStream_t stream)
                                  a.bincoming != nullptr && a.ranks_valid != 0);
         if (rc) return rc;
     }
-    if (a.n_r == 4) rc = a.l_max == 3 ? launch_wave<T, 4, 3>(a, csr, stream) : launch_wave<T, 4, 4>(a, csr, stream);
-    else rc = a.l_max == 3 ? launch_wave<T, 6, 3>(a, csr, stream) : launch_wave<T, 6, 4>(a, csr, stream);
+    if (a.n_r == 4) rc = a.l_max == 3 ? launch_wave<T, 4, 3>(a, lds_bytes, csr, stream) : launch_wave<T, 4, 4>(a, lds_bytes, csr, stream);
+    else rc = a.l_max == 3 ? launch_wave<T, 6, 3>(a, lds_bytes, csr, stream) : launch_wave<T, 6, 4>(a, lds_bytes, csr, stream);
     if (rc) return rc;
     if (a.force) return pair_csr_finish<T>(a.force, csr, stream, etot, virial, a.partial, a.B, a.nblocks);
     return finish_energy_virial<T>(etot, virial, a.partial, a.B, a.nblocks, stream);
 }
 
-template bool nep_wave_supported<float>(const NepArgs<float>&);
-template bool nep_wave_supported<double>(const NepArgs<double>&);
-template int nep_wave_nblocks<float>(const NepArgs<float>&);
-template int nep_wave_nblocks<double>(const NepArgs<double>&);
-template int nep_wave_run<float>(const NepArgs<float>&, float*, float*, hipStream_t);
-template int nep_wave_run<double>(const NepArgs<double>&, double*, double*, hipStream_t);
+template bool nep_wave_supported<float>(const NepArgs<float>&, size_t*);
+template bool nep_wave_supported<double>(const NepArgs<double>&, size_t*);
+template int nep_wave_run<float>(const NepArgs<float>&, size_t, float*, float*, hipStream_t);
+template int nep_wave_run<double>(const NepArgs<double>&, size_t, double*, double*, hipStream_t);
 
 }  // namespace a2p

@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 from ai2pot_amd import synth
-from test_gpu_nep import run_gpu
+from test_gpu_nep import check, run_gpu
+from test_gpu_nep_wave import _lists
 
 pytestmark = pytest.mark.gpu
 ROWS, U = 71, 72
@@ -29,10 +30,11 @@ def _copies(blk, copies, batch):
     return dict(nb, binum=np.full(batch, ROWS * copies - 1, np.int32), nghost=0)
 
 
-# fp32 at three species: up to 4096 rows four wavefronts, up to 8192 two workgroups of four, beyond it twelve wavefronts, beyond
-# 12288 several times four rows each; fp64 holds four wavefronts throughout.  One species: several workgroups of any size.
+# fp32 at three species: up to 2560 rows a wavefront each; then four rows each, up to 4096 four wavefronts to a workgroup, up to
+# 8192 two such workgroups, beyond it twelve wavefronts, beyond 12288 several times four rows each; fp64 from 1024 rows on four
+# wavefronts throughout.  One species: several workgroups of any size.
 @pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
-@pytest.mark.parametrize("ntypes,copies,batch", [(3, 1, 1), (3, 57, 1), (3, 58, 1), (3, 115, 1), (3, 116, 1), (3, 180, 1), (3, 600, 1),
+@pytest.mark.parametrize("ntypes,copies,batch", [(3, 1, 1), (3, 14, 1), (3, 36, 1), (3, 37, 1), (3, 57, 1), (3, 58, 1), (3, 115, 1), (3, 116, 1), (3, 180, 1), (3, 600, 1),
                                                  (3, 1, 61), (3, 3, 61), (1, 180, 1), (5, 60, 3)])
 def test_every_launch_gives_the_same(np_dtype, ntypes, copies, batch):
     blk = _block(np_dtype, ntypes)
@@ -56,3 +58,19 @@ def test_every_launch_gives_the_same(np_dtype, ntypes, copies, batch):
     scale = max(copies, 3) * eps * 1200
     assert np.abs(e - (e2 + (copies - 2) * per_e)).max() <= scale * np.abs(e3).max()
     assert np.abs(v - (v2 + (copies - 2) * per_v)).max() <= scale * np.abs(v3).max()
+
+
+@pytest.mark.parametrize("np_dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n_r,l_max,ntypes,H,nghost,skin", [(6, 4, 3, 50, 0, 0.0), (4, 3, 1, 30, 7, 1.0),
+                                                            (6, 3, 5, 65, 0, 1.0), (4, 4, 2, 7, 3, 0.0)])
+def test_tile_edges_of_four_atoms(oracle, np_dtype, n_r, l_max, ntypes, H, nghost, skin):
+    """Rows of 0 to 200 slots with 0 to 200 of them inside the angular cutoff (several tiles and several rounds of 64 pairs
+    beside rows of one), 39 structures of them: four rows to a wavefront in either precision."""
+    nb = _lists(np_dtype, ntypes, nghost, skin)
+    m = synth.nep_model(ntypes=ntypes, n_radial_basis=n_r, l_max=l_max, num_neurons=H, type_map=(1, 2, 3, 4, 5), sigma=0.12)
+    m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    ref = oracle.nep_efv(m, nb, np_dtype)
+    many = {k: np.concatenate([v] * 13) if isinstance(v, np.ndarray) else v for k, v in nb.items()}
+    e, f, v = run_gpu(m, many, np_dtype)
+    for k in range(0, 39, 3):
+        check((e[k:k + 3], f[k:k + 3], v[k:k + 3]), ref, np_dtype)
