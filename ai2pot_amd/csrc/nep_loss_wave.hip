@@ -15,7 +15,8 @@
 //
 // Bound: issue of the vector instructions and the chain of an atom, with two workgroups of four wavefronts per compute
 // unit (LDS).  64 structures of 128 atoms, fp32, 3 species, 50 neurons: 179 -> 59 us against 128 threads per atom, and
-// 25 -> 9.8 us for the sums over the atoms.
+// 25 -> 9.8 us for the sums over the atoms.  59 -> 52 by the next atom's first slots and the tables on their way early (tables
+// 8.9 -> 5.1 thousand cycles) and by a descriptor's moments read together (4.5 -> 2.3 of 25.6 thousand cycles an atom).
 #include "a2p_common.h"
 #include "nep_device.h"
 #include "nep_loss.h"
@@ -88,16 +89,41 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
     const int b = blockIdx.y, H = a.H, nt = a.ntypes;
     LossWaveLds<T> L;
     loss_wave_layout<T>(nt, H, NB, wave, smem_raw, L);
-    for (int i = tid; i < nt * H * WROW; i += LW_THREADS) {
-        const int r = i / WROW, j = i - r * WROW;
-        L.w0[i] = j < D ? a.w0[(size_t)r * D + j] : (T)0;
+    // What the next atom begins with, on its way while the one before is worked on: the atom, its number of neighbours, its
+    // first 64 slots (whether they hold a neighbour or not).
+    int center1, nn1, nj1;
+    T x1, y1, z1;
+    auto begin = [&](int ii) __attribute__((always_inline)) {
+        const size_t row = (size_t)b * a.P + min(ii, a.P - 1), pr = row * a.U + min(lane, a.U - 1);
+        center1 = a.bilist[row];
+        nn1 = a.bnumneigh[row];
+        nj1 = a.bfirstneigh[pr];
+        x1 = a.brcs[pr * 3]; y1 = a.brcs[pr * 3 + 1]; z1 = a.brcs[pr * 3 + 2];
+    };
+    begin(blockIdx.x * LW_WAVES + wave);
+    {
+        // The model's tables: the first values of every thread are all on their way before one is stored.
+        constexpr int W0 = sizeof(T) == 4 ? 16 : 8, C0 = 4;
+        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
+        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
+        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
+        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
+#pragma unroll
+        for (int u = 0; u < C0; u++) { const int i = tid + u * LW_THREADS; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
+#pragma unroll
+        for (int u = 0; u < W0; u++) { const int i = tid + u * LW_THREADS; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
+        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
+        if (tid < D) qs = a.q_scaler[tid];
+#pragma unroll
+        for (int u = 0; u < C0; u++) { const int i = tid + u * LW_THREADS; if (i < nc) put_coef(i, c0[u]); }
+#pragma unroll
+        for (int u = 0; u < W0; u++) { const int i = tid + u * LW_THREADS; if (i < nw0) put_w0(i, w0[u]); }
+        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
+        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
+        for (int i = tid + C0 * LW_THREADS; i < nc; i += LW_THREADS) put_coef(i, a.coeffs[i]);
+        for (int i = tid + W0 * LW_THREADS; i < nw0; i += LW_THREADS) put_w0(i, a.w0[i]);
+        for (int i = tid + LW_THREADS; i < nh; i += LW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
     }
-    for (int i = tid; i < nt * nt * NB * KC; i += LW_THREADS) {
-        const int p = i / (NB * KC);
-        L.coef[p * CROW + (i - p * NB * KC)] = a.coeffs[i];
-    }
-    for (int i = tid; i < nt * H; i += LW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
-    if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / a.q_scaler[tid] : (T)0;
     if (tid < LM) {
         const int l = l_of_lm(tid);
         L.wc[tid] = tid < NLM ? (T)(tid == l * l - 1 ? 1.0 : 2.0) * (T)kC3B[tid] : (T)0;
@@ -112,7 +138,7 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
 
     for (int ii = blockIdx.x * LW_WAVES + wave; ii < inum; ii += gridDim.x * LW_WAVES) {
         const size_t row = (size_t)b * a.P + ii;
-        int center = a.bilist[row], nn = a.bnumneigh[row];
+        int center = center1, nn = nn1;
         if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
         if ((unsigned)center >= (unsigned)a.P) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
         int ti = types[center];
@@ -138,10 +164,15 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
                     const int slot = slot0 + lane;
                     T x = (T)1, y = (T)0, z = (T)0, w[3] = {(T)0, (T)0, (T)0};
                     int tj = -1;
-                    if (slot < nn) {
+                    int nj = nj1;
+                    if (slot < nn) { x = x1; y = y1; z = z1; }
+                    if ((pass > 0 || slot0 > 0) && slot < nn) {
                         const size_t pr = row * a.U + slot;
-                        int nj = a.bfirstneigh[pr];
+                        nj = a.bfirstneigh[pr];
                         x = a.brcs[pr * 3]; y = a.brcs[pr * 3 + 1]; z = a.brcs[pr * 3 + 2];
+                    }
+                    if (pass == 0 && slot0 == 0) begin(ii + gridDim.x * LW_WAVES);
+                    if (slot < nn) {
                         if ((unsigned)nj >= (unsigned)a.P) { atomicOr(a.status, ST_BAD_NEIGHBOR); nj = center; }
                         tj = types[nj];
                         const T* fc = a.dFs + ((size_t)b * a.P + center) * 3;
@@ -315,18 +346,34 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
             if (d < D) {
                 T acc = (T)0;
                 if (d < NR) {
+#pragma unroll 2
                     for (int t = 0; t < nt; t++) {
                         const T *c = cti + t * CROW + d * KC, *f = L.F + t * RS + half * KC;
 #pragma unroll
-                        for (int k = 0; k < KC; k++) acc += c[k] * f[k];
+                        for (int k = 0; k < KC; k += 4) {
+                            T cv[4], fv[4];
+                            lds_load4(c + k, cv);
+                            lds_load4(f + k, fv);
+#pragma unroll
+                            for (int i = 0; i < 4; i++) acc += cv[i] * fv[i];
+                        }
                     }
                 } else {
                     const int n = (d - NR) / LC, l = (d - NR) % LC + 1;
-                    for (int m = l * l - 1; m < l * l + 2 * l; m++) {
-                        const T v = L.SS[n * TS + m];
-                        const T u = half ? (T)2 * (L.SS[(NAC + n) * TS + m] + L.SS[n * TS + LM + m]) : v;
-                        acc += L.wc[m] * v * u;
+                    // (a degree's moments all read before they are summed; beyond its last the weight is left out)
+                    const T* const sv = L.SS + n * TS + l * l - 1;
+                    const T* const wc = L.wc + l * l - 1;
+                    T v[2 * LC + 1], u[2 * LC + 1], w[2 * LC + 1];
+#pragma unroll
+                    for (int i = 0; i < 2 * LC + 1; i++) {
+                        const int m = min(i, 2 * l);
+                        v[i] = sv[m];
+                        u[i] = sv[NAC * TS + m] + sv[LM + m];
+                        w[i] = wc[m];
                     }
+#pragma unroll
+                    for (int i = 0; i < 2 * LC + 1; i++)
+                        if (i <= 2 * l) acc += w[i] * v[i] * (half ? (T)2 * u[i] : v[i]);
                 }
                 acc *= L.qs[d];                        // scaled descriptor and tangent
                 L.q[half * WROW + d] = acc;
