@@ -509,8 +509,8 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     // neighbours inside the angular cutoff: radial sums and angular moments
     walk_list<T, true>(a.cv, tile, lane, st, n_inner, true, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
         const int tj = min((bits >> CL_TYPE_SHIFT) & 15, nt - 1);
-        const T r = sqrt_t(x * x + y * y + z * z);
-        const T rinv = (T)1 / r;
+        T rinv;
+        const T r = length<false>(x * x + y * y + z * z, rinv);
         T f[KC], df[KC];
         radial_basis<T, KC, false>(r, rr_inv, KC, f, df);
 #pragma unroll
@@ -541,7 +541,8 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     // neighbours between the cutoffs: radial sums only
     walk_list<T, true>(a.cv, tile, lane, st, n_outer, false, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
         const int tj = min((bits >> CL_TYPE_SHIFT) & 15, nt - 1);
-        const T r = sqrt_t(x * x + y * y + z * z);
+        T unused;
+        const T r = length<false>(x * x + y * y + z * z, unused);
         T f[KC], df[KC];
         radial_basis<T, KC, false>(r, rr_inv, KC, f, df);
 #pragma unroll
@@ -677,8 +678,8 @@ nep_adjoint_kernel(const GatherArgs<T> a)
             // the place of this pair among the pairs that name atom j
             int place = 0;
             if (hand_over) place = atomicAdd(a.incoming + j, 1);
-            const T r = sqrt_t(x * x + y * y + z * z);
-            const T rinv = (T)1 / r;
+            T rinv;
+            const T r = length<false>(x * x + y * y + z * z, rinv);
             const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
             T f[KC], df[KC];
             T srad;
@@ -811,7 +812,8 @@ nep_gather_kernel(const GatherArgs<T> a)
         T lo[4], hi[4];
         ld4(a.rcc + ((size_t)j * NTC + ti) * KC, lo);
         ld4(a.rcc + ((size_t)j * NTC + ti) * KC + 4, hi);
-        const T r = sqrt_t(x * x + y * y + z * z);
+        T rinv;
+        const T r = length<false>(x * x + y * y + z * z, rinv);
         T ck[KC];
 #pragma unroll
         for (int k = 0; k < KC; k++) {
@@ -822,7 +824,7 @@ nep_gather_kernel(const GatherArgs<T> a)
         }
 #pragma unroll
         for (int k = 0; k < 4; k++) { ck[k] += lo[k]; ck[4 + k] += hi[k]; }
-        const T sr = radial_derivative_dot<T>(r, rr_inv, ck) / r;
+        const T sr = radial_derivative_dot<T>(r, rr_inv, ck) * rinv;
         const T gx = sr * x, gy = sr * y, gz = sr * z;
         fx += gx; fy += gy; fz += gz;
         vir[0] -= gx * x; vir[1] -= gx * y; vir[2] -= gx * z;

@@ -182,7 +182,8 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
                             w[q] = fc[q] - fn[q] - (dv[q * 3] * x + dv[q * 3 + 1] * y + dv[q * 3 + 2] * z);
                         if ((unsigned)tj >= (unsigned)nt) { atomicOr(a.status, ST_BAD_TYPE); tj = 0; }
                     }
-                    const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                    T rinv;
+                    const T r = length<false>(x * x + y * y + z * z, rinv);
                     const T uw = (w[0] * x + w[1] * y + w[2] * z) * rinv;
                     const bool in = slot < nn && r <= rr, inA = in && r <= ra;   // nepBasis.h:106, 135
                     const unsigned long long mA = __ballot(inA);
@@ -231,7 +232,8 @@ __global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepL
                         const int e = c0 + min(lane, n - 1);
                         ent_load(L.ent + e * 4, x, y, z, tj);
                         lds_load4(L.W + e * 4, w);
-                        const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                        T rinv;
+                    const T r = length<false>(x * x + y * y + z * z, rinv);
                         x *= rinv; y *= rinv; z *= rinv;
                         radial_basis<T, KC, true>(r, ra_inv, KC, fa, fad);
 #pragma unroll

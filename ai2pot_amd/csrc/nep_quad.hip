@@ -124,25 +124,6 @@ __device__ __forceinline__ void lds_load_even(const T* p, T (&o)[N])
     }
 }
 
-// r and 1 / r from r^2: the estimate of 1 / r and a Newton step for each, a third of the operations of square root and
-// division.  r^2 = 0 gives NaN, as 0 / 0 does; MIN keeps it from that.
-template <bool MIN>
-__device__ __forceinline__ float length(float d2, float& rinv)
-{
-    if (MIN) d2 = d2 < 1e-30f ? 1e-30f : d2;                    // (NaN stays)
-    const float y = __builtin_amdgcn_rsqf(d2), r0 = d2 * y;
-    const float r = r0 + (d2 - r0 * r0) * (0.5f * y);
-    rinv = y + y * (1.0f - r * y);
-    return r;
-}
-template <bool MIN>
-__device__ __forceinline__ double length(double d2, double& rinv)
-{
-    const double r = sqrt(d2);
-    rinv = 1.0 / r;
-    return r;
-}
-
 // What a lane of the wavefront wrote to LDS is read by the others behind this.
 __device__ __forceinline__ void wave_sync()
 {

@@ -132,7 +132,8 @@ __device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& se
         const int slot = t * NW_CAP + h * 64 + lane;
         const bool valid = slot < nn && (unsigned)nj[h] < (unsigned)NF;
         if (valid && (unsigned)tj[h] >= (unsigned)a.ntypes) { atomicOr(a.status, ST_BAD_TYPE); tj[h] = 0; }
-        const T r = sqrt_t(x[h] * x[h] + y[h] * y[h] + z[h] * z[h]);
+        T unused;
+        const T r = length<true>(x[h] * x[h] + y[h] * y[h] + z[h] * z[h], unused);
         const bool inA = valid && r <= ra && r <= rr;   // nepBasis.h:106, 135: beyond the radial cutoff a neighbour is skipped
         const bool inR = valid && !inA && r <= rr;
         int pos = 0;
@@ -246,7 +247,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 int tj;
                 ent_load(L.ent + (e < nA ? e : NW_CAP - 1 - (e - nA)) * 4, x, y, z, tj);
                 T f[KC], df[KC];
-                radial_basis<T, KC, false>(sqrt_t(x * x + y * y + z * z), rr_inv, KC, f, df);
+                T unused;
+                radial_basis<T, KC, false>(length<true>(x * x + y * y + z * z, unused), rr_inv, KC, f, df);
                 const T* c = cti + tj * CROW;
 #pragma unroll
                 for (int n = 0; n < NR; n++) {
@@ -264,7 +266,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 T x, y, z;
                 int tj;
                 ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
-                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                T rinv;
+                const T r = length<false>(x * x + y * y + z * z, rinv);
                 T f[KC], df[KC];
                 radial_basis<T, KC, false>(r, ra_inv, KC, f, df);
                 T c0[4], c1[4], g = (T)0;
@@ -382,7 +385,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 T x, y, z;
                 int tj;
                 ent_load(L.ent + min(e, nA - 1) * 4, x, y, z, tj);
-                const T r = sqrt_t(x * x + y * y + z * z), rinv = (T)1 / r;
+                T rinv;
+                const T r = length<false>(x * x + y * y + z * z, rinv);
                 const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
                 T f[KC], df[KC];
                 radial_basis<T, KC, true>(r, ra_inv, KC, f, df);
@@ -416,7 +420,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 T x, y, z;
                 int tj;
                 ent_load(L.ent + k * 4, x, y, z, tj);
-                const T r = sqrt_t(x * x + y * y + z * z);
+                T rinv;
+                const T r = length<false>(x * x + y * y + z * z, rinv);
                 T f[KC], df[KC];
                 radial_basis<T, KC, true>(r, rr_inv, KC, f, df);
                 T c0[4], c1[4], sr = (T)0;
@@ -426,7 +431,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 for (int i = 0; i < 4; i++) sr += c0[i] * df[i];
 #pragma unroll
                 for (int i = 0; i < 4; i++) sr += c1[i] * df[4 + i];
-                sr /= r;
+                sr *= rinv;
                 T gx = sr * x, gy = sr * y, gz = sr * z;
                 if (e < nA) { gx += L.ang[e * 3]; gy += L.ang[e * 3 + 1]; gz += L.ang[e * 3 + 2]; }
                 if (seg_g) {

@@ -365,6 +365,7 @@ def run_nep_md(args, kind, size, rebuild=True, via_ops=False):
         # the energy / force / virial operator as a whole, against the fp32 vector peak: whichever kernels serve it
         "nep_adjoint_kernel+nep_gather_kernel": valu,
         "nep_stage_kernel+nep_staged_kernel+reduce_sum": valu,
+        "nep_quad_kernel+reduce_sum": valu,
         "nep_wave_kernel+reduce_sum": valu,
         "nep_efv_kernel": valu,
         "nbl_lists": ("hbm", nbl_bytes_per_atom(nn_r, s, 200, rebuild) * n, "GB/s", PEAK_HBM_GBS, 1e9, "hbm"),
