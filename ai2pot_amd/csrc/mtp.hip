@@ -733,12 +733,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                 for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
             return;
         }
-        center = __builtin_amdgcn_readfirstlane(a.bilist[row]);
-        nn = __builtin_amdgcn_readfirstlane(a.bnumneigh[row]);
-        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
-        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-        ti = __builtin_amdgcn_readfirstlane(types[center]);
-        if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
+        const int center0 = a.bilist[row], nn0 = a.bnumneigh[row];         // on their way while the plan's arrays are fetched
 
         mgroups = a.mom_groups;       // uniform over the launch
         const unsigned* const bsrc = mgroups ? (const unsigned*)p.poly_pos : p.basic;
@@ -762,6 +757,12 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             for (int i = lane; i < p.npoly; i += NT) rws[i] = p.polys_mu[i];
             for (int i = lane; i <= nmus; i += NT) rws[p.npoly + i] = p.polys_end[i];
         }
+        center = __builtin_amdgcn_readfirstlane(center0);
+        nn = __builtin_amdgcn_readfirstlane(nn0);
+        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
+        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
+        ti = __builtin_amdgcn_readfirstlane(types[center]);
+        if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
         for (int i = lane; i < n_moms; i += NT) {
             M[i] = (T)0;
