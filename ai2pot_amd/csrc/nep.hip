@@ -451,8 +451,8 @@ constexpr long long quad_most() { return sizeof(T) == 4 ? 1ll << 62 : 49152; }
 // Atoms up to which a wavefront per atom beats four atoms per wavefront: its chain is a third shorter, and it repeats most of its
 // instructions for every atom, which costs nothing while a SIMD holds one to three wavefronts (fp32; fp64: one, by registers).
 // Kernel, 16 and 72 neighbours, us (one / four): fp32 108 atoms 12.1 / 16.0 and 16.0 / 23.0, 2000 15.1 / 16.4 and 23.5 / 27.4,
-// 3000 17.9 / 17.1 and 25.9 / 27.1, 4096 24.3 / 17.3 and 34.4 / 27.3; fp64 1000 16.8 / 20.5 and 22.9 / 34.1, 1500 29.7 / 20.6
-// and 37.9 / 35.4.
+// 3000 17.9 / 17.1 and 25.9 / 27.1, 4096 24.3 / 17.3 and 34.4 / 27.3; fp64 one for 1000 atoms 15.9 and 21.8, four for 1500 20.0 and
+// 29.8, where one takes 29 and 37.
 template <typename T>
 constexpr long long wave_most() { return sizeof(T) == 4 ? 2560 : 1024; }
 

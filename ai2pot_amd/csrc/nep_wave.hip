@@ -87,7 +87,7 @@ struct SegArgs {
 // Slots [128 t, 128 t + 128) of a row, of which `room` are read: lane = slot, both halves in flight.
 template <typename T>
 struct Slots {
-    int nj[2];
+    int nj[2], tj[2];
     T x[2], y[2], z[2];
 };
 template <typename T>
@@ -106,13 +106,19 @@ __device__ __forceinline__ void load_slots(const NepArgs<T>& a, int t, int lane,
         }
     }
 }
+// ... and the species of the neighbours
+template <typename T>
+__device__ __forceinline__ void load_species(const int* types, int NF, Slots<T>& o)
+{
+#pragma unroll
+    for (int h = 0; h < 2; h++) o.tj[h] = (unsigned)o.nj[h] < (unsigned)NF ? types[o.nj[h]] : -1;
+}
 // They into the wavefront's tile; nA / nR: entries at its front / back.
 template <typename T>
 __device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& seg, T* __restrict__ seg_g,
                                           const WaveLds<T>& L, int t, int lane, size_t row, int b, int NF, int nn, T rr,
                                           T ra, bool claim, const Slots<T>& in, int& nA, int& nR)
 {
-    const int* types = a.btypes + (size_t)b * NF;
     const unsigned long long lt = (1ull << lane) - 1ull;
     nA = 0; nR = 0;
     const int (&nj)[2] = in.nj;
@@ -123,8 +129,7 @@ __device__ __forceinline__ void load_tile(const NepArgs<T>& a, const SegArgs& se
         const int slot = t * NW_CAP + h * 64 + lane;
         const bool bad = slot < nn && (unsigned)nj[h] >= (unsigned)NF;
         if (bad) atomicOr(a.status, ST_BAD_NEIGHBOR);
-        tj[h] = -1;
-        if (slot < nn && !bad) tj[h] = types[nj[h]];
+        tj[h] = slot < nn && !bad ? in.tj[h] : -1;
     }
 #pragma unroll
     for (int h = 0; h < 2; h++) {
@@ -188,6 +193,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
     const int center1 = a.bilist[row1], nn1 = a.bnumneigh[row1];
     Slots<T> slots;
     load_slots<T>(a, 0, lane, row1, a.U, slots);
+    const int* const types = a.btypes + (size_t)b * NF;
+    int ti1;
     {
         // The model's tables: the first values of every thread are all on their way before one is stored.
         constexpr int W0 = sizeof(T) == 4 ? 16 : 8, C0 = 4;
@@ -201,6 +208,8 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
         for (int u = 0; u < W0; u++) { const int i = tid + u * NW_THREADS; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
         if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
         if (tid < D) qs = a.q_scaler[tid];
+        ti1 = types[(unsigned)center1 < (unsigned)NF ? center1 : 0];
+        load_species<T>(types, NF, slots);
 #pragma unroll
         for (int u = 0; u < C0; u++) { const int i = tid + u * NW_THREADS; if (i < nc) put_coef(i, c0[u]); }
 #pragma unroll
@@ -226,7 +235,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
         int center = ii == first ? center1 : a.bilist[row], nn = ii == first ? nn1 : a.bnumneigh[row];
         if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
         if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-        int ti = a.btypes[(size_t)b * NF + center];
+        int ti = ii == first && center == center1 ? ti1 : types[center];
         if ((unsigned)ti >= (unsigned)nt) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         const int ntiles = (nn + NW_CAP - 1) / NW_CAP;
         const T* const cti = L.coef + (size_t)ti * nt * CROW;
@@ -240,7 +249,10 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
         int nA = 0, nR = 0;
         for (int t = 0; t < ntiles; t++) {
             // (a row of several tiles is read again for the forces, and its pairs claim their places then)
-            if (t > 0 || ii != first) load_slots<T>(a, t, lane, row, nn, slots);
+            if (t > 0 || ii != first) {
+                load_slots<T>(a, t, lane, row, nn, slots);
+                load_species<T>(types, NF, slots);
+            }
             load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, ntiles == 1, slots, nA, nR);
             for (int e = lane; e < nA + nR; e += 64) {
                 T x, y, z;
@@ -378,6 +390,7 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
         for (int t = 0; t < ntiles; t++) {
             if (ntiles > 1) {
                 load_slots<T>(a, t, lane, row, nn, slots);
+                load_species<T>(types, NF, slots);
                 load_tile<T>(a, seg, seg_g, L, t, lane, row, b, NF, nn, rr, ra, true, slots, nA, nR);
             }
             for (int e0 = 0; e0 < nA; e0 += 16) {
