@@ -2270,13 +2270,13 @@ int plan_check(void* handle, MtpPlan** out)
 }
 
 // 256 threads per atom or 64 (the rule is at its definition)
-bool wide_atoms(int n_moms, bool loss, bool network);
+bool wide_atoms(int n_moms, bool loss, bool network, bool fp64);
 
 // Whether the atom kernel sums the basic moments by polynomials (basic_sums): each has a thread, and the sums of a group
 // of threads fit the place of the shortest table.  Otherwise each moment is formed by itself, from powers of z.
-bool poly_sums(const MtpPlanDevice& p, bool loss, bool network)
+bool poly_sums(const MtpPlanDevice& p, bool loss, bool network, bool fp64)
 {
-    return p.polys_len && p.poly_top <= MTP_POLY_MAX && p.npoly <= (wide_atoms(p.n_moms, loss, network) ? 256 : 64) &&
+    return p.polys_len && p.poly_top <= MTP_POLY_MAX && p.npoly <= (wide_atoms(p.n_moms, loss, network, fp64) ? 256 : 64) &&
            (loss ? 2 : 1) * p.ncoef_poly <= MTP_NC_MIN * (2 * (p.kmax + 1) + 2 * p.nmus + 4);
 }
 
@@ -2296,7 +2296,7 @@ void table_layout(MtpArgs<T>& a, bool loss, bool z_powers)
 template <typename T>
 void table_layout(MtpArgs<T>& a, bool loss)
 {
-    table_layout(a, loss, !poly_sums(a.p, loss, a.H > 0));
+    table_layout(a, loss, !poly_sums(a.p, loss, a.H > 0, sizeof(T) == 8));
 }
 
 template <typename T>
@@ -2354,17 +2354,18 @@ int g_keep_table = 1;      // (measurement switch: AI2POT_MTP_KEEP_TABLE=0)
 // 256 threads per atom or 64: a rule on the tables alone, so that a structure's results do not depend on the batch it is
 // in (the sums over neighbours are grouped by the threads).  Kernel times in us, 64 / 256 threads, fp64, energy / force /
 // virial (8,000 atoms; 250 atoms) and loss gradient (8,000; 250):
-//   level 8 (18 moments)   44 / 106   15.5 / 16.3   132 / 172   36 / 38
-//   level 10 (41)          49 / 113   19.0 / 17.5   185 / 188   39 / 41
-//   level 12 (84)          56 / 121   19.0 / 17.5   203 / 200   42 / 43
-//   level 14 (174)         82 / 130   28 / 19       301 / 249   53 / 47
-//   level 16 (350)        109 / 148   35 / 20       (loss: 256 threads before)
-//   level 18 (718)        194 / 183
+//   level 8 (18 moments)   40 / 90    13.9 / 14.9    89 / 125   24 / 29
+//   level 10 (41)          43 / 94    15.2 / 15.6   118 / 129   28 / 30
+//   level 12 (84)          48 / 101   16.1 / 15.9   154 / 139   32 / 30
+//   level 14 (174)         56 / 106   18.7 / 16.6   219 / 175   40 / 34
+//   level 16 (350)         78 / 124   24 / 17.7     243 / 188   48 / 37
+//   level 18 (718)        143 / 155   34 / 20       551 / 307   77 / 43
 // With a network the loss gradient has a weight per neuron and scalar moment besides (64 x 125 atoms; 2 x 60; 30 neurons):
-//   level 8  221 / 211 (10 neurons: 170 / 186)   46 / 40      level 10  273 / 230   51 / 44      level 12  304 / 247   56 / 46
-bool wide_atoms(int n_moms, bool loss, bool network)
+//   level 8  160 / 160, 28 / 24 (10 neurons: 112 / 139, 23 / 21)   level 10  185 / 168, 33 / 24   level 12  240 / 184, 38 / 25
+// fp32, level 12: 84 / 126, 31 / 30; 14: 108 / 138, 38 / 33; 18: 275 / 212, 77 / 41.
+bool wide_atoms(int n_moms, bool loss, bool network, bool fp64)
 {
-    return n_moms >= (loss ? (network ? 40 : 150) : 600);
+    return n_moms >= (loss ? (network ? 40 : fp64 ? 80 : 150) : 600);
 }
 
 template <typename T, bool LOSS, bool SEED = false>
@@ -2374,7 +2375,7 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         static const char* e = getenv("AI2POT_MTP_KEEP_TABLE");
         if (e) g_keep_table = e[0] != '0';
     }
-    const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0);
+    const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0, sizeof(T) == 8);
     const int groups = a.z_powers ? 0 : (wide ? 256 : 64) / std::max(a.p.npoly, 1);      // of a thread per polynomial
     const int kept_adjoints = std::max(a.p.n_moms, groups * a.p.ncoef_poly);
     auto lds_for = [&](int nc, size_t* main, int keep = 0) {
