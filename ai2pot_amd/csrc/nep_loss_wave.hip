@@ -13,14 +13,15 @@
 // dPhi/dW0 = sum over the atoms of a species of alpha q^T + beta qdot^T is left to the second kernel, as a matrix product
 // over the atoms: an atom's row carries the four vectors (144 values at 50 neurons) instead of the product (1100).
 //
-// Bound: issue of the vector instructions and the chain of an atom, with two workgroups of four wavefronts per compute
-// unit (LDS).  64 structures of 128 atoms, fp32, 3 species, 50 neurons: 179 -> 59 us against 128 threads per atom, and
+// Bound: issue of the vector instructions and the chain of an atom, with two workgroups (fp64: one) of four wavefronts per
+// compute unit (LDS).  64 structures of 128 atoms, fp32, 3 species, 50 neurons: 179 -> 59 us against 128 threads per atom, and
 // 25 -> 9.8 us for the sums over the atoms.  59 -> 52 by the next atom's first slots and the tables on their way early (tables
 // 8.9 -> 5.1 thousand cycles) and by a descriptor's moments read together (4.5 -> 2.3 of 25.6 thousand cycles an atom).
 #include "a2p_common.h"
 #include "nep_device.h"
 #include "nep_loss.h"
 #include "wave_ops.h"
+#include <climits>
 
 namespace a2p {
 using namespace nepdev;
@@ -28,6 +29,12 @@ using namespace wave;
 namespace {
 
 constexpr int LW_THREADS = 256, LW_WAVES = LW_THREADS / 64;
+// Workgroups per compute unit, what the LDS leaves: 53 KB of an fp32 workgroup's wavefronts and the tables, twice that in fp64.
+// A bound of two in fp64 buys no second workgroup and costs the loop over the atoms up to 63 spilled registers; and a grid for
+// two of them loads the tables a second time, with half of the atoms.  64 structures of 128 atoms, fp64, 3 species: 135 -> 117
+// us by the registers, -> 113 by the grid; 5 of 500: 71 -> 61 -> 48; 8 of 60 (one atom per wavefront): 21 -> 18.
+template <typename T>
+constexpr int LW_GROUPS = sizeof(T) == 4 ? 2 : 1;
 constexpr int KC = 8, NAC = 4;
 constexpr int WROW = 28;                     // row of w0 in LDS: see nep_wave.hip
 constexpr int CPAD = 4;
@@ -79,7 +86,7 @@ __host__ __device__ __forceinline__ size_t loss_wave_layout(int nt, int H, int n
 static_assert(CH * TS >= 64 * RS, "the radial table uses the angular one's place");
 
 template <typename T, int NR, int LC>
-__global__ void __launch_bounds__(LW_THREADS, 2) nep_loss_wave_kernel(const NepLossArgs<T> a)
+__global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel(const NepLossArgs<T> a)
 {
     constexpr int NLM = LC * LC + 2 * LC, NB = NR + NAC, D = NR + NAC * LC, CROW = NB * KC + CPAD;
     static_assert(D <= WROW && D <= 32, "descriptor count exceeds the padded row");
@@ -546,14 +553,31 @@ nep_loss_wave_reduce_kernel(const NepLossArgs<T> a, int sum_blocks, T* __restric
     }
 }
 
+// Workgroups per structure: the number with the shortest way through the device, in rounds of `room` workgroups, each the
+// atoms of a wavefront and the tables (a quarter of an atom: 4 of 14 us in fp64, 5 of 26 thousand cycles in fp32).  One round
+// unless the batch does not divide the room well: room / B workgroups each left 129 structures of 64 atoms on half of the device
+// (fp64: 208 us, now 151), 200 of 40 on 400 of the 512 places (fp32: 60 us, now 53), 300 of 30 in two rounds of which the second
+// was nearly empty (fp64 244 -> 152, fp32 89 -> 70).
+int loss_wave_blocks(int P, int B, int room)
+{
+    const int most = ceil_div(P, LW_WAVES);
+    int best = 1;
+    long long least = LLONG_MAX;
+    for (int round = 1; round <= ceil_div(B, room) + 3; round++) {
+        const int n = std::max(1, std::min<int>(most, (long long)round * room / B));
+        const long long way = (long long)ceil_div((long long)n * B, (long long)room) * (4ll * ceil_div(P, n * LW_WAVES) + 1);
+        if (way < least) { least = way; best = n; }
+    }
+    return best;
+}
+
 template <typename T, int NR, int LC>
 int launch_loss_wave(const NepLossArgs<T>& a, size_t lds, hipStream_t stream)
 {
     auto kern = nep_loss_wave_kernel<T, NR, LC>;
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    // an atom per wavefront until the batch has two workgroups per compute unit, from there on several
-    const int nblk = std::max(1, std::min(ceil_div(a.P, LW_WAVES), 512 / a.B));
+    const int nblk = loss_wave_blocks(a.P, a.B, LW_GROUPS<T> * 256);
     prof_begin("nep_loss_bwd_kernel", stream);
     hipLaunchKernelGGL(kern, dim3(nblk, a.B), dim3(LW_THREADS), lds, stream, a);
     prof_end(stream);
