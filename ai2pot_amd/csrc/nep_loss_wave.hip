@@ -150,6 +150,7 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
         if ((unsigned)center >= (unsigned)a.P) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
         int ti = types[center];
         if ((unsigned)ti >= (unsigned)nt) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
+        if (nn == 0) begin(ii + gridDim.x * LW_WAVES);        // (no first slots below, behind which the next row is fetched)
         const T* const cti = L.coef + (size_t)ti * nt * CROW;
         T* const grow = a.gpart + row * a.nrow;
         T* const g_alpha = grow + nt * NB * KC;
