@@ -775,8 +775,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     int nchunks, csize;
     {
         MTP_PHASE;
-        nchunks = __builtin_amdgcn_readfirstlane(small_div(nn + MTP_NC - 1, MTP_NC));
-        csize = nchunks > 1 ? __builtin_amdgcn_readfirstlane(small_div(nn + nchunks - 1, nchunks)) : max(nn, 1);
+        // (whole-number divisions: small_div cuts a row of two million and more into chunks longer than the table)
+        const unsigned n = nn, cap = MTP_NC, cuts = (n + cap - 1) / cap;
+        nchunks = (int)cuts;
+        csize = cuts > 1 ? (int)((n + cuts - 1) / cuts) : max(nn, 1);
     }
 
     // ---- basic moments (and their tangents) --------------------------------------------------

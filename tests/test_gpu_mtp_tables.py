@@ -96,3 +96,28 @@ def test_components_in_chunks_of_structures(oracle):
     alone = components(d)
     for whole, one in zip(components(batch), alone):
         assert torch.equal(whole, one.expand_as(whole))
+
+
+# A million neighbours and more in one row: lengths at which a single-precision quotient makes chunks of 33 for a table of
+# 32, or of 49 for 48 (with the reciprocal rounded to nearest or one place above), and one that it gets right.
+@pytest.mark.parametrize("level,n", [(10, 1 << 20), (10, 2618352), (10, 5449248), (8, 2625408), (20, 2074272), (20, 4154976)])
+def test_rows_of_millions(level, n):
+    """A row whose neighbours all lie beyond the cutoff but a few, the last one of every 1000th chunk: energies, forces and
+    virials of the row of those few."""
+    from ai2pot_amd import mtp_param
+    m = synth.mtp_model(mtp_param.mtp_param(level), 1, 6, 5.0, 1.5, 3210)
+    cap = 48 if level < 20 else 32
+    size = -(-n // -(-n // cap))
+    at = np.arange(size - 1, n, 1000 * size)
+    rng = np.random.default_rng(level)
+    few = rng.normal(size=(len(at), 3))
+    few *= (rng.uniform(2.0, 4.9, len(at)) / np.linalg.norm(few, axis=1))[:, None]
+    common = dict(binum=np.array([1], np.int32), bilist=np.zeros((1, 2), np.int32), btypes=np.zeros((1, 2), np.int32), nghost=0)
+    row = lambda r: dict(common, bnumneigh=np.array([[len(r), 0]], np.int32), bfirstneigh=np.ones((1, 2, len(r)), np.int32),
+                         brcs=np.stack([r, r])[None])
+    far = np.full((n, 3), 4.0)
+    far[at] = few
+    # sums of the same few hundred terms in another order
+    for got, want in zip(gpu_efv(m, row(far)), gpu_efv(m, row(few))):
+        assert np.abs(want).max() > 0
+        assert close(got, want)
