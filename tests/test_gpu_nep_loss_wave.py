@@ -106,6 +106,9 @@ def test_lone_atoms_of_a_large_structure(np_dtype, lone):
               bfirstneigh=rng.integers(0, P, (1, P, U)).astype(np.int32),
               brcs=(u * (r / np.linalg.norm(u, axis=3))[..., None]).astype(np_dtype),
               btypes=rng.integers(0, ntypes, (1, P)).astype(np.int32), nghost=0)
+    beyond = np.arange(U) >= rows[:, None]                  # padded entries hold anything
+    nb["bfirstneigh"][0, beyond] = rng.choice([-1, 1 << 30, P], beyond.sum())
+    nb["brcs"][0, beyond] = np.nan
     m = synth.nep_model(ntypes=ntypes, n_radial_basis=4, l_max=3, num_neurons=H, sigma=0.12)
     m["type_map"] = np.arange(1, ntypes + 1, dtype=np.int32)
     m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
