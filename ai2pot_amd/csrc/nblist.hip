@@ -461,8 +461,8 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
 // few) and bins one slab of the box, a plane of bins across x or a few, with its counters in LDS: the images in its slab
 // are listed and dealt to their bins, those in the slabs before it are only counted, which says where its records begin,
 // and every record is written once, to its final place (an image's place in its bin is the number of larger image numbers
-// there).  No workgroup waits for another.  4096 atoms take 14.5 us (one workgroup for the whole box: 31), of which extents
-// and grid 5, finding the images 4, dealing them 3.
+// there).  No workgroup waits for another.  4096 atoms take 14.5 us in lattice order (16.9 in no spatial order; one workgroup
+// for the whole box, in lattice order: 31), of which extents and grid 5, finding the images 4, dealing them 3.
 // Told axis by axis (diagonal lattice, at most three images an axis), an image is placed by comparisons with the edges of
 // the box and of the slab; the exactly rounded division decides next to an edge only, and for the bins of the slab's own.
 // Other lattices are tried image by image.  Images of a slab beyond its LDS (atoms crowded into a corner of the cell are

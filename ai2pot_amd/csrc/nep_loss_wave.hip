@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
                         ent_load(L.ent + e * 4, x, y, z, tj);
                         lds_load4(L.W + e * 4, w);
                         T rinv;
-                    const T r = length<false>(x * x + y * y + z * z, rinv);
+                        const T r = length<false>(x * x + y * y + z * z, rinv);
                         x *= rinv; y *= rinv; z *= rinv;
                         radial_basis<T, KC, true>(r, ra_inv, KC, fa, fad);
 #pragma unroll

@@ -18,10 +18,11 @@
 // Registers decide how many wavefronts a SIMD holds: each phase takes arguments, LDS addresses and the lane's place anew.  With
 // 60 values spilled for three wavefronts the kernel took 89 us at 20,011 atoms, with two 72, so 58.
 //
-// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms 34 -> 22 us, 20,011 with
-// skin lists 94 -> 57, 64 structures of 128 atoms 43 -> 25.  Of the 43 thousand cycles of a wavefront at 4096 atoms the tables
-// take 6.4, slots 7, angular pairs and moments 6, read-out 10, angular forces 2.2, radial forces 4.6.  Taken back: two neurons a
-// lane at a time (8 values spilled: 61 us), the neurons of dE/dq by fours (57 -> 58).
+// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 22 us
+// (28 now for the same atoms in no spatial order), 20,011 with skin lists 94 -> 57, 64 structures of 128 atoms 43 -> 25.
+// Of the 43 thousand cycles of a wavefront at 4096 atoms the tables take 6.4, slots 7, angular pairs and moments 6, read-out 10,
+// angular forces 2.2, radial forces 4.6.  Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq
+// by fours (57 -> 58).
 //
 // Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
 #include "a2p_common.h"
