@@ -50,6 +50,43 @@ struct NepArgs {
     int mb4 = 0, mb5 = 0;   // extension (generic kernel only): four- / five-body invariant per angular channel
 };
 
+// What the kernels that store a pair derivative straight into its target's segment know of the segments (PairCsr).
+struct SegArgs {
+    int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
+    int cap;       // capacity of a segment
+    int spare;     // entry that takes what overflows a segment
+    int mark;      // own sums are marked in the cursors (PairCsr)
+};
+
+// The model's tables in LDS, staged by the workgroup: w0 in rows of WROW values, the coefficients of a species pair in rows of
+// NB * KC + CPAD.  The first W0 and four values of every thread are all on their way before one is stored, behind them
+// whatever `early` asks for.
+template <int KC, int NB, int D, int WROW, int CPAD, int W0, typename T, typename Args, typename Lds, typename Early>
+__device__ __forceinline__ void stage_tables(Args& a, const Lds& L, int tid, int nthreads, Early early)
+{
+    constexpr int C0 = 4;
+    const int nt = a.ntypes, H = a.H, nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
+    T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
+    auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
+    auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * (NB * KC + CPAD) + (i - p * NB * KC)] = v; };
+#pragma unroll
+    for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
+#pragma unroll
+    for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
+    if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
+    if (tid < D) qs = a.q_scaler[tid];
+    early();
+#pragma unroll
+    for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; if (i < nc) put_coef(i, c0[u]); }
+#pragma unroll
+    for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; if (i < nw0) put_w0(i, w0[u]); }
+    if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
+    if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
+    for (int i = tid + C0 * nthreads; i < nc; i += nthreads) put_coef(i, a.coeffs[i]);
+    for (int i = tid + W0 * nthreads; i < nw0; i += nthreads) put_w0(i, a.w0[i]);
+    for (int i = tid + nthreads; i < nh; i += nthreads) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
+}
+
 // r and 1 / r from r^2: the estimate of 1 / r and a Newton step for each, a third of the operations of square root and
 // division, and no further from fp64 (forces 4.65e-7 with either).  Adjoint kernel of 1,048,576 atoms 631 -> 620 us, gather
 // kernel, which waits for memory, 334 -> 331.  r^2 = 0 gives NaN, as 0 / 0 does; MIN keeps it from that.

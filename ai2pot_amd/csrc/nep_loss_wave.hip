@@ -108,29 +108,7 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
         x1 = a.brcs[pr * 3]; y1 = a.brcs[pr * 3 + 1]; z1 = a.brcs[pr * 3 + 2];
     };
     begin(blockIdx.x * LW_WAVES + wave);
-    {
-        // The model's tables: the first values of every thread are all on their way before one is stored.
-        constexpr int W0 = sizeof(T) == 4 ? 16 : 8, C0 = 4;
-        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
-        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
-        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
-        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * LW_THREADS; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * LW_THREADS; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
-        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
-        if (tid < D) qs = a.q_scaler[tid];
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * LW_THREADS; if (i < nc) put_coef(i, c0[u]); }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * LW_THREADS; if (i < nw0) put_w0(i, w0[u]); }
-        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
-        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
-        for (int i = tid + C0 * LW_THREADS; i < nc; i += LW_THREADS) put_coef(i, a.coeffs[i]);
-        for (int i = tid + W0 * LW_THREADS; i < nw0; i += LW_THREADS) put_w0(i, a.w0[i]);
-        for (int i = tid + LW_THREADS; i < nh; i += LW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
-    }
+    stage_tables<KC, NB, D, WROW, CPAD, sizeof(T) == 4 ? 16 : 8, T>(a, L, tid, LW_THREADS, []() {});
     if (tid < LM) {
         const int l = l_of_lm(tid);
         L.wc[tid] = tid < NLM ? (T)(tid == l * l - 1 ? 1.0 : 2.0) * (T)kC3B[tid] : (T)0;

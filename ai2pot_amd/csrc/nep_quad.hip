@@ -106,13 +106,6 @@ struct WaveLds {
     }
 };
 
-struct SegArgs {
-    int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
-    int cap;       // capacity of a segment
-    int spare;     // entry that takes what overflows a segment
-    int mark;      // own sums are marked in the cursors (PairCsr)
-};
-
 // N values (N even) behind an address aligned to two of them
 template <typename T, int N>
 __device__ __forceinline__ void lds_load_even(const T* p, T (&o)[N])
@@ -235,33 +228,15 @@ nep_quad_kernel(const WaveArgs<T>)
     const int nwaves = blockDim.x >> 6, first = NW_ATOMS * (wave * gridDim.x + blockIdx.x), stride = NW_ATOMS * nwaves * gridDim.x;
     begin(first);
     {
-        // The model's tables: the first values of every thread are all on their way before one is stored.
         NW_PHASE;
         const int tid = threadIdx.x, nthreads = blockDim.x;
-        constexpr int W0 = 16, C0 = 4;
-        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
-        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1, bias = (T)0;
-        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
-        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
-        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
-        if (tid < nt) bias = a.bias[tid];
-        if (tid < D) qs = a.q_scaler[tid];
-        if constexpr (EARLY) begin_species();
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; if (i < nc) put_coef(i, c0[u]); }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; if (i < nw0) put_w0(i, w0[u]); }
-        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
+        T bias = (T)0;
+        stage_tables<KC, NB, D, WROW, CPAD, 16, T>(a, L, tid, nthreads, [&]() __attribute__((always_inline)) {
+            if (tid < nt) bias = a.bias[tid];
+            if constexpr (EARLY) begin_species();
+            if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)kC3B[tid] : (T)0;
+        });
         if (tid < nt) L.bias[tid] = bias;
-        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
-        if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)kC3B[tid] : (T)0;
-        for (int i = tid + C0 * nthreads; i < nc; i += nthreads) put_coef(i, a.coeffs[i]);
-        for (int i = tid + W0 * nthreads; i < nw0; i += nthreads) put_w0(i, a.w0[i]);
-        for (int i = tid + nthreads; i < nh; i += nthreads) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
         for (int i = tid + nthreads; i < nt; i += nthreads) L.bias[i] = a.bias[i];
     }
     __syncthreads();

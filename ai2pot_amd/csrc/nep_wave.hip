@@ -77,13 +77,6 @@ __host__ __device__ __forceinline__ size_t wave_lds_layout(int nt, int H, int nb
     return shared + own * NW_WAVES;
 }
 
-struct SegArgs {
-    int* cursor;   // [B * NF] entries claimed so far in each target's reduction segment, or null (no forces)
-    int cap;       // capacity of a segment
-    int spare;     // entry that takes what overflows a segment
-    int mark;      // own sums are marked in the cursors (PairCsr)
-};
-
 // Slots [128 t, 128 t + 128) of a row, of which `room` are read: lane = slot, both halves in flight.
 template <typename T>
 struct Slots {
@@ -195,31 +188,10 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
     load_slots<T>(a, 0, lane, row1, a.U, slots);
     const int* const types = a.btypes + (size_t)b * NF;
     int ti1;
-    {
-        // The model's tables: the first values of every thread are all on their way before one is stored.
-        constexpr int W0 = sizeof(T) == 4 ? 16 : 8, C0 = 4;
-        const int nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
-        T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
-        auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
-        auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * CROW + (i - p * NB * KC)] = v; };
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * NW_THREADS; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * NW_THREADS; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
-        if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
-        if (tid < D) qs = a.q_scaler[tid];
+    stage_tables<KC, NB, D, WROW, CPAD, sizeof(T) == 4 ? 16 : 8, T>(a, L, tid, NW_THREADS, [&]() __attribute__((always_inline)) {
         ti1 = types[(unsigned)center1 < (unsigned)NF ? center1 : 0];
         load_species<T>(types, NF, slots);
-#pragma unroll
-        for (int u = 0; u < C0; u++) { const int i = tid + u * NW_THREADS; if (i < nc) put_coef(i, c0[u]); }
-#pragma unroll
-        for (int u = 0; u < W0; u++) { const int i = tid + u * NW_THREADS; if (i < nw0) put_w0(i, w0[u]); }
-        if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
-        if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
-        for (int i = tid + C0 * NW_THREADS; i < nc; i += NW_THREADS) put_coef(i, a.coeffs[i]);
-        for (int i = tid + W0 * NW_THREADS; i < nw0; i += NW_THREADS) put_w0(i, a.w0[i]);
-        for (int i = tid + NW_THREADS; i < nh; i += NW_THREADS) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
-    }
+    });
     __syncthreads();
 
     const int inum = min(a.binum[b], a.P);            // (the loop below strides over the rows: none beyond the last)
