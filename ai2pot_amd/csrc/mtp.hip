@@ -1876,49 +1876,94 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         std::vector<int2> terms;
         bool too_long = false;
     };
-    auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level) {
+    // Cuts the lists of one level into pieces of at most `cap` terms and lays them out in rows of sixteen lanes.
+    struct Piece { int m, t0, n, rem; };
+    struct Level {
+        std::vector<Piece> lanes;                          // rows of sixteen, deepest first; whole groups of 64
+        std::vector<int> depth, steps;                     // of each group
+        double cost = 0;
+    };
+    auto pack_level = [&](const std::vector<std::vector<int2>>& lists, const std::vector<int>& members, int cap, int waves) {
+        struct List { int m, n, np, len; };
+        std::vector<List> ls;
+        for (int m : members) {
+            const int n = (int)lists[m].size(), np = (n + cap - 1) / cap;
+            ls.push_back({m, n, np, np ? (n + np - 1) / np : 0});       // pieces of equal length
+        }
+        auto deep = [](int n) { return (n + MTP_DEPTH_STEP - 1) / MTP_DEPTH_STEP * MTP_DEPTH_STEP; };
+        std::stable_sort(ls.begin(), ls.end(), [&](const List& x, const List& y) {
+            return deep(x.len) != deep(y.len) ? deep(x.len) > deep(y.len) : x.np > y.np;
+        });
+        Level lv;
+        std::vector<int> room;                             // free lanes of each row
+        for (const List& l : ls) {
+            if (l.np == 0) continue;
+            size_t r = 0;
+            int at;
+            if (l.np > 16) {                               // whole rows within a group (the last one has room left)
+                const size_t need = (l.np + 15) / 16;
+                while (room.size() % 4 + need > 4) room.push_back(16);
+                r = room.size();
+                for (size_t q = 0; q < need; q++) room.push_back(0);
+                room.back() = (int)need * 16 - l.np;
+                at = 0;
+            } else {
+                while (r < room.size() && room[r] < l.np) r++;
+                if (r == room.size()) room.push_back(16);
+                at = 16 - room[r];
+                room[r] -= l.np;
+            }
+            lv.lanes.resize(room.size() * 16, Piece{-1, 0, 0, 0});
+            for (int q = 0; q < l.np; q++)
+                lv.lanes[r * 16 + at + q] = {l.m, q * l.len, std::min(l.len, l.n - q * l.len), l.np - 1 - q};
+        }
+        while (lv.lanes.size() % 64) lv.lanes.push_back({-1, 0, 0, 0});
+        // what a wavefront issues: a term about ten instructions, a group about 25, a doubling step about nine; the workgroup
+        // waits for its slowest wavefront, and the others' share is what other workgroups can use meanwhile
+        std::vector<double> load(waves, 0.0);
+        double all = 0;
+        for (size_t g = 0; g < lv.lanes.size(); g += 64) {
+            int n = 0, rem = 0, steps = 0;
+            for (size_t q = g; q < g + 64; q++) { n = std::max(n, lv.lanes[q].n); rem = std::max(rem, lv.lanes[q].rem); }
+            while ((1 << steps) < rem + 1) steps++;
+            lv.depth.push_back(deep(n));
+            lv.steps.push_back(steps);
+            const double c = 10.0 * deep(n) + 25.0 + 9.0 * steps;
+            *std::min_element(load.begin(), load.end()) += c;
+            all += c;
+        }
+        lv.cost = *std::max_element(load.begin(), load.end()) + all / waves;
+        return lv;
+    };
+    auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level, int waves) {
         Ell e;
         for (const auto& members : by_level) {
             e.level.push_back((int)e.slot.size());
-            std::vector<int> ms = members;
-            std::stable_sort(ms.begin(), ms.end(),
-                             [&](int x, int y) { return lists[x].size() > lists[y].size(); });
-            // slots of the level: (list, first term, term count, pieces behind this one); the pieces of a list are
-            // adjacent and stay inside one group of 64 slots (one wavefront adds them up with shuffles)
-            struct Piece { int m, t0, n, rem; };
-            std::vector<Piece> pieces;
-            for (int m : ms) {
-                const int n = (int)lists[m].size();
-                const int np = (n + MTP_SLOT_CAP - 1) / MTP_SLOT_CAP;
-                if (np > 64) { e.too_long = true; continue; }
-                if ((int)(pieces.size() % 16) + np > 16)                  // a row of sixteen lanes, or from its beginning on
-                    while (pieces.size() % 16) pieces.push_back({-1, 0, 0, 0});
-                if ((int)(pieces.size() % 64) + np > 64)
-                    while (pieces.size() % 64) pieces.push_back({-1, 0, 0, 0});
-                for (int q = 0; q < np; q++)
-                    pieces.push_back({m, q * MTP_SLOT_CAP, std::min(MTP_SLOT_CAP, n - q * MTP_SLOT_CAP), np - 1 - q});
+            std::vector<int> ms;
+            for (int m : members) {
+                if ((int)lists[m].size() > 64 * MTP_SLOT_CAP) e.too_long = true;
+                else ms.push_back(m);
             }
-            for (size_t g0 = 0; g0 < pieces.size(); g0 += 64) {
-                const size_t g1 = std::min(pieces.size(), g0 + 64);
-                int depth = 0, longest = 1;
-                for (size_t q = g0; q < g1; q++) {
-                    depth = std::max(depth, pieces[q].n);
-                    longest = std::max(longest, pieces[q].rem + 1);
-                }
-                int steps = 0;                      // doubling steps that add up the pieces of this group's lists
-                while ((1 << steps) < longest) steps++;
-                depth = (depth + MTP_DEPTH_STEP - 1) / MTP_DEPTH_STEP * MTP_DEPTH_STEP;    // the sweeps fetch that many terms at a time
-                e.group.push_back(make_int4((int)e.terms.size(), depth, steps, 0));
-                e.terms.resize(e.terms.size() + (size_t)depth * 64, make_int2(0, 0));
-                for (size_t q = g0; q < g1; q++) {
-                    const Piece& pc = pieces[q];
+            Level best;
+            bool any = false;
+            for (int cap = MTP_DEPTH_STEP; cap <= MTP_SLOT_CAP; cap += MTP_DEPTH_STEP) {
+                bool fits = true;
+                for (int m : ms) fits = fits && (int)lists[m].size() <= 64 * cap;
+                if (!fits) continue;
+                Level lv = pack_level(lists, ms, cap, waves);
+                if (!any || lv.cost < best.cost) { best = std::move(lv); any = true; }
+            }
+            for (size_t g = 0; g < best.depth.size(); g++) {
+                e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], 0));
+                e.terms.resize(e.terms.size() + (size_t)best.depth[g] * 64, make_int2(0, 0));
+                for (size_t q = 0; q < 64; q++) {
+                    const Piece& pc = best.lanes[g * 64 + q];
                     for (int k = 0; k < pc.n; k++)
-                        e.terms[e.group.back().x + (size_t)k * 64 + (q - g0)] = lists[pc.m][pc.t0 + k];
+                        e.terms[e.group.back().x + (size_t)k * 64 + q] = lists[pc.m][pc.t0 + k];
                     e.slot.push_back(pc.n > 0 && pc.t0 == 0 ? pc.m : -1);      // the first piece of a list names the moment
                     e.lead.push_back(pc.rem);
                 }
             }
-            while (e.slot.size() % 64) { e.slot.push_back(-1); e.lead.push_back(0); }
         }
         e.level.push_back((int)e.slot.size());
         return e;
@@ -1977,8 +2022,8 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     }
     for (int m = 0; m < n_moms; m++)
         if (level[m] < n_levels && !rl[m].empty()) r_by[level[m]].push_back(m);
-    const Ell F = build_ell(fl, f_by), R = build_ell(rl, r_by);
-    A2P_REQUIRE(!F.too_long && !R.too_long, A2P_ERR_INVALID,
+    const Ell F[2] = {build_ell(fl, f_by, 1), build_ell(fl, f_by, 4)}, R[2] = {build_ell(rl, r_by, 1), build_ell(rl, r_by, 4)};
+    A2P_REQUIRE(!F[0].too_long && !R[0].too_long, A2P_ERR_INVALID,
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
     // monomial rows, their polynomials and the places of the basic moments among the coefficients (mtp_plan.h)
     std::vector<int> degree((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);      // highest c + 1 of (a, b, mu), 0: none
@@ -2113,15 +2158,15 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 for (int m : anc) node_of[m] = -1;
             }
             if (xl.empty()) xl.emplace_back();
-            const Ell ell = build_ell(xl, x_by);
+            const Ell ell = build_ell(xl, x_by, 4);
             h.stream = build_stream(ell, false, 4);
             A2P_REQUIRE(!ell.too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
                         64 * MTP_SLOT_CAP);
             std::vector<int> by_len = seeds;
             std::stable_sort(by_len.begin(), by_len.end(),
                              [&](int x, int y) { return seed_basic[x].size() > seed_basic[y].size(); });
-            struct Piece { int s, t0, n, rem; };
-            std::vector<Piece> pieces;
+            struct XPiece { int s, t0, n, rem; };
+            std::vector<XPiece> pieces;
             for (int s : by_len) {
                 const int len = (int)seed_basic[s].size();
                 const int np = std::max(1, (len + MTP_SLOT_CAP - 1) / MTP_SLOT_CAP);      // <= 64: n_basic < 64 * cap
@@ -2149,13 +2194,13 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 for (int half = 0; half < 64; half += 16) {
                     std::vector<std::vector<int>> lists(16);
                     for (int q = 0; q < 16; q++) {
-                        const Piece& pc = pieces[g0 + half + q];
+                        const XPiece& pc = pieces[g0 + half + q];
                         if (pc.n) lists[q].assign(seed_basic[pc.s].begin() + pc.t0, seed_basic[pc.s].begin() + pc.t0 + pc.n);
                     }
                     spread_over_banks(lists, depth, h.nodes, &h.bwords[h.bbase.back() + half], 64);
                 }
                 for (size_t q = g0; q < g0 + 64; q++) {
-                    const Piece& pc = pieces[q];
+                    const XPiece& pc = pieces[q];
                     h.seed.push_back(pc.s >= 0 && pc.t0 == 0 ? pc.s : -1);
                     h.brem.push_back(pc.rem);
                 }
@@ -2188,8 +2233,8 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     Stream fs[2], rs[2];
     StreamOff o_f[2], o_r[2];
     for (int i = 0; i < 2; i++) {
-        fs[i] = build_stream(F, true, i ? 4 : 1);
-        rs[i] = build_stream(R, false, i ? 4 : 1);
+        fs[i] = build_stream(F[i], true, i ? 4 : 1);
+        rs[i] = build_stream(R[i], false, i ? 4 : 1);
         o_f[i] = add_stream(fs[i]);
         o_r[i] = add_stream(rs[i]);
     }
