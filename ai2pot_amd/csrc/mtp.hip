@@ -31,6 +31,7 @@
 #include <mutex>
 #include <set>
 #include <string>
+#include <type_traits>
 
 namespace a2p {
 namespace {
@@ -115,6 +116,7 @@ struct MtpArgs {
     int grad_parts;     // loss gradient: parts of a chunk's neighbours that are summed at the same time
     int mom_groups;     // thread groups that share a row's neighbours in the sums of the basic moments (basic_sums), or 0
     int nc_cap;         // rows of the LDS neighbour table: a row is processed in chunks of at most nc_cap
+    int leaves_late;    // the streams are fwd_core and rev_leaf: moments that only the read-out reads are formed in the reverse sweep
     int keep_table;     // energy / force / virial kernel: the adjoints lie behind the table (mtp_table_region)
     // site-energy / descriptor mode (linearMtp.h:514-611, 821-890)
     T* e_sites;        // [B, P] per-row energies, or null
@@ -381,11 +383,11 @@ __device__ __forceinline__ T plan_entry(const T* base, unsigned off)
     return *(const T*)((const char*)base + (sizeof(T) == 8 ? off : off >> 1));
 }
 
-// A gather (mtp_plan.h: MtpStream): terms(words) for a step's terms of the thread's slot and done(slot, rem, steps) behind the
-// last of a group; a barrier behind every level.  What bounds it is the number of instructions a wavefront issues one after
-// the other, so the plan holds everything in the order of use; the words of the next two steps are on their way meanwhile,
-// also across a barrier (the plan does not depend on the moments).  Looking up each group's place, depth and moment when
-// its turn comes took 280 instead of 260 us for the whole kernel at level 20, 8192 atoms, 217 instead of 203 for the loss
+// A gather (mtp_plan.h: MtpStream): terms(words, leaf) for two terms of the thread's slot and done(slot, rem, steps, leaf)
+// behind the last of a group; a barrier behind every level.  What bounds it is the number of instructions a wavefront issues
+// one after the other, so the plan holds everything in the order of use; the words of the next two steps are on their way
+// meanwhile, also across a barrier (the plan does not depend on the moments).  Looking up each group's place, depth and moment
+// when its turn comes took 280 instead of 260 us for the whole kernel at level 20, 8192 atoms, 217 instead of 203 for the loss
 // gradient and 193 instead of 176 for the columns of the linear solver (level 16, 64 structures of 128 atoms).
 template <typename Stream, typename Terms, typename Done>
 __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& done)
@@ -397,25 +399,23 @@ __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& d
     if (n == 0) return;
     const A2P_CONSTANT int* ctrl = uniform_array(g.ctrl) + first;
     const int* sp = g.slots + (size_t)head[2] * 64 + lane;
-    const int2* tp = g.words + (size_t)first * (MTP_DEPTH_STEP * 64) + lane;
-    int2 a[MTP_DEPTH_STEP], b[MTP_DEPTH_STEP];
+    const int4* tp = g.words + (size_t)first * (MTP_DEPTH_STEP / 2 * 64) + lane;
+    int4 a[2], b[2];
     int slot = sp[0], next_slot = sp[64];              // (each array ends with two steps' worth of padding)
-#pragma unroll
-    for (int u = 0; u < MTP_DEPTH_STEP; u++) a[u] = tp[u * 64];
-#pragma unroll
-    for (int u = 0; u < MTP_DEPTH_STEP; u++) b[u] = tp[(MTP_DEPTH_STEP + u) * 64];
-    auto step = [&](int2 (&w)[MTP_DEPTH_STEP], int i) __attribute__((always_inline)) {
+    a[0] = tp[0]; a[1] = tp[64];
+    b[0] = tp[128]; b[1] = tp[192];
+    auto step = [&](int4 (&w)[2], int i) __attribute__((always_inline)) {
         const int c = ctrl[i];
-        terms(w);
-#pragma unroll
-        for (int u = 0; u < MTP_DEPTH_STEP; u++) w[u] = tp[(2 * MTP_DEPTH_STEP + u) * 64];
-        tp += MTP_DEPTH_STEP * 64;
-        if (c) {
-            done((slot & 0xffff) - 1, slot >> 16, (c >> 1) & 7);
+        if (c & MTP_CTRL_HALF) terms(w, std::integral_constant<int, 1>(), (c & MTP_CTRL_LEAF) != 0);
+        else terms(w, std::integral_constant<int, 2>(), (c & MTP_CTRL_LEAF) != 0);
+        w[0] = tp[256]; w[1] = tp[320];
+        tp += 128;
+        if (c & 1) {
+            done((slot & 0xffff) - 1, slot >> 16, (c >> 1) & 7, (c & MTP_CTRL_LEAF) != 0);
             slot = next_slot;
             sp += 64;
             next_slot = sp[64];
-            for (int k = c >> 4; k > 0; k--) __syncthreads();
+            for (int k = c >> 4 & 0xffff; k > 0; k--) __syncthreads();
         }
     };
 #pragma unroll 1
@@ -432,23 +432,23 @@ __device__ __forceinline__ void sweep_forward(Stream& g, T* M, T* Tg, int tid)
 {
     T acc = (T)0, tacc = (T)0;
     walk(g, tid,
-        [&](const int2 (&w)[MTP_DEPTH_STEP]) __attribute__((always_inline)) {
-            constexpr int C = MTP_DEPTH_STEP;
+        [&](const int4 (&w)[2], auto count, bool) __attribute__((always_inline)) {
+            constexpr int C = 2 * decltype(count)::value;
             T v0[C], v1[C], t0[C], t1[C];
 #pragma unroll
             for (int u = 0; u < C; u++) {
-                const unsigned m0 = (unsigned)w[u].x & 0xffffu, m1 = (unsigned)w[u].x >> 16;
+                const unsigned x = u & 1 ? w[u / 2].z : w[u / 2].x, m0 = x & 0xffffu, m1 = x >> 16;
                 v0[u] = plan_entry(M, m0); v1[u] = plan_entry(M, m1);
                 if (TANGENT) { t0[u] = plan_entry(Tg, m0); t1[u] = plan_entry(Tg, m1); }
             }
 #pragma unroll
             for (int u = 0; u < C; u++) {
-                const T mult = (T)w[u].y;
+                const T mult = (T)(u & 1 ? w[u / 2].w : w[u / 2].y);
                 acc += mult * v0[u] * v1[u];
                 if (TANGENT) tacc += t0[u] * mult * v1[u] + t1[u] * mult * v0[u];
             }
         },
-        [&](int dst, int rem, int steps) __attribute__((always_inline)) {
+        [&](int dst, int rem, int steps, bool) __attribute__((always_inline)) {
             if (steps) {
                 acc = piece_sum(acc, rem, steps);
                 if (TANGENT) tacc = piece_sum(tacc, rem, steps);
@@ -462,32 +462,44 @@ __device__ __forceinline__ void sweep_forward(Stream& g, T* M, T* Tg, int tid)
 }
 
 // reverse gather: X[m] += sum mult (X[dst] M[other] (+ A[dst] Tg[other] when MIXED))
-template <typename T, bool MIXED, typename Stream>
-__device__ __forceinline__ void sweep_reverse(Stream& g, const T* M, T* X, const T* A, const T* Tg, int tid)
+// LEAF: the stream also holds the products that nothing but the read-out reads (mtp_plan.h: rev_leaf), of
+// sums mult M[m0] M[m1], or, when MIXED, of their tangents sum mult (Tg[m0] M[m1] + M[m0] Tg[m1]); a leaf's sum goes to leaf().
+template <typename T, bool MIXED, bool LEAF, typename Stream, typename Leaf>
+__device__ __forceinline__ void sweep_reverse(Stream& g, const T* M, T* X, const T* A, const T* Tg, int tid, Leaf&& at_leaf)
 {
     T acc = (T)0;
     walk(g, tid,
-        [&](const int2 (&w)[MTP_DEPTH_STEP]) __attribute__((always_inline)) {
-            constexpr int C = MTP_DEPTH_STEP;
+        [&](const int4 (&w)[2], auto count, bool leaf) __attribute__((always_inline)) {
+            constexpr int C = 2 * decltype(count)::value;
+            const T* const b0 = !LEAF || !leaf ? X : MIXED ? Tg : M;
+            const T* const b1 = !LEAF || !leaf ? A : M;
             T v0[C], v1[C], t0[C], t1[C];
 #pragma unroll
             for (int u = 0; u < C; u++) {
-                const unsigned dst = (unsigned)w[u].x & 0xffffu, other = (unsigned)w[u].x >> 16;
-                v0[u] = plan_entry(X, dst); v1[u] = plan_entry(M, other);
-                if (MIXED) { t0[u] = plan_entry(A, dst); t1[u] = plan_entry(Tg, other); }
+                const unsigned x = u & 1 ? w[u / 2].z : w[u / 2].x, dst = x & 0xffffu, other = x >> 16;
+                v0[u] = plan_entry(b0, dst); v1[u] = plan_entry(M, other);
+                if (MIXED) { t0[u] = plan_entry(b1, dst); t1[u] = plan_entry(Tg, other); }
             }
 #pragma unroll
             for (int u = 0; u < C; u++) {
-                const T mult = (T)w[u].y;
+                const T mult = (T)(u & 1 ? w[u / 2].w : w[u / 2].y);
                 acc += v0[u] * mult * v1[u];
                 if (MIXED) acc += mult * t0[u] * t1[u];
             }
         },
-        [&](int src, int rem, int steps) __attribute__((always_inline)) {
+        [&](int src, int rem, int steps, bool leaf) __attribute__((always_inline)) {
             if (steps) acc = piece_sum(acc, rem, steps);
-            if (src >= 0) X[src] += acc;
+            if (src >= 0) {
+                if (LEAF && leaf) at_leaf(src, acc);
+                else X[src] += acc;
+            }
             acc = (T)0;
         });
+}
+template <typename T, typename Stream>
+__device__ __forceinline__ void sweep_reverse(Stream& g, const T* M, T* X, int tid)
+{
+    sweep_reverse<T, false, false>(g, M, X, (const T*)nullptr, (const T*)nullptr, tid, [](int, T) {});
 }
 
 // sum over the NT threads of a workgroup in a fixed order (wave sums, then wave 0 .. last)
@@ -924,8 +936,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             for (int s = lane; s < p.n_scalar; s += NT) A[p.mapping[s]] = a.row_seed[row * p.n_scalar + s];
         } else {
             for (int s = lane; s < p.n_scalar; s += NT) {
-                e_part += a.lin[s] * M[p.mapping[s]] / a.q_scaler[s];
-                A[p.mapping[s]] = a.lin[s] / a.q_scaler[s];
+                const int mw = p.mapping_leaf[s], m = mw & 0xffff;
+                const T w = a.lin[s] / a.q_scaler[s];
+                if (!a.leaves_late || mw == m) e_part += w * M[m];
+                A[m] = w;
             }
         }
         if (!LOSS && (a.e_sites || a.desc)) {
@@ -939,7 +953,12 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     }
     {
         MTP_PHASE;
-        sweep_reverse<T, false>(p.rev[NT / 256], M, A, (const T*)nullptr, (const T*)nullptr, lane);
+        // the leaves' moments: their part of the energy, or, for the loss gradient, the moments themselves
+        sweep_reverse<T, false, true>(p.rev[NT / 256], M, A, (const T*)nullptr, (const T*)nullptr, lane,
+            [&](int m, T v) __attribute__((always_inline)) {
+                if (LOSS) M[m] = v;
+                else e_part += A[m] * v;
+            });
     }
 
     if (!LOSS) {
@@ -1049,7 +1068,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             MTP_PHASE;
             cE = seeded ? (T)1 : (a.cE_per_atom ? a.cE[row] : a.cE[b]);
             // linearMtpLoss.h:417-434; the reference's network backward has no such term (Bm stays zero)
-            if (!no_tan && (a.H == 0 || a.nn_exact)) sweep_reverse<T, true>(p.rev[NT / 256], M, Bm, A, Tg, lane);
+            if (!no_tan && (a.H == 0 || a.nn_exact)) 
+                sweep_reverse<T, true, true>(p.rev[NT / 256], M, Bm, A, (const T*)Tg, lane,
+                    [&](int m, T v) __attribute__((always_inline)) { Tg[m] = v; });
         }
         {
             MTP_PHASE;
@@ -1390,7 +1411,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             if (p.x_root[s] >= 0) X[p.x_root[s]] = (T)1 / a.q_scaler[s];       // (the columns of this launch)
         }
         __syncthreads();
-        sweep_reverse<T, false>(p.x, M, X, (const T*)nullptr, (const T*)nullptr, lane);
+        sweep_reverse<T>(p.x, M, X, lane);
     }
 
     // Pair derivatives, four or eight neighbours at a time.  A wavefront forms, for one of them and every basic moment, the vector
@@ -1872,7 +1893,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     // Interleaved gather lists (see mtp_plan.h).  `lists[m]` holds the packed terms of moment m.
     struct Ell {
         std::vector<int> level, slot, lead;                // lead: pieces behind
-        std::vector<int4> group;                           // first term, depth, doubling steps
+        std::vector<int4> group;                           // first term, depth, doubling steps, MTP_CTRL_LEAF or 0
         std::vector<int2> terms;
         bool too_long = false;
     };
@@ -1890,7 +1911,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             const int n = (int)lists[m].size(), np = (n + cap - 1) / cap;
             ls.push_back({m, n, np, np ? (n + np - 1) / np : 0});       // pieces of equal length
         }
-        auto deep = [](int n) { return (n + MTP_DEPTH_STEP - 1) / MTP_DEPTH_STEP * MTP_DEPTH_STEP; };
+        auto deep = [](int n) { return (n + 1) / 2 * 2; };
         std::stable_sort(ls.begin(), ls.end(), [&](const List& x, const List& y) {
             return deep(x.len) != deep(y.len) ? deep(x.len) > deep(y.len) : x.np > y.np;
         });
@@ -1935,10 +1956,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         lv.cost = *std::max_element(load.begin(), load.end()) + all / waves;
         return lv;
     };
-    auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level, int waves) {
+    // (`leaves`: lists of another kind that go with the first level to be walked, the last of by_level)
+    auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level, int waves,
+                         const std::vector<std::vector<int2>>* leaf_lists = nullptr, const std::vector<int>* leaves = nullptr) {
         Ell e;
-        for (const auto& members : by_level) {
-            e.level.push_back((int)e.slot.size());
+        auto append = [&](const std::vector<std::vector<int2>>& lists, const std::vector<int>& members, int kind) {
             std::vector<int> ms;
             for (int m : members) {
                 if ((int)lists[m].size() > 64 * MTP_SLOT_CAP) e.too_long = true;
@@ -1946,7 +1968,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             }
             Level best;
             bool any = false;
-            for (int cap = MTP_DEPTH_STEP; cap <= MTP_SLOT_CAP; cap += MTP_DEPTH_STEP) {
+            for (int cap = 2; cap <= MTP_SLOT_CAP; cap += 2) {
                 bool fits = true;
                 for (int m : ms) fits = fits && (int)lists[m].size() <= 64 * cap;
                 if (!fits) continue;
@@ -1954,7 +1976,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 if (!any || lv.cost < best.cost) { best = std::move(lv); any = true; }
             }
             for (size_t g = 0; g < best.depth.size(); g++) {
-                e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], 0));
+                e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], kind));
                 e.terms.resize(e.terms.size() + (size_t)best.depth[g] * 64, make_int2(0, 0));
                 for (size_t q = 0; q < 64; q++) {
                     const Piece& pc = best.lanes[g * 64 + q];
@@ -1964,6 +1986,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                     e.lead.push_back(pc.rem);
                 }
             }
+        };
+        for (size_t l = 0; l < by_level.size(); l++) {
+            e.level.push_back((int)e.slot.size());
+            append(lists, by_level[l], 0);
+            if (leaves && l + 1 == by_level.size()) append(*leaf_lists, *leaves, MTP_CTRL_LEAF);
         }
         e.level.push_back((int)e.slot.size());
         return e;
@@ -1971,7 +1998,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     struct Stream {
         std::vector<int4> head;
         std::vector<int> ctrl, slots;
-        std::vector<int2> words;
+        std::vector<int4> words;
     };
     auto build_stream = [](const Ell& e, bool up, int waves) {
         Stream st;
@@ -1992,15 +2019,21 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 const int q = seq[w][i].first, g = seq[w][i].second;
                 const int barriers = (i + 1 < seq[w].size() ? seq[w][i + 1].first : levels) - q;
                 const int4 info = e.group[g];
-                st.words.insert(st.words.end(), e.terms.begin() + info.x, e.terms.begin() + info.x + (size_t)info.y * 64);
-                for (int k = MTP_DEPTH_STEP; k < info.y; k += MTP_DEPTH_STEP) st.ctrl.push_back(0);
-                st.ctrl.push_back(1 | info.z << 1 | barriers << 4);
+                // pairs of terms; a step holds two, the last of a group possibly one
+                for (int k = 0; k < info.y; k += 2)
+                    for (int l = 0; l < 64; l++) {
+                        const int2 u = e.terms[info.x + (size_t)k * 64 + l], v = e.terms[info.x + (size_t)(k + 1) * 64 + l];
+                        st.words.push_back(make_int4(u.x, u.y, v.x, v.y));
+                    }
+                if (info.y % MTP_DEPTH_STEP) st.words.resize(st.words.size() + 64, make_int4(0, 0, 0, 0));
+                for (int k = MTP_DEPTH_STEP; k < info.y; k += MTP_DEPTH_STEP) st.ctrl.push_back(info.w);
+                st.ctrl.push_back(1 | info.z << 1 | barriers << 4 | info.w | (info.y % MTP_DEPTH_STEP ? MTP_CTRL_HALF : 0));
                 for (int q64 = 0; q64 < 64; q64++)
                     st.slots.push_back((e.slot[g * 64 + q64] + 1) | e.lead[g * 64 + q64] << 16);
             }
             st.head.push_back(make_int4(first, (int)st.ctrl.size() - first, row, seq[w].empty() ? levels : seq[w][0].first));
         }
-        st.words.resize(st.words.size() + 2 * MTP_DEPTH_STEP * 64, make_int2(0, 0));     // requested ahead
+        st.words.resize(st.words.size() + MTP_DEPTH_STEP * 64, make_int4(0, 0, 0, 0));     // requested ahead
         st.ctrl.resize(st.ctrl.size() + 2, 0);
         st.slots.resize(st.slots.size() + 2 * 64, 0);
         return st;
@@ -2022,6 +2055,23 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     }
     for (int m = 0; m < n_moms; m++)
         if (level[m] < n_levels && !rl[m].empty()) r_by[level[m]].push_back(m);
+    // Leaves: scalar moments that no product reads.  Only the read-out needs them, so that the calls whose read-out is linear
+    // form them in the first step of the reverse sweep; the levels of the forward sweep that held nothing else are gone.
+    std::vector<char> is_source(n_moms, 0);
+    for (int e = 0; e < n_times; e++) is_source[times[e * 4]] = is_source[times[e * 4 + 1]] = 1;
+    std::vector<int> leaves, mapping_leaf(mapping, mapping + n_scalar);
+    for (int s = 0; s < n_scalar; s++) {
+        const int m = mapping[s];
+        if (m < n_basic || is_source[m] || fl[m].empty()) continue;
+        mapping_leaf[s] |= 1 << 16;
+        leaves.push_back(m);
+    }
+    std::vector<std::vector<int>> core_by = f_by;
+    for (auto& l : core_by)
+        l.erase(std::remove_if(l.begin(), l.end(), [&](int m) { return !is_source[m]; }), l.end());
+    while (!core_by.empty() && core_by.back().empty()) core_by.pop_back();
+    const Ell C[2] = {build_ell(fl, core_by, 1), build_ell(fl, core_by, 4)};
+    const Ell V[2] = {build_ell(rl, r_by, 1, &fl, &leaves), build_ell(rl, r_by, 4, &fl, &leaves)};
     const Ell F[2] = {build_ell(fl, f_by, 1), build_ell(fl, f_by, 4)}, R[2] = {build_ell(rl, r_by, 1), build_ell(rl, r_by, 4)};
     A2P_REQUIRE(!F[0].too_long && !R[0].too_long, A2P_ERR_INVALID,
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
@@ -2228,15 +2278,20 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     struct StreamOff { size_t head, ctrl, slots, words; };
     auto add_stream = [&](const Stream& st) {
         return StreamOff{add(st.head.data(), sizeof(int4) * st.head.size()), add(st.ctrl.data(), sizeof(int) * st.ctrl.size()),
-                         add(st.slots.data(), sizeof(int) * st.slots.size()), add(st.words.data(), sizeof(int2) * st.words.size())};
+                         add(st.slots.data(), sizeof(int) * st.slots.size()), add(st.words.data(), sizeof(int4) * st.words.size())};
     };
-    Stream fs[2], rs[2];
-    StreamOff o_f[2], o_r[2];
+    const size_t o_leaf = add(mapping_leaf.data(), sizeof(int) * n_scalar);
+    Stream fs[2], rs[2], cs[2], vs[2];
+    StreamOff o_f[2], o_r[2], o_c[2], o_v[2];
     for (int i = 0; i < 2; i++) {
         fs[i] = build_stream(F[i], true, i ? 4 : 1);
         rs[i] = build_stream(R[i], false, i ? 4 : 1);
         o_f[i] = add_stream(fs[i]);
         o_r[i] = add_stream(rs[i]);
+        cs[i] = build_stream(C[i], true, i ? 4 : 1);
+        vs[i] = build_stream(V[i], false, i ? 4 : 1);
+        o_c[i] = add_stream(cs[i]);
+        o_v[i] = add_stream(vs[i]);
     }
     const size_t o_rows = add(rows.data(), sizeof(int) * rows.size());
     const size_t o_poly = add(polys.data(), sizeof(int) * polys.size());
@@ -2275,9 +2330,11 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.basic = (const unsigned*)(base + o_basic);
     d.mapping = (const int*)(base + o_map);
     auto stream_at = [&](const StreamOff& o) {
-        return MtpStream{(const int4*)(base + o.head), (const int*)(base + o.ctrl), (const int*)(base + o.slots), (const int2*)(base + o.words)};
+        return MtpStream{(const int4*)(base + o.head), (const int*)(base + o.ctrl), (const int*)(base + o.slots), (const int4*)(base + o.words)};
     };
     for (int i = 0; i < 2; i++) { d.fwd[i] = stream_at(o_f[i]); d.rev[i] = stream_at(o_r[i]); }
+    for (int i = 0; i < 2; i++) { d.fwd_core[i] = stream_at(o_c[i]); d.rev_leaf[i] = stream_at(o_v[i]); }
+    d.mapping_leaf = (const int*)(base + o_leaf);
     d.x = MtpStream{nullptr, nullptr, nullptr, nullptr};
     d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
     d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
@@ -2385,7 +2442,7 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.cE = nullptr; a.dFs = nullptr; a.dVs = nullptr; a.gpart = nullptr; a.ngrad = 0;
     a.force = nullptr; a.seg_cursor = nullptr; a.seg_g = nullptr; a.seg_spare = 0; a.seg_cap = 0; a.seg_mark = 0;
     a.partial = nullptr;
-    a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0;
+    a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0; a.leaves_late = 0;
     a.nn_exact = 1;
     a.row_seed = nullptr; a.pair_out = nullptr;
     a.H = 0; a.w0 = nullptr; a.w1 = nullptr; a.q_shift = nullptr;
@@ -2423,6 +2480,11 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
         if (e) g_keep_table = e[0] != '0';
     }
     const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0, sizeof(T) == 8);
+    if (a.H == 0 && !a.row_seed && !a.e_sites && !a.desc && !a.energy_only) {
+        MtpArgs<T>& w = const_cast<MtpArgs<T>&>(a);
+        w.leaves_late = 1;
+        for (int i = 0; i < 2; i++) { w.p.fwd[i] = a.p.fwd_core[i]; w.p.rev[i] = a.p.rev_leaf[i]; }
+    }
     const int groups = a.z_powers ? 0 : (wide ? 256 : 64) / std::max(a.p.npoly, 1);      // of a thread per polynomial
     const int kept_adjoints = std::max(a.p.n_moms, groups * a.p.ncoef_poly);
     auto lds_for = [&](int nc, size_t* main, int keep = 0) {

@@ -19,24 +19,28 @@
 namespace a2p {
 
 constexpr int MTP_SLOT_CAP = 16;
-// Terms of a slot to a step of the sweeps.
+// Terms of a slot to a step of the sweeps; the last step of a group may hold half of them.
 constexpr int MTP_DEPTH_STEP = 4;
+// Marks of a control word: a step of half length, and a step of a group of leaves (rev_leaf).
+constexpr int MTP_CTRL_HALF = 1 << 30, MTP_CTRL_LEAF = 1 << 29;
 
 // A gather as the wavefronts of a workgroup walk it.  `lists[m]` holds the terms of moment m.  A slot holds up to
-// MTP_SLOT_CAP of them; a longer list is cut into consecutive slots (pieces), so that no lane walks a long list alone.  Slots
-// are grouped 64 at a time, one to a lane; the pieces of a list lie in one group, a list of up to sixteen within a row of
-// sixteen lanes and a longer one from the beginning of a row on, and the wavefront adds their sums (four doubling steps
-// within a row, two across).  Lists are sorted by length, so only a level's first groups hold cut ones.  The words of a
-// group are padded with zero terms to its depth (a multiple of MTP_DEPTH_STEP); a word packs x = 8 m0 | 8 m1 << 16 (byte
-// offsets into an array of doubles), y = multiplicity.
+// MTP_SLOT_CAP of them; a longer list is cut into pieces of equal length, so that no lane walks a long list alone.  Slots are
+// grouped 64 at a time, one to a lane; the pieces of a list lie in one group, a list of up to sixteen within a row of sixteen
+// lanes and a longer one from the beginning of a row on, and the wavefront adds their sums (four doubling steps within a row,
+// two across).  How long the pieces of a level are is what a wavefront issues for it at least (pack_level); rows are filled
+// first fit, deepest lists first.  The words of a group are padded with zero terms to its depth, an even number; a word packs
+// x = 8 m0 | 8 m1 << 16 (byte offsets into an array of doubles), y = multiplicity, and two terms of a lane lie together.
 // The groups of a level are dealt to the wavefronts, the deepest first and to the one with the least to do, and everything a
 // wavefront needs lies in the order in which it needs it: MTP_DEPTH_STEP x 64 words to a step, a control word for each step,
 // and a row of 64 slot words for each group.
+// (Lists cut at sixteen terms and laid out in order of length, in steps of four: 244 instead of 229 us for the call at level 20,
+// 8192 atoms, 304 instead of 286 for the training step at level 16, 64 structures of 128 atoms.)
 struct MtpStream {
     const int4* head;          // [wavefronts] first step, steps, first row of slots, barriers before the first step
-    const int* ctrl;           // 0, or behind the last step of a group: 1 | doubling steps << 1 | barriers to pass << 4
+    const int* ctrl;           // MTP_CTRL_ marks, and at the last step of a group 1 | doubling steps << 1 | barriers to pass << 4
     const int* slots;          // moment + 1 in the first piece of a list (0 elsewhere) | pieces of the list behind this one << 16
-    const int2* words;
+    const int4* words;
 };
 
 struct MtpPlanDevice {
@@ -49,6 +53,10 @@ struct MtpPlanDevice {
     // forward gather (terms of a product: its factors) and reverse gather (terms of a factor: x = 8 dst | 8 other << 16;
     // sources by level, from the last level to level 0), for workgroups of one wavefront and of four
     MtpStream fwd[2], rev[2];
+    // The same for a linear read-out: scalar moments that no product reads (leaves) are left out of the forward gather, and
+    // their lists stand with the first sources of the reverse one (control words marked, x = 8 m0 | 8 m1 << 16).
+    MtpStream fwd_core[2], rev_leaf[2];
+    const int* mapping_leaf;   // [n_scalar]   mapping | leaf << 16
     int max_level_slots;       // most slots of any level (forward or reverse)
     // Polynomials of the passes that own a neighbour per lane.  The basic moments (mu, a, b, c) with the same row (a, b) and
     // the same mu are the coefficients of a polynomial in z; its coefficients lie together, highest power first, up to
