@@ -375,6 +375,37 @@ __device__ __forceinline__ T piece_sum(T v, int rem, int steps)
     return v;
 }
 
+// The same for several values, a step for all of them at a time, so that their moves overlap.
+template <typename T, int N>
+__device__ __forceinline__ void piece_sums(T (&v)[N], int rem, int steps)
+{
+    T o[N];
+    auto add = [&](bool on) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < N; q++) v[q] += on ? o[q] : (T)0;
+    };
+#pragma unroll
+    for (int q = 0; q < N; q++) o[q] = wave::dpp_move<0x101>(v[q]);
+    add(rem >= 1);
+    if (steps <= 1) return;
+#pragma unroll
+    for (int q = 0; q < N; q++) o[q] = wave::dpp_move<0x102>(v[q]);
+    add(rem >= 2);
+    if (steps <= 2) return;
+#pragma unroll
+    for (int q = 0; q < N; q++) o[q] = wave::dpp_move<0x104>(v[q]);
+    add(rem >= 4);
+    if (steps <= 3) return;
+#pragma unroll
+    for (int q = 0; q < N; q++) o[q] = wave::dpp_move<0x108>(v[q]);
+    add(rem >= 8);
+    for (int d = 16; d < 1 << steps; d <<= 1) {
+#pragma unroll
+        for (int q = 0; q < N; q++) o[q] = __shfl_down(v[q], d, 64);
+        add(rem >= d);
+    }
+}
+
 // A plan term names its two moments by byte offsets into an array of doubles (index * 8): no shift between the
 // word and the LDS address in fp64.
 template <typename T>
@@ -1308,10 +1339,10 @@ struct CompArgs {
     const int* pair_off;    // [rows + 1] first pair of each row
     const int* nnc;         // [rows] checked neighbour count of each row (0 for rows that are not evaluated)
     T* desc;                // [rows, n_scalar] scalar moments
-    T* rowpart;             // [rows, 12, n_scalar] per row and column: sum of the pair derivatives (3), virial (9)
+    T* rowpart;             // [rows, 3, n_scalar] per row and column: sum of the pair derivatives
     int nc_cap, lds_basic_off;
     int node_region;        // entries of the node adjoints' place (even)
-    int batch;              // neighbours whose D vectors are formed together (even)
+    int batch;              // neighbours whose D vectors are formed together (four or eight)
     int d_over_nodes;       // all groups of pieces are worked on at once, so the D vectors take the place of the node adjoints
 };
 template <typename T>
@@ -1373,7 +1404,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
         nn = c.nnc[row];
         if (ii >= a.binum[b] || nn == 0) {                       // padded or refused row (k_rows flags the reasons)
             for (int s = lane; s < S; s += NT) c.desc[row * S + s] = (T)0;
-            for (int q = lane; q < 12 * S; q += NT) c.rowpart[row * 12 * S + q] = (T)0;
+            for (int q = lane; q < 3 * S; q += NT) c.rowpart[row * 3 * S + q] = (T)0;
             return;
         }
         pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
@@ -1421,30 +1452,35 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             c.desc[row * S + s] = M[p.mapping[s]];
             if (p.x_root[s] >= 0) X[p.x_root[s]] = (T)1 / a.q_scaler[s];       // (the columns of this launch)
         }
+        if (p.x_polys)                                                        // (at most as many as basic moments)
+            for (int i = lane; i < p.npoly; i += NT) bas[i] = p.polys_len[i];
         __syncthreads();
         sweep_reverse<T>(p.x, M, X, lane);
     }
 
-    // Pair derivatives, four or eight neighbours at a time.  A wavefront forms, for one of them and every basic moment, the vector
-    //   D_b = d(g_mu x^a y^b z^c)/dr_j = m (g' - k g / r) u + g / r grad_u m
-    // in LDS; then a lane owns a piece of a column's list of basic ancestors and sums adj * D_b over it for
-    // pairs of neighbours (three 16-byte reads and six FMAs per ancestor).  The lane keeps its words and their adjoints in registers over
-    // the whole row, and sums the column's force of the centre and virial as it goes.  Up to four groups of 64 pieces are
-    // worked on at once; fewer groups share out the neighbours.
-    // What bounds it: the LDS reads of D and the latency of their chains.  With a wavefront per neighbour for every
-    // group, words and adjoints fetched again for each neighbour and the row sums read back from memory at the end, the
-    // kernel took 494 instead of 374 us at level 16, 64 structures of 128 atoms (442 with neighbours one by one and 8-byte
-    // reads, 438 with the lists ordered, 384 with pairs of neighbours and 16-byte reads, 374 with eight at a time).
+    // Pair derivatives, four or eight neighbours at a time.  A thread forms, for one of them and the basic moments of a polynomial
+    // (mu, a, b, z^0 .. z^(len-1)), the vectors
+    //   D = d(g_mu x^a y^b z^c)/dr_j = m (g' - k g / r) u + g / r grad_u m
+    // in LDS; then a lane owns a piece of a column's list of basic ancestors and sums adj * D over it for
+    // pairs of neighbours (three 16-byte reads and six FMAs per ancestor, two ancestors' reads ahead).  The lane keeps its words and
+    // their adjoints in registers over the whole row, and sums the column's force of the centre as it goes.  Up to four groups of 64
+    // pieces are worked on at once; fewer groups share out the neighbours.
+    // What bounds it: the latency and the number of the LDS reads of D, and the registers (128) that hold them.  Level 16, 64
+    // structures of 128 atoms, thousands of a workgroup's cycles: 79 -> 66, of which D 16.9 -> 8.6 (a wavefront for a neighbour and a
+    // lane for a basic moment before: ten reads of the table and 25 operations for each), the sums 24.1 -> 16.6 (the reads of one
+    // ancestor at a time, the virial here instead of in comp_force_kernel, lists cut at sixteen words); the whole call 497 -> 467 us.
+    // The words asked for ahead of the sweep, which they outlive: spilled, 544.
     const int l64 = lane & 63, wv = __builtin_amdgcn_readfirstlane(lane >> 6);
     constexpr int NW = NT / 64;
-    int ngroups, at_once, shares, batch, plen;                 // plen: D of a pair of neighbours; the last six their displacements
+    int ngroups, at_once, shares, batch, log2_batch, plen;     // plen: D of a pair of neighbours
     T* D;
     {
         COMP_PHASE;
         ngroups = p.x_slots >> 6;
         at_once = min(ngroups, NW); shares = NW / at_once;
         batch = c.batch;
-        plen = n_basic * 6 + 6;
+        plen = n_basic * 6 + 6;                                // (the banks of the pairs apart)
+        log2_batch = batch == 8 ? 3 : 2;
         D = c.d_over_nodes ? X : (T*)smem_raw + (((tab - (T*)smem_raw) + (size_t)c.nc_cap * E + 1) & ~(size_t)1);
     }
     for (int g0 = 0; g0 < ngroups; g0 += NW) {
@@ -1469,9 +1505,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             for (int k = 0; k < MTP_SLOT_CAP; k += 2)
                 off[k / 2] = (int)(((unsigned)w[k] >> 16) * 6 | ((unsigned)w[k + 1] >> 16) * 6 << 16);
         }
-        T all[12];                                         // force of the centre (3), virial (9)
-#pragma unroll
-        for (int i = 0; i < 12; i++) all[i] = (T)0;
+        T all[3] = {(T)0, (T)0, (T)0};                     // force of the centre
         for (int c0 = 0; c0 < nn; c0 += chunk) {
             const int nc = min(chunk, nn - c0);
             __syncthreads();                               // the adjoints, or the last batch of D, have been read
@@ -1483,84 +1517,108 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             }
             for (int j0 = 0; j0 < nc; j0 += batch) {
                 if (j0) __syncthreads();
-                for (int jb = wv; jb < min(batch, nc - j0); jb += NW) {
+                {
                     COMP_PHASE;
-                    const int j = j0 + jb;
-                    const T* t = tab + j * E;
-                    T* Dw = D + (jb >> 1) * plen + (jb & 1) * 3;
-                    const T ux = t[OU + 0], uy = t[OU + 1], uz = t[OU + 2], rinv = t[OU + 3];
-                    for (int i = l64; i < n_basic; i += 64) {
-                        const unsigned bw = bas[i];
-                        const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
-                        const T gm = t[OG + mu], dg = t[ODG + mu];
-                        const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
-                        const T gs = xa * yb * zc * (dg - (T)(ea + eb + ec) * gm * rinv);
-                        const T gr = gm * rinv;
-                        Dw[i * 6 + 0] = gs * ux + gr * ((T)ea * t[OX + max(ea - 1, 0)] * yb * zc);
-                        Dw[i * 6 + 1] = gs * uy + gr * ((T)eb * xa * t[OY + max(eb - 1, 0)] * zc);
-                        Dw[i * 6 + 2] = gs * uz + gr * ((T)ec * xa * yb * t[OZ + max(ec - 1, 0)]);
+                    const int nb = min(batch, nc - j0);
+                    if (p.x_polys) {
+                        // thread <- (polynomial, neighbour of the batch): what its moments share is read and multiplied once
+                        // (longest first, and the wavefronts in turn from either end)
+                        for (int r = 0; r * NT < p.npoly * batch; r++) {
+                            const int task = r * NT + (r & 1 ? (NT - 64 - wv * 64) + l64 : lane), jb = task & (batch - 1);
+                            if (jb >= nb || task >= p.npoly * batch) continue;
+                            const unsigned pw = bas[task >> log2_batch];
+                            const T* t = tab + (j0 + jb) * E;
+                            const int mu = pw & 7, ea = (pw >> 3) & 31, eb = (pw >> 8) & 31, len = (pw >> 13) & 31;
+                            T* Dw = D + (jb >> 1) * plen + (jb & 1) * 3 + (int)(pw >> 18) * 6 + (len - 1) * 6;     // (highest power first)
+                            const T ux = t[OU + 0], uy = t[OU + 1], uz = t[OU + 2], rinv = t[OU + 3];
+                            const T gr = t[OG + mu] * rinv, xa = t[OX + ea], yb = t[OY + eb];
+                            const T xy = xa * yb, hx = gr * ((T)ea * t[OX + max(ea - 1, 0)] * yb), hy = gr * ((T)eb * xa * t[OY + max(eb - 1, 0)]),
+                                    hz = gr * xy, k0 = t[ODG + mu] - (T)(ea + eb) * gr;
+                            T zc = (T)1, zd = (T)0, n = (T)0;                  // z^c, c z^(c-1), c
+                            for (int i = 0; i < len; i++, Dw -= 6) {
+                                const T gs = xy * zc * (k0 - n * gr);
+                                Dw[0] = gs * ux + hx * zc;
+                                Dw[1] = gs * uy + hy * zc;
+                                Dw[2] = gs * uz + hz * zd;
+                                n += (T)1;
+                                zd = n * zc;
+                                zc *= uz;
+                            }
+                        }
+                    } else {
+                        for (int jb = wv; jb < nb; jb += NW) {
+                            const T* t = tab + (j0 + jb) * E;
+                            T* Dw = D + (jb >> 1) * plen + (jb & 1) * 3;
+                            const T ux = t[OU + 0], uy = t[OU + 1], uz = t[OU + 2], rinv = t[OU + 3];
+                            for (int i = l64; i < n_basic; i += 64) {
+                                const unsigned bw = bas[i];
+                                const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
+                                const T gm = t[OG + mu], dg = t[ODG + mu];
+                                const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
+                                const T gs = xa * yb * zc * (dg - (T)(ea + eb + ec) * gm * rinv);
+                                const T gr = gm * rinv;
+                                Dw[i * 6 + 0] = gs * ux + gr * ((T)ea * t[OX + max(ea - 1, 0)] * yb * zc);
+                                Dw[i * 6 + 1] = gs * uy + gr * ((T)eb * xa * t[OY + max(eb - 1, 0)] * zc);
+                                Dw[i * 6 + 2] = gs * uz + gr * ((T)ec * xa * yb * t[OZ + max(ec - 1, 0)]);
+                            }
+                        }
                     }
-                    if (l64 < 3) Dw[n_basic * 6 + l64] = rcs[(c0 + j) * 3 + l64];
                 }
                 __syncthreads();
                 if (!works) continue;
                 for (int jp = share * 2; jp < min(batch, nc - j0); jp += shares * 2) {
                     COMP_PHASE;
                     const T* Dp = D + (jp >> 1) * plen;
-                    T gr[6];
+                    T gr[6], dv[2][2][6];
 #pragma unroll
                     for (int q = 0; q < 6; q++) gr[q] = (T)0;
+                    // (the next two vectors are on their way while two are worked on)
+                    auto fetch = [&](T (&o)[2][6], int k) __attribute__((always_inline)) {
+                        load6(Dp + ((unsigned)off[k / 2] & 0xffffu), o[0]);
+                        load6(Dp + ((unsigned)off[k / 2] >> 16), o[1]);
+                    };
+                    fetch(dv[0], 0);
 #pragma unroll
-                    for (int k = 0; k < MTP_SLOT_CAP; k += 2)
+                    for (int k = 0; k < MTP_SLOT_CAP; k += 2) {
                         if (k < depth) {
+                            if (k + 2 < MTP_SLOT_CAP) fetch(dv[k / 2 + 1 & 1], k + 2 < MTP_SLOT_CAP ? k + 2 : 0);
 #pragma unroll
-                            for (int u = k; u < k + 2; u++) {
-                                T dv[6];
-                                load6(Dp + ((unsigned)off[u / 2] >> (u & 1) * 16 & 0xffffu), dv);
+                            for (int u = 0; u < 2; u++)
 #pragma unroll
-                                for (int q = 0; q < 6; q++) gr[q] += adj[u] * dv[q];
-                            }
+                                for (int q = 0; q < 6; q++) gr[q] += adj[k + u] * dv[k / 2 & 1][u][q];
                         }
-                    if (steps) {                            // a long list's pieces sit in neighbouring lanes
-#pragma unroll
-                        for (int q = 0; q < 6; q++) gr[q] = piece_sum(gr[q], rem, steps);
                     }
+                    if (steps) piece_sums(gr, rem, steps);          // a long list's pieces sit in neighbouring lanes
                     T* dst = c.pb + ((size_t)(pair0 + c0 + j0 + jp) * 3) * S + col;
 #pragma unroll
                     for (int o = 0; o < 2; o++) {
                         if (j0 + jp + o >= nc) continue;    // (the other half of D is not of this row)
-                        const T* dj = Dp + n_basic * 6 + o * 3;
 #pragma unroll
                         for (int q = 0; q < 3; q++) {
                             all[q] += gr[o * 3 + q];
-#pragma unroll
-                            for (int i = 0; i < 3; i++) all[3 + q * 3 + i] -= gr[o * 3 + q] * dj[i];
                             if (col >= 0) dst[(size_t)(o * 3 + q) * S] = gr[o * 3 + q];
                         }
                     }
                 }
             }
         }
-        // the shares of a group: four values of the others at a time through LDS
+        // the shares of a group, through LDS
         if (shares > 1) {
+            __syncthreads();
+            if (works && share > 0)
 #pragma unroll
-            for (int q0 = 0; q0 < 12; q0 += 4) {
-                __syncthreads();
-                if (works && share > 0)
+                for (int q = 0; q < 3; q++) D[((wv - at_once) * 3 + q) * 64 + l64] = all[q];
+            __syncthreads();
+            if (share == 0)
+                for (int o = wv; o < (shares - 1) * at_once; o += at_once)
 #pragma unroll
-                    for (int q = 0; q < 4; q++) D[((wv - at_once) * 4 + q) * 64 + l64] = all[q0 + q];
-                __syncthreads();
-                if (share == 0)
-                    for (int o = wv; o < (shares - 1) * at_once; o += at_once)
-#pragma unroll
-                        for (int q = 0; q < 4; q++) all[q0 + q] += D[(o * 4 + q) * 64 + l64];
-            }
+                    for (int q = 0; q < 3; q++) all[q] += D[(o * 3 + q) * 64 + l64];
         }
         if (works && share == 0 && col >= 0) {
             COMP_PHASE;
-            T* o = c.rowpart + row * 12 * S + col;
+            T* o = c.rowpart + row * 3 * S + col;
 #pragma unroll
-            for (int q = 0; q < 12; q++) o[(size_t)q * S] = all[q];
+            for (int q = 0; q < 3; q++) o[(size_t)q * S] = all[q];
         }
     }
 }
@@ -1592,12 +1650,11 @@ comp_rows_kernel(int B, int P, int U, int ntypes, const int* __restrict__ binum,
     nnc[row] = nn;
 }
 
-// The pairs that name each atom.  Each atom has room for `cap` of them (the row length of the list: enough for every list
+// The pairs that name each atom, by row * U + slot (B P U is below 2^31).  Each atom has room for `cap` of them (the row length of the list: enough for every list
 // built with one cutoff), so one pass lists them; when an atom is named more often (spill[0] counts what found no room)
 // the pass is repeated for counts only and then into segments of the right lengths (seg).
 __global__ void __launch_bounds__(256)
-comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int* __restrict__ pair_off,
-                     const int* __restrict__ bfirstneigh, int* __restrict__ cnt, const int* __restrict__ seg, int cap,
+comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int* __restrict__ bfirstneigh, int* __restrict__ cnt, const int* __restrict__ seg, int cap,
                      int* __restrict__ inc, int* __restrict__ spill)
 {
     const long long q = (long long)blockIdx.x * 256 + threadIdx.x;
@@ -1609,61 +1666,76 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
     const int tg = (row / P) * P + nj;
     const int place = atomicAdd(cnt + tg, 1);
     if (!inc) return;
-    if (seg) inc[seg[tg] + place] = pair_off[row] + j;
-    else if (place < cap) inc[(size_t)tg * cap + place] = pair_off[row] + j;
+    if (seg) inc[seg[tg] + place] = (int)q;
+    else if (place < cap) inc[(size_t)tg * cap + place] = (int)q;
     else atomicAdd(spill, 1);
 }
 
-// Force column of every atom: its own row's sum minus the pairs that name it, in the order of their numbers.  The pairs
-// arrive in any order: a workgroup (one wavefront) ranks those of its atom in LDS, up to COMP_SORT of them; a longer list
-// is walked from each number to the next larger one.  Columns from S on (species counts) are zero.
-// Bound by the reads of the pair derivatives; sorting the lists by insertion, one thread per atom, used to take as long as
-// they do (95 us beside 98 us at 64 structures of 128 atoms).
+// Force column of every atom: its own row's sum minus the pairs that name it, in the order of their places in the lists; on the
+// way these pairs' virial.  The pairs arrive in any order: a workgroup (one wavefront) ranks those of its atom in LDS, up to
+// COMP_SORT of them; a longer list is walked from each place to the next larger one.  Columns from S on (species counts) are
+// zero.
+// Bound by the reads of the pair derivatives, under which the virial's operations hide (in mtp_components_kernel they took a
+// fifth of its instructions and the registers of four more reads in flight); sorting the lists by insertion, one thread per
+// atom, used to take as long as they do (95 us beside 98 us at 64 structures of 128 atoms).
 constexpr int COMP_SORT = 256;
 
 template <typename T>
 __global__ void __launch_bounds__(64)
-comp_force_kernel(int S, int n, int cap, int row0, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
-                  const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ pb,
-                  const T* __restrict__ rowpart, T* __restrict__ fcomp)
+comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
+                  const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ brcs, const T* __restrict__ pb,
+                  const T* __restrict__ rowpart, T* __restrict__ vpart, T* __restrict__ fcomp)
 {
     __shared__ int list[COMP_SORT], order[COMP_SORT];
+    __shared__ T disp[COMP_SORT][3];
     const int t = blockIdx.x + row0, lane = threadIdx.x, col = blockIdx.y * 64 + lane, s = min(col, S - 1);
     const int* v = inc + (seg ? (size_t)seg[t] : (size_t)t * cap);
     const int m = seg ? seg[t + 1] - seg[t] : min(cnt[t], cap);
     const int r1 = row_of1[t], base = pair_off[row0];    // pb holds the pairs from row0 on
     const bool ranked = m <= COMP_SORT;
+    auto pair_of = [&](int q) __attribute__((always_inline)) { const int row = q / U; return pair_off[row] + (q - row * U) - base; };
     if (ranked) {
         for (int k = lane; k < m; k += 64) list[k] = v[k];
         __syncthreads();
         for (int k = lane; k < m; k += 64) {
-            const int x = list[k];
+            const int x = list[k], pair = pair_of(x);
+            const T* d = brcs + (size_t)x * 3;
+            const T dx = d[0], dy = d[1], dz = d[2];
             int r = 0;
             for (int i = 0; i < m; i++) r += list[i] < x;
-            order[r] = x;
+            order[r] = pair;
+            disp[r][0] = dx; disp[r][1] = dy; disp[r][2] = dz;
         }
         __syncthreads();
     }
-    T f[3] = {(T)0, (T)0, (T)0};
+    T f[3] = {(T)0, (T)0, (T)0}, vir[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) vir[i] = (T)0;
     if (r1 > 0) {
-        const T* o = rowpart + (size_t)(r1 - 1) * 12 * S + s;
+        const T* o = rowpart + (size_t)(r1 - 1) * 3 * S + s;
 #pragma unroll
         for (int i = 0; i < 3; i++) f[i] = o[(size_t)i * S];
     }
+    auto take = [&](const T (&g)[3], const T* d) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            f[i] -= g[i];
+#pragma unroll
+            for (int k = 0; k < 3; k++) vir[i * 3 + k] -= g[i] * d[k];
+        }
+    };
     if (ranked) {
         for (int k0 = 0; k0 < m; k0 += 4) {              // twelve loads in flight
             T g[4][3];
 #pragma unroll
             for (int u = 0; u < 4; u++) {
-                const T* src = pb + (size_t)(order[min(k0 + u, m - 1)] - base) * 3 * S + s;
+                const T* src = pb + (size_t)order[min(k0 + u, m - 1)] * 3 * S + s;
 #pragma unroll
                 for (int i = 0; i < 3; i++) g[u][i] = src[(size_t)i * S];
             }
 #pragma unroll
             for (int u = 0; u < 4; u++)
-                if (k0 + u < m)
-#pragma unroll
-                    for (int i = 0; i < 3; i++) f[i] -= g[u][i];
+                if (k0 + u < m) take(g[u], disp[k0 + u]);
         }
     } else {
         int last = -1;
@@ -1676,17 +1748,22 @@ comp_force_kernel(int S, int n, int cap, int row0, const int* __restrict__ pair_
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) next = min(next, __shfl_xor(next, off, 64));
             last = next;
-            const T* g = pb + (size_t)(next - base) * 3 * S + s;
+            const T* src = pb + (size_t)pair_of(next) * 3 * S + s;
+            T g[3];
 #pragma unroll
-            for (int i = 0; i < 3; i++) f[i] -= g[(size_t)i * S];
+            for (int i = 0; i < 3; i++) g[i] = src[(size_t)i * S];
+            take(g, brcs + (size_t)next * 3);
         }
     }
     if (col < n)
 #pragma unroll
         for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + col] = col < S ? f[i] : (T)0;
+    if (col < S)
+#pragma unroll
+        for (int i = 0; i < 9; i++) vpart[((size_t)t * 9 + i) * S + col] = vir[i];
 }
 
-// Energy and virial columns per structure: sums over the rows in row order, in two steps (blocks of COMP_ROWS rows, then
+// Energy and virial columns per structure: sums over the rows (virial: the atoms that the pairs name) in order, in two steps (blocks of COMP_ROWS rows, then
 // the blocks); part[B][nblocks][10][n].  Column S + t counts the rows whose centre has species t; its virial is zero.
 // The first step reads 80 bytes per row and column: short blocks (8 rows: 25 -> 8 us against 32 at 64 x 128 rows) keep
 // enough wavefronts in flight.
@@ -1696,7 +1773,7 @@ template <typename T>
 __global__ void __launch_bounds__(64)
 comp_structure_blocks_kernel(int S, int n, int P, int nblocks, const int* __restrict__ binum,
                              const int* __restrict__ bilist, const int* __restrict__ btypes, const T* __restrict__ desc,
-                             const T* __restrict__ rowpart, T* __restrict__ part)
+                             const T* __restrict__ vpart, T* __restrict__ part)
 {
     const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x, blk = blockIdx.z;
     if (s >= n) return;
@@ -1706,12 +1783,12 @@ comp_structure_blocks_kernel(int S, int n, int P, int nblocks, const int* __rest
     const int i0 = blk * COMP_ROWS, i1 = min(binum[b], i0 + COMP_ROWS);
     if (s < S) {
 #pragma unroll 4
-        for (int ii = i0; ii < i1; ii++) {
+        for (int ii = i0; ii < min(P, i0 + COMP_ROWS); ii++) {
             const size_t row = (size_t)b * P + ii;
-            e += desc[row * S + s];
-            const T* o = rowpart + row * 12 * S + s;
+            if (ii < i1) e += desc[row * S + s];
+            const T* o = vpart + row * 9 * S + s;
 #pragma unroll
-            for (int i = 0; i < 9; i++) v[i] += o[(size_t)(3 + i) * S];
+            for (int i = 0; i < 9; i++) v[i] += o[(size_t)i * S];
         }
     } else {
         int c[COMP_ROWS];
@@ -2154,6 +2231,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     }
     poly_items_off[n_poly_coef] = (int)poly_items.size();
 
+    const bool x_polys = polys_fit && n_poly_coef == n_basic;
     // nodes (scalar moment, ancestor) and their reverse gather (mtp_plan.h), for batches of scalar moments whose node
     // adjoints fit MTP_NODE_CAP entries of LDS
     struct XHost {
@@ -2214,7 +2292,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 }
                 for (int m : anc) {
                     if (level[m] < n_levels && !xl[node_of[m]].empty()) x_by[level[m]].push_back(node_of[m]);
-                    if (m < n_basic) seed_basic[s].push_back(node_of[m] | (m << 16));
+                    if (m < n_basic) seed_basic[s].push_back(node_of[m] | (x_polys ? poly_pos[m] : m) << 16);
                 }
                 for (int m : anc) node_of[m] = -1;
             }
@@ -2223,47 +2301,51 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             h.stream = build_stream(ell, false, 4);
             A2P_REQUIRE(!ell.too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
                         64 * MTP_SLOT_CAP);
-            std::vector<int> by_len = seeds;
-            std::stable_sort(by_len.begin(), by_len.end(),
-                             [&](int x, int y) { return seed_basic[x].size() > seed_basic[y].size(); });
-            struct XPiece { int s, t0, n, rem; };
-            std::vector<XPiece> pieces;
-            for (int s : by_len) {
-                const int len = (int)seed_basic[s].size();
-                const int np = std::max(1, (len + MTP_SLOT_CAP - 1) / MTP_SLOT_CAP);      // <= 64: n_basic < 64 * cap
-                if ((int)(pieces.size() % 16) + np > 16)                                  // as in the gathers (piece_sum)
-                    while (pieces.size() % 16) pieces.push_back({-1, 0, 0, 0});
-                if ((int)(pieces.size() % 64) + np > 64)
-                    while (pieces.size() % 64) pieces.push_back({-1, 0, 0, 0});
-                for (int q = 0; q < np; q++)
-                    pieces.push_back({s, q * MTP_SLOT_CAP, std::min(MTP_SLOT_CAP, len - q * MTP_SLOT_CAP), np - 1 - q});
+            // The lists of basic ancestors, cut and placed as the gathers' are.  A group costs its reads of D and some ten more for
+            // what it does once per pair of neighbours (and three for a doubling step); the groups of a round are worked on at the
+            // same time, fewer than four by several wavefronts each, and the reads of all of them share the LDS.  (Lists cut at
+            // sixteen words: 32 words deep instead of 24 at level 16.)
+            std::vector<std::vector<int2>> columns(n_scalar);
+            for (int s : seeds) {
+                for (int w : seed_basic[s]) columns[s].push_back(make_int2(w, 0));
+                if (columns[s].empty()) columns[s].push_back(make_int2(h.nodes, 0));      // (a column of zeros)
             }
-            while (pieces.empty() || pieces.size() % 64) pieces.push_back({-1, 0, 0, 0});
-            for (size_t g0 = 0; g0 < pieces.size(); g0 += 64) {
-                int depth = 0, most = 1;
-                for (size_t q = g0; q < g0 + 64; q++) {
-                    depth = std::max(depth, pieces[q].n);
-                    most = std::max(most, pieces[q].rem + 1);
+            Level best;
+            double best_cost = 0;
+            for (int cap = MTP_SLOT_CAP; cap >= 2; cap -= 2) {
+                bool fits = true;
+                for (int s : seeds) fits &= (int)columns[s].size() <= 64 * cap;
+                if (!fits) break;
+                Level lv = pack_level(columns, seeds, cap, 4);
+                const size_t n = lv.depth.size();
+                double cost = 0;
+                for (size_t g0 = 0; g0 < n; g0 += 4) {
+                    const size_t at_once = std::min<size_t>(n - g0, 4);
+                    double most = 0;
+                    for (size_t g = g0; g < g0 + at_once; g++) {
+                        const double one = lv.depth[g] + 10 + 3 * lv.steps[g];
+                        most = std::max(most, one);
+                        cost += 0.25 * one;
+                    }
+                    cost += most / (double)(4 / std::min<size_t>(n, 4));
                 }
-                int steps = 0;
-                while ((1 << steps) < most) steps++;
-                depth = (depth + 3) / 4 * 4;            // the kernel fetches four words at a time
+                if (best.depth.empty() || cost < best_cost) { best = std::move(lv); best_cost = cost; }
+            }
+            for (size_t g = 0; g < best.depth.size(); g++) {
+                const int depth = best.depth[g];
                 h.bbase.push_back((int)h.bwords.size());
                 h.bdepth.push_back(depth);
-                h.bsteps.push_back(steps);
+                h.bsteps.push_back(best.steps[g]);
                 h.bwords.resize(h.bwords.size() + (size_t)depth * 64, h.nodes);       // node `nodes` (a zero), basic moment 0
-                for (int half = 0; half < 64; half += 16) {
+                for (size_t row = g * 64; row < g * 64 + 64; row += 16) {
                     std::vector<std::vector<int>> lists(16);
-                    for (int q = 0; q < 16; q++) {
-                        const XPiece& pc = pieces[g0 + half + q];
-                        if (pc.n) lists[q].assign(seed_basic[pc.s].begin() + pc.t0, seed_basic[pc.s].begin() + pc.t0 + pc.n);
+                    for (size_t q = 0; q < 16; q++) {
+                        const Piece& pc = best.lanes[row + q];
+                        for (int k = 0; k < pc.n; k++) lists[q].push_back(columns[pc.m][pc.t0 + k].x);
+                        h.seed.push_back(pc.n > 0 && pc.t0 == 0 ? pc.m : -1);
+                        h.brem.push_back(pc.rem);
                     }
-                    spread_over_banks(lists, depth, h.nodes, &h.bwords[h.bbase.back() + half], 64);
-                }
-                for (size_t q = g0; q < g0 + 64; q++) {
-                    const XPiece& pc = pieces[q];
-                    h.seed.push_back(pc.s >= 0 && pc.t0 == 0 ? pc.s : -1);
-                    h.brem.push_back(pc.rem);
+                    spread_over_banks(lists, depth, h.nodes, &h.bwords[h.bbase.back() + (row - g * 64)], 64);
                 }
             }
             if (h.bwords.empty()) h.bwords.push_back(0);
@@ -2353,6 +2435,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.polys_mu = (const int*)(base + o_pmu); d.polys_end = (const int*)(base + o_pend);
     d.poly_src = (const int*)(base + o_psrc); d.poly_off = (const int*)(base + o_poff);
     d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
+    d.x_polys = x_polys;
     d.polys_len = polys_fit ? (const unsigned*)(base + o_plen) : nullptr;
     d.poly_top = poly_top;
     d.poly_unique = poly_unique;
@@ -2940,7 +3023,7 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
     const long long nslots = (long long)rows * U;
     prof_begin("mtp_components_lists", stream);
     hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U, (const int*)nnc,
-                       (const int*)pair_off, a.bfirstneigh, cnt, (const int*)nullptr, U, inc, spill);
+                       a.bfirstneigh, cnt, (const int*)nullptr, U, inc, spill);
     prof_end(stream);
     int found[2] = {0, 0};                  // the first sizes the pair buffer: one read-back per call
     rc = read_back(pair_off + rows, 2, found, stream);
@@ -2957,18 +3040,19 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         if (rc) return rc;
         inc = (int*)wsL;
         hipLaunchKernelGGL(comp_incoming_kernel, dim3(ceil_div(nslots, 256)), dim3(256), 0, stream, B, P, U,
-                           (const int*)nnc, (const int*)pair_off, a.bfirstneigh, cnt, (const int*)seg, U, inc, spill);
+                           (const int*)nnc, a.bfirstneigh, cnt, (const int*)seg, U, inc, spill);
         A2P_HIP_CHECK(hipGetLastError());
         in_seg = seg;
     }
-    // pair derivatives | row sums | scalar moments
-    const size_t n_pb = (size_t)std::max(npairs, 1) * 3 * S, n_rp = (size_t)rows * 12 * S, n_desc = (size_t)rows * S;
+    // pair derivatives | row sums | virial by named atom | scalar moments
+    const size_t n_pb = (size_t)std::max(npairs, 1) * 3 * S, n_rp = (size_t)rows * 3 * S, n_desc = (size_t)rows * S;
     void* wsT = nullptr;
-    rc = ws_get(WS_MTP, (n_pb + n_rp + n_desc) * sizeof(T), &wsT);
+    rc = ws_get(WS_MTP, (n_pb + 4 * n_rp + n_desc) * sizeof(T), &wsT);
     if (rc) return rc;
     T* pb = (T*)wsT;
     T* rowpart = pb + n_pb;
-    T* desc = rowpart + n_rp;
+    T* vpart = rowpart + n_rp;
+    T* desc = vpart + 3 * n_rp;
 
     CompArgs<T> c;
     c.pb = pb; c.pair_off = pair_off; c.nnc = nnc; c.desc = desc; c.rowpart = rowpart;
@@ -2987,12 +3071,12 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
             p.x_nodes = xb.nodes; p.x_slots = xb.slots; p.x_root = xb.root; p.x_seed = xb.seed;
             p.x = xb.x;
             p.x_bbase = xb.bbase; p.x_bdepth = xb.bdepth; p.x_bsteps = xb.bsteps; p.x_brem = xb.brem; p.x_bwords = xb.bwords;
-            // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 256
+            // LDS: moments | node adjoints | coefficients | table of nc rows | D of a batch of neighbours (or three shares' sums, 192
             // values each); then the packed basic moments.  With at most four groups of pieces the adjoints are in registers
             // when the first D is formed, and D takes their place (level 16: 36 instead of 46 KB).
             // Workgroups per CU count first, then the longest table that still allows them.
             c.batch = p.x_slots <= 128 ? 8 : 4;         // a pair of neighbours for every wavefront that shares a group
-            const int d_vals = std::max(c.batch * (3 * p.n_basic + 3), 768);
+            const int d_vals = std::max(c.batch * (3 * p.n_basic + 3), 576);
             c.d_over_nodes = p.x_slots <= 4 * 64;
             c.node_region = (std::max(p.x_nodes + 1, c.d_over_nodes ? d_vals : 0) + 1) & ~1;
             auto lds_for = [&](int nc, size_t* main) {
@@ -3018,9 +3102,9 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
             prof_end(stream);
         }
         prof_begin("mtp_components_sums", stream);
-        hipLaunchKernelGGL(comp_force_kernel<T>, dim3(nb * P, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, b0 * P,
+        hipLaunchKernelGGL(comp_force_kernel<T>, dim3(nb * P, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, U, b0 * P,
                            (const int*)pair_off, (const int*)row_of1,
-                           (const int*)cnt, in_seg, (const int*)inc, (const T*)pb, (const T*)rowpart, fcomp);
+                           (const int*)cnt, in_seg, (const int*)inc, a.brcs, (const T*)pb, (const T*)rowpart, vpart, fcomp);
         prof_end(stream);
     }
     prof_begin("mtp_components_sums", stream);
@@ -3029,7 +3113,7 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
     rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * n * sizeof(T), &wsP);
     if (rc) return rc;
     hipLaunchKernelGGL(comp_structure_blocks_kernel<T>, dim3(B, ceil_div(n, 64), nblocks), dim3(64), 0, stream, S, n, P,
-                       nblocks, a.binum, a.bilist, a.btypes, (const T*)desc, (const T*)rowpart, (T*)wsP);
+                       nblocks, a.binum, a.bilist, a.btypes, (const T*)desc, (const T*)vpart, (T*)wsP);
     hipLaunchKernelGGL(comp_structure_kernel<T>, dim3(B, ceil_div(n, 64)), dim3(64), 0, stream, n, S, nblocks, a.q_scaler,
                        (const T*)wsP, ecomp, vcomp);
     prof_end(stream);

@@ -81,11 +81,12 @@ struct MtpPlanDevice {
     // The basic ancestors of a scalar moment form a list of words node | basic << 16; lists are sorted by length, cut into
     // pieces of at most MTP_SLOT_CAP words, and dealt to slots, 64 slots a group, the pieces of a list in neighbouring
     // slots as in the gathers (the wavefront adds their sums, x_bsteps doubling steps).  A group's words are
-    // stored interleaved and padded to the group's depth with node x_nodes, whose adjoint is always zero: word k of
+    // stored interleaved and padded to the group's depth with node x_nodes, whose adjoint is always zero; `basic` is the moment's
+    // place among the polynomials' coefficients (poly_pos) when there are as many of them as basic moments (x_polys): word k of
     // slot q is x_bwords[x_bbase[q >> 6] + k * 64 + (q & 63)].
     // The scalar moments are dealt to batches whose nodes fit the kernel's LDS budget (MtpPlan::xbatches); the fields
     // below are those of the batch a launch works on (x_root is -1 for the scalar moments of other batches).
-    int x_nodes, x_slots;
+    int x_nodes, x_slots, x_polys;
     const int* x_root;         // [n_scalar] node (s, mapping[s])
     const int* x_seed;         // [x_slots]  scalar moment, in the slot of its list's first piece; -1 elsewhere
     const int* x_brem;         // [x_slots]  pieces of the same list behind this one

@@ -74,6 +74,41 @@ def test_components_by_group_and_row_length(oracle, level, U):
         assert close(a, b)
 
 
+@pytest.mark.parametrize("lists", ["whole", "rows left out", "one atom named by all"])
+@pytest.mark.parametrize("basic", [GAPS, TWICE, LONG, MANY, MANY + [(1, 0, 0, 8)]], ids=["gaps", "twice", "long", "many", "many, gap"])
+def test_components_of_irregular_tables(oracle, basic, lists):
+    """The vectors of the basic moments by polynomials and one by one, columns cut into pieces of any length, and the virial summed
+    over the atoms that the pairs name: atoms without a row of their own, and one with more pairs than are ranked in LDS.  All
+    columns from one pass against a pass per column, fp64 1e-10."""
+    from ai2pot_amd import _lib, ops
+    import torch
+    nt = 2
+    nb = synth.pack_batch([structure(oracle, n, (8.5, 9.0, 9.5), nt, 21 + n, 5.0) for n in (40, 23)])
+    if lists == "rows left out":
+        nb["binum"] = nb["binum"] - 17
+    if lists == "one atom named by all":
+        nb["bfirstneigh"] = np.where(nb["bfirstneigh"] >= 0, 5, nb["bfirstneigh"]).astype(np.int32)
+        assert nb["bnumneigh"][0].sum() > 256
+    m = synth.mtp_model(tables(basic), nt, 6, 5.0, 1.5, 3200)
+    m["q_scaler"] = np.linspace(0.8, 1.3, m["q_scaler"].size)
+    md = model_to_device(m, torch.float64)
+    d = to_device(nb, torch.float64)
+    args = (m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+            md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], d["binum"], d["bilist"], d["bnumneigh"],
+            d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"])
+    L = _lib.lib()
+    before = L.a2p_mtp_components_route(1)
+    try:
+        one = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+        L.a2p_mtp_components_route(0)
+        per_column = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+    finally:
+        L.a2p_mtp_components_route(before)
+    for a, b in zip(one, per_column):
+        assert np.abs(b).max() > 0
+        assert close(a, b)
+
+
 def test_components_in_chunks_of_structures(oracle):
     """Enough pair derivatives (level 16: 92 columns, more than 200 MB) that the structures are taken in chunks, the last
     one shorter: every structure equal to the call with that structure alone, bit for bit, in force columns too."""
