@@ -160,10 +160,46 @@ __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 // Lanes j < nc also return the neighbour's index, validity and displacement.
 enum TablePass { TAB_MOMENTS, TAB_TANGENTS, TAB_GRADIENT };
 
+// An array on its way to LDS: the first U entries of every thread are asked for together, and stored when the caller says.
+template <typename V, int NT, int U>
+struct Staged {
+    V v[U];
+    __device__ __forceinline__ void load(const V* src, int n, int lane)
+    {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (lane + u * NT < n) v[u] = src[lane + u * NT];
+    }
+    __device__ __forceinline__ void store(V* dst, const V* src, int n, int lane)
+    {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (lane + u * NT < n) dst[lane + u * NT] = v[u];
+        for (int i = lane + U * NT; i < n; i += NT) dst[i] = src[i];
+    }
+};
+
+// `ahead`: what a thread's first task begins with, read while the workgroup set itself up (is_ahead).
+template <typename T>
+struct TableAhead {
+    T x, y, z;
+    int nj, tj;          // the neighbour as it is listed, and the species of it (of the centre, where it is none)
+    __device__ __forceinline__ void entries(const T* rcs, const int* first, int lane, int c0, int nc)
+    {
+        const int jj = c0 + lane - small_div(lane, nc) * nc;
+        x = rcs[jj * 3 + 0]; y = rcs[jj * 3 + 1]; z = rcs[jj * 3 + 2];
+        nj = first[jj];
+    }
+    __device__ __forceinline__ void species(const int* types, int NF, int center)
+    {
+        tj = types[(unsigned)nj < (unsigned)NF ? nj : center];
+    }
+};
 template <typename T, TablePass PASS, int NT, typename Args>
 __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int lane, int nc, int c0,
                                             const T* rcs, const int* first, const int* types, int center,
-                                            int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true)
+                                            int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true,
+                                            const TableAhead<T>& ahead = TableAhead<T>(), bool is_ahead = false)
 {
     const int kmax = a.p.kmax, nmus = a.p.nmus, K = a.K;
     const int OG = a.OG, ODG = a.ODG, OU = a.OU, OW = a.OW, OF = a.OF, ODF = a.ODF;
@@ -171,11 +207,13 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
     *nj_out = center;
     if (lane < nc) {
         const int jj = c0 + lane;
-        const T x = rcs[jj * 3 + 0], y = rcs[jj * 3 + 1], z = rcs[jj * 3 + 2];
+        T x, y, z;
+        int nj;
+        if (is_ahead) { x = ahead.x; y = ahead.y; z = ahead.z; nj = ahead.nj; }
+        else { x = rcs[jj * 3 + 0]; y = rcs[jj * 3 + 1]; z = rcs[jj * 3 + 2]; nj = first[jj]; }
         d_out[0] = x; d_out[1] = y; d_out[2] = z;
-        int nj = first[jj];
         if ((unsigned)nj >= (unsigned)NF) { atomicOr(a.status, ST_BAD_NEIGHBOR); nj = center; }
-        if ((unsigned)types[nj] >= (unsigned)a.ntypes) atomicOr(a.status, ST_BAD_TYPE);
+        if ((unsigned)(is_ahead ? ahead.tj : types[nj]) >= (unsigned)a.ntypes) atomicOr(a.status, ST_BAD_TYPE);
         *nj_out = nj;
         *valid_out = !(sqrt_t(x * x + y * y + z * z) > a.rmax);      // mtpBasis.h:457, linearMtp.h:316
     }
@@ -192,7 +230,10 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
     for (int task = lane; task < ntask; task += NT) {
         const int role = small_div(task, nc), j = task - role * nc;
         const int jj = c0 + j;
-        const T x = rcs[jj * 3 + 0], y = rcs[jj * 3 + 1], z = rcs[jj * 3 + 2];
+        const bool known = is_ahead && task < NT;                         // (uniform: the first round)
+        T x, y, z;
+        if (known) { x = ahead.x; y = ahead.y; z = ahead.z; }
+        else { x = rcs[jj * 3 + 0]; y = rcs[jj * 3 + 1]; z = rcs[jj * 3 + 2]; }
         const T r = sqrt_t(x * x + y * y + z * z);
         T* t = tab + j * a.E;
         if (role == nrad) {                                            // powers of the unit vector
@@ -213,7 +254,7 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             t[OU + 0] = ux; t[OU + 1] = uy; t[OU + 2] = uz; t[OU + 3] = rinv;
             continue;
         }
-        int nj = first[jj];
+        int nj = known ? ahead.nj : first[jj];
         if ((unsigned)nj >= (unsigned)NF) nj = center;
         if (PASS != TAB_MOMENTS && role == nrad + 1) {
             // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386), kept as w . u and
@@ -254,7 +295,7 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             }
             continue;
         }
-        int tj = types[nj];
+        int tj = known ? ahead.tj : types[nj];
         if ((unsigned)tj >= (unsigned)a.ntypes) tj = 0;
         const int m1 = min(nmus, (role + 1) * share);
         for (int mu = role * share; mu < m1; mu += 2) {
@@ -773,6 +814,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     const int lane = threadIdx.x;     // thread in the workgroup
     const int ii = blockIdx.x, b = blockIdx.y;
     int center, nn, ti;
+    int nchunks, csize;               // the row is cut into equal chunks of at most nc_cap neighbours
+    TableAhead<T> ahead;              // (energies and forces; the loss gradient's registers do not hold it: 166 -> 175 us)
     int mgroups, mh, mtop = 0;        // sums of the basic moments: groups, the thread's group, the longest polynomial
     unsigned pword = 0;               // ... and the thread's polynomial
     {
@@ -788,59 +831,70 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         }
         const int center0 = a.bilist[row], nn0 = a.bnumneigh[row];         // on their way while the plan's arrays are fetched
 
+        // Three trips to memory: the row's head with the plan's arrays, the row's entries with the species of the centre, the
+        // coefficients with the neighbours' species.  (Five before, with the entries and their species behind the barrier: level 20, 8192
+        // atoms 228.8 -> 226.4 us, the training step of level 16, 64 structures of 128 atoms, 272.8 -> 270.5, the linear solver there
+        // 469 -> 462.)
         mgroups = a.mom_groups;       // uniform over the launch
         const unsigned* const bsrc = mgroups ? (const unsigned*)p.poly_pos : p.basic;
-        for (int i = lane; i < n_basic; i += NT) L.bas[i] = bsrc[i];
+        Staged<unsigned, NT, NT == 64 ? 4 : 2> basics;
+        basics.load(bsrc, n_basic, lane);
         mh = mgroups;
         if (mgroups) {
             mh = small_div(lane, p.npoly);
             if (mh < mgroups) pword = p.polys_len[lane - mh * p.npoly];
+        }
+        const bool flat = !LOSS && p.polys_len;
+        const int nwords = flat ? p.npoly : LOSS ? p.npoly : p.nrows + 1;
+        const int* const wsrc = flat ? (const int*)p.polys_len : LOSS ? p.polys_mu : p.rows;
+        Staged<int, NT, NT == 64 ? 2 : 1> words;
+        words.load(wsrc, nwords, lane);
+        center = __builtin_amdgcn_readfirstlane(center0);
+        nn = __builtin_amdgcn_readfirstlane(nn0);
+        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
+        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
+        const int ti0 = types[center];
+        {
+            // (whole-number divisions: small_div cuts a row of two million and more into chunks longer than the table)
+            const unsigned n = nn, cap = MTP_NC, cuts = (n + cap - 1) / cap;
+            nchunks = (int)cuts;
+            csize = cuts > 1 ? (int)((n + cuts - 1) / cuts) : max(nn, 1);
+        }
+        if (!LOSS && nn > 0) ahead.entries(rcs, first, lane, 0, min(csize, nn));
+        for (int i = lane; i < n_moms; i += NT) {
+            M[i] = (T)0;
+            if (LOSS) Tg[i] = (T)0;
+        }
+        basics.store(L.bas, bsrc, n_basic, lane);
+        words.store(L.rws, wsrc, nwords, lane);
+        if (!LOSS && !flat)
+            for (int i = lane; i < p.npoly; i += NT) L.rws[p.nrows + 1 + i] = p.polys[i];
+        if (LOSS)
+            for (int i = lane; i <= nmus; i += NT) L.rws[p.npoly + i] = p.polys_end[i];
+        if (mgroups) {
             const int len = (pword >> 13) & 31;
 #pragma unroll
             for (int c = 0; c < MTP_POLY_MAX; c++)
                 if (__any(len > c)) mtop = c + 1;
         }
-        int* const rws = L.rws;
-        if (!LOSS && p.polys_len) {
-            for (int i = lane; i < p.npoly; i += NT) rws[i] = (int)p.polys_len[i];
-        } else if (!LOSS) {
-            for (int i = lane; i <= p.nrows; i += NT) rws[i] = p.rows[i];
-            for (int i = lane; i < p.npoly; i += NT) rws[p.nrows + 1 + i] = p.polys[i];
-        } else {
-            for (int i = lane; i < p.npoly; i += NT) rws[i] = p.polys_mu[i];
-            for (int i = lane; i <= nmus; i += NT) rws[p.npoly + i] = p.polys_end[i];
-        }
-        center = __builtin_amdgcn_readfirstlane(center0);
-        nn = __builtin_amdgcn_readfirstlane(nn0);
-        if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
-        if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-        ti = __builtin_amdgcn_readfirstlane(types[center]);
+        ti = __builtin_amdgcn_readfirstlane(ti0);
         if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
-        for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
-        for (int i = lane; i < n_moms; i += NT) {
-            M[i] = (T)0;
-            if (LOSS) Tg[i] = (T)0;
-        }
+        const T* const csrc = a.coeffs + (size_t)ti * a.ntypes * nmus * K;
+        Staged<T, NT, NT == 64 ? 2 : 1> coefs;
+        coefs.load(csrc, a.ntypes * nmus * K, lane);
+        if (!LOSS && nn > 0) ahead.species(types, NF, center);
+        coefs.store(cf, csrc, a.ntypes * nmus * K, lane);
         __syncthreads();
     }
 
-    // The row is cut into equal chunks of at most nc_cap neighbours.
-    int nchunks, csize;
-    {
-        MTP_PHASE;
-        // (whole-number divisions: small_div cuts a row of two million and more into chunks longer than the table)
-        const unsigned n = nn, cap = MTP_NC, cuts = (n + cap - 1) / cap;
-        nchunks = (int)cuts;
-        csize = cuts > 1 ? (int)((n + cuts - 1) / cuts) : max(nn, 1);
-    }
-
     // ---- basic moments (and their tangents) --------------------------------------------------
-    for (int c0 = 0; c0 < nn; c0 += csize) {
+    for (int c0 = 0; nn > 0;) {
         const int nc = min(csize, nn - c0);
         {
             MTP_PHASE;
             int nj; bool valid; T d[3];
-            build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+            build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, true,
+                                                                      ahead, !LOSS);
             __syncthreads();
         }
         MTP_PHASE;
@@ -868,31 +922,37 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                 if (LOSS && !no_tan) Tg[i] += group_sum<T>(part + mgroups * p.ncoef_poly + pos, mgroups, p.ncoef_poly);
             }
             __syncthreads();
-            continue;
-        }
-        // (tables beyond the fields of polys_len)
-        for (int i = lane; i < n_basic; i += NT) {
-            const unsigned bw = L.bas[i];
-            const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
-            T acc = (T)0, tacc = (T)0;
-            for (int j = 0; j < nc; j++) {
-                const T* t = tab + j * E;
-                const T g = t[OG + mu];
-                const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
-                const T m = xa * yb * zc;
-                acc += g * m;
-                if (LOSS && !no_tan) {
-                    const T dg = t[ODG + mu], wu = t[OW + 3];
-                    const T gm = (T)ea * t[OX + max(ea - 1, 0)] * yb * zc * t[OW + 0] +
-                                 (T)eb * xa * t[OY + max(eb - 1, 0)] * zc * t[OW + 1] +
-                                 (T)ec * xa * yb * t[OZ + max(ec - 1, 0)] * t[OW + 2];
-                    tacc += wu * m * dg + g * gm;
+        } else {
+            // (tables beyond the fields of polys_len)
+            for (int i = lane; i < n_basic; i += NT) {
+                const unsigned bw = L.bas[i];
+                const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
+                T acc = (T)0, tacc = (T)0;
+                for (int j = 0; j < nc; j++) {
+                    const T* t = tab + j * E;
+                    const T g = t[OG + mu];
+                    const T xa = t[OX + ea], yb = t[OY + eb], zc = t[OZ + ec];
+                    const T m = xa * yb * zc;
+                    acc += g * m;
+                    if (LOSS && !no_tan) {
+                        const T dg = t[ODG + mu], wu = t[OW + 3];
+                        const T gm = (T)ea * t[OX + max(ea - 1, 0)] * yb * zc * t[OW + 0] +
+                                     (T)eb * xa * t[OY + max(eb - 1, 0)] * zc * t[OW + 1] +
+                                     (T)ec * xa * yb * t[OZ + max(ec - 1, 0)] * t[OW + 2];
+                        tacc += wu * m * dg + g * gm;
+                    }
                 }
+                M[i] += acc;
+                if (LOSS) Tg[i] += tacc;
             }
-            M[i] += acc;
-            if (LOSS) Tg[i] += tacc;
+            __syncthreads();
         }
-        __syncthreads();
+        c0 += csize;
+        if (c0 >= nn) break;
+        if (!LOSS) {                   // (not held over the sums)
+            ahead.entries(rcs, first, lane, c0, min(csize, nn - c0));
+            ahead.species(types, NF, center);
+        }
     }
 
     // ---- products, energy, adjoint ------------------------------------------------------------
@@ -1220,19 +1280,19 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                 }
                 __syncthreads();
                 for (int e = lane; e < n2; e += NT) gacc[e] += group_sum<T>(part + e, parts, n2);
-                continue;
-            }
-            // tj of each neighbour of the chunk, for the accumulation below
-            if (h == 0) tjs[j] = valid ? types[nj] : -1;
-            __syncthreads();
-            // lanes <- (mu, k): sequential over neighbours keeps the sum order fixed
-            for (int q = lane; q < n1; q += NT) {
-                const int mu = small_div(q, K), k = q - mu * K;
-                for (int jn = 0; jn < nc; jn++) {
-                    const int tj = tjs[jn];
-                    if (tj < 0) continue;
-                    const T* t = tab + jn * E;
-                    gacc[tj * n1 + q] += t[OF + k] * Pm[jn * nmus + mu] + t[ODF + k] * Qm[jn * nmus + mu];
+            } else {
+                // tj of each neighbour of the chunk, for the accumulation below
+                if (h == 0) tjs[j] = valid ? types[nj] : -1;
+                __syncthreads();
+                // lanes <- (mu, k): sequential over neighbours keeps the sum order fixed
+                for (int q = lane; q < n1; q += NT) {
+                    const int mu = small_div(q, K), k = q - mu * K;
+                    for (int jn = 0; jn < nc; jn++) {
+                        const int tj = tjs[jn];
+                        if (tj < 0) continue;
+                        const T* t = tab + jn * E;
+                        gacc[tj * n1 + q] += t[OF + k] * Pm[jn * nmus + mu] + t[ODF + k] * Qm[jn * nmus + mu];
+                    }
                 }
             }
         }
@@ -1398,7 +1458,8 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lane = threadIdx.x;
     const int ii = blockIdx.x, b = blockIdx.y + kernel_args<CompKernelArgs<T>>()->comp.b0;
-    int nn, pair0, center, ti;
+    int nn, pair0, center, ti, nchunks, chunk;
+    TableAhead<T> ahead;
     {
         COMP_PHASE;
         nn = c.nnc[row];
@@ -1409,26 +1470,31 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
         }
         pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
         center = a.bilist[row];
+        nchunks = (nn + c.nc_cap - 1) / c.nc_cap;
+        chunk = (nn + nchunks - 1) / nchunks;
+        Staged<unsigned, NT, 2> basics;
+        basics.load(p.basic, n_basic, lane);
+        ahead.entries(rcs, first, lane, 0, min(chunk, nn));
         if ((unsigned)center >= (unsigned)NF) center = 0;
         ti = types[center];
         if ((unsigned)ti >= (unsigned)a.ntypes) ti = 0;
-        for (int i = lane; i < n_basic; i += NT)
-            bas[i] = p.basic[i];
-        for (int q = lane; q < a.ntypes * nmus * K; q += NT) cf[q] = a.coeffs[(size_t)ti * a.ntypes * nmus * K + q];
+        const T* const csrc = a.coeffs + (size_t)ti * a.ntypes * nmus * K;
+        Staged<T, NT, 1> coefs;
+        coefs.load(csrc, a.ntypes * nmus * K, lane);
+        ahead.species(types, NF, center);
         for (int i = lane; i < n_moms; i += NT) M[i] = (T)0;
         for (int i = lane; i <= p.x_nodes; i += NT) X[i] = (T)0;
+        basics.store(bas, p.basic, n_basic, lane);
+        coefs.store(cf, csrc, a.ntypes * nmus * K, lane);
     }
     __syncthreads();
 
     // basic moments (as in mtp_atom_kernel)
-    const int MTP_NC = kernel_args<CompKernelArgs<T>>()->comp.nc_cap;
-    const int nchunks = (nn + MTP_NC - 1) / MTP_NC;
-    const int chunk = nchunks > 0 ? (nn + nchunks - 1) / nchunks : 1;
-    for (int c0 = 0; c0 < nn; c0 += chunk) {
+    for (int c0 = 0;;) {
         COMP_PHASE;
         const int nc = min(chunk, nn - c0);
         int nj; bool valid; T d[3];
-        build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+        build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, true, ahead, true);
         __syncthreads();
         for (int i = lane; i < n_basic; i += NT) {
             const unsigned bw = bas[i];
@@ -1441,6 +1507,10 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             M[i] += acc;
         }
         __syncthreads();
+        c0 += chunk;
+        if (c0 >= nn) break;
+        ahead.entries(rcs, first, lane, c0, min(chunk, nn - c0));
+        ahead.species(types, NF, center);
     }
     {
         COMP_PHASE;
