@@ -78,6 +78,8 @@ __host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_
 }
 // the coefficients of the pair-derivative pass's polynomials take the place of the moments when they fit
 __host__ __device__ inline bool mtp_polys_in_moments(int ncoef, int n_moms) { return ncoef <= n_moms; }
+// the tangents of a network's inputs wait in the place of P and Q (loss gradient) when they fit
+__host__ __device__ inline bool mtp_tangents_at_pq(int n_scalar, int nc, int nmus) { return n_scalar <= 2 * nc * nmus + nc; }
 constexpr int MTP_NGMAX = 16;     // most thread groups that share the basic moments of a chunk
 constexpr int MTP_KMAX = 16;      // radial basis size limit
 constexpr int MTP_NMUS_MAX = 8;   // radial function count limit
@@ -447,6 +449,24 @@ __device__ __forceinline__ void piece_sums(T (&v)[N], int rem, int steps)
     }
 }
 
+// Sums of items by neighbouring lanes: log2 of how many lanes an item gets of `nt` threads (at most sixteen), and the sum over
+// an item's lanes, in all of them.
+__device__ __forceinline__ int parts_log2(int nt, int items)
+{
+    int l = 0;
+    while (l < 4 && (items << (l + 1)) <= nt) l++;
+    return l;
+}
+template <typename T>
+__device__ __forceinline__ T parts_sum(T v, int log2_parts)
+{
+    if (log2_parts > 0) v += wave::dpp_move<0xB1>(v);      // quad_perm [1,0,3,2]
+    if (log2_parts > 1) v += wave::dpp_move<0x4E>(v);      // quad_perm [2,3,0,1]
+    if (log2_parts > 2) v += wave::dpp_move<0x141>(v);     // row_half_mirror
+    if (log2_parts > 3) v += wave::dpp_move<0x140>(v);     // row_mirror
+    return v;
+}
+
 // A plan term names its two moments by byte offsets into an array of doubles (index * 8): no shift between the
 // word and the LDS address in fp64.
 template <typename T>
@@ -806,8 +826,8 @@ struct AtomLds {
 // NT threads per centre atom: 64 or 256 (wide_atoms).  Five workgroups of 256 threads fit the LDS of a CU at level 20 and
 // the registers are kept to match (four: 321 us instead of 303 at 8192 atoms; six spill: 361).
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
-// (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.
-template <typename T, bool LOSS, int NT, bool SEED = false>
+// (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.  NET: the instances with a network read-out.
+template <typename T, bool LOSS, int NT, bool SEED = false, bool NET = false>
 __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) == 8 ? 6 : 1)) mtp_atom_kernel(const MtpArgs<T>)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -971,67 +991,109 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         __syncthreads();
         // network buffers (H > 0): inputs q[S]; per neuron w1 tanh', and in loss mode tanh, tanh', tanh'', tau
         T* nnb = L.net;
-        if (a.H > 0) {
+        if constexpr (NET) {
             // one tanh layer of the centre's species on the shifted, scaled scalar moments; the
             // adjoint is seeded with dE_i/dM_k = sum_p w1_p tanh'(h_p) w0_pk / q_scaler_k
             // (nnMtp.h:470-507).  Loss mode also needs the derivative of that seed along the tangent:
             // tau_p = sum_k w0_pk Tg_k / q_scaler_k is the tangent of h_p, and the adjoint of
             // D_w E = sum_p w1_p tanh'(h_p) tau_p  w.r.t. M_k is  sum_p w1_p tanh''(h_p) tau_p w0_pk / q_scaler_k,
             // the seed of the mixed sweep (nnMtpLoss.h:216-610 computes the same quantities atom by atom).
+            // A neuron's sum over the inputs, and an input's over the neurons, by 1, 2 .. 16 neighbouring lanes each, W weights
+            // of a lane on their way together, the first of either sum ahead of what it waits for.  What bounds it is the trips to
+            // the weights and the chain of their operations.  (A wavefront for four neurons at a time with sums over its 64 lanes,
+            // then a lane for an input: 10.8 of the 41 thousand cycles an atom takes at level 12 with 20 neurons, 9.3 of the 55 of the
+            // loss gradient; now 8.4 and 6.7.  Calls: 4000 atoms 47.3 -> 43.5 us, the training step of 40 structures of 100 atoms 156 ->
+            // 147; level 16, 30 neurons, 113 -> 108.6 and 232 -> 218.  Sixteen weights on their way: no faster; the next W behind
+            // them: level 16 108.7 -> 110.8.)
             const int S = p.n_scalar, H = a.H;
             T* qv = nnb;                          // [S] network inputs
             T* hv = nnb + S;                      // [H] pre-activations, then w1 * tanh'
-            T* n_th = hv + H;                     // loss mode: tanh, tanh', tanh'', tau   [H] each
+            T* n_th = hv + H;                     // loss mode: tanh, tanh', w1 tanh'' tau, tau   [H] each
             T* n_d1 = n_th + H;
-            T* n_d2 = n_d1 + H;
-            T* n_tau = n_d2 + H;
+            T* n_c2 = n_d1 + H;
+            T* n_tau = n_c2 + H;
+            // ... and the tangents of the inputs [S], where P and Q come in the last pass, or, when they do not fit there, where the
+            // seeds come after them
+            T* qt = mtp_tangents_at_pq(S, MTP_NC, nmus) ? L.pq : Bm;
             const T* w0 = a.w0 + (size_t)ti * H * S;
             const T* w1 = a.w1 + (size_t)ti * H;
-            for (int s = lane; s < S; s += NT) qv[s] = (M[p.mapping[s]] - a.q_shift[s]) / a.q_scaler[s];
+            constexpr int W = LOSS ? 4 : 8;       // (eight: 8 more values spilled by the loss gradient)
+            T w[W];
+            // weights of neuron n and the inputs k0, k0 + step ..; and of input k and the neurons from n0 on
+            auto row_weights = [&](int n, int k0, int step) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < W; u++) w[u] = k0 + u * step < S ? w0[(size_t)min(n, H - 1) * S + k0 + u * step] : (T)0;
+            };
+            auto column_weights = [&](int k, int n0, int step) __attribute__((always_inline)) {
+#pragma unroll
+                for (int u = 0; u < W; u++) w[u] = n0 + u * step < H ? w0[(size_t)(n0 + u * step) * S + min(k, S - 1)] : (T)0;
+            };
+            const int lh = parts_log2(NT, H), ph = 1 << lh, ls = parts_log2(NT, S), ps = 1 << ls;
+            const int hl = lane >> lh, hp = lane & (ph - 1), sl = lane >> ls, sp = lane & (ps - 1);
+            row_weights(hl, hp, ph);
+            const T w1_own = w1[min(lane, H - 1)];
+            for (int s = lane; s < S; s += NT) {
+                const int m = p.mapping[s];
+                const T scaler = a.q_scaler[s];
+                qv[s] = (M[m] - a.q_shift[s]) / scaler;
+                if (LOSS) qt[s] = Tg[m] / scaler;
+            }
             __syncthreads();
-            // a wavefront takes four neurons at a time, so that their weights' ways and their sums overlap
-            for (int n0 = (lane >> 6) * 4; n0 < H; n0 += NT / 64 * 4) {
-                T acc[4], tac[4];
+            for (int n0 = 0; n0 < H; n0 += NT >> lh) {
+                T acc = (T)0, tac = (T)0;
+                for (int k0 = 0; k0 < S; k0 += W * ph) {
+                    if (n0 + k0 > 0) row_weights(n0 + hl, k0 + hp, ph);
 #pragma unroll
-                for (int u = 0; u < 4; u++) acc[u] = tac[u] = (T)0;
-                for (int k = lane & 63; k < S; k += 64) {
-                    const T q = qv[k], t = LOSS ? Tg[p.mapping[k]] / a.q_scaler[k] : (T)0;
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const T w = w0[(size_t)min(n0 + u, H - 1) * S + k];
-                        acc[u] += w * q;
-                        if (LOSS) tac[u] += w * t;
+                    for (int u = 0; u < W; u++) {
+                        const int k = min(k0 + hp + u * ph, S - 1);
+                        acc += w[u] * qv[k];
+                        if (LOSS) tac += w[u] * qt[k];
                     }
                 }
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    acc[u] = wave::all_sum(acc[u]);
-                    if (LOSS) tac[u] = wave::all_sum(tac[u]);
-                    if ((lane & 63) == u && n0 + u < H) {
-                        hv[n0 + u] = acc[u];
-                        if (LOSS) n_tau[n0 + u] = tac[u];
-                    }
+                acc = parts_sum(acc, lh);
+                if (LOSS) tac = parts_sum(tac, lh);
+                if (hp == 0 && n0 + hl < H) {
+                    hv[n0 + hl] = acc;
+                    if (LOSS) n_tau[n0 + hl] = tac;
                 }
             }
+            column_weights(sl, sp, ps);
+            const int m_own = p.mapping[min(sl, S - 1)];
+            const T scaler_own = a.q_scaler[min(sl, S - 1)];
             __syncthreads();
             for (int n = lane; n < H; n += NT) {
-                const T th = tanh_t(hv[n]);
+                const T th = tanh_t(hv[n]), w1n = n == lane ? w1_own : w1[n];
                 const T d1 = (T)1 - th * th;
-                e_part += w1[n] * th;
-                hv[n] = w1[n] * d1;
-                if (LOSS) { n_th[n] = th; n_d1[n] = d1; n_d2[n] = (T)-2 * th * d1; }
-            }
-            __syncthreads();
-            for (int k = lane; k < S; k += NT) {
-                T acc = (T)0, bac = (T)0;
-#pragma unroll 4
-                for (int n = 0; n < H; n++) {
-                    const T w = w0[(size_t)n * S + k];
-                    acc += hv[n] * w;
-                    if (LOSS) bac += w1[n] * n_d2[n] * n_tau[n] * w;
+                e_part += w1n * th;
+                hv[n] = w1n * d1;
+                if (LOSS) {
+                    n_th[n] = th; n_d1[n] = d1;
+                    n_c2[n] = w1n * ((T)-2 * th * d1) * n_tau[n];
                 }
-                A[p.mapping[k]] = acc / a.q_scaler[k];
-                if (LOSS && a.nn_exact) Bm[p.mapping[k]] = bac / a.q_scaler[k];
+            }
+            if (LOSS && qt == Bm)
+                for (int s = lane; s < S; s += NT) qt[s] = (T)0;
+            __syncthreads();
+            for (int i0 = 0; i0 < S; i0 += NT >> ls) {
+                const int k = i0 + sl;
+                T acc = (T)0, bac = (T)0;
+                for (int n0 = 0; n0 < H; n0 += W * ps) {
+                    if (i0 + n0 > 0) column_weights(k, n0 + sp, ps);
+#pragma unroll
+                    for (int u = 0; u < W; u++) {
+                        const int n = min(n0 + sp + u * ps, H - 1);
+                        acc += hv[n] * w[u];
+                        if (LOSS) bac += n_c2[n] * w[u];
+                    }
+                }
+                acc = parts_sum(acc, ls);
+                if (LOSS) bac = parts_sum(bac, ls);
+                if (sp == 0 && k < S) {
+                    const int m = i0 > 0 ? p.mapping[k] : m_own;
+                    const T scaler = i0 > 0 ? a.q_scaler[k] : scaler_own;
+                    A[m] = acc / scaler;
+                    if (LOSS && a.nn_exact) Bm[m] = bac / scaler;
+                }
             }
         } else if (seeded) {
             for (int s = lane; s < p.n_scalar; s += NT) A[p.mapping[s]] = a.row_seed[row * p.n_scalar + s];
@@ -1056,7 +1118,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         MTP_PHASE;
         // the leaves' moments: their part of the energy, or, for the loss gradient, the moments (and tangents) themselves;
         // mixed adjoints: linearMtpLoss.h:417-434; the reference's network backward has none (Bm stays zero)
-        if (LOSS && !no_tan && (a.H == 0 || a.nn_exact))
+        if (LOSS && !no_tan && (!NET || a.nn_exact))
             sweep_reverse<T, LOSS, true>(p.rev[NT / 256], M, A, Bm, (const T*)Tg, lane,
                 [&](int m, T v, T t) __attribute__((always_inline)) { M[m] = v; Tg[m] = t; });
         else
@@ -1185,23 +1247,23 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             __syncthreads();         // other threads overwrite some of these entries below
             // everything but the coefficient block is written now: the pass over the neighbours below does
             // not read the moments or their tangents, and the group sums may take their place
-            if (a.H > 0) {
+            if constexpr (NET) {
                 // compact row of the centre species: coefficient block | w0[H, S] | w1[H] | bias
                 const int S = p.n_scalar, H = a.H, nblk = a.ntypes * nmus * K;
                 const T* qv = L.net;
                 const T* n_th = qv + S + H;
                 const T* n_d1 = n_th + H;
-                const T* n_d2 = n_d1 + H;
-                const T* n_tau = n_d2 + H;
+                const T* n_tau = n_d1 + 2 * H;
+                const bool at_pq = mtp_tangents_at_pq(S, MTP_NC, nmus);
                 const T* w1 = a.w1 + (size_t)ti * H;
                 const T* w0 = a.w0 + (size_t)ti * H * S;
                 for (int q = lane; q < H * S; q += NT) {
                     const int n = q / S, k = q - n * S;
-                    const T tk = Tg[p.mapping[k]] / a.q_scaler[k];
+                    const T tk = at_pq ? L.pq[k] : Tg[p.mapping[k]] / a.q_scaler[k], d2 = (T)-2 * n_th[n] * n_d1[n];
                     if (a.nn_exact)
-                        grow[nblk + q] = w1[n] * ((cE * n_d1[n] + n_d2[n] * n_tau[n]) * qv[k] + n_d1[n] * tk);
+                        grow[nblk + q] = w1[n] * ((cE * n_d1[n] + d2 * n_tau[n]) * qv[k] + n_d1[n] * tk);
                     else        // nnMtpLoss.h:560-585: only the k' = k term of tau
-                        grow[nblk + q] = w1[n] * (cE * n_d1[n] * qv[k] + tk * (n_d1[n] + n_d2[n] * w0[q] * qv[k]));
+                        grow[nblk + q] = w1[n] * (cE * n_d1[n] * qv[k] + tk * (n_d1[n] + d2 * w0[q] * qv[k]));
                 }
                 for (int n = lane; n < H; n += NT) grow[nblk + H * S + n] = cE * n_th[n] + n_d1[n] * n_tau[n];
                 if (lane == 0) grow[nblk + H * S + H] = cE;
@@ -1299,7 +1361,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         __syncthreads();
         MTP_PHASE;
         const T* const gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;
-        T* const grow = a.gpart + row * a.ngrad + (a.H > 0 ? 0 : (size_t)ti * a.ntypes * nmus * K);
+        T* const grow = a.gpart + row * a.ngrad + (NET ? 0 : (size_t)ti * a.ntypes * nmus * K);
         for (int q = lane; q < a.ntypes * nmus * K; q += NT) grow[q] = gacc[q];
     }
 }
@@ -2722,6 +2784,8 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
     auto kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
+    if constexpr (!SEED)
+        if (a.H > 0) kern = wide ? mtp_atom_kernel<T, LOSS, 256, false, true> : mtp_atom_kernel<T, LOSS, 64, false, true>;
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)lds));

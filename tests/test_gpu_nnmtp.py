@@ -146,6 +146,21 @@ def test_loss_step_complete_derivative(oracle, level, nt, H):
     assert np.array_equal(fwd["bloss"], got["bloss"]) and "dcoeffs" not in fwd
 
 
+@pytest.mark.parametrize("level", [8, 12, 16])              # 9, 29 and 92 inputs; 64 threads, and 256 for the loss gradient
+@pytest.mark.parametrize("H", [1, 4, 5, 16, 33, 65, 257])
+def test_readout_by_neighbouring_lanes(oracle, level, H):
+    """Neurons and inputs summed by sixteen lanes each down to one, and more of them than the workgroup has threads: energies,
+    forces, virials and the loss gradient against the oracle, fp64 1e-10."""
+    m, nb, labels = loss_inputs(oracle, level, 2, H, sizes=(13, 9))
+    e, f, v, _, _ = run(m, nb)
+    er, fr, vr, _ = oracle.nnmtp_efv(m, nb)
+    assert close(e, er) and close(f, fr) and close(v, vr)
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w, True), oracle.nnmtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dw0", "dw1", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
 @pytest.mark.parametrize("level,nt,H", [(8, 2, 7), (16, 3, 20)])
 def test_loss_step_reference_formulas(oracle, level, nt, H):
     """exact_gradient=False (the operators' default) against the committed output of the reference's
