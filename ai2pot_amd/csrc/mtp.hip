@@ -1810,64 +1810,104 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
 // Bound by the reads of the pair derivatives, under which the virial's operations hide (in mtp_components_kernel they took a
 // fifth of its instructions and the registers of four more reads in flight); sorting the lists by insertion, one thread per
 // atom, used to take as long as they do (95 us beside 98 us at 64 structures of 128 atoms).
-constexpr int COMP_SORT = 256;
+// With more than 64 columns a lane takes two of them, 64 apart, so that an atom's pairs are ranked once; the displacements of the
+// first COMP_DISP pairs lie in LDS (of 256: 20 instead of 32 wavefronts to a compute unit).  2 x 50 -> 2 x 41 us there.
+constexpr int COMP_SORT = 256, COMP_DISP = 128;
 
-template <typename T>
+template <typename T, int NC>
 __global__ void __launch_bounds__(64)
 comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
                   const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ brcs, const T* __restrict__ pb,
                   const T* __restrict__ rowpart, T* __restrict__ vpart, T* __restrict__ fcomp)
 {
     __shared__ int list[COMP_SORT], order[COMP_SORT];
-    __shared__ T disp[COMP_SORT][3];
-    const int t = blockIdx.x + row0, lane = threadIdx.x, col = blockIdx.y * 64 + lane, s = min(col, S - 1);
+    __shared__ T disp[COMP_DISP][3];
+    const int t = blockIdx.x + row0, lane = threadIdx.x, col0 = blockIdx.y * 64 * NC + lane;
     const int* v = inc + (seg ? (size_t)seg[t] : (size_t)t * cap);
     const int m = seg ? seg[t + 1] - seg[t] : min(cnt[t], cap);
     const int r1 = row_of1[t], base = pair_off[row0];    // pb holds the pairs from row0 on
     const bool ranked = m <= COMP_SORT;
+    int s[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) s[c] = min(col0 + c * 64, S - 1);
     auto pair_of = [&](int q) __attribute__((always_inline)) { const int row = q / U; return pair_off[row] + (q - row * U) - base; };
     if (ranked) {
         for (int k = lane; k < m; k += 64) list[k] = v[k];
         __syncthreads();
-        for (int k = lane; k < m; k += 64) {
+        int place[COMP_SORT / 64];
+#pragma unroll
+        for (int u = 0; u < COMP_SORT / 64; u++) {
+            const int k = u * 64 + lane;
+            if (u * 64 >= m) break;
+            if (k >= m) continue;
             const int x = list[k], pair = pair_of(x);
-            const T* d = brcs + (size_t)x * 3;
-            const T dx = d[0], dy = d[1], dz = d[2];
+            T d[3];
+#pragma unroll
+            for (int q = 0; q < 3; q++) d[q] = brcs[(size_t)x * 3 + q];
             int r = 0;
             for (int i = 0; i < m; i++) r += list[i] < x;
+            place[u] = r;
             order[r] = pair;
-            disp[r][0] = dx; disp[r][1] = dy; disp[r][2] = dz;
+            if (r < COMP_DISP)
+#pragma unroll
+                for (int q = 0; q < 3; q++) disp[r][q] = d[q];
         }
         __syncthreads();
-    }
-    T f[3] = {(T)0, (T)0, (T)0}, vir[9];
+        if (m > COMP_DISP) {                             // the places in the lists too, in order
+            int x[COMP_SORT / 64];
 #pragma unroll
-    for (int i = 0; i < 9; i++) vir[i] = (T)0;
-    if (r1 > 0) {
-        const T* o = rowpart + (size_t)(r1 - 1) * 3 * S + s;
+            for (int u = 0; u < COMP_SORT / 64; u++)
+                if (u * 64 + lane < m) x[u] = list[u * 64 + lane];
+            __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 3; i++) f[i] = o[(size_t)i * S];
-    }
-    auto take = [&](const T (&g)[3], const T* d) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 3; i++) {
-            f[i] -= g[i];
-#pragma unroll
-            for (int k = 0; k < 3; k++) vir[i * 3 + k] -= g[i] * d[k];
+            for (int u = 0; u < COMP_SORT / 64; u++)
+                if (u * 64 + lane < m) list[place[u]] = x[u];
+            __syncthreads();
         }
+    }
+    T f[NC][3], vir[NC][9];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) vir[c][i] = (T)0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) f[c][i] = r1 > 0 ? rowpart[((size_t)(r1 - 1) * 3 + i) * S + s[c]] : (T)0;
+    }
+    auto take = [&](const T (&g)[NC][3], T d0, T d1, T d2) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                f[c][i] -= g[c][i];
+                vir[c][i * 3 + 0] -= g[c][i] * d0;
+                vir[c][i * 3 + 1] -= g[c][i] * d1;
+                vir[c][i * 3 + 2] -= g[c][i] * d2;
+            }
+    };
+    auto fetch = [&](T (&g)[NC][3], int pair) __attribute__((always_inline)) {
+        const T* src = pb + (size_t)pair * 3 * S;
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) g[c][i] = src[(size_t)i * S + s[c]];
     };
     if (ranked) {
-        for (int k0 = 0; k0 < m; k0 += 4) {              // twelve loads in flight
-            T g[4][3];
+        for (int k0 = 0; k0 < m; k0 += 4) {              // twelve loads of a column in flight
+            T g[4][NC][3];
 #pragma unroll
-            for (int u = 0; u < 4; u++) {
-                const T* src = pb + (size_t)order[min(k0 + u, m - 1)] * 3 * S + s;
+            for (int u = 0; u < 4; u++) fetch(g[u], order[min(k0 + u, m - 1)]);
+            if (k0 + 4 <= COMP_DISP || m <= COMP_DISP) {
 #pragma unroll
-                for (int i = 0; i < 3; i++) g[u][i] = src[(size_t)i * S];
+                for (int u = 0; u < 4; u++)
+                    if (k0 + u < m) take(g[u], disp[k0 + u][0], disp[k0 + u][1], disp[k0 + u][2]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (k0 + u < m) {
+                        const T* d = brcs + (size_t)list[k0 + u] * 3;
+                        take(g[u], d[0], d[1], d[2]);
+                    }
             }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (k0 + u < m) take(g[u], disp[k0 + u]);
         }
     } else {
         int last = -1;
@@ -1880,19 +1920,22 @@ comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict_
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) next = min(next, __shfl_xor(next, off, 64));
             last = next;
-            const T* src = pb + (size_t)pair_of(next) * 3 * S + s;
-            T g[3];
-#pragma unroll
-            for (int i = 0; i < 3; i++) g[i] = src[(size_t)i * S];
-            take(g, brcs + (size_t)next * 3);
+            T g[NC][3];
+            fetch(g, pair_of(next));
+            const T* d = brcs + (size_t)next * 3;
+            take(g, d[0], d[1], d[2]);
         }
     }
-    if (col < n)
 #pragma unroll
-        for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + col] = col < S ? f[i] : (T)0;
-    if (col < S)
+    for (int c = 0; c < NC; c++) {
+        const int col = col0 + c * 64;
+        if (col < n)
 #pragma unroll
-        for (int i = 0; i < 9; i++) vpart[((size_t)t * 9 + i) * S + col] = vir[i];
+            for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + col] = col < S ? f[c][i] : (T)0;
+        if (col < S)
+#pragma unroll
+            for (int i = 0; i < 9; i++) vpart[((size_t)t * 9 + i) * S + col] = vir[c][i];
+    }
 }
 
 // Energy and virial columns per structure: sums over the rows (virial: the atoms that the pairs name) in order, in two steps (blocks of COMP_ROWS rows, then
@@ -3236,7 +3279,8 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
             prof_end(stream);
         }
         prof_begin("mtp_components_sums", stream);
-        hipLaunchKernelGGL(comp_force_kernel<T>, dim3(nb * P, ceil_div(n, 64)), dim3(64), 0, stream, S, n, U, U, b0 * P,
+        auto sums = n > 64 ? comp_force_kernel<T, 2> : comp_force_kernel<T, 1>;
+        hipLaunchKernelGGL(sums, dim3(nb * P, ceil_div(n, n > 64 ? 128 : 64)), dim3(64), 0, stream, S, n, U, U, b0 * P,
                            (const int*)pair_off, (const int*)row_of1,
                            (const int*)cnt, in_seg, (const int*)inc, a.brcs, (const T*)pb, (const T*)rowpart, vpart, fcomp);
         prof_end(stream);
