@@ -6,9 +6,10 @@
 // [X | y] is cut into blocks of rows; a workgroup takes a block, 32 rows at a time through LDS, and up to 24 of the 16 x 16
 // tiles of the upper triangle of [X | y]^T [X | y], six per wavefront in the accumulators of the matrix instructions
 // (16 x 16 x 4, the precision of X).  A second kernel adds the blocks' tiles in block order, in double, with the weights.
-// Bound by the matrix instructions (24,640 rows, 95 columns, fp64: 21 tiles x 6,160 instructions of 64 cycles on 1024 units)
-// and by the two launches; a batched library product per matrix with its concatenation, sum and scaling took 25 launches
-// and about 100 us for the same (27 + 10 us here).
+// Bound by the way of the rows through registers and LDS to the matrix instructions (24,640 rows, 95 columns, fp64: 21 tiles x 6,160
+// instructions of 64 cycles on 1024 units, 3.4 us) and by the two launches; a batched library product per matrix with its
+// concatenation, sum and scaling took 25 launches and about 100 us for the same.  Rows one pass ahead 27.8 -> 26.0 us, two blocks to
+// a compute unit 19.5; the sum of the blocks 10 -> 6.4.
 #include "a2p_common.h"
 #include "wave_ops.h"
 
@@ -61,23 +62,41 @@ __global__ void __launch_bounds__(256) gram_kernel(const GramArgs<T> a)
         tile_of(min(t0 + q, a.ntiles - 1), a.nc, ti[q], tj[q]);
         acc[q] = {0, 0, 0, 0};
     }
+    // Eight rows of a column per wavefront, all in flight (rows beyond the block and columns beyond y are zero).  Those of the
+    // first AHEAD columns of a lane are on their way while the rows before them are multiplied.
+    constexpr int AHEAD = 2, PER = GR_ROWS / 4;
+    auto fetch = [&](T (&v)[PER], int s0, int c) __attribute__((always_inline)) {
+        const T* const src = c < n ? X + c : y;
+        const long long step = c < n ? n : 1;
+#pragma unroll
+        for (int i = 0; i < PER; i++) v[i] = src[(r0 + min(s0 + wave * PER + i, rows - 1)) * step];
+    };
+    auto store = [&](T (&v)[PER], int s0, int c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            const int r = wave * PER + i;
+            tab[r * a.stride + c] = s0 + r >= rows || c > n ? (T)0 : v[i];
+        }
+    };
+    T ahead[AHEAD][PER];
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++)
+        if (lane + u * 64 < cols) fetch(ahead[u], 0, lane + u * 64);
     for (int s0 = 0; s0 < rows; s0 += GR_ROWS) {
         __syncthreads();
-        // eight rows per wavefront, all in flight (rows beyond the block and columns beyond y are zero)
-        for (int c = lane; c < cols; c += 64) {
-            T v[GR_ROWS / 4];
-            const T* const src = c < n ? X + c : y;
-            const long long step = c < n ? n : 1;
 #pragma unroll
-            for (int i = 0; i < GR_ROWS / 4; i++) {
-                const int r = s0 + wave * (GR_ROWS / 4) + i;
-                v[i] = src[(r0 + min(r, rows - 1)) * step];
-                if (r >= rows || c > n) v[i] = (T)0;
-            }
-#pragma unroll
-            for (int i = 0; i < GR_ROWS / 4; i++) tab[(wave * (GR_ROWS / 4) + i) * a.stride + c] = v[i];
+        for (int u = 0; u < AHEAD; u++)
+            if (lane + u * 64 < cols) store(ahead[u], s0, lane + u * 64);
+        for (int c = lane + AHEAD * 64; c < cols; c += 64) {
+            T v[PER];
+            fetch(v, s0, c);
+            store(v, s0, c);
         }
         __syncthreads();
+        if (s0 + GR_ROWS < rows)
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++)
+                if (lane + u * 64 < cols) fetch(ahead[u], s0 + GR_ROWS, lane + u * 64);
         for (int st = 0; st < GR_ROWS; st += 4) {
             const T* t = tab + (st + k4) * a.stride + c16;
 #pragma unroll
@@ -94,16 +113,18 @@ __global__ void __launch_bounds__(256) gram_kernel(const GramArgs<T> a)
     }
 }
 
-// One tile per workgroup: four threads per entry take a quarter of the blocks each.
+// A quarter of a tile per workgroup: sixteen threads per entry take a sixteenth of the blocks each.  Bound by its dependent loads (a
+// workgroup per tile with four threads per entry: 10 us for 198 blocks, this 4.6, and 6.4 for 394).
+constexpr int GS_PARTS = 16, GS_ENTRIES = 64;
 template <typename T>
-__global__ void __launch_bounds__(1024)
+__global__ void __launch_bounds__(GS_PARTS * GS_ENTRIES)
 gram_sum_kernel(const GramArgs<T> a, T* __restrict__ A, T* __restrict__ b)
 {
-    __shared__ double red[4][256];
-    const int e = threadIdx.x & 255, part = threadIdx.x >> 8, n = a.n;
+    __shared__ double red[GS_PARTS][GS_ENTRIES];
+    const int part = threadIdx.x / GS_ENTRIES, mine = threadIdx.x % GS_ENTRIES, e = blockIdx.y * GS_ENTRIES + mine, n = a.n;
     int ti, tj;
     tile_of(blockIdx.x, a.nc, ti, tj);
-    const int blocks = a.first_block[GR_SETS], run = (blocks + 3) / 4;
+    const int blocks = a.first_block[GR_SETS], run = (blocks + GS_PARTS - 1) / GS_PARTS;
     double sum = 0.0;
 #pragma unroll
     for (int k = 0; k < GR_SETS; k++) {
@@ -118,10 +139,13 @@ gram_sum_kernel(const GramArgs<T> a, T* __restrict__ A, T* __restrict__ b)
         }
         sum += a.w[k] * s;
     }
-    red[part][e] = sum;
+    red[part][mine] = sum;
     __syncthreads();
     if (part) return;
-    const T v = (T)(((red[0][e] + red[1][e]) + red[2][e]) + red[3][e]);
+    sum = red[0][mine];
+#pragma unroll
+    for (int q = 1; q < GS_PARTS; q++) sum += red[q][mine];
+    const T v = (T)sum;
     const int i = ti * 16 + (e >> 4), j = tj * 16 + (e & 15);
     if (i < n && j < n && i <= j) { A[(size_t)i * n + j] = v; A[(size_t)j * n + i] = v; }
     if (i < n && j == n) b[i] = v;
@@ -145,9 +169,10 @@ int normal_equations(int n, const long long* rows, const double* w, const T* con
         A2P_REQUIRE(rows[k] >= 0 && (rows[k] == 0 || (X[k] && y[k])), A2P_ERR_INVALID, "normal equations: null matrix");
         total += rows[k];
     }
-    // about one workgroup per compute unit over all tile groups; never less than one pass through LDS
+    // about two workgroups per compute unit over all tile groups (one: 26.0 + 4.6 us instead of 19.5 + 6.4 for 24,640 rows of 95
+    // columns); never less than one pass through LDS
     const int groups = ceil_div(a.ntiles, 4 * GR_TILES);
-    const long long want = std::max(32, 256 / groups);
+    const long long want = std::max(32, 512 / groups);
     const long long per = std::max<long long>(GR_ROWS, (total / want + GR_ROWS - 1) / GR_ROWS * GR_ROWS);
     A2P_REQUIRE(per < (1ll << 30), A2P_ERR_INVALID, "normal equations: too many rows");
     a.per_block = (int)per;
@@ -166,7 +191,7 @@ int normal_equations(int n, const long long* rows, const double* w, const T* con
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     prof_begin("gram", stream);
     if (blocks) hipLaunchKernelGGL(kern, dim3(blocks, groups), dim3(256), lds, stream, a);
-    hipLaunchKernelGGL(gram_sum_kernel<T>, dim3(a.ntiles), dim3(1024), 0, stream, a, A, b);
+    hipLaunchKernelGGL(gram_sum_kernel<T>, dim3(a.ntiles, 256 / GS_ENTRIES), dim3(GS_PARTS * GS_ENTRIES), 0, stream, a, A, b);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
