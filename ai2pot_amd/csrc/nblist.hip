@@ -62,6 +62,8 @@ struct Grid {
     int img_lo[3];    // image index ranges
     int img_dim[3];
     int nimg;
+    int diagonal;     // b is diagonal: a coordinate of an image depends on the image's index along its own axis only
+    unsigned inv_z, inv_yz;   // floor(m / img_dim[2]) = m * inv_z >> 16, of img_dim[1] * img_dim[2] likewise, for m < 32
     int N;
     int ext_bins;     // ceil(rcut / bin_size) = 2
     int is_cart;
@@ -361,10 +363,59 @@ __device__ __forceinline__ void entry_load(const double* p, double& x, double& y
     x = v0.x; y = v0.y; z = v1.x; bits = (int)__double_as_longlong(v1.y);
 }
 
-// One thread per atom walks its images (x outer, z inner: image m = (i * dim_y + j) * dim_z + k,
+// The images of an atom that can lie in the kept box (the comparisons of locate), a bit each; nimg <= IMAGE_BITS.  Axis by axis
+// where the lattice allows it: the products with its zeros add nothing to a coordinate, rounded or not.
+constexpr int IMAGE_BITS = 32;
+template <typename T>
+__device__ __forceinline__ unsigned images_in_reach(const Grid<T>& g, const T (&xp)[3], int i0, int i1)
+{
+    unsigned mask = 0;
+    if (g.diagonal) {
+        unsigned axis[3];
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            axis[a] = 0;
+            for (int q = 0; q < g.img_dim[a]; q++) {
+                const T c = add_rn(xp[a], mul_rn(g.b[a][a], (T)(g.img_lo[a] + q)));
+                if (!(c < g.keep_lo[a] || c > g.keep_hi[a])) axis[a] |= 1u << q;
+            }
+        }
+        for (int i = i0; i < i1; i++)
+            for (int j = 0; j < g.img_dim[1]; j++)
+                if (axis[0] >> i & axis[1] >> j & 1u) mask |= axis[2] << (i * g.img_dim[1] + j) * g.img_dim[2];
+        return mask;
+    }
+    int m = i0 * g.img_dim[1] * g.img_dim[2];
+    for (int i = i0; i < i1; i++)
+        for (int j = 0; j < g.img_dim[1]; j++)
+            for (int k = 0; k < g.img_dim[2]; k++, m++) {
+                bool in = true;
+#pragma unroll
+                for (int a = 0; a < 3; a++) {
+                    const T c = image_coord(xp[a], g.b[0][a], g.b[1][a], g.b[2][a], g.img_lo[0] + i, g.img_lo[1] + j, g.img_lo[2] + k);
+                    if (c < g.keep_lo[a] || c > g.keep_hi[a]) in = false;
+                }
+                if (in) mask |= 1u << m;
+            }
+    return mask;
+}
+template <typename T>
+__device__ __forceinline__ int locate(const Grid<T>& g, const T (&xp)[3], int m, T* c)
+{
+    const int i = (int)((unsigned)m * g.inv_yz >> 16), jk = m - i * g.img_dim[1] * g.img_dim[2];
+    const int j = (int)((unsigned)jk * g.inv_z >> 16);
+    return locate(g, xp, i, j, jk - j * g.img_dim[2], c);
+}
+
+// One thread per atom takes its images (x outer, z inner: image m = (i * dim_y + j) * dim_z + k,
 // supercell index m * N + p, structure.h:654-681).
 // With split > 1 (small structures, where a thread per atom leaves most of the chip idle) a thread takes one
 // x-layer of an atom's images: thread = atom * split + layer, split = img_dim[0].
+// Bound by the comparisons, and, at a face of the cell, by the trips to the bins one after the other: up to IMAGE_BITS images are
+// first told by comparisons alone (of 27 images of most atoms one is in reach), and those in reach then go to their bins
+// IMAGES_AT_ONCE together.  Image by image the two kernels took 24.3 + 37.9 instead of 22.4 + 35.0 us for 1,048,576 atoms in fp32, and
+// a build of 131,072 atoms in fp64 with sorted rows 244 instead of 236.
+constexpr int IMAGES_AT_ONCE = 4;
 template <typename T>
 __global__ void count_kernel(const Grid<T> g_in, const T* __restrict__ x, int* __restrict__ counts,
                              int* __restrict__ incoming, const GridDyn<T>* __restrict__ gd,
@@ -383,10 +434,17 @@ __global__ void count_kernel(const Grid<T> g_in, const T* __restrict__ x, int* _
         if (ilist) { ilist[p] = p; types_out[p] = types[p]; }
     }
     const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+    T c[3];
+    if (g.nimg <= IMAGE_BITS) {
+        for (unsigned mask = images_in_reach(g, xp, i0, i1); mask; mask &= mask - 1) {
+            const int bin = locate(g, xp, __ffs((int)mask) - 1, c);
+            if (bin >= 0) atomicAdd(&counts[bin], 1);
+        }
+        return;
+    }
     for (int i = i0; i < i1; i++)
         for (int j = 0; j < g.img_dim[1]; j++)
             for (int k = 0; k < g.img_dim[2]; k++) {
-                T c[3];
                 const int bin = locate(g, xp, i, j, k, c);
                 if (bin >= 0) atomicAdd(&counts[bin], 1);
             }
@@ -403,6 +461,27 @@ __global__ void fill_kernel(const Grid<T> g_in, const T* __restrict__ x, const i
     if (p >= g.N) return;
     const int i0 = split > 1 ? t - p * split : 0, i1 = split > 1 ? i0 + 1 : g.img_dim[0];
     const T xp[3] = {x[(size_t)p * 3], x[(size_t)p * 3 + 1], x[(size_t)p * 3 + 2]};
+    if (g.nimg <= IMAGE_BITS) {
+        unsigned mask = images_in_reach(g, xp, i0, i1);
+        while (mask) {
+            int bin[IMAGES_AT_ONCE], pos[IMAGES_AT_ONCE], im[IMAGES_AT_ONCE];
+            T c[IMAGES_AT_ONCE][3];
+#pragma unroll
+            for (int u = 0; u < IMAGES_AT_ONCE; u++) {
+                bin[u] = -1;
+                if (mask) {
+                    im[u] = __ffs((int)mask) - 1;
+                    mask &= mask - 1;
+                    bin[u] = locate(g, xp, im[u], c[u]);
+                }
+                if (bin[u] >= 0) pos[u] = atomicAdd(&cursor[bin[u]], 1);
+            }
+#pragma unroll
+            for (int u = 0; u < IMAGES_AT_ONCE; u++)
+                if (bin[u] >= 0) entry_store<T>(s_rec + (size_t)(offsets[bin[u]] + pos[u]) * 4, c[u][0], c[u][1], c[u][2], im[u] * g.N + p);
+        }
+        return;
+    }
     int m = i0 * g.img_dim[1] * g.img_dim[2];
     for (int i = i0; i < i1; i++)
         for (int j = 0; j < g.img_dim[1]; j++)
@@ -1773,6 +1852,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     A2P_REQUIRE(nimg * N < (1ll << 31), A2P_ERR_INVALID,
                 "nblist: %lld images x %d atoms exceeds the reference's int supercell index", nimg, N);
     g.nimg = (int)nimg;
+    g.inv_z = 65536u / g.img_dim[2] + 1;
+    g.inv_yz = 65536u / (g.img_dim[1] * g.img_dim[2]) + 1;
     g.ext_bins = (int)std::ceil(g.rcut / g.bin_size);          // binLinkedList.h:914-915
     A2P_REQUIRE(g.ext_bins >= 1 && g.ext_bins <= 3, A2P_ERR_INVALID, "nblist: unsupported bin stencil");
     g.inv_side = 1.0f / (float)(2 * g.ext_bins + 1);
@@ -1838,6 +1919,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     bool diagonal = true;
     for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) diagonal = diagonal && (i == j || g.b[i][j] == (T)0);
+    g.diagonal = diagonal ? 1 : 0;
     const bool separable = diagonal && g.img_dim[0] <= 3 && g.img_dim[1] <= 3 && g.img_dim[2] <= 3;
     bool small = !large && !(same && bound->large) && N <= NBS_ATOMS && (separable || (long long)N * g.nimg <= NBS_IMAGES);
     if (small) {

@@ -64,6 +64,24 @@ def test_unwrapped_coordinates_small_cell(oracle, dt):
     assert a[5].dtype == np.int32
 
 
+# 27, 27, 15, 45 and 75 images of an atom: told axis by axis, one by one, and, beyond 32 of them, in the order of the images;
+# atoms outside the cell; a thread for an x-layer of an atom's images and (66,000 atoms) for all of them
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("box,pbc,n", [
+    ([[40.0, 0, 0], [0, 45.0, 0], [0, 0, 50.0]], (True, True, True), 4500),
+    ([[40.0, 2.0, -1.0], [3.0, 45.0, 1.0], [-2.0, 1.0, 50.0]], (True, True, True), 4500),
+    ([[60.0, 0, 0], [0, 4.0, 0], [0, 0, 400.0]], (True, True, False), 4500),
+    ([[60.0, 0, 0], [0, 400.0, 0], [0, 0, 4.0]], (True, True, True), 4500),
+    ([[4.0, 0, 0], [0, 4.0, 0], [0, 0, 6000.0]], (True, True, True), 4500),
+    ([[100.0, 5.0, 0], [0, 110.0, 4.0], [3.0, 0, 120.0]], (True, True, True), 66000)])
+def test_images_in_reach(oracle, dt, box, pbc, n):
+    L = np.array(box)
+    fr = synth.rng_uniform(27, 3 * n).reshape(n, 3) * 1.1 - 0.05
+    ty = synth.rng_randint(28, n, 2)
+    args = (L.astype(dt), ty, (fr @ L).astype(dt), 5.0, 320)
+    assert_same(gpu_list(*args, pbc=pbc), oracle.nblist(*args, pbc=pbc))
+
+
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("umax", [56, 54, 2000])
 def test_row_capacities(oracle, dt, umax):
