@@ -65,6 +65,7 @@ struct Grid {
     int diagonal;     // b is diagonal: a coordinate of an image depends on the image's index along its own axis only
     unsigned inv_z, inv_yz;   // floor(m / img_dim[2]) = m * inv_z >> 16, of img_dim[1] * img_dim[2] likewise, for m < 32
     int N;
+    T in_below, out_from;     // rcut2 less and more 1e-6 of it: a squared length formed in T is in below the one, out from the other on
     int ext_bins;     // ceil(rcut / bin_size) = 2
     int is_cart;
     float inv_side;   // 1 / (2 ext_bins + 1), 1 / bin_size: for the pruning arithmetic of the
@@ -1095,7 +1096,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     static_assert(!COMPACT || (ROWBUF && !SORT && !RANK), "compact lists are cut from the row held in LDS");
     static_assert(!(SORT && RANK), "places belong to unsorted rows");
     const Grid<T> g = with_dyn(g_in, gd);
-    __shared__ int sh_start[NBL_BLOCK / 64][64];
+    __shared__ int sh_shift[NBL_BLOCK / 64][64];                             // entry of a column's candidate - its place in the list
     __shared__ int sh_base[NBL_BLOCK / 64][64];
     __shared__ unsigned char sh_col[NBL_BLOCK / 64][NBL_APW][NBL_ENT_CAP];   // column of each flat candidate
     extern __shared__ __align__(16) unsigned char sh_rows[];
@@ -1116,6 +1117,12 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         rb_first = (int*)(mine + (size_t)umax * (SORT ? 4 : 3) * sizeof(T));
         rb_rank = rb_first + umax;
     }
+    // vector of entry e, by a 24-bit product (umax is far below 2^20 where a row fits the LDS; the 32-bit one takes four slots)
+    auto rb_vec = [&](int e) __attribute__((always_inline)) { return (T*)((unsigned char*)rb_rcs + __umul24(e, 3 * sizeof(T))); };
+    // lanes of the mask below this one
+    auto place_in = [&](unsigned long long m) __attribute__((always_inline)) {
+        return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+    };
     // A row costs three dependent trips to memory (coordinates, column runs, candidates).  The
     // wavefront takes NBL_APW atoms: all their coordinates are loaded first, and the column runs of
     // the next atom are requested before the candidates of the current one are scanned.
@@ -1135,7 +1142,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             cs[a][d] = COMPACT ? ce.xs[(size_t)min(p0 + a, g.N - 1) * 3 + d] : x[(size_t)atom[a] * 3 + d];
     const int nruns = (2 * g.ext_bins + 1) * (2 * g.ext_bins + 1);
     // With at most 32 columns per atom the wave's two atoms are set up side by side, lanes 0-31 and 32-63 (their
-    // halves of sh_start / sh_base, their own flat list); with more, one after the other through the first
+    // halves of sh_shift / sh_base, their own flat list); with more, one after the other through the first
     // flat list, the column runs of the second requested before the candidates of the first are scanned.
     static_assert(NBL_APW == 2, "two atoms per wavefront");
     const bool paired = nruns <= 32;              // wave-uniform
@@ -1147,10 +1154,10 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         column_setup<T>(g, csel, lane & 31, offsets, start, len);
         if (sub >= np) len = 0;
         const int incl = wave_inclusive_scan(len);
-        totals[0] = __shfl(incl, 31, 64);
-        totals[1] = __shfl(incl, 63, 64) - totals[0];
+        totals[0] = __builtin_amdgcn_readlane(incl, 31);
+        totals[1] = __builtin_amdgcn_readlane(incl, 63) - totals[0];
         const int base = incl - len - (sub ? totals[0] : 0);
-        sh_start[wv][lane] = start;
+        sh_shift[wv][lane] = start - base;
         sh_base[wv][lane] = base;
         if ((sub ? totals[1] : totals[0]) <= NBL_ENT_CAP)
             for (int k = 0; k < len; k++) sh_col[wv][sub][base + k] = (unsigned char)(lane & 31);
@@ -1170,9 +1177,9 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     if (!paired) {
         if (ia + 1 < NBL_APW && ia + 1 < np) column_setup<T>(g, cs[ia + 1 < NBL_APW ? ia + 1 : ia], lane, offsets, nstart, nlen);
         const int incl = wave_inclusive_scan(len);
-        totals[ia] = __shfl(incl, 63, 64);
+        totals[ia] = __builtin_amdgcn_readlane(incl, 63);
         const int base = incl - len;
-        sh_start[wv][lane] = start;
+        sh_shift[wv][lane] = start - base;
         sh_base[wv][lane] = base;
         if (totals[ia] <= NBL_ENT_CAP)
             for (int k = 0; k < len; k++) sh_col[wv][0][base + k] = (unsigned char)lane;
@@ -1180,7 +1187,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     }
     const int total = totals[ia];
     const bool flat = total <= NBL_ENT_CAP;       // wave-uniform
-    const int so = paired ? ia * 32 : 0;          // the atom's part of sh_start / sh_base
+    const int so = paired ? ia * 32 : 0;          // the atom's part of sh_shift / sh_base
     const unsigned char* const cols = sh_col[wv][paired ? ia : 0];
 
     int cnt = 0;
@@ -1193,28 +1200,39 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     for (int c0 = 0; c0 < total; c0 += 64 * NBL_UNROLL) {
         int sj[NBL_UNROLL];
         T px[NBL_UNROLL], py[NBL_UNROLL], pz[NBL_UNROLL];
+        // No branch around the load: a lane past the end of the list reads the last candidate again and drops it
+        // below, and the loads of the trip's chunks stay back to back.  Sorted rows, whose kernel waits for its stores,
+        // leave out the chunks beyond the list (wave-uniform) from the third on: 131,072 atoms 167 -> 162 us in fp64,
+        // 121 -> 119 in fp32; compact ones gain nothing (whole step at 1,048,576 atoms 1635 us with and without).
+        // The list's length and the choice between the two searches are scalar, and the chunks' columns are read
+        // together: two waits for the LDS instead of two per chunk (with the rest of this loop: sorted list of 131,072
+        // atoms in fp64 236 -> 225 us a call, the step at 1,048,576 in fp32 1679 -> 1635).
+        auto beyond = [&](int u) __attribute__((always_inline)) { return SORT && u >= 2 && c0 + u * 64 >= total; };
+        int ent[NBL_UNROLL];
+        if (flat) {
+            int col[NBL_UNROLL];
 #pragma unroll
-        for (int u = 0; u < NBL_UNROLL; u++) {
-            // no branch around the load: a lane past the end of the list reads the last candidate again and
-            // drops it below, and the loads of the trip's chunks stay back to back.  Sorted rows, whose kernel waits for
-            // its stores, leave out the chunks beyond the list (wave-uniform) from the third on: 131,072 atoms 167 -> 162
-            // us in fp64, 121 -> 119 in fp32; unsorted and compact ones lose by it (611 -> 625 at 1,048,576).
-            if (SORT && u >= 2 && c0 + u * 64 >= total) break;         // (nor are they looked at below)
-            const int ci = min(c0 + u * 64 + lane, total - 1);
-            int ent;
-            if (flat) {
-                const int col = so + cols[ci];
-                ent = sh_start[wv][col] + (ci - sh_base[wv][col]);
-            } else {
+            for (int u = 0; u < NBL_UNROLL; u++) col[u] = cols[min(c0 + u * 64 + lane, total - 1)];
+#pragma unroll
+            for (int u = 0; u < NBL_UNROLL; u++) ent[u] = sh_shift[wv][so + col[u]] + min(c0 + u * 64 + lane, total - 1);
+        } else {
+#pragma unroll
+            for (int u = 0; u < NBL_UNROLL; u++) {
+                if (beyond(u)) break;
+                const int ci = min(c0 + u * 64 + lane, total - 1);
                 // last column whose base is <= ci
                 int lo = 0, hi = nruns - 1;
                 while (lo < hi) {
                     const int mid = (lo + hi + 1) >> 1;
                     if (sh_base[wv][so + mid] <= ci) lo = mid; else hi = mid - 1;
                 }
-                ent = sh_start[wv][so + lo] + (ci - sh_base[wv][so + lo]);
+                ent[u] = sh_shift[wv][so + lo] + ci;
             }
-            entry_load(s_rec + (size_t)ent * 4, px[u], py[u], pz[u], sj[u]);
+        }
+#pragma unroll
+        for (int u = 0; u < NBL_UNROLL; u++) {
+            if (beyond(u)) break;                                      // (nor are they looked at below)
+            entry_load(s_rec + (size_t)(unsigned)ent[u] * 4, px[u], py[u], pz[u], sj[u]);
         }
         // RANK: the pair's place among the pairs that name the same neighbour, claimed here so that
         // the force kernels need no atomics; the answers are collected after the chunk's last claim
@@ -1226,18 +1244,40 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             if (c0 + u * 64 >= total) break;                           // wave-uniform
             const bool have = c0 + u * 64 + lane < total;
             const T dx = sub_rn(px[u], c[0]), dy = sub_rn(py[u], c[1]), dz = sub_rn(pz[u], c[2]);
-            const double d2d = dist2_double(dx, dy, dz);
-            const T d2 = (T)d2d;                                       // `CoordType relative_distance2`
-            const bool in = have && ((double)d2 < g.rcut2) && ((double)d2 > kEpsilon);   // binLinkedList.h:1014-1017
-            const unsigned long long mask = __ballot(in);
-            const int rank = __popcll(mask & ((1ull << lane) - 1ull));
-            const int slot = cnt + rank;
+            // binLinkedList.h:1014-1017: the double-precision length, rounded to T, against the double-precision bounds.
+            // In fp32 the length in T decides unless it lies within 1e-6 of a bound (its error and the rounding of
+            // the other stay below 3e-7 together), and only a chunk with such a candidate forms the other: seven vector
+            // instructions instead of twelve, a third of which take more than one issue slot.
+            double d2d = 0.0;
+            bool in;
+            unsigned long long mask;
+            auto exact = [&]() __attribute__((always_inline)) {
+                d2d = dist2_double(dx, dy, dz);
+                const T d2 = (T)d2d;                                   // `CoordType relative_distance2`
+                in = have & ((double)d2 < g.rcut2) & ((double)d2 > kEpsilon);
+                mask = __builtin_amdgcn_ballot_w64(in);
+            };
+            if constexpr (sizeof(T) == 4 && !SORT) {
+                const T d2 = fma(dx, dx, fma(dy, dy, dz * dz));
+                const bool near = d2 < g.in_below, apart = d2 > (T)(kEpsilon * (1.0 + 1e-6));
+                in = have & near & apart;
+                // masks joined in scalar registers: a mask of a joint condition takes two vector instructions more
+                const unsigned long long row = __builtin_amdgcn_ballot_w64(have);
+                mask = row & __builtin_amdgcn_ballot_w64(near) & __builtin_amdgcn_ballot_w64(apart);
+                const unsigned long long maybe = row & __builtin_amdgcn_ballot_w64(d2 < g.out_from) &
+                                                 __builtin_amdgcn_ballot_w64(d2 > (T)(kEpsilon * (1.0 - 1e-6)));
+                if (mask != maybe) exact();                            // wave-uniform
+            } else {
+                exact();
+            }
+            const int slot = cnt + place_in(mask);
             if (in && slot < umax) {
                 if (ROWBUF) {
                     rb_first[slot] = sj[u];
-                    rb_rcs[slot * 3 + 0] = dx;
-                    rb_rcs[slot * 3 + 1] = dy;
-                    rb_rcs[slot * 3 + 2] = dz;
+                    T* const v = rb_vec(slot);
+                    v[0] = dx;
+                    v[1] = dy;
+                    v[2] = dz;
                 } else {
                     firstneigh[rowi + slot] = sj[u];                   // neighborList.h:561 (already mod natoms)
                     rcs[(rowi + slot) * 3 + 0] = dx;
@@ -1284,7 +1324,8 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             const int e = e0 + lane;
             const bool have = e < used;
             const int ee = have ? e : 0;
-            const T dx = rb_rcs[ee * 3 + 0], dy = rb_rcs[ee * 3 + 1], dz = rb_rcs[ee * 3 + 2];
+            const T* const vec = rb_vec(ee);
+            const T dx = vec[0], dy = vec[1], dz = vec[2];
             const int word = rb_first[ee];
             // The entry names its neighbour by position in the processing order (what the force kernels index their
             // per-atom arrays with), the record and the padded row by atom: one gather per entry.  The first 64
@@ -1293,8 +1334,8 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             // compact_symmetry_kernel reports; the consumers of the entries check the index they find.
             const int bits = ce.inv[word & (CL_IMAGE_BIT - 1)] | (word & ~CL_INDEX_MASK);
             const T d2 = dx * dx + dy * dy + dz * dz;
-            const bool in_outer = have && d2 <= ce.outer2;
-            const bool is_inner = in_outer && d2 <= ce.split2;
+            const bool in_outer = have & (d2 <= ce.outer2);
+            const bool is_inner = in_outer & (d2 <= ce.split2);
             // Both entries of a pair must fall on the same side of the inner cutoff (the force kernels treat the
             // two classes by different routes), but the two ends see vectors that differ by the rounding of their
             // images (a pair of atoms in the cell itself has exactly opposite vectors).  A position with an image
@@ -1303,11 +1344,11 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             // bit-identically; outside the band the two ends agree anyway.
             nearest = fmin(nearest, (in_outer && (word & CL_IMAGE_BIT)) ? fabs(d2 - ce.split2) : nearest);
             const bool is_outer = in_outer && !is_inner;
-            const unsigned long long mi = __ballot(is_inner), mo = __ballot(is_outer);
-            const unsigned long long below = (1ull << lane) - 1ull;
+            const unsigned long long m = __builtin_amdgcn_ballot_w64(have) & __builtin_amdgcn_ballot_w64(d2 <= ce.outer2);
+            const unsigned long long mi = m & __builtin_amdgcn_ballot_w64(d2 <= ce.split2), mo = m & ~mi;
             int slot = -1;
-            if (is_inner) slot = umax - 1 - (n_inner + __popcll(mi & below));
-            if (is_outer) slot = n_outer + __popcll(mo & below);
+            if (is_inner) slot = umax - 1 - (n_inner + place_in(mi));
+            if (is_outer) slot = n_outer + place_in(mo);
             if (e0 == 0) {                        // wave-uniform
                 first_dx = dx; first_dy = dy; first_dz = dz; first_bits = bits; first_slot = slot;
             } else if (slot >= 0) {
@@ -1316,7 +1357,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             n_inner += __popcll(mi);
             n_outer += __popcll(mo);
         }
-        const bool any_near = __ballot(nearest <= near_band) != 0ull;
+        const bool any_near = __builtin_amdgcn_ballot_w64(nearest <= near_band) != 0ull;
         if (lane == 0) {
             ce.n_outer[pos] = n_outer;
             ce.n_inner[pos] = n_inner | (any_near ? CL_NEAR_FLAG : 0);         // the flag: for compact_symmetry_kernel
@@ -1356,7 +1397,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             place[u] = less;
             tie |= have && same != 1;
         }
-        const bool tied_row = __ballot(tie) != 0ull;
+        const bool tied_row = __builtin_amdgcn_ballot_w64(tie) != 0ull;
         if (lane == 0) tied[p] = tied_row ? 1 : 0;
         if (!tied_row) {
             int ef[NBL_SORT_CAP / 64];
@@ -1830,6 +1871,8 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     g.is_cart = is_cart;
     g.rcut = (T)rcut_in;
     g.rcut2 = (double)g.rcut * (double)g.rcut;
+    g.in_below = (T)(g.rcut2 * (1.0 - 1e-6));
+    g.out_from = (T)(g.rcut2 * (1.0 + 1e-6));
     g.bin_size = g.rcut / 2;                                   // binLinkedList.h:664
     for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) g.b[i][j] = lattice[i * 3 + j];

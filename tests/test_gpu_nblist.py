@@ -83,6 +83,20 @@ def test_images_in_reach(oracle, dt, box, pbc, n):
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("n,umax", [(150, 152), (150, 154), (400, 404), (400, 402)])
+def test_distances_at_the_bounds(oracle, dt, n, umax):
+    """Neighbours within a few units of the last place of the cutoff, and of the length below which a pair is left out."""
+    u = synth.rng_uniform(41, 2 * n).reshape(n, 2)
+    z, phi = 2.0 * u[:, 0] - 1.0, 2.0 * np.pi * u[:, 1]
+    s = np.sqrt(1.0 - z * z)
+    d = np.stack([s * np.cos(phi), s * np.sin(phi), z], 1)
+    r = np.where(np.arange(n) % 5 == 0, np.sqrt(1e-3), 5.0) * (1.0 + (np.arange(n) % 33 - 16) * 2.0 ** -23)
+    pos = np.concatenate([[[13.0, 13.0, 13.0]], 13.0 + d * r[:, None]]).astype(dt)
+    args = ((26.0 * np.eye(3)).astype(dt), np.zeros(n + 1, dtype=np.int32), pos, 5.0, umax)
+    assert_same(gpu_list(*args), oracle.nblist(*args))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("umax", [56, 54, 2000])
 def test_row_capacities(oracle, dt, umax):
     """Capacities that take the LDS row buffer (multiple of 4, small), the direct stores (not a
