@@ -977,13 +977,28 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
                                              const int* __restrict__ offsets, int& start, int& len)
 {
     int cb[3];
+    bool sure = false;
+    if constexpr (sizeof(T) == 4) {
+        // The bins by the reciprocal, unless a quotient lies within 1e-3 of a whole number (its error is below
+        // 2e-7 of itself): a third of the instructions of three divisions.
+        T off = (T)0;                              // the farthest of the quotients' fractions from a half
 #pragma unroll
-    for (int a = 0; a < 3; a++) cb[a] = bin_of(c[a], g.mn[a], g.bin_size);
+        for (int a = 0; a < 3; a++) {
+            const T q = sub_rn(c[a], g.mn[a]) * g.inv_bin, f = floorf(q);
+            cb[a] = (int)f;
+            off = fmaxf(off, fabsf((q - f) - (T)0.5));
+        }
+        sure = max(max(g.nbin[0], g.nbin[1]), g.nbin[2]) < 4096 && __builtin_amdgcn_ballot_w64(!(off < (T)0.499)) == 0ull;   // wave-uniform
+    }
+    if (!sure) {
+#pragma unroll
+        for (int a = 0; a < 3; a++) cb[a] = bin_of(c[a], g.mn[a], g.bin_size);
+    }
     const int e = g.ext_bins, side = 2 * e + 1, nruns = side * side;
     start = 0; len = 0;
     if (lane < nruns) {
         const int lq = (int)(((float)lane + 0.5f) * g.inv_side);     // lane / side for small integers
-        const int bx = cb[0] + lq - e, by = cb[1] + (lane - lq * side) - e;
+        const int bx = cb[0] + lq - e, by = cb[1] + (lane - (int)__umul24(lq, side)) - e;
         int zlo = cb[2] - e, zhi = cb[2] + e;
         // bins outside the reference's grid are skipped (binLinkedList.h:952-968); inside it the
         // box kept here covers every bin within `e` of a centre atom
@@ -998,22 +1013,25 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
             const float bs = (float)g.bin_size, inv_bs = g.inv_bin, rc2 = (float)g.rcut2 * 1.00001f;
             float lat2 = 0.0f;
             const int bxy[2] = {bx, by};
+            // a thousandth of a bin and 1e-5 of the coordinates (rel, the atom's own and the origin: the atom's own is no
+            // longer than the other two together)
+            auto tolerance = [&](int a, float rel) __attribute__((always_inline)) {
+                return fmaf(2.0e-5f, fabsf(rel), fmaf(2.0e-5f, fabsf((float)g.mn[a]), 1.0e-3f * bs));
+            };
 #pragma unroll
             for (int a = 0; a < 2; a++) {
                 const float rel = (float)c[a] - (float)g.mn[a];
-                const float tol = 1.0e-3f * bs + 1.0e-5f * (fabsf(rel) + fabsf((float)c[a]) + fabsf((float)g.mn[a]));
-                const float lo = (float)bxy[a] * bs;
-                const float d = fmaxf(fmaxf(lo - rel, rel - (lo + bs)) - tol, 0.0f);
-                lat2 += d * d;
+                const float t = fmaf((float)bxy[a], bs, 0.5f * bs - rel);       // the column's middle from the atom
+                const float d = fmaxf(fabsf(t) - (0.5f * bs + tolerance(a, rel)), 0.0f);
+                lat2 = fmaf(d, d, lat2);
             }
             if (lat2 > rc2) ok = false;
             else {
                 const float rel = (float)c[2] - (float)g.mn[2];
-                const float tol = 1.0e-3f * bs + 1.0e-5f * (fabsf(rel) + fabsf((float)c[2]) + fabsf((float)g.mn[2]));
                 // the hardware square root is within an ulp; the tolerance is five orders above that
-                const float reach = __builtin_amdgcn_sqrtf(rc2 - lat2) + tol;
-                zlo = max(zlo, (int)floorf((rel - reach) * inv_bs - 1.0e-3f));
-                zhi = min(zhi, (int)floorf((rel + reach) * inv_bs + 1.0e-3f));
+                const float reach = __builtin_amdgcn_sqrtf(rc2 - lat2) + tolerance(2, rel);
+                zlo = max(zlo, (int)floorf(fmaf(rel - reach, inv_bs, -1.0e-3f)));
+                zhi = min(zhi, (int)floorf(fmaf(rel + reach, inv_bs, 1.0e-3f)));
             }
         }
         if (ok && zlo <= zhi) {
@@ -1025,6 +1043,29 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
 }
 
 constexpr int NBL_APW = 2;         // consecutive centre atoms per wavefront
+
+// cols[base .. base + len) = the lane's column, for the runs of all lanes at once, which lie back to back.  Every lane with a run
+// writes the first NBL_RUN places from its base on, the last one first, whether they are its own or not: a place belongs to the
+// lane with the nearest base before it, whose write comes last.  No comparison per place (a loop over each lane's own run took
+// four vector instructions per step); `cols` has NBL_RUN bytes behind its last place.  With the bins by the reciprocal and the
+// columns' distances in fused operations a wavefront of the compact kernel issues 503 vector instructions instead of 565:
+// 574 -> 566 us at 1,048,576 atoms (the LDS is busy for 0.72 of it, HBM at 3.7 TB/s).
+constexpr int NBL_RUN = 16;
+__device__ __forceinline__ void run_columns(unsigned char* cols, int base, int len, int col)
+{
+    // (volatile: the writes stay single and in this order)
+    typedef volatile __attribute__((address_space(3))) unsigned char lds_byte;
+    lds_byte* const at = (lds_byte*)(cols + base);
+    if (__builtin_amdgcn_ballot_w64(len > NBL_RUN) != 0ull)                    // wave-uniform
+        for (int k = NBL_RUN; k < len; k++) at[k] = (unsigned char)col;
+#pragma unroll
+    for (int k0 = NBL_RUN - 4; k0 >= 0; k0 -= 4)
+        if (k0 == 0 || __builtin_amdgcn_ballot_w64(len > k0) != 0ull)          // wave-uniform
+            if (len > 0) {
+#pragma unroll
+                for (int k = k0 + 3; k >= k0; k--) at[k] = (unsigned char)col;
+            }
+}
 
 // Compact lists (compact_list.h) written next to, or instead of, the padded rows.  The wavefront
 // that holds a finished row in LDS sorts its entries into the two ends of the position's slots:
@@ -1098,7 +1139,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     const Grid<T> g = with_dyn(g_in, gd);
     __shared__ int sh_shift[NBL_BLOCK / 64][64];                             // entry of a column's candidate - its place in the list
     __shared__ int sh_base[NBL_BLOCK / 64][64];
-    __shared__ unsigned char sh_col[NBL_BLOCK / 64][NBL_APW][NBL_ENT_CAP];   // column of each flat candidate
+    __shared__ unsigned char sh_col[NBL_BLOCK / 64][NBL_APW][NBL_ENT_CAP + NBL_RUN];   // column of each flat candidate
     extern __shared__ __align__(16) unsigned char sh_rows[];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // the wave's first position, in a scalar register: the loads of its atoms' indices and coordinates are then
@@ -1159,8 +1200,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         const int base = incl - len - (sub ? totals[0] : 0);
         sh_shift[wv][lane] = start - base;
         sh_base[wv][lane] = base;
-        if ((sub ? totals[1] : totals[0]) <= NBL_ENT_CAP)
-            for (int k = 0; k < len; k++) sh_col[wv][sub][base + k] = (unsigned char)(lane & 31);
+        run_columns(sh_col[wv][sub], base, (sub ? totals[1] : totals[0]) <= NBL_ENT_CAP ? len : 0, lane & 31);
         __builtin_amdgcn_wave_barrier();
     } else {
         column_setup<T>(g, cs[0], lane, offsets, start, len);
@@ -1181,8 +1221,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         const int base = incl - len;
         sh_shift[wv][lane] = start - base;
         sh_base[wv][lane] = base;
-        if (totals[ia] <= NBL_ENT_CAP)
-            for (int k = 0; k < len; k++) sh_col[wv][0][base + k] = (unsigned char)lane;
+        if (totals[ia] <= NBL_ENT_CAP) run_columns(sh_col[wv][0], base, len, lane);
         __builtin_amdgcn_wave_barrier();
     }
     const int total = totals[ia];
@@ -1372,7 +1411,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         // keys per 16-byte read in fp32), and the entries go from registers to their places.  A row with equal
         // distances keeps the order it was found in and is flagged for sort_tied_rows_kernel, which repeats the
         // reference's own sequence of moves.  Bound by the padded rows written: 131072 atoms, 36 neighbours, fp64,
-        // umax 200 take 0.156 ms (4.7 TB/s); rows through global memory, a sort by a thread per row and a gather took
+        // umax 200 take 0.145 ms (5.1 TB/s); rows through global memory, a sort by a thread per row and a gather took
         // 0.176 + 0.898 + 0.241 ms.
         __builtin_amdgcn_wave_barrier();
         const int used = min(cnt, umax);          // wave-uniform, at most NBL_SORT_CAP

@@ -97,6 +97,18 @@ def test_distances_at_the_bounds(oracle, dt, n, umax):
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("sort", [False, True])
+def test_atoms_on_the_faces_of_bins(oracle, dt, sort):
+    """Atoms within a few units of the last place of the faces of their bins (half a cutoff wide, from half a unit below the
+    lowest image on)."""
+    k = np.stack(np.meshgrid(*[np.arange(10.0)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    ulps = np.floor(synth.rng_uniform(43, k.size).reshape(k.shape) * 9.0) - 4.0
+    pos = np.concatenate([[[0.0, 0.0, 0.0]], (2.5 * k + 2.0) * (1.0 + ulps * 2.0 ** -23)]).astype(dt)
+    args = ((25.0 * np.eye(3)).astype(dt), np.zeros(len(pos), dtype=np.int32), pos, 5.0, 80)
+    assert_same(gpu_list(*args, sort=sort), oracle.nblist(*args, sort=sort))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("umax", [56, 54, 2000])
 def test_row_capacities(oracle, dt, umax):
     """Capacities that take the LDS row buffer (multiple of 4, small), the direct stores (not a
