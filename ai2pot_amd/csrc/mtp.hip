@@ -1045,9 +1045,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                     if (n0 + k0 > 0) row_weights(n0 + hl, k0 + hp, ph);
 #pragma unroll
                     for (int u = 0; u < W; u++) {
-                        const int k = min(k0 + hp + u * ph, S - 1);
-                        acc += w[u] * qv[k];
-                        if (LOSS) tac += w[u] * qt[k];
+                        const int k = k0 + hp + u * ph, own = min(k, S - 1);
+                        const T q = qv[own], t = LOSS ? qt[own] : (T)0;
+                        acc += w[u] * (k < S ? q : (T)0);                   // (an input may be infinite)
+                        if (LOSS) tac += w[u] * (k < S ? t : (T)0);
                     }
                 }
                 acc = parts_sum(acc, lh);
@@ -1081,9 +1082,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                     if (i0 + n0 > 0) column_weights(k, n0 + sp, ps);
 #pragma unroll
                     for (int u = 0; u < W; u++) {
-                        const int n = min(n0 + sp + u * ps, H - 1);
-                        acc += hv[n] * w[u];
-                        if (LOSS) bac += n_c2[n] * w[u];
+                        const int n = n0 + sp + u * ps, own = min(n, H - 1);
+                        const T h = hv[own], c = LOSS ? n_c2[own] : (T)0;
+                        acc += w[u] * (n < H ? h : (T)0);
+                        if (LOSS) bac += w[u] * (n < H ? c : (T)0);
                     }
                 }
                 acc = parts_sum(acc, ls);

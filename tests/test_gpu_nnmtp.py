@@ -161,6 +161,26 @@ def test_readout_by_neighbouring_lanes(oracle, level, H):
         assert close(got[k], ref[k]), k
 
 
+@pytest.mark.parametrize("level", [8, 12, 16, 20])
+@pytest.mark.parametrize("H", [3, 20, 65])
+def test_readout_of_an_infinite_input(oracle, level, H):
+    """An input that overflows (the last one: lanes with no input of their own must not count it) saturates every neuron at
+    plus or minus one: energies are sums of the second layer's weights and the forces vanish.  fp64 1e-13: H additions."""
+    m, nb, _ = loss_inputs(oracle, level, 2, H, sizes=(13, 9))
+    m["q_scaler"] = m["q_scaler"].copy()
+    m["q_scaler"][-1] = 5e-324
+    lin = dict(m); lin["scaling"] = 1.0; lin["linear_coeffs"] = np.zeros(m["q_scaler"].size)
+    last = oracle.mtp_esites(lin, nb)[1][..., -1] - m["q_shifter"][-1]
+    w0, w1 = np.reshape(m["w0"], (2, H, -1)), np.reshape(m["w1"], (2, H))
+    ref = np.zeros(last.shape)
+    for b, n in enumerate(nb["binum"]):
+        for ii in range(n):
+            t = nb["btypes"][b, nb["bilist"][b, ii]]
+            ref[b, ii] = m["type_bias"][t] + np.sum(w1[t] * np.sign(w0[t, :, -1] * last[b, ii]))
+    e, f, v, es, _ = run(m, nb)
+    assert close(es, ref, 1e-13) and close(e, ref.sum(1), 1e-13) and not f.any() and not v.any()
+
+
 @pytest.mark.parametrize("level,nt,H", [(8, 2, 7), (16, 3, 20)])
 def test_loss_step_reference_formulas(oracle, level, nt, H):
     """exact_gradient=False (the operators' default) against the committed output of the reference's
