@@ -1001,10 +1001,14 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             // A neuron's sum over the inputs, and an input's over the neurons, by 1, 2 .. 16 neighbouring lanes each, W weights
             // of a lane on their way together, the first of either sum ahead of what it waits for.  What bounds it is the trips to
             // the weights and the chain of their operations.  (A wavefront for four neurons at a time with sums over its 64 lanes,
-            // then a lane for an input: 10.8 of the 41 thousand cycles an atom takes at level 12 with 20 neurons, 9.3 of the 55 of the
-            // loss gradient; now 8.4 and 6.7.  Calls: 4000 atoms 47.3 -> 43.5 us, the training step of 40 structures of 100 atoms 156 ->
-            // 147; level 16, 30 neurons, 113 -> 108.6 and 232 -> 218.  Sixteen weights on their way: no faster; the next W behind
-            // them: level 16 108.7 -> 110.8.)
+            // then a lane for an input, against this, in us of the kernel: level 12, 20 neurons, 3000 atoms 37.6 and 33.6, 200 atoms
+            // 25.6 and 23.1, the loss gradient of 16 structures of 64 atoms 45.5 and 41.2; level 20, 60 neurons, 152 and 143, 37.6
+            // and 35.8, 221 and 198.)
+            // At least two lanes to a neuron from 9 inputs on, four from 24 on, eight in fp32 from 128 on, in as many rounds as that
+            // takes: fewer lanes read a few bytes of each of many rows at a time, whose lines are gone before they are used up
+            // (one lane, two, four, eight; 3000 atoms: level 8, 9 inputs, 60 neurons 27.5, 27.2, 28.5, 32.0 us; level 10, 16
+            // inputs, 100 neurons 42.8, 38.4, 39.2, 43.8; level 12, 29 inputs, 200 neurons 64.3, 56.0, 55.5, 64.6; level 20, 288
+            // inputs, 200 neurons 463, 319, 250, 256, in fp32 383, 376, 179, 157).
             const int S = p.n_scalar, H = a.H;
             T* qv = nnb;                          // [S] network inputs
             T* hv = nnb + S;                      // [H] pre-activations, then w1 * tanh'
@@ -1019,18 +1023,39 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             const T* w1 = a.w1 + (size_t)ti * H;
             constexpr int W = LOSS ? 4 : 8;       // (eight: 8 more values spilled by the loss gradient)
             T w[W];
-            // weights of neuron n and the inputs k0, k0 + step ..; and of input k and the neurons from n0 on
-            auto row_weights = [&](int n, int k0, int step) __attribute__((always_inline)) {
-#pragma unroll
-                for (int u = 0; u < W; u++) w[u] = k0 + u * step < S ? w0[(size_t)min(n, H - 1) * S + k0 + u * step] : (T)0;
-            };
-            auto column_weights = [&](int k, int n0, int step) __attribute__((always_inline)) {
-#pragma unroll
-                for (int u = 0; u < W; u++) w[u] = n0 + u * step < H ? w0[(size_t)(n0 + u * step) * S + min(k, S - 1)] : (T)0;
-            };
-            const int lh = parts_log2(NT, H), ph = 1 << lh, ls = parts_log2(NT, S), ps = 1 << ls;
+            const int lh = max(parts_log2(NT, H), S <= 8 ? 0 : S < 24 ? 1 : sizeof(T) == 4 && S >= 128 ? 3 : 2), ph = 1 << lh, ls = parts_log2(NT, S), ps = 1 << ls;
             const int hl = lane >> lh, hp = lane & (ph - 1), sl = lane >> ls, sp = lane & (ps - 1);
-            row_weights(hl, hp, ph);
+            // the wavefront's first neuron and input of a round
+            const int hw = __builtin_amdgcn_readfirstlane(lane) >> lh, sw = __builtin_amdgcn_readfirstlane(lane) >> ls;
+            // weights of neuron n and the inputs k0, k0 + ph ..; and of input k and the neurons n0, n0 + ps ..
+            auto row_weights = [&](int n, int k0) __attribute__((always_inline)) {
+                const unsigned at = __umul24(min(n, H - 1), S);
+#pragma unroll
+                for (int u = 0; u < W; u++) w[u] = w0[at + min(k0 + u * ph, S - 1)];
+            };
+            auto column_weights = [&](int k, int n0) __attribute__((always_inline)) {
+                const unsigned at = min(k, S - 1);
+#pragma unroll
+                for (int u = 0; u < W; u++) w[u] = w0[__umul24(min(n0 + u * ps, H - 1), S) + at];
+            };
+            // W of the products of a sum: acc += w q[first + u step], below `end` (others may be infinite), and tac += w t[..]
+            auto products = [&](T& acc, T& tac, const T* q, const T* t, int first, int step, int end, bool whole) __attribute__((always_inline)) {
+                if (whole)                                     // wave-uniform
+#pragma unroll
+                    for (int u = 0; u < W; u++) {
+                        acc += w[u] * q[first + u * step];
+                        if (LOSS) tac += w[u] * t[first + u * step];
+                    }
+                else
+#pragma unroll
+                    for (int u = 0; u < W; u++) {
+                        const int i = first + u * step, own = min(i, end - 1);
+                        const T v = w[u] * q[own], d = LOSS ? w[u] * t[own] : (T)0;
+                        acc += i < end ? v : (T)0;
+                        if (LOSS) tac += i < end ? d : (T)0;
+                    }
+            };
+            row_weights(hl, hp);
             const T w1_own = w1[min(lane, H - 1)];
             for (int s = lane; s < S; s += NT) {
                 const int m = p.mapping[s];
@@ -1039,17 +1064,11 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                 if (LOSS) qt[s] = Tg[m] / scaler;
             }
             __syncthreads();
-            for (int n0 = 0; n0 < H; n0 += NT >> lh) {
+            for (int n0 = 0; n0 + hw < H; n0 += NT >> lh) {
                 T acc = (T)0, tac = (T)0;
                 for (int k0 = 0; k0 < S; k0 += W * ph) {
-                    if (n0 + k0 > 0) row_weights(n0 + hl, k0 + hp, ph);
-#pragma unroll
-                    for (int u = 0; u < W; u++) {
-                        const int k = k0 + hp + u * ph, own = min(k, S - 1);
-                        const T q = qv[own], t = LOSS ? qt[own] : (T)0;
-                        acc += w[u] * (k < S ? q : (T)0);                   // (an input may be infinite)
-                        if (LOSS) tac += w[u] * (k < S ? t : (T)0);
-                    }
+                    if (n0 + k0 > 0) row_weights(n0 + hl, k0 + hp);
+                    products(acc, tac, qv, qt, k0 + hp, ph, S, k0 + W * ph <= S);
                 }
                 acc = parts_sum(acc, lh);
                 if (LOSS) tac = parts_sum(tac, lh);
@@ -1058,7 +1077,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                     if (LOSS) n_tau[n0 + hl] = tac;
                 }
             }
-            column_weights(sl, sp, ps);
+            column_weights(sl, sp);
             const int m_own = p.mapping[min(sl, S - 1)];
             const T scaler_own = a.q_scaler[min(sl, S - 1)];
             __syncthreads();
@@ -1075,18 +1094,12 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             if (LOSS && qt == Bm)
                 for (int s = lane; s < S; s += NT) qt[s] = (T)0;
             __syncthreads();
-            for (int i0 = 0; i0 < S; i0 += NT >> ls) {
+            for (int i0 = 0; i0 + sw < S; i0 += NT >> ls) {
                 const int k = i0 + sl;
                 T acc = (T)0, bac = (T)0;
                 for (int n0 = 0; n0 < H; n0 += W * ps) {
-                    if (i0 + n0 > 0) column_weights(k, n0 + sp, ps);
-#pragma unroll
-                    for (int u = 0; u < W; u++) {
-                        const int n = n0 + sp + u * ps, own = min(n, H - 1);
-                        const T h = hv[own], c = LOSS ? n_c2[own] : (T)0;
-                        acc += w[u] * (n < H ? h : (T)0);
-                        if (LOSS) bac += w[u] * (n < H ? c : (T)0);
-                    }
+                    if (i0 + n0 > 0) column_weights(k, n0 + sp);
+                    products(acc, bac, hv, n_c2, n0 + sp, ps, H, n0 + W * ps <= H);
                 }
                 acc = parts_sum(acc, ls);
                 if (LOSS) bac = parts_sum(bac, ls);
@@ -1121,10 +1134,10 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         // the leaves' moments: their part of the energy, or, for the loss gradient, the moments (and tangents) themselves;
         // mixed adjoints: linearMtpLoss.h:417-434; the reference's network backward has none (Bm stays zero)
         if (LOSS && !no_tan && (!NET || a.nn_exact))
-            sweep_reverse<T, LOSS, true>(p.rev[NT / 256], M, A, Bm, (const T*)Tg, lane,
+            sweep_reverse<T, LOSS, !NET>(p.rev[NT / 256], M, A, Bm, (const T*)Tg, lane,
                 [&](int m, T v, T t) __attribute__((always_inline)) { M[m] = v; Tg[m] = t; });
         else
-            sweep_reverse<T, false, true>(p.rev[NT / 256], M, A, (T*)nullptr, (const T*)nullptr, lane,
+            sweep_reverse<T, false, !NET>(p.rev[NT / 256], M, A, (T*)nullptr, (const T*)nullptr, lane,
                 [&](int m, T v, T) __attribute__((always_inline)) {
                     if (LOSS) M[m] = v;
                     else e_part += A[m] * v;
@@ -1256,17 +1269,25 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                 const T* n_th = qv + S + H;
                 const T* n_d1 = n_th + H;
                 const T* n_tau = n_d1 + 2 * H;
-                const bool at_pq = mtp_tangents_at_pq(S, MTP_NC, nmus);
                 const T* w1 = a.w1 + (size_t)ti * H;
                 const T* w0 = a.w0 + (size_t)ti * H * S;
-                for (int q = lane; q < H * S; q += NT) {
-                    const int n = q / S, k = q - n * S;
-                    const T tk = at_pq ? L.pq[k] : Tg[p.mapping[k]] / a.q_scaler[k], d2 = (T)-2 * n_th[n] * n_d1[n];
+                auto weight_gradient = [&](int q, int n, int k, T tk) __attribute__((always_inline)) {
+                    const T d2 = (T)-2 * n_th[n] * n_d1[n];
                     if (a.nn_exact)
                         grow[nblk + q] = w1[n] * ((cE * n_d1[n] + d2 * n_tau[n]) * qv[k] + n_d1[n] * tk);
                     else        // nnMtpLoss.h:560-585: only the k' = k term of tau
                         grow[nblk + q] = w1[n] * (cE * n_d1[n] * qv[k] + tk * (n_d1[n] + d2 * w0[q] * qv[k]));
-                }
+                };
+                if (mtp_tangents_at_pq(S, MTP_NC, nmus))
+                    for (int q = lane; q < H * S; q += NT) {
+                        const int n = q / S, k = q - n * S;
+                        weight_gradient(q, n, k, L.pq[k]);
+                    }
+                else        // (many inputs: a thread forms its input's tangent once; an entry at a time, level 22, 20 neurons: 328 -> 296 us)
+                    for (int k = lane; k < S; k += NT) {
+                        const T tk = Tg[p.mapping[k]] / a.q_scaler[k];
+                        for (int n = 0; n < H; n++) weight_gradient(n * S + k, n, k, tk);
+                    }
                 for (int n = lane; n < H; n += NT) grow[nblk + H * S + n] = cE * n_th[n] + n_d1[n] * n_tau[n];
                 if (lane == 0) grow[nblk + H * S + H] = cE;
             } else if (!seeded) {

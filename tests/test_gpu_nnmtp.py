@@ -161,6 +161,52 @@ def test_readout_by_neighbouring_lanes(oracle, level, H):
         assert close(got[k], ref[k]), k
 
 
+@pytest.mark.parametrize("level", [14, 18, 20])            # 52, 163 and 288 inputs: 64 threads, 256, and more inputs than those
+@pytest.mark.parametrize("H", [1, 15, 16, 17, 64, 65, 200])
+def test_readout_in_rounds(oracle, level, H):
+    """Neurons in more rounds than one, with wavefronts that have none in the last, and a second round of inputs, in both precisions:
+    energies, forces and virials against the oracle, fp64 1e-10, fp32 1e-4 and 1e-3 as above."""
+    m, nb, _ = loss_inputs(oracle, level, 2, H, sizes=(13, 9))
+    er, fr, vr, esr = oracle.nnmtp_efv(m, nb)
+    for dt, te, tf in ((np.float64, 1e-10, 1e-10), (np.float32, 1e-4, 1e-3)):
+        e, f, v, es, _ = run(m, nb, dt)
+        assert close(e, er, te) and close(es, esr, te) and close(f, fr, tf) and close(v, vr, tf)
+
+
+def many_inputs(oracle, S, H):
+    """A table of one radial function whose first S basic moments are the scalar ones: more than 96 inputs leave no room for the
+    tangents of the inputs where they wait otherwise."""
+    basic = [(0, a, b, c) for a in range(9) for b in range(9 - a) for c in range(9 - a - b)]
+    tables = dict(alpha_moments_count=len(basic), alpha_index_basic=np.array(basic, np.int32),
+                  alpha_index_times=np.zeros((0, 4), np.int32), alpha_moment_mapping=np.arange(S, dtype=np.int32), nmus=1)
+    _, nb, labels = loss_inputs(oracle, 8, 2, H, sizes=(11, 7))
+    return synth.nnmtp_model(tables, 2, 6, H, 5.0, 1.5, 3400), nb, labels
+
+
+@pytest.mark.parametrize("S", [96, 97, 130])
+@pytest.mark.parametrize("H", [1, 5])
+def test_loss_step_of_many_inputs(oracle, S, H):
+    """The complete derivative against the oracle, fp64 1e-10; and, with both formulas, the gradient with and without inputs
+    whose weights are zero."""
+    m, nb, labels = many_inputs(oracle, S, H)
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w, True), oracle.nnmtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dw0", "dw1", "dbias"):
+        assert close(got[k], ref[k]), k
+    few = many_inputs(oracle, 90, H)[0]
+    w0 = np.zeros((2, H, S))
+    w0[:, :, :90] = np.reshape(few["w0"], (2, H, 90))
+    m = dict(m, coeffs=few["coeffs"], w0=w0.reshape(np.shape(m["w0"])), w1=few["w1"], type_bias=few["type_bias"])
+    for k in ("q_shifter", "q_scaler"):
+        m[k] = np.concatenate([few[k], m[k][90:]])
+    for exact in (False, True):
+        a, b = gpu_loss(m, nb, labels, w, exact), gpu_loss(few, nb, labels, w, exact)
+        B = len(nb["binum"])
+        assert close(a["dw0"].reshape(B, 2, H, S)[..., :90], b["dw0"].reshape(B, 2, H, 90), 1e-12)
+        for k in ("bloss", "dcoeffs", "dw1", "dbias"):
+            assert close(a[k], b[k], 1e-12), k
+
+
 @pytest.mark.parametrize("level", [8, 12, 16, 20])
 @pytest.mark.parametrize("H", [3, 20, 65])
 def test_readout_of_an_infinite_input(oracle, level, H):
