@@ -28,6 +28,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <set>
 #include <string>
@@ -2133,6 +2134,9 @@ void spread_over_banks(const std::vector<std::vector<int>>& lists, int depth, in
     }
 }
 
+// 256 threads per atom or 64 (the rule is at its definition)
+bool wide_atoms(int n_moms, bool loss, bool network, bool fp64);
+
 int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const int* times, int n_scalar,
                 const int* mapping, MtpPlan** out)
 {
@@ -2176,36 +2180,57 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         seen[mapping[s]] = 1;
     }
     A2P_REQUIRE(n_moms < 8192, A2P_ERR_INVALID, "mtp plan: more than 8191 moments");    // 16-bit byte offsets
-    // Interleaved gather lists (see mtp_plan.h).  `lists[m]` holds the packed terms of moment m.
+    // Packed terms of each moment, in the order given.
+    struct Lists {
+        std::vector<int> off;
+        std::vector<int2> terms;
+        Lists(int n, const std::vector<std::pair<int, int2>>& given) : off((size_t)n + 2, 0), terms(given.size())
+        {
+            for (const auto& t : given) off[(size_t)t.first + 2]++;
+            for (int m = 0; m < n; m++) off[(size_t)m + 2] += off[(size_t)m + 1];
+            for (const auto& t : given) terms[(size_t)off[(size_t)t.first + 1]++] = t.second;
+        }
+        int size(int m) const { return off[(size_t)m + 1] - off[m]; }
+        const int2* of(int m) const { return terms.data() + off[m]; }
+    };
+    // Interleaved gather lists (see mtp_plan.h).
     struct Ell {
         std::vector<int> level, slot, lead;                // lead: pieces behind
         std::vector<int4> group;                           // first term, depth, doubling steps, MTP_CTRL_LEAF or 0
         std::vector<int2> terms;
-        bool too_long = false;
     };
     // Cuts the lists of one level into pieces of at most `cap` terms and lays them out in rows of sixteen lanes.
     struct Piece { int m, t0, n, rem; };
     struct Level {
         std::vector<Piece> lanes;                          // rows of sixteen, deepest first; whole groups of 64
         std::vector<int> depth, steps;                     // of each group
-        double cost = 0;
     };
-    auto pack_level = [&](const std::vector<std::vector<int2>>& lists, const std::vector<int>& members, int cap, int waves) {
+    auto pieces_of = [](int n, int cap) { return n <= cap ? (n > 0 ? 1 : 0) : (n + cap - 1) / cap; };
+    // (`placed` off: the groups' depths and doubling steps alone, all that the choice of a cut needs)
+    auto pack_level = [&](const Lists& lists, const std::vector<int>& members, int cap, bool placed) {
         struct List { int m, n, np, len; };
-        std::vector<List> ls;
-        for (int m : members) {
-            const int n = (int)lists[m].size(), np = (n + cap - 1) / cap;
-            ls.push_back({m, n, np, np ? (n + np - 1) / np : 0});       // pieces of equal length
-        }
         auto deep = [](int n) { return (n + 1) / 2 * 2; };
-        std::stable_sort(ls.begin(), ls.end(), [&](const List& x, const List& y) {
-            return deep(x.len) != deep(y.len) ? deep(x.len) > deep(y.len) : x.np > y.np;
-        });
+        // deepest pieces first, of those the lists of most pieces
+        std::vector<List> given, ls(members.size());
+        given.reserve(members.size());
+        int most = 0;
+        for (int m : members) {
+            const int n = lists.size(m), np = pieces_of(n, cap);
+            given.push_back({m, n, np, np > 1 ? (n + np - 1) / np : n});        // pieces of equal length
+            most = std::max(most, np);
+        }
+        auto key = [&](const List& l) { return (cap - deep(l.len)) / 2 * (most + 1) + most - l.np; };
+        std::vector<int> place((size_t)(cap / 2 + 1) * (most + 1) + 1, 0);
+        for (const List& l : given) place[key(l) + 1]++;
+        for (size_t k = 1; k < place.size(); k++) place[k] += place[k - 1];
+        for (const List& l : given) ls[place[key(l)]++] = l;
         Level lv;
         std::vector<int> room;                             // free lanes of each row
+        size_t from[17] = {0};                             // rows before from[n] have no room for n pieces (room only shrinks)
+        auto steps_of = [](int pieces) { int k = 0; while ((1 << k) < pieces) k++; return k; };
         for (const List& l : ls) {
             if (l.np == 0) continue;
-            size_t r = 0;
+            size_t r;
             int at;
             if (l.np > 16) {                               // whole rows within a group (the last one has room left)
                 const size_t need = (l.np + 15) / 16;
@@ -2215,68 +2240,92 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 room.back() = (int)need * 16 - l.np;
                 at = 0;
             } else {
+                r = from[l.np];
                 while (r < room.size() && room[r] < l.np) r++;
+                from[l.np] = r;
                 if (r == room.size()) room.push_back(16);
                 at = 16 - room[r];
                 room[r] -= l.np;
             }
-            lv.lanes.resize(room.size() * 16, Piece{-1, 0, 0, 0});
+            if (lv.depth.size() <= r / 4) { lv.depth.resize(r / 4 + 1, 0); lv.steps.resize(r / 4 + 1, 0); }
+            lv.depth[r / 4] = std::max(lv.depth[r / 4], deep(l.len));
+            lv.steps[r / 4] = std::max(lv.steps[r / 4], steps_of(l.np));
+            if (!placed) continue;
+            if (lv.lanes.size() < room.size() * 16) lv.lanes.resize(room.size() * 16, Piece{-1, 0, 0, 0});
             for (int q = 0; q < l.np; q++)
                 lv.lanes[r * 16 + at + q] = {l.m, q * l.len, std::min(l.len, l.n - q * l.len), l.np - 1 - q};
         }
         while (lv.lanes.size() % 64) lv.lanes.push_back({-1, 0, 0, 0});
-        // what a wavefront issues: a term about ten instructions, a group about 25, a doubling step about nine; the workgroup
-        // waits for its slowest wavefront, and the others' share is what other workgroups can use meanwhile
+        return lv;
+    };
+    // what a wavefront issues: a term about ten instructions, a group about 25, a doubling step about nine; the workgroup
+    // waits for its slowest wavefront, and the others' share is what other workgroups can use meanwhile
+    auto level_cost = [](const Level& lv, int waves) {
         std::vector<double> load(waves, 0.0);
         double all = 0;
-        for (size_t g = 0; g < lv.lanes.size(); g += 64) {
-            int n = 0, rem = 0, steps = 0;
-            for (size_t q = g; q < g + 64; q++) { n = std::max(n, lv.lanes[q].n); rem = std::max(rem, lv.lanes[q].rem); }
-            while ((1 << steps) < rem + 1) steps++;
-            lv.depth.push_back(deep(n));
-            lv.steps.push_back(steps);
-            const double c = 10.0 * deep(n) + 25.0 + 9.0 * steps;
+        for (size_t g = 0; g < lv.depth.size(); g++) {
+            const double c = 10.0 * lv.depth[g] + 25.0 + 9.0 * lv.steps[g];
             *std::min_element(load.begin(), load.end()) += c;
             all += c;
         }
-        lv.cost = *std::max_element(load.begin(), load.end()) + all / waves;
-        return lv;
+        return *std::max_element(load.begin(), load.end()) + all / waves;
     };
-    // (`leaves`: lists of another kind that go with the first level to be walked, the last of by_level)
-    auto build_ell = [&](const std::vector<std::vector<int2>>& lists, const std::vector<std::vector<int>>& by_level, int waves,
-                         const std::vector<std::vector<int2>>* leaf_lists = nullptr, const std::vector<int>* leaves = nullptr) {
+    // A level as a workgroup of one wavefront and one of four walk it best.
+    struct Best { Level lv[2]; };
+    bool too_long = false;
+    auto best_level = [&](const Lists& lists, const std::vector<int>& members) {
+        std::vector<int> ms;
+        int longest = 0;
+        for (int m : members) {
+            if (lists.size(m) > 64 * MTP_SLOT_CAP) { too_long = true; continue; }
+            ms.push_back(m);
+            longest = std::max(longest, lists.size(m));
+        }
+        double cost[2] = {-1, -1};
+        int cut[2] = {MTP_SLOT_CAP, MTP_SLOT_CAP};
+        long long pieces = -1;
+        for (int cap = 2; cap <= MTP_SLOT_CAP; cap += 2) {
+            if (longest > 64 * cap) continue;
+            long long np = 0;
+            for (int m : ms) np += pieces_of(lists.size(m), cap);
+            if (np == pieces) continue;                    // (as many pieces of every list: the same layout)
+            pieces = np;
+            const Level lv = pack_level(lists, ms, cap, false);
+            for (int i = 0; i < 2; i++) {
+                const double c = level_cost(lv, i ? 4 : 1);
+                if (cost[i] < 0 || c < cost[i]) { cut[i] = cap; cost[i] = c; }
+            }
+        }
+        Best best;
+        for (int i = 0; i < 2; i++) best.lv[i] = i && cut[1] == cut[0] ? best.lv[0] : pack_level(lists, ms, cut[i], true);
+        return best;
+    };
+    auto best_levels = [&](const Lists& lists, const std::vector<std::vector<int>>& by_level) {
+        std::vector<Best> out;
+        for (const auto& members : by_level) out.push_back(best_level(lists, members));
+        return out;
+    };
+    // (`leaves`: lists of another kind that go with the first level to be walked, the last of them)
+    auto build_ell = [](const Lists& lists, const std::vector<Best>& levels, int wide,
+                        const Lists* leaf_lists = nullptr, const Best* leaves = nullptr) {
         Ell e;
-        auto append = [&](const std::vector<std::vector<int2>>& lists, const std::vector<int>& members, int kind) {
-            std::vector<int> ms;
-            for (int m : members) {
-                if ((int)lists[m].size() > 64 * MTP_SLOT_CAP) e.too_long = true;
-                else ms.push_back(m);
-            }
-            Level best;
-            bool any = false;
-            for (int cap = 2; cap <= MTP_SLOT_CAP; cap += 2) {
-                bool fits = true;
-                for (int m : ms) fits = fits && (int)lists[m].size() <= 64 * cap;
-                if (!fits) continue;
-                Level lv = pack_level(lists, ms, cap, waves);
-                if (!any || lv.cost < best.cost) { best = std::move(lv); any = true; }
-            }
+        auto append = [&](const Lists& lists, const Level& best, int kind) {
             for (size_t g = 0; g < best.depth.size(); g++) {
                 e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], kind));
                 e.terms.resize(e.terms.size() + (size_t)best.depth[g] * 64, make_int2(0, 0));
                 for (size_t q = 0; q < 64; q++) {
                     const Piece& pc = best.lanes[g * 64 + q];
                     for (int k = 0; k < pc.n; k++)
-                        e.terms[e.group.back().x + (size_t)k * 64 + q] = lists[pc.m][pc.t0 + k];
+                        e.terms[e.group.back().x + (size_t)k * 64 + q] = lists.of(pc.m)[pc.t0 + k];
                     e.slot.push_back(pc.n > 0 && pc.t0 == 0 ? pc.m : -1);      // the first piece of a list names the moment
                     e.lead.push_back(pc.rem);
                 }
             }
         };
-        for (size_t l = 0; l < by_level.size(); l++) {
+        for (size_t l = 0; l < levels.size(); l++) {
             e.level.push_back((int)e.slot.size());
-            append(lists, by_level[l], 0);
-            if (leaves && l + 1 == by_level.size()) append(*leaf_lists, *leaves, MTP_CTRL_LEAF);
+            append(lists, levels[l].lv[wide], 0);
+            if (leaves && l + 1 == levels.size()) append(*leaf_lists, leaves->lv[wide], MTP_CTRL_LEAF);
         }
         e.level.push_back((int)e.slot.size());
         return e;
@@ -2325,22 +2374,25 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         return st;
     };
     // forward: terms per destination in file order; level l >= 1 at index l - 1
-    std::vector<std::vector<int2>> fl(n_moms), rl(n_moms);
+    std::vector<std::pair<int, int2>> given;
     for (int e = 0; e < n_times; e++) {
         const int* q = times + e * 4;
-        fl[q[3]].push_back(make_int2((q[0] * 8) | ((q[1] * 8) << 16), q[2]));
+        given.emplace_back(q[3], make_int2((q[0] * 8) | ((q[1] * 8) << 16), q[2]));
     }
+    const Lists fl(n_moms, given);
     std::vector<std::vector<int>> f_by(n_levels), r_by(n_levels);
     for (int m = n_basic; m < n_moms; m++)
-        if (level[m] >= 1 && !fl[m].empty()) f_by[level[m] - 1].push_back(m);
+        if (level[m] >= 1 && fl.size(m)) f_by[level[m] - 1].push_back(m);
     // reverse: terms per source in reverse file order
+    given.clear();
     for (int e = n_times - 1; e >= 0; e--) {
         const int* q = times + e * 4;
-        rl[q[1]].push_back(make_int2((q[3] * 8) | ((q[0] * 8) << 16), q[2]));     // adj[m1] += adj[dst] mult M[m0]
-        rl[q[0]].push_back(make_int2((q[3] * 8) | ((q[1] * 8) << 16), q[2]));     // adj[m0] += adj[dst] mult M[m1]
+        given.emplace_back(q[1], make_int2((q[3] * 8) | ((q[0] * 8) << 16), q[2]));     // adj[m1] += adj[dst] mult M[m0]
+        given.emplace_back(q[0], make_int2((q[3] * 8) | ((q[1] * 8) << 16), q[2]));     // adj[m0] += adj[dst] mult M[m1]
     }
+    const Lists rl(n_moms, given);
     for (int m = 0; m < n_moms; m++)
-        if (level[m] < n_levels && !rl[m].empty()) r_by[level[m]].push_back(m);
+        if (level[m] < n_levels && rl.size(m)) r_by[level[m]].push_back(m);
     // Leaves: scalar moments that no product reads.  Only the read-out needs them, so that the calls whose read-out is linear
     // form them in the first step of the reverse sweep; the levels of the forward sweep that held nothing else are gone.
     std::vector<char> is_source(n_moms, 0);
@@ -2348,7 +2400,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     std::vector<int> leaves, mapping_leaf(mapping, mapping + n_scalar);
     for (int s = 0; s < n_scalar; s++) {
         const int m = mapping[s];
-        if (m < n_basic || is_source[m] || fl[m].empty()) continue;
+        if (m < n_basic || is_source[m] || !fl.size(m)) continue;
         mapping_leaf[s] |= 1 << 16;
         leaves.push_back(m);
     }
@@ -2356,11 +2408,27 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     for (auto& l : core_by)
         l.erase(std::remove_if(l.begin(), l.end(), [&](int m) { return !is_source[m]; }), l.end());
     while (!core_by.empty() && core_by.back().empty()) core_by.pop_back();
-    const Ell C[2] = {build_ell(fl, core_by, 1), build_ell(fl, core_by, 4)};
-    const Ell V[2] = {build_ell(rl, r_by, 1, &fl, &leaves), build_ell(rl, r_by, 4, &fl, &leaves)};
-    const Ell F[2] = {build_ell(fl, f_by, 1), build_ell(fl, f_by, 4)}, R[2] = {build_ell(rl, r_by, 1), build_ell(rl, r_by, 4)};
-    A2P_REQUIRE(!F[0].too_long && !R[0].too_long, A2P_ERR_INVALID,
+    const std::vector<Best> f_best = best_levels(fl, f_by), r_best = best_levels(rl, r_by);
+    std::vector<Best> c_best;
+    for (size_t l = 0; l < core_by.size(); l++)
+        c_best.push_back(core_by[l].size() == f_by[l].size() ? f_best[l] : best_level(fl, core_by[l]));
+    const Best leaf_best = best_level(fl, leaves);
+    A2P_REQUIRE(!too_long, A2P_ERR_INVALID,
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
+    // The streams that a launch can ask for: those of the widths that wide_atoms gives for as many moments, and the forward one
+    // of four wavefronts for the components.  (Host time of a plan with all of them and every cut laid out for each by itself
+    // 1.83 ms for level 16 and 14.2 for level 20, this 0.78 and 4.2.)
+    bool reached[2] = {false, false};
+    for (int q = 0; q < 8; q++) reached[wide_atoms(n_moms, q & 1, q & 2, q & 4)] = true;
+    Stream fs[2], rs[2], cs[2], vs[2];
+    for (int i = 0; i < 2; i++) {
+        const int waves = i ? 4 : 1;
+        if (reached[i] || i == 1) fs[i] = build_stream(build_ell(fl, f_best, i), true, waves);
+        if (!reached[i]) continue;
+        rs[i] = build_stream(build_ell(rl, r_best, i), false, waves);
+        cs[i] = build_stream(build_ell(fl, c_best, i), true, waves);
+        vs[i] = build_stream(build_ell(rl, r_best, i, &fl, &leaf_best), false, waves);
+    }
     // monomial rows, their polynomials and the places of the basic moments among the coefficients (mtp_plan.h)
     std::vector<int> degree((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);      // highest c + 1 of (a, b, mu), 0: none
     for (int i = 0; i < n_basic; i++) {
@@ -2441,7 +2509,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     if (n_basic < 64 * MTP_SLOT_CAP) {
         std::vector<std::vector<int>> terms_of(n_moms);
         for (int e = 0; e < n_times; e++) terms_of[times[e * 4 + 3]].push_back(e);
-        std::vector<int> node_of(n_moms, -1), anc, stack;
+        std::vector<int> node_of(n_moms, -1), anc, stack, terms;
         auto ancestors = [&](int s, int first_node) {          // fills anc and node_of; returns the number of nodes
             anc.clear();
             stack.assign(1, mapping[s]);
@@ -2473,48 +2541,52 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             xhosts.emplace_back();
             XHost& h = xhosts.back();
             h.root.assign(n_scalar, -1);
-            std::vector<std::vector<int2>> xl;
-            std::vector<std::vector<int>> x_by(n_levels);
-            std::vector<std::vector<int>> seed_basic(n_scalar);
+            std::vector<std::pair<int, int2>> given, words;
+            std::vector<std::pair<int, int>> by_level;
             for (int s : seeds) {
                 const int cnt = ancestors(s, h.nodes);
                 h.nodes += cnt;
-                xl.resize(h.nodes);
                 h.root[s] = node_of[mapping[s]];
-                for (int e = n_times - 1; e >= 0; e--) {          // reverse file order, as in the reverse gather above
+                terms.clear();
+                for (int m : anc) terms.insert(terms.end(), terms_of[m].begin(), terms_of[m].end());
+                std::sort(terms.begin(), terms.end(), std::greater<int>());       // reverse file order, as in the reverse gather above
+                for (int e : terms) {
                     const int* q = times + e * 4;
-                    if (node_of[q[3]] < 0) continue;
                     const int nd = node_of[q[3]];
-                    xl[node_of[q[1]]].push_back(make_int2((nd * 8) | ((q[0] * 8) << 16), q[2]));
-                    xl[node_of[q[0]]].push_back(make_int2((nd * 8) | ((q[1] * 8) << 16), q[2]));
+                    given.emplace_back(node_of[q[1]], make_int2((nd * 8) | ((q[0] * 8) << 16), q[2]));
+                    given.emplace_back(node_of[q[0]], make_int2((nd * 8) | ((q[1] * 8) << 16), q[2]));
                 }
+                bool any = false;
                 for (int m : anc) {
-                    if (level[m] < n_levels && !xl[node_of[m]].empty()) x_by[level[m]].push_back(node_of[m]);
-                    if (m < n_basic) seed_basic[s].push_back(node_of[m] | (x_polys ? poly_pos[m] : m) << 16);
+                    if (level[m] < n_levels) by_level.emplace_back(level[m], node_of[m]);
+                    if (m >= n_basic) continue;
+                    words.emplace_back(s, make_int2(node_of[m] | (x_polys ? poly_pos[m] : m) << 16, 0));
+                    any = true;
                 }
+                if (!any) words.emplace_back(s, make_int2(-1, 0));           // (a column of zeros)
                 for (int m : anc) node_of[m] = -1;
             }
-            if (xl.empty()) xl.emplace_back();
-            const Ell ell = build_ell(xl, x_by, 4);
-            h.stream = build_stream(ell, false, 4);
-            A2P_REQUIRE(!ell.too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
+            const Lists xl(h.nodes, given);
+            std::vector<std::vector<int>> x_by(n_levels);
+            for (const auto& q : by_level)
+                if (xl.size(q.second)) x_by[q.first].push_back(q.second);
+            h.stream = build_stream(build_ell(xl, best_levels(xl, x_by), 1), false, 4);
+            A2P_REQUIRE(!too_long, A2P_ERR_INVALID, "mtp plan: a moment takes part in more than %d products",
                         64 * MTP_SLOT_CAP);
             // The lists of basic ancestors, cut and placed as the gathers' are.  A group costs its reads of D and some ten more for
             // what it does once per pair of neighbours (and three for a doubling step); the groups of a round are worked on at the
             // same time, fewer than four by several wavefronts each, and the reads of all of them share the LDS.  (Lists cut at
             // sixteen words: 32 words deep instead of 24 at level 16.)
-            std::vector<std::vector<int2>> columns(n_scalar);
-            for (int s : seeds) {
-                for (int w : seed_basic[s]) columns[s].push_back(make_int2(w, 0));
-                if (columns[s].empty()) columns[s].push_back(make_int2(h.nodes, 0));      // (a column of zeros)
-            }
+            for (auto& w : words)
+                if (w.second.x < 0) w.second.x = h.nodes;
+            const Lists columns(n_scalar, words);
             Level best;
             double best_cost = 0;
             for (int cap = MTP_SLOT_CAP; cap >= 2; cap -= 2) {
                 bool fits = true;
-                for (int s : seeds) fits &= (int)columns[s].size() <= 64 * cap;
+                for (int s : seeds) fits &= columns.size(s) <= 64 * cap;
                 if (!fits) break;
-                Level lv = pack_level(columns, seeds, cap, 4);
+                Level lv = pack_level(columns, seeds, cap, true);
                 const size_t n = lv.depth.size();
                 double cost = 0;
                 for (size_t g0 = 0; g0 < n; g0 += 4) {
@@ -2539,7 +2611,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                     std::vector<std::vector<int>> lists(16);
                     for (size_t q = 0; q < 16; q++) {
                         const Piece& pc = best.lanes[row + q];
-                        for (int k = 0; k < pc.n; k++) lists[q].push_back(columns[pc.m][pc.t0 + k].x);
+                        for (int k = 0; k < pc.n; k++) lists[q].push_back(columns.of(pc.m)[pc.t0 + k].x);
                         h.seed.push_back(pc.n > 0 && pc.t0 == 0 ? pc.m : -1);
                         h.brem.push_back(pc.rem);
                     }
@@ -2572,15 +2644,10 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                          add(st.slots.data(), sizeof(int) * st.slots.size()), add(st.words.data(), sizeof(int4) * st.words.size())};
     };
     const size_t o_leaf = add(mapping_leaf.data(), sizeof(int) * n_scalar);
-    Stream fs[2], rs[2], cs[2], vs[2];
     StreamOff o_f[2], o_r[2], o_c[2], o_v[2];
     for (int i = 0; i < 2; i++) {
-        fs[i] = build_stream(F[i], true, i ? 4 : 1);
-        rs[i] = build_stream(R[i], false, i ? 4 : 1);
         o_f[i] = add_stream(fs[i]);
         o_r[i] = add_stream(rs[i]);
-        cs[i] = build_stream(C[i], true, i ? 4 : 1);
-        vs[i] = build_stream(V[i], false, i ? 4 : 1);
         o_c[i] = add_stream(cs[i]);
         o_v[i] = add_stream(vs[i]);
     }
@@ -2664,9 +2731,6 @@ int plan_check(void* handle, MtpPlan** out)
     *out = (MtpPlan*)handle;
     return A2P_OK;
 }
-
-// 256 threads per atom or 64 (the rule is at its definition)
-bool wide_atoms(int n_moms, bool loss, bool network, bool fp64);
 
 // Whether the atom kernel sums the basic moments by polynomials (basic_sums): each has a thread, and the sums of a group
 // of threads fit the place of the shortest table.  Otherwise each moment is formed by itself, from powers of z.
