@@ -2829,17 +2829,17 @@ bool wide_atoms(int n_moms, bool loss, bool network, bool fp64)
 }
 
 template <typename T, bool LOSS, bool SEED = false>
-int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
+int launch_atoms(const MtpArgs<T>& args, hipStream_t stream)
 {
+    MtpArgs<T> a = args;         // (what belongs to this launch alone is set here)
     {
         static const char* e = getenv("AI2POT_MTP_KEEP_TABLE");
         if (e) g_keep_table = e[0] != '0';
     }
     const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0, sizeof(T) == 8);
     if (a.H == 0 && !a.row_seed && !a.e_sites && !a.desc && !a.energy_only) {
-        MtpArgs<T>& w = const_cast<MtpArgs<T>&>(a);
-        w.leaves_late = 1;
-        for (int i = 0; i < 2; i++) { w.p.fwd[i] = a.p.fwd_core[i]; w.p.rev[i] = a.p.rev_leaf[i]; }
+        a.leaves_late = 1;
+        for (int i = 0; i < 2; i++) { a.p.fwd[i] = a.p.fwd_core[i]; a.p.rev[i] = a.p.rev_leaf[i]; }
     }
     const int groups = a.z_powers ? 0 : (wide ? 256 : 64) / std::max(a.p.npoly, 1);      // of a thread per polynomial
     const int kept_adjoints = std::max(a.p.n_moms, groups * a.p.ncoef_poly);
@@ -2876,41 +2876,40 @@ int launch_atoms(const MtpArgs<T>& a, hipStream_t stream)
                 const size_t l = lds_for(nc, &m, kept_adjoints);
                 if (per_cu(l) >= want) { keep = 1; nc_cap = nc; lds = l; lds_main = m; break; }
             }
-        const_cast<MtpArgs<T>&>(a).keep_table = keep;
+        a.keep_table = keep;
     }
     {
-        MtpArgs<T>& w = const_cast<MtpArgs<T>&>(a);
         const MtpPlanDevice& p = a.p;
         const int nt = wide ? 256 : 64;
-        const int keep = !LOSS && w.keep_table != 0 ? kept_adjoints : 0;
-        w.lds_basic_off = (int)lds_main;
-        w.nc_cap = nc_cap;
+        const int keep = !LOSS && a.keep_table != 0 ? kept_adjoints : 0;
+        a.lds_basic_off = (int)lds_main;
+        a.nc_cap = nc_cap;
         // moments | (loss mode: their tangents) | coefficients | region of the neighbour table | ...
-        w.at_Tg = p.n_moms;
-        w.at_cf = w.at_Tg + (LOSS ? p.n_moms : 0);
-        w.at_tab = w.at_cf + a.ntypes * p.nmus * a.K;
+        a.at_Tg = p.n_moms;
+        a.at_cf = a.at_Tg + (LOSS ? p.n_moms : 0);
+        a.at_tab = a.at_cf + a.ntypes * p.nmus * a.K;
         // the adjoints share the table's region, behind the sweeps' partial sums, or lie behind the table
-        w.at_A = w.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt)
+        a.at_A = a.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt)
                                   : mtp_adjoint_offset((LOSS ? 2 : 1) * p.max_level_slots));
-        w.at_Bm = w.at_A + p.n_moms;
+        a.at_Bm = a.at_A + p.n_moms;
         // Partial sums of the thread groups, needed only in the last pass over the neighbours, when the moments (and, in
         // loss mode, their tangents) are dead: a long enough moment vector lends them its place.  Energy / force / virial
         // kernel: they are written over the table once it has been read.
-        w.at_gred = !LOSS ? w.at_tab : mtp_gred_in_moments(LOSS, p.n_moms) ? 0 : w.at_tab + nc_cap * a.E;
-        w.at_Ab = w.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, p.max_level_slots, nt, keep);
-        w.at_Bb = w.at_Ab + p.ncoef_poly;
-        w.at_pq = LOSS ? w.at_Bb + p.ncoef_poly : w.at_Ab;
-        w.at_net = w.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);
-        w.at_polys = mtp_polys_in_moments(p.ncoef_poly, p.n_moms) ? 0 : w.at_pq + (a.H > 0 ? p.n_scalar + a.H : 0);
+        a.at_gred = !LOSS ? a.at_tab : mtp_gred_in_moments(LOSS, p.n_moms) ? 0 : a.at_tab + nc_cap * a.E;
+        a.at_Ab = a.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, p.max_level_slots, nt, keep);
+        a.at_Bb = a.at_Ab + p.ncoef_poly;
+        a.at_pq = LOSS ? a.at_Bb + p.ncoef_poly : a.at_Ab;
+        a.at_net = a.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);
+        a.at_polys = mtp_polys_in_moments(p.ncoef_poly, p.n_moms) ? 0 : a.at_pq + (a.H > 0 ? p.n_scalar + a.H : 0);
     }
     if (LOSS) {
         // the group sums' place: the moments and their tangents, or 1024 entries behind the table
         const int n1 = a.p.nmus * a.K, place = mtp_gred_in_moments(true, a.p.n_moms) ? 2 * a.p.n_moms : 1024;
-        const_cast<MtpArgs<T>&>(a).grad_parts = std::max(1, std::min((wide ? 256 : 64) / n1, place / (a.ntypes * n1)));
+        a.grad_parts = std::max(1, std::min((wide ? 256 : 64) / n1, place / (a.ntypes * n1)));
     }
     // as many groups of a thread per polynomial as the workgroup has, and as the place of their sums holds
     const int room = !LOSS && a.keep_table ? kept_adjoints : mtp_table_entries(nc_cap, a.E, LOSS, a.p.n_moms, wide ? 256 : 64);
-    const_cast<MtpArgs<T>&>(a).mom_groups = std::min(groups, room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1));
+    a.mom_groups = std::min(groups, room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1));
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
     auto kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
