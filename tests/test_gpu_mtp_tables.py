@@ -109,6 +109,58 @@ def test_components_of_irregular_tables(oracle, basic, lists):
         assert close(a, b)
 
 
+def components_by_both_routes(m, nb):
+    """Energy, force and virial columns from one pass over the atoms, and from a pass per column."""
+    from ai2pot_amd import _lib, ops
+    import torch
+    md = model_to_device(m, torch.float64)
+    d = to_device(nb, torch.float64)
+    args = (m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+            md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], d["binum"], d["bilist"], d["bnumneigh"],
+            d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"])
+    L = _lib.lib()
+    before = L.a2p_mtp_components_route(1)
+    try:
+        one = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+        L.a2p_mtp_components_route(0)
+        per_column = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+    finally:
+        L.a2p_mtp_components_route(before)
+    return one, per_column
+
+
+@pytest.mark.parametrize("level", [8, 16])                        # 11 columns and 94: one of them to a lane, and two
+@pytest.mark.parametrize("pairs", [63, 64, 65, 127, 128, 129, 130, 255, 256, 257])
+def test_components_by_pairs_that_name_an_atom(oracle, level, pairs):
+    """An atom named by as many pairs as a wavefront ranks at a time, as have their displacements in LDS, and as are ranked at
+    all, one more and one less: all columns from one pass against a pass per column, fp64 1e-10."""
+    m, nb, _ = loss_inputs(oracle, level, 2, sizes=(40, 23))
+    first = nb["bfirstneigh"].copy()
+    first[0][first[0] == 5] = 6
+    used = np.argwhere(np.arange(first.shape[2]) < nb["bnumneigh"][0][:, None])
+    for ii, u in used[::len(used) // pairs][:pairs]:              # (over all rows, at places of any order)
+        first[0, ii, u] = 5
+    nb = dict(nb, bfirstneigh=first)
+    assert sum((first[0, i, :n] == 5).sum() for i, n in enumerate(nb["bnumneigh"][0])) == pairs
+    for a, b in zip(*components_by_both_routes(m, nb)):
+        assert np.abs(b).max() > 0
+        assert close(a, b)
+
+
+# a power of z left out and a moment given twice: as many coefficients as basic moments, though not one for each
+ONE_OF_EACH = [(0, 0, 0, 0), (0, 0, 0, 2), (0, 1, 0, 0), (0, 1, 0, 0), (1, 0, 0, 0), (1, 0, 0, 1)]
+
+
+def test_as_many_coefficients_as_basic_moments(oracle):
+    test_irregular_basic_moments(oracle, ONE_OF_EACH)
+    nt = 2
+    nb = synth.pack_batch([structure(oracle, n, (8.5, 9.0, 9.5), nt, 21 + n, 5.0) for n in (40, 23)])
+    m = synth.mtp_model(tables(ONE_OF_EACH), nt, 6, 5.0, 1.5, 3200)
+    for a, b in zip(*components_by_both_routes(m, nb)):
+        assert np.abs(b).max() > 0
+        assert close(a, b)
+
+
 def test_components_in_chunks_of_structures(oracle):
     """Enough pair derivatives (level 16: 92 columns, more than 200 MB) that the structures are taken in chunks, the last
     one shorter: every structure equal to the call with that structure alone, bit for bit, in force columns too."""
