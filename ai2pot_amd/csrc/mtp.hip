@@ -1002,9 +1002,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             // A neuron's sum over the inputs, and an input's over the neurons, by 1, 2 .. 16 neighbouring lanes each, W weights
             // of a lane on their way together, the first of either sum ahead of what it waits for.  What bounds it is the trips to
             // the weights and the chain of their operations.  (A wavefront for four neurons at a time with sums over its 64 lanes,
-            // then a lane for an input, against this, in us of the kernel: level 12, 20 neurons, 3000 atoms 37.6 and 33.6, 200 atoms
-            // 25.6 and 23.1, the loss gradient of 16 structures of 64 atoms 45.5 and 41.2; level 20, 60 neurons, 152 and 143, 37.6
-            // and 35.8, 221 and 198.)
+            // then a lane for an input, against this, in us of the kernel: level 12, 20 neurons, 3000 atoms 37.6 and 33.9, 200 atoms
+            // 25.6 and 23.5, the loss gradient of 16 structures of 64 atoms 45.5 and 41.4; level 20, 60 neurons, 152 and 141, 37.6
+            // and 36.0, 221 and 195.)
             // At least two lanes to a neuron from 9 inputs on, four from 24 on, eight in fp32 from 128 on, in as many rounds as that
             // takes: fewer lanes read a few bytes of each of many rows at a time, whose lines are gone before they are used up
             // (one lane, two, four, eight; 3000 atoms: level 8, 9 inputs, 60 neurons 27.5, 27.2, 28.5, 32.0 us; level 10, 16
@@ -1806,9 +1806,9 @@ comp_rows_kernel(int B, int P, int U, int ntypes, const int* __restrict__ binum,
     nnc[row] = nn;
 }
 
-// The pairs that name each atom, by row * U + slot (B P U is below 2^31).  Each atom has room for `cap` of them (the row length of the list: enough for every list
-// built with one cutoff), so one pass lists them; when an atom is named more often (spill[0] counts what found no room)
-// the pass is repeated for counts only and then into segments of the right lengths (seg).
+// The pairs that name each atom, by row * U + slot (B P U is below 2^31).  Each atom has room for `cap` of them (the row length
+// of the list: enough for every list built with one cutoff), so one pass lists them; when an atom is named more often (spill[0]
+// counts what found no room) the pass is repeated for counts only and then into segments of the right lengths (seg).
 __global__ void __launch_bounds__(256)
 comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int* __restrict__ bfirstneigh, int* __restrict__ cnt, const int* __restrict__ seg, int cap,
                      int* __restrict__ inc, int* __restrict__ spill)
@@ -1835,7 +1835,10 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
 // fifth of its instructions and the registers of four more reads in flight); sorting the lists by insertion, one thread per
 // atom, used to take as long as they do (95 us beside 98 us at 64 structures of 128 atoms).
 // With more than 64 columns a lane takes two of them, 64 apart, so that an atom's pairs are ranked once; the displacements of the
-// first COMP_DISP pairs lie in LDS (of 256: 20 instead of 32 wavefronts to a compute unit).  2 x 50 -> 2 x 41 us there.
+// first COMP_DISP pairs lie in LDS (of 256: 20 instead of 32 wavefronts to a compute unit).  2 x 50 -> 2 x 41 us there.  One column
+// to a lane and two, 6,400 atoms: 53 columns 40.0 and 42.9 us, 65 67.6 and 56.4, 93 85.1 and 72.7, 127 109.5 and 97.5, 151 136.6 and
+// 136.4, 261 243.6 and 249.3 (a last block half of which has no column); fp32 24.9 and 27.0, 38.2 and 28.5, 52.8 and 38.0, 65.5 and
+// 52.6, 83.3 and 75.4, 130.5 and 122.7; 160 atoms, 93 columns 11.6 and 12.8.
 constexpr int COMP_SORT = 256, COMP_DISP = 128;
 
 template <typename T, int NC>
@@ -2093,8 +2096,7 @@ std::set<MtpPlan*> g_plans;
 // the words (node | basic << 16) of lane q, at most `depth` of them; out[k * stride + q] is the lane's word of step k, or
 // a word of the node `zero_node` where it has none.  16 lanes read from the 64 banks at a time, and lanes that name basic
 // moments of the same remainder mod 16 wait for each other unless they name the same one.  Greedy: the lanes with the
-// fewest steps to spare choose first, each the moment whose banks are least taken.  (Longest waits summed over the steps
-// at level 16: 185 as the lists come, 114 ordered; there are 112 steps.)
+// fewest steps to spare choose first, each the moment whose banks are least taken.
 void spread_over_banks(const std::vector<std::vector<int>>& lists, int depth, int zero_node, int* out, int stride)
 {
     constexpr int LANES = 16;

@@ -78,8 +78,8 @@ struct MtpPlanDevice {
     // ancestor of scalar moment s: mapping[s] itself, or a factor of a product among its ancestors.  The adjoint
     // sweeps of all read-outs e_s together are one reverse gather over the nodes, laid out like the reverse gather
     // above (a term packs x = 8 node(dst) | 8 other << 16 with `other` a moment, y = mult).
-    // The basic ancestors of a scalar moment form a list of words node | basic << 16; lists are sorted by length, cut into
-    // pieces of at most MTP_SLOT_CAP words, and dealt to slots, 64 slots a group, the pieces of a list in neighbouring
+    // The basic ancestors of a scalar moment form a list of words node | basic << 16; lists are cut into pieces of equal length,
+    // at most MTP_SLOT_CAP words, and placed first fit, deepest first, 64 slots a group, the pieces of a list in neighbouring
     // slots as in the gathers (the wavefront adds their sums, x_bsteps doubling steps).  A group's words are
     // stored interleaved and padded to the group's depth with node x_nodes, whose adjoint is always zero; `basic` is the moment's
     // place among the polynomials' coefficients (poly_pos) when there are as many of them as basic moments (x_polys): word k of

@@ -1286,7 +1286,8 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
             // binLinkedList.h:1014-1017: the double-precision length, rounded to T, against the double-precision bounds.
             // In fp32 the length in T decides unless it lies within 1e-6 of a bound (its error and the rounding of
             // the other stay below 3e-7 together), and only a chunk with such a candidate forms the other: seven vector
-            // instructions instead of twelve, a third of which take more than one issue slot.
+            // instructions instead of twelve, a third of which take more than one issue slot.  Sorted rows keep the other: its
+            // root is the key they are put in order by.
             double d2d = 0.0;
             bool in;
             unsigned long long mask;
