@@ -40,7 +40,7 @@ __device__ __forceinline__ void tile_of(int t, int nc, int& i, int& j)
     j = i + t;
 }
 
-template <typename T>
+template <typename T, int AHEAD>
 __global__ void __launch_bounds__(256) gram_kernel(const GramArgs<T> a)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(256) gram_kernel(const GramArgs<T> a)
     }
     // Eight rows of a column per wavefront, all in flight (rows beyond the block and columns beyond y are zero).  Those of the
     // first AHEAD columns of a lane are on their way while the rows before them are multiplied.
-    constexpr int AHEAD = 2, PER = GR_ROWS / 4;
+    constexpr int PER = GR_ROWS / 4;
     auto fetch = [&](T (&v)[PER], int s0, int c) __attribute__((always_inline)) {
         const T* const src = c < n ? X + c : y;
         const long long step = c < n ? n : 1;
@@ -113,10 +113,13 @@ __global__ void __launch_bounds__(256) gram_kernel(const GramArgs<T> a)
     }
 }
 
-// A quarter of a tile per workgroup: sixteen threads per entry take a sixteenth of the blocks each.  Bound by its dependent loads (a
-// workgroup per tile with four threads per entry: 10 us for 198 blocks, this 4.6, and 6.4 for 394).
-constexpr int GS_PARTS = 16, GS_ENTRIES = 64;
-template <typename T>
+// A quarter of a tile per workgroup, GS_PARTS threads per entry, each for its share of the blocks.  Bound by its dependent loads
+// while there are few tiles (sixteen threads per entry, four, and a workgroup per tile with four: 94 columns, 24,576 rows 8.7, 10.4 and
+// 18.5 us; 127 columns 7.1, 7.7 and 12.0), and by the workgroups and what they write from a workgroup for every compute unit on,
+// where four threads per entry suffice (164 columns, 66 tiles, 8.8, 7.4 and 10.6; 290 columns 9.2, 7.6 and 8.3; 503 columns, 3,072 rows
+// 18.9, 8.7 and 11.1).
+constexpr int GS_ENTRIES = 64, GS_MANY = 64;         // entries of a workgroup; tiles from which four threads per entry are taken
+template <typename T, int GS_PARTS>
 __global__ void __launch_bounds__(GS_PARTS * GS_ENTRIES)
 gram_sum_kernel(const GramArgs<T> a, T* __restrict__ A, T* __restrict__ b)
 {
@@ -186,12 +189,16 @@ int normal_equations(int n, const long long* rows, const double* w, const T* con
     int rc = ws_get(WS_MISC, (size_t)std::max(blocks, 1) * a.ntiles * 256 * sizeof(T), &ws);
     if (rc) return rc;
     a.part = (T*)ws;
-    auto kern = gram_kernel<T>;
+    // columns of a lane that are asked for one pass ahead: two, and one beyond 256 columns, of which a lane has five or more (one and
+    // two: 127 columns, 24,576 rows 32.2 and 31.7 us; 290, 120,000 rows 581 and 600; 503, 24,576 rows 618 and 634)
+    auto kern = a.nc > 16 ? gram_kernel<T, 1> : gram_kernel<T, 2>;
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     prof_begin("gram", stream);
     if (blocks) hipLaunchKernelGGL(kern, dim3(blocks, groups), dim3(256), lds, stream, a);
-    hipLaunchKernelGGL(gram_sum_kernel<T>, dim3(a.ntiles, 256 / GS_ENTRIES), dim3(GS_PARTS * GS_ENTRIES), 0, stream, a, A, b);
+    const int parts = a.ntiles < GS_MANY ? 16 : 4;
+    auto sum = parts == 16 ? gram_sum_kernel<T, 16> : gram_sum_kernel<T, 4>;
+    hipLaunchKernelGGL(sum, dim3(a.ntiles, 256 / GS_ENTRIES), dim3(parts * GS_ENTRIES), 0, stream, a, A, b);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;

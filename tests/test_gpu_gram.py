@@ -43,6 +43,15 @@ def test_normal_equations(dtype, n, rows):
     assert np.array_equal(A, A.T)
 
 
+# 55 and 66 tiles: the last column count with sixteen threads to an entry of the blocks' sum, and the first ones with four, from
+# fewer blocks than those to more
+@pytest.mark.parametrize("dtype", ["float64", "float32"])
+@pytest.mark.parametrize("n,rows", [(159, (1, 33, 9)), (159, (9, 24576, 81)), (160, (1, 0, 0)), (160, (1, 33, 9)),
+                                    (175, (9, 24576, 81)), (176, (3, 150, 27))])
+def test_sum_of_the_blocks(dtype, n, rows):
+    test_normal_equations(dtype, n, rows)
+
+
 @pytest.mark.parametrize("named", [9, 300])
 def test_an_atom_named_by_many_pairs(oracle, named):
     import torch
