@@ -1003,8 +1003,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             // of a lane on their way together, the first of either sum ahead of what it waits for.  What bounds it is the trips to
             // the weights and the chain of their operations.  (A wavefront for four neurons at a time with sums over its 64 lanes,
             // then a lane for an input, against this, in us of the kernel: level 12, 20 neurons, 3000 atoms 37.6 and 33.9, 200 atoms
-            // 25.6 and 23.5, the loss gradient of 16 structures of 64 atoms 45.5 and 41.4; level 20, 60 neurons, 152 and 141, 37.6
-            // and 36.0, 221 and 195.)
+            // 25.6 and 23.5, the loss gradient of 16 structures of 64 atoms 45.5 and 41.4; level 20, 60 neurons, 152 and 143, 37.6
+            // and 36.0, 221 and 197.)
             // At least two lanes to a neuron from 9 inputs on, four from 24 on, eight in fp32 from 128 on, in as many rounds as that
             // takes: fewer lanes read a few bytes of each of many rows at a time, whose lines are gone before they are used up
             // (one lane, two, four, eight; 3000 atoms: level 8, 9 inputs, 60 neurons 27.5, 27.2, 28.5, 32.0 us; level 10, 16
@@ -1039,22 +1039,36 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
 #pragma unroll
                 for (int u = 0; u < W; u++) w[u] = w0[__umul24(min(n0 + u * ps, H - 1), S) + at];
             };
-            // W of the products of a sum: acc += w q[first + u step], below `end` (others may be infinite), and tac += w t[..]
+            // W of the products of a sum: acc += w q[first + u step], below `end` (others may be infinite), and tac += w t[..]; by
+            // halves, as the sums of the lanes (one after the other: energies in fp32 up to a tenth further from fp64)
             auto products = [&](T& acc, T& tac, const T* q, const T* t, int first, int step, int end, bool whole) __attribute__((always_inline)) {
+                T v[W], d[LOSS ? W : 1];
                 if (whole)                                     // wave-uniform
 #pragma unroll
                     for (int u = 0; u < W; u++) {
-                        acc += w[u] * q[first + u * step];
-                        if (LOSS) tac += w[u] * t[first + u * step];
+                        v[u] = w[u] * q[first + u * step];
+                        if constexpr (LOSS) d[u] = w[u] * t[first + u * step];
                     }
                 else
 #pragma unroll
                     for (int u = 0; u < W; u++) {
                         const int i = first + u * step, own = min(i, end - 1);
-                        const T v = w[u] * q[own], d = LOSS ? w[u] * t[own] : (T)0;
-                        acc += i < end ? v : (T)0;
-                        if (LOSS) tac += i < end ? d : (T)0;
+                        v[u] = w[u] * q[own];
+                        if (i >= end) v[u] = (T)0;
+                        if constexpr (LOSS) {
+                            d[u] = w[u] * t[own];
+                            if (i >= end) d[u] = (T)0;
+                        }
                     }
+#pragma unroll
+                for (int n = W / 2; n > 0; n >>= 1)
+#pragma unroll
+                    for (int u = 0; u < n; u++) {
+                        v[u] += v[u + n];
+                        if constexpr (LOSS) d[u] += d[u + n];
+                    }
+                acc += v[0];
+                if constexpr (LOSS) tac += d[0];
             };
             row_weights(hl, hp);
             const T w1_own = w1[min(lane, H - 1)];
