@@ -373,14 +373,12 @@ nep_efv_kernel(const NepArgs<T> a)
 #pragma unroll
                         for (int mp = 0; mp < 2 * l + 1; mp++) {
                             const int m = l * l - 1 + mp;
-                            if (l <= l_max) srad += (Ad[m] - (T)l * rinv * A[m]) * bl[m];
+                            if (l <= l_max) srad += Ad[m] * bl[m];
                             else A[m] = (T)0;
                         }
-                    T wx = (T)0, wy = (T)0, wz = (T)0;
-                    blm_grad_dot<T, LC>(ux, uy, uz, A, wx, wy, wz);
-                    const T gx = srad * ux + wx * rinv;
-                    const T gy = srad * uy + wy * rinv;
-                    const T gz = srad * uz + wz * rinv;
+                    T wx, wy, wz, gx, gy, gz;
+                    blm_gradient<T, LC>(ux, uy, uz, A, wx, wy, wz);
+                    pair_gradient(srad, wx, wy, wz, ux, uy, uz, rinv, gx, gy, gz);
                     grow[jj * 3 + 0] += gx; grow[jj * 3 + 1] += gy; grow[jj * 3 + 2] += gz;
                     fx += gx; fy += gy; fz += gz;
                     vir[0] -= gx * x; vir[1] -= gx * y; vir[2] -= gx * z;

@@ -143,7 +143,22 @@ __device__ __forceinline__ void cos_sin_pi(T t, T& c, T& s)
     c = quarter_sine((T)1 - (t + t));
     s = quarter_sine(m + m);
 }
-__device__ __forceinline__ float tanh_t(float x) { return tanhf(x); }
+// tanh: below 0.7 x + x^3 p(x^2), p of least relative error (1.6e-8), else 1 - 2 / (exp(2 |x|) + 1) by the chip's exp2 and
+// reciprocal; both and a choice, 20 operations.  The library's takes a branch for either side and an argument of exp in two parts,
+// 35 operations of which a wavefront with both kinds of argument issues all; both are within 1.6 units of the last place, with
+// 1.8e-8 for the mean error.
+__device__ __forceinline__ float tanh_t(float x)
+{
+    const float a = fabsf(x), y = a * a;
+    float p = -0.00513857882f;
+    p = p * y + 0.0200918801f;
+    p = p * y - 0.0535588302f;
+    p = p * y + 0.133291095f;
+    p = p * y - 0.333331913f;
+    const float small = a * y * p + a;
+    const float large = 1.0f - 2.0f * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(a * 2.88539008f) + 1.0f);
+    return copysignf(a < 0.7f ? small : large, x);
+}
 __device__ __forceinline__ double tanh_t(double x) { return tanh(x); }
 __device__ __forceinline__ float sqrt_t(float x) { return sqrtf(x); }
 __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
@@ -175,86 +190,121 @@ __device__ __forceinline__ void radial_basis(T r, T rc_inv, int K, T (&f)[KC], T
     }
 }
 
-// b_lm(u) for unit vector u, flat index l*l-1+mp (nep_utilities.h:110-203 with r = 1)
+// h = fc / 2 and T_k, so that f_k = h (T_k + 1): for sums of the functions themselves, sum h T_k + sum h.
+template <typename T, int KC>
+__device__ __forceinline__ T radial_terms(T r, T rc_inv, T (&t)[KC])
+{
+    const T u = r * rc_inv;
+    const T xr = u - (T)1;
+    const T x = (T)2 * xr * xr - (T)1, x2 = x + x;
+    T cs, sn;
+    cos_sin_pi(u, cs, sn);
+    t[0] = (T)1; t[1] = x;
+#pragma unroll
+    for (int k = 2; k < KC; k++) t[k] = x2 * t[k - 1] - t[k - 2];
+    return (T)0.25 * cs + (T)0.25;
+}
+
+// b_lm(u) for unit vector u, flat index l*l-1+mp (nep_utilities.h:110-203 with r = 1).  With C_m + i S_m = (x + i y)^m the pair
+// of mp = 2 m - 1, 2 m is C_m and S_m times a polynomial in z of degree l - m: 37 operations for the 24 of l <= 4.
 template <typename T, int LC>
 __device__ __forceinline__ void blm_values(T x, T y, T z, T (&b)[LC * LC + 2 * LC])
 {
-    const T x2 = x * x, y2 = y * y, z2 = z * z;
+    const T z2 = z * z, c2 = x * x - y * y, s2 = (x + x) * y;
     if (LC >= 1) { b[0] = z; b[1] = x; b[2] = y; }
     if (LC >= 2) {
-        b[3] = (T)3 * z2 - (T)1; b[4] = x * z; b[5] = y * z; b[6] = x2 - y2; b[7] = (T)2 * x * y;
+        b[3] = (T)3 * z2 - (T)1; b[4] = x * z; b[5] = y * z; b[6] = c2; b[7] = s2;
     }
+    const T c3 = x * c2 - y * s2, s3 = x * s2 + y * c2;
     if (LC >= 3) {
-        b[8] = ((T)5 * z2 - (T)3) * z;
-        b[9] = ((T)5 * z2 - (T)1) * x;
-        b[10] = ((T)5 * z2 - (T)1) * y;
-        b[11] = (x2 - y2) * z;
-        b[12] = (T)2 * x * y * z;
-        b[13] = (x2 - (T)3 * y2) * x;
-        b[14] = ((T)3 * x2 - y2) * y;
+        const T p1 = (T)5 * z2 - (T)1;
+        b[8] = (p1 - (T)2) * z; b[9] = p1 * x; b[10] = p1 * y; b[11] = c2 * z; b[12] = s2 * z; b[13] = c3; b[14] = s3;
     }
     if (LC >= 4) {
+        const T p1 = ((T)7 * z2 - (T)3) * z, p2 = (T)7 * z2 - (T)1;
         b[15] = ((T)35 * z2 - (T)30) * z2 + (T)3;
-        b[16] = ((T)7 * z2 - (T)3) * x * z;
-        b[17] = ((T)7 * z2 - (T)3) * y * z;
-        b[18] = ((T)7 * z2 - (T)1) * (x2 - y2);
-        b[19] = ((T)7 * z2 - (T)1) * (T)2 * x * y;
-        b[20] = (x2 - (T)3 * y2) * x * z;
-        b[21] = ((T)3 * x2 - y2) * y * z;
-        b[22] = (x2 - y2) * (x2 - y2) - (T)4 * x2 * y2;
-        b[23] = (T)4 * (x2 - y2) * x * y;
+        b[16] = p1 * x; b[17] = p1 * y; b[18] = p2 * c2; b[19] = p2 * s2; b[20] = c3 * z; b[21] = s3 * z;
+        b[22] = c2 * c2 - s2 * s2; b[23] = (c2 + c2) * s2;
     }
 }
 
-// w += sum_lm a[lm] * grad b_lm(u): Cartesian gradients of the homogeneous polynomials
-// b_lm, evaluated on the unit sphere (nep_utilities.h:206-379 with r = 1)
+// Gradient of sum_lm a[lm] b_lm, the b_lm as blm_values forms them.  They are the solid harmonics on the unit sphere only, so
+// what counts is the part across u (across()).  With P_m(z), Q_m(z) the sums of the a[lm] that go with C_m and S_m it is
+//   x: sum m (C_{m-1} P_m + S_{m-1} Q_m),  y: sum m (C_{m-1} Q_m - S_{m-1} P_m),  z: sum C_m P_m' + S_m Q_m'
+// Some 60 operations; the gradients of the homogeneous polynomials (nep_utilities.h:206-379) taken one by one are 150.
 template <typename T, int LC>
-__device__ __forceinline__ void blm_grad_dot(T x, T y, T z, const T (&a)[LC * LC + 2 * LC], T& wx,
-                                             T& wy, T& wz)
+__device__ __forceinline__ void blm_gradient(T x, T y, T z, const T (&a)[LC * LC + 2 * LC], T& wx, T& wy, T& wz)
 {
-    const T x2 = x * x, y2 = y * y, z2 = z * z;
-    const T xy = x * y, xz = x * z, yz = y * z;
-    if (LC >= 1) { wz += a[0]; wx += a[1]; wy += a[2]; }
+    const T z2 = z * z, c2 = x * x - y * y, s2 = (x + x) * y;
+    const T c3 = x * c2 - y * s2, s3 = x * s2 + y * c2;
+    T P1 = a[1], Q1 = a[2];                                   // m = 1
+    wz = a[0];
+    T dP1 = (T)0, dQ1 = (T)0;
     if (LC >= 2) {
-        wx += a[3] * ((T)-2 * x) + a[4] * z + a[6] * ((T)2 * x) + a[7] * ((T)2 * y);
-        wy += a[3] * ((T)-2 * y) + a[5] * z - a[6] * ((T)2 * y) + a[7] * ((T)2 * x);
-        wz += a[3] * ((T)4 * z) + a[4] * x + a[5] * y;
+        P1 += a[4] * z; Q1 += a[5] * z;
+        wz += a[3] * ((T)6 * z);
+        dP1 = a[4]; dQ1 = a[5];
     }
     if (LC >= 3) {
-        const T c = (T)5 * z2 - (T)1;
-        wx += a[8] * ((T)-6 * xz) + a[9] * (c - (T)2 * x2) + a[10] * ((T)-2 * xy) +
-              a[11] * ((T)2 * xz) + a[12] * ((T)2 * yz) + a[13] * ((T)3 * (x2 - y2)) +
-              a[14] * ((T)6 * xy);
-        wy += a[8] * ((T)-6 * yz) + a[9] * ((T)-2 * xy) + a[10] * (c - (T)2 * y2) +
-              a[11] * ((T)-2 * yz) + a[12] * ((T)2 * xz) + a[13] * ((T)-6 * xy) +
-              a[14] * ((T)3 * (x2 - y2));
-        wz += a[8] * ((T)9 * z2 - (T)3) + a[9] * ((T)8 * xz) + a[10] * ((T)8 * yz) +
-              a[11] * (x2 - y2) + a[12] * ((T)2 * xy);
+        const T p1 = (T)5 * z2 - (T)1, d1 = (T)10 * z;
+        P1 += a[9] * p1; Q1 += a[10] * p1;
+        wz += a[8] * ((T)15 * z2 - (T)3);
+        dP1 += a[9] * d1; dQ1 += a[10] * d1;
     }
     if (LC >= 4) {
-        const T z3 = z2 * z, x3 = x2 * x, y3 = y2 * y;
-        const T c73 = (T)7 * z3 - (T)3 * z;
-        wx += a[15] * ((T)-60 * x * z2 + (T)12 * x) + a[16] * ((T)-6 * x2 * z + c73) +
-              a[17] * ((T)-6 * xy * z) +
-              a[18] * ((T)-2 * x3 + (T)2 * x * y2 + (T)14 * x * z2 - (T)2 * x) +
-              a[19] * ((T)-4 * x2 * y + (T)14 * y * z2 - (T)2 * y) + a[20] * ((T)3 * (x2 - y2) * z) +
-              a[21] * ((T)6 * xy * z) + a[22] * ((T)4 * x3 - (T)12 * x * y2) +
-              a[23] * ((T)12 * x2 * y - (T)4 * y3);
-        wy += a[15] * ((T)-60 * y * z2 + (T)12 * y) + a[16] * ((T)-6 * xy * z) +
-              a[17] * ((T)-6 * y2 * z + c73) +
-              a[18] * ((T)-2 * x2 * y + (T)2 * y3 - (T)14 * y * z2 + (T)2 * y) +
-              a[19] * ((T)-4 * x * y2 + (T)14 * x * z2 - (T)2 * x) + a[20] * ((T)-6 * xy * z) +
-              a[21] * ((T)3 * (x2 - y2) * z) + a[22] * ((T)4 * y3 - (T)12 * x2 * y) +
-              a[23] * ((T)4 * x3 - (T)12 * x * y2);
-        wz += a[15] * ((T)80 * z3 - (T)48 * z) + a[16] * ((T)15 * x * z2 - (T)3 * x) +
-              a[17] * ((T)15 * y * z2 - (T)3 * y) + a[18] * ((T)12 * z * (x2 - y2)) +
-              a[19] * ((T)24 * xy * z) + a[20] * ((x2 - (T)3 * y2) * x) +
-              a[21] * (((T)3 * x2 - y2) * y);
+        const T p1 = ((T)7 * z2 - (T)3) * z, d1 = (T)21 * z2 - (T)3;
+        P1 += a[16] * p1; Q1 += a[17] * p1;
+        wz += a[15] * (((T)140 * z2 - (T)60) * z);
+        dP1 += a[16] * d1; dQ1 += a[17] * d1;
     }
+    wx = P1; wy = Q1;
+    if (LC >= 2) wz += x * dP1 + y * dQ1;
+    if (LC >= 2) {
+        T P2 = a[6], Q2 = a[7];
+        if (LC >= 3) { P2 += a[11] * z; Q2 += a[12] * z; }
+        if (LC >= 4) { const T p2 = (T)7 * z2 - (T)1; P2 += a[18] * p2; Q2 += a[19] * p2; }
+        const T x2 = x + x, y2 = y + y;
+        wx += x2 * P2 + y2 * Q2;
+        wy += x2 * Q2 - y2 * P2;
+    }
+    if (LC >= 3) {
+        T P3 = a[13], Q3 = a[14], dP2 = a[11], dQ2 = a[12];
+        if (LC >= 4) {
+            const T d2 = (T)14 * z;
+            P3 += a[20] * z; Q3 += a[21] * z;
+            dP2 += a[18] * d2; dQ2 += a[19] * d2;
+        }
+        wz += c2 * dP2 + s2 * dQ2;
+        const T c23 = (T)3 * c2, s23 = (T)3 * s2;
+        wx += c23 * P3 + s23 * Q3;
+        wy += c23 * Q3 - s23 * P3;
+    }
+    if (LC >= 4) {
+        wz += c3 * a[20] + s3 * a[21];
+        const T c34 = (T)4 * c3, s34 = (T)4 * s3;
+        wx += c34 * a[22] + s34 * a[23];
+        wy += c34 * a[23] - s34 * a[22];
+    }
+}
+
+// The compiler forms what depends on x from here on anew, instead of holding what blm_values has formed of it already (the
+// kernels whose registers are full).
+template <typename T>
+__device__ __forceinline__ void forget(T& x, T& y, T& z) { asm volatile("" : "+v"(x), "+v"(y), "+v"(z)); }
+
+// Derivative along the pair vector of a function g(r) b(u): `along` = g' b for its length, w = g grad b for its direction, of
+// which the part across u counts: along u + (w - (w . u) u) / r.
+template <typename T>
+__device__ __forceinline__ void pair_gradient(T along, T wx, T wy, T wz, T ux, T uy, T uz, T rinv, T& gx, T& gy, T& gz)
+{
+    const T s = along - (wx * ux + wy * uy + wz * uz) * rinv;
+    gx = s * ux + wx * rinv;
+    gy = s * uy + wy * rinv;
+    gz = s * uz + wz * rinv;
 }
 
 // d[lm] = w . grad b_lm(u): the directional derivative of every homogeneous polynomial b_lm along
-// w, evaluated on the unit sphere (the same gradients as blm_grad_dot, taken apart per lm)
+// w, evaluated on the unit sphere (the gradients of nep_utilities.h:206-379 with r = 1)
 template <typename T, int LC>
 __device__ __forceinline__ void blm_dir_derivs(T x, T y, T z, T wx, T wy, T wz, T (&d)[LC * LC + 2 * LC])
 {

@@ -613,13 +613,11 @@ nep_quad_kernel(const WaveArgs<T>)
                         }
                         srad += dg[c] * tc;
                     }
-                    T wx = (T)0, wy = (T)0, wz = (T)0;
-                    blm_grad_dot<T, LC>(ux, uy, uz, P, wx, wy, wz);
-                    const T along = srad - (wx * ux + wy * uy + wz * uz) * rinv;
+                    T wx, wy, wz;
+                    forget(ux, uy, uz);
+                    blm_gradient<T, LC>(ux, uy, uz, P, wx, wy, wz);
                     T* const rw = L.ang + lane * 3;
-                    rw[0] = along * ux + wx * rinv;
-                    rw[1] = along * uy + wy * rinv;
-                    rw[2] = along * uz + wz * rinv;
+                    pair_gradient(srad, wx, wy, wz, ux, uy, uz, rinv, rw[0], rw[1], rw[2]);
                 }
                 wave_sync();
                 // -- lane = neighbour of the atom: the radial part, the pair's force; behind the last angular pairs also the

@@ -633,19 +633,16 @@ nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, int* __r
                     for (int k = 0; k < 4; k++) { g += c1v[k] * f[4 + k]; dg += c1v[k] * df[4 + k]; }
 #pragma unroll
                     for (int m = 0; m < NLM; m++) { A[m] += S[n][m] * g; Ad[m] += S[n][m] * dg; }
+                    if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
                 }
                 T bl[NLM];
                 blm_values<T, LC>(ux, uy, uz, bl);
 #pragma unroll
-                for (int l = 1; l <= LC; l++)
-#pragma unroll
-                    for (int mp = 0; mp < 2 * l + 1; mp++) {
-                        const int m = l * l - 1 + mp;
-                        srad += (Ad[m] - (T)l * rinv * A[m]) * bl[m];
-                    }
-                T wx = (T)0, wy = (T)0, wz = (T)0;
-                blm_grad_dot<T, LC>(ux, uy, uz, A, wx, wy, wz);
-                emit(store, valid, place, x, y, z, srad * ux + wx * rinv, srad * uy + wy * rinv, srad * uz + wz * rinv);
+                for (int m = 0; m < NLM; m++) srad += Ad[m] * bl[m];
+                T wx, wy, wz, gx, gy, gz;
+                blm_gradient<T, LC>(ux, uy, uz, A, wx, wy, wz);
+                pair_gradient(srad, wx, wy, wz, ux, uy, uz, rinv, gx, gy, gz);
+                emit(store, valid, place, x, y, z, gx, gy, gz);
             });
         };
         if (seg_g) pass2(std::true_type{});

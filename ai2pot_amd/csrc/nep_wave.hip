@@ -384,19 +384,12 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
                 for (int k = 0; k < 4; k++) { g += c1[k] * f[4 + k]; dg += c1[k] * df[4 + k]; }
                 T bl[NLM];
                 blm_values<T, LC>(ux, uy, uz, bl);
-                T srad = (T)0;
+                T sb = (T)0, wx, wy, wz, gx, gy, gz;
 #pragma unroll
-                for (int l = 1; l <= LC; l++) {
-                    T sl = (T)0;
-#pragma unroll
-                    for (int mp = 0; mp < 2 * l + 1; mp++) sl += S[l * l - 1 + mp] * bl[l * l - 1 + mp];
-                    srad += (dg - (T)l * rinv * g) * sl;
-                }
-                T wx = (T)0, wy = (T)0, wz = (T)0;
-                blm_grad_dot<T, LC>(ux, uy, uz, S, wx, wy, wz);
-                const T gr = g * rinv;
-                const T gx = quad_sum(srad * ux + wx * gr), gy = quad_sum(srad * uy + wy * gr),
-                        gz = quad_sum(srad * uz + wz * gr);
+                for (int m = 0; m < NLM; m++) sb += S[m] * bl[m];
+                blm_gradient<T, LC>(ux, uy, uz, S, wx, wy, wz);
+                pair_gradient(dg * sb, wx, wy, wz, ux, uy, uz, g * rinv, gx, gy, gz);
+                gx = quad_sum(gx); gy = quad_sum(gy); gz = quad_sum(gz);
                 if (e < nA && chan == 0) { L.ang[e * 3] = gx; L.ang[e * 3 + 1] = gy; L.ang[e * 3 + 2] = gz; }
             }
             __builtin_amdgcn_wave_barrier();
