@@ -20,6 +20,10 @@
 //                        are gathered and nothing is stored per pair; then the slots of the atom are summed
 //                        (in fixed point, so that the result does not depend on which pair got which
 //                        place) and the force is written.
+// What bounds the first is the issue of vector instructions (0.97 of its cycles), the second the texture path.  Neither may keep
+// anything in scratch memory: a wavefront's few spilled values are written to HBM and read again, 16,384 wavefronts of them
+// (1,048,576 atoms, 3 species, fp32: 584 -> 546 and 331 -> 322 us by taking the last 24 and 16 bytes a lane out; 200 and 36 bytes
+// for a list's first chunk on its way earlier cost 100 and 55 us).
 // Atoms are processed in the Morton order of the list build and workgroups are dealt to the XCDs in contiguous
 // runs.  The lists are read in 8 KiB chunks (8 slots of 64 positions), staged through LDS by each wavefront
 // for itself: global loads are contiguous, LDS reads are one 16-byte entry per lane.
@@ -40,6 +44,8 @@ namespace {
 constexpr int CB = 256;                 // positions (threads) per workgroup
 constexpr int KC = 8, NAC = 4, LC = 4, NLM = 24, FDP = 24;
 constexpr int NSLOT = 32;               // depth of the slot array: places 0 .. NSLOT-1 of every atom
+constexpr int SLOTS_AT_ONCE = 4;
+static_assert(NSLOT % SLOTS_AT_ONCE == 0, "a batch ends with the array");
 constexpr int STP = CL_CHUNK + 1;       // staged slots per position, padded: 16-byte reads of 8 lanes hit 8 banks
 
 template <typename T>
@@ -154,23 +160,22 @@ __device__ __forceinline__ void chunk_store(T* __restrict__ st, int lane, const 
 
 // Walks one of the two lists of the wavefront's 64 positions: chunk after chunk through the staging
 // buffer, every lane making the trips of the longest list; body(valid, x, y, z, bits).  A lane past
-// the end of its own list gets a unit vector and valid = false.  With AHEAD the next chunk is requested
+// the end of its own list gets a unit vector and valid = false.  The next chunk is requested
 // before the trips of the current one and waits in registers (32 of them) meanwhile.
-template <typename T, bool AHEAD = false, typename Body>
+template <typename T, typename Body>
 __device__ __forceinline__ void walk_list(const CompactView<T>& cv, int tile, int lane, T* st, int n, bool inner,
                                           Body&& body)
 {
     const int trips = __builtin_amdgcn_readfirstlane(wave_max(n));
     T v[CL_CHUNK][4];
-    if (AHEAD && trips > 0)
+    if (trips > 0)
         chunk_load<T>(cv.entries + compact_chunk_offset<T>(cv.nch, tile, inner ? cv.nch - 1 : 0), lane, v);
     for (int c = 0; c * CL_CHUNK < trips; c++) {
         const int chunk = inner ? cv.nch - 1 - c : c;
-        if (!AHEAD) chunk_load<T>(cv.entries + compact_chunk_offset<T>(cv.nch, tile, chunk), lane, v);
         __builtin_amdgcn_wave_barrier();
         chunk_store<T>(st, lane, v);
         __builtin_amdgcn_wave_barrier();
-        if (AHEAD && (c + 1) * CL_CHUNK < trips)
+        if ((c + 1) * CL_CHUNK < trips)
             chunk_load<T>(cv.entries + compact_chunk_offset<T>(cv.nch, tile, inner ? chunk - 1 : chunk + 1), lane, v);
         for (int s = 0; s < CL_CHUNK; s++) {
             const int e = c * CL_CHUNK + s;
@@ -183,24 +188,46 @@ __device__ __forceinline__ void walk_list(const CompactView<T>& cv, int tile, in
     }
 }
 
-// position -> atom, species, list lengths; with the checks
-template <typename T>
-__device__ __forceinline__ bool position_header(const GatherArgs<T>& a, int p, int& atom, int& ti, int& n_outer,
-                                                int& n_inner)
+// A table into LDS by the workgroup, eight values of a thread on their way together.
+template <int NTHREADS, typename T, typename Get>
+__device__ __forceinline__ void stage(T* dst, int n, int tid, Get&& get)
 {
-    atom = 0; ti = 0; n_outer = 0; n_inner = 0;
-    if (p >= a.cv.natoms) return false;
-    atom = a.cv.order[p];
-    if ((unsigned)atom >= (unsigned)a.cv.natoms) { atomicOr(a.status, ST_BAD_NEIGHBOR); atom = 0; return false; }
-    ti = a.types[atom];
-    if ((unsigned)ti >= (unsigned)a.ntypes) { atomicOr(a.status, ST_BAD_TYPE); ti = 0; return false; }
-    n_outer = a.cv.n_outer[p];
-    n_inner = a.cv.n_inner[p];
-    if (n_outer < 0 || n_inner < 0 || n_outer + n_inner > a.cv.umax) {
-        atomicOr(a.status, ST_NEIGH_OVERFLOW);
-        n_outer = 0; n_inner = 0;
+    for (int i0 = tid; i0 < n; i0 += 8 * NTHREADS) {
+        T v[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v[u] = get(min(i0 + u * NTHREADS, n - 1));
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (i0 + u * NTHREADS < n) dst[i0 + u * NTHREADS] = v[u];
     }
-    return true;
+}
+
+// position -> atom, species, list lengths; with the checks.  (Returned as a value: references to the caller's variables, set on
+// several ways out, keep these in scratch memory, which goes out to HBM and back.)
+struct Header {
+    bool active;
+    int atom, ti, n_outer, n_inner;
+};
+template <typename T>
+__device__ __forceinline__ Header position_header(const GatherArgs<T>& a, int p)
+{
+    Header h = {false, 0, 0, 0, 0};
+    const bool inside = p < a.cv.natoms;
+    const int at = inside ? a.cv.order[p] : 0, no = inside ? a.cv.n_outer[p] : 0, ni = inside ? a.cv.n_inner[p] : 0;
+    const bool named = (unsigned)at < (unsigned)a.cv.natoms;
+    const int ti = inside && named ? a.types[at] : 0;
+    const bool known = (unsigned)ti < (unsigned)a.ntypes, fits = no >= 0 && ni >= 0 && no + ni <= a.cv.umax;
+    int bad = 0;
+    if (!named) bad = ST_BAD_NEIGHBOR;
+    else if (!known) bad = ST_BAD_TYPE;
+    else if (!fits) bad = ST_NEIGH_OVERFLOW;
+    if (inside && bad) atomicOr(a.status, bad);
+    h.active = inside && named && known;
+    h.atom = named ? at : 0;
+    h.ti = h.active ? ti : 0;
+    h.n_outer = h.active && fits ? no : 0;
+    h.n_inner = h.active && fits ? ni : 0;
+    return h;
 }
 
 // Exact, order-independent sum of a few floating-point values: fixed point in 64-bit integers.
@@ -461,13 +488,13 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int p = blk * CB + tid;
-    const int tile = p >> 6;
+    const int tile = __builtin_amdgcn_readfirstlane(p >> 6);
     const int nt = a.ntypes, H = a.H;
     AdjointLds<T> L;
     adjoint_lds<T>(nt, NTC, H, NB, smem_raw, L, HM);
     T* const st = L.stage + (size_t)wv * 64 * STP * 4;
 
-    for (int i = tid; i < nt * nt * NB * KC; i += CB) L.coef[i] = a.coeffs[i];
+    stage<CB>(L.coef, nt * nt * NB * KC, tid, [&](int i) { return a.coeffs[i]; });
     if constexpr (HM) {
         // [species][HM_HP neurons][FDP] and its transpose [species][FDP][HM_HPT], zeros beyond H and DC
         for (int i = tid; i < nt * HM_HP * FDP; i += CB) {
@@ -482,16 +509,15 @@ nep_adjoint_kernel(const GatherArgs<T> a)
             L.w1[i] = n < H ? a.w1[t * H + n] : (T)0;
         }
     } else {
-        for (int i = tid; i < nt * H * FDP; i += CB) {
+        stage<CB>(L.w0, nt * H * FDP, tid, [&](int i) {
             const int r = i / FDP, j = i - r * FDP;
-            L.w0[i] = j < DC ? a.w0[(size_t)r * DC + j] : (T)0;
-        }
+            return j < DC ? a.w0[r * DC + j] : (T)0;
+        });
         for (int i = tid; i < nt * H; i += CB) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
     }
     if (tid < FDP) L.qs[tid] = tid < DC ? (T)1 / a.q_scaler[tid] : (T)0;
 
-    int atom, ti, n_outer, n_inner;
-    const bool active = position_header<T>(a, p, atom, ti, n_outer, n_inner);
+    const auto [active, atom, ti, n_outer, n_inner] = position_header<T>(a, p);
     const T rr_inv = (T)1 / a.rr, ra_inv = (T)1 / a.ra;
 
     T F[NTC][KC];                 // radial functions summed per neighbour species
@@ -519,7 +545,7 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     __syncthreads();
 
     // neighbours inside the angular cutoff: radial sums and angular moments
-    walk_list<T, true>(a.cv, tile, lane, st, n_inner, true, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
+    walk_list<T>(a.cv, tile, lane, st, n_inner, true, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
         const int tj = min((bits >> CL_TYPE_SHIFT) & 15, nt - 1);
         T rinv;
         const T r = length<false>(x * x + y * y + z * z, rinv);
@@ -545,7 +571,8 @@ nep_adjoint_kernel(const GatherArgs<T> a)
         }
     });
     // neighbours between the cutoffs: radial sums only
-    walk_list<T, true>(a.cv, tile, lane, st, n_outer, false, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
+    const bool derivs = a.force || a.want_virial;
+    walk_list<T>(a.cv, tile, lane, st, n_outer, false, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
         const int tj = min((bits >> CL_TYPE_SHIFT) & 15, nt - 1);
         T unused;
         const T r = length<false>(x * x + y * y + z * z, unused);
@@ -674,9 +701,9 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     T vir[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) vir[i] = (T)0;
-    if (a.force || a.want_virial) {
+    if (derivs) {
         const bool hand_over = a.force != nullptr;
-        walk_list<T, true>(a.cv, tile, lane, st, n_inner, true, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
+        walk_list<T>(a.cv, tile, lane, st, n_inner, true, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
             int j = bits & CL_INDEX_MASK;
             if (valid && j >= a.cv.natoms) { atomicOr(a.status, ST_BAD_NEIGHBOR); valid = false; }
             if (!valid) return;
@@ -699,7 +726,8 @@ nep_adjoint_kernel(const GatherArgs<T> a)
             const T* ci = L.coef + ((ti * nt + tj) * NB + NR) * KC;
             // the channels' moments' adjoints: A = sum g_n s_n for the direction, sum g_n' (s_n . b) for the length.  (Vector
             // operations of a pair 654 -> 532 by that and blm_gradient; 1,048,576 atoms with the sums of h T_k above and tanh_t:
-            // 19,070 -> 17,360 of a wavefront, kernel 606 -> 584 us.)
+            // 19,070 -> 17,360 of a wavefront, kernel 606 -> 584 us.)  The channels one after the other: mixed by the compiler they
+            // hold the coefficients of all four, and what does not fit the registers goes to scratch memory.
             T A[NLM], bl[NLM];
             if (sizeof(T) == 8) forget(ux, uy, uz);
             blm_values<T, LC>(ux, uy, uz, bl);
@@ -719,7 +747,7 @@ nep_adjoint_kernel(const GatherArgs<T> a)
 #pragma unroll
                 for (int m = 0; m < NLM; m++) { A[m] += S[n][m] * g; sb += S[n][m] * bl[m]; }
                 srad += dg * sb;
-                if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_sched_barrier(0);
             }
             T wx, wy, wz, gx, gy, gz, vx = ux, vy = uy, vz = uz;
             if (sizeof(T) == 8) forget(vx, vy, vz);
@@ -784,14 +812,14 @@ nep_gather_kernel(const GatherArgs<T> a)
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int blk = xcd_block(blockIdx.x, gridDim.x);
     const int p = blk * CB + tid;
-    const int tile = p >> 6;
+    const int tile = __builtin_amdgcn_readfirstlane(p >> 6);
     const int nt = a.ntypes;
     GatherLds<T> L;
     gather_lds<T>(smem_raw, L);
     T* const st = L.stage + (size_t)wv * 64 * STP * 4;
 
-    int atom, ti, n_outer, n_inner;
-    const bool active = position_header<T>(a, p, atom, ti, n_outer, n_inner);
+    const int claimed = p < a.cv.natoms && a.force ? a.incoming[p] : 0;
+    const auto [active, atom, ti, n_outer, n_inner] = position_header<T>(a, p);
     const T rr_inv = (T)1 / a.rr;
 
     // own contracted radial coefficients, one array per neighbour species (separate arrays: a select between
@@ -810,7 +838,7 @@ nep_gather_kernel(const GatherArgs<T> a)
 #pragma unroll
     for (int i = 0; i < 9; i++) vir[i] = (T)0;
     // g_ij - g_ji = (cc_i[t_j] + cc_j[t_i]) . f'(r) r_ij / r
-    walk_list<T, true>(a.cv, tile, lane, st, n_outer, false, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
+    walk_list<T>(a.cv, tile, lane, st, n_outer, false, [&](bool valid, T x, T y, T z, int bits) __attribute__((always_inline)) {
         const int j = bits & CL_INDEX_MASK;
         if (valid && j >= a.cv.natoms) { atomicOr(a.status, ST_BAD_NEIGHBOR); valid = false; }
         if (!valid) return;                  // lanes past the end of their list issue no loads
@@ -840,15 +868,22 @@ nep_gather_kernel(const GatherArgs<T> a)
 
     // what the neighbours inside the angular cutoff handed over: F_i -= sum_j g_ji
     if (p < a.cv.natoms && a.force) {
-        const int n = a.incoming[p];
+        const int n = claimed;
         a.incoming[p] = 0;                                  // the next call finds the counters at zero
         FixedSum<T> sx, sy, sz;
         double mag = 0.0;                                   // NaN or inf in a slot makes this NaN or inf
-        for (int t = 0; t < min(n, NSLOT); t++) {
-            T v[4];
-            ld4_stream(a.slots + ((size_t)t * a.cv.natoms + p) * 4, v);        // read once
-            mag += fabs((double)v[0]) + fabs((double)v[1]) + fabs((double)v[2]);
-            sx.add(v[0]); sy.add(v[1]); sz.add(v[2]);
+        // SLOTS_AT_ONCE of them on their way together: one after the other each waits for a trip to memory
+        for (int t0 = 0; t0 < min(n, NSLOT); t0 += SLOTS_AT_ONCE) {
+            T s[SLOTS_AT_ONCE][4];
+#pragma unroll
+            for (int u = 0; u < SLOTS_AT_ONCE; u++)
+                if (t0 + u < n) ld4_stream(a.slots + ((size_t)(t0 + u) * a.cv.natoms + p) * 4, s[u]);        // read once
+#pragma unroll
+            for (int u = 0; u < SLOTS_AT_ONCE; u++)
+                if (t0 + u < n) {
+                    mag += fabs((double)s[u][0]) + fabs((double)s[u][1]) + fabs((double)s[u][2]);
+                    sx.add(s[u][0]); sy.add(s[u][1]); sz.add(s[u][2]);
+                }
         }
         bool ok = mag < kFixedSumLimit;
         if (n > NSLOT) {
