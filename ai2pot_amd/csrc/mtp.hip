@@ -26,6 +26,7 @@
 #include "wave_ops.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -476,46 +477,109 @@ __device__ __forceinline__ T plan_entry(const T* base, unsigned off)
     return *(const T*)((const char*)base + (sizeof(T) == 8 ? off : off >> 1));
 }
 
-// A gather (mtp_plan.h: MtpStream): terms(words, leaf) for two terms of the thread's slot and done(slot, rem, steps, leaf)
-// behind the last of a group; a barrier behind every level.  What bounds it is the number of instructions a wavefront issues
-// one after the other, so the plan holds everything in the order of use; the words of the next two steps are on their way
-// meanwhile, also across a barrier (the plan does not depend on the moments).  Looking up each group's place, depth and moment
-// when its turn comes took 280 instead of 260 us for the whole kernel at level 20, 8192 atoms, 217 instead of 203 for the loss
-// gradient and 193 instead of 176 for the columns of the linear solver (level 16, 64 structures of 128 atoms).
+// A gather (mtp_plan.h: MtpStream): terms(words, leaf, next) for a step, with next() where it has read its words, and done(moment,
+// rem, steps, leaf) behind the last of a group; a barrier behind every level.  What bounds it is the instructions a wavefront issues
+// one after the other and, with few wavefronts, the way of a step through one, so the plan holds everything in the order of use, and
+// the words of the next two steps are on their way, also across a barrier (the plan does not depend on the moments).
+// That takes some care, or the compiler waits for what it has only just asked for: every load of the loop is made in every step
+// (with one that only some make, the next group's moments or control words, it does not know how many lie behind the words it waits
+// for), the loop has one way out, what is loaded into is free by then (or it goes elsewhere, and copies wait for it), and none of a
+// load's registers is lent to something else meanwhile.  So a step brings its moments along in the multiplicities, the
+// control words of 64 steps lie in a vector register, and an odd step is walked ahead of the loop.
+// Energies and forces of level 20, 8192 atoms, 236 -> 224 us (216 atoms: 28.3 -> 26.9), of level 16, 64 structures of 128 atoms,
+// 90.3 -> 87.7, the loss gradient there 161 -> 159.5; with two products to a multiplicity (step_terms), 14 instead of 24 vector
+// instructions for the four of a step.  (The words of a step in an order that keeps the LDS free of bank conflicts, 1.2 lanes to a
+// bank instead of 2.1: no change.)
 template <typename Stream, typename Terms, typename Done>
 __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& done)
 {
+    typedef int int4_t __attribute__((ext_vector_type(4)));
+    struct Step { int4_t w[2]; };
     const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const A2P_CONSTANT int* const head = uniform_array((const int*)g.head) + wave * 4;
     const int first = head[0], n = head[1];
+    const A2P_CONSTANT char* at = (const A2P_CONSTANT char*)(const A2P_CONSTANT int4*)uniform_array(g.words + (size_t)first * MTP_STEP_WORDS);
+    const unsigned at_lane = (unsigned)lane * 16u;
+    auto load = [&](Step& s, int k) __attribute__((always_inline)) {       // (two steps behind the last)
+        s.w[0] = *(const A2P_CONSTANT int4_t*)(at + k * MTP_STEP_WORDS * 16 + at_lane);
+        s.w[1] = *(const A2P_CONSTANT int4_t*)(at + k * MTP_STEP_WORDS * 16 + 64 * 16 + at_lane);
+    };
+    // An odd step is walked ahead of the loop, which takes two at a time and has one way out (on another one the compiler sees
+    // the loads of one step alone behind the words it waits for).
+    const int odd = n & 1;
+    Step a, b, single;
+    int ctrl = 0;
+    if (n > 0) {                                       // in the order in which they are waited for
+        ctrl = g.ctrl[first + lane];                   // (64 words behind the last)
+        __builtin_amdgcn_sched_barrier(0);
+        if (odd) {
+            load(single, 0);
+            at += MTP_STEP_WORDS * 16;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        load(a, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(b, 1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     for (int k = head[3]; k > 0; k--) __syncthreads();
-    if (n == 0) return;
-    const A2P_CONSTANT int* ctrl = uniform_array(g.ctrl) + first;
-    const int* sp = g.slots + (size_t)head[2] * 64 + lane;
-    const int4* tp = g.words + (size_t)first * (MTP_DEPTH_STEP / 2 * 64) + lane;
-    int4 a[2], b[2];
-    int slot = sp[0], next_slot = sp[64];              // (each array ends with two steps' worth of padding)
-    a[0] = tp[0]; a[1] = tp[64];
-    b[0] = tp[128]; b[1] = tp[192];
-    auto step = [&](int4 (&w)[2], int i) __attribute__((always_inline)) {
-        const int c = ctrl[i];
-        if (c & MTP_CTRL_HALF) terms(w, std::integral_constant<int, 1>(), (c & MTP_CTRL_LEAF) != 0);
-        else terms(w, std::integral_constant<int, 2>(), (c & MTP_CTRL_LEAF) != 0);
-        w[0] = tp[256]; w[1] = tp[320];
-        tp += 128;
-        if (c & 1) {
-            done((slot & 0xffff) - 1, slot >> 16, (c >> 1) & 7, (c & MTP_CTRL_LEAF) != 0);
-            slot = next_slot;
-            sp += 64;
-            next_slot = sp[64];
+    auto step = [&](Step& s, int i, bool ahead) __attribute__((always_inline)) {
+        const int c = __builtin_amdgcn_readlane(ctrl, i);
+        int slot;
+        const bool leaf = (c & MTP_CTRL_LEAF) != 0;
+        terms(s.w, leaf, [&]() __attribute__((always_inline)) {
+            slot = s.w[0].z - 1;
+            // (w[1].z, of no use, keeps its register: given to another value, this one would wait for the load)
+            asm volatile("" : "+v"(slot) : "v"(s.w[1].z) : "memory");
+            if (!ahead) return;
+            load(s, 2);
+            at += MTP_STEP_WORDS * 16;
+            asm volatile("" : "+s"(at));               // (a lane's address formed anew each step takes no vector instruction)
+        });
+        if (__builtin_expect(c & 1, 0)) {
+            done((int)(short)slot, slot >> 16, (c >> 1) & 7, leaf);
             for (int k = c >> 4 & 0xffff; k > 0; k--) __syncthreads();
         }
     };
+    if (n == 0) return;
+    if (odd) step(single, 0, false);
+    for (int i = odd, base = 0; i < n; base = i) {
+        if (base > 0) ctrl = g.ctrl[first + base + lane];
+        asm volatile("" : "+v"(ctrl));                 // (waited for here, not in the loop)
+        const int end = min(n, base + 64 - (i - base));
 #pragma unroll 1
-    for (int i = 0; i < n; i += 2) {
-        step(a, i);
-        if (i + 1 == n) break;
-        step(b, i + 1);
+        for (; i < end; i += 2) {
+            step(a, i - base, true);
+            step(b, i - base + 1, true);
+        }
+    }
+}
+
+// The terms of a step, two pairs of products (mtp_plan.h): acc += mult (a[x0] b[y0] + a[x1] b[y1]), and, with BOTH,
+// tac += mult (ta[x0] b[y0] + a[x0] tb[y0] + ta[x1] b[y1] + a[x1] tb[y1]).  next() stands where the words have been read: the
+// multiplicities are taken out of them before, for words that are held beyond the load of the next ones send these to other
+// registers, and the copies at the end of a step wait for them.
+template <typename T, bool BOTH, typename Words, typename Next>
+__device__ __forceinline__ void step_terms(const Words (&w)[2], const T* a, const T* b, const T* ta, const T* tb, T& acc, T& tac, Next&& next)
+{
+    constexpr int C = MTP_DEPTH_STEP;
+    T v0[C], v1[C], t0[C], t1[C], mult[C / 2];
+#pragma unroll
+    for (int u = 0; u < C; u++) {
+        const unsigned x = u & 1 ? w[u / 2].y : w[u / 2].x, i0 = x & 0xffffu, i1 = x >> 16;
+        v0[u] = plan_entry(a, i0); v1[u] = plan_entry(b, i1);
+        if (BOTH) { t0[u] = plan_entry(ta, i0); t1[u] = plan_entry(tb, i1); }
+    }
+#pragma unroll
+    for (int u = 0; u < C / 2; u++) {
+        mult[u] = (T)__hiloint2double(w[u].w, 0);
+        asm volatile("" : "+v"(mult[u]));
+    }
+    next();
+#pragma unroll
+    for (int u = 0; u < C; u += 2) {
+        acc += mult[u / 2] * (v0[u] * v1[u] + v0[u + 1] * v1[u + 1]);
+        if (BOTH) tac += mult[u / 2] * ((t0[u] * v1[u] + v0[u] * t1[u]) + (t0[u + 1] * v1[u + 1] + v0[u + 1] * t1[u + 1]));
     }
 }
 
@@ -525,21 +589,8 @@ __device__ __forceinline__ void sweep_forward(Stream& g, T* M, T* Tg, int tid)
 {
     T acc = (T)0, tacc = (T)0;
     walk(g, tid,
-        [&](const int4 (&w)[2], auto count, bool) __attribute__((always_inline)) {
-            constexpr int C = 2 * decltype(count)::value;
-            T v0[C], v1[C], t0[C], t1[C];
-#pragma unroll
-            for (int u = 0; u < C; u++) {
-                const unsigned x = u & 1 ? w[u / 2].z : w[u / 2].x, m0 = x & 0xffffu, m1 = x >> 16;
-                v0[u] = plan_entry(M, m0); v1[u] = plan_entry(M, m1);
-                if (TANGENT) { t0[u] = plan_entry(Tg, m0); t1[u] = plan_entry(Tg, m1); }
-            }
-#pragma unroll
-            for (int u = 0; u < C; u++) {
-                const T mult = (T)(u & 1 ? w[u / 2].w : w[u / 2].y);
-                acc += mult * v0[u] * v1[u];
-                if (TANGENT) tacc += t0[u] * mult * v1[u] + t1[u] * mult * v0[u];
-            }
+        [&](const auto& w, bool, auto next) __attribute__((always_inline)) {
+            step_terms<T, TANGENT>(w, M, M, Tg, Tg, acc, tacc, next);
         },
         [&](int dst, int rem, int steps, bool) __attribute__((always_inline)) {
             if (steps) {
@@ -564,25 +615,8 @@ __device__ __forceinline__ void sweep_reverse(Stream& g, const T* M, T* A, T* X,
 {
     T acc = (T)0, xacc = (T)0;
     walk(g, tid,
-        [&](const int4 (&w)[2], auto count, bool leaf) __attribute__((always_inline)) {
-            constexpr int C = 2 * decltype(count)::value;
-            const T* const b0 = LEAF && leaf ? M : A;
-            const T* const b1 = LEAF && leaf ? Tg : X;
-            T v0[C], v1[C], t0[C], t1[C];
-#pragma unroll
-            for (int u = 0; u < C; u++) {
-                const unsigned x = u & 1 ? w[u / 2].z : w[u / 2].x, dst = x & 0xffffu, other = x >> 16;
-                v0[u] = plan_entry(b0, dst); v1[u] = plan_entry(M, other);
-                if (MIXED) { t0[u] = plan_entry(b1, dst); t1[u] = plan_entry(Tg, other); }
-            }
-#pragma unroll
-            for (int u = 0; u < C; u++) {
-                const T mult = (T)(u & 1 ? w[u / 2].w : w[u / 2].y);
-                if (MIXED) xacc += t0[u] * mult * v1[u];
-                const T a = v0[u] * mult;
-                acc += a * v1[u];
-                if (MIXED) xacc += a * t1[u];
-            }
+        [&](const auto& w, bool leaf, auto next) __attribute__((always_inline)) {
+            step_terms<T, MIXED>(w, LEAF && leaf ? M : A, M, LEAF && leaf ? Tg : X, Tg, acc, xacc, next);
         },
         [&](int src, int rem, int steps, bool leaf) __attribute__((always_inline)) {
             if (steps) {
@@ -2196,24 +2230,63 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         seen[mapping[s]] = 1;
     }
     A2P_REQUIRE(n_moms < 8192, A2P_ERR_INVALID, "mtp plan: more than 8191 moments");    // 16-bit byte offsets
-    // Packed terms of each moment, in the order given.
+    // Packed terms of each moment, in the order given; a list of products (mtp_plan.h) in pairs of the same multiplicity, whose
+    // lower half as a double is zero: one that takes more than 21 bits is the sum of two.
+    struct Term { int x; double mult; };
     struct Lists {
         std::vector<int> off;
-        std::vector<int2> terms;
-        Lists(int n, const std::vector<std::pair<int, int2>>& given) : off((size_t)n + 2, 0), terms(given.size())
+        std::vector<Term> terms;
+        int longest = 0;                                   // as given
+        Lists(int n, const std::vector<std::pair<int, Term>>& given, bool products)
         {
+            fill(n, given);
+            for (int m = 0; m < n; m++) longest = std::max(longest, size(m));
+            if (!products) return;
+            auto low = [](const Term& t) { return std::fabs(t.mult) < 1 << 20 ? 0.0 : std::fmod(t.mult, 2048.0); };
+            if (std::any_of(terms.begin(), terms.end(), [&](const Term& t) { return low(t) != 0.0; })) {
+                std::vector<std::pair<int, Term>> cut;
+                for (const auto& t : given) {
+                    const double l = low(t.second);
+                    cut.emplace_back(t.first, Term{t.second.x, t.second.mult - l});
+                    if (l != 0.0) cut.emplace_back(t.first, Term{t.second.x, l});
+                }
+                fill(n, cut);
+            }
+            std::vector<Term> pairs;
+            pairs.reserve(2 * terms.size());
+            for (int m = 0; m < n; m++) {
+                const auto begin = terms.begin() + off[m], end = terms.begin() + off[(size_t)m + 1];
+                if (end - begin > 32) std::stable_sort(begin, end, [](const Term& x, const Term& y) { return x.mult < y.mult; });
+                else                                       // (no buffer of its own)
+                    for (auto t = begin; t != end; ++t)
+                        for (auto u = t; u != begin && u->mult < (u - 1)->mult; --u) std::swap(*u, *(u - 1));
+                off[m] = (int)pairs.size();
+                for (auto t = begin; t != end; ++t) {
+                    pairs.push_back(*t);
+                    if ((pairs.size() - off[m]) % 2 == 0 || (t + 1 != end && (t + 1)->mult == t->mult)) continue;
+                    pairs.back().mult *= 0.5;              // (alone: twice, each time half)
+                    pairs.push_back(pairs.back());
+                }
+            }
+            off[n] = off[(size_t)n + 1] = (int)pairs.size();
+            terms = std::move(pairs);
+        }
+        void fill(int n, const std::vector<std::pair<int, Term>>& given)
+        {
+            off.assign((size_t)n + 2, 0);
+            terms.resize(given.size());
             for (const auto& t : given) off[(size_t)t.first + 2]++;
             for (int m = 0; m < n; m++) off[(size_t)m + 2] += off[(size_t)m + 1];
             for (const auto& t : given) terms[(size_t)off[(size_t)t.first + 1]++] = t.second;
         }
         int size(int m) const { return off[(size_t)m + 1] - off[m]; }
-        const int2* of(int m) const { return terms.data() + off[m]; }
+        const Term* of(int m) const { return terms.data() + off[m]; }
     };
     // Interleaved gather lists (see mtp_plan.h).
     struct Ell {
         std::vector<int> level, slot, lead;                // lead: pieces behind
         std::vector<int4> group;                           // first term, depth, doubling steps, MTP_CTRL_LEAF or 0
-        std::vector<int2> terms;
+        std::vector<Term> terms;
     };
     // Cuts the lists of one level into pieces of at most `cap` terms and lays them out in rows of sixteen lanes.
     struct Piece { int m, t0, n, rem; };
@@ -2232,7 +2305,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         int most = 0;
         for (int m : members) {
             const int n = lists.size(m), np = pieces_of(n, cap);
-            given.push_back({m, n, np, np > 1 ? (n + np - 1) / np : n});        // pieces of equal length
+            given.push_back({m, n, np, np > 1 ? deep((n + np - 1) / np) : n});        // pieces of equal length, of whole pairs
             most = std::max(most, np);
         }
         auto key = [&](const List& l) { return (cap - deep(l.len)) / 2 * (most + 1) + most - l.np; };
@@ -2274,13 +2347,13 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         while (lv.lanes.size() % 64) lv.lanes.push_back({-1, 0, 0, 0});
         return lv;
     };
-    // what a wavefront issues: a term about ten instructions, a group about 25, a doubling step about nine; the workgroup
+    // what a wavefront issues: a step of four terms about twenty instructions, a group about 25, a doubling step about nine; the workgroup
     // waits for its slowest wavefront, and the others' share is what other workgroups can use meanwhile
     auto level_cost = [](const Level& lv, int waves) {
         std::vector<double> load(waves, 0.0);
         double all = 0;
         for (size_t g = 0; g < lv.depth.size(); g++) {
-            const double c = 10.0 * lv.depth[g] + 25.0 + 9.0 * lv.steps[g];
+            const double c = 20.0 * ((lv.depth[g] + 3) / 4) + 25.0 + 9.0 * lv.steps[g];
             *std::min_element(load.begin(), load.end()) += c;
             all += c;
         }
@@ -2293,14 +2366,15 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         std::vector<int> ms;
         int longest = 0;
         for (int m : members) {
-            if (lists.size(m) > 64 * MTP_SLOT_CAP) { too_long = true; continue; }
             ms.push_back(m);
             longest = std::max(longest, lists.size(m));
         }
         double cost[2] = {-1, -1};
         int cut[2] = {MTP_SLOT_CAP, MTP_SLOT_CAP};
         long long pieces = -1;
-        for (int cap = 2; cap <= MTP_SLOT_CAP; cap += 2) {
+        if (lists.longest > 64 * MTP_SLOT_CAP) { too_long = true; return Best(); }
+        // (the longest lists hold more in pairs than as they were given)
+        for (int cap = 2; cap <= MTP_SLOT_CAP || cost[0] < 0; cap += 2) {
             if (longest > 64 * cap) continue;
             long long np = 0;
             for (int m : ms) np += pieces_of(lists.size(m), cap);
@@ -2328,7 +2402,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         auto append = [&](const Lists& lists, const Level& best, int kind) {
             for (size_t g = 0; g < best.depth.size(); g++) {
                 e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], kind));
-                e.terms.resize(e.terms.size() + (size_t)best.depth[g] * 64, make_int2(0, 0));
+                e.terms.resize(e.terms.size() + (size_t)best.depth[g] * 64, Term{0, 0.0});
                 for (size_t q = 0; q < 64; q++) {
                     const Piece& pc = best.lanes[g * 64 + q];
                     for (int k = 0; k < pc.n; k++)
@@ -2348,7 +2422,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     };
     struct Stream {
         std::vector<int4> head;
-        std::vector<int> ctrl, slots;
+        std::vector<int> ctrl;
         std::vector<int4> words;
     };
     auto build_stream = [](const Ell& e, bool up, int waves) {
@@ -2365,37 +2439,37 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             }
         }
         for (int w = 0; w < waves; w++) {
-            const int first = (int)st.ctrl.size(), row = (int)st.slots.size() / 64;
+            const int first = (int)st.ctrl.size();
             for (size_t i = 0; i < seq[w].size(); i++) {
                 const int q = seq[w][i].first, g = seq[w][i].second;
                 const int barriers = (i + 1 < seq[w].size() ? seq[w][i + 1].first : levels) - q;
                 const int4 info = e.group[g];
-                // pairs of terms; a step holds two, the last of a group possibly one
-                for (int k = 0; k < info.y; k += 2)
-                    for (int l = 0; l < 64; l++) {
-                        const int2 u = e.terms[info.x + (size_t)k * 64 + l], v = e.terms[info.x + (size_t)(k + 1) * 64 + l];
-                        st.words.push_back(make_int4(u.x, u.y, v.x, v.y));
-                    }
-                if (info.y % MTP_DEPTH_STEP) st.words.resize(st.words.size() + 64, make_int4(0, 0, 0, 0));
-                for (int k = MTP_DEPTH_STEP; k < info.y; k += MTP_DEPTH_STEP) st.ctrl.push_back(info.w);
-                st.ctrl.push_back(1 | info.z << 1 | barriers << 4 | info.w | (info.y % MTP_DEPTH_STEP ? MTP_CTRL_HALF : 0));
-                for (int q64 = 0; q64 < 64; q64++)
-                    st.slots.push_back((e.slot[g * 64 + q64] + 1) | e.lead[g * 64 + q64] << 16);
+                // pairs of terms, two to a step, and the slots' moments
+                for (int k = 0; k < info.y; k += MTP_DEPTH_STEP) {
+                    for (int t = k; t < k + MTP_DEPTH_STEP; t += 2)
+                        for (int l = 0; l < 64; l++) {
+                            if (t >= info.y) { st.words.push_back(make_int4(0, 0, 0, 0)); continue; }
+                            const Term &u = e.terms[info.x + (size_t)t * 64 + l], &v = e.terms[info.x + (size_t)(t + 1) * 64 + l];
+                            unsigned long long bits;
+                            std::memcpy(&bits, &u.mult, sizeof(bits));
+                            st.words.push_back(make_int4(u.x, v.x, t == k ? ((e.slot[g * 64 + l] & 0xffff) | e.lead[g * 64 + l] << 16) + 1 : 0, (int)(bits >> 32)));
+                        }
+                    st.ctrl.push_back(info.w | (k + MTP_DEPTH_STEP < info.y ? 0 : 1 | info.z << 1 | barriers << 4));
+                }
             }
-            st.head.push_back(make_int4(first, (int)st.ctrl.size() - first, row, seq[w].empty() ? levels : seq[w][0].first));
+            st.head.push_back(make_int4(first, (int)st.ctrl.size() - first, 0, seq[w].empty() ? levels : seq[w][0].first));
         }
-        st.words.resize(st.words.size() + MTP_DEPTH_STEP * 64, make_int4(0, 0, 0, 0));     // requested ahead
-        st.ctrl.resize(st.ctrl.size() + 2, 0);
-        st.slots.resize(st.slots.size() + 2 * 64, 0);
+        st.words.resize(st.words.size() + 2 * MTP_STEP_WORDS, make_int4(0, 0, 0, 0));      // requested ahead
+        st.ctrl.resize(st.ctrl.size() + 64, 0);
         return st;
     };
     // forward: terms per destination in file order; level l >= 1 at index l - 1
-    std::vector<std::pair<int, int2>> given;
+    std::vector<std::pair<int, Term>> given;
     for (int e = 0; e < n_times; e++) {
         const int* q = times + e * 4;
-        given.emplace_back(q[3], make_int2((q[0] * 8) | ((q[1] * 8) << 16), q[2]));
+        given.emplace_back(q[3], Term{(q[0] * 8) | ((q[1] * 8) << 16), (double)q[2]});
     }
-    const Lists fl(n_moms, given);
+    const Lists fl(n_moms, given, true);
     std::vector<std::vector<int>> f_by(n_levels), r_by(n_levels);
     for (int m = n_basic; m < n_moms; m++)
         if (level[m] >= 1 && fl.size(m)) f_by[level[m] - 1].push_back(m);
@@ -2403,10 +2477,10 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     given.clear();
     for (int e = n_times - 1; e >= 0; e--) {
         const int* q = times + e * 4;
-        given.emplace_back(q[1], make_int2((q[3] * 8) | ((q[0] * 8) << 16), q[2]));     // adj[m1] += adj[dst] mult M[m0]
-        given.emplace_back(q[0], make_int2((q[3] * 8) | ((q[1] * 8) << 16), q[2]));     // adj[m0] += adj[dst] mult M[m1]
+        given.emplace_back(q[1], Term{(q[3] * 8) | ((q[0] * 8) << 16), (double)q[2]});     // adj[m1] += adj[dst] mult M[m0]
+        given.emplace_back(q[0], Term{(q[3] * 8) | ((q[1] * 8) << 16), (double)q[2]});     // adj[m0] += adj[dst] mult M[m1]
     }
-    const Lists rl(n_moms, given);
+    const Lists rl(n_moms, given, true);
     for (int m = 0; m < n_moms; m++)
         if (level[m] < n_levels && rl.size(m)) r_by[level[m]].push_back(m);
     // Leaves: scalar moments that no product reads.  Only the read-out needs them, so that the calls whose read-out is linear
@@ -2433,7 +2507,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
     // The streams that a launch can ask for: those of the widths that wide_atoms gives for as many moments, and the forward one
     // of four wavefronts for the components.  (Host time of a plan with all of them and every cut laid out for each by itself
-    // 1.83 ms for level 16 and 14.2 for level 20, this 0.78 and 4.2.)
+    // 1.83 ms for level 16 and 14.2 for level 20, with the streams reached alone 0.78 and 4.2, in pairs of a multiplicity 1.2 and 5.6.)
     bool reached[2] = {false, false};
     for (int q = 0; q < 8; q++) reached[wide_atoms(n_moms, q & 1, q & 2, q & 4)] = true;
     Stream fs[2], rs[2], cs[2], vs[2];
@@ -2557,7 +2631,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             xhosts.emplace_back();
             XHost& h = xhosts.back();
             h.root.assign(n_scalar, -1);
-            std::vector<std::pair<int, int2>> given, words;
+            std::vector<std::pair<int, Term>> given, words;
             std::vector<std::pair<int, int>> by_level;
             for (int s : seeds) {
                 const int cnt = ancestors(s, h.nodes);
@@ -2569,20 +2643,20 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 for (int e : terms) {
                     const int* q = times + e * 4;
                     const int nd = node_of[q[3]];
-                    given.emplace_back(node_of[q[1]], make_int2((nd * 8) | ((q[0] * 8) << 16), q[2]));
-                    given.emplace_back(node_of[q[0]], make_int2((nd * 8) | ((q[1] * 8) << 16), q[2]));
+                    given.emplace_back(node_of[q[1]], Term{(nd * 8) | ((q[0] * 8) << 16), (double)q[2]});
+                    given.emplace_back(node_of[q[0]], Term{(nd * 8) | ((q[1] * 8) << 16), (double)q[2]});
                 }
                 bool any = false;
                 for (int m : anc) {
                     if (level[m] < n_levels) by_level.emplace_back(level[m], node_of[m]);
                     if (m >= n_basic) continue;
-                    words.emplace_back(s, make_int2(node_of[m] | (x_polys ? poly_pos[m] : m) << 16, 0));
+                    words.emplace_back(s, Term{node_of[m] | (x_polys ? poly_pos[m] : m) << 16, 0.0});
                     any = true;
                 }
-                if (!any) words.emplace_back(s, make_int2(-1, 0));           // (a column of zeros)
+                if (!any) words.emplace_back(s, Term{-1, 0.0});           // (a column of zeros)
                 for (int m : anc) node_of[m] = -1;
             }
-            const Lists xl(h.nodes, given);
+            const Lists xl(h.nodes, given, true);
             std::vector<std::vector<int>> x_by(n_levels);
             for (const auto& q : by_level)
                 if (xl.size(q.second)) x_by[q.first].push_back(q.second);
@@ -2595,7 +2669,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
             // sixteen words: 32 words deep instead of 24 at level 16.)
             for (auto& w : words)
                 if (w.second.x < 0) w.second.x = h.nodes;
-            const Lists columns(n_scalar, words);
+            const Lists columns(n_scalar, words, false);
             Level best;
             double best_cost = 0;
             for (int cap = MTP_SLOT_CAP; cap >= 2; cap -= 2) {
@@ -2654,10 +2728,10 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                          ((unsigned)basic[i * 4 + 3] << 24);
     const size_t o_basic = add(basic_words.data(), sizeof(unsigned) * n_basic);
     const size_t o_map = add(mapping, sizeof(int) * n_scalar);
-    struct StreamOff { size_t head, ctrl, slots, words; };
+    struct StreamOff { size_t head, ctrl, words; };
     auto add_stream = [&](const Stream& st) {
         return StreamOff{add(st.head.data(), sizeof(int4) * st.head.size()), add(st.ctrl.data(), sizeof(int) * st.ctrl.size()),
-                         add(st.slots.data(), sizeof(int) * st.slots.size()), add(st.words.data(), sizeof(int4) * st.words.size())};
+                         add(st.words.data(), sizeof(int4) * st.words.size())};
     };
     const size_t o_leaf = add(mapping_leaf.data(), sizeof(int) * n_scalar);
     StreamOff o_f[2], o_r[2], o_c[2], o_v[2];
@@ -2704,12 +2778,12 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.basic = (const unsigned*)(base + o_basic);
     d.mapping = (const int*)(base + o_map);
     auto stream_at = [&](const StreamOff& o) {
-        return MtpStream{(const int4*)(base + o.head), (const int*)(base + o.ctrl), (const int*)(base + o.slots), (const int4*)(base + o.words)};
+        return MtpStream{(const int4*)(base + o.head), (const int*)(base + o.ctrl), (const int4*)(base + o.words)};
     };
     for (int i = 0; i < 2; i++) { d.fwd[i] = stream_at(o_f[i]); d.rev[i] = stream_at(o_r[i]); }
     for (int i = 0; i < 2; i++) { d.fwd_core[i] = stream_at(o_c[i]); d.rev_leaf[i] = stream_at(o_v[i]); }
     d.mapping_leaf = (const int*)(base + o_leaf);
-    d.x = MtpStream{nullptr, nullptr, nullptr, nullptr};
+    d.x = MtpStream{nullptr, nullptr, nullptr};
     d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
     d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
     d.rows = (const int*)(base + o_rows); d.polys = (const int*)(base + o_poly);

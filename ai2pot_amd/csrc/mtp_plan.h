@@ -19,28 +19,29 @@
 namespace a2p {
 
 constexpr int MTP_SLOT_CAP = 16;
-// Terms of a slot to a step of the sweeps; the last step of a group may hold half of them.
-constexpr int MTP_DEPTH_STEP = 4;
-// Marks of a control word: a step of half length, and a step of a group of leaves (rev_leaf).
-constexpr int MTP_CTRL_HALF = 1 << 30, MTP_CTRL_LEAF = 1 << 29;
+// Terms of a slot to a step of the sweeps, and the words of a step: the terms by pairs, 64 lanes each.
+constexpr int MTP_DEPTH_STEP = 4, MTP_STEP_WORDS = MTP_DEPTH_STEP / 2 * 64;
+// Mark of a control word: a step of a group of leaves (rev_leaf).
+constexpr int MTP_CTRL_LEAF = 1 << 29;
 
-// A gather as the wavefronts of a workgroup walk it.  `lists[m]` holds the terms of moment m.  A slot holds up to
-// MTP_SLOT_CAP of them; a longer list is cut into pieces of equal length, so that no lane walks a long list alone.  Slots are
+// A gather as the wavefronts of a workgroup walk it.  `lists[m]` holds the terms of moment m, in pairs of the same multiplicity
+// (one without a partner twice, each time half).  A slot holds up to MTP_SLOT_CAP of them; a longer list is cut into pieces of
+// equal length, so that no lane walks a long list alone.  Slots are
 // grouped 64 at a time, one to a lane; the pieces of a list lie in one group, a list of up to sixteen within a row of sixteen
 // lanes and a longer one from the beginning of a row on, and the wavefront adds their sums (four doubling steps within a row,
 // two across).  How long the pieces of a level are is what a wavefront issues for it at least (pack_level); rows are filled
-// first fit, deepest lists first.  The words of a group are padded with zero terms to its depth, an even number; a word packs
-// x = 8 m0 | 8 m1 << 16 (byte offsets into an array of doubles), y = multiplicity, and two terms of a lane lie together.
+// first fit, deepest lists first.  The words of a group are padded with zero terms to its depth; a word is a pair: x, y = 8 m0 | 8 m1
+// << 16 of its terms (byte offsets into an array of doubles), w = upper half of the multiplicity as a double, whose lower half is
+// zero, z = slot word in the first word of a step.
 // The groups of a level are dealt to the wavefronts, the deepest first and to the one with the least to do, and everything a
-// wavefront needs lies in the order in which it needs it: MTP_DEPTH_STEP x 64 words to a step, a control word for each step,
-// and a row of 64 slot words for each group.
+// wavefront needs lies in the order in which it needs it: MTP_STEP_WORDS words to a step, and a control word for each step.
 // (Lists cut at sixteen terms and laid out in order of length, in steps of four: 244 instead of 229 us for the call at level 20,
 // 8192 atoms, 304 instead of 286 for the training step at level 16, 64 structures of 128 atoms.)
 struct MtpStream {
-    const int4* head;          // [wavefronts] first step, steps, first row of slots, barriers before the first step
-    const int* ctrl;           // MTP_CTRL_ marks, and at the last step of a group 1 | doubling steps << 1 | barriers to pass << 4
-    const int* slots;          // moment + 1 in the first piece of a list (0 elsewhere) | pieces of the list behind this one << 16
-    const int4* words;
+    const int4* head;          // [wavefronts] first step, steps, unused, barriers before the first step
+    const int* ctrl;           // MTP_CTRL_LEAF, and at the last step of a group 1 | doubling steps << 1 | barriers to pass << 4
+    const int4* words;         // slot word: (moment in the first piece of a list, -1 elsewhere) & 0xffff | pieces of the list behind this one
+                               // << 16, plus one
 };
 
 struct MtpPlanDevice {
@@ -50,11 +51,11 @@ struct MtpPlanDevice {
     // device arrays
     const unsigned* basic;     // [n_basic]    mu | a << 8 | b << 16 | c << 24
     const int* mapping;        // [n_scalar]
-    // forward gather (terms of a product: its factors) and reverse gather (terms of a factor: x = 8 dst | 8 other << 16;
+    // forward gather (terms of a product: its factors) and reverse gather (terms of a factor: 8 dst | 8 other << 16;
     // sources by level, from the last level to level 0), for workgroups of one wavefront and of four
     MtpStream fwd[2], rev[2];
     // The same for a linear read-out: scalar moments that no product reads (leaves) are left out of the forward gather, and
-    // their lists stand with the first sources of the reverse one (control words marked, x = 8 m0 | 8 m1 << 16).
+    // their lists stand with the first sources of the reverse one (control words marked, 8 m0 | 8 m1 << 16).
     MtpStream fwd_core[2], rev_leaf[2];
     const int* mapping_leaf;   // [n_scalar]   mapping | leaf << 16
     int max_level_slots;       // most slots of any level (forward or reverse)
@@ -77,7 +78,7 @@ struct MtpPlanDevice {
     // The one-hot adjoints of all scalar moments at once (linear-solver components).  A node (s, m) is moment m as an
     // ancestor of scalar moment s: mapping[s] itself, or a factor of a product among its ancestors.  The adjoint
     // sweeps of all read-outs e_s together are one reverse gather over the nodes, laid out like the reverse gather
-    // above (a term packs x = 8 node(dst) | 8 other << 16 with `other` a moment, y = mult).
+    // above (a term packs 8 node(dst) | 8 other << 16 with `other` a moment).
     // The basic ancestors of a scalar moment form a list of words node | basic << 16; lists are cut into pieces of equal length,
     // at most MTP_SLOT_CAP words, and placed first fit, deepest first, 64 slots a group, the pieces of a list in neighbouring
     // slots as in the gathers (the wavefront adds their sums, x_bsteps doubling steps).  A group's words are

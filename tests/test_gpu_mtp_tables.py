@@ -45,6 +45,35 @@ def test_irregular_basic_moments(oracle, basic):
         assert close(got[k], ref[k]), k
 
 
+@pytest.mark.parametrize("levels", [1, 2, 5, 62, 63, 64, 65, 129, 130])
+def test_products_by_number_of_levels_and_multiplicity(oracle, levels):
+    """Products that depend on the one before, so that a wavefront makes as many steps as there are levels, odd and even, less and
+    more than the 64 whose control words it holds at a time; lists with one, two and three products of a multiplicity, among them
+    negative ones and one beyond 21 bits.  Energies, forces, virials and loss gradients against the oracle: fp64, 1e-10."""
+    nt, nbasic = 2, len(GAPS)
+    times = []
+    for k in range(levels):                                       # sums that stay of the order of a product of two
+        at = nbasic + k
+        times += [(at - 1 if k else 1, 0, 1, at), (2, 3, -3, at), (4, 5, 1, at), (1, 3, 2, at)]
+    last = nbasic + levels
+    times += [(0, 0, (1 << 21) + 1, last), (1, 1, -(1 << 21), last), (last - 1, 2, 1, last)]
+    t = dict(alpha_moments_count=last + 1, alpha_index_basic=np.array(GAPS, np.int32),
+             alpha_index_times=np.array(times, np.int32), alpha_moment_mapping=np.array(sorted({0, 2, nbasic, last - 1, last}), np.int32), nmus=2)
+    nb = synth.pack_batch([structure(oracle, n, (8.5, 9.0, 9.5), nt, 21 + n, 5.0) for n in (12, 7)])
+    m = synth.mtp_model(t, nt, 6, 5.0, 1.5, 3200)
+    m["q_scaler"] = np.linspace(0.8, 1.3, m["q_scaler"].size)
+    m["linear_coeffs"][-1] *= 1e-6                                # of the order of the others
+    for got, ref in zip(gpu_efv(m, nb), oracle.mtp_efv(m, nb)):
+        assert np.isfinite(ref).all() and close(got, ref)
+    B, P = nb["bilist"].shape
+    labels = dict(energy=synth.rng_normal(1, B, -4 * 12, 3), force=synth.rng_normal(2, B * P * 3).reshape(B, P, 3),
+                  virial=synth.rng_normal(3, B * 9, 0, 0.5).reshape(B, 9))
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w), oracle.mtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dlinear", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
 @pytest.mark.parametrize("level", [8, 14, 16, 18])                # 1, 1, 2 and 4 groups of 64 pieces
 @pytest.mark.parametrize("U", [1, 2, 3, 9, None])
 def test_components_by_group_and_row_length(oracle, level, U):
