@@ -59,31 +59,44 @@ struct SegArgs {
 };
 
 // The model's tables in LDS, staged by the workgroup: w0 in rows of WROW values, the coefficients of a species pair in rows of
-// NB * KC + CPAD.  The first W0 and four values of every thread are all on their way before one is stored, behind them
-// whatever `early` asks for.
+// NB * KC + CPAD.  The first W0 and four values of every thread, four to a load, are all on their way before one is stored, behind
+// them whatever `early` asks for.  No load stands behind a branch: a thread beyond the end takes the last four again.
 template <int KC, int NB, int D, int WROW, int CPAD, int W0, typename T, typename Args, typename Lds, typename Early>
 __device__ __forceinline__ void stage_tables(Args& a, const Lds& L, int tid, int nthreads, Early early)
 {
-    constexpr int C0 = 4;
-    const int nt = a.ntypes, H = a.H, nw0 = nt * H * D, nc = nt * nt * NB * KC, nh = nt * H;
-    T w0[W0], c0[C0], b0 = (T)0, w1 = (T)0, qs = (T)1;
-    auto put_w0 = [&](int i, T v) __attribute__((always_inline)) { const int r = i / D; L.w0[r * WROW + (i - r * D)] = v; };
-    auto put_coef = [&](int i, T v) __attribute__((always_inline)) { const int p = i / (NB * KC); L.coef[p * (NB * KC + CPAD) + (i - p * NB * KC)] = v; };
+    constexpr int W4 = W0 / 4, NC = NB * KC;
+    static_assert(W0 % 4 == 0 && D >= 4 && NC >= 4, "four values cross one end of a row at most");
+    struct alignas(sizeof(T)) Four { T v[4]; };
+    const int nt = a.ntypes, H = a.H, nw0 = nt * H * D, nc = nt * nt * NC, nh = nt * H;
+    auto take = [&](const T* p, int n, int u) __attribute__((always_inline)) {
+        return *reinterpret_cast<const Four*>(p + min((tid + u * nthreads) * 4, n - 4));
+    };
+    auto put = [&](T* dst, auto row, auto pad, int n, int u, const Four& o) __attribute__((always_inline)) {
+        constexpr int ROW = decltype(row)::value, PAD = decltype(pad)::value;
+        const int i = min((tid + u * nthreads) * 4, n - 4), r = i / ROW, c = i - r * ROW;
 #pragma unroll
-    for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; c0[u] = i < nc ? a.coeffs[i] : (T)0; }
+        for (int k = 0; k < 4; k++) dst[i + k + (r + (c + k >= ROW ? 1 : 0)) * PAD] = o.v[k];
+    };
+    auto put_w0 = [&](int u, const Four& o) __attribute__((always_inline)) {
+        put(L.w0, std::integral_constant<int, D>{}, std::integral_constant<int, WROW - D>{}, nw0, u, o);
+    };
+    auto put_coef = [&](int u, const Four& o) __attribute__((always_inline)) {
+        put(L.coef, std::integral_constant<int, NC>{}, std::integral_constant<int, CPAD>{}, nc, u, o);
+    };
+    const Four c0 = take(a.coeffs, nc, 0);
+    Four w0[W4];
 #pragma unroll
-    for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; w0[u] = i < nw0 ? a.w0[i] : (T)0; }
-    if (tid < nh) { b0 = a.b0[tid]; w1 = a.w1[tid]; }
-    if (tid < D) qs = a.q_scaler[tid];
+    for (int u = 0; u < W4; u++) w0[u] = take(a.w0, nw0, u);
+    const T b0 = a.b0[min(tid, nh - 1)], w1 = a.w1[min(tid, nh - 1)], qs = a.q_scaler[min(tid, D - 1)];
     early();
+    put_coef(0, c0);
 #pragma unroll
-    for (int u = 0; u < C0; u++) { const int i = tid + u * nthreads; if (i < nc) put_coef(i, c0[u]); }
-#pragma unroll
-    for (int u = 0; u < W0; u++) { const int i = tid + u * nthreads; if (i < nw0) put_w0(i, w0[u]); }
+    for (int u = 0; u < W4; u++)
+        if (u * nthreads * 4 < nw0) put_w0(u, w0[u]);
     if (tid < nh) { L.b0[tid] = b0; L.w1[tid] = w1; }
     if (tid < WROW) L.qs[tid] = tid < D ? (T)1 / qs : (T)0;
-    for (int i = tid + C0 * nthreads; i < nc; i += nthreads) put_coef(i, a.coeffs[i]);
-    for (int i = tid + W0 * nthreads; i < nw0; i += nthreads) put_w0(i, a.w0[i]);
+    for (int u = 1; (tid + u * nthreads) * 4 < nc; u++) put_coef(u, take(a.coeffs, nc, u));
+    for (int u = W4; (tid + u * nthreads) * 4 < nw0; u++) put_w0(u, take(a.w0, nw0, u));
     for (int i = tid + nthreads; i < nh; i += nthreads) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
 }
 

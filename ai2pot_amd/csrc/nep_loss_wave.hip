@@ -108,16 +108,23 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
         x1 = a.brcs[pr * 3]; y1 = a.brcs[pr * 3 + 1]; z1 = a.brcs[pr * 3 + 2];
     };
     begin(blockIdx.x * LW_WAVES + wave);
-    stage_tables<KC, NB, D, WROW, CPAD, sizeof(T) == 4 ? 16 : 8, T>(a, L, tid, LW_THREADS, []() {});
+    int inum;
+    T cE;
+    stage_tables<KC, NB, D, WROW, CPAD, sizeof(T) == 4 ? 16 : 8, T>(a, L, tid, LW_THREADS, [&]() __attribute__((always_inline)) {
+        inum = min(uniform_array(a.binum)[b], a.P);
+        cE = uniform_array(a.cE)[b];
+    });
     if (tid < LM) {
         const int l = l_of_lm(tid);
         L.wc[tid] = tid < NLM ? (T)(tid == l * l - 1 ? 1.0 : 2.0) * (T)kC3B[tid] : (T)0;
     }
+    const int* types = a.btypes + (size_t)b * a.P;
+    // The species of the next atom is asked for ahead of its turn too.
+    auto species = [&]() __attribute__((always_inline)) { return types[(unsigned)center1 < (unsigned)a.P ? center1 : 0]; };
+    int ti1 = species();
     __syncthreads();
 
-    const int inum = min(a.binum[b], a.P);
-    const T cE = a.cE[b], rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
-    const int* types = a.btypes + (size_t)b * a.P;
+    const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
     const T* dv = a.dVs + (size_t)b * 9;
     const unsigned long long lt = (1ull << lane) - 1ull;
 
@@ -126,7 +133,7 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
         int center = center1, nn = nn1;
         if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
         if ((unsigned)center >= (unsigned)a.P) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-        int ti = types[center];
+        int ti = center == center1 ? ti1 : types[center];
         if ((unsigned)ti >= (unsigned)nt) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         if (nn == 0) begin(ii + gridDim.x * LW_WAVES);        // (no first slots below, behind which the next row is fetched)
         const T* const cti = L.coef + (size_t)ti * nt * CROW;
@@ -409,6 +416,8 @@ __global__ void __launch_bounds__(LW_THREADS, LW_GROUPS<T>) nep_loss_wave_kernel
                 if (lane < D) { L.ab[lane] = av * L.qs[lane]; L.ab[WROW + lane] = bv * L.qs[lane]; }
             }
             __builtin_amdgcn_wave_barrier();
+
+            ti1 = species();                           // (of the next row, which was fetched behind the first slots of this)
 
             // ---- radial coefficients' gradient; [sigma tau ; tau 0] over the moments
             for (int o = lane; o < nt * NR * KC; o += 64) {

@@ -18,10 +18,10 @@
 // Registers decide how many wavefronts a SIMD holds: each phase takes arguments, LDS addresses and the lane's place anew.  With
 // 60 values spilled for three wavefronts the kernel took 89 us at 20,011 atoms, with two 72, so 58.
 //
-// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 22 us
-// (28 now for the same atoms in no spatial order), 20,011 with skin lists 94 -> 57, 64 structures of 128 atoms 43 -> 25.
-// Of the 43 thousand cycles of a wavefront at 4096 atoms the tables take 6.4, slots 7, angular pairs and moments 6, read-out 10,
-// angular forces 2.2, radial forces 4.6.  Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq
+// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 21.7 us
+// (28 for the same atoms in no spatial order), 20,011 with skin lists 94 -> 56.5, 64 structures of 128 atoms 43 -> 24.5.
+// Of the 42 thousand cycles of a wavefront at 4096 atoms the tables take 5.2 (8.2 with a load to a value and the number of rows
+// waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6.  Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq
 // by fours (57 -> 58).
 //
 // Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
@@ -172,15 +172,10 @@ nep_quad_kernel(const WaveArgs<T>)
     constexpr int NLM = A::NLM, MG = A::MG, XYZ = A::XYZ, NB = NR + NAC, D = NR + NAC * LC, CROW = NB * KC + CPAD;
     static_assert(D <= WROW && D <= 16 + 8, "descriptor count exceeds the padded row or the lanes of dE/dq");
     extern __shared__ __align__(16) unsigned char smem_raw[];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int b = blockIdx.y, nwaves = blockDim.x >> 6, first = NW_ATOMS * (wave * gridDim.x + blockIdx.x), stride = NW_ATOMS * nwaves * gridDim.x;
     int inum;
     bool derivs, claims;
-    {
-        NW_PHASE;
-        inum = min(a.binum[b], a.P);                  // (the loop below strides over the rows: none beyond the last)
-        derivs = a.force != nullptr || a.want_virial;
-        claims = derivs && seg.cursor;
-    }
     double e_sum = 0.0, v_sum[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) v_sum[i] = 0.0;
@@ -190,8 +185,7 @@ nep_quad_kernel(const WaveArgs<T>)
     constexpr int V = 2, STEP = V * NW_LANES;              // slots of a lane in flight, of an atom per trip
     int center1, nn1, ti1, nj[V], nj1[V], tj[V];
     T x[V], y[V], z[V], x1[V], y1[V], z1[V];
-    auto load = [&](int base, int room, int slot0, int (&n)[V], T (&px)[V], T (&py)[V], T (&pz)[V]) __attribute__((always_inline)) {
-        NW_PHASE;
+    auto load = [&](auto& a, int s, int base, int room, int slot0, int (&n)[V], T (&px)[V], T (&py)[V], T (&pz)[V]) __attribute__((always_inline)) {
 #pragma unroll
         for (int v = 0; v < V; v++) {
             const int slot = slot0 + v * NW_LANES + s;
@@ -208,8 +202,8 @@ nep_quad_kernel(const WaveArgs<T>)
         const int row = b * a.P + min(i0 + g, a.P - 1);
         center1 = a.bilist[row];
         nn1 = a.bnumneigh[row];
-        load(row * U, U, 0, nj, x, y, z);
-        load(row * U, U, STEP, nj1, x1, y1, z1);
+        load(a, s, row * U, U, 0, nj, x, y, z);
+        load(a, s, row * U, U, STEP, nj1, x1, y1, z1);
     };
     auto species = [&](const int (&n)[V], int (&t)[V]) __attribute__((always_inline)) {
         NW_PHASE;
@@ -217,27 +211,29 @@ nep_quad_kernel(const WaveArgs<T>)
 #pragma unroll
         for (int v = 0; v < V; v++) t[v] = (unsigned)n[v] < (unsigned)NF ? types[n[v]] : 0;
     };
-    // Their species too in fp64, where a SIMD holds one wavefront and nothing else hides the wait (4096 atoms with 72 neighbours
-    // 37.1 -> 30.8 us); in fp32 it only delays the tables (22.0 -> 22.4).
-    constexpr bool EARLY = sizeof(T) == 8;
+    // Their species too, asked for when the tables have been stored: what comes before them in the wavefront's loads is there by then.
     auto begin_species = [&]() __attribute__((always_inline)) {
         NW_PHASE;
         ti1 = a.btypes[(size_t)b * NF + ((unsigned)center1 < (unsigned)NF ? center1 : 0)];
         species(nj, tj);
     };
-    const int nwaves = blockDim.x >> 6, first = NW_ATOMS * (wave * gridDim.x + blockIdx.x), stride = NW_ATOMS * nwaves * gridDim.x;
     begin(first);
     {
         NW_PHASE;
         const int tid = threadIdx.x, nthreads = blockDim.x;
-        T bias = (T)0;
+        T bias;
+        double c3b;
         stage_tables<KC, NB, D, WROW, CPAD, 16, T>(a, L, tid, nthreads, [&]() __attribute__((always_inline)) {
-            if (tid < nt) bias = a.bias[tid];
-            if constexpr (EARLY) begin_species();
-            if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)kC3B[tid] : (T)0;
+            bias = a.bias[min(tid, nt - 1)];
+            c3b = kC3B[min(tid, NLM - 1)];
+            derivs = a.force != nullptr || a.want_virial;
+            claims = derivs && seg.cursor;
+            inum = min(uniform_array(a.binum)[b], a.P);       // (the loop below strides over the rows: none beyond the last)
         });
+        if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)c3b : (T)0;
         if (tid < nt) L.bias[tid] = bias;
         for (int i = tid + nthreads; i < nt; i += nthreads) L.bias[i] = a.bias[i];
+        begin_species();
     }
     __syncthreads();
 
@@ -250,7 +246,7 @@ nep_quad_kernel(const WaveArgs<T>)
             if (!act) { center = 0; nn = 0; }
             if (nn > U) { if (s == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = U; }
             if ((unsigned)center >= (unsigned)NF) { if (s == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-            ti = EARLY && center == center1 ? ti1 : a.btypes[(size_t)b * NF + center];
+            ti = center == center1 ? ti1 : a.btypes[(size_t)b * NF + center];
             if ((unsigned)ti >= (unsigned)nt) { if (s == 0 && act) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         }
         const int ntiles = max(1, (most_of_atoms(nn) + NW_CAP - 1) / NW_CAP);
@@ -283,17 +279,17 @@ nep_quad_kernel(const WaveArgs<T>)
                 const unsigned below = (1u << s) - 1u;
                 const int room = min(U - t * NW_CAP, NW_CAP);
                 if (jt > 0) {
-                    load(base, room, 0, nj, x, y, z);
-                    load(base, room, STEP, nj1, x1, y1, z1);
+                    load(a, s, base, room, 0, nj, x, y, z);
+                    load(a, s, base, room, STEP, nj1, x1, y1, z1);
+                    species(nj, tj);
                 }
-                if (jt > 0 || !EARLY) species(nj, tj);
                 const int trips = (most_of_atoms(tn) + STEP - 1) / STEP;
 #pragma unroll 1
                 for (int k = 0; k < trips; k++) {
                     const int slot0 = k * STEP + s;
                     int nj2[V];
                     T x2[V], y2[V], z2[V];
-                    load(base, tn, (k + 2) * STEP, nj2, x2, y2, z2);
+                    load(a, s, base, tn, (k + 2) * STEP, nj2, x2, y2, z2);
                     int tj1[V];
                     species(nj1, tj1);
                     bool valid[V], inA[V], inR[V];
@@ -706,7 +702,7 @@ nep_quad_kernel(const WaveArgs<T>)
             if (act && seg.mark && s == 3) pair_mark_own(&seg.cursor[b * NF + center]);
         }
         begin(i0 + stride);
-        if constexpr (EARLY) begin_species();
+        begin_species();
     }
 
     // ---- workgroup partial sums of energy and virial (fp64): 16 threads to a sum, lanes 4 k .. 4 k + 3 of every wavefront

@@ -187,14 +187,14 @@ nep_wave_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g)
     Slots<T> slots;
     load_slots<T>(a, 0, lane, row1, a.U, slots);
     const int* const types = a.btypes + (size_t)b * NF;
-    int ti1;
+    int ti1, inum;
     stage_tables<KC, NB, D, WROW, CPAD, sizeof(T) == 4 ? 16 : 8, T>(a, L, tid, NW_THREADS, [&]() __attribute__((always_inline)) {
         ti1 = types[(unsigned)center1 < (unsigned)NF ? center1 : 0];
         load_species<T>(types, NF, slots);
+        inum = min(uniform_array(a.binum)[b], a.P);   // (the loop below strides over the rows: none beyond the last)
     });
     __syncthreads();
 
-    const int inum = min(a.binum[b], a.P);            // (the loop below strides over the rows: none beyond the last)
     const T rr = a.rr, ra = a.ra, rr_inv = (T)1 / rr, ra_inv = (T)1 / ra;
     const bool derivs = a.force != nullptr || a.want_virial;
     const int quad = lane >> 2, chan = lane & 3;       // neighbour within a round of 16, angular channel
