@@ -203,6 +203,14 @@ __device__ __forceinline__ const A2P_CONSTANT S* kernel_args() { return (const A
 template <typename S>
 __device__ __forceinline__ const A2P_CONSTANT S* uniform_array(const S* p) { return (const A2P_CONSTANT S*)(uintptr_t)p; }
 
+// Workgroups are handed to the 8 XCDs round robin; giving XCD k the k-th contiguous run of blocks
+// keeps neighbours in space on one L2.
+__device__ __forceinline__ int xcd_block(int w, int nb)
+{
+    const int per = nb >> 3, rem = nb & 7, k = w & 7;
+    return k * per + min(k, rem) + (w >> 3);
+}
+
 // The same reduction for a producer that stores each pair derivative straight into its target's segment, without the
 // intermediate [row, slot, 3] array (pair_fixed_begin, the producer, pair_csr_finish).
 // Capacity of the fixed reduction segments: umax unless the calling thread asked for more with

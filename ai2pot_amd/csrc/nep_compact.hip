@@ -132,14 +132,6 @@ __device__ __forceinline__ T radial_derivative_dot(T r, T rc_inv, const T (&a)[K
 
 __host__ __device__ __forceinline__ size_t lds16(size_t bytes) { return (bytes + 15) & ~(size_t)15; }
 
-// Workgroups are handed to the 8 XCDs round robin; giving XCD k the k-th contiguous run of blocks
-// keeps neighbours in space on one L2.
-__device__ __forceinline__ int xcd_block(int w, int nb)
-{
-    const int per = nb >> 3, rem = nb & 7, k = w & 7;
-    return k * per + min(k, rem) + (w >> 3);
-}
-
 // One chunk (8 slots of the tile's 64 positions, contiguous in memory) on its way into the wavefront's
 // staging buffer (position-major with STP slots per position): contiguous loads, then 16-byte LDS stores.
 template <typename T>
@@ -517,7 +509,9 @@ nep_adjoint_kernel(const GatherArgs<T> a)
     }
     if (tid < FDP) L.qs[tid] = tid < DC ? (T)1 / a.q_scaler[tid] : (T)0;
 
-    const auto [active, atom, ti, n_outer, n_inner] = position_header<T>(a, p);
+    const Header head = position_header<T>(a, p);
+    const bool active = head.active;
+    const int atom = head.atom, ti = head.ti, n_outer = head.n_outer, n_inner = head.n_inner;
     const T rr_inv = (T)1 / a.rr, ra_inv = (T)1 / a.ra;
 
     T F[NTC][KC];                 // radial functions summed per neighbour species
@@ -819,7 +813,9 @@ nep_gather_kernel(const GatherArgs<T> a)
     T* const st = L.stage + (size_t)wv * 64 * STP * 4;
 
     const int claimed = p < a.cv.natoms && a.force ? a.incoming[p] : 0;
-    const auto [active, atom, ti, n_outer, n_inner] = position_header<T>(a, p);
+    const Header head = position_header<T>(a, p);
+    const bool active = head.active;
+    const int atom = head.atom, ti = head.ti, n_outer = head.n_outer, n_inner = head.n_inner;
     const T rr_inv = (T)1 / a.rr;
 
     // own contracted radial coefficients, one array per neighbour species (separate arrays: a select between

@@ -19,7 +19,7 @@
 // 60 values spilled for three wavefronts the kernel took 89 us at 20,011 atoms, with two 72, so 58.
 //
 // Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 21.7 us
-// (28 for the same atoms in no spatial order), 20,011 with skin lists 94 -> 56.5, 64 structures of 128 atoms 43 -> 24.5.
+// (28 for the same atoms in no spatial order), 20,011 with skin lists 94 -> 53, 64 structures of 128 atoms 43 -> 24.5.
 // Of the 42 thousand cycles of a wavefront at 4096 atoms the tables take 5.2 (8.2 with a load to a value and the number of rows
 // waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6.  Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq
 // by fours (57 -> 58).
@@ -144,6 +144,7 @@ struct WaveArgs {
     SegArgs seg;
     T* seg_g;
     WaveAt at;
+    int runs;                        // rows dealt to the workgroups in runs (wave_shape)
 };
 // The lane's place, found anew by each phase as well (again() of a2p_common.h): what the phases derive from it does not fit the registers
 // of three wavefronts per SIMD either.
@@ -173,9 +174,22 @@ nep_quad_kernel(const WaveArgs<T>)
     static_assert(D <= WROW && D <= 16 + 8, "descriptor count exceeds the padded row or the lanes of dE/dq");
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int b = blockIdx.y, nwaves = blockDim.x >> 6, first = NW_ATOMS * (wave * gridDim.x + blockIdx.x), stride = NW_ATOMS * nwaves * gridDim.x;
-    int inum;
+    const int nwaves = blockDim.x >> 6;
+    int b, blk, inum, last, first, stride;         // structure, workgroup of it; rows, and of the wavefront: end, first, distance
     bool derivs, claims;
+    {
+        NW_PHASE;
+        const int nblocks = a.nblocks;
+        b = blockIdx.y; blk = blockIdx.x; last = a.P;
+        first = NW_ATOMS * (wave * nblocks + blk); stride = NW_ATOMS * nwaves * nblocks;
+        if (K_.runs) {
+            const int at = xcd_block(b * nblocks + blk, nblocks * gridDim.y);
+            b = at / nblocks; blk = at - b * nblocks;
+            const int sets = (last + NW_ATOMS - 1) / NW_ATOMS, per = sets / nblocks, more = sets - per * nblocks, set0 = blk * per + min(blk, more);
+            first = NW_ATOMS * (set0 + wave); stride = NW_ATOMS * nwaves;
+            last = NW_ATOMS * (set0 + per + (blk < more ? 1 : 0));
+        }
+    }
     double e_sum = 0.0, v_sum[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) v_sum[i] = 0.0;
@@ -237,7 +251,7 @@ nep_quad_kernel(const WaveArgs<T>)
     }
     __syncthreads();
 
-    for (int i0 = first; i0 < inum; i0 += stride) {
+    for (int i0 = first; i0 < min(inum, last); i0 += stride) {
         int center = center1, nn = nn1, ti, base0;
         {
             NW_PHASE;
@@ -724,7 +738,7 @@ nep_quad_kernel(const WaveArgs<T>)
             for (int i = 0; i < 4; i++) v += theirs[i];
         }
         v = row_sum(v);
-        if (s == 0) a.partial[ev_partial(a.nblocks, b, blockIdx.x, c)] = v;
+        if (s == 0) a.partial[ev_partial(a.nblocks, b, blk, c)] = v;
     }
 }
 #undef NW_PHASE
@@ -732,19 +746,26 @@ nep_quad_kernel(const WaveArgs<T>)
 // Wavefronts of a workgroup, workgroups of a structure.  A workgroup to a compute unit, which shares the model's tables, or two
 // where they have room; as many rows for each wavefront as it takes with the most wavefronts a compute unit holds, and then no
 // more wavefronts than that takes (four stage the tables faster than one).
-struct WaveShape { int waves, nblocks; size_t lds; WaveAt at; };
+// Up to eight sets to a compute unit the rows are dealt out one set to a workgroup in turn; beyond, every workgroup takes a run of
+// consecutive rows and every XCD a run of workgroups, so that neighbours in the list's order share their species, cursors and
+// segments' lines in one cache.  In turn and in runs, us: one structure of 9,000 atoms 34.9 and 32.1, 20,011 with ghosts 57.0
+// and 52.9, 32,768 68.1 and 66.0; 8 of 2,500 61.4 and 47.6, 32 of 640 60.1 and 47.7, 64 of 400 66.2 and 59.7, 128 of 128 44.4
+// and 41.1; fp64 20,011 100 and 98.  With fewer sets all rows of a neighbourhood claim their places at once, from one XCD: 4,096
+// atoms 21.9 and 23.1, 6,000 25.0 and 26.0, 8,192 26.6 and 26.7, 64 structures of 128 24.8 and 29.4.  (XCDs in runs and workgroups in
+// turn: 20,011 atoms 51.4, 32,768 82.9.)
+struct WaveShape { int waves, nblocks, runs; size_t lds; WaveAt at; };
 template <typename T>
 WaveShape wave_shape(const NepArgs<T>& a)
 {
     const WaveAt at = a.l_max == 3 ? wave_at<T, 3>(a.ntypes, a.H, a.n_r + NAC) : wave_at<T, 4>(a.ntypes, a.H, a.n_r + NAC);
     const int most = std::min(wave_cap<T>(), (160 * 1024 - std::min(at.shared, 160 * 1024)) / at.own);
-    if (most < 1) return {0, 0, 0, at};
+    if (most < 1) return {0, 0, 0, 0, at};
     const int per = std::max(1, ceil_div(a.P, NW_ATOMS));                    // sets of four rows of a structure
     const long long sets = (long long)a.B * per;
     int waves = std::min(most, (int)std::min<long long>((sets + 256 * 4 - 1) / (256 * 4) * 4, wave_cap<T>())), held = 1;
     if (waves == 8 && 2 * (at.shared + 4 * at.own) <= 160 * 1024) { waves = 4; held = 2; }
     const int nblocks = std::min(ceil_div(per, waves), std::max(1, held * 256 / std::max(a.B, 1)));
-    return {waves, nblocks, (size_t)at.shared + (size_t)waves * at.own, at};
+    return {waves, nblocks, sets > 8 * 256, (size_t)at.shared + (size_t)waves * at.own, at};
 }
 
 template <typename T, int NR, int LC>
@@ -756,7 +777,7 @@ int launch_wave(const NepArgs<T>& a, const PairCsr& csr, hipStream_t stream)
     if (w.lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)w.lds));
     prof_begin("nep_quad_kernel", stream);
-    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at});
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at, w.runs});
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;

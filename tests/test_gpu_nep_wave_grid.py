@@ -74,3 +74,26 @@ def test_tile_edges_of_four_atoms(oracle, np_dtype, n_r, l_max, ntypes, H, nghos
     e, f, v = run_gpu(m, many, np_dtype)
     for k in range(0, 39, 3):
         check((e[k:k + 3], f[k:k + 3], v[k:k + 3]), ref, np_dtype)
+
+
+@pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("copies,batch", [(29, 4), (2, 61), (1, 130)])
+def test_rows_in_runs_and_in_turn(np_dtype, copies, batch):
+    """Above 2048 sets of four rows a workgroup takes a run of rows: every structure as it comes out alone, with from none to
+    all of its rows in use."""
+    m = synth.nep_model(ntypes=3, num_neurons=30, type_map=(1, 2, 3, 4, 5), sigma=0.12)
+    m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
+    nb = _copies(_block(np_dtype, 3), copies, batch)
+    P = nb["bilist"].shape[1]
+    nb["binum"] = (np.arange(batch) * 37 % (P + 1)).astype(np.int32)
+    nb["binum"][-1] = P
+    assert batch * -(-P // 4) > 2048
+    e, f, v = run_gpu(m, nb, np_dtype)
+    eps = np.finfo(np_dtype).eps
+    for b in (0, 1, batch // 2, batch - 1):
+        one = {k: a[b:b + 1] if isinstance(a, np.ndarray) else a for k, a in nb.items()}
+        e1, f1, v1 = run_gpu(m, one, np_dtype)
+        # (the roundings of test_every_launch_gives_the_same; the sums of a structure grow with its rows)
+        assert np.abs(f[b] - f1[0]).max() <= 1200 * eps * np.abs(f1).max()
+        assert np.abs(e[b] - e1[0]).max() <= 1200 * eps * copies * max(np.abs(e1).max(), 1.0)
+        assert np.abs(v[b] - v1[0]).max() <= 1200 * eps * copies * max(np.abs(v1).max(), 1.0)
