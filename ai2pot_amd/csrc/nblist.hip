@@ -416,6 +416,8 @@ __device__ __forceinline__ int locate(const Grid<T>& g, const T (&xp)[3], int m,
 // first told by comparisons alone (of 27 images of most atoms one is in reach), and those in reach then go to their bins
 // IMAGES_AT_ONCE together.  Image by image the two kernels took 24.3 + 37.9 instead of 22.4 + 35.0 us for 1,048,576 atoms in fp32, and
 // a build of 131,072 atoms in fp64 with sorted rows 244 instead of 236.
+// The second one's workgroups go to the XCDs in runs, so that a bin's records are written through one L2: 34.8 -> 29.7 us there, 13.5 ->
+// 12.3 at 131,072 atoms in fp64 (the first one, which only counts, 8.2 -> 9.4 that way).
 constexpr int IMAGES_AT_ONCE = 4;
 template <typename T>
 __global__ void count_kernel(const Grid<T> g_in, const T* __restrict__ x, int* __restrict__ counts,
@@ -457,7 +459,7 @@ __global__ void fill_kernel(const Grid<T> g_in, const T* __restrict__ x, const i
                             const GridDyn<T>* __restrict__ gd, int split)
 {
     const Grid<T> g = with_dyn(g_in, gd);
-    const int t = blockIdx.x * NBL_BLOCK + threadIdx.x;
+    const int t = xcd_block(blockIdx.x, gridDim.x) * NBL_BLOCK + threadIdx.x;
     const int p = split > 1 ? t / split : t;
     if (p >= g.N) return;
     const int i0 = split > 1 ? t - p * split : 0, i1 = split > 1 ? i0 + 1 : g.img_dim[0];
@@ -885,11 +887,12 @@ __device__ __forceinline__ unsigned spread3(unsigned v)      // 10 bits -> every
 
 // xs[position] = x[order[position]]: the list kernel then reads its atoms' coordinates without first
 // waiting for the order; and the inverse of the order
+// (workgroups to the XCDs in runs: 10.9 -> 8.5 us at 1,048,576 atoms)
 template <typename T>
 __global__ void sorted_coords_kernel(int N, const T* __restrict__ x, const int* __restrict__ order, T* __restrict__ xs,
                                      int* __restrict__ inv)
 {
-    const int p = blockIdx.x * NBL_BLOCK + threadIdx.x;
+    const int p = xcd_block(blockIdx.x, gridDim.x) * NBL_BLOCK + threadIdx.x;
     if (p >= N) return;
     const int at = min(max(order[p], 0), N - 1);
     inv[at] = p;                                  // atom -> position: the index the compact entries carry
@@ -1142,9 +1145,11 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     __shared__ unsigned char sh_col[NBL_BLOCK / 64][NBL_APW][NBL_ENT_CAP + NBL_RUN];   // column of each flat candidate
     extern __shared__ __align__(16) unsigned char sh_rows[];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // (In processing order an XCD takes a run of workgroups, as the kernels behind do: 569 -> 556 us at 1,048,576 atoms; in the
+    // caller's order that gained nothing, sorted rows of 131,072 atoms 141 -> 144 us.)
     // the wave's first position, in a scalar register: the loads of its atoms' indices and coordinates are then
     // scalar loads
-    const int p0 = __builtin_amdgcn_readfirstlane((blockIdx.x * (NBL_BLOCK / 64) + wv) * NBL_APW);
+    const int p0 = __builtin_amdgcn_readfirstlane(((COMPACT ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * (NBL_BLOCK / 64) + wv) * NBL_APW);
     if (p0 >= g.N) return;                        // whole wave leaves together
     const int np = min(NBL_APW, g.N - p0);
     T* rb_rcs = nullptr;

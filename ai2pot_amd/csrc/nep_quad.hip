@@ -21,8 +21,8 @@
 // Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 21.7 us
 // (28 for the same atoms in no spatial order), 20,011 with skin lists 94 -> 53, 64 structures of 128 atoms 43 -> 24.5.
 // Of the 42 thousand cycles of a wavefront at 4096 atoms the tables take 5.2 (8.2 with a load to a value and the number of rows
-// waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6.  Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq
-// by fours (57 -> 58).
+// waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6.
+// Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq by fours (57 -> 58).
 //
 // Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
 #include "a2p_common.h"
