@@ -305,8 +305,7 @@ int finish_energy_virial(T* etot, T* virial, const double* partial, int B, int n
 int fill_zero(void* ptr, size_t bytes, hipStream_t stream);
 int fill_zero2(void* ptr, size_t bytes, void* ptr2, size_t bytes2, hipStream_t stream);   // two ranges, one launch
 
-// out[i] = in[0] + ... + in[i-1] for i < n (out must not alias in); tmp holds
-// scan_tmp_ints(n) ints, and tmp[ceil(n/2048)] receives the total.
+// out[i] = in[0] + ... + in[i-1] for i < n (out must not alias in); tmp holds scan_tmp_ints(n) ints.
 int scan_tmp_ints(int n);
 int exclusive_scan_i32(const int* in, int* out, int n, int* tmp, hipStream_t stream);
 

@@ -210,34 +210,6 @@ __device__ __forceinline__ void extents_of_axis(const Grid<T>& g, int a, T* out)
     out[9 + a] = hi > (T)INT_MIN ? hi : (T)INT_MIN;
 }
 
-// 6 wavefronts, one per extreme of the atoms, then the extents (minima of the image coordinates, their maxima, minima and
-// maxima of the centre atoms, three axes each)
-template <typename T>
-__global__ void minmax_finish_kernel(const Grid<T> g, const T* __restrict__ partial, int nblocks, T* __restrict__ out)
-{
-    __shared__ T ext[12];
-    const int q = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const bool is_min = q < 3;
-    T r = is_min ? (T)INFINITY : (T)-INFINITY;
-    for (int k0 = lane; k0 < nblocks; k0 += 64 * 8) {
-        T o[8];                                    // eight loads in flight
-#pragma unroll
-        for (int u = 0; u < 8; u++) o[u] = partial[(size_t)min(k0 + 64 * u, nblocks - 1) * 6 + q];
-#pragma unroll
-        for (int u = 0; u < 8; u++) r = is_min ? (o[u] < r ? o[u] : r) : (o[u] > r ? o[u] : r);
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const T o = __shfl_xor(r, off, 64);
-        r = is_min ? (o < r ? o : r) : (o > r ? o : r);
-    }
-    if (lane == 0) ext[6 + q] = r;
-    __syncthreads();
-    if (threadIdx.x < 3) extents_of_axis<T>(g, (int)threadIdx.x, ext);
-    __syncthreads();
-    if (threadIdx.x < 12) out[threadIdx.x] = ext[threadIdx.x];
-}
-
 // ---- 1b. bin grid from the extents, on the device (builds that do not read the extents back) ----------
 // The arithmetic of find_pl_info4nblist and of the bin counts (structure.h:1013-1061, binLinkedList.h:685-688) as
 // the host does it in the synchronised build, in T with correctly rounded operations.  The box must fit the
@@ -274,24 +246,54 @@ __device__ __forceinline__ bool grid_axis(const Grid<T>& g, const T* ext, GridDy
     return ok;
 }
 
+// 6 wavefronts, one per extreme of the atoms, then the extents (minima of the image coordinates, their maxima, minima and
+// maxima of the centre atoms, three axes each).  They go to the host by the kernel itself (slot, where there is one: out holds
+// them for a copy otherwise), or become the grid here (gd; three axes side by side): one launch less than with a kernel that
+// posts them or sets up the grid behind this one (with the scan's two, below, a step of 20,000 atoms 102 -> 96 us, of 1,048,576
+// 1515 -> 1503, a list of 8,000 75 -> 69).
 template <typename T>
-__global__ void grid_setup_kernel(const Grid<T> g, const T* __restrict__ ext, GridDyn<T>* __restrict__ gd, int cap0,
-                                  int cap1, int cap2, double big_bound, int* __restrict__ status)
+__global__ void __launch_bounds__(6 * 64)
+minmax_finish_kernel(const Grid<T> g, const T* __restrict__ partial, int nblocks, T* __restrict__ out, int* slot, int seq,
+                     GridDyn<T>* __restrict__ gd, int cap0, int cap1, int cap2, double big_bound, int* __restrict__ status)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const int cap[3] = {cap0, cap1, cap2};
-    bool ok = true;
-    long long nregion = 1;
-    for (int a = 0; a < 3; a++) {
-        if (!grid_axis<T>(g, ext, gd, a, cap[a], big_bound)) ok = false;
-        nregion *= gd->rdim[a] > 0 ? gd->rdim[a] : 0;
+    __shared__ T ext[12];
+    __shared__ GridDyn<T> dyn;
+    __shared__ int sh_ok[3];
+    const int tid = (int)threadIdx.x, q = tid >> 6, lane = tid & 63;
+    const bool is_min = q < 3;
+    T r = is_min ? (T)INFINITY : (T)-INFINITY;
+    for (int k0 = lane; k0 < nblocks; k0 += 64 * 8) {
+        T o[8];                                    // eight loads in flight
+#pragma unroll
+        for (int u = 0; u < 8; u++) o[u] = partial[(size_t)min(k0 + 64 * u, nblocks - 1) * 6 + q];
+#pragma unroll
+        for (int u = 0; u < 8; u++) r = is_min ? (o[u] < r ? o[u] : r) : (o[u] > r ? o[u] : r);
     }
-    if (!ok) {
-        for (int a = 0; a < 3; a++) { gd->rdim[a] = 0; gd->keep_lo[a] = (T)1; gd->keep_hi[a] = (T)-1; }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+        const T o = __shfl_xor(r, off, 64);
+        r = is_min ? (o < r ? o : r) : (o > r ? o : r);
+    }
+    if (lane == 0) ext[6 + q] = r;
+    __syncthreads();
+    if (tid < 3) {
+        extents_of_axis<T>(g, tid, ext);
+        if (gd) sh_ok[tid] = grid_axis<T>(g, ext, &dyn, tid, tid == 0 ? cap0 : tid == 1 ? cap1 : cap2, big_bound) ? 1 : 0;
+    }
+    __syncthreads();
+    if (tid < 12) out[tid] = ext[tid];
+    if (tid != 0) return;
+    if (slot) read_back_store(slot, seq, (const int*)ext, (int)(sizeof(ext) / 4));
+    if (!gd) return;
+    long long nregion = 1;
+    for (int a = 0; a < 3; a++) nregion *= dyn.rdim[a] > 0 ? dyn.rdim[a] : 0;
+    if (!(sh_ok[0] && sh_ok[1] && sh_ok[2])) {
+        for (int a = 0; a < 3; a++) { dyn.rdim[a] = 0; dyn.keep_lo[a] = (T)1; dyn.keep_hi[a] = (T)-1; }
         nregion = 0;
         atomicOr(status, ST_GRID_BOUND);
     }
-    gd->nregion = (int)nregion;
+    dyn.nregion = (int)nregion;
+    *gd = dyn;
 }
 
 // ---- 2 / 4. binning of (atom, image) pairs ---------------------------------------------------
@@ -1866,7 +1868,7 @@ struct CompactOut {
 // ---- builds that do not read the extents back (a2p_nblist_sync_free) -----------------------------------
 // The synchronised build remembers, per host thread, the bin box it found for a structure (device, natoms, lattice,
 // cutoff, periodicity).  With the switch on, a later build of the same structure sizes its launches and scratch
-// arrays for that box plus a margin, derives the actual box on the device (grid_setup_kernel) and never waits
+// arrays for that box plus a margin, derives the actual box on the device (minmax_finish_kernel) and never waits
 // for the stream; a box that outgrows the bound empties the lists and raises ST_GRID_BOUND.
 struct GridBound {
     bool valid = false;
@@ -2120,9 +2122,13 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(mm_blocks), dim3(NBL_BLOCK), 0, stream, g, coords, x_out,
                        partial);
     prof_end(stream);
-    prof_begin("nbl_coords_minmax", stream);
-    hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(6 * 64), 0, stream, g, (const T*)partial, mm_blocks, ext_dev);
-    prof_end(stream);
+    auto finish = [&](int* slot, int seq, double big) -> hipError_t {
+        prof_begin("nbl_coords_minmax", stream);
+        hipLaunchKernelGGL(minmax_finish_kernel<T>, dim3(1), dim3(6 * 64), 0, stream, g, (const T*)partial, mm_blocks, ext_dev, slot, seq, gd,
+                           cap[0], cap[1], cap[2], big, status);
+        prof_end(stream);
+        return hipGetLastError();
+    };
     if (sync_free) {
         for (int a = 0; a < 3; a++) {
             g.rdim[a] = cap[a];                         // host copies of the box serve launch and scratch sizes only
@@ -2133,11 +2139,16 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         rc = ws_get(WS_GRID, 256, &wsG);
         if (rc) return rc;
         gd = (GridDyn<T>*)wsG;
-        hipLaunchKernelGGL(grid_setup_kernel<T>, dim3(1), dim3(64), 0, stream, g, (const T*)ext_dev, gd, cap[0], cap[1],
-                           cap[2], big_coord, status);
+        A2P_HIP_CHECK(finish(nullptr, 0, big_coord));
     } else {
         T ext[12];
-        rc = read_back(ext_dev, (int)(sizeof(ext) / 4), ext, stream);
+        ReadBack rb;
+        int* const slot = read_back_take((int)(sizeof(ext) / 4), stream, &rb);
+        rb.src = ext_dev;                               // (copied when no slot is free)
+        const hipError_t launched = finish(slot, rb.seq, 0.0);
+        if (launched != hipSuccess) read_back_drop(rb);
+        A2P_HIP_CHECK(launched);
+        rc = read_back_wait(rb, ext);
         if (rc) return rc;
 
         // find_pl_info4nblist + bin counts (structure.h:1013-1061, binLinkedList.h:685-688)
