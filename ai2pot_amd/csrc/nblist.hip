@@ -153,12 +153,16 @@ __device__ __forceinline__ void image_extremes(const Grid<T>& g, int a, T c_lo, 
 // kernel waits for, and the kernel behind it has fewer values to compare
 // (1,048,576 atoms, fp32: 19.1 -> 10.9 and 13.5 -> 4.6 us with 1024 instead of 4096 workgroups; 7.3 and 4.5 since the images'
 // extremes are taken from the atoms' and Cartesian coordinates are not copied).
+// On the way it clears the bins' counters and cursors, `nclear` times four of them: a launch less (a step of 9,000 atoms 81 -> 78 us,
+// of 20,000 96 -> 94.5; 1,048,576: 6.8 -> 8.4 us instead of 5.7 apart).  (Counting the counters down again instead of a cursor: the
+// kernel that places the records 5.5 -> 7.4 and 29.4 -> 31.5 us.)
 constexpr int MINMAX_BLOCKS = 1024;
 
 template <typename T>
 __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coords, T* __restrict__ x,
-                                     T* __restrict__ partial)
+                                     T* __restrict__ partial, int4* __restrict__ counts, int nclear)
 {
+    for (int i = blockIdx.x * NBL_BLOCK + threadIdx.x; i < nclear; i += gridDim.x * NBL_BLOCK) counts[i] = make_int4(0, 0, 0, 0);
     __shared__ T sh[NBL_BLOCK / 64][6];
     T v[6];                                             // minima and maxima of the atoms (a NaN is passed by)
 #pragma unroll
@@ -2117,10 +2121,33 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     int split = 1, *cursor = nullptr;
     dim3 image_grid;
     if (!small) {
+    // Workspace B: counts[room] | cursor[room] (and up to three behind it) | offsets[room] | scan tmp, for as many bins as atoms inside the cell can have, or as the bound
+    // allows for, and one; counts and cursors are cleared before the box is known, unless they are many to an atom.
+    double bins = 1;
+    for (int a = 0; a < 3; a++) {
+        const double len = std::fabs((double)g.b[0][a]) + std::fabs((double)g.b[1][a]) + std::fabs((double)g.b[2][a]);
+        bins *= sync_free ? (double)cap[a] : std::ceil(len / (double)g.bin_size) + 2 + 2 * g.ext_bins;
+    }
+    int room = bins < 8.0 * N + 16384 && bins < (double)(1 << 28) ? (int)bins + 1 : 0;
+    int *counts = nullptr, *tmp = nullptr;
+    auto bin_room = [&](int n) -> int {
+        void* wsB = nullptr;
+        const int got = ws_get(WS_NBL_B, ((size_t)n * 3 + 4 + scan_tmp_ints(n)) * sizeof(int), &wsB);
+        if (got) return got;
+        counts = (int*)wsB;
+        cursor = counts + n;
+        offsets = cursor + n + 4;
+        tmp = offsets + n;
+        return A2P_OK;
+    };
+    if (room) {
+        rc = bin_room(room);
+        if (rc) return rc;
+    }
     prof_begin("nbl_coords_minmax", stream);
     const int mm_blocks = std::min(nblocks, MINMAX_BLOCKS);
     hipLaunchKernelGGL(coords_minmax_kernel<T>, dim3(mm_blocks), dim3(NBL_BLOCK), 0, stream, g, coords, x_out,
-                       partial);
+                       partial, (int4*)counts, (2 * room + 3) / 4);
     prof_end(stream);
     auto finish = [&](int* slot, int seq, double big) -> hipError_t {
         prof_begin("nbl_coords_minmax", stream);
@@ -2185,19 +2212,12 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     }
     const int nb1 = (int)nregion + 1;
 
-    // workspace B: counts[nb1] | offsets[nb1] | cursor[nb1] | scan tmp, then (after the count is
-    // known) the image records s_rec[total][4], and for sort: keys[N*umax] | order[N*umax] | tmp rows
-    const int ntmp = scan_tmp_ints(nb1);
-    size_t ints = (size_t)nb1 * 3 + ntmp;
-    void* wsB = nullptr;
-    rc = ws_get(WS_NBL_B, ints * sizeof(int), &wsB);
-    if (rc) return rc;
-    int* counts = (int*)wsB;
-    offsets = counts + nb1;
-    cursor = offsets + nb1;
-    int* tmp = cursor + nb1;
-    rc = fill_zero2(counts, (size_t)nb1 * sizeof(int), cursor, (size_t)nb1 * sizeof(int), stream);
-    if (rc) return rc;
+    if (nb1 > room) {
+        rc = bin_room(nb1);
+        if (rc) return rc;
+        rc = fill_zero(counts, 2 * (size_t)nb1 * sizeof(int), stream);
+        if (rc) return rc;
+    }
     // binning: a thread per atom, or per x-layer of an atom's images while the structure is small
     split = (N < 65536 && g.img_dim[0] > 1) ? g.img_dim[0] : 1;
     image_grid = dim3(ceil_div((long long)N * split, NBL_BLOCK));

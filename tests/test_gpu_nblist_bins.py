@@ -12,8 +12,10 @@ RCUT, UMAX, N = 6.0, 200, 4999                       # (more atoms than are binn
 
 # bins of half the cutoff; one more than their number is summed up: in tiles of 4096 by one launch up to 16 of them, in tiles of
 # 2048 by two up to 2048 of them, by three beyond
-@pytest.mark.parametrize("dims", [(63, 65, 1), (64, 64, 1), (64, 64, 15), (64, 16, 64), (41, 40, 41), (255, 128, 128), (256, 128, 128)])
-def test_every_pair_once(dims):
+# Their counters are cleared ahead for the bins of a cell's size (none for the largest boxes): half a cell has fewer than there are.
+@pytest.mark.parametrize("dims,cell", [((63, 65, 1), 1.0), ((64, 64, 1), 1.0), ((64, 64, 15), 1.0), ((64, 64, 15), 0.5), ((64, 16, 64), 1.0), ((41, 40, 41), 1.0),
+                                       ((255, 128, 128), 1.0), ((256, 128, 128), 1.0)])
+def test_every_pair_once(dims, cell):
     rng = np.random.default_rng(sum(dims))
     top = (np.array(dims) - 0.5) * RCUT / 2           # the corners fix the box
     # places 1.5 apart, moved by up to 0.5: none closer than 0.5; a third of the atoms in a part of the box, so that the largest
@@ -27,7 +29,7 @@ def test_every_pair_once(dims):
     x = np.concatenate([[[0.0] * 3, top], np.minimum((x + 0.5) * 1.5 + rng.uniform(-0.5, 0.5, x.shape), top - 0.01)])
     x = x[np.linalg.norm(x - top, axis=1) + (np.arange(len(x)) == 1) > 0.6]
     n = len(x)
-    lattice = np.diag(top + 40.0)
+    lattice = np.diag((top + 40.0) * cell)
     out = find_info4mlff_device(lattice, torch.zeros(n, dtype=torch.int32, device="cuda:0"), torch.from_numpy(x).to("cuda:0"), RCUT, UMAX,
                                 True, (False, False, False))
     count, first = out[2].cpu().numpy().reshape(n), out[3].cpu().numpy().reshape(n, UMAX)
