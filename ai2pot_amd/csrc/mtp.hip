@@ -2373,8 +2373,9 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         int cut[2] = {MTP_SLOT_CAP, MTP_SLOT_CAP};
         long long pieces = -1;
         if (lists.longest > 64 * MTP_SLOT_CAP) { too_long = true; return Best(); }
-        // (the longest lists hold more in pairs than as they were given)
-        for (int cap = 2; cap <= MTP_SLOT_CAP || cost[0] < 0; cap += 2) {
+        // (whole steps: between them a cut makes more pieces and no fewer steps; the longest lists hold more in pairs than as they
+        // were given)
+        for (int cap = MTP_DEPTH_STEP; cap <= MTP_SLOT_CAP || cost[0] < 0; cap += MTP_DEPTH_STEP) {
             if (longest > 64 * cap) continue;
             long long np = 0;
             for (int m : ms) np += pieces_of(lists.size(m), cap);
@@ -2399,6 +2400,13 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     auto build_ell = [](const Lists& lists, const std::vector<Best>& levels, int wide,
                         const Lists* leaf_lists = nullptr, const Best* leaves = nullptr) {
         Ell e;
+        size_t terms = 0, lanes = 0;
+        auto count = [&](const Level& lv) { for (int d : lv.depth) { terms += (size_t)d * 64; lanes += 64; } };
+        for (const Best& b : levels) count(b.lv[wide]);
+        if (leaves) count(leaves->lv[wide]);
+        e.terms.reserve(terms);
+        e.slot.reserve(lanes);
+        e.lead.reserve(lanes);
         auto append = [&](const Lists& lists, const Level& best, int kind) {
             for (size_t g = 0; g < best.depth.size(); g++) {
                 e.group.push_back(make_int4((int)e.terms.size(), best.depth[g], best.steps[g], kind));
@@ -2438,6 +2446,10 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 seq[w].push_back({q, g});
             }
         }
+        size_t steps = 2;
+        for (const int4& info : e.group) steps += (info.y + MTP_DEPTH_STEP - 1) / MTP_DEPTH_STEP;
+        st.words.reserve(steps * MTP_STEP_WORDS);
+        st.ctrl.reserve(steps + 64);
         for (int w = 0; w < waves; w++) {
             const int first = (int)st.ctrl.size();
             for (size_t i = 0; i < seq[w].size(); i++) {
@@ -2507,7 +2519,7 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
     // The streams that a launch can ask for: those of the widths that wide_atoms gives for as many moments, and the forward one
     // of four wavefronts for the components.  (Host time of a plan with all of them and every cut laid out for each by itself
-    // 1.83 ms for level 16 and 14.2 for level 20, with the streams reached alone 0.78 and 4.2, in pairs of a multiplicity 1.2 and 5.6.)
+    // 1.83 ms for level 16 and 14.2 for level 20, with the streams reached alone 0.78 and 4.2, in pairs of a multiplicity 0.77 and 4.1.)
     bool reached[2] = {false, false};
     for (int q = 0; q < 8; q++) reached[wide_atoms(n_moms, q & 1, q & 2, q & 4)] = true;
     Stream fs[2], rs[2], cs[2], vs[2];
