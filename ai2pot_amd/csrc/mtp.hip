@@ -1876,9 +1876,12 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
 }
 
 // Force column of every atom: its own row's sum minus the pairs that name it, in the order of their places in the lists; on the
-// way these pairs' virial.  The pairs arrive in any order: a workgroup (one wavefront) ranks those of its atom in LDS, up to
-// COMP_SORT of them; a longer list is walked from each place to the next larger one.  Columns from S on (species counts) are
-// zero.
+// way these pairs' virial.  The pairs arrive in any order: a wavefront ranks those of its atom in LDS, up to COMP_SORT of them; a
+// longer list is walked from each place to the next larger one.  Columns from S on (species counts) are zero.  A workgroup takes
+// COMP_ROWS atoms in a row and sums up their virials, and the energies of as many rows, in order: written by each wavefront and
+// summed by a kernel of its own they were 55 MB out and in at 64 structures of 128 atoms, 15 us beside 2 x 42, and the kernel that
+// sums the workgroups took 8 with a thread to a column, now 5 with one to each of its ten values; the call 421 -> 402 us.  (Eight
+// atoms to a workgroup: two of them fit no compute unit at the 156 registers of two columns in fp64, and at 128 112 bytes spill.)
 // Bound by the reads of the pair derivatives, under which the virial's operations hide (in mtp_components_kernel they took a
 // fifth of its instructions and the registers of four more reads in flight); sorting the lists by insertion, one thread per
 // atom, used to take as long as they do (95 us beside 98 us at 64 structures of 128 atoms).
@@ -1887,20 +1890,42 @@ comp_incoming_kernel(int B, int P, int U, const int* __restrict__ nnc, const int
 // to a lane and two, 6,400 atoms: 53 columns 40.0 and 42.9 us, 65 67.6 and 56.4, 93 85.1 and 72.7, 127 109.5 and 97.5, 151 136.6 and
 // 136.4, 261 243.6 and 249.3 (a last block half of which has no column); fp32 24.9 and 27.0, 38.2 and 28.5, 52.8 and 38.0, 65.5 and
 // 52.6, 83.3 and 75.4, 130.5 and 122.7; 160 atoms, 93 columns 11.6 and 12.8.
-constexpr int COMP_SORT = 256, COMP_DISP = 128;
+constexpr int COMP_SORT = 256, COMP_DISP = 128, COMP_ROWS = 4;
 
 template <typename T, int NC>
-__global__ void __launch_bounds__(64)
-comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
+__global__ void __launch_bounds__(64 * COMP_ROWS, 3)
+comp_force_kernel(int S, int n, int P, int cap, int U, int b0, const int* __restrict__ binum, const int* __restrict__ bilist,
+                  const int* __restrict__ btypes, const int* __restrict__ pair_off, const int* __restrict__ row_of1, const int* __restrict__ cnt,
                   const int* __restrict__ seg, const int* __restrict__ inc, const T* __restrict__ brcs, const T* __restrict__ pb,
-                  const T* __restrict__ rowpart, T* __restrict__ vpart, T* __restrict__ fcomp)
+                  const T* __restrict__ rowpart, const T* __restrict__ desc, T* __restrict__ part, T* __restrict__ fcomp)
 {
-    __shared__ int list[COMP_SORT], order[COMP_SORT];
-    __shared__ T disp[COMP_DISP][3];
-    const int t = blockIdx.x + row0, lane = threadIdx.x, col0 = blockIdx.y * 64 * NC + lane;
+    struct Own { int list[COMP_SORT], order[COMP_SORT]; T disp[COMP_DISP][3]; };
+    constexpr int COLS = 64 * NC;
+    __shared__ union { Own own[COMP_ROWS]; T vir[COMP_ROWS][3][COLS]; } sh;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int nblocks = (P + COMP_ROWS - 1) / COMP_ROWS, bb = blockIdx.x / nblocks, blk = blockIdx.x - bb * nblocks, b = b0 + bb;
+    const int first = b * P + blk * COMP_ROWS, t = first + wave, col0 = blockIdx.y * COLS + lane;
+    const bool there = blk * COMP_ROWS + wave < P;
+    int* const list = sh.own[wave].list;
+    int* const order = sh.own[wave].order;
+    T (* const disp)[3] = sh.own[wave].disp;
+    auto wave_sync = [&]() __attribute__((always_inline)) {           // (what a wavefront keeps in LDS is its own)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    T f[NC][3], vir[NC][9];
+#pragma unroll
+    for (int c = 0; c < NC; c++) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) vir[c][i] = (T)0;
+#pragma unroll
+        for (int i = 0; i < 3; i++) f[c][i] = (T)0;
+    }
+    if (there) {
     const int* v = inc + (seg ? (size_t)seg[t] : (size_t)t * cap);
     const int m = seg ? seg[t + 1] - seg[t] : min(cnt[t], cap);
-    const int r1 = row_of1[t], base = pair_off[row0];    // pb holds the pairs from row0 on
+    const int r1 = row_of1[t], base = pair_off[(size_t)b0 * P];          // pb holds the pairs from structure b0 on
     const bool ranked = m <= COMP_SORT;
     int s[NC];
 #pragma unroll
@@ -1908,7 +1933,7 @@ comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict_
     auto pair_of = [&](int q) __attribute__((always_inline)) { const int row = q / U; return pair_off[row] + (q - row * U) - base; };
     if (ranked) {
         for (int k = lane; k < m; k += 64) list[k] = v[k];
-        __syncthreads();
+        wave_sync();
         int place[COMP_SORT / 64];
 #pragma unroll
         for (int u = 0; u < COMP_SORT / 64; u++) {
@@ -1927,27 +1952,23 @@ comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict_
 #pragma unroll
                 for (int q = 0; q < 3; q++) disp[r][q] = d[q];
         }
-        __syncthreads();
+        wave_sync();
         if (m > COMP_DISP) {                             // the places in the lists too, in order
             int x[COMP_SORT / 64];
 #pragma unroll
             for (int u = 0; u < COMP_SORT / 64; u++)
                 if (u * 64 + lane < m) x[u] = list[u * 64 + lane];
-            __syncthreads();
+            wave_sync();
 #pragma unroll
             for (int u = 0; u < COMP_SORT / 64; u++)
                 if (u * 64 + lane < m) list[place[u]] = x[u];
-            __syncthreads();
+            wave_sync();
         }
     }
-    T f[NC][3], vir[NC][9];
 #pragma unroll
-    for (int c = 0; c < NC; c++) {
-#pragma unroll
-        for (int i = 0; i < 9; i++) vir[c][i] = (T)0;
+    for (int c = 0; c < NC; c++)
 #pragma unroll
         for (int i = 0; i < 3; i++) f[c][i] = r1 > 0 ? rowpart[((size_t)(r1 - 1) * 3 + i) * S + s[c]] : (T)0;
-    }
     auto take = [&](const T (&g)[NC][3], T d0, T d1, T d2) __attribute__((always_inline)) {
 #pragma unroll
         for (int c = 0; c < NC; c++)
@@ -2007,71 +2028,63 @@ comp_force_kernel(int S, int n, int cap, int U, int row0, const int* __restrict_
         if (col < n)
 #pragma unroll
             for (int i = 0; i < 3; i++) fcomp[((size_t)t * 3 + i) * n + col] = col < S ? f[c][i] : (T)0;
-        if (col < S)
-#pragma unroll
-            for (int i = 0; i < 9; i++) vpart[((size_t)t * 9 + i) * S + col] = vir[c][i];
     }
-}
-
-// Energy and virial columns per structure: sums over the rows (virial: the atoms that the pairs name) in order, in two steps (blocks of COMP_ROWS rows, then
-// the blocks); part[B][nblocks][10][n].  Column S + t counts the rows whose centre has species t; its virial is zero.
-// The first step reads 80 bytes per row and column: short blocks (8 rows: 25 -> 8 us against 32 at 64 x 128 rows) keep
-// enough wavefronts in flight.
-constexpr int COMP_ROWS = 8;
-
-template <typename T>
-__global__ void __launch_bounds__(64)
-comp_structure_blocks_kernel(int S, int n, int P, int nblocks, const int* __restrict__ binum,
-                             const int* __restrict__ bilist, const int* __restrict__ btypes, const T* __restrict__ desc,
-                             const T* __restrict__ vpart, T* __restrict__ part)
-{
-    const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x, blk = blockIdx.z;
-    if (s >= n) return;
-    T e = (T)0, v[9];
+    }
+    // the sums of the atoms of the workgroup, in order: three components at a time through the lists' place
+    T* const out = part + ((size_t)b * nblocks + blk) * 10 * n;
+    const int here = min(COMP_ROWS, P - blk * COMP_ROWS);
 #pragma unroll
-    for (int i = 0; i < 9; i++) v[i] = (T)0;
-    const int i0 = blk * COMP_ROWS, i1 = min(binum[b], i0 + COMP_ROWS);
-    if (s < S) {
-#pragma unroll 4
-        for (int ii = i0; ii < min(P, i0 + COMP_ROWS); ii++) {
-            const size_t row = (size_t)b * P + ii;
-            if (ii < i1) e += desc[row * S + s];
-            const T* o = vpart + row * 9 * S + s;
+    for (int q = 0; q < 3; q++) {
+        __syncthreads();
+        if (there)
 #pragma unroll
-            for (int i = 0; i < 9; i++) v[i] += o[(size_t)i * S];
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int i = 0; i < 3; i++) sh.vir[wave][i][c * 64 + lane] = vir[c][q * 3 + i];
+        __syncthreads();
+        for (int o = threadIdx.x; o < 3 * COLS; o += 64 * COMP_ROWS) {
+            const int i = o / COLS, c = o - i * COLS, col = blockIdx.y * COLS + c;
+            if (col >= n) continue;
+            T sum = (T)0;
+            if (col < S)
+                for (int w = 0; w < here; w++) sum += sh.vir[w][i][c];
+            out[(size_t)(1 + q * 3 + i) * n + col] = sum;
         }
-    } else {
-        int c[COMP_ROWS];
-#pragma unroll
-        for (int u = 0; u < COMP_ROWS; u++) c[u] = i0 + u < i1 ? bilist[(size_t)b * P + i0 + u] : -1;
-#pragma unroll
-        for (int u = 0; u < COMP_ROWS; u++)
-            if ((unsigned)c[u] < (unsigned)P && btypes[(size_t)b * P + c[u]] == s - S) e += (T)1;
     }
-    T* o = part + ((size_t)b * nblocks + blk) * 10 * n + s;
-    o[0] = e;
+    // ... and the energies of the rows; column S + t counts those whose centre has species t
+    const int rows = min(COMP_ROWS, binum[b] - blk * COMP_ROWS);
+    for (int c = threadIdx.x; c < COLS; c += 64 * COMP_ROWS) {
+        const int col = blockIdx.y * COLS + c;
+        if (col >= n) continue;
+        T e = (T)0;
+        if (col < S) {
 #pragma unroll
-    for (int i = 0; i < 9; i++) o[(size_t)(1 + i) * n] = v[i];
+            for (int u = 0; u < COMP_ROWS; u++)
+                if (u < rows) e += desc[(size_t)(first + u) * S + col];
+        } else {
+            for (int u = 0; u < rows; u++) {
+                const int center = bilist[first + u];
+                if ((unsigned)center < (unsigned)P && btypes[(size_t)b * P + center] == col - S) e += (T)1;
+            }
+        }
+        out[col] = e;
+    }
 }
 
+// Energy and virial columns per structure: the workgroups' sums (comp_force_kernel) in order; part[B][nblocks][10][n].
 template <typename T>
 __global__ void __launch_bounds__(64)
 comp_structure_kernel(int n, int S, int nblocks, const T* __restrict__ q_scaler, const T* __restrict__ part,
                       T* __restrict__ ecomp, T* __restrict__ vcomp)
 {
-    const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x;
+    const int b = blockIdx.x, s = blockIdx.y * 64 + threadIdx.x, i = blockIdx.z;        // (a component to a workgroup)
     if (s >= n) return;
-    T acc[10];
-#pragma unroll
-    for (int i = 0; i < 10; i++) acc[i] = (T)0;
-    for (int blk = 0; blk < nblocks; blk++) {
-        const T* o = part + ((size_t)b * nblocks + blk) * 10 * n + s;
-#pragma unroll
-        for (int i = 0; i < 10; i++) acc[i] += o[(size_t)i * n];
-    }
-    ecomp[(size_t)b * n + s] = s < S ? acc[0] / q_scaler[s] : acc[0];
-#pragma unroll
-    for (int i = 0; i < 9; i++) vcomp[((size_t)b * 9 + i) * n + s] = acc[1 + i];
+    const T* const o = part + ((size_t)b * nblocks * 10 + i) * n + s;
+    T acc = (T)0;
+#pragma unroll 16
+    for (int blk = 0; blk < nblocks; blk++) acc += o[(size_t)blk * 10 * n];
+    if (i == 0) ecomp[(size_t)b * n + s] = s < S ? acc / q_scaler[s] : acc;
+    else vcomp[((size_t)b * 9 + i - 1) * n + s] = acc;
 }
 
 // counts[b, t] += 1 for every evaluated row whose centre has species t (integer atomics: exact in any order)
@@ -3409,15 +3422,18 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         A2P_HIP_CHECK(hipGetLastError());
         in_seg = seg;
     }
-    // pair derivatives | row sums | virial by named atom | scalar moments
+    // pair derivatives | row sums | scalar moments
     const size_t n_pb = (size_t)std::max(npairs, 1) * 3 * S, n_rp = (size_t)rows * 3 * S, n_desc = (size_t)rows * S;
     void* wsT = nullptr;
-    rc = ws_get(WS_MTP, (n_pb + 4 * n_rp + n_desc) * sizeof(T), &wsT);
+    rc = ws_get(WS_MTP, (n_pb + n_rp + n_desc) * sizeof(T), &wsT);
     if (rc) return rc;
     T* pb = (T*)wsT;
     T* rowpart = pb + n_pb;
-    T* vpart = rowpart + n_rp;
-    T* desc = vpart + 3 * n_rp;
+    T* desc = rowpart + n_rp;
+    const int nblocks = ceil_div(P, COMP_ROWS);
+    void* wsP = nullptr;
+    rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * n * sizeof(T), &wsP);
+    if (rc) return rc;
 
     CompArgs<T> c;
     c.pb = pb; c.pair_off = pair_off; c.nnc = nnc; c.desc = desc; c.rowpart = rowpart;
@@ -3468,19 +3484,13 @@ int mtp_lin_components_nodes(MtpPlan* plan, MtpArgs<T>& a, int S, int n, T* ecom
         }
         prof_begin("mtp_components_sums", stream);
         auto sums = n > 64 ? comp_force_kernel<T, 2> : comp_force_kernel<T, 1>;
-        hipLaunchKernelGGL(sums, dim3(nb * P, ceil_div(n, n > 64 ? 128 : 64)), dim3(64), 0, stream, S, n, U, U, b0 * P,
-                           (const int*)pair_off, (const int*)row_of1,
-                           (const int*)cnt, in_seg, (const int*)inc, a.brcs, (const T*)pb, (const T*)rowpart, vpart, fcomp);
+        hipLaunchKernelGGL(sums, dim3(nb * nblocks, ceil_div(n, n > 64 ? 128 : 64)), dim3(64 * COMP_ROWS), 0, stream, S, n, P, U, U, b0, a.binum, a.bilist,
+                           a.btypes, (const int*)pair_off, (const int*)row_of1, (const int*)cnt, in_seg, (const int*)inc, a.brcs, (const T*)pb,
+                           (const T*)rowpart, (const T*)desc, (T*)wsP, fcomp);
         prof_end(stream);
     }
     prof_begin("mtp_components_sums", stream);
-    const int nblocks = ceil_div(P, COMP_ROWS);
-    void* wsP = nullptr;
-    rc = ws_get(WS_MISC, (size_t)B * nblocks * 10 * n * sizeof(T), &wsP);
-    if (rc) return rc;
-    hipLaunchKernelGGL(comp_structure_blocks_kernel<T>, dim3(B, ceil_div(n, 64), nblocks), dim3(64), 0, stream, S, n, P,
-                       nblocks, a.binum, a.bilist, a.btypes, (const T*)desc, (const T*)vpart, (T*)wsP);
-    hipLaunchKernelGGL(comp_structure_kernel<T>, dim3(B, ceil_div(n, 64)), dim3(64), 0, stream, n, S, nblocks, a.q_scaler,
+    hipLaunchKernelGGL(comp_structure_kernel<T>, dim3(B, ceil_div(n, 64), 10), dim3(64), 0, stream, n, S, nblocks, a.q_scaler,
                        (const T*)wsP, ecomp, vcomp);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());

@@ -489,6 +489,29 @@ def test_components_in_one_pass_equal_a_pass_per_column(oracle, level, nt, U):
         assert np.array_equal(a, c)                      # bit-reproducible
 
 
+@pytest.mark.parametrize("level", [10, 16])
+@pytest.mark.parametrize("sizes", [(1,), (3, 2), (4,), (5, 1), (8, 6, 3), (9,)])
+def test_components_of_few_atoms(oracle, level, sizes):
+    """Rows of structures that fill the sets of four which are summed together, begin one or leave one short."""
+    from ai2pot_amd import _lib, ops
+    import torch
+    m, nb, _ = loss_inputs(oracle, level, 2, sizes=sizes)
+    md, d = model_to_device(m, torch.float64), to_device(nb, torch.float64)
+    args = (m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+            md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], d["binum"], d["bilist"], d["bnumneigh"],
+            d["bfirstneigh"], d["brcs"], d["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"])
+    L = _lib.lib()
+    before = L.a2p_mtp_components_route(1)
+    try:
+        one = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+        L.a2p_mtp_components_route(0)
+        per_column = [t.cpu().numpy() for t in ops.mtp_lin_components(*args)]
+    finally:
+        L.a2p_mtp_components_route(before)
+    for a, b in zip(one, per_column):
+        assert close(a, b)
+
+
 def test_components_in_single_precision(oracle):
     """The fp32 instance of the one-pass components against the fp64 one (the plan's byte offsets are halved for
     4-byte moments)."""
