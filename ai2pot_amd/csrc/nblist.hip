@@ -25,6 +25,7 @@
 // operations with the *_rn intrinsics: no fused multiply-add may change a rounding.
 #include "a2p_common.h"
 #include "compact_list.h"
+#include "wave_ops.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -59,6 +60,7 @@ struct Grid {
     int nbin[3];      // the reference's bin counts
     int rlo[3];       // bin box kept here: [rlo, rlo + rdim)
     int rdim[3];
+    int zstride;      // offsets from one column of bins to the next: rdim[2], or one more where a column has an end of its own
     int img_lo[3];    // image index ranges
     int img_dim[3];
     int nimg;
@@ -81,7 +83,7 @@ template <typename T>
 struct GridDyn {
     T mn[3], keep_lo[3], keep_hi[3];
     int nbin[3], rlo[3], rdim[3];
-    int nregion;
+    int nregion, zstride;
 };
 
 template <typename T>
@@ -94,6 +96,7 @@ __device__ __forceinline__ Grid<T> with_dyn(const Grid<T>& in, const GridDyn<T>*
             g.mn[a] = gd->mn[a]; g.keep_lo[a] = gd->keep_lo[a]; g.keep_hi[a] = gd->keep_hi[a];
             g.nbin[a] = gd->nbin[a]; g.rlo[a] = gd->rlo[a]; g.rdim[a] = gd->rdim[a];
         }
+        g.zstride = gd->zstride;
     }
     return g;
 }
@@ -297,6 +300,7 @@ minmax_finish_kernel(const Grid<T> g, const T* __restrict__ partial, int nblocks
         atomicOr(status, ST_GRID_BOUND);
     }
     dyn.nregion = (int)nregion;
+    dyn.zstride = dyn.rdim[2];
     *gd = dyn;
 }
 
@@ -547,12 +551,14 @@ __global__ void binsort_kernel(int nbins, const int* __restrict__ offsets, T* __
 // Such a build is bound by the latency of nine short launches and of the wait for the extents (51 us of GPU time for
 // 4096 atoms, of which 38 in kernels).  Here every workgroup finds the extents and the grid for itself (the atoms are
 // few) and bins one slab of the box, a plane of bins across x or a few, with its counters in LDS: the images in its slab
-// are listed and dealt to their bins, those in the slabs before it are only counted, which says where its records begin,
-// and every record is written once, to its final place (an image's place in its bin is the number of larger image numbers
-// there).  No workgroup waits for another.  4096 atoms take 14.5 us in lattice order (16.9 in no spatial order; one workgroup
-// for the whole box, in lattice order: 31), of which extents and grid 5, finding the images 4, dealing them 3.
-// Told axis by axis (diagonal lattice, at most three images an axis), an image is placed by comparisons with the edges of
-// the box and of the slab; the exactly rounded division decides next to an edge only, and for the bins of the slab's own.
+// are listed and dealt to their bins, and every record is written once, to its final place (an image's place in its bin is the
+// number of larger image numbers there).  No workgroup waits for another: a slab's records have a place of their own, which has
+// room for every image that can be in it, and a column of bins ends with an offset of its own (zstride).  With the records of all
+// slabs back to back every workgroup counted the images before its own, of all atoms along all axes: 10 of 29 thousand cycles;
+// 4096 atoms in lattice order 14.5 -> 11.0 us, a step of theirs 47.7 -> 43.2, with the box on its way to the host before the images
+// are looked for.  (One workgroup for the whole box: 31.)
+// Told axis by axis (diagonal lattice, at most three images an axis), an image is kept by comparisons with the edges of
+// the slab, and exactly rounded division decides among those.
 // Other lattices are tried image by image.  Images of a slab beyond its LDS (atoms crowded into a corner of the cell are
 // within reach of eight cells each) pass through global memory instead.  What the grid turned out to be goes to the host
 // while the rest runs; a box beyond the LDS empties the lists and is reported, and the host then takes the general route.
@@ -577,13 +583,27 @@ __device__ __forceinline__ unsigned image_triple(const Grid<T>& g, int im)
 // posted to the host: [0] 1 if the lists are complete, [1..3] the box, [4..5] the largest |coordinate| kept (a double)
 constexpr int NBS_WORDS = 6;
 
+// the least or the largest over the wavefront, in every lane (a NaN is passed by)
+template <typename T>
+__device__ __forceinline__ T wave_extreme(T r, bool is_min)
+{
+    auto take = [&](T o) __attribute__((always_inline)) { r = is_min ? (o < r ? o : r) : (o > r ? o : r); };
+    take(wave::dpp_move<0x128>(r));                // row_ror: 8, 4, 2, 1
+    take(wave::dpp_move<0x124>(r));
+    take(wave::dpp_move<0x122>(r));
+    take(wave::dpp_move<0x121>(r));
+    take(__shfl_xor(r, 16, 64));
+    take(__shfl_xor(r, 32, 64));
+    return r;
+}
+
 template <typename T>
 __global__ void __launch_bounds__(NBS_THREADS)
 small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restrict__ x, GridDyn<T>* __restrict__ gd,
                   int* __restrict__ offsets, T* __restrict__ s_rec, const int* __restrict__ types, int* __restrict__ ilist,
                   int* __restrict__ types_out, int* __restrict__ incoming, int mark_types, int separable, int cap0, int cap1,
                   int cap2, double big_bound, int raise, int* __restrict__ status, int* slot, int seq,
-                  int* __restrict__ spare, int spare_images)
+                  int* __restrict__ spare, int room)
 {
     extern __shared__ __align__(16) unsigned char sh_small[];
     int* const cnt = (int*)sh_small;                             // per bin: count, then end of the bin's records
@@ -591,46 +611,48 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     int* const num = found + NBS_CAP;                            // ... and by bin
     unsigned short* const bin_of_found = (unsigned short*)(num + NBS_CAP);
     unsigned short* const work = bin_of_found + NBS_CAP;         // atom | image along x << 12
-    static_assert(NBS_LDS >= 6 * NBS_THREADS * sizeof(double), "the extremes pass through the counters' LDS");
+    static_assert(NBS_THREADS / 64 == 16, "waves 0 .. 5 and from 8 on");
+    static_assert(2 * NBS_CAP * sizeof(int) >= 6 * NBS_THREADS * sizeof(double), "the extremes pass through the place of the image numbers");
     __shared__ T ext[12];
     __shared__ GridDyn<T> dyn;
-    __shared__ int sh_ok[3], sh_scan[3][NBS_THREADS / 64], sh_bad, sh_found, sh_work;
+    __shared__ int sh_ok[3], sh_scan[NBS_THREADS / 64], sh_bad[NBS_THREADS / 64], sh_found, sh_work;
     __shared__ unsigned sh_triple[NBS_TRIPLES];                  // image number -> (i, j, k), 10 bits each
     const int tid = (int)threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int N = g_in.N;
-    if (tid == 0) { sh_bad = 0; sh_found = 0; sh_work = 0; }
-    __syncthreads();
+    if (tid == 0) { sh_found = 0; sh_work = 0; }
 
     // 1. coordinates, extents (image_extremes: those of the atoms are enough)
     constexpr int PER = NBS_ATOMS / NBS_THREADS;
     const int chunk = (N + (int)gridDim.x - 1) / (int)gridDim.x;          // the atoms whose outputs this workgroup writes
     const int own0 = chunk * (int)blockIdx.x, own1 = min(own0 + chunk, N);
-    T lo[3], hi[3];
+    static_assert(NBS_BINS % (4 * NBS_THREADS) == 0, "counters cleared by fours");
+#pragma unroll
+    for (int i = 0; i < NBS_BINS / 4; i += NBS_THREADS) ((int4*)cnt)[i + tid] = make_int4(0, 0, 0, 0);
+    if (tid < min(g_in.nimg, NBS_TRIPLES)) sh_triple[tid] = image_triple(g_in, tid);
+    T lo[3], hi[3], along[PER];                                  // (their coordinates along x)
     bool bad = false;
 #pragma unroll
     for (int a = 0; a < 3; a++) { lo[a] = (T)INFINITY; hi[a] = (T)-INFINITY; }
 #pragma unroll
     for (int r = 0; r < PER; r++) {
         const int p = tid + r * NBS_THREADS;
-        if (p >= N) break;
+        along[r] = (T)4.0e30;
+        if (p >= N) continue;
         T c[3];
         cart_coords<T>(g_in, coords, p, c);
+        along[r] = c[0];
 #pragma unroll
         for (int a = 0; a < 3; a++) {
             bad = bad || !(fabs((double)c[a]) < 1.0e30);           // the comparisons below pass a NaN by
             lo[a] = c[a] < lo[a] ? c[a] : lo[a];
             hi[a] = c[a] > hi[a] ? c[a] : hi[a];
         }
-        if (p >= own0 && p < own1) {
-            if (x) { x[(size_t)p * 3] = c[0]; x[(size_t)p * 3 + 1] = c[1]; x[(size_t)p * 3 + 2] = c[2]; }
-            if (ilist) { ilist[p] = p; types_out[p] = types[p]; }  // neighborList.h:548-553
-            if (incoming) incoming[p] = 0;                         // counted up by the list kernel
-        }
     }
-    if (bad) sh_bad = 1;
+    const bool any_bad = __any(bad);
+    if (lane == 0) sh_bad[wv] = any_bad ? 1 : 0;
     // each extreme is taken over the threads' values by one wavefront: six reductions by shuffles in every
     // wavefront would be a chain of 36
-    T* const sh_v = (T*)sh_small;                                // [6][NBS_THREADS], before the counters
+    T* const sh_v = (T*)found;                                   // [6][NBS_THREADS]
 #pragma unroll
     for (int a = 0; a < 3; a++) { sh_v[a * NBS_THREADS + tid] = lo[a]; sh_v[(3 + a) * NBS_THREADS + tid] = hi[a]; }
     __syncthreads();
@@ -642,12 +664,18 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         T r = o[0];
 #pragma unroll
         for (int w = 1; w < NBS_THREADS / 64; w++) r = is_min ? (o[w] < r ? o[w] : r) : (o[w] > r ? o[w] : r);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const T t = __shfl_xor(r, off, 64);
-            r = is_min ? (t < r ? t : r) : (t > r ? t : r);
-        }
+        r = wave_extreme(r, is_min);
         if (lane == 0) ext[6 + wv] = r;
+    } else if (wv >= 8) {                                        // meanwhile, others
+        for (int p = own0 + tid - NBS_THREADS / 2; p < own1; p += NBS_THREADS / 2) {
+            if (x) {
+                T c[3];
+                cart_coords<T>(g_in, coords, p, c);
+                x[(size_t)p * 3] = c[0]; x[(size_t)p * 3 + 1] = c[1]; x[(size_t)p * 3 + 2] = c[2];
+            }
+            if (ilist) { ilist[p] = p; types_out[p] = types[p]; }  // neighborList.h:548-553
+            if (incoming) incoming[p] = 0;                         // counted up by the list kernel
+        }
     }
     __syncthreads();
     if (tid < 3) {
@@ -656,20 +684,36 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     }
     __syncthreads();
     const long long nregion_ll = (long long)max(dyn.rdim[0], 0) * max(dyn.rdim[1], 0) * max(dyn.rdim[2], 0);
-    bool ok = !sh_bad && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform, alike in all workgroups
+    int bads = 0;
+#pragma unroll
+    for (int w = 0; w < NBS_THREADS / 64; w++) bads |= sh_bad[w];
+    const bool ok = !bads && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform, alike in all workgroups
     const Grid<T> g = with_dyn<T>(g_in, &dyn);
     const int nx = ok ? g.rdim[0] : 0, plane = ok ? g.rdim[1] * g.rdim[2] : 0;
     const int planes = (nx + (int)gridDim.x - 1) / (int)gridDim.x;
     const int x0 = min(planes * (int)blockIdx.x, nx), x1 = min(x0 + planes, nx);
-    if (blockIdx.x > 0 && x0 >= x1) return;                      // no slab; the first workgroup reports
+    if (tid == 0 && blockIdx.x == 0) {                           // (the first workgroup reports)
+        GridDyn<T> out = dyn;                                    // (the others still read theirs)
+        if (!ok) {
+            for (int a = 0; a < 3; a++) { out.rdim[a] = 0; out.keep_lo[a] = (T)1; out.keep_hi[a] = (T)-1; }
+            if (raise) atomicOr(status, ST_GRID_BOUND);
+        }
+        out.nregion = ok ? nx * plane : 0;
+        out.zstride = out.rdim[2] + 1;
+        double big = 0;
+        for (int a = 0; a < 3; a++) big = fmax(big, fmax(fabs((double)out.keep_lo[a]), fabs((double)out.keep_hi[a])));
+        *gd = out;
+        if (slot) {
+            const long long bits = __double_as_longlong(big);
+            const int words[NBS_WORDS] = {ok ? 1 : 0, out.rdim[0], out.rdim[1], out.rdim[2], (int)(bits & 0xffffffffll),
+                                          (int)(bits >> 32)};
+            read_back_store(slot, seq, words, NBS_WORDS);
+        }
+    }
+    if (!ok || x0 >= x1) return;                                 // (no box, no slab)
     const int nbins = (x1 - x0) * plane;
 
-    for (int i = tid; i < nbins; i += NBS_THREADS) cnt[i] = 0;
-    if (tid < min(g.nimg, NBS_TRIPLES)) sh_triple[tid] = image_triple(g, tid);
-    __syncthreads();
-
-    // 2. images: found (in the slab), before it, in the box
-    int before = 0, all = 0;
+    // 2. images in the slab
     auto image = [&](int im, int p, int b) __attribute__((always_inline)) {      // bin b of the slab
         atomicAdd(&cnt[b], 1);
         const int k = atomicAdd(&sh_found, 1);
@@ -678,26 +722,7 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
             bin_of_found[k] = (unsigned short)b;
         }
     };
-    if (ok && separable) {
-        // An image at distance v from the middle of the kept interval is outside the box for sure when |v| > reach, inside
-        // when |v| < inner, and likewise before the slab when v < from, behind it when v > to.  The margins are that of
-        // keep_lo, a hundred times the rounding of the binning, and of this arithmetic.
-        T shift[3][3], reach[3], inner[3], from, to;
-#pragma unroll
-        for (int a = 0; a < 3; a++) {
-            const double lo_edge = (double)g.mn[a] + (double)g.rlo[a] * (double)g.bin_size;
-            const double margin = lo_edge - (double)g.keep_lo[a];
-            const double mid = 0.5 * ((double)g.keep_lo[a] + (double)g.keep_hi[a]);
-            reach[a] = (T)((double)g.keep_hi[a] - mid);
-            inner[a] = (T)((double)g.keep_hi[a] - mid - 2.0 * margin);
-            if (a == 0) {
-                from = (T)(lo_edge + (double)x0 * (double)g.bin_size - margin - mid);
-                to = (T)(lo_edge + (double)x1 * (double)g.bin_size + margin - mid);
-            }
-#pragma unroll
-            for (int i = 0; i < 3; i++)
-                shift[a][i] = i < g.img_dim[a] ? (T)((double)g.b[a][a] * (double)(g.img_lo[a] + i) - mid) : (T)4.0e30;
-        }
+    if (separable) {
         // the coordinate along axis a of the image that is i cells along it (the other axes' indices only add zeros, their
         // lattice components along this axis vanish), its bin, and whether it is inside, exactly
         auto at = [&](T ca, int a, int i) __attribute__((always_inline)) -> T {
@@ -709,50 +734,25 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
             const int b = bin(ci, a);
             return b >= 0 && b < g.rdim[a];
         };
-        T ahead_c[3];
-        if (tid < N) cart_coords<T>(g, coords, tid, ahead_c);
-#pragma unroll 1
-        for (int p = tid, next = tid; p < N; p = next) {
-            T c[3];
+        // An image below `from` or above `to` is not in the slab for sure: the margins are that of keep_lo, a hundred times the
+        // rounding of the binning, and of this arithmetic.
+        const double lo_edge = (double)g.mn[0] + (double)g.rlo[0] * (double)g.bin_size, margin = lo_edge - (double)g.keep_lo[0];
+        const T from = (T)(lo_edge + (double)x0 * (double)g.bin_size - margin), to = (T)(lo_edge + (double)x1 * (double)g.bin_size + margin);
+        T shift[3];
 #pragma unroll
-            for (int a = 0; a < 3; a++) c[a] = ahead_c[a];
-            next += NBS_THREADS;
-            if (next < N) cart_coords<T>(g, coords, next, ahead_c);        // on its way while this one is placed
-            int n[3], sure[3], ahead = 0, upto = 0;
+        for (int i = 0; i < 3; i++) shift[i] = i < g.img_dim[0] ? (T)((double)g.b[0][0] * (double)(g.img_lo[0] + i)) : (T)4.0e30;
 #pragma unroll
-            for (int a = 0; a < 3; a++) {
-                n[a] = sure[a] = 0;
+        for (int r = 0; r < PER; r++) {
+            const int p = tid + r * NBS_THREADS;
 #pragma unroll
-                for (int i = 0; i < 3; i++) {
-                    const T v = c[a] + shift[a][i], d = v < (T)0 ? -v : v;
-                    n[a] += d <= reach[a] ? 1 : 0;
-                    sure[a] += d < inner[a] ? 1 : 0;
-                    if (a == 0) {
-                        ahead += d < inner[a] && v < from ? 1 : 0;
-                        upto += d <= reach[a] && v <= to ? 1 : 0;
-                    }
-                }
-                if (a > 0 && n[a] != sure[a]) {
-                    n[a] = 0;
-#pragma unroll 1
-                    for (int i = 0; i < g.img_dim[a]; i++) n[a] += inside(at(c[a], a, i), a) ? 1 : 0;
-                }
+            for (int i = 0; i < 3; i++) {
+                const T v = along[r] + shift[i];
+                if (!(v >= from && v <= to) || p >= N || i >= g.img_dim[0]) continue;
+                const T ci = at(along[r], 0, i);
+                if (!inside(ci, 0)) continue;
+                const int b = bin(ci, 0);
+                if (b >= x0 && b < x1) work[atomicAdd(&sh_work, 1)] = (unsigned short)(p | i << NBS_ATOM_BITS);
             }
-            const int n12 = n[1] * n[2];
-            if ((n[0] != sure[0] || upto != ahead) && n12 > 0) {           // next to an edge of the box, or in the slab
-                n[0] = ahead = 0;
-#pragma unroll 1
-                for (int i = 0; i < g.img_dim[0]; i++) {
-                    const T ci = at(c[0], 0, i);
-                    if (!inside(ci, 0)) continue;
-                    n[0]++;
-                    const int b = bin(ci, 0);
-                    if (b < x0) ahead++;
-                    else if (b < x1) work[atomicAdd(&sh_work, 1)] = (unsigned short)(p | i << NBS_ATOM_BITS);
-                }
-            }
-            all += n[0] * n12;
-            before += ahead * n12;
         }
         __syncthreads();
         // the slab's own, all lanes busy
@@ -771,7 +771,7 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
                 if (inside(cz, 2)) image((i * g.img_dim[1] + j) * g.img_dim[2] + k, p, bxy * g.rdim[2] + bin(cz, 2));
             }
         }
-    } else if (ok) {
+    } else {
 #pragma unroll 1
         for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
             const int m = w / N, p = w - m * N;
@@ -779,58 +779,44 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
             T xp[3], ci[3];
             cart_coords<T>(g, coords, p, xp);
             const int b = locate(g, xp, ij / g.img_dim[1], ij % g.img_dim[1], k, ci);
-            if (b < 0) continue;
-            all++;
-            if (b < x0 * plane) before++;
-            else if (b < x1 * plane) image(m, p, b - x0 * plane);
+            if (b >= x0 * plane && b < x1 * plane) image(m, p, b - x0 * plane);
         }
     }
-    before = wave_sum(before);
-    all = wave_sum(all);
-    if (lane == 0) { sh_scan[1][wv] = before; sh_scan[2][wv] = all; }
     __syncthreads();
 
-    // 3. prefix sum in place: a thread takes consecutive bins
+    // 3. prefix sum in place: a thread takes consecutive bins.  A slab's records have a place of their own, and every column of
+    // bins an end of its own behind its last one.
     const int per = (nbins + NBS_THREADS - 1) / NBS_THREADS;
     const int b0 = min(tid * per, nbins), b1 = min(b0 + per, nbins);
     int mine = 0;
     for (int b = b0; b < b1; b++) mine += cnt[b];
     const int incl = wave_inclusive_scan(mine);
-    if (lane == 63) sh_scan[0][wv] = incl;
+    if (lane == 63) sh_scan[wv] = incl;
     __syncthreads();
-    int run = incl - mine, own = 0, base = 0, total = 0;
+    int run = incl - mine, own = 0;
     for (int w = 0; w < NBS_THREADS / 64; w++) {
-        const int t = sh_scan[0][w];
+        const int t = sh_scan[w];
         run += w < wv ? t : 0;
         own += t;
-        base += sh_scan[1][w];
-        total += sh_scan[2][w];
     }
-    ok = ok && total <= spare_images;                            // (the room for records)
-    for (int b = b0; b < b1; b++) {
-        const int n = cnt[b];
-        cnt[b] = run;
-        if (ok) offsets[x0 * plane + b] = base + run;
-        run += n;
-    }
-    if (tid == 0 && blockIdx.x == 0) {
-        if (!ok) {
-            for (int a = 0; a < 3; a++) { dyn.rdim[a] = 0; dyn.keep_lo[a] = (T)1; dyn.keep_hi[a] = (T)-1; }
-            if (raise) atomicOr(status, ST_GRID_BOUND);
-        }
-        dyn.nregion = ok ? nx * plane : 0;
-        if (ok) offsets[nx * plane] = total;
-        double big = 0;
-        for (int a = 0; a < 3; a++) big = fmax(big, fmax(fabs((double)dyn.keep_lo[a]), fabs((double)dyn.keep_hi[a])));
-        *gd = dyn;
-        if (slot) {
-            const long long bits = __double_as_longlong(big);
-            const int words[NBS_WORDS] = {ok ? 1 : 0, dyn.rdim[0], dyn.rdim[1], dyn.rdim[2], (int)(bits & 0xffffffffll),
-                                          (int)(bits >> 32)};
-            read_back_store(slot, seq, words, NBS_WORDS);
+    const int base = (int)blockIdx.x * room;
+    const bool fits = own <= room;                               // (always: small_room)
+    {
+        const int nz = g.rdim[2], q0 = b0 / nz;
+        int z = b0 - q0 * nz;
+        int* o = offsets + (x0 * g.rdim[1] + q0) * (nz + 1) + z;
+        for (int b = b0; b < b1; b++) {
+            const int n = cnt[b];
+            cnt[b] = run;
+            *o++ = base + (fits ? run : 0);
+            run += n;
+            if (++z == nz) { *o++ = base + (fits ? run : 0); z = 0; }
         }
     }
-    if (!ok) return;
+    if (!fits) {
+        if (tid == 0) atomicOr(status, ST_GRID_BOUND);
+        return;
+    }
     __syncthreads();
 
     // 4. image numbers to their bins, 5. records in descending image number within a bin (head insertion,
@@ -863,7 +849,7 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     }
     // more images than LDS: their numbers go through global memory, to places of this slab's own
     int* const by_bin = spare + base;
-    int* const bins = spare + spare_images + base;
+    int* const bins = spare + NBS_SLABS * room + base;
 #pragma unroll 1
     for (int w = tid; w < N * g.nimg; w += NBS_THREADS) {
         const int m = w / N, p = w - m * N;
@@ -1044,7 +1030,7 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
             }
         }
         if (ok && zlo <= zhi) {
-            const int col = ((bx - g.rlo[0]) * g.rdim[1] + (by - g.rlo[1])) * g.rdim[2] - g.rlo[2];
+            const int col = ((bx - g.rlo[0]) * g.rdim[1] + (by - g.rlo[1])) * g.zstride - g.rlo[2];
             start = offsets[col + zlo];
             len = offsets[col + zhi + 1] - start;
         }
@@ -1971,6 +1957,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     int* status = (int*)flags;
 
     for (int a = 0; a < 3; a++) { g.mn[a] = 0; g.nbin[a] = 0; g.rlo[a] = 0; g.rdim[a] = 0; }
+    g.zstride = 0;
     // the bin box: read back from the extents, or bounded by the box of the last synchronised build of this structure
     int device = 0;
     A2P_HIP_CHECK(hipGetDevice(&device));
@@ -2073,17 +2060,19 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
     GridDyn<T>* gd = nullptr;
     int* offsets = nullptr;
     long long total = 0;
-    int spare_images = 0;                               // images the binning in one launch has room for
+    int small_room = 0;                                 // images that a slab of the binning in one launch has room for
     if (small) {
         posted = !sync_free;
         void* wsG = nullptr;
         rc = ws_get(WS_GRID, 256, &wsG);
-        // one by one there are at most NBS_IMAGES images; told by axis, every one of them may be in reach
-        spare_images = std::max(NBS_IMAGES, N * g.nimg);
+        // A slab has room for every image that can be in it: one along x to an atom while it is thinner than the cell.
+        const int planes = ceil_div(cap[0], NBS_SLABS);
+        const bool thin = separable && (double)planes * (double)g.bin_size < 0.99 * std::fabs((double)g.b[0][0]);
+        small_room = N * g.img_dim[1] * g.img_dim[2] * (thin ? 1 : g.img_dim[0]);
         if (rc == A2P_OK)
-            rc = ws_get(WS_NBL_B, ((size_t)NBS_BINS + 1 + 2 * (size_t)spare_images) * sizeof(int), (void**)&offsets);
+            rc = ws_get(WS_NBL_B, (2 * (size_t)NBS_BINS + 2 * (size_t)NBS_SLABS * small_room) * sizeof(int), (void**)&offsets);
         gd = (GridDyn<T>*)wsG;
-        total = spare_images;
+        total = (long long)NBS_SLABS * small_room;
     }
 
     if (small && rc == A2P_OK) {
@@ -2101,7 +2090,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             hipLaunchKernelGGL(small_bins_kernel<T>, dim3(NBS_SLABS), dim3(NBS_THREADS), NBS_LDS, stream, g, coords, x_out, gd, offsets,
                                (T*)wsC0, types, want_rows ? ilist : (int*)nullptr, types_out, incoming, co ? 1 : 0,
                                separable ? 1 : 0, cap[0], cap[1], cap[2], bound_of_coords, sync_free ? 1 : 0, status,
-                               posted ? post_slot : nullptr, post.seq, offsets + NBS_BINS + 1, spare_images);
+                               posted ? post_slot : nullptr, post.seq, offsets + 2 * NBS_BINS, small_room);
             prof_end(stream);
             if (hipGetLastError() != hipSuccess) rc = A2P_ERR_HIP;
         }
@@ -2210,6 +2199,7 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             big_coord = std::max(big_coord, std::max(std::fabs((double)g.keep_lo[a]), std::fabs((double)g.keep_hi[a])));
         remember({g.rdim[0], g.rdim[1], g.rdim[2]}, big_coord);
     }
+    g.zstride = g.rdim[2];
     const int nb1 = (int)nregion + 1;
 
     if (nb1 > room) {
