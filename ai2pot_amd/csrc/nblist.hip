@@ -1038,6 +1038,9 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
 }
 
 constexpr int NBL_APW = 2;         // consecutive centre atoms per wavefront
+// Up to NBL_SINGLE atoms they leave the chip half empty, and a wavefront takes one: a step of 4,000 atoms 42.1 -> 41.0 us, of 2,000 36.5 ->
+// 35.1, but of 9,000 71.7 -> 72.6.
+constexpr int NBL_SINGLE = 4096;
 
 // cols[base .. base + len) = the lane's column, for the runs of all lanes at once, which lie back to back.  Every lane with a run
 // writes the first NBL_RUN places from its base on, the last one first, whether they are its own or not: a place belongs to the
@@ -1120,30 +1123,30 @@ __device__ T pair_symmetric_d2(const Grid<T>& g, const T* __restrict__ x, const 
     return add_rn(add_rn(mul_rn(w0, w0), mul_rn(w1, w1)), mul_rn(w2, w2));
 }
 
-template <typename T, bool SORT, bool ROWBUF, bool RANK, bool COMPACT = false>
+template <typename T, bool SORT, bool ROWBUF, bool RANK, bool COMPACT = false, int APW = 2>
 __global__ void __launch_bounds__(NBL_BLOCK)
 lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict__ types,
              const int* __restrict__ offsets, const T* __restrict__ s_rec,
              int umax, int* __restrict__ ilist, int* __restrict__ numneigh, int* __restrict__ firstneigh,
              T* __restrict__ rcs, int* __restrict__ types_out, T* __restrict__ keys,
              int* __restrict__ status, int update, int* __restrict__ rank_out, int* __restrict__ incoming,
-             const CompactEmit<T> ce, const GridDyn<T>* __restrict__ gd, int* __restrict__ tied = nullptr)
+             const CompactEmit<T> ce, const GridDyn<T>* __restrict__ gd, int* __restrict__ tied)
 {
     static_assert(!COMPACT || (ROWBUF && !SORT && !RANK), "compact lists are cut from the row held in LDS");
     static_assert(!(SORT && RANK), "places belong to unsorted rows");
     const Grid<T> g = with_dyn(g_in, gd);
     __shared__ int sh_shift[NBL_BLOCK / 64][64];                             // entry of a column's candidate - its place in the list
     __shared__ int sh_base[NBL_BLOCK / 64][64];
-    __shared__ unsigned char sh_col[NBL_BLOCK / 64][NBL_APW][NBL_ENT_CAP + NBL_RUN];   // column of each flat candidate
+    __shared__ unsigned char sh_col[NBL_BLOCK / 64][APW][NBL_ENT_CAP + NBL_RUN];   // column of each flat candidate
     extern __shared__ __align__(16) unsigned char sh_rows[];
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // (In processing order an XCD takes a run of workgroups, as the kernels behind do: 569 -> 556 us at 1,048,576 atoms; in the
     // caller's order that gained nothing, sorted rows of 131,072 atoms 141 -> 144 us.)
     // the wave's first position, in a scalar register: the loads of its atoms' indices and coordinates are then
     // scalar loads
-    const int p0 = __builtin_amdgcn_readfirstlane(((COMPACT ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * (NBL_BLOCK / 64) + wv) * NBL_APW);
+    const int p0 = __builtin_amdgcn_readfirstlane(((COMPACT ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * (NBL_BLOCK / 64) + wv) * APW);
     if (p0 >= g.N) return;                        // whole wave leaves together
-    const int np = min(NBL_APW, g.N - p0);
+    const int np = min(APW, g.N - p0);
     T* rb_rcs = nullptr;
     int* rb_first = nullptr;
     int* rb_rank = nullptr;
@@ -1162,19 +1165,19 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
         return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
     };
     // A row costs three dependent trips to memory (coordinates, column runs, candidates).  The
-    // wavefront takes NBL_APW atoms: all their coordinates are loaded first, and the column runs of
+    // wavefront takes APW atoms: all their coordinates are loaded first, and the column runs of
     // the next atom are requested before the candidates of the current one are scanned.
-    T cs[NBL_APW][3];
-    int atom[NBL_APW];                            // the atom behind each of the wave's positions
+    T cs[APW][3];
+    int atom[APW];                            // the atom behind each of the wave's positions
 #pragma unroll
-    for (int a = 0; a < NBL_APW; a++) {
+    for (int a = 0; a < APW; a++) {
         const int q = min(p0 + a, g.N - 1);
         // the caller may write the order: an index outside the structure must not reach an address
         // (compact_symmetry_kernel reports it)
         atom[a] = COMPACT ? min(max(ce.order[q], 0), g.N - 1) : q;
     }
 #pragma unroll
-    for (int a = 0; a < NBL_APW; a++)
+    for (int a = 0; a < APW; a++)
 #pragma unroll
         for (int d = 0; d < 3; d++)
             cs[a][d] = COMPACT ? ce.xs[(size_t)min(p0 + a, g.N - 1) * 3 + d] : x[(size_t)atom[a] * 3 + d];
@@ -1182,29 +1185,30 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     // With at most 32 columns per atom the wave's two atoms are set up side by side, lanes 0-31 and 32-63 (their
     // halves of sh_shift / sh_base, their own flat list); with more, one after the other through the first
     // flat list, the column runs of the second requested before the candidates of the first are scanned.
-    static_assert(NBL_APW == 2, "two atoms per wavefront");
+    static_assert(APW == 2 || APW == 1, "two atoms per wavefront, or one");
     const bool paired = nruns <= 32;              // wave-uniform
     int start, len;
-    int totals[NBL_APW] = {0, 0};
+    int totals[APW] = {};
     if (paired) {
         const int sub = lane >> 5;
-        const T csel[3] = {sub ? cs[1][0] : cs[0][0], sub ? cs[1][1] : cs[0][1], sub ? cs[1][2] : cs[0][2]};
+        constexpr int SECOND = APW - 1;
+        const T csel[3] = {sub ? cs[SECOND][0] : cs[0][0], sub ? cs[SECOND][1] : cs[0][1], sub ? cs[SECOND][2] : cs[0][2]};
         column_setup<T>(g, csel, lane & 31, offsets, start, len);
         if (sub >= np) len = 0;
         const int incl = wave_inclusive_scan(len);
         totals[0] = __builtin_amdgcn_readlane(incl, 31);
-        totals[1] = __builtin_amdgcn_readlane(incl, 63) - totals[0];
+        if (APW > 1) totals[APW - 1] = __builtin_amdgcn_readlane(incl, 63) - totals[0];
         const int base = incl - len - (sub ? totals[0] : 0);
         sh_shift[wv][lane] = start - base;
         sh_base[wv][lane] = base;
-        run_columns(sh_col[wv][sub], base, (sub ? totals[1] : totals[0]) <= NBL_ENT_CAP ? len : 0, lane & 31);
+        run_columns(sh_col[wv][APW > 1 ? sub : 0], base, (sub ? totals[APW - 1] : totals[0]) <= NBL_ENT_CAP ? len : 0, lane & 31);
         __builtin_amdgcn_wave_barrier();
     } else {
         column_setup<T>(g, cs[0], lane, offsets, start, len);
     }
     const T near_band = ce.near_band;
 #pragma unroll
-    for (int ia = 0; ia < NBL_APW; ia++) {
+    for (int ia = 0; ia < APW; ia++) {
     if (ia >= np) break;                          // wave-uniform
     const int pos = p0 + ia;                      // position in processing order
     const int p = atom[ia];                       // atom, row of the padded outputs
@@ -1212,7 +1216,7 @@ lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict_
     const T (&c)[3] = cs[ia];
     int nstart = 0, nlen = 0;
     if (!paired) {
-        if (ia + 1 < NBL_APW && ia + 1 < np) column_setup<T>(g, cs[ia + 1 < NBL_APW ? ia + 1 : ia], lane, offsets, nstart, nlen);
+        if (ia + 1 < APW && ia + 1 < np) column_setup<T>(g, cs[ia + 1 < APW ? ia + 1 : ia], lane, offsets, nstart, nlen);
         const int incl = wave_inclusive_scan(len);
         totals[ia] = __builtin_amdgcn_readlane(incl, 63);
         const int base = incl - len;
@@ -2311,40 +2315,41 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
             ce.near_band = (T)(2.0 * co->split * dr + dr * dr);
         }
     }
-    const int list_blocks = ceil_div(N, (NBL_BLOCK / 64) * NBL_APW);
     prof_begin("nbl_lists", stream);
     const size_t rows_lds = rowbuf_bytes<T>(umax, rank != nullptr) * (NBL_BLOCK / 64);
     const bool rowbuf = !sort && umax % 4 == 0 && rows_lds <= 32 * 1024 && (uintptr_t)firstneigh % 16 == 0 &&
                         (uintptr_t)rcs % 16 == 0 && (uintptr_t)rank % 16 == 0;
+    const bool single = !co && N <= NBL_SINGLE && (sort_in_place || rowbuf);
+    const int list_blocks = ceil_div(N, (NBL_BLOCK / 64) * (single ? 1 : NBL_APW));
     if (co)
         hipLaunchKernelGGL((lists_kernel<T, false, true, false, true>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds,
                            stream, g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out,
-                           keys, status, update, nullptr, nullptr, ce, (const GridDyn<T>*)gd);
+                           keys, status, update, nullptr, nullptr, ce, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (sort_in_place)
-        hipLaunchKernelGGL((lists_kernel<T, true, true, false>), dim3(list_blocks), dim3(NBL_BLOCK),
+        hipLaunchKernelGGL((single ? lists_kernel<T, true, true, false, false, 1> : lists_kernel<T, true, true, false, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK),
                            rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64), stream, g, x, types, offsets, s_rec, umax,
                            ilist, numneigh, firstneigh, rcs, types_out, keys, status, update, nullptr, nullptr,
                            CompactEmit<T>{}, (const GridDyn<T>*)gd, tied);
     else if (sort)
-        hipLaunchKernelGGL((lists_kernel<T, true, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, true, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, tmp_first, tmp_rcs, types_out, keys,
-                           status, 0, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd);
+                           status, 0, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rowbuf && rank)
-        hipLaunchKernelGGL((lists_kernel<T, false, true, true>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
+        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, true, false, 1> : lists_kernel<T, false, true, true, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
                            g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
-                           status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd);
+                           status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rowbuf)
-        hipLaunchKernelGGL((lists_kernel<T, false, true, false>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
+        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, false, false, 1> : lists_kernel<T, false, true, false, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
                            g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
-                           status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd);
+                           status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rank)
-        hipLaunchKernelGGL((lists_kernel<T, false, false, true>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, false, false, true, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
-                           status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd);
+                           status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else
-        hipLaunchKernelGGL((lists_kernel<T, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, false, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
-                           status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd);
+                           status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     prof_end(stream);
     if (co) {
         prof_begin("nbl_symmetry", stream);
