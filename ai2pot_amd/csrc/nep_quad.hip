@@ -18,11 +18,14 @@
 // Registers decide how many wavefronts a SIMD holds: each phase takes arguments, LDS addresses and the lane's place anew.  With
 // 60 values spilled for three wavefronts the kernel took 89 us at 20,011 atoms, with two 72, so 58.
 //
-// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 21.7 us
-// (28 for the same atoms in no spatial order), 20,011 with skin lists 94 -> 53, 64 structures of 128 atoms 43 -> 24.5.
-// Of the 42 thousand cycles of a wavefront at 4096 atoms the tables take 5.2 (8.2 with a load to a value and the number of rows
-// waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6.
-// Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq by fours (57 -> 58).
+// Measured (fp32, 6 radial functions, l_max 4, 47 neighbours) against a wavefront per atom: 4096 atoms in lattice order 34 -> 20.7 us
+// (28 for the same atoms in no spatial order, when those took 22), 20,011 with skin lists 94 -> 52, 64 structures of 128 atoms 43 -> 24.
+// Of the 42 thousand cycles of a wavefront at 4096 atoms the tables took 5.2 (8.2 with a load to a value and the number of rows
+// waited for before the first), its rows' heads 1, slots 7.3, angular pairs and moments 6, read-out 9, angular forces 2, radial forces 6,
+// and the claims with their answers 3, a row behind the last 1.3, before their entries were read four at a time and it was not begun:
+// 21.4 -> 20.7 us, 53.2 -> 51.9 at 20,011.
+// Taken back: two neurons a lane at a time (8 values spilled: 61 us), the neurons of dE/dq by fours (57 -> 58), the first entries
+// of the radial forces ahead of the angular ones (20 bytes spilled), descriptors scaled by the lane that sums them (no change).
 //
 // Formulas: source/descriptor/nep/include/{nepBasis.h:57-196; nep.h:320-529}.
 #include "a2p_common.h"
@@ -251,7 +254,8 @@ nep_quad_kernel(const WaveArgs<T>)
     }
     __syncthreads();
 
-    for (int i0 = first; i0 < min(inum, last); i0 += stride) {
+    last = min(inum, last);
+    for (int i0 = first; i0 < last;) {
         int center = center1, nn = nn1, ti, base0;
         {
             NW_PHASE;
@@ -429,14 +433,24 @@ nep_quad_kernel(const WaveArgs<T>)
                     // -- the pairs claim their places; the answers are stored when the forces' turn comes (the loads above
                     // would wait for them)
                     NW_PHASE;
+                    // (half of the entries read at a time, and then their claims)
 #pragma unroll
-                    for (int k = 0; k < NW_TRIPS; k++) {
-                        const int e = k * NW_LANES + s;
-                        rk[k] = 0;
-                        if (k * NW_LANES < n_most && e < n_own) {
-                            const int2 w = ent[entry(e)];
-                            if (a.brank && a.ranks_valid) rk[k] = a.brank[base + (w.y & 0xffff)];
-                            else rk[k] = pair_claim_raw(&seg.cursor[b * NF + w.x]);
+                    for (int k0 = 0; k0 < NW_TRIPS; k0 += NW_TRIPS / 2) {
+                        if (k0 * NW_LANES >= n_most && k0 > 0) {
+#pragma unroll
+                            for (int k = k0; k < k0 + NW_TRIPS / 2; k++) rk[k] = 0;
+                            break;
+                        }
+                        int2 w[NW_TRIPS / 2];
+#pragma unroll
+                        for (int k = 0; k < NW_TRIPS / 2; k++) w[k] = ent[entry(min((k0 + k) * NW_LANES + s, max(n_own - 1, 0)))];
+#pragma unroll
+                        for (int k = k0; k < k0 + NW_TRIPS / 2; k++) {
+                            rk[k] = 0;
+                            if (k * NW_LANES + s < n_own) {
+                                if (a.brank && a.ranks_valid) rk[k] = a.brank[base + (w[k - k0].y & 0xffff)];
+                                else rk[k] = pair_claim_raw(&seg.cursor[b * NF + w[k - k0].x]);
+                            }
                         }
                     }
                 }
@@ -588,15 +602,20 @@ nep_quad_kernel(const WaveArgs<T>)
                 if (claim && it == (mom ? nch - 1 : 0)) {
                     NW_PHASE;
 #pragma unroll
-                    for (int k = 0; k < NW_TRIPS; k++) {
-                        const int e = k * NW_LANES + s;
-                        if (k * NW_LANES < n_most && e < n_own) {
-                            int2* const w = &ent[entry(e)];
-                            const int tg = b * NF + w->x, r = pair_rank(rk[k]);
-                            if (a.brank && !a.ranks_valid) a.brank[base + (w->y & 0xffff)] = r;
+                    for (int k0 = 0; k0 < NW_TRIPS; k0 += NW_TRIPS / 2) {
+                        if (k0 * NW_LANES >= n_most) break;
+                        int2 w[NW_TRIPS / 2];
+#pragma unroll
+                        for (int k = 0; k < NW_TRIPS / 2; k++) w[k] = ent[entry(min((k0 + k) * NW_LANES + s, max(n_own - 1, 0)))];
+#pragma unroll
+                        for (int k = k0; k < k0 + NW_TRIPS / 2; k++) {
+                            const int e = k * NW_LANES + s;
+                            if (e >= n_own) continue;
+                            const int tg = b * NF + w[k - k0].x, r = pair_rank(rk[k]);
+                            if (a.brank && !a.ranks_valid) a.brank[base + (w[k - k0].y & 0xffff)] = r;
                             const bool fits = (unsigned)r < (unsigned)seg.cap;
                             if (!fits) atomicOr(a.status, ST_SEG_OVERFLOW);
-                            w->x = fits ? tg * seg.cap + r : seg.spare;
+                            ent[entry(e)].x = fits ? tg * seg.cap + r : seg.spare;
                         }
                     }
                 }
@@ -715,7 +734,9 @@ nep_quad_kernel(const WaveArgs<T>)
             if (act && s < 3) a.force[((size_t)b * NF + center) * 3 + s] = s == 0 ? fx : s == 1 ? fy : fz;
             if (act && seg.mark && s == 3) pair_mark_own(&seg.cursor[b * NF + center]);
         }
-        begin(i0 + stride);
+        i0 += stride;
+        if (i0 >= last) break;                           // (no row behind the last one is waited for)
+        begin(i0);
         begin_species();
     }
 
