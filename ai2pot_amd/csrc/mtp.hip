@@ -875,21 +875,16 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     unsigned pword = 0;               // ... and the thread's polynomial
     {
         MTP_PHASE;
-        if (ii >= a.binum[b]) {                  // padded row: contributes nothing
-            if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
-            if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
-            if (!LOSS && a.desc)
-                for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
-            if (LOSS)
-                for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
-            return;
-        }
-        const int center0 = a.bilist[row], nn0 = a.bnumneigh[row];         // on their way while the plan's arrays are fetched
+        // (scalar loads, on their way while the plan's arrays are asked for; a padded row has places in the lists as well)
+        const int inum = uniform_array(a.binum)[b];
+        center = uniform_array(a.bilist)[row];
+        nn = uniform_array(a.bnumneigh)[row];
 
         // Three trips to memory: the row's head with the plan's arrays, the row's entries with the species of the centre, the
         // coefficients with the neighbours' species.  (Five before, with the entries and their species behind the barrier: level 20, 8192
         // atoms 228.8 -> 226.4 us, the training step of level 16, 64 structures of 128 atoms, 272.8 -> 270.5, the linear solver there
         // 469 -> 462.)
+        // (The number of rows was a trip of its own ahead of these: level 10, 216 atoms 29.5 -> 29.1 us, the solver 403 -> 401.)
         mgroups = a.mom_groups;       // uniform over the launch
         const unsigned* const bsrc = mgroups ? (const unsigned*)p.poly_pos : p.basic;
         Staged<unsigned, NT, NT == 64 ? 4 : 2> basics;
@@ -904,11 +899,18 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         const int* const wsrc = flat ? (const int*)p.polys_len : LOSS ? p.polys_mu : p.rows;
         Staged<int, NT, NT == 64 ? 2 : 1> words;
         words.load(wsrc, nwords, lane);
-        center = __builtin_amdgcn_readfirstlane(center0);
-        nn = __builtin_amdgcn_readfirstlane(nn0);
+        if (ii >= inum) {                  // padded row: contributes nothing
+            if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
+            if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
+            if (!LOSS && a.desc)
+                for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
+            if (LOSS)
+                for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
+            return;
+        }
         if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
         if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
-        const int ti0 = types[center];
+        ti = uniform_array(types)[center];
         {
             // (whole-number divisions: small_div cuts a row of two million and more into chunks longer than the table)
             const unsigned n = nn, cap = MTP_NC, cuts = (n + cap - 1) / cap;
@@ -932,7 +934,6 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             for (int c = 0; c < MTP_POLY_MAX; c++)
                 if (__any(len > c)) mtop = c + 1;
         }
-        ti = __builtin_amdgcn_readfirstlane(ti0);
         if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         const T* const csrc = a.coeffs + (size_t)ti * a.ntypes * nmus * K;
         Staged<T, NT, NT == 64 ? 2 : 1> coefs;
@@ -1596,21 +1597,22 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
     TableAhead<T> ahead;
     {
         COMP_PHASE;
-        nn = c.nnc[row];
-        if (ii >= a.binum[b] || nn == 0) {                       // padded or refused row (k_rows flags the reasons)
+        nn = uniform_array(c.nnc)[row];
+        pair0 = uniform_array(c.pair_off)[row] - uniform_array(c.pair_off)[(size_t)c.b0 * a.P];     // of the structures of this launch
+        center = uniform_array(a.bilist)[row];
+        const int inum = uniform_array(a.binum)[b];
+        Staged<unsigned, NT, 2> basics;
+        basics.load(p.basic, n_basic, lane);
+        if (ii >= inum || nn == 0) {                       // padded or refused row (k_rows flags the reasons)
             for (int s = lane; s < S; s += NT) c.desc[row * S + s] = (T)0;
             for (int q = lane; q < 3 * S; q += NT) c.rowpart[row * 3 * S + q] = (T)0;
             return;
         }
-        pair0 = c.pair_off[row] - c.pair_off[(size_t)c.b0 * a.P];     // of the structures of this launch
-        center = a.bilist[row];
         nchunks = (nn + c.nc_cap - 1) / c.nc_cap;
         chunk = (nn + nchunks - 1) / nchunks;
-        Staged<unsigned, NT, 2> basics;
-        basics.load(p.basic, n_basic, lane);
         ahead.entries(rcs, first, lane, 0, min(chunk, nn));
         if ((unsigned)center >= (unsigned)NF) center = 0;
-        ti = types[center];
+        ti = uniform_array(types)[center];
         if ((unsigned)ti >= (unsigned)a.ntypes) ti = 0;
         const T* const csrc = a.coeffs + (size_t)ti * a.ntypes * nmus * K;
         Staged<T, NT, 1> coefs;
