@@ -473,19 +473,16 @@ template <typename T>
 __global__ void finish_partials_kernel(T* out, const double* partial, int nblocks, int src_stride,
                                        int out_stride)
 {
-    __shared__ double sh[256];
+    __shared__ double sh[4];
     const int b = blockIdx.y, c = blockIdx.x;
     const double* src = partial + ((size_t)b * nblocks) * src_stride + c;
     // fixed assignment of blocks to threads, fixed tree: the result does not depend on timing
     double acc = 0.0;
     for (int k = threadIdx.x; k < nblocks; k += 256) acc += src[(size_t)k * src_stride];
-    sh[threadIdx.x] = acc;
+    acc = wave_sum(acc);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if ((int)threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[(size_t)b * out_stride + c] = (T)sh[0];
+    if (threadIdx.x == 0) out[(size_t)b * out_stride + c] = (T)((sh[0] + sh[1]) + (sh[2] + sh[3]));
 }
 
 template <typename T>

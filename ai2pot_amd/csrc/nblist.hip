@@ -152,6 +152,17 @@ __device__ __forceinline__ void image_extremes(const Grid<T>& g, int a, T c_lo, 
     v_hi = image_coord(c_hi, g.b[0][a], g.b[1][a], g.b[2][a], hi[0], hi[1], hi[2]);
 }
 
+// the least or the largest over the wavefront, in every lane (a NaN is passed by)
+template <typename T>
+__device__ __forceinline__ T wave_extreme(T r, bool is_min)
+{
+    auto take = [&](T o) __attribute__((always_inline)) { r = is_min ? (o < r ? o : r) : (o > r ? o : r); };
+    wave::over_row(r, take);
+    take(__shfl_xor(r, 16, 64));
+    take(__shfl_xor(r, 32, 64));
+    return r;
+}
+
 // Four workgroups per CU: beyond that a thread takes several atoms before the sums across lanes, which are what the
 // kernel waits for, and the kernel behind it has fewer values to compare
 // (1,048,576 atoms, fp32: 19.1 -> 10.9 and 13.5 -> 4.6 us with 1024 instead of 4096 workgroups; 7.3 and 4.5 since the images'
@@ -183,12 +194,7 @@ __global__ void coords_minmax_kernel(const Grid<T> g, const T* __restrict__ coor
 #pragma unroll
     for (int q = 0; q < 6; q++) {
         const bool is_min = q < 3;
-        T r = v[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            T o = __shfl_xor(r, off, 64);
-            r = is_min ? (o < r ? o : r) : (o > r ? o : r);
-        }
+        const T r = wave_extreme(v[q], is_min);
         if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6][q] = r;
     }
     __syncthreads();
@@ -276,11 +282,7 @@ minmax_finish_kernel(const Grid<T> g, const T* __restrict__ partial, int nblocks
 #pragma unroll
         for (int u = 0; u < 8; u++) r = is_min ? (o[u] < r ? o[u] : r) : (o[u] > r ? o[u] : r);
     }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        const T o = __shfl_xor(r, off, 64);
-        r = is_min ? (o < r ? o : r) : (o > r ? o : r);
-    }
+    r = wave_extreme(r, is_min);
     if (lane == 0) ext[6 + q] = r;
     __syncthreads();
     if (tid < 3) {
@@ -582,20 +584,6 @@ __device__ __forceinline__ unsigned image_triple(const Grid<T>& g, int im)
 
 // posted to the host: [0] 1 if the lists are complete, [1..3] the box, [4..5] the largest |coordinate| kept (a double)
 constexpr int NBS_WORDS = 6;
-
-// the least or the largest over the wavefront, in every lane (a NaN is passed by)
-template <typename T>
-__device__ __forceinline__ T wave_extreme(T r, bool is_min)
-{
-    auto take = [&](T o) __attribute__((always_inline)) { r = is_min ? (o < r ? o : r) : (o > r ? o : r); };
-    take(wave::dpp_move<0x128>(r));                // row_ror: 8, 4, 2, 1
-    take(wave::dpp_move<0x124>(r));
-    take(wave::dpp_move<0x122>(r));
-    take(wave::dpp_move<0x121>(r));
-    take(__shfl_xor(r, 16, 64));
-    take(__shfl_xor(r, 32, 64));
-    return r;
-}
 
 template <typename T>
 __global__ void __launch_bounds__(NBS_THREADS)

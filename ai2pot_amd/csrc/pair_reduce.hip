@@ -324,11 +324,7 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restric
 #pragma unroll
         for (int k = 0; k < 4; k++) larger(gx[k], gy[k], gz[k]);
         others([&](const T* g) __attribute__((always_inline)) { larger(g[0], g[1], g[2]); });
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
-            const float o = __shfl_xor(mf, off, 64);
-            mf = (mf != mf || o != o) ? NAN : fmaxf(mf, o);
-        }
+        wave::over_row(mf, [&](float o) __attribute__((always_inline)) { mf = (mf != mf || o != o) ? NAN : fmaxf(mf, o); });
         const bool finite = mf < 3.0e38f && mf == mf;
         double s0 = 0.0, s1 = 0.0, s2 = 0.0;
         const bool any = finite && mf > 0.0f;
@@ -349,12 +345,9 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restric
                 s2 += ((double)g[2] + C) - C;
             });
         }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
-            s0 += __shfl_xor(s0, off, 64);
-            s1 += __shfl_xor(s1, off, 64);
-            s2 += __shfl_xor(s2, off, 64);
-        }
+        wave::over_row(s0, [&](double o) __attribute__((always_inline)) { s0 += o; });
+        wave::over_row(s1, [&](double o) __attribute__((always_inline)) { s1 += o; });
+        wave::over_row(s2, [&](double o) __attribute__((always_inline)) { s2 += o; });
         if (sub == 0) {
             if (!finite) {
                 fo[0] = fo[1] = fo[2] = (T)NAN;
@@ -372,8 +365,7 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restric
 #pragma unroll
         for (int k = 0; k < 4; k++) larger(gx[k], gy[k], gz[k]);
         others([&](const T* g) __attribute__((always_inline)) { larger(g[0], g[1], g[2]); });
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+        wave::over_row(m, [&](double o) __attribute__((always_inline)) { m = fmax(m, o); });
         long long s0 = 0, s1 = 0, s2 = 0;
         double scale = 0.0;
         const bool finite = m < 1.0e300 && m == m;
@@ -393,12 +385,9 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restric
                 s2 += __double2ll_rn(g[2] * scale);
             });
         }
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
-            s0 += shfl_xor_ll(s0, off);
-            s1 += shfl_xor_ll(s1, off);
-            s2 += shfl_xor_ll(s2, off);
-        }
+        wave::over_row(s0, [&](long long o) __attribute__((always_inline)) { s0 += o; });
+        wave::over_row(s1, [&](long long o) __attribute__((always_inline)) { s1 += o; });
+        wave::over_row(s2, [&](long long o) __attribute__((always_inline)) { s2 += o; });
         if (sub == 0) {
             if (!finite) {
                 fo[0] = fo[1] = fo[2] = (T)NAN;

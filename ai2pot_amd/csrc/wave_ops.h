@@ -1,70 +1,10 @@
-// Pieces of the kernels that give an atom a wavefront: sums across lanes, 16-byte LDS accesses, 16 x 16 x 4 matrix
-// instructions of either precision.
+// Pieces of the kernels that give an atom a wavefront: 16-byte LDS accesses, 16 x 16 x 4 matrix instructions of either
+// precision.
 #pragma once
 #include "a2p_common.h"
 
 namespace a2p {
 namespace wave {
-
-// ---- cross-lane sums -----------------------------------------------------------------------------
-template <int CTRL>
-__device__ __forceinline__ int dpp_move(int v)
-{
-    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_move(float v) { return __int_as_float(dpp_move<CTRL>(__float_as_int(v))); }
-template <int CTRL>
-__device__ __forceinline__ double dpp_move(double v)
-{
-    const long long b = __double_as_longlong(v);
-    const int lo = dpp_move<CTRL>((int)(b & 0xffffffffll));
-    const int hi = dpp_move<CTRL>((int)(b >> 32));
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-// v[lane] + v[lane ^ 16] and v[lane] + v[lane ^ 32]: the swap of a value with its copy leaves one half's rows in the
-// first and the other half's in the second
-template <int ROWS>
-__device__ __forceinline__ void swap_rows(unsigned v, unsigned& a, unsigned& b)
-{
-    const auto r = ROWS == 16 ? __builtin_amdgcn_permlane16_swap(v, v, false, false)
-                              : __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    a = r[0]; b = r[1];
-}
-template <int ROWS>
-__device__ __forceinline__ float add_rows(float v)
-{
-    unsigned a, b;
-    swap_rows<ROWS>(__float_as_uint(v), a, b);
-    return __uint_as_float(a) + __uint_as_float(b);
-}
-template <int ROWS>
-__device__ __forceinline__ double add_rows(double v)
-{
-    const unsigned long long w = (unsigned long long)__double_as_longlong(v);
-    unsigned al, bl, ah, bh;
-    swap_rows<ROWS>((unsigned)w, al, bl);
-    swap_rows<ROWS>((unsigned)(w >> 32), ah, bh);
-    return __longlong_as_double((long long)((unsigned long long)ah << 32 | al)) +
-           __longlong_as_double((long long)((unsigned long long)bh << 32 | bl));
-}
-template <typename T>
-__device__ __forceinline__ T quad_sum(T v)          // the four lanes of a quad
-{
-    v += dpp_move<0xB1>(v);    // quad_perm [1,0,3,2]
-    v += dpp_move<0x4E>(v);    // quad_perm [2,3,0,1]
-    return v;
-}
-template <typename T>
-__device__ __forceinline__ T sum_over_quads(T v)    // the sixteen lanes with the same place in their quad
-{
-    v += dpp_move<0x124>(v);   // row_ror:4
-    v += dpp_move<0x128>(v);   // row_ror:8
-    v = add_rows<16>(v);
-    return add_rows<32>(v);
-}
-template <typename T>
-__device__ __forceinline__ T all_sum(T v) { return sum_over_quads(quad_sum(v)); }
 
 // ---- LDS -----------------------------------------------------------------------------------------
 __device__ __forceinline__ void lds_load4(const float* p, float (&o)[4])
