@@ -152,3 +152,34 @@ def test_virial_reports_its_own_rows_only():
     finally:
         fvt.set_validate(True)
     fvt.check_status(want)
+
+
+@pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("U", [1, 21, 63, 64, 65, 130])
+def test_gradients_of_many_rows_equal_those_of_few(np_dtype, U):
+    """Above 2047 rows a wavefront's values leave in whole lines: 45 structures of 47 rows and each of some alone, bit for bit."""
+    import torch
+    from ai2pot_amd import ops
+    B, P = 45, 47
+    rng = np.random.default_rng(U)
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
+    binum = np.full(B, P, np.int32)
+    binum[::3] = 40
+    lists = [t(binum), t(np.tile(np.arange(P, dtype=np.int32), (B, 1))), t(rng.integers(0, U + 1, (B, P)).astype(np.int32)),
+             t(rng.integers(0, P, (B, P, U)).astype(np.int32))]
+    rcs, dei = (t(rng.normal(size=(B, P, U, 3)).astype(np_dtype)) for _ in range(2))
+    gf, gv = t(rng.normal(size=(B, P, 3)).astype(np_dtype)), t(rng.normal(size=(B, 3, 3)).astype(np_dtype))
+
+    def grads(k):
+        r, d = rcs[k].clone().requires_grad_(True), dei[k].clone().requires_grad_(True)
+        l = [a[k].contiguous() for a in lists]
+        f = ops.ForceSrOp(*l, 0, U, d)[0]
+        v = ops.VirialSrOp(l[2], r, U, d)[0]
+        by_force = torch.autograd.grad(f, d, gf[k].reshape(f.shape), retain_graph=True)[0]
+        by_virial = torch.autograd.grad(v, [r, d], gv[k].reshape(v.shape))
+        return by_force, *by_virial
+
+    every = grads(slice(0, B))
+    for b in (0, 1, 17, B - 1):
+        for a, one in zip(every, grads(slice(b, b + 1))):
+            assert torch.equal(a[b:b + 1], one)
