@@ -307,6 +307,7 @@ struct PairCsr {
     void* seg_g = nullptr;
     int n = 0;          // B * (P + nghost) targets
     int seg_cap = 0;
+    int runs = 0;       // no ghosts among the targets
     int mark = 0;
     PairCsr() = default;
     PairCsr(const PairCsr&) = delete;
