@@ -2054,7 +2054,7 @@ comp_force_kernel(int S, int n, int P, int cap, int U, int b0, const int* __rest
         }
     }
     // ... and the energies of the rows; column S + t counts those whose centre has species t
-    const int rows = min(COMP_ROWS, binum[b] - blk * COMP_ROWS);
+    const int rows = min(here, binum[b] - blk * COMP_ROWS);
     for (int c = threadIdx.x; c < COLS; c += 64 * COMP_ROWS) {
         const int col = blockIdx.y * COLS + c;
         if (col >= n) continue;

@@ -512,6 +512,23 @@ def test_components_of_few_atoms(oracle, level, sizes):
         assert close(a, b)
 
 
+def test_components_of_a_count_beyond_the_rows(oracle):
+    """A structure that is said to have more rows than the lists hold: those of the lists are evaluated, and neither the next
+    structure's nor what lies behind the last one's (sizes of which a set of four leaves some over)."""
+    import torch
+    from ai2pot_amd import ops
+    m, nb, _ = loss_inputs(oracle, 10, 2, sizes=(9, 9, 9))
+    md, d = model_to_device(m, torch.float64), to_device(nb, torch.float64)
+    assert d["bilist"].shape[1] == 9
+    run = lambda binum: [t.cpu().numpy() for t in ops.mtp_lin_components(
+        m["chebyshev_size"], m["scaling"], md["coeffs"], m["alpha_moments_count"], md["alpha_index_basic"],
+        md["alpha_index_times"], md["alpha_moment_mapping"], m["nmus"], binum, d["bilist"], d["bnumneigh"], d["bfirstneigh"],
+        d["brcs"], d["btypes"], md["type_map"], m["rmax"], m["rmin"], md["q_scaler"], validate=False)]
+    for beyond in (1, 3, 9):
+        for a, b in zip(run(d["binum"] + beyond), run(d["binum"])):
+            assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
 def test_components_in_single_precision(oracle):
     """The fp32 instance of the one-pass components against the fp64 one (the plan's byte offsets are halved for
     4-byte moments)."""
