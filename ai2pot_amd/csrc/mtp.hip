@@ -1451,7 +1451,7 @@ mtp_grad_reduce_kernel(int P, int ncoef, int nlin, int nbias, const int* __restr
     const int ngrad = ncoef + nlin + nbias;
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= ngrad) return;
-    const int inum = binum[b];
+    const int inum = min(binum[b], P);
     T acc = (T)0;
     const T* src = gpart + (size_t)b * P * ngrad + q;
     int ii = 0;
@@ -1482,7 +1482,7 @@ nnmtp_grad_reduce_kernel(int P, int NF, int nblk, int HS, int H, int ntypes, con
     const int nrow = nblk + HS + H + 1;
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= nrow) return;
-    const int inum = binum[b];
+    const int inum = min(binum[b], P);
     T acc = (T)0;
     // eight rows in flight; the rows of other species are skipped, the order of the sum is the atom order
     for (int i0 = 0; i0 < inum; i0 += 8) {

@@ -70,7 +70,7 @@ nep_efv_kernel(const NepArgs<T> a)
     for (int i = tid; i < D; i += NEP_BLOCK) s_qs[i] = a.q_scaler[i];
     __syncthreads();
 
-    const int inum = a.binum[b];
+    const int inum = min(a.binum[b], a.P);
     const bool active = ii < inum;
     const size_t row = (size_t)b * a.P + ii;
     int center = 0, ti = 0, nn = 0;

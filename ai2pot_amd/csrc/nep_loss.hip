@@ -338,7 +338,7 @@ nep_grad_reduce_kernel(NepLossArgs<T> a, T* __restrict__ dcoeffs, T* __restrict_
         else if (e < n_c + n_w0 + 2 * n_h) { const int r = e - n_c - n_w0 - n_h; t = r / H; q = ncl + H * D + H + r - t * H; out = dw1 ? dw1 + (size_t)b * n_h + r : nullptr; }
         else { t = e - n_c - n_w0 - 2 * n_h; q = a.nrow - 1; out = dbias ? dbias + (size_t)b * nt + t : nullptr; }
     }
-    const int inum = a.binum[b];
+    const int inum = min(a.binum[b], a.P);
     const int run = ((inum + 3) / 4 + 7) / 8 * 8;
     const int i_end = min(inum, (part + 1) * run);
     T acc = (T)0;

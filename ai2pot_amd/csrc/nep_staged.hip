@@ -265,7 +265,7 @@ nep_stage_kernel(const NepArgs<T> a, const SegArgs seg, T* __restrict__ seg_g, T
     StageLds<T> L;
     stage_lds_layout<T>(smem_raw, L);
 
-    const bool active = ii < a.binum[b];
+    const bool active = ii < min(a.binum[b], a.P);
     const size_t rowbase = (size_t)b * a.P + r0;
     int center, ti, nn;
     row_header<T>(a, active, rowbase + tid, b, NF, center, ti, nn);
@@ -384,7 +384,7 @@ nep_staged_kernel(const NepArgs<T> a, T* __restrict__ seg_g, int spare, int* __r
     for (int i = tid; i < nt * H; i += FB) { L.b0[i] = a.b0[i]; L.w1[i] = a.w1[i]; }
     if (tid < FDP) L.qs[tid] = tid < DC ? (T)1 / a.q_scaler[tid] : (T)0;
 
-    const bool active = ii < a.binum[b];
+    const bool active = ii < min(a.binum[b], a.P);
     const size_t row = (size_t)b * a.P + (size_t)blockIdx.x * FB + tid;
     int center, ti, nn;
     row_header<T>(a, active, row, b, NF, center, ti, nn);

@@ -175,3 +175,56 @@ def test_nep_loss_with_isolated_atoms(oracle):
     an = sum(got[gk] @ np.ravel(d[pk]) for gk, pk in zip(GRADS, PARAMS))
     assert np.allclose(an, fd, rtol=2e-6, atol=1e-9), (an, fd)
     assert not got[GRADS[0]][1].any()                 # no pair: no coefficient gradient from the second structure
+
+
+# A structure that is said to have more rows than the lists hold: those of the lists are evaluated, and nothing behind them is read
+# (the operators refuse such a count unless they are told not to look at the lists).
+@pytest.mark.parametrize("np_dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,n_r,beyond", [(70, 5, 1), (70, 5, 200), (49153, 6, 1), (49153, 6, 300)])
+def test_nep_rows_beyond_the_lists(monkeypatch, np_dtype, n, n_r, beyond):
+    """n_r = 5 takes the kernel for any shape, 49,153 atoms in fp64 the staged one (fp32: four atoms to a wavefront); the last
+    workgroup of both has rows to spare."""
+    from ai2pot_amd import ops
+    monkeypatch.setattr(ops, "_validate_batch", lambda *a: None)
+    B, U = 2, 8
+    m = synth.nep_model(n_radial_basis=n_r, seed=77)
+    first = np.full((B, n, U), -1, np.int32)
+    near = np.array([-3, -2, -1, 1, 2, 3])
+    first[:, :, :6] = (np.arange(n)[:, None] + near) % n
+    rcs = np.zeros((B, n, U, 3), np_dtype)
+    rcs[:, :, :6, 0] = 1.9 * near
+    rcs[:, :, :6, 1:] = 0.3 * synth.rng_normal(5, B * n * 6 * 2).reshape(B, n, 6, 2)
+    nb = dict(binum=np.full(B, n, np.int32), bilist=np.tile(np.arange(n, dtype=np.int32), (B, 1)),
+              bnumneigh=np.full((B, n), 6, np.int32), bfirstneigh=first, brcs=rcs,
+              btypes=synth.rng_randint(6, B * n, 3).reshape(B, n).astype(np.int32), nghost=0, umax=U)
+    want = run_gpu(m, nb, np_dtype)
+    got = run_gpu(m, dict(nb, binum=nb["binum"] + beyond), np_dtype)
+    for a, b in zip(got, want):
+        assert np.abs(b).max() > 0 and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("model", ["nep", "mtp", "nnmtp"])
+def test_loss_rows_beyond_the_lists(oracle, monkeypatch, model):
+    """The errors are divided by the number of rows: twice as many halve the loss and its gradients, to the last bit."""
+    import test_gpu_mtp
+    import test_gpu_nep_loss
+    import test_gpu_nnmtp
+    from ai2pot_amd import ops
+    monkeypatch.setattr(ops, "_validate_batch", lambda *a: None)
+    w = (1.0, 0.7, 0.3)
+    if model == "nep":                                # (three angular functions: the kernel for any shape)
+        m, nb, labels = test_gpu_nep_loss.larger_case(oracle, 2, (41, 41), l_max=2, n_a=3)
+        run = lambda lists: test_gpu_nep_loss.gpu_loss(m, lists, labels, w)
+    elif model == "mtp":
+        m, nb, labels = test_gpu_mtp.loss_inputs(oracle, 10, 2, sizes=(37, 37))
+        run = lambda lists: test_gpu_mtp.gpu_loss(m, lists, labels, w)
+    else:
+        m, nb, labels = test_gpu_nnmtp.loss_inputs(oracle, 8, 2, 7, sizes=(37, 37))
+        run = lambda lists: test_gpu_nnmtp.gpu_loss(m, lists, labels, w, True)
+    assert (nb["binum"] == nb["bilist"].shape[1]).all()
+    want, got = run(nb), run(dict(nb, binum=2 * nb["binum"]))
+    for k in want:
+        if k in ("energy", "force", "virial"):
+            assert np.array_equal(got[k], want[k]), k
+        elif k != "rmse":
+            assert np.abs(want[k]).max() > 0 and np.array_equal(got[k], want[k] / 2), k
