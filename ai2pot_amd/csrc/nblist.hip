@@ -675,7 +675,11 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
     int bads = 0;
 #pragma unroll
     for (int w = 0; w < NBS_THREADS / 64; w++) bads |= sh_bad[w];
-    const bool ok = !bads && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS;      // uniform, alike in all workgroups
+    // (room for one image along x to an atom: coordinates so large that their rounding counts beside the cell could leave two in a
+    // slab a hundredth thinner than it; the margin of keep_lo is twenty times what rounding does to a distance along x)
+    const double lo_edge = (double)dyn.mn[0] + (double)dyn.rlo[0] * (double)g_in.bin_size, margin = lo_edge - (double)dyn.keep_lo[0];
+    const bool fits = room == N * g_in.nimg || margin < 0.2 * fabs((double)g_in.b[0][0]);
+    const bool ok = !bads && sh_ok[0] && sh_ok[1] && sh_ok[2] && nregion_ll < NBS_BINS && fits;      // uniform, alike in all workgroups
     const Grid<T> g = with_dyn<T>(g_in, &dyn);
     const int nx = ok ? g.rdim[0] : 0, plane = ok ? g.rdim[1] * g.rdim[2] : 0;
     const int planes = (nx + (int)gridDim.x - 1) / (int)gridDim.x;
@@ -724,7 +728,6 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         };
         // An image below `from` or above `to` is not in the slab for sure: the margins are that of keep_lo, a hundred times the
         // rounding of the binning, and of this arithmetic.
-        const double lo_edge = (double)g.mn[0] + (double)g.rlo[0] * (double)g.bin_size, margin = lo_edge - (double)g.keep_lo[0];
         const T from = (T)(lo_edge + (double)x0 * (double)g.bin_size - margin), to = (T)(lo_edge + (double)x1 * (double)g.bin_size + margin);
         T shift[3];
 #pragma unroll
@@ -788,7 +791,6 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         own += t;
     }
     const int base = (int)blockIdx.x * room;
-    const bool fits = own <= room;                               // (always: small_room)
     {
         const int nz = g.rdim[2], q0 = b0 / nz;
         int z = b0 - q0 * nz;
@@ -796,14 +798,10 @@ small_bins_kernel(const Grid<T> g_in, const T* __restrict__ coords, T* __restric
         for (int b = b0; b < b1; b++) {
             const int n = cnt[b];
             cnt[b] = run;
-            *o++ = base + (fits ? run : 0);
+            *o++ = base + run;
             run += n;
-            if (++z == nz) { *o++ = base + (fits ? run : 0); z = 0; }
+            if (++z == nz) { *o++ = base + run; z = 0; }
         }
-    }
-    if (!fits) {
-        if (tid == 0) atomicOr(status, ST_GRID_BOUND);
-        return;
     }
     __syncthreads();
 
@@ -2057,10 +2055,17 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         posted = !sync_free;
         void* wsG = nullptr;
         rc = ws_get(WS_GRID, 256, &wsG);
-        // A slab has room for every image that can be in it: one along x to an atom while it is thinner than the cell.
-        const int planes = ceil_div(cap[0], NBS_SLABS);
-        const bool thin = separable && (double)planes * (double)g.bin_size < 0.99 * std::fabs((double)g.b[0][0]);
-        small_room = N * g.img_dim[1] * g.img_dim[2] * (thin ? 1 : g.img_dim[0]);
+        // A slab has room for every image that can be in it: one along x to an atom while it is thinner than the cell (4096 atoms,
+        // three images an axis, fp64: 38 MB of records and 9 of image numbers in all slabs; 3.5 and 0.9 with the slabs back to back).
+        // With a second try at hand, a box that would make slabs thicker than that is left to it: a cell told axis by axis is two
+        // bins long at least, so that the box has 32 bins along it at least, of which its atoms inside the cell take 8.
+        const double thin = 0.99 * std::fabs((double)g.b[0][0]) / (double)g.bin_size;       // planes
+        int planes = ceil_div(cap[0], NBS_SLABS);
+        if (separable && !sync_free && g.img_dim[0] > 1 && planes > thin) {
+            planes = (int)thin;
+            cap[0] = planes * NBS_SLABS;
+        }
+        small_room = N * g.img_dim[1] * g.img_dim[2] * (separable && planes <= thin ? 1 : g.img_dim[0]);
         if (rc == A2P_OK)
             rc = ws_get(WS_NBL_B, (2 * (size_t)NBS_BINS + 2 * (size_t)NBS_SLABS * small_room) * sizeof(int), (void**)&offsets);
         gd = (GridDyn<T>*)wsG;

@@ -187,3 +187,37 @@ def test_more_than_a_thousand_images_along_an_axis(oracle, dt, axis, spacing):
     pbc = [a == axis for a in range(3)]
     args = (lat.astype(dt), np.zeros(1, np.int32), x.astype(dt), 3.0, 1300)
     assert_same(gpu_list(*args, pbc=pbc), oracle.nblist(*args, pbc=pbc))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_workspace_of_a_short_cell(oracle, dt):
+    """A slab of the box has room for one image along x to an atom, also where the cell is four bins long: 32 slabs of nine images
+    to an atom, 16 bytes (fp64 32) a record and 8 for the images' numbers, and an eighth that a workspace is allocated
+    ahead.  Atoms six cells away along x, where a slab would hold
+    several of an atom's images, are listed as well."""
+    import ctypes
+    from ai2pot_amd import _lib
+    n, L = 3800, np.array([12.0, 80.0, 80.0])
+    f = np.stack([np.arange(n) % 5 / 5, np.arange(n) // 5 % 28 / 28, np.arange(n) // 140 / 28], 1) + 0.02 * synth.rng_uniform(9, 3 * n).reshape(n, 3)
+    ty = synth.rng_randint(4, n, 2)
+    held = _lib.lib().a2p_workspace_bytes
+    held.restype = ctypes.c_size_t
+    _lib.check(_lib.lib().a2p_workspace_release())
+    x = f * L
+    for far in (0.0, 2.0, 6.0, 0.0):
+        x[::7, 0] = f[::7, 0] * L[0] + far * L[0]
+        args = (np.diag(L).astype(dt), ty, x.astype(dt), 6.0, 120)
+        assert_same(gpu_list(*args), oracle.nblist(*args))
+        assert held() < 32 * 9 * n * (8 + 4 * np.dtype(dt).itemsize) * 9 // 8 + (4 << 20)
+
+
+def test_coordinates_whose_rounding_counts_beside_the_cell(oracle):
+    """fp32, 2 ** 22 A from the origin: coordinates are half an A apart there, and images of an atom a cell and a half."""
+    n = 60
+    L, f = jittered(n, 11, density=0.02)
+    lat, ty = np.diag(L).astype(np.float32), synth.rng_randint(3, n, 2)
+    site = np.stack(np.unravel_index(np.arange(n), (4, 4, 4)), 1)
+    for at in (0.0, 2.0 ** 12, 2.0 ** 17, 2.0 ** 22):
+        x = (site * np.float32(L.min() / 4) + np.float32(at) * np.array([1, 0, 0])).astype(np.float32)
+        args = (lat, ty, x, 5.0, 200)
+        assert_same(gpu_list(*args), oracle.nblist(*args))
