@@ -202,15 +202,17 @@ __device__ __forceinline__ T quad_sum(T v)          // the four lanes of a quad
 template <typename T>
 __device__ __forceinline__ T sum_over_quads(T v)    // the sixteen lanes with the same place in their quad
 {
-    v += dpp_move<0x124>(v);   // row_ror:4
+    // the longer way round first: lanes eight apart then hold the same bits, and so do, behind the shorter one, lanes four apart
+    // (the other way about, neighbouring quads add the same four values in two orders, and end a rounding apart)
     v += dpp_move<0x128>(v);   // row_ror:8
+    v += dpp_move<0x124>(v);   // row_ror:4
     v = add_rows<16>(v);
     return add_rows<32>(v);
 }
 template <typename T>
 __device__ __forceinline__ T all_sum(T v) { return sum_over_quads(quad_sum(v)); }
 // `take(o)` with the value of the lane 8, 4, 2 and 1 behind in the row of sixteen, which folds it into v: in the end v is folded over
-// the row, in each of its lanes
+// the row, in each of its lanes, with the same bits (each way round is half of the one before, as in sum_over_quads)
 template <typename T, typename Take>
 __device__ __forceinline__ void over_row(T& v, Take&& take)
 {
@@ -223,6 +225,7 @@ __device__ __forceinline__ void over_row(T& v, Take&& take)
 
 // By data-parallel moves: through the LDS, six round trips and two moves a double each, a wavefront's nine virial sums took most of
 // their kernel (virial_rows_kernel, 4,000 rows, 8.2 -> 4.7 us; reduce_kernel at 20,011 atoms, over rows of sixteen, 6.7 -> 6.1).
+// Every lane holds the sum, with the same bits.
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) { return wave::all_sum(v); }
 
