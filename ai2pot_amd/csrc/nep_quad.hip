@@ -784,11 +784,11 @@ nep_quad_kernel(const WaveArgs<T>)
 // and 41.1; fp64 20,011 100 and 98.  With fewer sets all rows of a neighbourhood claim their places at once, from one XCD: 4,096
 // atoms 21.9 and 23.1, 6,000 25.0 and 26.0, 8,192 26.6 and 26.7, 64 structures of 128 24.8 and 29.4.  (XCDs in runs and workgroups in
 // turn: 20,011 atoms 51.4, 32,768 82.9.)  Runs go by the lists' places, for the number of rows in use comes with the tables; with a quarter
-of the places empty or more by that number, which takes the first rows' loads once more.  In turn, by places alone and so, us: 8 structures
-of 2,500 places with 1,870 in use 43.8, 39.4 and 41.4, with 1,500 36.2, 37.9 and 35.7, with 800 28.4, 36.2 and 27.4; 64 of 400 with 300
-43.2, 48.7 and 40.7, with 150 27.5, 46.0 and 26.9; one of 20,000 with 5,000 23.3, 37.2 and 23.7; fp64 8 of 2,500 with 800 42.3, 91.0 and 41.7;
-sizes from a third of the places up, 32 of 640 45.8, 39.8 and 42.0, 128 of 128 34.7, 34.0 and 34.8.  (From half of them empty: 8 of 2,500 with
-1,500 38.2, 64 of 400 with 300 48.8.)
+// of the places empty or more by that number, which takes the first rows' loads once more.  In turn, by places alone and so, us: 8 structures
+// of 2,500 places with 1,870 in use 43.8, 39.4 and 41.4, with 1,500 36.2, 37.9 and 35.7, with 800 28.4, 36.2 and 27.4; 64 of 400 with 300
+// 43.2, 48.7 and 40.7, with 150 27.5, 46.0 and 26.9; one of 20,000 with 5,000 23.3, 37.2 and 23.7; fp64 8 of 2,500 with 800 42.3, 91.0 and 41.7;
+// sizes from a third of the places up, 32 of 640 45.8, 39.8 and 42.0, 128 of 128 34.7, 34.0 and 34.8.  (From half of them empty: 8 of 2,500 with
+// 1,500 38.2, 64 of 400 with 300 48.8.)
 struct WaveShape { int waves, nblocks, runs; size_t lds; WaveAt at; };
 template <typename T>
 WaveShape wave_shape(const NepArgs<T>& a)
