@@ -25,7 +25,6 @@
 // operations with the *_rn intrinsics: no fused multiply-add may change a rounding.
 #include "a2p_common.h"
 #include "compact_list.h"
-#include "wave_ops.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -1025,7 +1024,10 @@ __device__ __forceinline__ void column_setup(const Grid<T>& g, const T (&c)[3], 
 
 constexpr int NBL_APW = 2;         // consecutive centre atoms per wavefront
 // Up to NBL_SINGLE atoms they leave the chip half empty, and a wavefront takes one: a step of 4,000 atoms 42.1 -> 41.0 us, of 2,000 36.5 ->
-// 35.1, but of 9,000 71.7 -> 72.6.
+// 35.1, but of 9,000 71.7 -> 72.6.  Kernel, two atoms and one, us: a step's update 4,096 atoms 7.0 and 5.4 (fp64 8.4 and 6.4), 6,144 8.1 and 6.7
+// (9.6 and 8.8), 8,192 8.7 and 7.7 (10.5 and 11.1), 12,000 with the events around it 11.8 and 13.1 (14.1 and 15.3); sorted rows 4,096 9.6 and
+// 8.5 (10.6 and 9.9), 5,500 11.8 and 11.2 (12.4 and 13.1).  So they cross near 5,000 atoms in fp64 and beyond 8,192 in fp32; the line
+// is where one is the better in all of these.
 constexpr int NBL_SINGLE = 4096;
 
 // cols[base .. base + len) = the lane's column, for the runs of all lanes at once, which lie back to back.  Every lane with a run
@@ -1109,7 +1111,7 @@ __device__ T pair_symmetric_d2(const Grid<T>& g, const T* __restrict__ x, const 
     return add_rn(add_rn(mul_rn(w0, w0), mul_rn(w1, w1)), mul_rn(w2, w2));
 }
 
-template <typename T, bool SORT, bool ROWBUF, bool RANK, bool COMPACT = false, int APW = 2>
+template <typename T, bool SORT, bool ROWBUF, bool RANK, bool COMPACT = false, int APW = NBL_APW>
 __global__ void __launch_bounds__(NBL_BLOCK)
 lists_kernel(const Grid<T> g_in, const T* __restrict__ x, const int* __restrict__ types,
              const int* __restrict__ offsets, const T* __restrict__ s_rec,
@@ -2319,28 +2321,28 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
                            stream, g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out,
                            keys, status, update, nullptr, nullptr, ce, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (sort_in_place)
-        hipLaunchKernelGGL((single ? lists_kernel<T, true, true, false, false, 1> : lists_kernel<T, true, true, false, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK),
+        hipLaunchKernelGGL((single ? lists_kernel<T, true, true, false, false, 1> : lists_kernel<T, true, true, false>), dim3(list_blocks), dim3(NBL_BLOCK),
                            rowbuf_bytes<T>(umax, false, true) * (NBL_BLOCK / 64), stream, g, x, types, offsets, s_rec, umax,
                            ilist, numneigh, firstneigh, rcs, types_out, keys, status, update, nullptr, nullptr,
                            CompactEmit<T>{}, (const GridDyn<T>*)gd, tied);
     else if (sort)
-        hipLaunchKernelGGL((lists_kernel<T, true, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, true, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, tmp_first, tmp_rcs, types_out, keys,
                            status, 0, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rowbuf && rank)
-        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, true, false, 1> : lists_kernel<T, false, true, true, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
+        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, true, false, 1> : lists_kernel<T, false, true, true>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
                            g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
                            status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rowbuf)
-        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, false, false, 1> : lists_kernel<T, false, true, false, false, 2>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
+        hipLaunchKernelGGL((single ? lists_kernel<T, false, true, false, false, 1> : lists_kernel<T, false, true, false>), dim3(list_blocks), dim3(NBL_BLOCK), rows_lds, stream,
                            g, x, types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
                            status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else if (rank)
-        hipLaunchKernelGGL((lists_kernel<T, false, false, true, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, false, false, true>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
                            status, update, rank, incoming, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     else
-        hipLaunchKernelGGL((lists_kernel<T, false, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
+        hipLaunchKernelGGL((lists_kernel<T, false, false, false>), dim3(list_blocks), dim3(NBL_BLOCK), 0, stream, g, x,
                            types, offsets, s_rec, umax, ilist, numneigh, firstneigh, rcs, types_out, keys,
                            status, update, nullptr, nullptr, CompactEmit<T>{}, (const GridDyn<T>*)gd, (int*)nullptr);
     prof_end(stream);
