@@ -18,11 +18,16 @@
 namespace a2p {
 namespace {
 
-// Rows of three values to a slot, a lane to a slot.  Many rows are bound by what they write: 64 slots' values pass through the
-// wavefront's LDS (WHOLE), so that each store writes whole lines, where three stores would write every third value each.  4,000 rows of
-// 200 slots in fp64: force_bwd_kernel 8.2 -> 6.8 us, virial_bwd_kernel 10.7 -> 8.7.  Few are bound by the wavefront's chain, which
-// that makes longer: 900 rows in fp32 3.36 and 3.56, 3.43 and 3.99.
-constexpr long long FVT_WHOLE = 2048;                    // rows
+// Rows of three values to a slot, a lane to a slot.  Many rows in fp64 are bound by what they write: 64 slots' values pass through the
+// wavefront's LDS (WHOLE), so that each store writes whole lines, where three stores would write every third value each.  Few are
+// bound by the wavefront's chain, which that makes longer, and so are rows in fp32, whose lines the L2 puts together as they come.
+// Kernels without and with it, us, force and virial: fp64, 200 slots, 600 rows 3.40 and 3.52, 4.04 and 3.80; 900 3.68 and 3.60, 4.64 and 4.08;
+// 2,000 5.3 and 4.8, 7.4 and 5.7; 4,000 7.6 and 6.4, 10.6 and 8.6; 32,000 43.7 and 39.4, 92.6 and 60.2; 64 slots, 1,400 rows 3.28 and 3.40, 3.76 and
+// 3.60; 2,400 3.80 and 3.76, 4.64 and 4.40; 32,000 15.3 and 15.2, 23.6 and 23.9.  fp32, 200 slots, 2,000 rows 3.56 and 3.72, 4.28 and 4.68;
+// 4,000 5.0 and 4.8, 6.0 and 6.1; 32,000 18.6 and 19.0, 30.8 and 35.3; 64 slots, 4,000 rows 3.3 and 3.6, 3.7 and 4.1.
+constexpr long long FVT_WHOLE = 1 << 17;                 // slots, fp64
+template <typename T>
+constexpr bool whole_lines() { return sizeof(T) == 8; }
 template <typename T, bool WHOLE>
 __device__ __forceinline__ void store_slots(T* __restrict__ out, T* sh, int lane, int n, T v0, T v1, T v2)
 {
@@ -174,7 +179,7 @@ int force_bwd(int B, int P, int U, int nghost, const int* binum, const int* bili
                 "fvt force backward: null pointer");
     if (B == 0 || P == 0) return A2P_OK;
     prof_begin("fvt_force_bwd", stream);
-    auto kern = (long long)B * P >= FVT_WHOLE ? force_bwd_kernel<T, true> : force_bwd_kernel<T, false>;
+    auto kern = (long long)B * P * U >= FVT_WHOLE ? force_bwd_kernel<T, whole_lines<T>()> : force_bwd_kernel<T, false>;
     hipLaunchKernelGGL(kern, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
                        grad_dei, grad_force, B, P, U, P + nghost, binum, bilist, bnumneigh, bfirstneigh);
     prof_end(stream);
@@ -225,7 +230,7 @@ int virial_bwd(int B, int P, int U, const int* bnumneigh, const T* rcs, const T*
                 "fvt virial backward: null pointer");
     if (B == 0 || P == 0) return A2P_OK;
     prof_begin("fvt_virial_bwd", stream);
-    auto kern = (long long)B * P >= FVT_WHOLE ? virial_bwd_kernel<T, true> : virial_bwd_kernel<T, false>;
+    auto kern = (long long)B * P * U >= FVT_WHOLE ? virial_bwd_kernel<T, whole_lines<T>()> : virial_bwd_kernel<T, false>;
     hipLaunchKernelGGL(kern, dim3(ceil_div((long long)B * P * 64, 256)), dim3(256), 0, stream,
                        grad_dei, grad_rcs, grad_virial, dei, rcs, B, P, U, bnumneigh);
     prof_end(stream);

@@ -157,10 +157,11 @@ def test_virial_reports_its_own_rows_only():
 @pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
 @pytest.mark.parametrize("U", [1, 21, 63, 64, 65, 130])
 def test_gradients_of_many_rows_equal_those_of_few(np_dtype, U):
-    """Above 2047 rows a wavefront's values leave in whole lines: 45 structures of 47 rows and each of some alone, bit for bit."""
+    """In fp64, from 131,072 slots on, a wavefront's values leave in whole lines: 45 or more structures of 47 rows and each of some
+    alone, bit for bit."""
     import torch
     from ai2pot_amd import ops
-    B, P = 45, 47
+    B, P = max(45, (1 << 17) // (47 * U) + 1), 47
     rng = np.random.default_rng(U)
     t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda:0")
     binum = np.full(B, P, np.int32)
