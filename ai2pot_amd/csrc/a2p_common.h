@@ -342,7 +342,7 @@ template <typename T>
 int finish_partials(T* out, const double* partial, int B, int nblocks, int ncomp, int src_stride,
                     int out_stride, hipStream_t stream, bool timed = true);
 
-// One workgroup of 256 threads: component c (0 energy, 1..9 virial) of structure b from
+// One workgroup of 256 threads, `sh` for its four wavefronts: component c (0 energy, 1..9 virial) of structure b from
 // partial[ev_partial(..)], summed over the blocks by a fixed tree (fp64).  A component's shares lie together: with the ten
 // of a block together, a workgroup fetched ten times the lines it used (8192 blocks of an MTP call: 9.4 -> 5.3 us for the
 // reduction they share a launch with, 12.7 before the sixteen loads in flight).

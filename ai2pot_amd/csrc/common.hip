@@ -501,7 +501,7 @@ int finish_partials(T* out, const double* partial, int B, int nblocks, int ncomp
 template <typename T>
 __global__ void finish_ev_kernel(T* etot, T* virial, const double* partial, int nblocks)
 {
-    __shared__ double sh[256];
+    __shared__ double sh[4];
     finish_ev_body<T>(etot, virial, partial, nblocks, blockIdx.y, blockIdx.x, sh);
 }
 

@@ -49,17 +49,14 @@ __host__ __device__ inline bool mtp_gred_in_moments(bool loss, int n_moms)
 {
     return loss ? 2 * n_moms >= 512 : n_moms >= 1024;
 }
-// entries of the region that holds the neighbour table (+ group sums) and doubles as the sweeps' partial sums.
+// entries of the region that holds the neighbour table (+ group sums).
 // In the energy / force / virial kernel the group sums (4 per thread) are written over the table once every
 // thread has finished reading it.
-// The adjoints live in this region too, behind the partial sums (mtp_adjoint_offset): they are needed from the end of
+// The adjoints live in this region too, behind the scratch of a block sum (MTP_AT_ADJOINTS): they are needed from the end of
 // the forward sweep to the last pass over the neighbours, which is when the neighbour table is not.  That pass needs
 // the adjoints of the basic moments only: the energy / force / virial kernel moves them to its polynomials, the
 // loss kernel moves them behind the region first.
-__host__ __device__ inline int mtp_adjoint_offset(int max_level_slots)
-{
-    return ((max_level_slots > 8 ? max_level_slots : 8) + 1) & ~1;     // at least the scratch of a block sum
-}
+constexpr int MTP_AT_ADJOINTS = 8;
 // keep (energy / force / virial kernel, when the LDS allows it without costing a workgroup per CU): the adjoints lie
 // behind the table instead of inside it, so that a row of one chunk finds its table still in place in the last pass; keep
 // is the number of entries there (0: inside).
@@ -69,12 +66,10 @@ __host__ __device__ inline int mtp_table_entries(int nc, int E, bool loss, int n
     if (!loss && a < nt * 4) a = nt * 4;          // four group sums per thread
     return (a + 1) & ~1;
 }
-__host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_moms, int max_level_slots, int nt,
-                                                int keep = 0)
+__host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_moms, int nt, int keep = 0)
 {
     const int a = mtp_table_entries(nc, E, loss, n_moms, nt);
-    // loss mode: two partial-sum arrays, then the adjoints and the mixed adjoints
-    const int b = loss ? mtp_adjoint_offset(2 * max_level_slots) + 2 * n_moms : mtp_adjoint_offset(max_level_slots) + n_moms;
+    const int b = MTP_AT_ADJOINTS + (loss ? 2 : 1) * n_moms;         // loss mode: the adjoints and the mixed adjoints
     if (keep) return a + keep;
     return a > b ? a : b;
 }
@@ -486,7 +481,7 @@ __device__ __forceinline__ T plan_entry(const T* base, unsigned off)
 // for), the loop has one way out, what is loaded into is free by then (or it goes elsewhere, and copies wait for it), and none of a
 // load's registers is lent to something else meanwhile.  So a step brings its moments along in the multiplicities, the
 // control words of 64 steps lie in a vector register, and an odd step is walked ahead of the loop.
-// Energies and forces of level 20, 8192 atoms, 236 -> 224 us (216 atoms: 28.3 -> 26.9), of level 16, 64 structures of 128 atoms,
+// Kernel of energies and forces, level 20, 8192 atoms, 236 -> 222 us (216 atoms: 28.3 -> 26.9), of level 16, 64 structures of 128 atoms,
 // 90.3 -> 87.7, the loss gradient there 161 -> 159.5; with two products to a multiplicity (step_terms), 14 instead of 24 vector
 // instructions for the four of a step.  (The words of a step in an order that keeps the LDS free of bank conflicts, 1.2 lanes to a
 // bank instead of 2.1: no change.)
@@ -2811,7 +2806,6 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     for (int i = 0; i < 2; i++) { d.fwd_core[i] = stream_at(o_c[i]); d.rev_leaf[i] = stream_at(o_v[i]); }
     d.mapping_leaf = (const int*)(base + o_leaf);
     d.x = MtpStream{nullptr, nullptr, nullptr};
-    d.max_level_slots = 0;       // the sweeps keep no partial sums in LDS
     d.nrows = (int)rows.size() - 1; d.npoly = (int)polys.size(); d.ncoef_poly = n_poly_coef;
     d.rows = (const int*)(base + o_rows); d.polys = (const int*)(base + o_poly);
     d.polys_mu = (const int*)(base + o_pmu); d.polys_end = (const int*)(base + o_pend);
@@ -2880,8 +2874,7 @@ template <typename T>
 size_t lds_bytes(const MtpPlanDevice& p, int E, bool loss, int ntypes, int K, int H, int MTP_NC, int nt,
                  int keep = 0)
 {
-    // the neighbour table and the group sums double as the sweeps' partial-sum arrays
-    const size_t tabs = (size_t)mtp_table_region(MTP_NC, E, loss, p.n_moms, p.max_level_slots, nt, keep);
+    const size_t tabs = (size_t)mtp_table_region(MTP_NC, E, loss, p.n_moms, nt, keep);
     size_t n = (size_t)p.n_moms * (loss ? 2 : 1) + tabs + (loss ? 2 * (size_t)p.ncoef_poly : 0) +
                (size_t)ntypes * p.nmus * K;   // + the coefficient copy
     // loss mode: P, Q, the neighbour types and the per-atom coefficient-gradient block
@@ -3005,15 +2998,14 @@ int launch_atoms(const MtpArgs<T>& args, hipStream_t stream)
         a.at_Tg = p.n_moms;
         a.at_cf = a.at_Tg + (LOSS ? p.n_moms : 0);
         a.at_tab = a.at_cf + a.ntypes * p.nmus * a.K;
-        // the adjoints share the table's region, behind the sweeps' partial sums, or lie behind the table
-        a.at_A = a.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt)
-                                  : mtp_adjoint_offset((LOSS ? 2 : 1) * p.max_level_slots));
+        // the adjoints share the table's region, or lie behind the table
+        a.at_A = a.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt) : MTP_AT_ADJOINTS);
         a.at_Bm = a.at_A + p.n_moms;
         // Partial sums of the thread groups, needed only in the last pass over the neighbours, when the moments (and, in
         // loss mode, their tangents) are dead: a long enough moment vector lends them its place.  Energy / force / virial
         // kernel: they are written over the table once it has been read.
         a.at_gred = !LOSS ? a.at_tab : mtp_gred_in_moments(LOSS, p.n_moms) ? 0 : a.at_tab + nc_cap * a.E;
-        a.at_Ab = a.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, p.max_level_slots, nt, keep);
+        a.at_Ab = a.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, nt, keep);
         a.at_Bb = a.at_Ab + p.ncoef_poly;
         a.at_pq = LOSS ? a.at_Bb + p.ncoef_poly : a.at_Ab;
         a.at_net = a.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);

@@ -38,7 +38,7 @@ constexpr int MTP_CTRL_LEAF = 1 << 29;
 // (Lists cut at sixteen terms and laid out in order of length, in steps of four: 244 instead of 229 us for the call at level 20,
 // 8192 atoms, 304 instead of 286 for the training step at level 16, 64 structures of 128 atoms.)
 struct MtpStream {
-    const int4* head;          // [wavefronts] first step, steps, unused, barriers before the first step
+    const int4* head;          // [wavefronts] first step, steps, (16 bytes to a load), barriers before the first step
     const int* ctrl;           // MTP_CTRL_LEAF, and at the last step of a group 1 | doubling steps << 1 | barriers to pass << 4
     const int4* words;         // slot word: (moment in the first piece of a list, -1 elsewhere) & 0xffff | pieces of the list behind this one
                                // << 16, plus one
@@ -58,7 +58,6 @@ struct MtpPlanDevice {
     // their lists stand with the first sources of the reverse one (control words marked, 8 m0 | 8 m1 << 16).
     MtpStream fwd_core[2], rev_leaf[2];
     const int* mapping_leaf;   // [n_scalar]   mapping | leaf << 16
-    int max_level_slots;       // most slots of any level (forward or reverse)
     // Polynomials of the passes that own a neighbour per lane.  The basic moments (mu, a, b, c) with the same row (a, b) and
     // the same mu are the coefficients of a polynomial in z; its coefficients lie together, highest power first, up to
     // the highest power in the tables (powers the tables leave out: zero).

@@ -274,7 +274,7 @@ reduce_kernel(T* __restrict__ force, const T* __restrict__ seg_g, int* __restric
         read_back_store(post.slot, post.seq, &word, 1);
     }
     if ((int)blockIdx.x >= reduce_blocks) {
-        __shared__ double sh[256];
+        __shared__ double sh[4];
         const int id = (int)blockIdx.x - reduce_blocks;
         finish_ev_body<T>(etot, virial, partial, nblocks, id / 10, id % 10, sh);
         return;
