@@ -147,7 +147,6 @@ struct WaveArgs {
     SegArgs seg;
     T* seg_g;
     WaveAt at;
-    int runs;                        // rows dealt to the workgroups in runs (wave_shape)
 };
 // The lane's place, found anew by each phase as well (again() of a2p_common.h): what the phases derive from it does not fit the registers
 // of three wavefronts per SIMD either.
@@ -168,7 +167,9 @@ __device__ __forceinline__ int lane_again()
     [[maybe_unused]] const int chan = s & 3, mg = s >> 2;                      /* angular channel, MG of its moments */ \
     [[maybe_unused]] int2* const ent = L.ent + g * NW_CAP
 
-template <typename T, int NR, int LC>
+// RUNS: rows dealt to the workgroups in runs (wave_shape).  An instance of its own: the loads that only it makes on the way to the first
+// rows cost the others a wait (fp64, 4,019 atoms 21.8 -> 22.4 us).
+template <typename T, int NR, int LC, bool RUNS>
 __global__ void __launch_bounds__(64 * wave_cap<T>(), sizeof(T) == 4 ? 3 : 1)
 nep_quad_kernel(const WaveArgs<T>)
 {
@@ -190,7 +191,7 @@ nep_quad_kernel(const WaveArgs<T>)
         const int nblocks = a.nblocks;
         b = blockIdx.y; blk = blockIdx.x; last = a.P;
         first = NW_ATOMS * (wave * nblocks + blk); stride = NW_ATOMS * nwaves * nblocks;
-        if (K_.runs) {
+        if constexpr (RUNS) {
             const int at = xcd_block(b * nblocks + blk, nblocks * gridDim.y);
             b = at / nblocks; blk = at - b * nblocks;
             run_of(last, nblocks);
@@ -244,23 +245,27 @@ nep_quad_kernel(const WaveArgs<T>)
         const int tid = threadIdx.x, nthreads = blockDim.x;
         T bias;
         double c3b;
+        [[maybe_unused]] int sample = 0;
         stage_tables<KC, NB, D, WROW, CPAD, 16, T>(a, L, tid, nthreads, [&]() __attribute__((always_inline)) {
             bias = a.bias[min(tid, nt - 1)];
             c3b = kC3B[min(tid, NLM - 1)];
             derivs = a.force != nullptr || a.want_virial;
             claims = derivs && seg.cursor;
             inum = min(uniform_array(a.binum)[b], a.P);       // (the loop below strides over the rows: none beyond the last)
+            if (RUNS) sample = a.binum[(unsigned)lane * gridDim.y / 64];
         });
         if (tid < 4 * MG) L.cw[tid] = tid < NLM ? ((tid == 0 || tid == 3 || tid == 8 || tid == 15) ? (T)1 : (T)2) * (T)c3b : (T)0;
         if (tid < nt) L.bias[tid] = bias;
         for (int i = tid + nthreads; i < nt; i += nthreads) L.bias[i] = a.bias[i];
-        // A structure that leaves a quarter of its places empty is divided by its own number of rows, once that is there
-        // (wave_shape).
-        if (K_.runs && inum <= a.P - a.P / 4) {
+        // Where all structures (of up to 64 looked at) leave a quarter of their places empty, they are divided by their own numbers of rows,
+        // now that these are there (wave_shape).
+        if (RUNS && !__any(sample > a.P - a.P / 4)) {
             run_of(max(inum, 0), a.nblocks);
             begin(first);
+            begin_species();
+        } else {
+            begin_species();
         }
-        begin_species();
     }
     __syncthreads();
 
@@ -783,12 +788,12 @@ nep_quad_kernel(const WaveArgs<T>)
 // and 52.9, 32,768 68.1 and 66.0; 8 of 2,500 61.4 and 47.6, 32 of 640 60.1 and 47.7, 64 of 400 66.2 and 59.7, 128 of 128 44.4
 // and 41.1; fp64 20,011 100 and 98.  With fewer sets all rows of a neighbourhood claim their places at once, from one XCD: 4,096
 // atoms 21.9 and 23.1, 6,000 25.0 and 26.0, 8,192 26.6 and 26.7, 64 structures of 128 24.8 and 29.4.  (XCDs in runs and workgroups in
-// turn: 20,011 atoms 51.4, 32,768 82.9.)  Runs go by the lists' places, for the number of rows in use comes with the tables; with a quarter
-// of the places empty or more by that number, which takes the first rows' loads once more.  In turn, by places alone and so, us: 8 structures
-// of 2,500 places with 1,870 in use 43.8, 39.4 and 41.4, with 1,500 36.2, 37.9 and 35.7, with 800 28.4, 36.2 and 27.4; 64 of 400 with 300
-// 43.2, 48.7 and 40.7, with 150 27.5, 46.0 and 26.9; one of 20,000 with 5,000 23.3, 37.2 and 23.7; fp64 8 of 2,500 with 800 42.3, 91.0 and 41.7;
-// sizes from a third of the places up, 32 of 640 45.8, 39.8 and 42.0, 128 of 128 34.7, 34.0 and 34.8.  (From half of them empty: 8 of 2,500 with
-// 1,500 38.2, 64 of 400 with 300 48.8.)
+// turn: 20,011 atoms 51.4, 32,768 82.9.)  Runs go by the lists' places, for the numbers of rows in use
+// come with the tables; where these show that all structures leave a quarter of their places empty, by those numbers, which takes the first rows'
+// loads once more.  In turn, by places alone and so, us: 8 structures of 2,500 places with 1,870 in use 43.8, 38.9 and 41.4, with 1,500 36.2,
+// 38.0 and 35.3, with 800 28.4, 36.3 and 28.1; 64 of 400 with 300 43.2, 48.7 and 41.2, with 150 27.5, 46.1 and 27.6; one of 20,000 with 5,000 23.3, 37.4
+// and 24.0; fp64 8 of 2,500 with 800 42.3, 91.0 and 42.1.  A structure with all of its places in use takes as long whatever the others do: sizes
+// from a third of the places up, 32 of 640 45.8 in turn, 39.6 by places, 42.0 with the smaller ones by their rows, 128 of 128 34.7, 34.1 and 34.8.
 struct WaveShape { int waves, nblocks, runs; size_t lds; WaveAt at; };
 template <typename T>
 WaveShape wave_shape(const NepArgs<T>& a)
@@ -808,12 +813,12 @@ template <typename T, int NR, int LC>
 int launch_wave(const NepArgs<T>& a, const PairCsr& csr, hipStream_t stream)
 {
     SegArgs seg{csr.cursor, csr.seg_cap, csr.n * csr.seg_cap, csr.mark};
-    auto kern = nep_quad_kernel<T, NR, LC>;
     const WaveShape w = wave_shape<T>(a);
+    auto kern = w.runs ? nep_quad_kernel<T, NR, LC, true> : nep_quad_kernel<T, NR, LC, false>;
     if (w.lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)w.lds));
     prof_begin("nep_quad_kernel", stream);
-    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at, w.runs});
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at});
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;

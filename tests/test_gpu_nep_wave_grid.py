@@ -100,13 +100,19 @@ def test_rows_in_runs_and_in_turn(np_dtype, copies, batch):
 
 
 @pytest.mark.parametrize("np_dtype", [np.float32, np.float64])
-def test_runs_of_structures_with_places_to_spare(np_dtype):
-    """Runs of rows by the places of the lists, and by the rows in use where these leave a quarter of the places empty."""
+@pytest.mark.parametrize("copies,batch,most", [(29, 8, 0), (29, 8, 1), (1, 130, 0)])
+def test_runs_of_structures_with_places_to_spare(np_dtype, copies, batch, most):
+    """Runs of rows by the places of the lists, and by the rows in use where all structures leave a quarter of the places empty (up to
+    64 of them are looked at: the second of 130 is not, and uses all of its places)."""
     m = synth.nep_model(ntypes=3, num_neurons=30, type_map=(1, 2, 3, 4, 5), sigma=0.12)
     m["q_scaler"] = np.linspace(5.0, 10.0, m["q_scaler"].size)
-    nb = _copies(_block(np_dtype, 3), 29, 8)
+    nb = _copies(_block(np_dtype, 3), copies, batch)
     P = nb["bilist"].shape[1]
-    nb["binum"] = np.array([0, 1, 5, 515, P - P // 4 - 1, P - P // 4, P - P // 4 + 1, P], np.int32)
+    top = P - P // 4 + most
+    assert batch * -(-P // 4) > 2048
+    nb["binum"] = np.resize(np.array([0, 1, 5, top // 3, top - 1, top - 2, top - 4, top], np.int32), batch)
+    if batch > 64:
+        nb["binum"][1] = P
     e, f, v = run_gpu(m, nb, np_dtype)
     eps = np.finfo(np_dtype).eps
     for b in range(8):
@@ -114,5 +120,8 @@ def test_runs_of_structures_with_places_to_spare(np_dtype):
         e1, f1, v1 = run_gpu(m, one, np_dtype)
         # (the roundings of test_every_launch_gives_the_same; the sums of a structure grow with its rows)
         assert np.abs(f[b] - f1[0]).max() <= 1200 * eps * np.abs(f1).max()
-        assert np.abs(e[b] - e1[0]).max() <= 1200 * eps * 29 * max(np.abs(e1).max(), 1.0)
-        assert np.abs(v[b] - v1[0]).max() <= 1200 * eps * 29 * max(np.abs(v1).max(), 1.0)
+        assert np.abs(e[b] - e1[0]).max() <= 1200 * eps * copies * max(np.abs(e1).max(), 1.0)
+        assert np.abs(v[b] - v1[0]).max() <= 1200 * eps * copies * max(np.abs(v1).max(), 1.0)
+    for b in range(8, batch):
+        if b % 8 != 1:
+            assert abs(e[b] - e[b % 8]) <= 1200 * eps * copies * max(abs(e[b % 8]), 1.0)
