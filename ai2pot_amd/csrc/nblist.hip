@@ -2010,6 +2010,9 @@ int nblist_build(const T* lattice, const int* types, const T* coords, int N, dou
         // its counters in LDS
         for (int a = 0; a < 3 && sync_free; a++) small = small && cap[a] <= NBS_AXIS;
         if (sync_free) small = small && (long long)cap[0] * cap[1] * cap[2] < NBS_BINS;
+        // ... and its margin (grid_axis, from above) small beside the cell, which small_bins_kernel asks for
+        const double cell = std::fabs((double)g.b[0][0]), length = (double)cap[0] * (double)g.bin_size + 8.0 * cell;
+        if (sync_free) small = small && 1.0e-3 * (double)g.bin_size + 1.0e-5 * (2.0 * big_coord + length) < 0.2 * cell;
     }
     // sorted rows: put in order by the wavefronts that build them while a row fits their registers and LDS (the four
     // rows of a workgroup in 48 KB: three workgroups per CU at least) and can be written with 16-byte stores;

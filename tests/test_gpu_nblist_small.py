@@ -217,7 +217,22 @@ def test_coordinates_whose_rounding_counts_beside_the_cell(oracle):
     L, f = jittered(n, 11, density=0.02)
     lat, ty = np.diag(L).astype(np.float32), synth.rng_randint(3, n, 2)
     site = np.stack(np.unravel_index(np.arange(n), (4, 4, 4)), 1)
+    import torch
+    from ai2pot_amd import _lib
+    from ai2pot_amd.nblist import find_info4mlff_device
     for at in (0.0, 2.0 ** 12, 2.0 ** 17, 2.0 ** 22):
         x = (site * np.float32(L.min() / 4) + np.float32(at) * np.array([1, 0, 0])).astype(np.float32)
         args = (lat, ty, x, 5.0, 200)
-        assert_same(gpu_list(*args), oracle.nblist(*args))
+        want = oracle.nblist(*args)
+        for k in range(2):                               # (the second knows the box of the first, and that it goes the general way)
+            assert_same(gpu_list(*args), want)
+        # without a synchronisation there is no second try: such a structure takes the general route at once
+        t, c = torch.from_numpy(ty.astype(np.int32)).to("cuda:0"), torch.from_numpy(x).to("cuda:0")
+        before = _lib.lib().a2p_nblist_sync_free(1)
+        try:
+            for k in range(2):
+                got = find_info4mlff_device(lat, t, c, 5.0, 200, check=False)
+                _lib.check_status(torch.cuda.current_stream().cuda_stream)
+                assert_same(tuple(o.cpu().numpy() if hasattr(o, "cpu") else o for o in got), want)
+        finally:
+            _lib.lib().a2p_nblist_sync_free(before)
