@@ -147,6 +147,7 @@ struct WaveArgs {
     SegArgs seg;
     T* seg_g;
     WaveAt at;
+    int runs;                        // rows dealt to the workgroups in runs (wave_shape)
 };
 // The lane's place, found anew by each phase as well (again() of a2p_common.h): what the phases derive from it does not fit the registers
 // of three wavefronts per SIMD either.
@@ -168,7 +169,8 @@ __device__ __forceinline__ int lane_again()
     [[maybe_unused]] int2* const ent = L.ent + g * NW_CAP
 
 // RUNS: rows dealt to the workgroups in runs (wave_shape).  An instance of its own: the loads that only it makes on the way to the first
-// rows cost the others a wait (fp64, 4,019 atoms 21.8 -> 22.4 us).
+// rows cost the others a wait (fp64, 4,019 atoms 21.6 -> 22.4 us).  The others ask for `runs` all the same, which is never set there: without
+// that branch the compiler lays their first loads out otherwise, at 21.8.
 template <typename T, int NR, int LC, bool RUNS>
 __global__ void __launch_bounds__(64 * wave_cap<T>(), sizeof(T) == 4 ? 3 : 1)
 nep_quad_kernel(const WaveArgs<T>)
@@ -191,7 +193,7 @@ nep_quad_kernel(const WaveArgs<T>)
         const int nblocks = a.nblocks;
         b = blockIdx.y; blk = blockIdx.x; last = a.P;
         first = NW_ATOMS * (wave * nblocks + blk); stride = NW_ATOMS * nwaves * nblocks;
-        if constexpr (RUNS) {
+        if (RUNS || K_.runs) {
             const int at = xcd_block(b * nblocks + blk, nblocks * gridDim.y);
             b = at / nblocks; blk = at - b * nblocks;
             run_of(last, nblocks);
@@ -818,7 +820,7 @@ int launch_wave(const NepArgs<T>& a, const PairCsr& csr, hipStream_t stream)
     if (w.lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)w.lds));
     prof_begin("nep_quad_kernel", stream);
-    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at});
+    hipLaunchKernelGGL(kern, dim3(a.nblocks, a.B), dim3(64 * w.waves), w.lds, stream, WaveArgs<T>{a, seg, (T*)csr.seg_g, w.at, w.runs});
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
