@@ -26,10 +26,12 @@
 #include "wave_ops.h"
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <map>
 #include <mutex>
 #include <set>
 #include <string>
@@ -41,6 +43,7 @@ namespace {
 constexpr int MTP_NC = 32;        // neighbours per chunk (rows of the LDS table); the energy / force / virial
 constexpr int MTP_NC_MAX = 48;    // the launch picks between MTP_NC_MIN and MTP_NC_MAX rows (launch_atoms)
 constexpr int MTP_NC_MIN = 16;
+constexpr int MTP_SCRATCH = 16;
 
 // The group sums of the last pass over the neighbours (four per thread for the pair derivatives, two
 // for the loss gradient) live in the moment vector (loss mode: moments and tangents) when it is long
@@ -49,28 +52,19 @@ __host__ __device__ inline bool mtp_gred_in_moments(bool loss, int n_moms)
 {
     return loss ? 2 * n_moms >= 512 : n_moms >= 1024;
 }
-// entries of the region that holds the neighbour table (+ group sums).
+// General tables (a kernel that is not TILED): entries of the region that holds the neighbour table (+ group sums).
 // In the energy / force / virial kernel the group sums (4 per thread) are written over the table once every
 // thread has finished reading it.
-// The adjoints live in this region too, behind the scratch of a block sum (MTP_AT_ADJOINTS): they are needed from the end of
+// The adjoints live in this region too: they are needed from the end of
 // the forward sweep to the last pass over the neighbours, which is when the neighbour table is not.  That pass needs
 // the adjoints of the basic moments only: the energy / force / virial kernel moves them to its polynomials, the
 // loss kernel moves them behind the region first.
-constexpr int MTP_AT_ADJOINTS = 8;
-// keep (energy / force / virial kernel, when the LDS allows it without costing a workgroup per CU): the adjoints lie
-// behind the table instead of inside it, so that a row of one chunk finds its table still in place in the last pass; keep
-// is the number of entries there (0: inside).
-__host__ __device__ inline int mtp_table_entries(int nc, int E, bool loss, int n_moms, int nt)
+__host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_moms, int nt)
 {
     int a = loss ? nc * E + (mtp_gred_in_moments(loss, n_moms) ? 0 : (256 / 32) * 32 * 4) : nc * E;
     if (!loss && a < nt * 4) a = nt * 4;          // four group sums per thread
-    return (a + 1) & ~1;
-}
-__host__ __device__ inline int mtp_table_region(int nc, int E, bool loss, int n_moms, int nt, int keep = 0)
-{
-    const int a = mtp_table_entries(nc, E, loss, n_moms, nt);
-    const int b = MTP_AT_ADJOINTS + (loss ? 2 : 1) * n_moms;         // loss mode: the adjoints and the mixed adjoints
-    if (keep) return a + keep;
+    a = (a + 1) & ~1;
+    const int b = (loss ? 2 : 1) * n_moms;         // loss mode: the adjoints and the mixed adjoints
     return a > b ? a : b;
 }
 // the coefficients of the pair-derivative pass's polynomials take the place of the moments when they fit
@@ -108,15 +102,13 @@ struct MtpArgs {
     T* gpart;          // [B, P, ngrad] per-atom gradient rows (ngrad = ncoef + n_scalar + ntypes)
     int ngrad;
     // Places in LDS, in entries (AtomLds), and in a row of the neighbour table: worked out once for the launch.
-    int at_Tg, at_cf, at_tab, at_A, at_Bm, at_gred, at_Ab, at_Bb, at_pq, at_polys, at_net;
+    int at_Tg, at_cf, at_tab, at_A, at_Bm, at_gred, at_Ab, at_Bb, at_pq, at_polys, at_net, at_part, at_scratch;
     int OY, OZ, OG, ODG, OU, OW, OF, ODF;
-    int z_powers;       // the table holds the powers of z (else z alone, and OZ + 1 is its place)
-    int lds_basic_off;  // byte offset of the packed basic-moment table in LDS
+    int PE;             // entries of a neighbour's powers: a table of their own at the beginning of the LDS, or E
+    int lds_basic_off;  // byte offset of the packed basic-moment table in LDS (general tables)
     int grad_parts;     // loss gradient: parts of a chunk's neighbours that are summed at the same time
-    int mom_groups;     // thread groups that share a row's neighbours in the sums of the basic moments (basic_sums), or 0
     int nc_cap;         // rows of the LDS neighbour table: a row is processed in chunks of at most nc_cap
     int leaves_late;    // the streams are fwd_core and rev_leaf: moments that only the read-out reads are formed in the reverse sweep
-    int keep_table;     // energy / force / virial kernel: the adjoints lie behind the table (mtp_table_region)
     // site-energy / descriptor mode (linearMtp.h:514-611, 821-890)
     T* e_sites;        // [B, P] per-row energies, or null
     T* desc;           // [B, P, n_scalar] scalar moments, or null
@@ -146,9 +138,10 @@ __device__ __forceinline__ float sqrt_t(float x) { return sqrtf(x); }
 __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 
 // Per-neighbour table for neighbours [c0, c0+nc) of the row.
-// Layout per neighbour (E entries of T): ux^0..kmax | uy^.. | (z_powers) uz^.. | g[nmus] | dg[nmus] |
-// ux uy uz 1/r | (loss mode) vx vy vz w.u | f[K] | df[K]
-// PASS says what the pass that follows reads: TAB_MOMENTS powers, g, dg; TAB_TANGENTS also w; TAB_GRADIENT powers, w, f, df.
+// Layout per neighbour: in `pw` (stride a.PE) ux^0..kmax | uy^.. | uz^..; in `tab` (E entries of T, the places in MtpArgs) ux uy uz 1/r |
+// g[nmus] | dg[nmus] | (loss mode) vx vy vz w.u | f[K] | df[K].  The two are one table where a.PE is E.
+// PASS says what the passes that follow read: TAB_MOMENTS powers, g, dg; TAB_TANGENTS also w; TAB_ALL also f, df; TAB_GRADIENT powers, w,
+// f, df.  Without `powers` the powers are left out.
 // The threads form groups of nc, a neighbour to a thread.  Groups share the radial functions, two to a Chebyshev
 // recurrence (coefficients from the LDS copy `cf` of the centre species' block); more than two where the workgroup has no
 // room for their groups beside those of the powers, of w and of f.  What bounds it is the issue of fp64 instructions, so a
@@ -157,7 +150,7 @@ __device__ __forceinline__ double sqrt_t(double x) { return sqrt(x); }
 // kernel at level 20, 8192 atoms, 118 instead of 111 at level 16, 64 structures of 128 atoms, and 252 instead of 244 for
 // the loss gradient there; early claims and row-swap sums at the end included.)
 // Lanes j < nc also return the neighbour's index, validity and displacement.
-enum TablePass { TAB_MOMENTS, TAB_TANGENTS, TAB_GRADIENT };
+enum TablePass { TAB_MOMENTS, TAB_TANGENTS, TAB_ALL, TAB_GRADIENT };
 
 // An array on its way to LDS: the first U entries of every thread are asked for together, and stored when the caller says.
 template <typename V, int NT, int U>
@@ -195,9 +188,9 @@ struct TableAhead {
     }
 };
 template <typename T, TablePass PASS, int NT, typename Args>
-__device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int lane, int nc, int c0,
+__device__ __forceinline__ void build_table(Args& a, T* tab, T* pw, const T* cf, int lane, int nc, int c0,
                                             const T* rcs, const int* first, const int* types, int center,
-                                            int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true,
+                                            int b, int NF, int* nj_out, bool* valid_out, T* d_out, bool fill = true, bool powers = true,
                                             const TableAhead<T>& ahead = TableAhead<T>(), bool is_ahead = false)
 {
     const int kmax = a.p.kmax, nmus = a.p.nmus, K = a.K;
@@ -218,7 +211,8 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
     }
     if (!fill) return;                      // the table is in place, only the lanes' own neighbours are returned
     // groups [0, nrad) radial functions, then powers, then w, then f
-    constexpr int OTHERS = PASS == TAB_MOMENTS ? 1 : (PASS == TAB_TANGENTS ? 2 : 3);
+    constexpr bool WITH_W = PASS != TAB_MOMENTS, WITH_F = PASS == TAB_ALL || PASS == TAB_GRADIENT;
+    constexpr int OTHERS = 1 + (WITH_W ? 1 : 0) + (WITH_F ? 1 : 0);
     int share = 0, nrad = 0;
     if (PASS != TAB_GRADIENT) {
         nrad = max(1, min((nmus + 1) / 2, __builtin_amdgcn_readfirstlane(small_div(NT, nc)) - OTHERS));
@@ -239,15 +233,11 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             const T rinv = (T)1 / r;
             const T ux = x * rinv, uy = y * rinv, uz = z * rinv;
             T px = (T)1, py = (T)1, pz = (T)1;
-            if (a.z_powers) {
+            if (powers) {
+                T* const q = pw + j * a.PE;
                 for (int k = 0; k <= kmax; k++) {
-                    t[k] = px; t[kmax + 1 + k] = py; t[2 * (kmax + 1) + k] = pz;
+                    q[k] = px; q[kmax + 1 + k] = py; q[2 * (kmax + 1) + k] = pz;
                     px *= ux; py *= uy; pz *= uz;
-                }
-            } else {
-                for (int k = 0; k <= kmax; k++) {
-                    t[k] = px; t[kmax + 1 + k] = py;
-                    px *= ux; py *= uy;
                 }
             }
             t[OU + 0] = ux; t[OU + 1] = uy; t[OU + 2] = uz; t[OU + 3] = rinv;
@@ -255,7 +245,7 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
         }
         int nj = known ? ahead.nj : first[jj];
         if ((unsigned)nj >= (unsigned)NF) nj = center;
-        if (PASS != TAB_MOMENTS && role == nrad + 1) {
+        if (WITH_W && role == nrad + 1) {
             // w_a = dFs[centre]_a - dFs[neighbour]_a - sum_b dVs[a,b] r_b   (linearMtpLoss.h:371-386), kept as w . u and
             // v = (w - (w . u) u) / r: the monomials are homogeneous, k m = u . grad m, so D_w m = (w . u) m' + v . grad m
             const T* fc = a.dFs + ((size_t)b * a.P + center) * 3;
@@ -284,7 +274,7 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             ds = a.scaling * a.inv_span * ((T)-30 * u * u * u * u + (T)60 * u * u * u - (T)30 * u * u);
         }
         const T sx = s * (T)2 * a.inv_span;
-        if (PASS == TAB_GRADIENT) {
+        if (WITH_F && role == nrad + 2) {
             T t0 = (T)1, t1 = xx, d0 = (T)0, d1 = (T)1;
             for (int k = 0; k < K; k++) {
                 t[OF + k] = s * t0;
@@ -294,6 +284,7 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
             }
             continue;
         }
+        if (PASS == TAB_GRADIENT) continue;
         int tj = known ? ahead.tj : types[nj];
         if ((unsigned)tj >= (unsigned)a.ntypes) tj = 0;
         const int m1 = min(nmus, (role + 1) * share);
@@ -317,78 +308,203 @@ __device__ __forceinline__ void build_table(Args& a, T* tab, const T* cf, int la
     }
 }
 
-// Basic moments of the polynomial (mu, a, b, z^0 .. z^(len-1)) that the thread owns (mtp_plan.h: polys_len), over every
-// ng-th neighbour of a chunk from the h-th on: four LDS reads per polynomial and neighbour and two operations per moment;
-// a thread per basic moment takes four reads and three operations each (tangents: eleven reads and twenty operations; the
-// loss gradient of level 16, 64 structures of 128 atoms, ~ 10 of 230 us longer; energies and forces within 1 %).
-// With TANGENT also D_w M = sum (w . u) g' m + g v . grad m.  `top` is the length of the wavefront's longest polynomial;
-// what a shorter one sums up beyond its length is not used.
-// (A copy of the loop for every second length: one for all, ended by a test behind each power, becomes selects.)
-constexpr int MTP_POLY_MAX = 10;       // longest polynomial (levels up to 22)
-template <typename T, bool TANGENT, int N>
-__device__ __forceinline__ void basic_loop(const T* tab, int E, int nc, int h, int ng, int mu, int ea, int eb, int OX, int OY,
-                                           int OZ, int OG, int ODG, int OW, T (&acc)[MTP_POLY_MAX],
-                                           T (&tacc)[TANGENT ? MTP_POLY_MAX : 1])
+// Basic moments M_(mu,a,b,c) = sum_j (x^a y^b)_j (g_mu z^c)_j of a chunk's neighbours as products of matrices, tile by tile of rows (a, b)
+// and columns (mu, c) (mtp_plan.h), and, with tangents, D_w M = sum_j (x^a y^b) ((w . u) g' z^c + g v_z c z^(c-1)) + (v_x a x^(a-1) y^b +
+// v_y b x^a y^(b-1)) (g z^c).  Four neighbours to an instruction; the sums stay in its accumulators over all chunks of the row.  A
+// wavefront takes up to tiles_of tiles; with fewer tiles than wavefronts these share the neighbours.
+// What bounds it: the matrix instructions, 64 cycles each in fp64 during which the SIMD issues nothing else (as many FMAs as the vector
+// instructions make in that time), with a third of the places of the tiles in use; but the operands of a tile cost 6 LDS reads and some 14
+// vector instructions per four neighbours, where a thread per polynomial in z read four values per neighbour and moment row.
+constexpr int tiles_of(bool loss, int nt) { return loss && nt == 64 ? 1 : 2; }
+struct TileShare {
+    int first, split, nsplit;            // the wavefront's first tile; its share of the neighbours and how many there are
+    template <int NT>
+    static __device__ __forceinline__ TileShare of(int ntiles, int wave)
+    {
+        constexpr int W = NT / 64;
+        if (ntiles >= W) return {wave, 0, 1};
+        const int s = wave >= 2 * ntiles ? (wave >= 3 * ntiles ? 3 : 2) : (wave >= ntiles ? 1 : 0);       // (at most three tiles)
+        return {wave - s * ntiles, s, ntiles == 1 ? W : W / 2 >= ntiles ? 2 : 1};
+    }
+};
+// The exponents of the lane's row and column of a tile.
+template <typename T>
+__device__ __forceinline__ unsigned tile_word(const unsigned* ops, int tile, int lane)
 {
-#pragma unroll 1
-    for (int j = h; j < nc; j += ng) {
-        const T* t = tab + j * E;
-        const T xa = t[OX + ea], yb = t[OY + eb], z = t[OZ + 1], g = t[OG + mu];
-        const T ab = xa * yb;
-        T p = g * ab;
-        if (!TANGENT) {
+    // (in single precision the lane's places are rows 4 (l / 16) + v of the product: its rows in the order that makes them those of the plan)
+    const unsigned own = ops[tile * 64 + lane];
+    if (sizeof(T) == 8) return own;
+    return (ops[tile * 64 + (lane & 3) * 4 + (lane >> 2 & 3)] & 0x3ffu) | (own & ~0x3ffu);
+}
+template <typename T, bool TANGENT, int NT, int TILES, typename Args>
+__device__ __forceinline__ void tile_products(Args& a, const T* tab, const T* pw, int tid, int nc, const TileShare& ts, const unsigned (&word)[TILES],
+                                              typename wave::Acc<T>::type (&m)[TILES], typename wave::Acc<T>::type (&d)[TILES])
+{
+    const int kq = (tid & 63) >> 4, E = a.E, PE = a.PE, n1 = a.p.kmax + 1, ntiles = a.p.ntiles;
+    if (ts.split >= ts.nsplit) return;
+    const int steps = (nc + 3) >> 2;
+    const int k0 = ts.nsplit == 1 ? 0 : ts.split * steps / ts.nsplit, k1 = ts.nsplit == 1 ? steps : (ts.split + 1) * steps / ts.nsplit;
 #pragma unroll
-            for (int c = 0; c < N; c++) {
-                acc[c] += p;
-                if (c + 1 < N) p *= z;
-            }
-        } else {
-            const T q = t[OW + 3] * t[ODG + mu] * ab +
-                        g * (((T)ea * t[OX + max(ea - 1, 0)] * yb) * t[OW + 0] + ((T)eb * xa * t[OY + max(eb - 1, 0)]) * t[OW + 1]);
-            const T pv = p * t[OW + 2];
-            T zc = (T)1, dz = (T)0;                              // z^c and its derivative
-#pragma unroll
-            for (int c = 0; c < N; c++) {
-                acc[c] += p * zc;
-                tacc[c] += q * zc + pv * dz;
-                dz = dz * z + zc;
-                zc *= z;
+    for (int u = 0; u < TILES; u++) {
+        if (ts.first + u * (NT / 64) >= ntiles || (u > 0 && ts.nsplit > 1)) break;
+        const int ea = word[u] & 31, eb = word[u] >> 5 & 31, mu = word[u] >> 10 & 7, ec = word[u] >> 13;
+        const T *const px = pw + ea, *const py = pw + n1 + eb, *const pz = pw + 2 * n1 + ec, *const pg = tab + a.OG + mu;
+#pragma unroll 2
+        for (int k = k0; k < k1; k++) {
+            const int j = k * 4 + kq;
+            const bool on = j < nc;
+            const unsigned jj = on ? j : nc - 1, ap = __umul24(jj, PE), at = __umul24(jj, E);
+            const T xa = px[ap], yb = py[ap], zc = pz[ap], g = pg[at];
+            const T row = xa * yb, col = on ? g * zc : (T)0;
+            m[u] = wave::mma(row, col, m[u]);
+            if (TANGENT) {
+                const T xm = px[(int)ap - (ea > 0)], ym = py[(int)ap - (eb > 0)], zm = pz[(int)ap - (ec > 0)], dg = pg[at + a.ODG - a.OG];
+                const T *const w = tab + at + a.OW;
+                const T rowd = ((T)ea * w[0]) * (xm * yb) + ((T)eb * w[1]) * (xa * ym);
+                const T cold = on ? (w[3] * dg) * zc + ((T)ec * w[2]) * (g * zm) : (T)0;
+                d[u] = wave::mma(row, cold, d[u]);
+                d[u] = wave::mma(rowd, col, d[u]);
             }
         }
     }
 }
-template <typename T, bool TANGENT>
-__device__ __forceinline__ void basic_sums(const T* tab, int E, int nc, int h, int ng, unsigned word, int top, int OX, int OY,
-                                           int OZ, int OG, int ODG, int OW, T (&acc)[MTP_POLY_MAX],
-                                           T (&tacc)[TANGENT ? MTP_POLY_MAX : 1])
+// A wavefront's sums to their moments.
+template <typename T, int NT, int TILES, typename Plan>
+__device__ __forceinline__ void tile_store(Plan& p, T* dst, int tid, const TileShare& ts, const typename wave::Acc<T>::type (&m)[TILES])
 {
-    const int mu = word & 7, ea = (word >> 3) & 31, eb = (word >> 8) & 31;
+    if (ts.split >= ts.nsplit) return;
 #pragma unroll
-    for (int c = 0; c < MTP_POLY_MAX; c++) {
-        acc[c] = (T)0;
-        if (TANGENT) tacc[c] = (T)0;
+    for (int u = 0; u < TILES; u++) {
+        const int tile = ts.first + u * (NT / 64);
+        if (tile >= p.ntiles || (u > 0 && ts.nsplit > 1)) break;
+        const uint2 at = p.tile_place[tile * 64 + (tid & 63)];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const unsigned i = (v < 2 ? at.x : at.y) >> (v & 1 ? 16 : 0) & 0xffffu;
+            if (i != MTP_NO_MOMENT) dst[i] = m[u][v];
+        }
     }
-    if (h >= ng) nc = 0;
-    if (top <= 2) basic_loop<T, TANGENT, 2>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
-    else if (top <= 4) basic_loop<T, TANGENT, 4>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
-    else if (top <= 6) basic_loop<T, TANGENT, 6>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
-    else if (top <= 8) basic_loop<T, TANGENT, 8>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
-    else basic_loop<T, TANGENT, 10>(tab, E, nc, h, ng, mu, ea, eb, OX, OY, OZ, OG, ODG, OW, acc, tacc);
 }
 
-// A thread's sums to its group's coefficients in `part` [ng][ncoef] (highest power first), and a coefficient's sum over the
-// groups, in their order.
+// A unit (mtp_plan.h): the polynomial of degree M in x and t whose coefficients stand at `c`, with its derivatives, and, with BOTH, the
+// value of the one at `cb`.  G lanes to a neighbour: with one, t = y; with two, t = xy and the powers of t take two degrees each.
+// Nested Horner's rule without a branch: two FMAs per coefficient (three), three per power of t (four).
 template <typename T>
-__device__ __forceinline__ void basic_part(T* part, const T (&acc)[MTP_POLY_MAX], int h, int ng, unsigned word, int ncoef)
+struct UnitSums { T v, x, t, b; };
+template <int G>
+constexpr int unit_size(int M)
 {
-    const int len = (word >> 13) & 31;
-    T* const mine = part + h * ncoef + (word >> 18) + (len - 1);
-    if (h < ng) {
+    int n = 0;
+    for (int b = 0; b <= (G == 2 ? M / 2 : M); b++) n += M - G * b + 1;
+    return n;
+}
+// The coefficients come by lots, one ahead of the one in use (all at once they take a hundred registers).
+template <typename T, int G, int M, bool BOTH>
+__device__ __forceinline__ UnitSums<T> unit_poly(const T* c, const T* cb, T x, T t)
+{
+    constexpr int TOP = G == 2 ? M / 2 : M, N = unit_size<G>(M), AHEAD = BOTH ? 2 : 4;
+    UnitSums<T> s = {(T)0, (T)0, (T)0, (T)0};
+    T lot[2][AHEAD], lotb[2][BOTH ? AHEAD : 1];
+    auto fetch = [&](int i0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int c = 0; c < MTP_POLY_MAX; c++)
-            if (c < len) mine[-c] = acc[c];
+        for (int u = 0; u < AHEAD; u++) {
+            if (i0 + u >= N) continue;
+            lot[i0 / AHEAD & 1][u] = c[i0 + u];
+            if (BOTH) lotb[i0 / AHEAD & 1][u] = cb[i0 + u];
+        }
+    };
+    fetch(0);
+    T v = (T)0, d = (T)0, vb = (T)0;
+    int b = TOP, k = 0;                                 // row, place in it
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        if (i % AHEAD == 0) {
+            // (nothing of the lots before is left for later, and no later lot is asked for yet)
+            if (i > 0) asm volatile("" : "+v"(v), "+v"(d), "+v"(s.v), "+v"(s.x), "+v"(s.t) : : "memory");
+            if (BOTH && i > 0) asm volatile("" : "+v"(vb), "+v"(s.b) : : "memory");
+            fetch(i + AHEAD);
+        }
+        const T ci = lot[i / AHEAD & 1][i % AHEAD];
+        const T cbi = BOTH ? lotb[i / AHEAD & 1][BOTH ? i % AHEAD : 0] : (T)0;
+        if (k == 0) {
+            v = ci; d = (T)0; vb = cbi;
+        } else {
+            d = k == 1 ? v : d * x + v;
+            v = v * x + ci;
+            if (BOTH) vb = vb * x + cbi;
+        }
+        if (++k == M - G * b + 1) {
+            if (b == TOP) {
+                s.v = v; s.x = d; s.b = vb;
+            } else {
+                s.t = b == TOP - 1 ? s.v : s.t * t + s.v;
+                s.v = s.v * t + v;
+                s.x = s.x * t + d;
+                if (BOTH) s.b = s.b * t + vb;
+            }
+            b--;
+            k = 0;
+        }
+    }
+    return s;
+}
+template <typename T, int G, bool BOTH>
+__device__ __forceinline__ UnitSums<T> unit_sums(int M, const T*& c, const T*& cb, T x, T t)
+{
+    UnitSums<T> s;
+#define MTP_UNIT(N) case N: s = unit_poly<T, G, N, BOTH>(c, cb, x, t); c += unit_size<G>(N); if (BOTH) cb += unit_size<G>(N); break;
+    switch (M) {
+        MTP_UNIT(1) MTP_UNIT(2) MTP_UNIT(3) MTP_UNIT(4) MTP_UNIT(5) MTP_UNIT(6) MTP_UNIT(7) MTP_UNIT(8) MTP_UNIT(9)
+        default: s = unit_poly<T, G, 0, BOTH>(c, cb, x, t); c++; if (BOTH) cb++;
+    }
+#undef MTP_UNIT
+    static_assert(MTP_NEST_MAX == 9, "a case for every degree");
+    return s;
+}
+
+// The wavefront's units at the lane's neighbour, whose table row is t: with A = sum adj m over the basic moments m of a mu, taken as a
+// polynomial in (x, y, z), `done` receives mu, the share's number, A, its gradient, and, with BOTH, the value B of the second coefficients.
+// With two lanes to a neighbour (G), the upper 32 lanes of the wavefront have x and y exchanged, and each lane the sums of its half.
+// All lanes of a wavefront take the same way, so that what describes a unit costs scalar instructions only, and read the same one or two
+// coefficients.  What bounds it is the issue of the FMAs: a lane per (neighbour, share of the polynomials in z of all rows (a, b)) before
+// took six LDS reads and some thirty instructions per polynomial beside its FMAs, of which polynomials of different lengths left some idle.
+template <typename T, int G, bool BOTH, typename Done>
+__device__ __forceinline__ void nested(const T* coef, const T* coefb, int prog, int n, T x, T y, T z, Done&& done)
+{
+    const T t = G == 2 ? x * y : y;
+    T r = (T)0, rx = (T)0, rt = (T)0, rz = (T)0, rb = (T)0;
+#pragma unroll 1
+    for (int i = 0; i < n; i++) {
+        const int w = __builtin_amdgcn_readlane(prog, i);
+        const UnitSums<T> s = unit_sums<T, G, BOTH>(w & 15, coef, coefb, x, t);
+        rz = rz * z + r;
+        r = r * z + s.v;
+        rx = rx * z + s.x;
+        rt = rt * z + s.t;
+        if (BOTH) rb = rb * z + s.b;
+        if (w & 128) {
+            for (int k = w >> 8 & 31; k > 0; k--) {            // (the next powers of z are another wavefront's)
+                rz = rz * z + r;
+                r *= z; rx *= z; rt *= z;
+                if (BOTH) rb *= z;
+            }
+            done(w >> 4 & 7, w >> 13, r, rx, rt, rz, rb);
+            r = rx = rt = rz = rb = (T)0;
+        }
     }
 }
+// The coefficients of the units out of the adjoints of the basic moments.
+template <typename T, int NT, typename Plan>
+__device__ __forceinline__ void unit_coefficients(Plan& p, int G, T* dst, const T* A, int tid)
+{
+    const int n = p.nstream[G - 1];
+    const unsigned short* const src = p.stream_src[G - 1];
+    for (int i = tid; i < n; i += NT) {
+        const int m = src[i];
+        dst[i] = m == MTP_NO_MOMENT ? (T)0 : A[m];
+    }
+}
+
 template <typename T>
 __device__ __forceinline__ T group_sum(const T* src, int ng, int ncoef)
 {
@@ -716,49 +832,6 @@ __device__ __forceinline__ void pair_walk(const T* __restrict__ t, const T* __re
     }
 }
 
-// The same sums polynomial by polynomial, longest first (mtp_plan.h: polys_len): every ng-th one, so that the lanes of a
-// wavefront walk polynomials of about the same length.  With V, D the value and derivative in z the polynomial adds
-//   gs += x^a y^b g' V,  w_x += a x^(a-1) y^b g V,  w_y += b x^a y^(b-1) g V,  w_z += x^a y^b g D
-// and the monomials are homogeneous, k m = u . grad m, so -(u . w) / r completes gs at the end.  What bounds it is the chain
-// of LDS reads and operations of a polynomial: its word is read while the one before is worked on, and its values in one go.
-// (Row by row, the radial functions of a row together, the whole kernel took 102 us instead of 98 for 64 x 128 atoms at level
-// 16, 260 instead of 255 for 8192 atoms at level 20 and 17.6 instead of 16.6 for 216 at level 10.)
-template <typename T>
-__device__ __forceinline__ void poly_walk(const T* __restrict__ t, const T* __restrict__ coef, const unsigned* __restrict__ words,
-                                          int npoly, int h, int ng, int OX, int OY, int OZ, int OG, int ODG, T ux, T uy, T uz,
-                                          T rinv, T& gs, T& wx, T& wy, T& wz)
-{
-    const T z = t[OZ + 1];
-    unsigned next = words[h];
-#pragma unroll 1
-    for (int s = h; s < npoly;) {
-        const unsigned pw = next;
-        s += ng;
-        if (s < npoly) next = words[s];
-        const int mu = pw & 7, ea = (pw >> 3) & 31, eb = (pw >> 8) & 31;
-        int len = (pw >> 13) & 31;
-        const T* c = coef + (pw >> 18);                          // highest power first
-        const T g = t[OG + mu], dg = t[ODG + mu], xa = t[OX + ea], yb = t[OY + eb], xm = t[OX + max(ea - 1, 0)],
-                ym = t[OY + max(eb - 1, 0)];
-        T v = (T)0, d = (T)0;
-        if (len & 1) v = *c++;
-#pragma unroll 1
-        for (len >>= 1; len > 0; len--, c += 2) {
-            const T c0 = c[0], c1 = c[1];
-            d = d * z + v;
-            v = v * z + c0;
-            d = d * z + v;
-            v = v * z + c1;
-        }
-        const T xy = xa * yb, gv = g * v;
-        gs += xy * dg * v;
-        wx += (T)ea * xm * yb * gv;
-        wy += (T)eb * xa * ym * gv;
-        wz += xy * g * d;
-    }
-    gs -= (ux * wx + uy * wy + uz * wz) * rinv;
-}
-
 // The polynomials of a neighbour for the loss gradient: every ng-th one of a radial function's from the s-th on.  With
 // A = sum adj m, B = sum (cE adj + mixed) m over the basic moments of mu and k m = u . grad m (m is homogeneous),
 //   P_mu = B + (w - (w . u) u) . grad A / r,   Q_mu = (w . u) A.
@@ -799,14 +872,14 @@ __device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __re
     Q *= wu;
 }
 
-// The workgroup's LDS: moments | (loss mode: their tangents) | coefficients of the centre species | region of the neighbour
-// table | ...
-template <typename T, bool LOSS, int NT>
+// The workgroup's LDS (launch_atoms): moments | (loss mode: their tangents) | adjoints | (mixed adjoints), in whose place the powers of the
+// neighbours' unit vectors stand before | coefficients of the centre species | neighbour table | ...
+// General tables: moments | tangents | coefficients | neighbour table, in whose place the adjoints come after it | ...
+template <typename T, bool LOSS>
 struct AtomLds {
-    T *M, *Tg, *cf, *tab, *A, *Bm, *gred, *Ab, *Bb, *pq, *polys, *net;
+    T *M, *Tg, *cf, *tab, *A, *Bm, *gred, *Ab, *Bb, *pq, *polys, *net, *part, *scratch;
     unsigned* bas;
     int* rws;
-    bool keep;
     template <typename Args>
     __device__ __forceinline__ AtomLds(Args& a, unsigned char* smem)
     {
@@ -814,8 +887,6 @@ struct AtomLds {
         Tg = M + a.at_Tg;
         cf = M + a.at_cf;                       // [ntypes][nmus][K]
         tab = M + a.at_tab;
-        // the adjoints (loss mode: and the mixed adjoints) share the table's region, or lie behind the table (keep)
-        keep = !LOSS && a.keep_table != 0;      // uniform over the launch
         A = M + a.at_A;
         Bm = M + a.at_Bm;
         gred = M + a.at_gred;                   // partial sums of the thread groups
@@ -826,8 +897,10 @@ struct AtomLds {
         pq = M + a.at_pq;
         polys = M + a.at_polys;                 // energy / force / virial: coefficients of the polynomials
         net = M + a.at_net;                     // network inputs and per-neuron values
-        // behind everything else: (mu, a, b, c) of every basic moment, one byte each, or its place among the coefficients
-        // (mom_groups); monomial rows and polynomials of the pair-derivative walk
+        part = M + a.at_part;                   // sums of the basic moments by wavefronts that share a tile
+        scratch = M + a.at_scratch;             // a value per wavefront; sums over the pairs of a row's chunks so far
+        // general tables, behind everything else: (mu, a, b, c) of every basic moment, one byte each; monomial rows and polynomials of
+        // the pair-derivative walk
         bas = (unsigned*)(smem + a.lds_basic_off);
         rws = (int*)(bas + a.p.n_basic);
     }
@@ -843,8 +916,9 @@ struct AtomLds {
     [[maybe_unused]] auto& p = a.p;                                                                                        \
     [[maybe_unused]] const bool seeded = (SEED || LOSS) && a.row_seed != nullptr;                                          \
     [[maybe_unused]] const bool no_tan = LOSS && a.no_tangent != 0;                 /* uniform over the launch */          \
-    [[maybe_unused]] const AtomLds<T, LOSS, NT> L(a, smem_raw);                                                            \
+    [[maybe_unused]] const AtomLds<T, LOSS> L(a, smem_raw);                                                            \
     [[maybe_unused]] T *const M = L.M, *const Tg = L.Tg, *const cf = L.cf, *const tab = L.tab, *const A = L.A, *const Bm = L.Bm; \
+    [[maybe_unused]] T* const pw = TILED ? M : tab;                                                                        \
     [[maybe_unused]] const int NF = a.P + a.nghost, n_moms = p.n_moms, n_basic = p.n_basic, nmus = p.nmus, kmax = p.kmax,  \
                                K = a.K, E = a.E, MTP_NC = a.nc_cap;                                                        \
     [[maybe_unused]] const int OX = 0, OY = a.OY, OZ = a.OZ, OG = a.OG, ODG = a.ODG, OU = a.OU, OW = a.OW, OF = a.OF, ODF = a.ODF; \
@@ -857,7 +931,9 @@ struct AtomLds {
 // the registers are kept to match (four: 321 us instead of 303 at 8192 atoms; six spill: 361).
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
 // (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.  NET: the instances with a network read-out.
-template <typename T, bool LOSS, int NT, bool SEED = false, bool NET = false>
+// TILED: the passes over the neighbours by matrix products and nested polynomials (mtp_plan.h: ntiles), where the tables fit them; the
+// others go by basic moments and by polynomials in z, with 256 threads.
+template <typename T, bool LOSS, int NT, bool SEED = false, bool NET = false, bool TILED = true>
 __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) == 8 ? 6 : 1)) mtp_atom_kernel(const MtpArgs<T>)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
@@ -866,8 +942,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     int center, nn, ti;
     int nchunks, csize;               // the row is cut into equal chunks of at most nc_cap neighbours
     TableAhead<T> ahead;              // (energies and forces; the loss gradient's registers do not hold it: 166 -> 175 us)
-    int mgroups, mh, mtop = 0;        // sums of the basic moments: groups, the thread's group, the longest polynomial
-    unsigned pword = 0;               // ... and the thread's polynomial
+    constexpr int TILES = tiles_of(LOSS, NT);
+    unsigned tword[TILES];        // the lane's rows and columns of the wavefront's tiles
+    const int wave = __builtin_amdgcn_readfirstlane(lane >> 6), l64 = lane & 63;
     {
         MTP_PHASE;
         // (scalar loads, on their way while the plan's arrays are asked for; a padded row has places in the lists as well)
@@ -880,20 +957,18 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         // atoms 228.8 -> 226.4 us, the training step of level 16, 64 structures of 128 atoms, 272.8 -> 270.5, the linear solver there
         // 469 -> 462.)
         // (The number of rows was a trip of its own ahead of these: level 10, 216 atoms 29.5 -> 29.1 us, the solver 403 -> 401.)
-        mgroups = a.mom_groups;       // uniform over the launch
-        const unsigned* const bsrc = mgroups ? (const unsigned*)p.poly_pos : p.basic;
         Staged<unsigned, NT, NT == 64 ? 4 : 2> basics;
-        basics.load(bsrc, n_basic, lane);
-        mh = mgroups;
-        if (mgroups) {
-            mh = small_div(lane, p.npoly);
-            if (mh < mgroups) pword = p.polys_len[lane - mh * p.npoly];
-        }
-        const bool flat = !LOSS && p.polys_len;
-        const int nwords = flat ? p.npoly : LOSS ? p.npoly : p.nrows + 1;
-        const int* const wsrc = flat ? (const int*)p.polys_len : LOSS ? p.polys_mu : p.rows;
+        const int nwords = LOSS ? p.npoly : p.nrows + 1;
+        const int* const wsrc = LOSS ? p.polys_mu : p.rows;
         Staged<int, NT, NT == 64 ? 2 : 1> words;
-        words.load(wsrc, nwords, lane);
+        if constexpr (TILED) {
+            const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
+#pragma unroll
+            for (int u = 0; u < TILES; u++) tword[u] = tile_word<T>(p.tile_ops, min(ts.first + u * (NT / 64), p.ntiles - 1), l64);
+        } else {
+            basics.load(p.basic, n_basic, lane);
+            words.load(wsrc, nwords, lane);
+        }
         if (ii >= inum) {                  // padded row: contributes nothing
             if (!LOSS && a.partial && lane < 10) a.partial[ev_partial(a.P, b, ii, lane)] = 0.0;
             if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
@@ -913,21 +988,17 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             csize = cuts > 1 ? (int)((n + cuts - 1) / cuts) : max(nn, 1);
         }
         if (!LOSS && nn > 0) ahead.entries(rcs, first, lane, 0, min(csize, nn));
-        for (int i = lane; i < n_moms; i += NT) {
-            M[i] = (T)0;
-            if (LOSS) Tg[i] = (T)0;
-        }
-        basics.store(L.bas, bsrc, n_basic, lane);
-        words.store(L.rws, wsrc, nwords, lane);
-        if (!LOSS && !flat)
-            for (int i = lane; i < p.npoly; i += NT) L.rws[p.nrows + 1 + i] = p.polys[i];
-        if (LOSS)
-            for (int i = lane; i <= nmus; i += NT) L.rws[p.npoly + i] = p.polys_end[i];
-        if (mgroups) {
-            const int len = (pword >> 13) & 31;
-#pragma unroll
-            for (int c = 0; c < MTP_POLY_MAX; c++)
-                if (__any(len > c)) mtop = c + 1;
+        if constexpr (!TILED) {
+            for (int i = lane; i < n_moms; i += NT) {
+                M[i] = (T)0;
+                if (LOSS) Tg[i] = (T)0;
+            }
+            basics.store(L.bas, p.basic, n_basic, lane);
+            words.store(L.rws, wsrc, nwords, lane);
+            if (!LOSS)
+                for (int i = lane; i < p.npoly; i += NT) L.rws[p.nrows + 1 + i] = p.polys[i];
+            else
+                for (int i = lane; i <= nmus; i += NT) L.rws[p.npoly + i] = p.polys_end[i];
         }
         if ((unsigned)ti >= (unsigned)a.ntypes) { if (lane == 0) atomicOr(a.status, ST_BAD_TYPE); ti = 0; nn = 0; }
         const T* const csrc = a.coeffs + (size_t)ti * a.ntypes * nmus * K;
@@ -939,42 +1010,45 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     }
 
     // ---- basic moments (and their tangents) --------------------------------------------------
-    for (int c0 = 0; nn > 0;) {
-        const int nc = min(csize, nn - c0);
-        {
-            MTP_PHASE;
-            int nj; bool valid; T d[3];
-            build_table<T, LOSS ? TAB_TANGENTS : TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, true,
-                                                                      ahead, !LOSS);
-            __syncthreads();
-        }
+    [[maybe_unused]] typename wave::Acc<T>::type msum[TILES], dsum[TILES];
+    auto table = [&](int c0, int nc) __attribute__((always_inline)) {
         MTP_PHASE;
-        if (mgroups) {
-            // the groups' sums pass through the table's place, or through the adjoints' when the table stays
-            T* const part = L.keep ? A : tab;
-            T macc[MTP_POLY_MAX];
-            if (LOSS && !no_tan) {
-                T mtan[LOSS ? MTP_POLY_MAX : 1];
-                basic_sums<T, LOSS>(tab, E, nc, mh, mgroups, pword, mtop, OX, OY, OZ, OG, ODG, OW, macc, mtan);
-                if constexpr (LOSS) {
-                    __syncthreads();
-                    basic_part<T>(part + mgroups * p.ncoef_poly, mtan, mh, mgroups, pword, p.ncoef_poly);
-                }
-            } else {
-                T none[1];
-                basic_sums<T, false>(tab, E, nc, mh, mgroups, pword, mtop, OX, OY, OZ, OG, ODG, OW, macc, none);
-                if (!L.keep) __syncthreads();
-            }
-            basic_part<T>(part, macc, mh, mgroups, pword, p.ncoef_poly);
+        int nj; bool valid; T d[3];
+        build_table<T, LOSS ? (TILED ? TAB_ALL : TAB_TANGENTS) : TAB_MOMENTS, NT>(a, tab, pw, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid,
+                                                                              d, true, true, ahead, !LOSS);
+        __syncthreads();
+    };
+    auto next_ahead = [&](int c0) __attribute__((always_inline)) {
+        if (LOSS) return;              // (not held over the sums)
+        MTP_PHASE;
+        ahead.entries(rcs, first, lane, c0, min(csize, nn - c0));
+        ahead.species(types, NF, center);
+    };
+    if constexpr (TILED) {
+        auto products = [&](int nc) __attribute__((always_inline)) {
+            MTP_PHASE;
+            const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
+            if (LOSS && !no_tan) tile_products<T, LOSS, NT, TILES>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
+            else tile_products<T, false, NT, TILES>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
             __syncthreads();
-            for (int i = lane; i < n_basic; i += NT) {
-                const int pos = L.bas[i];
-                M[i] += group_sum<T>(part + pos, mgroups, p.ncoef_poly);
-                if (LOSS && !no_tan) Tg[i] += group_sum<T>(part + mgroups * p.ncoef_poly + pos, mgroups, p.ncoef_poly);
-            }
-            __syncthreads();
-        } else {
-            // (tables beyond the fields of polys_len)
+        };
+        // (the first chunk, of most rows the only one, by itself: sums held over the table's phase do not fit the registers)
+        if (nn > 0) table(0, min(csize, nn));
+#pragma unroll
+        for (int u = 0; u < TILES; u++) msum[u] = dsum[u] = {0, 0, 0, 0};
+        if (nn > 0) products(min(csize, nn));
+#pragma unroll 1
+        for (int c0 = csize; c0 < nn; c0 += csize) {
+            next_ahead(c0);
+            table(c0, min(csize, nn - c0));
+            products(min(csize, nn - c0));
+        }
+    } else {
+        for (int c0 = 0; c0 < nn; c0 += csize) {
+            const int nc = min(csize, nn - c0);
+            if (c0 > 0) next_ahead(c0);
+            table(c0, nc);
+            MTP_PHASE;
             for (int i = lane; i < n_basic; i += NT) {
                 const unsigned bw = L.bas[i];
                 const int mu = bw & 255, ea = (bw >> 8) & 255, eb = (bw >> 16) & 255, ec = bw >> 24;
@@ -998,11 +1072,25 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             }
             __syncthreads();
         }
-        c0 += csize;
-        if (c0 >= nn) break;
-        if (!LOSS) {                   // (not held over the sums)
-            ahead.entries(rcs, first, lane, c0, min(csize, nn - c0));
-            ahead.species(types, NF, center);
+    }
+    if constexpr (TILED) {             // the powers are dead: the moments take their place
+        MTP_PHASE;
+        const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
+        const int per = LOSS ? 2 * n_basic : n_basic;
+        tile_store<T, NT, TILES>(p, ts.split == 0 ? M : L.part + (ts.split - 1) * per, lane, ts, msum);
+        if (LOSS) tile_store<T, NT, TILES>(p, ts.split == 0 ? Tg : L.part + (ts.split - 1) * per + n_basic, lane, ts, dsum);
+        for (int i = n_basic + lane; i < n_moms; i += NT) {
+            M[i] = (T)0;
+            if (LOSS) Tg[i] = (T)0;
+        }
+        __syncthreads();
+        if (ts.nsplit > 1) {
+            for (int i = lane; i < n_basic; i += NT)
+                for (int k = 0; k + 1 < ts.nsplit; k++) {
+                    M[i] += L.part[k * per + i];
+                    if (LOSS) Tg[i] += L.part[k * per + n_basic + i];
+                }
+            __syncthreads();
         }
     }
 
@@ -1168,7 +1256,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         if (!LOSS && (a.e_sites || a.desc)) {
             if (a.desc)                                          // linearMtp.h:884-885: unscaled scalar moments
                 for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = M[p.mapping[s]];
-            const T e_row = block_sum<T, NT>(e_part, tab, lane) + a.bias[ti];      // the table is idle between the sweeps
+            const T e_row = block_sum<T, NT>(e_part, L.scratch, lane) + a.bias[ti];
             if (a.e_sites && lane == 0) a.e_sites[row] = e_row;  // linearMtp.h:594-599
             if (a.energy_only) return;
         }
@@ -1191,27 +1279,35 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
 
     if (!LOSS) {
         // ---- pair derivatives ------------------------------------------------------------------
-        // The adjoints of the basic moments as polynomial coefficients; the moments are dead
-        // Within a chunk of nc neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one
-        // per monomial row) share the rows, so a short chunk still keeps the workgroup busy.
+        // The adjoints of the basic moments as polynomial coefficients; the moments are dead.  Nested polynomials: two lanes to a neighbour
+        // where a chunk has no more than 32, one otherwise; the wavefronts share the units.  General tables: within a chunk of nc
+        // neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one per monomial row) share the rows.
+        const int halves = csize <= 32 ? 2 : 1;
+        [[maybe_unused]] int prog = 0;
         {
             MTP_PHASE;
-            scatter_polys<T, NT>(p, L.polys, A, lane);
+            if constexpr (TILED) {
+                unit_coefficients<T, NT>(p, halves, L.polys, A, lane);
+                prog = p.units[NT / 256][2 * (NT / 64) + lane];
+            } else {
+                scatter_polys<T, NT>(p, L.polys, A, lane);
+            }
         }
-        T fx = (T)0, fy = (T)0, fz = (T)0;
-        T vir[9];
-#pragma unroll
-        for (int q = 0; q < 9; q++) vir[q] = (T)0;
+        // Sums over the pairs, chunk by chunk, in wavefront 0's place in LDS (held by lane from chunk to chunk they cost the walk 24 registers).
+        if (lane < 12) {
+            MTP_PHASE;
+            L.scratch[4 + lane] = (T)0;
+        }
         for (int c0 = 0; c0 < nn; c0 += csize) {
             const int nc = min(csize, nn - c0);
             int nj; bool valid; T d[3] = {(T)0, (T)0, (T)0};
             __syncthreads();
-            // (a row of one chunk finds the table of the first pass still in place when the adjoints lie behind it)
+            // (nested polynomials: a row of one chunk finds the table of the first pass still in place)
             {
                 MTP_PHASE;
-                build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
-                                          !(L.keep && nchunks == 1));
-                __syncthreads();
+                build_table<T, TAB_MOMENTS, NT>(a, tab, pw, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d,
+                                          !TILED || nchunks > 1, !TILED);
+                if (!TILED || nchunks > 1) __syncthreads();
             }
             T gs = (T)0, wx = (T)0, wy = (T)0, wz = (T)0;
             T ux = (T)0, uy = (T)0, uz = (T)0, rinv = (T)0;
@@ -1220,30 +1316,69 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             int rk = 0, ng, h, j;
             {
                 MTP_PHASE;
-                ng = min(small_div(NT, nc), p.polys_len ? p.npoly : p.nrows);
-                h = small_div(lane, nc); j = lane - h * nc;
                 if (a.seg_cursor && lane < nc) rk = pair_claim_raw(&a.seg_cursor[b * NF + nj]);
-                if (h < ng) {
-                    const T* t = tab + j * E;
+                if constexpr (TILED) {
+                    ng = NT / 64; h = wave; j = halves == 2 ? l64 & 31 : l64;
+                    const T* t = tab + min(j, nc - 1) * E;
                     ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
-                    if (p.polys_len)
-                        poly_walk<T>(t, L.polys, (const unsigned*)L.rws, p.npoly, h, ng, OX, OY, OZ, OG, ODG, ux, uy, uz, rinv, gs, wx, wy, wz);
-                    else
+                    const int n = uniform_array(p.units[NT / 256])[2 * wave], at = uniform_array(p.units[NT / 256])[2 * wave + 1];
+                    T wt = (T)0;
+                    auto add = [&](int mu, int, T r, T rx, T rt, T rz, T) __attribute__((always_inline)) {
+                        const T g = t[OG + mu], dg = t[ODG + mu];
+                        gs += dg * r;
+                        wx += g * rx; wt += g * rt; wz += g * rz;
+                    };
+                    if (halves == 2) {
+                        const bool up = l64 >= 32;
+                        const T x = up ? uy : ux, y = up ? ux : uy;
+                        nested<T, 2, false>(L.polys + (at >> 16) + (up ? p.half_at : 0), (const T*)nullptr, prog, n, x, y, uz, add);
+                        wx += y * wt;
+                        wy = x * wt;
+                        const T sw = up ? wy : wx;
+                        wy = up ? wx : wy;
+                        wx = sw;
+                        gs = wave::add_rows<32>(gs); wx = wave::add_rows<32>(wx); wy = wave::add_rows<32>(wy); wz = wave::add_rows<32>(wz);
+                    } else {
+                        nested<T, 1, false>(L.polys + (at & 0xffff), (const T*)nullptr, prog, n, ux, uy, uz, add);
+                        wy = wt;
+                    }
+                } else {
+                    ng = min(small_div(NT, nc), p.nrows);
+                    h = small_div(lane, nc); j = lane - h * nc;
+                    if (h < ng) {
+                        const T* t = tab + j * E;
+                        ux = t[OU + 0]; uy = t[OU + 1]; uz = t[OU + 2]; rinv = t[OU + 3];
                         pair_walk<T>(t, L.polys, L.rws, L.rws + p.nrows + 1, p.nrows, h, ng, OX, OY, OZ, OG, ODG, rinv, gs, wx, wy, wz);
+                    }
                 }
             }
-            __syncthreads();            // every thread has read its table row: the group sums take its place
+            if (!TILED) __syncthreads();            // every thread has read its table row: the group sums take its place
             MTP_PHASE;
             // group sums in the order h = 0 .. ng-1
-            {
+            if (!TILED) {
                 T* gr = L.gred + lane * 4;
                 gr[0] = gs; gr[1] = wx; gr[2] = wy; gr[3] = wz;
+            } else if (NT > 64 && h > 0 && l64 < nc) {
+                T* gr = L.gred + ((h - 1) * nc + l64) * 4;
+                gr[0] = gs; gr[1] = wx; gr[2] = wy; gr[3] = wz;
             }
-            __syncthreads();
-            if (h == 0) {
-                for (int hh = 1; hh < ng; hh++) {
-                    const T* gr = L.gred + (hh * nc + j) * 4;
-                    gs += gr[0]; wx += gr[1]; wy += gr[2]; wz += gr[3];
+            if (!TILED || NT > 64) __syncthreads();
+            T fv[12];
+#pragma unroll
+            for (int q = 0; q < 12; q++) fv[q] = (T)0;
+            if (TILED ? lane < nc : h == 0) {
+                if constexpr (TILED) {
+#pragma unroll
+                    for (int w = 0; w < NT / 64 - 1; w++) {
+                        const T* gr = L.gred + (w * nc + j) * 4;
+                        gs += gr[0]; wx += gr[1]; wy += gr[2]; wz += gr[3];
+                    }
+                    gs -= (ux * wx + uy * wy + uz * wz) * rinv;        // the monomials are homogeneous: k m = u . grad m
+                } else {
+                    for (int hh = 1; hh < ng; hh++) {
+                        const T* gr = L.gred + (hh * nc + j) * 4;
+                        gs += gr[0]; wx += gr[1]; wy += gr[2]; wz += gr[3];
+                    }
                 }
                 T gx = gs * ux + wx * rinv;
                 T gy = gs * uy + wy * rinv;
@@ -1260,25 +1395,33 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
                     T* dst = a.pair_out + (row * a.U + c0 + j) * 3;
                     dst[0] = gx; dst[1] = gy; dst[2] = gz;
                 }
-                fx += gx; fy += gy; fz += gz;
-                vir[0] -= gx * d[0]; vir[1] -= gx * d[1]; vir[2] -= gx * d[2];
-                vir[3] -= gy * d[0]; vir[4] -= gy * d[1]; vir[5] -= gy * d[2];
-                vir[6] -= gz * d[0]; vir[7] -= gz * d[1]; vir[8] -= gz * d[2];
+                fv[0] = gx; fv[1] = gy; fv[2] = gz;
+                fv[3] = -gx * d[0]; fv[4] = -gx * d[1]; fv[5] = -gx * d[2];
+                fv[6] = -gy * d[0]; fv[7] = -gy * d[1]; fv[8] = -gy * d[2];
+                fv[9] = -gz * d[0]; fv[10] = -gz * d[1]; fv[11] = -gz * d[2];
+            }
+            if (lane < 64) {
+                T* const kept = L.scratch + 4;
+#pragma unroll
+                for (int q = 0; q < 12; q++) {
+                    fv[q] = wave::all_sum(fv[q]) + kept[q];
+                    kept[q] = fv[q];
+                }
             }
         }
         MTP_PHASE;
         // only the threads of group 0 (inside wave 0) hold force and virial terms: the other wavefronts are done
-        const double e_atom = (double)block_sum<T, NT>(e_part, L.gred, lane);
+        const double e_atom = (double)block_sum<T, NT>(e_part, L.scratch, lane);
         if (lane >= 64) return;
-        fx = wave::all_sum(fx); fy = wave::all_sum(fy); fz = wave::all_sum(fz);
+        const T* const fvsum = L.scratch + 4;
         double out[10];
         out[0] = e_atom + (seeded ? 0.0 : (double)a.bias[ti]);
 #pragma unroll
-        for (int q = 0; q < 9; q++) out[1 + q] = (double)wave::all_sum(vir[q]);
+        for (int q = 0; q < 9; q++) out[1 + q] = (double)fvsum[3 + q];
         if (lane == 0) {
             if (!SEED || a.force) {
                 T* fo = a.force + ((size_t)b * NF + center) * 3;
-                fo[0] = fx; fo[1] = fy; fo[2] = fz;
+                fo[0] = fvsum[0]; fo[1] = fvsum[1]; fo[2] = fvsum[2];
                 if (a.seg_mark) pair_mark_own(&a.seg_cursor[b * NF + center]);
             }
             if (!SEED || a.partial) {
@@ -1292,6 +1435,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     // ---- loss gradient ------------------------------------------------------------------------
     if (LOSS) {
         T cE;
+        const int halves = csize <= 32 ? 2 : 1;
+        [[maybe_unused]] int prog = 0;
         {
             MTP_PHASE;
             cE = seeded ? (T)1 : (a.cE_per_atom ? a.cE[row] : a.cE[b]);
@@ -1299,8 +1444,21 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         {
             MTP_PHASE;
             // the last pass needs the adjoints of the basic moments while the table is back in its region
-            scatter_polys<T, NT>(p, L.Ab, A, lane);
-            scatter_polys<T, NT>(p, L.Bb, Bm, lane);
+            if constexpr (TILED) {
+                // (B's coefficients: cE times the adjoints plus the mixed ones)
+                const int n = p.nstream[halves - 1];
+                const unsigned short* const src = p.stream_src[halves - 1];
+                for (int i = lane; i < n; i += NT) {
+                    const int m = src[i];
+                    const T av = m == MTP_NO_MOMENT ? (T)0 : A[m];
+                    L.Ab[i] = av;
+                    L.Bb[i] = m == MTP_NO_MOMENT ? (T)0 : cE * av + Bm[m];
+                }
+                prog = p.units[NT / 256][2 * (NT / 64) + lane];
+            } else {
+                scatter_polys<T, NT>(p, L.Ab, A, lane);
+                scatter_polys<T, NT>(p, L.Bb, Bm, lane);
+            }
             const int ncoef = a.ntypes * a.ntypes * nmus * K;
             T* grow = a.gpart + row * a.ngrad;
             for (int q = lane; q < a.ngrad; q += NT) grow[q] = (T)0;
@@ -1348,15 +1506,63 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
             // equal chunks and as many thread groups per chunk as fit, as in the pair-derivative pass
             const int nc = min(csize, nn - c0);
             const int ng = min(small_div(NT, nc), MTP_NGMAX);
-            const int h = small_div(lane, nc), j = lane - h * nc;
+            const int h = TILED ? (lane < nc ? 0 : 1) : small_div(lane, nc), j = TILED ? lane : lane - h * nc;
             int nj; bool valid; T d[3];
             __syncthreads();
             {
                 MTP_PHASE;
-                build_table<T, TAB_GRADIENT, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
-                __syncthreads();
+                build_table<T, TAB_GRADIENT, NT>(a, tab, pw, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, !TILED || nchunks > 1, !TILED);
+                if (!TILED || nchunks > 1) __syncthreads();
             }
-            {
+            if constexpr (TILED) {
+                MTP_PHASE;
+                // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  With A = sum adj m, B = sum (cE adj + mixed) m
+                // over the basic moments of mu and k m = u . grad m (m is homogeneous),
+                //   P_mu = B + (w - (w . u) u) . grad A / r,   Q_mu = (w . u) A.
+                const T* t = tab + min(halves == 2 ? l64 & 31 : l64, nc - 1) * E;
+                const T x = t[OU + 0], y = t[OU + 1], z = t[OU + 2];
+                const T vx = no_tan ? (T)0 : t[OW + 0], vy = no_tan ? (T)0 : t[OW + 1], vz = no_tan ? (T)0 : t[OW + 2], wu = no_tan ? (T)0 : t[OW + 3];
+                const bool up = halves == 2 && l64 >= 32, whole = p.nshares[NT / 256] == nmus && NT == 64;
+                // along x (y in the upper half) at constant t, and along t
+                const T hx = up ? vy : vx, ht = halves == 2 ? vx * y + vy * x : vy;
+                const int n = uniform_array(p.units[NT / 256])[2 * wave], at = uniform_array(p.units[NT / 256])[2 * wave + 1];
+                auto add = [&](int mu, int share, T r, T rx, T rt, T rz, T rb) __attribute__((always_inline)) {
+                    T P = rb + hx * rx + ht * rt + vz * rz, Q = wu * r;
+                    if (halves == 2) { P = wave::add_rows<32>(P); Q = wave::add_rows<32>(Q); }
+                    if (l64 < nc) {
+                        if (whole) {
+                            L.pq[l64 * nmus + mu] = P;
+                            L.pq[MTP_NC * nmus + l64 * nmus + mu] = Q;
+                        } else {
+                            T* o = L.gred + (share * nc + l64) * 2;
+                            o[0] = P; o[1] = Q;
+                        }
+                    }
+                };
+                if (halves == 2) {
+                    const int o = (at >> 16) + (up ? p.half_at : 0);
+                    nested<T, 2, true>(L.Ab + o, L.Bb + o, prog, n, up ? y : x, up ? x : y, z, add);
+                } else {
+                    nested<T, 1, true>(L.Ab + (at & 0xffff), L.Bb + (at & 0xffff), prog, n, x, y, z, add);
+                }
+                __syncthreads();
+                if (!whole) {
+                    for (int q = lane; q < nc * nmus; q += NT) {
+                        const int mu = small_div(q, nc), jn = q - mu * nc;
+                        const unsigned long long shares = p.mu_shares[NT / 256];
+                        int k0 = 0;
+                        for (int m = 0; m < mu; m++) k0 += (int)(shares >> (8 * m)) & 255;
+                        T P = (T)0, Q = (T)0;
+                        for (int k = k0; k < k0 + ((int)(shares >> (8 * mu)) & 255); k++) {
+                            P += L.gred[(k * nc + jn) * 2];
+                            Q += L.gred[(k * nc + jn) * 2 + 1];
+                        }
+                        L.pq[jn * nmus + mu] = P;
+                        L.pq[MTP_NC * nmus + jn * nmus + mu] = Q;
+                    }
+                    __syncthreads();
+                }
+            } else {
                 MTP_PHASE;
                 // P_mu(j), Q_mu(j): linearMtpLoss.h:438-536 with the k-sum factored out.  The groups take the polynomials in
                 // turn, on from one mu to the next.  (All of a thread's sums kept to the end, with one round of group sums:
@@ -1625,7 +1831,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
         COMP_PHASE;
         const int nc = min(chunk, nn - c0);
         int nj; bool valid; T d[3];
-        build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, true, ahead, true);
+        build_table<T, TAB_MOMENTS, NT>(a, tab, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d, true, true, ahead, true);
         __syncthreads();
         for (int i = lane; i < n_basic; i += NT) {
             const unsigned bw = bas[i];
@@ -1713,7 +1919,7 @@ __global__ void __launch_bounds__(NT, 4) mtp_components_kernel(const CompKernelA
             if (nchunks > 1) {                             // (a single chunk's table is still in place)
                 COMP_PHASE;
                 int nj; bool valid; T d[3];
-                build_table<T, TAB_MOMENTS, NT>(a, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
+                build_table<T, TAB_MOMENTS, NT>(a, tab, tab, cf, lane, nc, c0, rcs, first, types, center, b, NF, &nj, &valid, d);
                 __syncthreads();
             }
             for (int j0 = 0; j0 < nc; j0 += batch) {
@@ -2194,8 +2400,15 @@ void spread_over_banks(const std::vector<std::vector<int>>& lists, int depth, in
     }
 }
 
-// 256 threads per atom or 64 (the rule is at its definition)
+// 256 threads per atom or 64 (the rule is at its definition), and whether a launch then goes by tiles and nested polynomials: others take
+// 256 threads
 bool wide_atoms(int n_moms, bool loss, bool network, bool fp64);
+bool tiled_launch(int ntiles, bool loss, bool wide) { return ntiles > 0 && ntiles <= tiles_of(loss, wide ? 256 : 64) * (wide ? 4 : 1); }
+bool wide_launch(int n_moms, int ntiles, bool loss, bool network, bool fp64)
+{
+    const bool wide = wide_atoms(n_moms, loss, network, fp64);
+    return wide || !tiled_launch(ntiles, loss, wide);
+}
 
 int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const int* times, int n_scalar,
                 const int* mapping, MtpPlan** out)
@@ -2527,20 +2740,6 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const Best leaf_best = best_level(fl, leaves);
     A2P_REQUIRE(!too_long, A2P_ERR_INVALID,
                 "mtp plan: a moment takes part in more than %d products; this level is too large", 64 * MTP_SLOT_CAP);
-    // The streams that a launch can ask for: those of the widths that wide_atoms gives for as many moments, and the forward one
-    // of four wavefronts for the components.  (Host time of a plan with all of them and every cut laid out for each by itself
-    // 1.83 ms for level 16 and 14.2 for level 20, with the streams reached alone 0.78 and 4.2, in pairs of a multiplicity 0.77 and 4.1.)
-    bool reached[2] = {false, false};
-    for (int q = 0; q < 8; q++) reached[wide_atoms(n_moms, q & 1, q & 2, q & 4)] = true;
-    Stream fs[2], rs[2], cs[2], vs[2];
-    for (int i = 0; i < 2; i++) {
-        const int waves = i ? 4 : 1;
-        if (reached[i] || i == 1) fs[i] = build_stream(build_ell(fl, f_best, i), true, waves);
-        if (!reached[i]) continue;
-        rs[i] = build_stream(build_ell(rl, r_best, i), false, waves);
-        cs[i] = build_stream(build_ell(fl, c_best, i), true, waves);
-        vs[i] = build_stream(build_ell(rl, r_best, i, &fl, &leaf_best), false, waves);
-    }
     // monomial rows, their polynomials and the places of the basic moments among the coefficients (mtp_plan.h)
     std::vector<int> degree((size_t)(kmax + 1) * (kmax + 1) * nmus, 0);      // highest c + 1 of (a, b, mu), 0: none
     for (int i = 0; i < n_basic; i++) {
@@ -2583,11 +2782,9 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     }
     std::vector<unsigned> polys_len;                              // longest first, for the sums of the basic moments
     const bool polys_fit = n_poly_coef < (1 << 14);               // (kmax <= 24, nmus <= 8)
-    int poly_top = 0;
     for (size_t r = 0; r < row_ab.size(); r++)
         for (int q = rows[r] >> 16; q < rows[r + 1] >> 16; q++) {
             const int mu = polys[q] & 15, len = (polys[q] >> 4) & 255, beg = polys[q] >> 12;
-            poly_top = std::max(poly_top, len);
             polys_len.push_back((unsigned)mu | (unsigned)row_ab[r].first << 3 | (unsigned)row_ab[r].second << 8 |
                                 (unsigned)len << 13 | (unsigned)beg << 18);
         }
@@ -2608,6 +2805,134 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
         poly_items.insert(poly_items.end(), poly_lists[e].begin(), poly_lists[e].end());
     }
     poly_items_off[n_poly_coef] = (int)poly_items.size();
+
+    // tiles of the matrix products and units of the nested polynomials (mtp_plan.h)
+    std::vector<unsigned> tile_ops;
+    std::vector<uint2> tile_place;
+    std::vector<unsigned short> stream_src[2];
+    std::vector<int> units[2];
+    int ntiles = 0, half_at = 0, nshares[2] = {0, 0};
+    unsigned long long mu_shares[2] = {0, 0};
+    std::vector<int> mu_degree(nmus, -1);
+    for (int i = 0; i < n_basic; i++) {
+        const int* q = basic + i * 4;
+        mu_degree[q[0]] = std::max(mu_degree[q[0]], q[1] + q[2] + q[3]);
+    }
+    int nunits = 0;
+    for (int m = 0; m < nmus; m++) nunits += mu_degree[m] + 1;
+    if (poly_unique && kmax <= MTP_NEST_MAX && nunits <= MTP_UNITS_MAX && n_basic < MTP_NO_MOMENT) {
+        std::map<std::array<int, 4>, int> at;                      // (mu, a, b, c) -> basic moment
+        std::map<std::pair<int, int>, int> in_row, in_col;
+        for (int i = 0; i < n_basic; i++) {
+            const int* q = basic + i * 4;
+            at[{q[0], q[1], q[2], q[3]}] = i;
+            in_row[{q[1], q[2]}]++;
+            in_col[{q[0], q[3]}]++;
+        }
+        auto moment = [&](int mu, int a, int b, int c) {
+            const auto f = at.find({mu, a, b, c});
+            return f == at.end() ? MTP_NO_MOMENT : f->second;
+        };
+        auto by_count = [](const std::map<std::pair<int, int>, int>& of) {
+            std::vector<std::pair<int, int>> v;
+            for (const auto& e : of) v.push_back(e.first);
+            std::stable_sort(v.begin(), v.end(), [&](const auto& x, const auto& y) { return of.at(x) > of.at(y); });
+            return v;
+        };
+        const std::vector<std::pair<int, int>> trow = by_count(in_row), tcol = by_count(in_col);
+        for (size_t c0 = 0; c0 < tcol.size(); c0 += 16)
+            for (size_t r0 = 0; r0 < trow.size(); r0 += 16) {
+                std::vector<uint2> place(64);
+                bool any = false;
+                for (int l = 0; l < 64; l++) {
+                    unsigned p[4];
+                    for (int v = 0; v < 4; v++) {
+                        const size_t r = r0 + 4 * v + l / 16, c = c0 + l % 16;
+                        p[v] = r < trow.size() && c < tcol.size() ? moment(tcol[c].first, trow[r].first, trow[r].second, tcol[c].second) : MTP_NO_MOMENT;
+                        any = any || p[v] != MTP_NO_MOMENT;
+                    }
+                    place[l] = make_uint2(p[0] | p[1] << 16, p[2] | p[3] << 16);
+                }
+                if (!any) continue;
+                ntiles++;
+                tile_place.insert(tile_place.end(), place.begin(), place.end());
+                for (int l = 0; l < 64; l++) {
+                    const auto& r = trow[std::min(r0 + l % 16, trow.size() - 1)];
+                    const auto& c = tcol[std::min(c0 + l % 16, tcol.size() - 1)];
+                    tile_ops.push_back((unsigned)r.first | (unsigned)r.second << 5 | (unsigned)c.first << 10 | (unsigned)c.second << 13);
+                }
+            }
+        struct Unit { int mu, c, M, cost, at[2]; };
+        std::vector<Unit> list;
+        std::vector<unsigned short> half[2];
+        for (int m = 0; m < nmus; m++)
+            for (int c = mu_degree[m]; c >= 0; c--) {
+                const int M = mu_degree[m] - c;
+                list.push_back({m, c, M, 5 * (M + 1) * (M + 2) / 4 + 3 * (M + 1) + 9, {(int)stream_src[0].size(), (int)half[0].size()}});
+                for (int b = M; b >= 0; b--)
+                    for (int a = M - b; a >= 0; a--) stream_src[0].push_back((unsigned short)moment(m, a, b, c));
+                for (int b = M / 2; b >= 0; b--)
+                    for (int e = M - 2 * b; e >= 0; e--) {
+                        half[0].push_back((unsigned short)moment(m, b + e, b, c));
+                        half[1].push_back((unsigned short)(e > 0 ? moment(m, b, b + e, c) : MTP_NO_MOMENT));
+                    }
+            }
+        // (lanes of the two halves read a coefficient each, and often the next one too: their banks apart)
+        half_at = (int)half[0].size();
+        while (half_at % 32 < 4 || half_at % 32 > 28) half_at++;
+        stream_src[1] = half[0];
+        stream_src[1].resize(half_at, MTP_NO_MOMENT);
+        stream_src[1].insert(stream_src[1].end(), half[1].begin(), half[1].end());
+        for (int w = 0; w < 2; w++) {
+            const int waves = w ? 4 : 1;
+            // runs of units, the dearest as cheap as can be: the smallest bound that needs no more wavefronts than there are
+            std::vector<int> first(1, 0);
+            int total = 0, bound = 0;
+            for (const Unit& u : list) { total += u.cost; bound = std::max(bound, u.cost); }
+            for (bound = std::max(bound, total / waves);; bound++) {
+                first.assign(1, 0);
+                int sum = 0;
+                for (int i = 0; i < (int)list.size(); i++) {
+                    if (sum + list[i].cost > bound) { first.push_back(i); sum = 0; }
+                    sum += list[i].cost;
+                }
+                if ((int)first.size() <= waves) break;
+            }
+            first.resize(waves + 1, (int)list.size());
+            std::vector<int> words((size_t)waves * 64, 0);
+            int share = -1;
+            for (int k = 0; k < waves; k++) {
+                const int i0 = first[k], i1 = first[k + 1];
+                units[w].push_back(i1 - i0);
+                units[w].push_back(i0 < i1 ? list[i0].at[0] | list[i0].at[1] << 16 : 0);
+                for (int i = i0; i < i1; i++) {
+                    if (i == i0 || list[i].mu != list[i - 1].mu) {
+                        share++;
+                        mu_shares[w] += 1ull << (8 * list[i].mu);
+                    }
+                    const int end = i + 1 == i1 || list[i + 1].mu != list[i].mu;
+                    words[(size_t)k * 64 + i - i0] = list[i].M | list[i].mu << 4 | end << 7 | list[i].c << 8 | share << 13;
+                }
+            }
+            units[w].insert(units[w].end(), words.begin(), words.end());
+            nshares[w] = share + 1;
+        }
+    }
+
+    // The streams that a launch can ask for: those of the widths that wide_launch gives for as many moments, and the forward one
+    // of four wavefronts for the components.  (Host time of a plan with all of them and every cut laid out for each by itself
+    // 1.83 ms for level 16 and 14.2 for level 20, with the streams reached alone 0.78 and 4.2, in pairs of a multiplicity 0.77 and 4.1.)
+    bool reached[2] = {false, false};
+    for (int q = 0; q < 8; q++) reached[wide_launch(n_moms, ntiles, q & 1, q & 2, q & 4)] = true;
+    Stream fs[2], rs[2], cs[2], vs[2];
+    for (int i = 0; i < 2; i++) {
+        const int waves = i ? 4 : 1;
+        if (reached[i] || i == 1) fs[i] = build_stream(build_ell(fl, f_best, i), true, waves);
+        if (!reached[i]) continue;
+        rs[i] = build_stream(build_ell(rl, r_best, i), false, waves);
+        cs[i] = build_stream(build_ell(fl, c_best, i), true, waves);
+        vs[i] = build_stream(build_ell(rl, r_best, i, &fl, &leaf_best), false, waves);
+    }
 
     const bool x_polys = polys_fit && n_poly_coef == n_basic;
     // nodes (scalar moment, ancestor) and their reverse gather (mtp_plan.h), for batches of scalar moments whose node
@@ -2772,6 +3097,13 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     const size_t o_pit = add(poly_items.data(), sizeof(int) * poly_items.size());
     const size_t o_ppos = add(poly_pos.data(), sizeof(int) * poly_pos.size());
     const size_t o_plen = add(polys_len.data(), sizeof(unsigned) * polys_len.size());
+    const size_t o_tops = add(tile_ops.data(), sizeof(unsigned) * tile_ops.size());
+    const size_t o_tplace = add(tile_place.data(), sizeof(uint2) * tile_place.size());
+    size_t o_ssrc[2], o_unit[2];
+    for (int i = 0; i < 2; i++) {
+        o_ssrc[i] = add(stream_src[i].data(), sizeof(unsigned short) * stream_src[i].size());
+        o_unit[i] = add(units[i].data(), sizeof(int) * units[i].size());
+    }
     struct XOff { size_t root, seed, bbase, bdepth, bsteps, brem, bwords; StreamOff x; };
     std::vector<XOff> xoffs;
     for (const XHost& h : xhosts) {
@@ -2813,8 +3145,17 @@ int plan_create(int n_moms, int n_basic, const int* basic, int n_times, const in
     d.poly_items = (const int*)(base + o_pit); d.poly_pos = (const int*)(base + o_ppos);
     d.x_polys = x_polys;
     d.polys_len = polys_fit ? (const unsigned*)(base + o_plen) : nullptr;
-    d.poly_top = poly_top;
     d.poly_unique = poly_unique;
+    d.ntiles = ntiles; d.half_at = half_at;
+    d.tile_ops = (const unsigned*)(base + o_tops);
+    d.tile_place = (const uint2*)(base + o_tplace);
+    for (int i = 0; i < 2; i++) {
+        d.nstream[i] = (int)stream_src[i].size();
+        d.stream_src[i] = (const unsigned short*)(base + o_ssrc[i]);
+        d.units[i] = (const int*)(base + o_unit[i]);
+        d.nshares[i] = nshares[i];
+        d.mu_shares[i] = mu_shares[i];
+    }
     d.x_nodes = 0; d.x_slots = 0;                // set per batch by the components call (MtpPlan::xbatches)
     for (size_t i = 0; i < xhosts.size(); i++) {
         const XOff& o = xoffs[i];
@@ -2843,45 +3184,84 @@ int plan_check(void* handle, MtpPlan** out)
     return A2P_OK;
 }
 
-// Whether the atom kernel sums the basic moments by polynomials (basic_sums): each has a thread, and the sums of a group
-// of threads fit the place of the shortest table.  Otherwise each moment is formed by itself, from powers of z.
-bool poly_sums(const MtpPlanDevice& p, bool loss, bool network, bool fp64)
-{
-    return p.polys_len && p.poly_top <= MTP_POLY_MAX && p.npoly <= (wide_atoms(p.n_moms, loss, network, fp64) ? 256 : 64) &&
-           (loss ? 2 : 1) * p.ncoef_poly <= MTP_NC_MIN * (2 * (p.kmax + 1) + 2 * p.nmus + 4);
-}
-
-// The entries of a row of the neighbour table.
-template <typename T>
-void table_layout(MtpArgs<T>& a, bool loss, bool z_powers)
-{
-    const MtpPlanDevice& p = a.p;
-    a.z_powers = z_powers ? 1 : 0;
-    a.OY = p.kmax + 1;
-    a.OG = (z_powers ? 3 : 2) * (p.kmax + 1);
-    a.ODG = a.OG + p.nmus; a.OU = a.ODG + p.nmus; a.OW = a.OU + 4; a.OF = a.OW + 4; a.ODF = a.OF + a.K;
-    a.OZ = z_powers ? 2 * (p.kmax + 1) : a.OU + 1;
-    a.E = a.OU + 4 + (loss ? 4 + 2 * a.K : 0);
-    if ((a.E & 1) == 0) a.E++;        // odd stride: neighbours land in different LDS banks
-}
+// The entries of a row of the neighbour table, the powers among them (general tables, components).
 template <typename T>
 void table_layout(MtpArgs<T>& a, bool loss)
 {
-    table_layout(a, loss, !poly_sums(a.p, loss, a.H > 0, sizeof(T) == 8));
+    const MtpPlanDevice& p = a.p;
+    a.OY = p.kmax + 1;
+    a.OZ = 2 * (p.kmax + 1);
+    a.OG = 3 * (p.kmax + 1);
+    a.ODG = a.OG + p.nmus; a.OU = a.ODG + p.nmus; a.OW = a.OU + 4; a.OF = a.OW + 4; a.ODF = a.OF + a.K;
+    a.E = a.OU + 4 + (loss ? 4 + 2 * a.K : 0);
+    a.E |= 1;                         // odd stride: neighbours land in different LDS banks
+    a.PE = a.E;
 }
 
+// LDS of a workgroup of the atom kernel for tables of nc rows, in entries; sets the places in `a` (AtomLds).
+// General tables: moments | (loss mode: their tangents) | coefficients | region of the neighbour table | ...
 template <typename T>
-size_t lds_bytes(const MtpPlanDevice& p, int E, bool loss, int ntypes, int K, int H, int MTP_NC, int nt,
-                 int keep = 0)
+size_t general_lds(MtpArgs<T>& a, bool loss, int nc)
 {
-    const size_t tabs = (size_t)mtp_table_region(MTP_NC, E, loss, p.n_moms, nt, keep);
-    size_t n = (size_t)p.n_moms * (loss ? 2 : 1) + tabs + (loss ? 2 * (size_t)p.ncoef_poly : 0) +
-               (size_t)ntypes * p.nmus * K;   // + the coefficient copy
-    // loss mode: P, Q, the neighbour types and the per-atom coefficient-gradient block
-    if (loss) n += 2 * (size_t)MTP_NC * p.nmus + MTP_NC + (size_t)ntypes * p.nmus * K;
-    if (H > 0) n += (size_t)p.n_scalar + (loss ? 5 : 1) * (size_t)H;     // network inputs and per-neuron values
-    if (!loss && !mtp_polys_in_moments(p.ncoef_poly, p.n_moms)) n += (size_t)p.ncoef_poly;
-    return n * sizeof(T) + 64;      // the packed basic-moment table (4 n_basic bytes) follows
+    const MtpPlanDevice& p = a.p;
+    const int nt = 256, ncf = a.ntypes * p.nmus * a.K;
+    table_layout(a, loss);
+    a.at_Tg = p.n_moms;
+    a.at_cf = a.at_Tg + (loss ? p.n_moms : 0);
+    a.at_tab = a.at_cf + ncf;
+    a.at_A = a.at_tab;
+    a.at_Bm = a.at_A + p.n_moms;
+    // Partial sums of the thread groups, needed only in the last pass over the neighbours, when the moments (and, in
+    // loss mode, their tangents) are dead: a long enough moment vector lends them its place.  Energy / force / virial
+    // kernel: they are written over the table once it has been read.
+    a.at_gred = !loss ? a.at_tab : mtp_gred_in_moments(loss, p.n_moms) ? 0 : a.at_tab + nc * a.E;
+    a.at_Ab = a.at_tab + mtp_table_region(nc, a.E, loss, p.n_moms, nt);
+    a.at_Bb = a.at_Ab + p.ncoef_poly;
+    a.at_pq = loss ? a.at_Bb + p.ncoef_poly : a.at_Ab;
+    a.at_net = a.at_pq + (loss ? 2 * nc * p.nmus + nc + ncf : 0);
+    const int net = a.H > 0 ? p.n_scalar + (loss ? 5 : 1) * a.H : 0;
+    const bool inside = mtp_polys_in_moments(p.ncoef_poly, p.n_moms);
+    a.at_polys = inside ? 0 : a.at_net + net;
+    a.at_part = 0;
+    a.at_scratch = a.at_net + net + (!loss && !inside ? p.ncoef_poly : 0);
+    if (loss) {
+        // the group sums' place: the moments and their tangents, or 1024 entries behind the table
+        const int n1 = p.nmus * a.K, place = mtp_gred_in_moments(true, p.n_moms) ? 2 * p.n_moms : 1024;
+        a.grad_parts = std::max(1, std::min(nt / n1, place / (a.ntypes * n1)));
+    }
+    return (size_t)a.at_scratch + MTP_SCRATCH;
+}
+// moments | (tangents) | adjoints | (mixed adjoints), with the powers of the neighbours' unit vectors in their place before and sums of
+// wavefronts over those already dead | coefficients | neighbour table | ...
+template <typename T>
+size_t tiled_lds(MtpArgs<T>& a, bool loss, bool wide, int nc)
+{
+    const MtpPlanDevice& p = a.p;
+    const int vec = loss ? 2 : 1, n1 = p.nmus * a.K, ncf = a.ntypes * n1, stream = std::max(p.nstream[0], p.nstream[1]);
+    const int shared = wide && p.ntiles < 4 ? 4 / p.ntiles : 1;          // wavefronts to a tile (TileShare)
+    a.OU = 0; a.OG = 4; a.ODG = a.OG + p.nmus; a.OW = a.ODG + p.nmus; a.OF = a.OW + 4; a.ODF = a.OF + a.K;
+    a.OY = a.OZ = 0;
+    a.E = (loss ? a.ODF + a.K : a.OW) | 1;
+    a.PE = 3 * (p.kmax + 1) | 1;
+    a.at_Tg = p.n_moms;
+    a.at_A = vec * p.n_moms;
+    a.at_Bm = a.at_A + p.n_moms;
+    a.at_part = a.at_gred = a.at_A;
+    const int sums = loss ? 2 * nc * p.nshares[wide ? 1 : 0] : wide ? 3 * 4 * nc : 0;
+    const int dead = std::max(vec * p.n_moms, std::max((shared - 1) * vec * p.n_basic, sums));
+    const int region = std::max(vec * p.n_moms + dead, nc * a.PE);
+    if (loss) a.grad_parts = std::max(1, std::min((wide ? 256 : 64) / n1, (region - a.at_gred) / ncf));
+    a.at_cf = (region + 1) & ~1;
+    a.at_tab = a.at_cf + ncf;
+    a.at_Ab = a.at_tab + nc * a.E;
+    a.at_Bb = a.at_Ab + stream;
+    a.at_pq = loss ? a.at_Bb + stream : a.at_Ab;
+    a.at_net = a.at_pq + (loss ? 2 * nc * p.nmus + nc + ncf : 0);
+    const int net = a.H > 0 ? p.n_scalar + (loss ? 5 : 1) * a.H : 0;
+    const bool inside = stream <= p.n_moms;
+    a.at_polys = inside ? 0 : a.at_net + net;
+    a.at_scratch = a.at_net + net + (!loss && !inside ? stream : 0);
+    return (size_t)a.at_scratch + MTP_SCRATCH;
 }
 
 template <typename T>
@@ -2908,7 +3288,7 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.cE = nullptr; a.dFs = nullptr; a.dVs = nullptr; a.gpart = nullptr; a.ngrad = 0;
     a.force = nullptr; a.seg_cursor = nullptr; a.seg_g = nullptr; a.seg_spare = 0; a.seg_cap = 0; a.seg_mark = 0;
     a.partial = nullptr;
-    a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.keep_table = 0; a.leaves_late = 0;
+    a.e_sites = nullptr; a.desc = nullptr; a.energy_only = 0; a.cE_per_atom = 0; a.no_tangent = 0; a.leaves_late = 0; a.grad_parts = 1;
     a.nn_exact = 1;
     a.row_seed = nullptr; a.pair_out = nullptr;
     a.H = 0; a.w0 = nullptr; a.w1 = nullptr; a.q_shift = nullptr;
@@ -2918,8 +3298,6 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
     a.status = (int*)ws;
     return A2P_OK;
 }
-
-int g_keep_table = 1;      // (measurement switch: AI2POT_MTP_KEEP_TABLE=0)
 
 // 256 threads per atom or 64: a rule on the tables alone, so that a structure's results do not depend on the batch it is
 // in (the sums over neighbours are grouped by the threads).  Kernel times in us, 64 / 256 threads, fp64, energy / force /
@@ -2942,88 +3320,44 @@ template <typename T, bool LOSS, bool SEED = false>
 int launch_atoms(const MtpArgs<T>& args, hipStream_t stream)
 {
     MtpArgs<T> a = args;         // (what belongs to this launch alone is set here)
-    {
-        static const char* e = getenv("AI2POT_MTP_KEEP_TABLE");
-        if (e) g_keep_table = e[0] != '0';
-    }
-    const bool wide = wide_atoms(a.p.n_moms, LOSS, a.H > 0, sizeof(T) == 8);
+    const bool tiled = tiled_launch(a.p.ntiles, LOSS, wide_atoms(a.p.n_moms, LOSS, a.H > 0, sizeof(T) == 8));
+    const bool wide = wide_launch(a.p.n_moms, a.p.ntiles, LOSS, a.H > 0, sizeof(T) == 8);
     if (a.H == 0 && !a.row_seed && !a.e_sites && !a.desc && !a.energy_only) {
         a.leaves_late = 1;
         for (int i = 0; i < 2; i++) { a.p.fwd[i] = a.p.fwd_core[i]; a.p.rev[i] = a.p.rev_leaf[i]; }
     }
-    const int groups = a.z_powers ? 0 : (wide ? 256 : 64) / std::max(a.p.npoly, 1);      // of a thread per polynomial
-    const int kept_adjoints = std::max(a.p.n_moms, groups * a.p.ncoef_poly);
-    auto lds_for = [&](int nc, size_t* main, int keep = 0) {
-        *main = (lds_bytes<T>(a.p, a.E, LOSS, a.ntypes, a.K, a.H, nc, wide ? 256 : 64, keep) + 15) / 16 * 16;
+    auto lds_for = [&](int nc) {
+        const size_t n = (tiled ? tiled_lds<T>(a, LOSS, wide, nc) : general_lds<T>(a, LOSS, nc)) * sizeof(T);
+        if (tiled) return n;
         // the packed basic-moment table and the polynomials, with the monomial rows or the run of every mu
-        return *main + ((size_t)a.p.n_basic + a.p.npoly + 1 + (LOSS ? a.p.nmus : a.p.nrows)) * sizeof(unsigned);
+        a.lds_basic_off = (int)((n + 15) / 16 * 16);
+        return a.lds_basic_off + ((size_t)a.p.n_basic + a.p.npoly + 1 + (LOSS ? a.p.nmus : a.p.nrows)) * sizeof(unsigned);
     };
-    size_t lds_main = 0;
-    int nc_cap = MTP_NC;
-    size_t lds = lds_for(nc_cap, &lds_main);
-    // Rows of the neighbour table (energy / force / virial kernel; the loss kernels keep MTP_NC): the kernel waits on
-    // dependent LDS reads and barriers, so workgroups per CU count first (level 16: 12 -> 16 workgroups, 0.136 -> 0.122 ms
-    // although rows of more than 20 neighbours then take two chunks), and among the tables that allow as many
-    // workgroups as the registers do (four or five waves per SIMD), or as the shortest table does, the longest is taken
-    // (level 20: a row of 35 neighbours in one chunk instead of two, 0.45 -> 0.41 ms).
-    if (!LOSS) {
+    // Rows of the neighbour table: the kernel waits on dependent LDS reads and barriers, so workgroups per CU count first, and among the
+    // tables that allow as many workgroups as the registers do, or as the shortest table does (loss gradient: one of MTP_NC rows), the
+    // longest is taken.
+    size_t lds = 0;
+    {
         // LDS is handed out in pieces of 1280 bytes on this chip
         auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
-        size_t m = 0;
-        const size_t by_registers = wide ? 5 : 16;
-        const size_t want = std::min(by_registers, per_cu(lds_for(MTP_NC_MIN, &m)));
-        for (int nc : {MTP_NC_MAX, 40, 32, 24, 20, MTP_NC_MIN}) {
-            const size_t l = lds_for(nc, &m);
-            if (per_cu(l) >= want || nc == MTP_NC_MIN) { nc_cap = nc; lds = l; lds_main = m; break; }
+        const size_t by_registers = (wide ? 1 : 4) * (LOSS ? 6 : wide ? 5 : 4);
+        const size_t want = std::min(by_registers, std::max<size_t>(1, per_cu(lds_for(LOSS ? MTP_NC : MTP_NC_MIN))));
+        for (int nc : {MTP_NC_MAX, 40, MTP_NC, 24, 20, MTP_NC_MIN}) {
+            lds = lds_for(nc);
+            a.nc_cap = nc;
+            if (per_cu(lds) >= want) break;
         }
-        // The table kept through the sweeps (adjoints behind it) saves a row of one chunk its second table build: taken
-        // when a table of at least 32 rows fits that way at the same number of workgroups per CU (level 20: 0.387 ->
-        // 0.368 ms, level 10: 0.026 -> 0.023 ms; at level 16 the sixteen workgroups per CU count for more).  Not in the
-        // modes that use the table's place as scratch between the sweeps (site energies, descriptors).
-        int keep = 0;
-        if (!a.e_sites && !a.desc && !a.energy_only && g_keep_table)
-            for (int nc : {MTP_NC_MAX, 40, 32}) {
-                const size_t l = lds_for(nc, &m, kept_adjoints);
-                if (per_cu(l) >= want) { keep = 1; nc_cap = nc; lds = l; lds_main = m; break; }
-            }
-        a.keep_table = keep;
     }
-    {
-        const MtpPlanDevice& p = a.p;
-        const int nt = wide ? 256 : 64;
-        const int keep = !LOSS && a.keep_table != 0 ? kept_adjoints : 0;
-        a.lds_basic_off = (int)lds_main;
-        a.nc_cap = nc_cap;
-        // moments | (loss mode: their tangents) | coefficients | region of the neighbour table | ...
-        a.at_Tg = p.n_moms;
-        a.at_cf = a.at_Tg + (LOSS ? p.n_moms : 0);
-        a.at_tab = a.at_cf + a.ntypes * p.nmus * a.K;
-        // the adjoints share the table's region, or lie behind the table
-        a.at_A = a.at_tab + (keep ? mtp_table_entries(nc_cap, a.E, LOSS, p.n_moms, nt) : MTP_AT_ADJOINTS);
-        a.at_Bm = a.at_A + p.n_moms;
-        // Partial sums of the thread groups, needed only in the last pass over the neighbours, when the moments (and, in
-        // loss mode, their tangents) are dead: a long enough moment vector lends them its place.  Energy / force / virial
-        // kernel: they are written over the table once it has been read.
-        a.at_gred = !LOSS ? a.at_tab : mtp_gred_in_moments(LOSS, p.n_moms) ? 0 : a.at_tab + nc_cap * a.E;
-        a.at_Ab = a.at_tab + mtp_table_region(nc_cap, a.E, LOSS, p.n_moms, nt, keep);
-        a.at_Bb = a.at_Ab + p.ncoef_poly;
-        a.at_pq = LOSS ? a.at_Bb + p.ncoef_poly : a.at_Ab;
-        a.at_net = a.at_pq + (LOSS ? 2 * nc_cap * p.nmus + nc_cap + a.ntypes * p.nmus * a.K : 0);
-        a.at_polys = mtp_polys_in_moments(p.ncoef_poly, p.n_moms) ? 0 : a.at_pq + (a.H > 0 ? p.n_scalar + a.H : 0);
-    }
-    if (LOSS) {
-        // the group sums' place: the moments and their tangents, or 1024 entries behind the table
-        const int n1 = a.p.nmus * a.K, place = mtp_gred_in_moments(true, a.p.n_moms) ? 2 * a.p.n_moms : 1024;
-        a.grad_parts = std::max(1, std::min((wide ? 256 : 64) / n1, place / (a.ntypes * n1)));
-    }
-    // as many groups of a thread per polynomial as the workgroup has, and as the place of their sums holds
-    const int room = !LOSS && a.keep_table ? kept_adjoints : mtp_table_entries(nc_cap, a.E, LOSS, a.p.n_moms, wide ? 256 : 64);
-    a.mom_groups = std::min(groups, room / std::max((LOSS ? 2 : 1) * a.p.ncoef_poly, 1));
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
-    auto kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
+    auto kern = mtp_atom_kernel<T, LOSS, 256, SEED, false, false>;
     if constexpr (!SEED)
-        if (a.H > 0) kern = wide ? mtp_atom_kernel<T, LOSS, 256, false, true> : mtp_atom_kernel<T, LOSS, 64, false, true>;
+        if (a.H > 0) kern = mtp_atom_kernel<T, LOSS, 256, false, true, false>;
+    if (tiled) {
+        kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
+        if constexpr (!SEED)
+            if (a.H > 0) kern = wide ? mtp_atom_kernel<T, LOSS, 256, false, true> : mtp_atom_kernel<T, LOSS, 64, false, true>;
+    }
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
                                           (int)lds));
@@ -3072,7 +3406,6 @@ int mtp_efv(void* handle, int K, double scaling, const T* coeffs, const T* lin, 
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
     a.e_sites = e_sites;
-    table_layout(a, false);
     void* ws = nullptr;
     rc = ws_get(WS_PARTIAL, (size_t)B * P * 10 * sizeof(double), &ws);
     if (rc) return rc;
@@ -3148,7 +3481,6 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
-    table_layout(a, true);
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
@@ -3213,7 +3545,6 @@ int nnmtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft,
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
-    table_layout(a, true);
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = nrow;
     a.nn_exact = exact ? 1 : 0;
     rc = launch_atoms<T, true>(a, stream);
@@ -3244,7 +3575,6 @@ int mtp_esites(void* handle, int K, double scaling, const T* coeffs, const T* li
     rc = set_net(a, net);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
-    table_layout(a, false);
     a.e_sites = e_sites; a.desc = desc; a.energy_only = 1;
     return launch_atoms<T, false>(a, stream);
 }
@@ -3279,7 +3609,6 @@ int mtp_esites_bwd(void* handle, int K, double scaling, const T* coeffs, const T
     T* gpart = (T*)ws + nzero;
     rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
     if (rc) return rc;
-    table_layout(a, true);
     a.cE = gout; a.cE_per_atom = 1; a.no_tangent = 1; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
@@ -3317,7 +3646,6 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         rc = fill_zero(drcs, (size_t)B * P * U * 3 * sizeof(T), stream);
         if (rc) return rc;
         MtpArgs<T> e = a;
-        table_layout(e, false);
         e.pair_out = drcs;
         rc = launch_atoms<T, false, true>(e, stream);
         if (rc) return rc;
@@ -3335,7 +3663,6 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
         if (rc) return rc;
         MtpArgs<T> g = a;
-        table_layout(g, true);
         g.dFs = dFs; g.dVs = dVs; g.gpart = gpart; g.ngrad = ncoef; g.no_tangent = 1;
         rc = launch_atoms<T, true>(g, stream);
         if (rc) return rc;
@@ -3516,7 +3843,7 @@ int mtp_lin_components(void* handle, int K, double scaling, const T* coeffs, int
                        rmin, B, P, U, 0, binum, bilist, bnumneigh, bfirstneigh, brcs, btypes, false);
         if (rc) return rc;
         A2P_REQUIRE(q_scaler, A2P_ERR_INVALID, "mtp components: null q_scaler");
-        table_layout(a, false, true);     // (the kernel forms derivatives of each basic moment)
+        table_layout(a, false);     // (the kernel forms derivatives of each basic moment)
         return mtp_lin_components_nodes<T>(plan, a, S, n, ecomp, fcomp, vcomp, stream);
     }
     rc = fill_zero(ecomp, (size_t)B * n * sizeof(T), stream);
@@ -3610,7 +3937,6 @@ int nnmtp_esites_bwd(void* handle, int K, const MtpNet<T>& net, const T* coeffs,
     T* gpart = (T*)ws + nzero;
     rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
     if (rc) return rc;
-    table_layout(a, true);
     a.cE = gout; a.cE_per_atom = 1; a.no_tangent = 1; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = nrow;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;

@@ -19,6 +19,7 @@
 namespace a2p {
 
 constexpr int MTP_SLOT_CAP = 16;
+constexpr int MTP_NEST_MAX = 9, MTP_UNITS_MAX = 64, MTP_NO_MOMENT = 0xffff;
 // Terms of a slot to a step of the sweeps, and the words of a step: the terms by pairs, 64 lanes each.
 constexpr int MTP_DEPTH_STEP = 4, MTP_STEP_WORDS = MTP_DEPTH_STEP / 2 * 64;
 // Mark of a control word: a step of a group of leaves (rev_leaf).
@@ -58,6 +59,25 @@ struct MtpPlanDevice {
     // their lists stand with the first sources of the reverse one (control words marked, 8 m0 | 8 m1 << 16).
     MtpStream fwd_core[2], rev_leaf[2];
     const int* mapping_leaf;   // [n_scalar]   mapping | leaf << 16
+    // The passes over the neighbours (mtp.hip: tile_products, nested).  ntiles is 0 where the tables do not fit them: a basic moment
+    // that occurs twice, a degree beyond MTP_NEST_MAX, more than MTP_UNITS_MAX units.
+    // Sums of the basic moments as matrix products: rows (a, b) and columns (mu, c), those with the most moments first, in tiles of
+    // 16 x 16, of which only those with a moment are formed.  Lane l supplies row l % 16 and column l % 16 of a tile and receives row
+    // 4 v + l / 16 of its column in place v.
+    int ntiles;
+    const unsigned* tile_ops;              // [ntiles][64] a | b << 5 | mu << 10 | c << 13 of the lane's row and column
+    const uint2* tile_place;               // [ntiles][64] basic moments of the lane's four places, 16 bits each (0xffff: none)
+    // Sums over the basic moments at one neighbour: for every (mu, c), c downwards, a unit, the polynomial of degree M = deg(mu) - c in x
+    // and y whose coefficients are the adjoints, with zeros for moments that the tables leave out.  stream[0]: b downwards, a downwards.
+    // stream[1], for two lanes to a neighbour: the moments with a >= b and those with a < b, each in powers of xy downwards and
+    // then of x, or of y, downwards (the second half at half_at, with zeros for a = b).
+    int nstream[2], half_at;
+    const unsigned short* stream_src[2];   // [nstream] basic moment behind a coefficient (0xffff: none)
+    // Units dealt to the wavefronts, one or four, in runs of about equal cost: [wavefronts] {units, first coefficient in stream[0] | in
+    // stream[1] << 16}, then [wavefronts][64] M | mu << 4 | last of its mu in the run << 7 | c << 8 | share << 13, shares of the mus numbered.
+    const int* units[2];
+    int nshares[2];                        // shares in all
+    unsigned long long mu_shares[2];       // shares of each mu, eight bits each
     // Polynomials of the passes that own a neighbour per lane.  The basic moments (mu, a, b, c) with the same row (a, b) and
     // the same mu are the coefficients of a polynomial in z; its coefficients lie together, highest power first, up to
     // the highest power in the tables (powers the tables leave out: zero).
@@ -69,7 +89,6 @@ struct MtpPlanDevice {
     const int* poly_pos;       // [n_basic] coefficient of each basic moment
     const unsigned* polys_len; // [npoly] the same, longest first: mu | a << 3 | b << 8 | length << 13 | first coefficient << 18
                                // (null: a coefficient does not fit its field)
-    int poly_top;              // length of the longest
     int poly_unique;           // no two basic moments share a coefficient (the usual case: a plain scatter fills them)
     const int* poly_src;       // [ncoef_poly] basic moment behind the coefficient, -1 none, -2 several (poly_off / items)
     const int* poly_off;       // [ncoef_poly+1]
