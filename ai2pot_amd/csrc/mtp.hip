@@ -349,7 +349,6 @@ __device__ __forceinline__ void tile_products(Args& a, const T* tab, const T* pw
         if (ts.first + u * (NT / 64) >= ntiles || (u > 0 && ts.nsplit > 1)) break;
         const int ea = word[u] & 31, eb = word[u] >> 5 & 31, mu = word[u] >> 10 & 7, ec = word[u] >> 13;
         const T *const px = pw + ea, *const py = pw + n1 + eb, *const pz = pw + 2 * n1 + ec, *const pg = tab + a.OG + mu;
-#pragma unroll 2
         for (int k = k0; k < k1; k++) {
             const int j = k * 4 + kq;
             const bool on = j < nc;
@@ -872,6 +871,12 @@ __device__ __forceinline__ void loss_walk(const T* __restrict__ t, const T* __re
     Q *= wu;
 }
 
+// Wavefronts per SIMD that the registers are kept to.  Energies and forces with 256 threads: five (four: level 20, 8192 atoms 174 -> 195
+// us; six spill: 266), with 64: four (five: level 16, 64 structures of 128 atoms 67 -> 90).  Loss gradient in fp64: five, which takes 95
+// registers without a spill (six, as long as its sums went by polynomials in z: 136 registers spilled, level 16 165 -> 133; four: 149), in
+// fp32 six (without a limit some went to the accumulation registers and back: level 20, 32 x 128 atoms 123 -> 115).
+constexpr int waves_of(bool fp64, bool loss, int nt) { return loss ? (fp64 ? 5 : 6) : nt == 256 ? 5 : 4; }
+
 // The workgroup's LDS (launch_atoms): moments | (loss mode: their tangents) | adjoints | (mixed adjoints), in whose place the powers of the
 // neighbours' unit vectors stand before | coefficients of the centre species | neighbour table | ...
 // General tables: moments | tangents | coefficients | neighbour table, in whose place the adjoints come after it | ...
@@ -927,14 +932,15 @@ struct AtomLds {
     [[maybe_unused]] const T* const rcs = a.brcs + row * a.U * 3;                                                          \
     [[maybe_unused]] const int* const types = a.btypes + (size_t)b * NF
 
-// NT threads per centre atom: 64 or 256 (wide_atoms).  Five workgroups of 256 threads fit the LDS of a CU at level 20 and
-// the registers are kept to match (four: 321 us instead of 303 at 8192 atoms; six spill: 361).
+// NT threads per centre atom: 64 or 256 (wide_atoms).
 // SEED: the instance of the energy / force / virial kernel that can start its adjoint sweep from per-row weights
 // (row_seed, pair_out); the loss-gradient kernel tests the pointer at run time.  NET: the instances with a network read-out.
-// TILED: the passes over the neighbours by matrix products and nested polynomials (mtp_plan.h: ntiles), where the tables fit them; the
-// others go by basic moments and by polynomials in z, with 256 threads.
-template <typename T, bool LOSS, int NT, bool SEED = false, bool NET = false, bool TILED = true>
-__global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) == 8 ? 6 : 1)) mtp_atom_kernel(const MtpArgs<T>)
+// TILES: the passes over the neighbours by matrix products, as many tiles to a wavefront, and nested polynomials (mtp_plan.h: ntiles),
+// where the tables fit them; the others (0) go by basic moments and by polynomials in z, with 256 threads.  (Two tiles to a wavefront where
+// one does, 32 registers of sums without use: the loss gradient of a network at level 10, 32 x 100 atoms 63 -> 62 us, fp32, level 16, 64 x
+// 128 atoms 116 -> 104, fp32 energies and forces of level 8 29.5 -> 25.5.)
+template <typename T, bool LOSS, int NT, bool SEED = false, bool NET = false, int TILES = 1>
+__global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_atom_kernel(const MtpArgs<T>)
 {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int lane = threadIdx.x;     // thread in the workgroup
@@ -942,8 +948,9 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     int center, nn, ti;
     int nchunks, csize;               // the row is cut into equal chunks of at most nc_cap neighbours
     TableAhead<T> ahead;              // (energies and forces; the loss gradient's registers do not hold it: 166 -> 175 us)
-    constexpr int TILES = tiles_of(LOSS, NT);
-    unsigned tword[TILES];        // the lane's rows and columns of the wavefront's tiles
+    constexpr bool TILED = TILES > 0;
+    constexpr int NTILE = TILED ? TILES : 1;
+    unsigned tword[NTILE];        // the lane's rows and columns of the wavefront's tiles
     const int wave = __builtin_amdgcn_readfirstlane(lane >> 6), l64 = lane & 63;
     {
         MTP_PHASE;
@@ -964,7 +971,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         if constexpr (TILED) {
             const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
 #pragma unroll
-            for (int u = 0; u < TILES; u++) tword[u] = tile_word<T>(p.tile_ops, min(ts.first + u * (NT / 64), p.ntiles - 1), l64);
+            for (int u = 0; u < NTILE; u++) tword[u] = tile_word<T>(p.tile_ops, min(ts.first + u * (NT / 64), p.ntiles - 1), l64);
         } else {
             basics.load(p.basic, n_basic, lane);
             words.load(wsrc, nwords, lane);
@@ -1010,7 +1017,7 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
     }
 
     // ---- basic moments (and their tangents) --------------------------------------------------
-    [[maybe_unused]] typename wave::Acc<T>::type msum[TILES], dsum[TILES];
+    [[maybe_unused]] typename wave::Acc<T>::type msum[NTILE], dsum[NTILE];
     auto table = [&](int c0, int nc) __attribute__((always_inline)) {
         MTP_PHASE;
         int nj; bool valid; T d[3];
@@ -1028,14 +1035,14 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         auto products = [&](int nc) __attribute__((always_inline)) {
             MTP_PHASE;
             const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
-            if (LOSS && !no_tan) tile_products<T, LOSS, NT, TILES>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
-            else tile_products<T, false, NT, TILES>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
+            if (LOSS && !no_tan) tile_products<T, LOSS, NT, NTILE>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
+            else tile_products<T, false, NT, NTILE>(a, tab, pw, lane, nc, ts, tword, msum, dsum);
             __syncthreads();
         };
         // (the first chunk, of most rows the only one, by itself: sums held over the table's phase do not fit the registers)
         if (nn > 0) table(0, min(csize, nn));
 #pragma unroll
-        for (int u = 0; u < TILES; u++) msum[u] = dsum[u] = {0, 0, 0, 0};
+        for (int u = 0; u < NTILE; u++) msum[u] = dsum[u] = {0, 0, 0, 0};
         if (nn > 0) products(min(csize, nn));
 #pragma unroll 1
         for (int c0 = csize; c0 < nn; c0 += csize) {
@@ -1077,8 +1084,8 @@ __global__ void __launch_bounds__(NT, (!LOSS ? (NT == 256 ? 5 : 4) : sizeof(T) =
         MTP_PHASE;
         const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
         const int per = LOSS ? 2 * n_basic : n_basic;
-        tile_store<T, NT, TILES>(p, ts.split == 0 ? M : L.part + (ts.split - 1) * per, lane, ts, msum);
-        if (LOSS) tile_store<T, NT, TILES>(p, ts.split == 0 ? Tg : L.part + (ts.split - 1) * per + n_basic, lane, ts, dsum);
+        tile_store<T, NT, NTILE>(p, ts.split == 0 ? M : L.part + (ts.split - 1) * per, lane, ts, msum);
+        if (LOSS) tile_store<T, NT, NTILE>(p, ts.split == 0 ? Tg : L.part + (ts.split - 1) * per + n_basic, lane, ts, dsum);
         for (int i = n_basic + lane; i < n_moms; i += NT) {
             M[i] = (T)0;
             if (LOSS) Tg[i] = (T)0;
@@ -3311,6 +3318,8 @@ int fill_args(MtpArgs<T>& a, MtpPlan* plan, int K, double scaling, const T* coef
 // With a network the loss gradient has a weight per neuron and scalar moment besides (64 x 125 atoms; 2 x 60; 30 neurons):
 //   level 8  160 / 160, 28 / 24 (10 neurons: 112 / 139, 23 / 21)   level 10  185 / 168, 33 / 24   level 12  240 / 184, 38 / 25
 // fp32, level 12: 84 / 126, 31 / 30; 14: 108 / 138, 38 / 33; 18: 275 / 212, 77 / 41.
+// Those were the kernels that went by polynomials in z; the loss gradients by tiles and nested polynomials (64 x 128 atoms; 4 x 60):
+//   level 10  86 / 103, 28 / 15   level 12  93 / 105, 27 / 15   level 12 in fp32  60 / 85
 bool wide_atoms(int n_moms, bool loss, bool network, bool fp64)
 {
     return n_moms >= (loss ? (network ? 40 : fp64 ? 80 : 150) : 600);
@@ -3340,7 +3349,7 @@ int launch_atoms(const MtpArgs<T>& args, hipStream_t stream)
     {
         // LDS is handed out in pieces of 1280 bytes on this chip
         auto per_cu = [](size_t l) { return (size_t)(160 * 1024) / ((l + 1279) / 1280 * 1280); };
-        const size_t by_registers = (wide ? 1 : 4) * (LOSS ? 6 : wide ? 5 : 4);
+        const size_t by_registers = (wide ? 1 : 4) * waves_of(sizeof(T) == 8, LOSS, wide ? 256 : 64);
         const size_t want = std::min(by_registers, std::max<size_t>(1, per_cu(lds_for(LOSS ? MTP_NC : MTP_NC_MIN))));
         for (int nc : {MTP_NC_MAX, 40, MTP_NC, 24, 20, MTP_NC_MIN}) {
             lds = lds_for(nc);
@@ -3350,13 +3359,22 @@ int launch_atoms(const MtpArgs<T>& args, hipStream_t stream)
     }
     A2P_REQUIRE(lds <= 160 * 1024, A2P_ERR_INVALID,
                 "mtp: %d moments need %zu bytes of LDS per atom; this level is too large", a.p.n_moms, lds);
-    auto kern = mtp_atom_kernel<T, LOSS, 256, SEED, false, false>;
+    auto kern = mtp_atom_kernel<T, LOSS, 256, SEED, false, 0>;
     if constexpr (!SEED)
-        if (a.H > 0) kern = mtp_atom_kernel<T, LOSS, 256, false, true, false>;
+        if (a.H > 0) kern = mtp_atom_kernel<T, LOSS, 256, false, true, 0>;
     if (tiled) {
-        kern = wide ? mtp_atom_kernel<T, LOSS, 256, SEED> : mtp_atom_kernel<T, LOSS, 64, SEED>;
+        // (as many tiles to a wavefront as the tables take)
+        const bool two = a.p.ntiles > (wide ? 4 : 1);
+        auto pick = [&](auto net) {
+            constexpr bool N = decltype(net)::value;
+            auto narrow = mtp_atom_kernel<T, LOSS, 64, SEED, N, 1>;
+            if constexpr (!LOSS)
+                if (two) narrow = mtp_atom_kernel<T, LOSS, 64, SEED, N, 2>;
+            return !wide ? narrow : two ? mtp_atom_kernel<T, LOSS, 256, SEED, N, 2> : mtp_atom_kernel<T, LOSS, 256, SEED, N, 1>;
+        };
+        kern = pick(std::false_type());
         if constexpr (!SEED)
-            if (a.H > 0) kern = wide ? mtp_atom_kernel<T, LOSS, 256, false, true> : mtp_atom_kernel<T, LOSS, 64, false, true>;
+            if (a.H > 0) kern = pick(std::true_type());
     }
     if (lds > 48 * 1024)
         A2P_HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,

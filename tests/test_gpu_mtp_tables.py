@@ -4,7 +4,7 @@ few neighbours (pairs of neighbours that have no second one)."""
 import numpy as np
 import pytest
 
-from ai2pot_amd import synth
+from ai2pot_amd import mtp_param, synth
 from test_gpu_mtp import close, gpu_efv, gpu_loss, loss_inputs, model_to_device, structure
 from conftest import to_device
 
@@ -39,6 +39,30 @@ def test_irregular_basic_moments(oracle, basic):
     B, P = nb["bilist"].shape
     labels = dict(energy=synth.rng_normal(1, B, -4 * 40, 3), force=synth.rng_normal(2, B * P * 3).reshape(B, P, 3),
                   virial=synth.rng_normal(3, B * 9, 0, 0.5).reshape(B, 9))
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w), oracle.mtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dlinear", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
+ROWS = [0, 1, 2, 3, 4, 5, 15, 16, 17, 23, 24, 25, 31, 32, 33, 40, 41, 47, 48, 49, 63, 64, 65, 80]
+
+
+@pytest.mark.parametrize("level", [8, 12, 16, 20, 22])            # 1, 1, 2, 4 and 5 tiles: one or two to a wavefront, or shared by four and two
+def test_passes_by_row_length(oracle, level):
+    """The sums of the basic moments and the pair derivatives for rows that fill a matrix product, half a wavefront, a wavefront and
+    the neighbour table, one neighbour more and one less.  Energies, forces, virials and loss gradients against the oracle: fp64, 1e-10."""
+    nt, rc = 2, 7.0
+    nb = dict(synth.pack_batch([structure(oracle, len(ROWS), (7.0, 7.2, 7.4), nt, 57, rc, umax=140)]))
+    assert nb["bnumneigh"].min() >= max(ROWS)
+    nb["bnumneigh"] = np.array([ROWS], np.int32)
+    m = synth.mtp_model(mtp_param.mtp_param(level), nt, 8, rc, 1.5, 3300 + level, lo=-0.05, hi=0.05)
+    m["q_scaler"] = np.linspace(0.8, 1.3, m["q_scaler"].size)
+    for got, ref in zip(gpu_efv(m, nb), oracle.mtp_efv(m, nb)):
+        assert close(got, ref)
+    n = len(ROWS)
+    labels = dict(energy=synth.rng_normal(1, 1, -4 * n, 3), force=synth.rng_normal(2, n * 3).reshape(1, n, 3),
+                  virial=synth.rng_normal(3, 9, 0, 0.5).reshape(1, 9))
     w = (1.0, 0.7, 0.3)
     got, ref = gpu_loss(m, nb, labels, w), oracle.mtp_loss_step(m, nb, w, labels)
     for k in ("bloss", "dcoeffs", "dlinear", "dbias"):
