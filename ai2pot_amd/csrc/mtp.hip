@@ -369,14 +369,14 @@ __device__ __forceinline__ void tile_products(Args& a, const T* tab, const T* pw
 }
 // A wavefront's sums to their moments.
 template <typename T, int NT, int TILES, typename Plan>
-__device__ __forceinline__ void tile_store(Plan& p, T* dst, int tid, const TileShare& ts, const typename wave::Acc<T>::type (&m)[TILES])
+__device__ __forceinline__ void tile_store(Plan& p, T* dst, const TileShare& ts, const uint2 (&place)[TILES], const typename wave::Acc<T>::type (&m)[TILES])
 {
     if (ts.split >= ts.nsplit) return;
 #pragma unroll
     for (int u = 0; u < TILES; u++) {
         const int tile = ts.first + u * (NT / 64);
         if (tile >= p.ntiles || (u > 0 && ts.nsplit > 1)) break;
-        const uint2 at = p.tile_place[tile * 64 + (tid & 63)];
+        const uint2 at = place[u];
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const unsigned i = (v < 2 ? at.x : at.y) >> (v & 1 ? 16 : 0) & 0xffffu;
@@ -492,17 +492,30 @@ __device__ __forceinline__ void nested(const T* coef, const T* coefb, int prog, 
         }
     }
 }
-// The coefficients of the units out of the adjoints of the basic moments.
-template <typename T, int NT, typename Plan>
-__device__ __forceinline__ void unit_coefficients(Plan& p, int G, T* dst, const T* A, int tid)
-{
-    const int n = p.nstream[G - 1];
-    const unsigned short* const src = p.stream_src[G - 1];
-    for (int i = tid; i < n; i += NT) {
-        const int m = src[i];
-        dst[i] = m == MTP_NO_MOMENT ? (T)0 : A[m];
+// The moments behind a thread's first coefficients of the units, on their way during the reverse sweep (with the places of the tiles'
+// sums during these: level 20, 8192 atoms 176 -> 174 us, level 12, 64 x 128 atoms 43.2 -> 40.9), and the coefficients out of the
+// adjoints of the basic moments: set(place, moment) for each.
+template <int NT>
+struct UnitSources {
+    static constexpr int U = NT == 64 ? 4 : 2;
+    int m[U];
+    template <typename Plan>
+    __device__ __forceinline__ void load(Plan& p, int G, int tid)
+    {
+        const int n = p.nstream[G - 1];
+#pragma unroll
+        for (int u = 0; u < U; u++) m[u] = p.stream_src[G - 1][min(tid + u * NT, n - 1)];
     }
-}
+    template <typename Plan, typename Set>
+    __device__ __forceinline__ void each(Plan& p, int G, int tid, Set&& set) const
+    {
+        const int n = p.nstream[G - 1];
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (tid + u * NT < n) set(tid + u * NT, m[u]);
+        for (int i = tid + U * NT; i < n; i += NT) set(i, (int)p.stream_src[G - 1][i]);
+    }
+};
 
 template <typename T>
 __device__ __forceinline__ T group_sum(const T* src, int ng, int ncoef)
@@ -598,7 +611,8 @@ __device__ __forceinline__ T plan_entry(const T* base, unsigned off)
 // control words of 64 steps lie in a vector register, and an odd step is walked ahead of the loop.
 // Kernel of energies and forces, level 20, 8192 atoms, 236 -> 222 us (216 atoms: 28.3 -> 26.9), of level 16, 64 structures of 128 atoms,
 // 90.3 -> 87.7, the loss gradient there 161 -> 159.5; with two products to a multiplicity (step_terms), 14 instead of 24 vector
-// instructions for the four of a step.  (The words of a step in an order that keeps the LDS free of bank conflicts, 1.2 lanes to a
+// instructions for the four of a step; with the words' address formed without vector instructions and the second multiplicity as it was
+// loaded, level 20, 8192 atoms 174 -> 169.5, the components of level 16 134 -> 131.  (The words of a step in an order that keeps the LDS free of bank conflicts, 1.2 lanes to a
 // bank instead of 2.1: no change.)
 template <typename Stream, typename Terms, typename Done>
 __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& done)
@@ -609,7 +623,7 @@ __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& d
     const A2P_CONSTANT int* const head = uniform_array((const int*)g.head) + wave * 4;
     const int first = head[0], n = head[1];
     const A2P_CONSTANT char* at = (const A2P_CONSTANT char*)(const A2P_CONSTANT int4*)uniform_array(g.words + (size_t)first * MTP_STEP_WORDS);
-    const unsigned at_lane = (unsigned)lane * 16u;
+    unsigned at_lane = (unsigned)lane * 16u;
     auto load = [&](Step& s, int k) __attribute__((always_inline)) {       // (two steps behind the last)
         s.w[0] = *(const A2P_CONSTANT int4_t*)(at + k * MTP_STEP_WORDS * 16 + at_lane);
         s.w[1] = *(const A2P_CONSTANT int4_t*)(at + k * MTP_STEP_WORDS * 16 + 64 * 16 + at_lane);
@@ -642,9 +656,11 @@ __device__ __forceinline__ void walk(Stream& g, int tid, Terms&& terms, Done&& d
             // (w[1].z, of no use, keeps its register: given to another value, this one would wait for the load)
             asm volatile("" : "+v"(slot) : "v"(s.w[1].z) : "memory");
             if (!ahead) return;
-            load(s, 2);
+            // (a lane's address takes no vector instruction where it is formed anew each step, of the wavefront's and 32 bits of
+            // the lane's, with an offset of less than 4096 bytes)
             at += MTP_STEP_WORDS * 16;
-            asm volatile("" : "+s"(at));               // (a lane's address formed anew each step takes no vector instruction)
+            asm volatile("" : "+s"(at), "+v"(at_lane));
+            load(s, 1);
         });
         if (__builtin_expect(c & 1, 0)) {
             done((int)(short)slot, slot >> 16, (c >> 1) & 7, leaf);
@@ -682,7 +698,7 @@ __device__ __forceinline__ void step_terms(const Words (&w)[2], const T* a, cons
     }
 #pragma unroll
     for (int u = 0; u < C / 2; u++) {
-        mult[u] = (T)__hiloint2double(w[u].w, 0);
+        mult[u] = (T)__hiloint2double(w[u].w, u == 0 ? 0 : w[u].z);
         asm volatile("" : "+v"(mult[u]));
     }
     next();
@@ -1018,6 +1034,7 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
 
     // ---- basic moments (and their tangents) --------------------------------------------------
     [[maybe_unused]] typename wave::Acc<T>::type msum[NTILE], dsum[NTILE];
+    [[maybe_unused]] uint2 tplace[NTILE];
     auto table = [&](int c0, int nc) __attribute__((always_inline)) {
         MTP_PHASE;
         int nj; bool valid; T d[3];
@@ -1032,6 +1049,12 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
         ahead.species(types, NF, center);
     };
     if constexpr (TILED) {
+        {
+            MTP_PHASE;
+            const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
+#pragma unroll
+            for (int u = 0; u < NTILE; u++) tplace[u] = p.tile_place[min(ts.first + u * (NT / 64), p.ntiles - 1) * 64 + l64];
+        }
         auto products = [&](int nc) __attribute__((always_inline)) {
             MTP_PHASE;
             const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
@@ -1084,8 +1107,8 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
         MTP_PHASE;
         const TileShare ts = TileShare::of<NT>(p.ntiles, wave);
         const int per = LOSS ? 2 * n_basic : n_basic;
-        tile_store<T, NT, NTILE>(p, ts.split == 0 ? M : L.part + (ts.split - 1) * per, lane, ts, msum);
-        if (LOSS) tile_store<T, NT, NTILE>(p, ts.split == 0 ? Tg : L.part + (ts.split - 1) * per + n_basic, lane, ts, dsum);
+        tile_store<T, NT, NTILE>(p, ts.split == 0 ? M : L.part + (ts.split - 1) * per, ts, tplace, msum);
+        if (LOSS) tile_store<T, NT, NTILE>(p, ts.split == 0 ? Tg : L.part + (ts.split - 1) * per + n_basic, ts, tplace, dsum);
         for (int i = n_basic + lane; i < n_moms; i += NT) {
             M[i] = (T)0;
             if (LOSS) Tg[i] = (T)0;
@@ -1269,6 +1292,14 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
         }
         __syncthreads();
     }
+    const int halves = csize <= 32 ? 2 : 1;       // lanes to a neighbour in the last passes
+    [[maybe_unused]] int prog = 0;
+    [[maybe_unused]] UnitSources<NT> sources;
+    if constexpr (TILED) {
+        MTP_PHASE;
+        sources.load(p, halves, lane);
+        prog = p.units[NT / 256][2 * (NT / 64) + lane];
+    }
     {
         MTP_PHASE;
         // the leaves' moments: their part of the energy, or, for the loss gradient, the moments (and tangents) themselves;
@@ -1289,13 +1320,10 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
         // The adjoints of the basic moments as polynomial coefficients; the moments are dead.  Nested polynomials: two lanes to a neighbour
         // where a chunk has no more than 32, one otherwise; the wavefronts share the units.  General tables: within a chunk of nc
         // neighbours thread = group h * nc + neighbour j, and the groups (as many as fit, at most one per monomial row) share the rows.
-        const int halves = csize <= 32 ? 2 : 1;
-        [[maybe_unused]] int prog = 0;
         {
             MTP_PHASE;
             if constexpr (TILED) {
-                unit_coefficients<T, NT>(p, halves, L.polys, A, lane);
-                prog = p.units[NT / 256][2 * (NT / 64) + lane];
+                sources.each(p, halves, lane, [&](int i, int m) __attribute__((always_inline)) { L.polys[i] = m == MTP_NO_MOMENT ? (T)0 : A[m]; });
             } else {
                 scatter_polys<T, NT>(p, L.polys, A, lane);
             }
@@ -1323,6 +1351,9 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
             int rk = 0, ng, h, j;
             {
                 MTP_PHASE;
+                // (no load on its way beside the claims: a register of one, needed for something else, would wait for all of them.  vmcnt(0),
+                // which the claims' addresses wait for anyway.  Level 10, 216 atoms 14.3 -> 13.6 us, level 16, 64 x 128 atoms 66.2 -> 64.7)
+                __builtin_amdgcn_s_waitcnt(0x0f70);
                 if (a.seg_cursor && lane < nc) rk = pair_claim_raw(&a.seg_cursor[b * NF + nj]);
                 if constexpr (TILED) {
                     ng = NT / 64; h = wave; j = halves == 2 ? l64 & 31 : l64;
@@ -1392,6 +1423,7 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
                 T gz = gs * uz + wz * rinv;
                 if (!valid) { gx = (T)0; gy = (T)0; gz = (T)0; }
                 if (a.seg_cursor) {
+                    asm volatile("" : "+v"(rk));         // (its bits taken apart here, not where the answer is on its way)
                     rk = pair_rank(rk);
                     const bool fits = (unsigned)rk < (unsigned)a.seg_cap;
                     T* dst = a.seg_g + (size_t)(fits ? (b * NF + nj) * a.seg_cap + rk : a.seg_spare) * 3;
@@ -1442,8 +1474,6 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
     // ---- loss gradient ------------------------------------------------------------------------
     if (LOSS) {
         T cE;
-        const int halves = csize <= 32 ? 2 : 1;
-        [[maybe_unused]] int prog = 0;
         {
             MTP_PHASE;
             cE = seeded ? (T)1 : (a.cE_per_atom ? a.cE[row] : a.cE[b]);
@@ -1453,15 +1483,11 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
             // the last pass needs the adjoints of the basic moments while the table is back in its region
             if constexpr (TILED) {
                 // (B's coefficients: cE times the adjoints plus the mixed ones)
-                const int n = p.nstream[halves - 1];
-                const unsigned short* const src = p.stream_src[halves - 1];
-                for (int i = lane; i < n; i += NT) {
-                    const int m = src[i];
+                sources.each(p, halves, lane, [&](int i, int m) __attribute__((always_inline)) {
                     const T av = m == MTP_NO_MOMENT ? (T)0 : A[m];
                     L.Ab[i] = av;
                     L.Bb[i] = m == MTP_NO_MOMENT ? (T)0 : cE * av + Bm[m];
-                }
-                prog = p.units[NT / 256][2 * (NT / 64) + lane];
+                });
             } else {
                 scatter_polys<T, NT>(p, L.Ab, A, lane);
                 scatter_polys<T, NT>(p, L.Bb, Bm, lane);
