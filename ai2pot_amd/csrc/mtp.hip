@@ -99,7 +99,7 @@ struct MtpArgs {
     const T* cE;       // [B]        2 e_w / N (E - E_dft)
     const T* dFs;      // [B, P, 3]  2 f_w / (3N) (F - F_dft)
     const T* dVs;      // [B, 9]     2 v_w / (9N) (V - V_dft)
-    T* gpart;          // [B, P, ngrad] per-atom gradient rows (ngrad = ncoef + n_scalar + ntypes)
+    T* gpart;          // [B, P, ngrad] per-atom gradient rows: coefficient block of the centre's species | bias | linear coefficients
     int ngrad;
     // Places in LDS, in entries (AtomLds), and in a row of the neighbour table: worked out once for the launch.
     int at_Tg, at_cf, at_tab, at_A, at_Bm, at_gred, at_Ab, at_Bb, at_pq, at_polys, at_net, at_part, at_scratch;
@@ -548,9 +548,11 @@ template <typename T, int N>
 __device__ __forceinline__ void piece_sums(T (&v)[N], int rem, int steps)
 {
     T o[N];
-    auto add = [&](bool on) __attribute__((always_inline)) {
+    auto add = [&](bool on) __attribute__((always_inline)) {        // (selected values: twelve instructions more for six)
+        if (on) {
 #pragma unroll
-        for (int q = 0; q < N; q++) v[q] += on ? o[q] : (T)0;
+            for (int q = 0; q < N; q++) v[q] += o[q];
+        }
     };
 #pragma unroll
     for (int q = 0; q < N; q++) o[q] = wave::dpp_move<0x101>(v[q]);
@@ -997,9 +999,7 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
             if (!LOSS && a.e_sites && lane == 0) a.e_sites[row] = (T)0;
             if (!LOSS && a.desc)
                 for (int s = lane; s < p.n_scalar; s += NT) a.desc[row * p.n_scalar + s] = (T)0;
-            if (LOSS)
-                for (int q = lane; q < a.ngrad; q += NT) a.gpart[row * a.ngrad + q] = (T)0;
-            return;
+            return;                        // (its gradient row is not read)
         }
         if (nn > a.U) { if (lane == 0) atomicOr(a.status, ST_NEIGH_OVERFLOW); nn = a.U; }
         if ((unsigned)center >= (unsigned)NF) { if (lane == 0) atomicOr(a.status, ST_BAD_NEIGHBOR); center = 0; nn = 0; }
@@ -1492,15 +1492,13 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
                 scatter_polys<T, NT>(p, L.Ab, A, lane);
                 scatter_polys<T, NT>(p, L.Bb, Bm, lane);
             }
-            const int ncoef = a.ntypes * a.ntypes * nmus * K;
-            T* grow = a.gpart + row * a.ngrad;
-            for (int q = lane; q < a.ngrad; q += NT) grow[q] = (T)0;
-            __syncthreads();         // other threads overwrite some of these entries below
+            const int nblk = a.ntypes * nmus * K;
+            T* const grow = a.gpart + row * a.ngrad;
             // everything but the coefficient block is written now: the pass over the neighbours below does
             // not read the moments or their tangents, and the group sums may take their place
             if constexpr (NET) {
-                // compact row of the centre species: coefficient block | w0[H, S] | w1[H] | bias
-                const int S = p.n_scalar, H = a.H, nblk = a.ntypes * nmus * K;
+                // coefficient block of the centre's species | w0[H, S] | w1[H] | bias
+                const int S = p.n_scalar, H = a.H;
                 const T* qv = L.net;
                 const T* n_th = qv + S + H;
                 const T* n_d1 = n_th + H;
@@ -1529,8 +1527,8 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
             } else if (!seeded) {
                 // linear coefficients and bias: linearMtpLoss.h:539-554
                 for (int s = lane; s < p.n_scalar; s += NT)
-                    grow[ncoef + s] = (cE * M[p.mapping[s]] + Tg[p.mapping[s]]) / a.q_scaler[s];
-                if (lane == 0) grow[ncoef + p.n_scalar + ti] = cE;
+                    grow[nblk + 1 + s] = (cE * M[p.mapping[s]] + Tg[p.mapping[s]]) / a.q_scaler[s];
+                if (lane == 0) grow[nblk] = cE;
             }
             T* gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;          // [ntypes][nmus][K] for this centre type
             for (int q = lane; q < a.ntypes * nmus * K; q += NT) gacc[q] = (T)0;
@@ -1668,80 +1666,108 @@ __global__ void __launch_bounds__(NT, waves_of(sizeof(T) == 8, LOSS, NT)) mtp_at
         __syncthreads();
         MTP_PHASE;
         const T* const gacc = L.pq + 2 * MTP_NC * nmus + MTP_NC;
-        T* const grow = a.gpart + row * a.ngrad + (NET ? 0 : (size_t)ti * a.ntypes * nmus * K);
+        T* const grow = a.gpart + row * a.ngrad;
         for (int q = lane; q < a.ntypes * nmus * K; q += NT) grow[q] = gacc[q];
     }
 }
 #undef MTP_PHASE
 
-// out[b, q] = sum over atoms ii < binum[b] of gpart[b, ii, q], in atom order
+// Sums of the gradient rows of a structure's atoms: a lane for an entry, a wavefront for each of four runs of the rows, which is summed in
+// atom order, then the runs.  What bounds it is the trips to memory one after the other, then the rows' bytes: 64 x 128 atoms of three
+// species at level 16 8.4 -> 6.6 us (and 131 -> 128.5 for the loss gradient, which writes half as much), of a network with 20 neurons
+// 42 -> 24.6, 5 x 47 atoms at level 12 7.1 -> 4.0 (a thread for an entry and all rows, eight of them on their way, before; the rows of a
+// linear potential with the blocks of all species).
+constexpr int GRAD_RUNS = 4;
+// Over the rows of species t (all for t < 0) entry `own`; the sum is in the threads of the first wavefront.
 template <typename T>
-__global__ void __launch_bounds__(256)
-mtp_grad_reduce_kernel(int P, int ncoef, int nlin, int nbias, const int* __restrict__ binum,
-                       const T* __restrict__ gpart, T* __restrict__ dcoeffs, T* __restrict__ dlin,
-                       T* __restrict__ dbias)
+__device__ __forceinline__ T grad_rows_sum(int P, int NF, int nrow, int own, int b, int t, const int* __restrict__ binum, const int* __restrict__ bilist,
+                                           const int* __restrict__ btypes, const T* __restrict__ gpart)
 {
-    const int b = blockIdx.y;
-    const int ngrad = ncoef + nlin + nbias;
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= ngrad) return;
-    const int inum = min(binum[b], P);
+    __shared__ T runs[GRAD_RUNS - 1][64];
+    const int lane = threadIdx.x & 63, run = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int inum = max(min(binum[b], P), 0), i1 = (int)((long long)(run + 1) * inum / GRAD_RUNS);
     T acc = (T)0;
-    const T* src = gpart + (size_t)b * P * ngrad + q;
-    int ii = 0;
-    for (; ii + 8 <= inum; ii += 8) {            // eight rows in flight, added in atom order
-        T v[8];
+    // of 64 rows those of the species, sixteen on their way; the others are not read
+    for (int i0 = (int)((long long)run * inum / GRAD_RUNS); i0 < i1; i0 += 64) {
+        const int i = i0 + lane;
+        bool mine = i < i1;
+        if (t >= 0) {
+            const int c = bilist[(size_t)b * P + min(i, i1 - 1)];
+            const bool ok = mine && (unsigned)c < (unsigned)NF;
+            mine = ok && btypes[(size_t)b * NF + (ok ? c : 0)] == t;
+        }
+        unsigned long long left = __ballot(mine);
+        const T* const src = gpart + ((size_t)b * P + i0) * nrow + own;
+        while (left) {
+            T v[16];
+            const int n = __popcll(left);
+            int k = __builtin_ctzll(left);
 #pragma unroll
-        for (int u = 0; u < 8; u++) v[u] = src[(size_t)(ii + u) * ngrad];
+            for (int u = 0; u < 16; u++) {
+                v[u] = src[(size_t)k * nrow];
+                left &= left - 1;                    // (the last one again where there are fewer)
+                if (left) k = __builtin_ctzll(left);
+            }
 #pragma unroll
-        for (int u = 0; u < 8; u++) acc += v[u];
+            for (int u = 0; u < 16; u++) acc += u < n ? v[u] : (T)0;
+        }
     }
-    for (; ii < inum; ii++) acc += src[(size_t)ii * ngrad];
-    if (q < ncoef) { if (dcoeffs) dcoeffs[(size_t)b * ncoef + q] = acc; }
-    else if (q < ncoef + nlin) { if (dlin) dlin[(size_t)b * nlin + q - ncoef] = acc; }
-    else if (dbias) dbias[(size_t)b * nbias + q - ncoef - nlin] = acc;
+    if (run > 0) runs[run - 1][lane] = acc;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k + 1 < GRAD_RUNS; k++) acc += runs[k][lane];
+    return acc;
 }
 
-// The same for the compact rows of the neural-network MTP: row = [coefficient block of the centre
-// species | w0[H, S] | w1[H] | bias]; out[b] is laid out coeffs[ntypes^2 nmus K] | w0[ntypes H S] |
-// w1[ntypes H] | bias[ntypes].  Thread q of block (x, t, b) sums entry q of the rows of species t.
+// Linear potentials: row = [coefficient block of the centre's species | bias | linear coefficients], of which a launch without `dlin` and
+// `dbias` may have the block alone.  Block x < ntypes * per takes the block and bias of a species, the others the linear coefficients.
 template <typename T>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(64 * GRAD_RUNS)
+mtp_grad_reduce_kernel(int P, int NF, int nblk, int nlin, int ntypes, int nrow, const int* __restrict__ binum, const int* __restrict__ bilist,
+                       const int* __restrict__ btypes, const T* __restrict__ gpart, T* __restrict__ dcoeffs, T* __restrict__ dlin,
+                       T* __restrict__ dbias)
+{
+    const int b = blockIdx.y, per = (nblk + 64) / 64, x = blockIdx.x, lane = threadIdx.x & 63;
+    const bool block = x < ntypes * per;
+    const int t = block ? x / per : -1, q = (block ? x - t * per : x - ntypes * per) * 64 + lane;
+    const int at = block ? q : nblk + 1 + q, end = block ? min(nblk + 1, nrow) : nblk + 1 + nlin;
+    const T acc = grad_rows_sum<T>(P, NF, nrow, min(at, end - 1), b, t, binum, bilist, btypes, gpart);
+    if (threadIdx.x >= 64 || at >= end) return;
+    if (!block) { if (dlin) dlin[(size_t)b * nlin + q] = acc; }
+    else if (q < nblk) { if (dcoeffs) dcoeffs[((size_t)b * ntypes + t) * nblk + q] = acc; }
+    else if (dbias) dbias[(size_t)b * ntypes + t] = acc;
+}
+
+// Network potentials: row = [coefficient block of the centre's species | w0[H, S] | w1[H] | bias]; out[b] is laid out
+// coeffs[ntypes^2 nmus K] | w0[ntypes H S] | w1[ntypes H] | bias[ntypes].  Block (x, t, b) sums the rows of species t.
+template <typename T>
+__global__ void __launch_bounds__(64 * GRAD_RUNS)
 nnmtp_grad_reduce_kernel(int P, int NF, int nblk, int HS, int H, int ntypes, const int* __restrict__ binum,
                          const int* __restrict__ bilist, const int* __restrict__ btypes,
                          const T* __restrict__ gpart, T* __restrict__ dcoeffs, T* __restrict__ dw0,
                          T* __restrict__ dw1, T* __restrict__ dbias)
 {
-    const int b = blockIdx.z, t = blockIdx.y;
-    const int nrow = nblk + HS + H + 1;
-    const int q = blockIdx.x * 256 + threadIdx.x;
-    if (q >= nrow) return;
-    const int inum = min(binum[b], P);
-    T acc = (T)0;
-    // eight rows in flight; the rows of other species are skipped, the order of the sum is the atom order
-    for (int i0 = 0; i0 < inum; i0 += 8) {
-        int c[8], ty[8];
-        T v[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) c[u] = bilist[(size_t)b * P + min(i0 + u, inum - 1)];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const bool ok = i0 + u < inum && (unsigned)c[u] < (unsigned)NF;
-            ty[u] = btypes[(size_t)b * NF + (ok ? c[u] : 0)];
-            if (!ok) ty[u] = -1;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {            // (a row of another species is not read)
-            v[u] = (T)0;
-            if (ty[u] == t) v[u] = gpart[((size_t)b * P + min(i0 + u, inum - 1)) * nrow + q];
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) acc += v[u];
-    }
+    const int b = blockIdx.z, t = blockIdx.y, nrow = nblk + HS + H + 1, q = blockIdx.x * 64 + (threadIdx.x & 63);
+    const T acc = grad_rows_sum<T>(P, NF, nrow, min(q, nrow - 1), b, t, binum, bilist, btypes, gpart);
+    if (threadIdx.x >= 64 || q >= nrow) return;
     if (q < nblk) { if (dcoeffs) dcoeffs[((size_t)b * ntypes + t) * nblk + q] = acc; }
     else if (q < nblk + HS) { if (dw0) dw0[((size_t)b * ntypes + t) * HS + q - nblk] = acc; }
     else if (q < nblk + HS + H) { if (dw1) dw1[((size_t)b * ntypes + t) * H + q - nblk - HS] = acc; }
     else if (dbias) dbias[(size_t)b * ntypes + t] = acc;
+}
+// Length of a linear potential's row, and its sums.
+template <typename T>
+int mtp_grad_row(const MtpArgs<T>& a, bool readout) { return a.ntypes * a.p.nmus * a.K + (readout ? 1 + a.p.n_scalar : 0); }
+template <typename T>
+int mtp_grad_reduce(const MtpArgs<T>& a, bool readout, T* dcoeffs, T* dlin, T* dbias, hipStream_t stream)
+{
+    const int nblk = a.ntypes * a.p.nmus * a.K, nlin = readout ? a.p.n_scalar : 0;
+    prof_begin("mtp_grad_reduce", stream);
+    hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(a.ntypes * ((nblk + 64) / 64) + ceil_div(nlin, 64), a.B), dim3(64 * GRAD_RUNS), 0, stream, a.P,
+                       a.P + a.nghost, nblk, nlin, a.ntypes, a.ngrad, a.binum, a.bilist, a.btypes, a.gpart, dcoeffs, dlin, dbias);
+    prof_end(stream);
+    A2P_HIP_CHECK(hipGetLastError());
+    return A2P_OK;
 }
 
 // dst[(i * ncols) + col] = src[i] for i < n: one column of a row-major matrix
@@ -3504,8 +3530,7 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
     rc = fill_args(a, plan, K, scaling, coeffs, lin, bias, nmus, ntypes, q_scaler, rmax, rmin, B, P, U, 0,
                    binum, bilist, bnumneigh, bfirstneigh, brcs, btypes);
     if (rc) return rc;
-    const int ncoef = ntypes * ntypes * nmus * K;
-    const int ngrad = ncoef + a.p.n_scalar + ntypes;
+    const int ngrad = mtp_grad_row(a, true);
     const bool want_grad = dcoeffs || dlin || dbias;
     // workspace: cE[B] | dVs[B*9] | dFs[B*P*3] | gpart[B*P*ngrad] | sq[B*3] (double)
     size_t nT = (size_t)B + (size_t)B * 9 + (size_t)B * P * 3 + (want_grad ? (size_t)B * P * ngrad : 0);
@@ -3528,12 +3553,7 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
-    prof_begin("mtp_grad_reduce", stream);
-    hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(ceil_div(ngrad, 256), B), dim3(256), 0, stream, P, ncoef,
-                       a.p.n_scalar, ntypes, binum, gpart, dcoeffs, dlin, dbias);
-    prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
-    return A2P_OK;
+    return mtp_grad_reduce<T>(a, true, dcoeffs, dlin, dbias, stream);
 }
 
 // Training loss of the neural-network MTP: E/F/V, per-structure loss and the per-structure gradients
@@ -3594,7 +3614,7 @@ int nnmtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft,
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
     prof_begin("mtp_grad_reduce", stream);
-    hipLaunchKernelGGL(nnmtp_grad_reduce_kernel<T>, dim3(ceil_div(nrow, 256), ntypes, B), dim3(256), 0, stream, P, P,
+    hipLaunchKernelGGL(nnmtp_grad_reduce_kernel<T>, dim3(ceil_div(nrow, 64), ntypes, B), dim3(64 * GRAD_RUNS), 0, stream, P, P,
                        nblk, H * S, H, ntypes, binum, bilist, btypes, gpart, dcoeffs, dw0, dw1, dbias);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
@@ -3641,8 +3661,7 @@ int mtp_esites_bwd(void* handle, int K, double scaling, const T* coeffs, const T
                    binum, bilist, bnumneigh, bfirstneigh, brcs, btypes);
     if (rc) return rc;
     if (B == 0 || P == 0) return A2P_OK;
-    const int ncoef = ntypes * ntypes * nmus * K;
-    const int ngrad = ncoef + a.p.n_scalar + ntypes;
+    const int ngrad = mtp_grad_row(a, true);
     // workspace: dVs[B*9] | dFs[(B*P + nghost)*3] (both zero) | gpart[B*P*ngrad]
     const size_t nzero = (size_t)B * 9 + ((size_t)B * P + nghost) * 3;
     void* ws = nullptr;
@@ -3656,12 +3675,7 @@ int mtp_esites_bwd(void* handle, int K, double scaling, const T* coeffs, const T
     a.cE = gout; a.cE_per_atom = 1; a.no_tangent = 1; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
-    prof_begin("mtp_grad_reduce", stream);
-    hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(ceil_div(ngrad, 256), B), dim3(256), 0, stream, P, ncoef,
-                       a.p.n_scalar, ntypes, binum, gpart, dcoeffs, dlin, dbias);
-    prof_end(stream);
-    A2P_HIP_CHECK(hipGetLastError());
-    return A2P_OK;
+    return mtp_grad_reduce<T>(a, true, dcoeffs, dlin, dbias, stream);
 }
 
 // Backward of the legacy basis operator (mtpBasisOp.cc:220-326; mtpBasis.h:359-394 contracts the dense derivative
@@ -3695,11 +3709,11 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         if (rc) return rc;
     }
     if (dcoeffs) {
-        const int ncoef = ntypes * ntypes * nmus * K;
-        // workspace: dVs[B*9] | dFs[(B*P + nghost)*3] (both zero) | gpart[B*P*ncoef]
+        const int ngrad = mtp_grad_row(a, false);
+        // workspace: dVs[B*9] | dFs[(B*P + nghost)*3] (both zero) | gpart[B*P*ngrad]
         const size_t nzero = (size_t)B * 9 + ((size_t)B * P + nghost) * 3;
         void* ws = nullptr;
-        rc = ws_get(WS_MTP, (nzero + (size_t)B * P * ncoef) * sizeof(T), &ws);
+        rc = ws_get(WS_MTP, (nzero + (size_t)B * P * ngrad) * sizeof(T), &ws);
         if (rc) return rc;
         T* dVs = (T*)ws;
         T* dFs = dVs + (size_t)B * 9;
@@ -3707,14 +3721,11 @@ int mtp_basis_bwd(void* handle, int K, double scaling, const T* coeffs, int nmus
         rc = fill_zero(ws, ((nzero * sizeof(T) + 3) / 4) * 4, stream);
         if (rc) return rc;
         MtpArgs<T> g = a;
-        g.dFs = dFs; g.dVs = dVs; g.gpart = gpart; g.ngrad = ncoef; g.no_tangent = 1;
+        g.dFs = dFs; g.dVs = dVs; g.gpart = gpart; g.ngrad = ngrad; g.no_tangent = 1;
         rc = launch_atoms<T, true>(g, stream);
         if (rc) return rc;
-        prof_begin("mtp_grad_reduce", stream);
-        hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(ceil_div(ncoef, 256), B), dim3(256), 0, stream, P, ncoef, 0, 0,
-                           binum, gpart, dcoeffs, (T*)nullptr, (T*)nullptr);
-        prof_end(stream);
-        A2P_HIP_CHECK(hipGetLastError());
+        rc = mtp_grad_reduce<T>(g, false, dcoeffs, (T*)nullptr, (T*)nullptr, stream);
+        if (rc) return rc;
     }
     return A2P_OK;
 }
@@ -3985,7 +3996,7 @@ int nnmtp_esites_bwd(void* handle, int K, const MtpNet<T>& net, const T* coeffs,
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
     prof_begin("mtp_grad_reduce", stream);
-    hipLaunchKernelGGL(nnmtp_grad_reduce_kernel<T>, dim3(ceil_div(nrow, 256), ntypes, B), dim3(256), 0, stream, P,
+    hipLaunchKernelGGL(nnmtp_grad_reduce_kernel<T>, dim3(ceil_div(nrow, 64), ntypes, B), dim3(64 * GRAD_RUNS), 0, stream, P,
                        P + nghost, nblk, H * S, H, ntypes, binum, bilist, btypes, gpart, dcoeffs, dw0, dw1, dbias);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());

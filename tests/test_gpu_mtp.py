@@ -217,6 +217,23 @@ def test_loss_step(oracle, level, nt):
     assert np.array_equal(fwd["bloss"], got["bloss"]) and "dcoeffs" not in fwd
 
 
+@pytest.mark.parametrize("sizes", [(1, 2, 3), (4, 5, 16), (63, 68), (256, 257), (275, 15)], ids=str)
+def test_gradients_by_number_of_rows(oracle, sizes):
+    """The rows' gradients are summed in four runs, 64 rows and then sixteen of a species at a time: structures that leave runs empty, fill
+    them, or have one row more.  fp64 against the oracle, 1e-10."""
+    boxes = [max(4.0, (n / 0.05) ** (1 / 3)) for n in sizes]
+    nb = synth.pack_batch([structure(oracle, n, (a, a, a), 3, 41 + n, 4.0) for n, a in zip(sizes, boxes)])
+    B, P = nb["bilist"].shape
+    m = synth.mtp_model(mtp_param.mtp_param(8), 3, 8, 4.0, 1.0, 3108)
+    m["q_scaler"] = np.linspace(0.8, 1.3, m["q_scaler"].size)
+    labels = dict(energy=synth.rng_normal(1, B, -4 * 40, 3), force=synth.rng_normal(2, B * P * 3).reshape(B, P, 3),
+                  virial=synth.rng_normal(3, B * 9, 0, 0.5).reshape(B, 9))
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w), oracle.mtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dlinear", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
 def test_loss_level16_against_golden(oracle):
     """Level 16 (configuration 4's level) against the committed output of the reference's own
     find_loss_backward (tests/golden/mtp.npz), where the oracle's forward-mode derivative is slow."""

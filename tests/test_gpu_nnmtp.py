@@ -146,6 +146,21 @@ def test_loss_step_complete_derivative(oracle, level, nt, H):
     assert np.array_equal(fwd["bloss"], got["bloss"]) and "dcoeffs" not in fwd
 
 
+@pytest.mark.parametrize("sizes", [(1, 2, 3), (4, 5, 16), (63, 68), (256, 257), (275, 15)], ids=str)
+def test_gradients_by_number_of_rows(oracle, sizes):
+    """The rows' gradients are summed in four runs, 64 rows and then sixteen of a species at a time, as those of the linear potentials."""
+    boxes = [max(4.0, (n / 0.05) ** (1 / 3)) for n in sizes]
+    nb = synth.pack_batch([structure(oracle, n, (a, a, a), 3, 41 + n, 4.0) for n, a in zip(sizes, boxes)])
+    B, P = nb["bilist"].shape
+    m = synth.nnmtp_model(mtp_param.mtp_param(8), 3, 8, 5, 4.0, 1.0, 3408, lo=-0.05, hi=0.05)
+    labels = dict(energy=synth.rng_normal(1, B, -4 * 40, 3), force=synth.rng_normal(2, B * P * 3).reshape(B, P, 3),
+                  virial=synth.rng_normal(3, B * 9, 0, 0.5).reshape(B, 9))
+    w = (1.0, 0.7, 0.3)
+    got, ref = gpu_loss(m, nb, labels, w, True), oracle.nnmtp_loss_step(m, nb, w, labels)
+    for k in ("bloss", "dcoeffs", "dw0", "dw1", "dbias"):
+        assert close(got[k], ref[k]), k
+
+
 @pytest.mark.parametrize("level", [8, 12, 16])              # 9, 29 and 92 inputs; 64 threads, and 256 for the loss gradient
 @pytest.mark.parametrize("H", [1, 4, 5, 16, 33, 65, 257])
 def test_readout_by_neighbouring_lanes(oracle, level, H):
