@@ -56,12 +56,22 @@ loss_forward_kernel(int P, const int* __restrict__ binum, const int* __restrict_
 }
 
 // One wavefront: the structures' squared errors by lane, then by a fixed tree (a single thread over 64 structures took
-// 8 us, all of it the latency of its loads).
+// 8 us, all of it the latency of its loads).  Where the gradient is wanted too, a workgroup of its last kernel does this (5 us for a launch
+// of its own between two kernels that do not need it).
 template <typename T>
-__global__ void __launch_bounds__(64)
-loss_rmse_kernel(int B, const int* __restrict__ binum, const double* __restrict__ sq, T* __restrict__ rmse)
+struct LossRmse {
+    int B;
+    const int* binum;
+    const double* sq;
+    T* rmse;
+};
+template <typename T>
+__device__ __forceinline__ void loss_rmse(const LossRmse<T>& r, int lane)
 {
-    const int lane = (int)threadIdx.x;
+    const int B = r.B;
+    const int* const binum = r.binum;
+    const double* const sq = r.sq;
+    T* const rmse = r.rmse;
     double e = 0, f = 0, v = 0, nf = 0;
     for (int b = lane; b < B; b += 64) {
         e += sq[b * 3]; f += sq[b * 3 + 1]; v += sq[b * 3 + 2];
@@ -74,6 +84,8 @@ loss_rmse_kernel(int B, const int* __restrict__ binum, const double* __restrict_
         rmse[2] = (T)sqrt(v / (9.0 * B));
     }
 }
+template <typename T>
+__global__ void __launch_bounds__(64) loss_rmse_kernel(const LossRmse<T> r) { loss_rmse(r, (int)threadIdx.x); }
 
 }  // namespace losskern
 }  // namespace a2p

@@ -1725,9 +1725,13 @@ template <typename T>
 __global__ void __launch_bounds__(64 * GRAD_RUNS)
 mtp_grad_reduce_kernel(int P, int NF, int nblk, int nlin, int ntypes, int nrow, const int* __restrict__ binum, const int* __restrict__ bilist,
                        const int* __restrict__ btypes, const T* __restrict__ gpart, T* __restrict__ dcoeffs, T* __restrict__ dlin,
-                       T* __restrict__ dbias)
+                       T* __restrict__ dbias, const losskern::LossRmse<T> errors)
 {
     const int b = blockIdx.y, per = (nblk + 64) / 64, x = blockIdx.x, lane = threadIdx.x & 63;
+    if (x * 64 >= ntypes * per * 64 + nlin) {               // (a workgroup per structure too many, of which the first has the batch's errors)
+        if (b == 0 && threadIdx.x < 64) losskern::loss_rmse(errors, lane);
+        return;
+    }
     const bool block = x < ntypes * per;
     const int t = block ? x / per : -1, q = (block ? x - t * per : x - ntypes * per) * 64 + lane;
     const int at = block ? q : nblk + 1 + q, end = block ? min(nblk + 1, nrow) : nblk + 1 + nlin;
@@ -1759,12 +1763,12 @@ nnmtp_grad_reduce_kernel(int P, int NF, int nblk, int HS, int H, int ntypes, con
 template <typename T>
 int mtp_grad_row(const MtpArgs<T>& a, bool readout) { return a.ntypes * a.p.nmus * a.K + (readout ? 1 + a.p.n_scalar : 0); }
 template <typename T>
-int mtp_grad_reduce(const MtpArgs<T>& a, bool readout, T* dcoeffs, T* dlin, T* dbias, hipStream_t stream)
+int mtp_grad_reduce(const MtpArgs<T>& a, bool readout, T* dcoeffs, T* dlin, T* dbias, hipStream_t stream, const losskern::LossRmse<T>& errors = {})
 {
     const int nblk = a.ntypes * a.p.nmus * a.K, nlin = readout ? a.p.n_scalar : 0;
     prof_begin("mtp_grad_reduce", stream);
-    hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(a.ntypes * ((nblk + 64) / 64) + ceil_div(nlin, 64), a.B), dim3(64 * GRAD_RUNS), 0, stream, a.P,
-                       a.P + a.nghost, nblk, nlin, a.ntypes, a.ngrad, a.binum, a.bilist, a.btypes, a.gpart, dcoeffs, dlin, dbias);
+    hipLaunchKernelGGL(mtp_grad_reduce_kernel<T>, dim3(a.ntypes * ((nblk + 64) / 64) + ceil_div(nlin, 64) + (errors.rmse ? 1 : 0), a.B), dim3(64 * GRAD_RUNS), 0, stream, a.P,
+                       a.P + a.nghost, nblk, nlin, a.ntypes, a.ngrad, a.binum, a.bilist, a.btypes, a.gpart, dcoeffs, dlin, dbias, errors);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     return A2P_OK;
@@ -3546,14 +3550,15 @@ int mtp_loss(void* handle, double e_w, double f_w, double v_w, const T* e_dft, c
     prof_begin("mtp_loss_forward", stream);
     hipLaunchKernelGGL(losskern::loss_forward_kernel<T>, dim3(B), dim3(256), 0, stream, P, binum, bilist, (T)e_w,
                        (T)f_w, (T)v_w, etot, e_dft, force, f_dft, virial, v_dft, bloss, cE, dFs, dVs, sq, 1);
-    if (rmse) hipLaunchKernelGGL(losskern::loss_rmse_kernel<T>, dim3(1), dim3(64), 0, stream, B, binum, sq, rmse);
+    const losskern::LossRmse<T> errors{B, binum, sq, rmse};
+    if (rmse && !want_grad) hipLaunchKernelGGL(losskern::loss_rmse_kernel<T>, dim3(1), dim3(64), 0, stream, errors);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;
     a.cE = cE; a.dFs = dFs; a.dVs = dVs; a.gpart = gpart; a.ngrad = ngrad;
     rc = launch_atoms<T, true>(a, stream);
     if (rc) return rc;
-    return mtp_grad_reduce<T>(a, true, dcoeffs, dlin, dbias, stream);
+    return mtp_grad_reduce<T>(a, true, dcoeffs, dlin, dbias, stream, errors);
 }
 
 // Training loss of the neural-network MTP: E/F/V, per-structure loss and the per-structure gradients

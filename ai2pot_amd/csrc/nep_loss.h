@@ -1,6 +1,7 @@
 // What the kernels of the NEP training loss share (nep_loss.hip: any shape; nep_loss_wave.hip: the common shapes).
 #pragma once
 #include "a2p_common.h"
+#include "loss_kernels.h"
 
 namespace a2p {
 namespace nepdev {
@@ -19,6 +20,7 @@ struct NepLossArgs {
     int nrow;
     int E;             // table entries per neighbour (generic kernel)
     int* status;
+    losskern::LossRmse<T> errors;      // (rmse null: not wanted, or a launch of its own)
 };
 
 __device__ __forceinline__ int l_of_lm(int m) { return m < 3 ? 1 : m < 8 ? 2 : m < 15 ? 3 : 4; }

@@ -434,7 +434,8 @@ int nep_loss(double e_w, double f_w, double v_w, const T* e_dft, const T* f_dft,
     prof_begin("nep_loss_forward", stream);
     hipLaunchKernelGGL(losskern::loss_forward_kernel<T>, dim3(B), dim3(256), 0, stream, P, binum, bilist, (T)e_w,
                        (T)f_w, (T)v_w, etot, e_dft, force, f_dft, virial, v_dft, bloss, cE, dFs, dVs, sq, 0);
-    if (rmse) hipLaunchKernelGGL(losskern::loss_rmse_kernel<T>, dim3(1), dim3(64), 0, stream, B, binum, sq, rmse);
+    a.errors = {B, binum, sq, rmse};
+    if (rmse && !(wave && want_grad)) hipLaunchKernelGGL(losskern::loss_rmse_kernel<T>, dim3(1), dim3(64), 0, stream, a.errors);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
     if (!want_grad) return A2P_OK;

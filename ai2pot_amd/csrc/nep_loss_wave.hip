@@ -463,6 +463,10 @@ nep_loss_wave_reduce_kernel(const NepLossArgs<T> a, int sum_blocks, T* __restric
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, c16 = lane & 15, k4 = lane >> 4;
     const int t = blockIdx.y, b = blockIdx.z, nt = a.ntypes, H = a.H, D = a.D;
     const int ncl = nt * (a.n_r + a.n_a) * a.K, job = blockIdx.x;
+    if (job >= sum_blocks + (H + 63) / 64) {                   // (one more for the batch's errors)
+        if (t == 0 && b == 0 && wave == 0) losskern::loss_rmse(a.errors, lane);
+        return;
+    }
     const bool sums = job < sum_blocks;
     const int e = min(job * 64 + lane, ncl + 2 * H - 1);         // element of a row
     const int p0 = (job - sum_blocks) * 64 + wave * 16, p = min(p0 + c16, H - 1);
@@ -601,7 +605,7 @@ int nep_loss_wave_run(const NepLossArgs<T>& a, size_t lds_bytes, T* dcoeffs, T* 
     if (rc) return rc;
     const int sum_blocks = ceil_div(a.ntypes * (a.n_r + a.n_a) * a.K + 2 * a.H, 64);
     prof_begin("nep_grad_reduce", stream);
-    hipLaunchKernelGGL(nep_loss_wave_reduce_kernel<T>, dim3(sum_blocks + ceil_div(a.H, 64), a.ntypes, a.B), dim3(256), 0,
+    hipLaunchKernelGGL(nep_loss_wave_reduce_kernel<T>, dim3(sum_blocks + ceil_div(a.H, 64) + (a.errors.rmse ? 1 : 0), a.ntypes, a.B), dim3(256), 0,
                        stream, a, sum_blocks, dcoeffs, dw0, db0, dw1, dbias);
     prof_end(stream);
     A2P_HIP_CHECK(hipGetLastError());
