@@ -3,20 +3,20 @@
 //
 // One workgroup (64 threads, or 256 for the larger levels) per centre atom; the moment vector M,
 // its adjoint and (for the loss gradient) the tangent and mixed vectors live in LDS.  Neighbours
-// are processed in equal chunks of at most 32 to 48: a per-neighbour table (powers of the unit vector, contracted
+// are processed in equal chunks of at most 16 to 48: a per-neighbour table (powers of the unit vector, contracted
 // radial functions g_mu(r) = sum_k c[ti,tj,mu,k] f_k(r) and their r-derivatives) is staged
 // in LDS, then
-//   basic moments : lane <- basic moment i,  M_i += sum_j g_mu(r_j) ux^a uy^b uz^c
-//                   (x^a y^b z^c / r^(a+b+c) of the reference, include/mtpBasis.h:472-519,
+//   basic moments : M_(mu,a,b,c) = sum_j g_mu(r_j) ux^a uy^b uz^c as products of matrices over the neighbours, rows (a, b)
+//                   and columns (mu, c)     (x^a y^b z^c / r^(a+b+c) of the reference, include/mtpBasis.h:472-519,
 //                    written with the unit vector u = r_ij / r)
 //   products      : level-ordered gather over the host-built plan (mtp_plan.h)
 //   energy        : E_i = bias[t] + sum_s lin[s] M[map[s]] / q_scaler[s]  (linearMtp.h:281-285)
 //   adjoint       : seed + reverse gather                                  (linearMtp.h:292-306)
-//   pair forces   : lane <- (neighbour, a share of the monomial rows x^a y^b z^*):
+//   pair forces   : lane <- neighbour (or half of one), wavefronts share the (mu, c):
 //                   dE_i/dr_ij = u sum_i adj_i m_i (g' - k g / r) + (1/r) sum_i adj_i g grad_u m_i
-//                   with the adjoints gathered by monomial and z^c by recurrence (pair_walk; three uniform
-//                   LDS reads per monomial instead of ten scattered ones per basic moment)
+//                   by polynomials nested in (x, y, z) whose coefficients are the adjoints
 //                   -> reduction segments of the neighbours (a2p::PairCsr), summed without float atomics
+// Tables that the products and the nested polynomials do not fit (mtp_plan.h: ntiles) go by basic moments and by polynomials in z.
 // The loss gradient adds the tangent sweep (include/linearMtpLoss.h:371-398), the mixed
 // adjoint (:417-434) and the coefficient-gradient pass (:438-536) in the same structure;
 // per-structure gradients are accumulated per workgroup and summed by a second kernel.
